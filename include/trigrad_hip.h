@@ -327,6 +327,20 @@ int tg_render_forward(const tg_real *vertices, const int32_t *indices, const tg_
                       tg_real *last_depth, uint16_t *fragments, uint64_t *hit_masks,
                       const tg_real *batch_bounds, const int32_t *far_start, const uint32_t *list_status, void *stream);
 
+/* Per-pixel order with the blend order saved whatever max_layers is: a pixel blends an entry of its tile's list at
+ * most once, so a tile with a list of n entries is given n rows of `order_pool`, a row holding one uint16 list position
+ * per pixel of a tile (rounded up to whole waves).  tg_order_pool_words: the uint16 words of the pool (with more than
+ * 65535 triangles lists can be longer than 16 bits count, and the positions' high halves take as many words again).
+ * The pool is private to tg_render_forward_pooled and tg_render_backward_pooled; words of layers that are not blended
+ * are never touched. */
+int64_t tg_order_pool_words(int64_t n_keys, int64_t n_triangles, int tile_w, int tile_h);
+int tg_render_forward_pooled(const tg_real *vertices, const int32_t *indices, int32_t n_triangles, const tg_real *colors,
+                             const tg_real *opacities, const int32_t *sorted_ids, const int32_t *offsets, int64_t n_keys,
+                             const tg_real *bary, int width, int height, int tile_w, int tile_h,
+                             tg_real early_stopping_threshold, int max_layers, tg_real *image, tg_real *depthmap,
+                             tg_real *final_weights, int32_t *ends, int32_t *last, tg_real *last_depth, uint16_t *order_pool,
+                             const tg_real *batch_bounds, const int32_t *far_start, const uint32_t *list_status, void *stream);
+
 /* ---- (5) backward ----------------------------------------------------------- */
 
 /* Accumulates into grad_vertices (V,4), grad_colors (V,3), grad_opacities (V),
@@ -349,6 +363,15 @@ int tg_render_backward(const tg_real *grad_image, const tg_real *grad_depthmap, 
                        tg_real early_stopping_threshold, int per_pixel_sort, int max_layers, tg_real *grad_vertices,
                        tg_real *grad_colors, tg_real *grad_opacities, int vertex_stride, int color_stride,
                        int opacity_stride, void *stream);
+
+/* The same with the blend order in the pool that tg_render_forward_pooled filled. */
+int tg_render_backward_pooled(const tg_real *grad_image, const tg_real *grad_depthmap, const tg_real *vertices,
+                              const int32_t *indices, int32_t n_triangles, const tg_real *colors, const tg_real *opacities,
+                              const int32_t *sorted_ids, const int32_t *offsets, int64_t n_keys, const tg_real *bary,
+                              const tg_real *image, const tg_real *depthmap, const tg_real *final_weights, const int32_t *ends,
+                              const int32_t *last, const uint16_t *order_pool, int width, int height, int tile_w, int tile_h,
+                              tg_real early_stopping_threshold, int max_layers, tg_real *grad_vertices, tg_real *grad_colors,
+                              tg_real *grad_opacities, int vertex_stride, int color_stride, int opacity_stride, void *stream);
 
 /* The (V,8) block that tg_render_backward accumulates into with strides
  * (8, 8, 8) -> the three dense arrays the reference's render_backward returns

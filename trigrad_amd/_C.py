@@ -96,6 +96,9 @@ MAX_SAVED_LAYERS = 32  # TG_MAX_SAVED_LAYERS of the C header
 # blend order (16-bit planes, see saved_blend_order) and the backward pass walks it in reverse instead of
 # selecting the fragments again.  False trades the memory for the re-selection.
 SAVE_BLEND_ORDER = True
+# With more layers than that the order goes to a pool that holds one word per (pixel, entry of its tile's list)
+# (tg_order_pool_words), as long as the pool takes no more bytes than this; else the backward pass selects again.
+ORDER_POOL_MAX_BYTES = 4 << 30
 # Without per_pixel_sort the forward pass saves which list entries cover which pixel (one bit per pair it
 # looked at) and the backward pass reads that back instead of repeating the inside tests.
 SAVE_HIT_MASKS = True
@@ -579,11 +582,28 @@ def verify_finished_frames():
     verify_frames(wait=False)
 
 
+class Resume(tuple):
+    """(last, last_depth, status_check, fragments, hit_masks), and as an attribute the pool with the blend order of a
+    pass with more than MAX_SAVED_LAYERS layers (None: no such order was saved)."""
+    order_pool = None
+
+
+def _order_pool(n_keys, n_triangles, tile_width, tile_height, device):
+    """A pool for the blend order of n_keys list entries, or None if it would be too large.  Its size is rounded up to an
+    eighth of a power of two, so that a scene whose K drifts from frame to frame gets the same block of memory again."""
+    words = int(_lib.load(32).tg_order_pool_words(n_keys, n_triangles, tile_width, tile_height))
+    if words == 0 or words * 2 > ORDER_POOL_MAX_BYTES:
+        return None
+    step = 1 << max(words.bit_length() - 4, 10)
+    return torch.empty((-(-words // step) * step,), dtype=torch.int16, device=device)
+
+
 def _forward_full(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
-                  early_stopping_threshold, disable_timing, per_pixel_sort, max_layers):
+                  early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward=True):
     """render_forward's eight results plus `resume` = (last, last_depth, status_check, fragments, hit_masks):
     what the backward pass needs for its reverse traversal (fragments / hit_masks are None unless the blend
-    order / the hit masks were saved) and the status word of the list kernels on its way to the host."""
+    order / the hit masks were saved) and the status word of the list kernels on its way to the host.
+    for_backward=False: no backward pass will follow, nothing is saved for it."""
     _need_cuda(vertices, indices, colors, opacities)
     verify_finished_frames()
     bits = _bits(vertices)
@@ -601,10 +621,12 @@ def _forward_full(vertices, indices, colors, opacities, width, height, tile_widt
         depthmap = torch.empty((height, width), dtype=real, device=dev)
         final_weights = torch.empty((height, width), dtype=real, device=dev)
         ends = torch.empty((height, width), dtype=torch.int32, device=dev)
-        last = torch.empty((height, width), dtype=torch.int32, device=dev)
-        last_depth = torch.empty((height, width), dtype=real, device=dev) if per_pixel_sort else None
-        save_order = bool(per_pixel_sort) and SAVE_BLEND_ORDER and 0 < int(max_layers) <= MAX_SAVED_LAYERS
-        fragments = torch.empty((2 * int(max_layers), height, width), dtype=torch.int16, device=dev) if save_order else None
+        last = torch.empty((height, width), dtype=torch.int32, device=dev) if for_backward else None
+        last_depth = torch.empty((height, width), dtype=real, device=dev) if per_pixel_sort and for_backward else None
+        save_order = bool(per_pixel_sort) and SAVE_BLEND_ORDER and for_backward
+        fragments = order_pool = None
+        if save_order and 0 < int(max_layers) <= MAX_SAVED_LAYERS:
+            fragments = torch.empty((2 * int(max_layers), height, width), dtype=torch.int16, device=dev)
 
         timer.start("per_tile_lists")
         T = num_tiles(width, height, tile_width, tile_height)
@@ -666,25 +688,35 @@ def _forward_full(vertices, indices, colors, opacities, width, height, tile_widt
                                           _ptr(sorted_ids), _ptr(offsets), T, _ptr(triangle_low), _ptr(batch_bounds),
                                           _ptr(far_start), _stream(vertices)), "tg_list_bounds", bits)
         hit_masks = None
-        if not per_pixel_sort and SAVE_HIT_MASKS:
+        if not per_pixel_sort and SAVE_HIT_MASKS and for_backward:
             words = int(lib.tg_hit_mask_words(K, width, height, tile_width, tile_height))
             hit_masks = torch.empty((words,), dtype=torch.int64, device=dev)
-        _lib.check(lib.tg_render_forward(
-            _ptr(vertices), _ptr(indices), _ptr(colors), _ptr(opacities), _ptr(sorted_ids), _ptr(offsets), _ptr(bary_transforms),
-            width, height, tile_width, tile_height, float(early_stopping_threshold), int(bool(per_pixel_sort)), int(max_layers),
-            _ptr(image), _ptr(depthmap), _ptr(final_weights), _ptr(ends), _ptr(last), _ptr(last_depth), _ptr(fragments),
-            _ptr(hit_masks), _ptr(batch_bounds), _ptr(far_start), _ptr(sort_status), _stream(vertices)), "tg_render_forward", bits)
+        if save_order and fragments is None and K > 0:
+            order_pool = _order_pool(K, indices.shape[0], tile_width, tile_height, dev)
+        if order_pool is not None:
+            _lib.check(lib.tg_render_forward_pooled(
+                _ptr(vertices), _ptr(indices), indices.shape[0], _ptr(colors), _ptr(opacities), _ptr(sorted_ids), _ptr(offsets), K,
+                _ptr(bary_transforms), width, height, tile_width, tile_height, float(early_stopping_threshold), int(max_layers),
+                _ptr(image), _ptr(depthmap), _ptr(final_weights), _ptr(ends), _ptr(last), _ptr(last_depth), _ptr(order_pool),
+                _ptr(batch_bounds), _ptr(far_start), _ptr(sort_status), _stream(vertices)), "tg_render_forward_pooled", bits)
+        else:
+            _lib.check(lib.tg_render_forward(
+                _ptr(vertices), _ptr(indices), _ptr(colors), _ptr(opacities), _ptr(sorted_ids), _ptr(offsets), _ptr(bary_transforms),
+                width, height, tile_width, tile_height, float(early_stopping_threshold), int(bool(per_pixel_sort)), int(max_layers),
+                _ptr(image), _ptr(depthmap), _ptr(final_weights), _ptr(ends), _ptr(last), _ptr(last_depth), _ptr(fragments),
+                _ptr(hit_masks), _ptr(batch_bounds), _ptr(far_start), _ptr(sort_status), _stream(vertices)), "tg_render_forward", bits)
         timings = timer.stop()
         if not disable_timing:  # the timer has waited for the stream anyway
             if status_check.failed() and not _tickets_forced:
                 # the lists are invalid (and the image NaN): the whole frame once more, its tiles numbered by ticket
                 force_tickets(True)
                 return _forward_full(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
-                                     early_stopping_threshold, disable_timing, per_pixel_sort, max_layers)
+                                     early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward)
             status_check.checked = False
             status_check.verify()
-    return (image, depthmap, final_weights, sorted_ids, offsets, bary_transforms, ends, timings,
-            (last, last_depth, status_check, fragments, hit_masks))
+    resume = Resume((last, last_depth, status_check, fragments, hit_masks))
+    resume.order_pool = order_pool
+    return image, depthmap, final_weights, sorted_ids, offsets, bary_transforms, ends, timings, resume
 
 
 def render_forward(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
@@ -754,6 +786,7 @@ def render_backward(grad_output, grad_depthmap, vertices, indices, colors, opaci
             resume = _resume_by_forward(*tensors[2:9], width, height, tile_width, tile_height, early_stopping_threshold,
                                         per_pixel_sort, max_layers)
         last, last_depth, status_check, fragments, hit_masks = resume
+        order_pool = getattr(resume, "order_pool", None)
         if status_check is not None:
             status_check.verify()
         tensors.append(last.contiguous())
@@ -775,10 +808,17 @@ def render_backward(grad_output, grad_depthmap, vertices, indices, colors, opaci
             grad_vertices = torch.zeros((V, sv), dtype=vertices.dtype, device=dev)[:, :4]
             grad_colors = torch.zeros((V, sc), dtype=vertices.dtype, device=dev)[:, :3]
             grad_opacities = torch.zeros((V, so), dtype=vertices.dtype, device=dev)[:, 0]
-        _lib.check(lib.tg_render_backward(
-            *[_ptr(t) for t in tensors], _ptr(last_depth), _ptr(fragments), _ptr(hit_masks), width, height, tile_width, tile_height,
-            float(early_stopping_threshold), int(bool(per_pixel_sort)), int(max_layers), _ptr(grad_vertices), _ptr(grad_colors),
-            _ptr(grad_opacities), *strides, _stream(vertices)), "tg_render_backward", bits)
+        if order_pool is not None:
+            p = [_ptr(t) for t in tensors]
+            _lib.check(lib.tg_render_backward_pooled(
+                *p[:4], indices.shape[0], *p[4:8], sorted_ids.numel(), *p[8:], _ptr(order_pool), width, height, tile_width, tile_height,
+                float(early_stopping_threshold), int(max_layers), _ptr(grad_vertices), _ptr(grad_colors), _ptr(grad_opacities), *strides,
+                _stream(vertices)), "tg_render_backward_pooled", bits)
+        else:
+            _lib.check(lib.tg_render_backward(
+                *[_ptr(t) for t in tensors], _ptr(last_depth), _ptr(fragments), _ptr(hit_masks), width, height, tile_width, tile_height,
+                float(early_stopping_threshold), int(bool(per_pixel_sort)), int(max_layers), _ptr(grad_vertices), _ptr(grad_colors),
+                _ptr(grad_opacities), *strides, _stream(vertices)), "tg_render_backward", bits)
         if strides == (8, 8, 8):
             grad_vertices = torch.empty((V, 4), dtype=vertices.dtype, device=dev)
             grad_colors = torch.empty((V, 3), dtype=vertices.dtype, device=dev)

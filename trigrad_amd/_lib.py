@@ -58,7 +58,10 @@ SIGNATURES = {
     "tg_list_bounds": (_i, [_p, _i32, _p, _i32, _p, _p, _p, _i, _p, _p, _p, _p]),
     "tg_hit_mask_words": (_sz, [_i64, _i, _i, _i, _i]),
     "tg_render_forward": (_i, [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _f, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
+    "tg_order_pool_words": (_i64, [_i64, _i64, _i, _i]),
+    "tg_render_forward_pooled": (_i, [_p, _p, _i32, _p, _p, _p, _p, _i64, _p, _i, _i, _i, _i, _f, _i] + [_p] * 11),
     "tg_render_backward": (_i, [_p] * 17 + [_i, _i, _i, _i, _f, _i, _i, _p, _p, _p, _i, _i, _i, _p]),
+    "tg_render_backward_pooled": (_i, [_p] * 4 + [_i32] + [_p] * 4 + [_i64] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p, _p, _p, _i, _i, _i, _p]),
     "tg_split_gradient_block": (_i, [_p, _i64, _p, _p, _p, _p]),
     "tg_barycentric": (None, [_p] * 5),
     "tg_barycentric_backward": (None, [_p] * 6),

@@ -31,7 +31,7 @@ struct BackwardArgs {
     const int32_t *ends;
     const int32_t *last;
     const real *last_depth;
-    const uint16_t *fragments;  // saved by the forward pass (low halves, then high halves for long lists), or null
+    OrderStore order;          // the blend order saved by the forward pass
     const uint64_t *hit_masks; // saved by the tile-order forward pass, or null
     real *grad_vertices;
     real *grad_colors;
@@ -832,11 +832,11 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
         st = load_back_state(g, p);
         n = min(g.ends[p.index], a.max_layers);  // render.cu:642
     }
-    const int64_t plane = (int64_t)a.W * a.H;
-    const bool long_list = end - start > 0xffff;  // then the positions' high halves were saved as well
+    const int64_t plane = order_stride(g.order, a);
+    const bool long_list = end - start > kShortList;  // then the positions' high halves were saved as well
     // The list positions of my steps, one after the other: step s is layer n - 1 - s, a plane further down each time.
-    const uint16_t *next_layer = g.fragments + ((int64_t)(n - 1) * plane + (p.valid ? p.index : 0));
-    const int64_t high_halves = (int64_t)a.max_layers * plane;
+    const uint16_t *next_layer = g.order.low + ((int64_t)(n - 1) * plane + order_first(g.order, p, start, blockIdx.z * blockDim.x + tid));
+    const int64_t high_halves = g.order.high;
     int steps_read = 0;
     auto next_position = [&]() {
         int position = -1;  // no such step: below every threshold
@@ -1008,11 +1008,11 @@ size_t backward_pixel_order_lds_bytes(int n_threads) { return pixel_order_lds_by
 
 using namespace tg;
 
-extern "C" int tg_render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices,
+static int render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices,
                                   const int32_t *indices, const real *colors, const real *opacities,
                                   const int32_t *sorted_ids, const int32_t *offsets, const real *bary, const real *image,
                                   const real *depthmap, const real *final_weights, const int32_t *ends, const int32_t *last,
-                                  const real *last_depth, const uint16_t *fragments, const uint64_t *hit_masks, int width,
+                                  const real *last_depth, const OrderStore &order, const uint64_t *hit_masks, int width,
                                   int height, int tile_w,
                                   int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers, real *grad_vertices,
                                   real *grad_colors, real *grad_opacities, int vertex_stride, int color_stride,
@@ -1020,7 +1020,7 @@ extern "C" int tg_render_backward(const real *grad_image, const real *grad_depth
     if (int e = check_raster_args("tg_render_backward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!grad_image || !vertices || !indices || !colors || !opacities || !offsets || !bary || !image ||
         !depthmap || !final_weights || !ends || !last || !grad_vertices || !grad_colors || !grad_opacities ||
-        (per_pixel_sort && !last_depth && !fragments)) {
+        (per_pixel_sort && !last_depth && !order.low)) {
         set_error("tg_render_backward: null pointer");
         return TG_E_ARG;
     }
@@ -1035,7 +1035,7 @@ extern "C" int tg_render_backward(const real *grad_image, const real *grad_depth
     RasterArgs a{(const real4 *)vertices, indices, colors, opacities, sorted_ids, offsets, bary, nullptr, nullptr,
                  width, height, tile_w, tile_h, early_stopping_threshold, max_layers};
     BackwardArgs g{(const real4 *)grad_image, grad_depthmap, (const real4 *)image, depthmap, final_weights, ends, last,
-                   last_depth, fragments, per_pixel_sort ? nullptr : hit_masks, grad_vertices, grad_colors, grad_opacities,
+                   last_depth, order, per_pixel_sort ? nullptr : hit_masks, grad_vertices, grad_colors, grad_opacities,
                    vertex_stride, color_stride, opacity_stride};
     hipStream_t s = (hipStream_t)stream;
     const int layout = (vertex_stride == 4 && color_stride == 3 && opacity_stride == 1)   ? kGradDense
@@ -1052,11 +1052,7 @@ extern "C" int tg_render_backward(const real *grad_image, const real *grad_depth
         TG_LAUNCH_BACKWARD(backward_tile_order_kernel, tl.grid, dim3(tl.threads), 0);
         return check_launch("backward_tile_order_kernel");
     }
-    if (fragments) {
-        if (max_layers > TG_MAX_SAVED_LAYERS) {
-            set_error("tg_render_backward: saved fragments need max_layers <= %d", TG_MAX_SAVED_LAYERS);
-            return TG_E_ARG;
-        }
+    if (order.low) {
         const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, kTileThreads);
         TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), 0);
         return check_launch("backward_saved_order_kernel");
@@ -1071,6 +1067,43 @@ extern "C" int tg_render_backward(const real *grad_image, const real *grad_depth
     TG_LAUNCH_BACKWARD(backward_pixel_order_kernel, tl.grid, dim3(tl.threads), lds);
     return check_launch("backward_pixel_order_kernel");
 #undef TG_LAUNCH_BACKWARD
+}
+
+extern "C" int tg_render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices,
+                                  const int32_t *indices, const real *colors, const real *opacities,
+                                  const int32_t *sorted_ids, const int32_t *offsets, const real *bary, const real *image,
+                                  const real *depthmap, const real *final_weights, const int32_t *ends, const int32_t *last,
+                                  const real *last_depth, const uint16_t *fragments, const uint64_t *hit_masks, int width,
+                                  int height, int tile_w, int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers,
+                                  real *grad_vertices, real *grad_colors, real *grad_opacities, int vertex_stride, int color_stride,
+                                  int opacity_stride, void *stream) {
+    if (fragments && per_pixel_sort && max_layers > TG_MAX_SAVED_LAYERS) {
+        set_error("tg_render_backward: saved fragments need max_layers <= %d", TG_MAX_SAVED_LAYERS);
+        return TG_E_ARG;
+    }
+    const OrderStore order{const_cast<uint16_t *>(fragments), (int64_t)max_layers * width * height, 0};
+    return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
+                           final_weights, ends, last, last_depth, order, hit_masks, width, height, tile_w, tile_h,
+                           early_stopping_threshold, per_pixel_sort, max_layers, grad_vertices, grad_colors, grad_opacities,
+                           vertex_stride, color_stride, opacity_stride, stream);
+}
+
+extern "C" int tg_render_backward_pooled(const real *grad_image, const real *grad_depthmap, const real *vertices,
+                                         const int32_t *indices, int32_t n_triangles, const real *colors, const real *opacities,
+                                         const int32_t *sorted_ids, const int32_t *offsets, int64_t n_keys, const real *bary,
+                                         const real *image, const real *depthmap, const real *final_weights, const int32_t *ends,
+                                         const int32_t *last, const uint16_t *order_pool, int width, int height, int tile_w, int tile_h,
+                                         real early_stopping_threshold, int max_layers, real *grad_vertices, real *grad_colors,
+                                         real *grad_opacities, int vertex_stride, int color_stride, int opacity_stride, void *stream) {
+    if (!order_pool || n_keys < 0 || n_triangles < 0) {
+        set_error("tg_render_backward_pooled: null order pool or negative count");
+        return TG_E_ARG;
+    }
+    const int pixels = order_pool_pixels(tile_w, tile_h);
+    const OrderStore order{const_cast<uint16_t *>(order_pool), n_triangles > kShortList ? n_keys * pixels : 0, pixels};
+    return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
+                           final_weights, ends, last, nullptr, order, nullptr, width, height, tile_w, tile_h, early_stopping_threshold,
+                           1, max_layers, grad_vertices, grad_colors, grad_opacities, vertex_stride, color_stride, opacity_stride, stream);
 }
 
 extern "C" int tg_split_gradient_block(const real *block, int64_t n_vertices, real *grad_vertices, real *grad_colors,

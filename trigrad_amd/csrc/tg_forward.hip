@@ -23,10 +23,7 @@ struct ForwardOut {
     int32_t *ends;
     int32_t *last;
     real *last_depth;
-    // Blend order, may be null: 2 * max_layers planes of H * W 16-bit words.  Plane l holds the low half of the
-    // list position (relative to the tile's start) of every pixel's layer l; plane max_layers + l the high half,
-    // written and read only in tiles whose list is longer than kShortList.
-    uint16_t *fragments;
+    OrderStore order;    // blend order: list positions relative to the tile's start
     uint64_t *hit_masks; // tile order: which list entries cover which pixel, 64 entries per word (see hit_mask_chunk); may be null
     const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
 };
@@ -154,7 +151,6 @@ __device__ __forceinline__ void topk_insert(const TopKOf<Pos> &tk, int cap, int 
 
 constexpr int kSelectBatch = 128;       // list entries staged per batch where positions take an int
 constexpr int kSelectBatchShort = 64;   // ... and where they take 16 bits
-constexpr int kShortList = 0xffff;      // longest tile list whose positions fit 16 bits
 constexpr int kLongListGroups = 256;    // workgroups that look for the tiles with longer lists
 
 // The per-pixel-order forward pass of one tile.  Pos: how a candidate's list position (from the tile's
@@ -177,6 +173,8 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_x, tile_y);
     publish_wave_rect(p, s_rects);
+    const int64_t order_step = order_stride(out.order, a);
+    const int64_t order_at = order_first(out.order, p, start, blockIdx.z * blockDim.x + threadIdx.x);
 
     PixelState s;
     real last_depth = -__builtin_inff();  // render.cu:585-586
@@ -290,12 +288,12 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                         real b0, b1, b2;
                         bary_apply(r[u].m, p.px, p.py, b0, b1, b2);
                         if (!bary_inside(b0, b1, b2)) continue;  // cannot happen: the selection tested it
-                        if (out.fragments) {
-                            const int64_t plane = (int64_t)a.W * a.H, at = (int64_t)s.blended * plane + p.index;
+                        if (out.order.low) {
+                            const int64_t at = order_at + (int64_t)s.blended * order_step;
                             const int rel = tk.j(i0 + u);
-                            out.fragments[at] = (uint16_t)rel;
+                            out.order.low[at] = (uint16_t)rel;
                             if (sizeof(Pos) > sizeof(uint16_t) && end - start > kShortList)
-                                out.fragments[(int64_t)a.max_layers * plane + at] = (uint16_t)(rel >> 16);
+                                out.order.low[out.order.high + at] = (uint16_t)(rel >> 16);
                         }
                         blend_fragment(s, r[u], b0, b1, b2);
                     }
@@ -421,11 +419,11 @@ extern "C" size_t tg_hit_mask_words(int64_t n_keys, int width, int height, int t
     return (size_t)(tiles * tl.grid.z + (n_keys / kWave + tiles + 1) * (int64_t)tl.grid.z * tl.threads);
 }
 
-extern "C" int tg_render_forward(const real *vertices, const int32_t *indices, const real *colors, const real *opacities,
+static int render_forward(const real *vertices, const int32_t *indices, const real *colors, const real *opacities,
                                  const int32_t *sorted_ids, const int32_t *offsets, const real *bary, int width, int height,
                                  int tile_w, int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers,
                                  real *image, real *depthmap, real *final_weights, int32_t *ends, int32_t *last,
-                                 real *last_depth, uint16_t *fragments, uint64_t *hit_masks, const real *batch_bounds,
+                                 real *last_depth, const OrderStore &order, uint64_t *hit_masks, const real *batch_bounds,
                                  const int32_t *far_start, const uint32_t *list_status, void *stream) {
     if (int e = check_raster_args("tg_render_forward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!vertices || !indices || !colors || !opacities || !offsets || !bary || !image || !depthmap || !final_weights || !ends) {
@@ -443,11 +441,7 @@ extern "C" int tg_render_forward(const real *vertices, const int32_t *indices, c
         set_error("tg_render_forward: batch_bounds come with far_start");
         return TG_E_ARG;
     }
-    if (fragments && (!per_pixel_sort || max_layers > TG_MAX_SAVED_LAYERS)) {
-        set_error("tg_render_forward: fragments are saved only with per_pixel_sort and max_layers <= %d", TG_MAX_SAVED_LAYERS);
-        return TG_E_ARG;
-    }
-    ForwardOut o{(real4 *)image, depthmap, final_weights, ends, last, last_depth, fragments, per_pixel_sort ? nullptr : hit_masks,
+    ForwardOut o{(real4 *)image, depthmap, final_weights, ends, last, last_depth, order, per_pixel_sort ? nullptr : hit_masks,
                  list_status};
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
     const dim3 grid = tl.grid;
@@ -479,4 +473,43 @@ extern "C" int tg_render_forward(const real *vertices, const int32_t *indices, c
     TG_LAUNCH(forward_pixel_order_long_lists_kernel, dim3(min(tiles, kLongListGroups), 1, grid.z), dim3(n_threads), lds, s, a, o,
               (int)grid.x, (int)grid.y);
     return check_launch("forward_pixel_order_long_lists_kernel");
+}
+
+extern "C" int tg_render_forward(const real *vertices, const int32_t *indices, const real *colors, const real *opacities,
+                                 const int32_t *sorted_ids, const int32_t *offsets, const real *bary, int width, int height,
+                                 int tile_w, int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers,
+                                 real *image, real *depthmap, real *final_weights, int32_t *ends, int32_t *last,
+                                 real *last_depth, uint16_t *fragments, uint64_t *hit_masks, const real *batch_bounds,
+                                 const int32_t *far_start, const uint32_t *list_status, void *stream) {
+    if (fragments && (!per_pixel_sort || max_layers > TG_MAX_SAVED_LAYERS)) {
+        set_error("tg_render_forward: fragments are saved only with per_pixel_sort and max_layers <= %d", TG_MAX_SAVED_LAYERS);
+        return TG_E_ARG;
+    }
+    const OrderStore order{fragments, (int64_t)max_layers * width * height, 0};
+    return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
+                          early_stopping_threshold, per_pixel_sort, max_layers, image, depthmap, final_weights, ends, last, last_depth,
+                          order, hit_masks, batch_bounds, far_start, list_status, stream);
+}
+
+extern "C" int64_t tg_order_pool_words(int64_t n_keys, int64_t n_triangles, int tile_w, int tile_h) {
+    if (n_keys < 0 || n_triangles < 0 || tile_w <= 0 || tile_h <= 0 || tile_w * tile_h > kMaxTilePixels) return 0;
+    // a triangle is in a tile's list once, so no list is longer than the number of triangles
+    return n_keys * order_pool_pixels(tile_w, tile_h) * (n_triangles > kShortList ? 2 : 1);
+}
+
+extern "C" int tg_render_forward_pooled(const real *vertices, const int32_t *indices, int32_t n_triangles, const real *colors,
+                                        const real *opacities, const int32_t *sorted_ids, const int32_t *offsets, int64_t n_keys,
+                                        const real *bary, int width, int height, int tile_w, int tile_h, real early_stopping_threshold,
+                                        int max_layers, real *image, real *depthmap, real *final_weights, int32_t *ends, int32_t *last,
+                                        real *last_depth, uint16_t *order_pool, const real *batch_bounds, const int32_t *far_start,
+                                        const uint32_t *list_status, void *stream) {
+    if (!order_pool || n_keys < 0 || n_triangles < 0) {
+        set_error("tg_render_forward_pooled: null order pool or negative count");
+        return TG_E_ARG;
+    }
+    const int pixels = order_pool_pixels(tile_w, tile_h);
+    const OrderStore order{order_pool, n_triangles > kShortList ? n_keys * pixels : 0, pixels};
+    return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
+                          early_stopping_threshold, 1, max_layers, image, depthmap, final_weights, ends, last, last_depth, order, nullptr,
+                          batch_bounds, far_start, list_status, stream);
 }

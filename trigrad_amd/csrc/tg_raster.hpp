@@ -18,6 +18,7 @@ constexpr int kBoundSpan = 256;     // list entries per depth bound (tg_list_bou
 constexpr int kLayers = 32;         // per-pixel selection batch (render.cu:570, :655)
 constexpr int kMaxTilePixels = 1024;  // tile_w * tile_h limit of the API (wrapper.py:143)
 constexpr int kTileThreads = 256;     // workgroup size limit
+constexpr int kShortList = 0xffff;    // longest tile list whose positions fit 16 bits
 constexpr int kGatherAhead = 4;       // records a lane of a per-pixel-order kernel fetches together
 
 struct RasterArgs {
@@ -176,6 +177,26 @@ __device__ __forceinline__ int64_t hit_mask_chunk(int start, int tile, int relat
 __device__ __forceinline__ int64_t hit_mask_head_index(int tile) { return (int64_t)tile * gridDim.z + blockIdx.z; }
 __device__ __forceinline__ int64_t hit_mask_head_words() { return (int64_t)gridDim.x * gridDim.y * gridDim.z; }
 
+// Where the saved blend order of a pixel lies: layer l of the pixel at low[l * stride], and, in tiles whose list holds more
+// than kShortList entries, the high half of its list position at high[l * stride].  Two layouts:
+//   planes  (max_layers <= TG_MAX_SAVED_LAYERS) one image plane per layer, the high halves in as many planes behind them
+//   pool    (any number of layers) a pixel blends an entry of its tile's list at most once, so a tile with a list of n
+//           entries is given n rows of one word per pixel: row `start + l` of the pool is layer l of the tile whose list
+//           starts at `start`, and n_keys rows hold every tile's.  Nothing has to be counted or allocated on the device, and
+//           what is never blended is never touched.
+struct OrderStore {
+    uint16_t *low;      // null: no order saved
+    int64_t high;       // words from a low half to its high half; 0: no list is that long
+    int pool_pixels;    // pool: words per row (pixels of a tile, whole waves); 0: planes
+};
+__device__ __forceinline__ int64_t order_stride(const OrderStore &o, const RasterArgs &a) {
+    return o.pool_pixels ? o.pool_pixels : (int64_t)a.W * a.H;
+}
+// t: the pixel's number inside its tile
+__device__ __forceinline__ int64_t order_first(const OrderStore &o, const PixelCoord &p, int list_start, int t) {
+    return o.pool_pixels ? (int64_t)list_start * o.pool_pixels + t : (p.valid ? p.index : 0);
+}
+
 // Batch bounds: word batch_bound_index(start, tile, p) holds, for the tile whose
 // list starts at `start`, a lower bound of the per-pixel depth of every entry at
 // relative position >= p (p a multiple of kBoundSpan) and < far_start[tile].  From
@@ -216,6 +237,7 @@ struct TileLaunch { dim3 grid; int threads; };
 TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_threads);
 int pixel_order_threads(int preferred);
 size_t pixel_order_lds_bytes(int n_threads, int staged_entries, size_t position_bytes = sizeof(int));
+inline int order_pool_pixels(int tile_w, int tile_h) { return ceil_div(tile_w * tile_h, kWave) * kWave; }
 int check_raster_args(const char *fn, int width, int height, int tile_w, int tile_h, int max_layers);
 
 // ---- per-wave culling ------------------------------------------------------------------

@@ -52,16 +52,19 @@ class Renderer(Function):
             ctx.skipped = False
             (image, depthmap, final_weights, sorted_ids, offsets, bary_transforms, ends, timings, resume) = _C._forward_full(
                 vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
-                not record_timing, per_pixel_sort, max_layers)
+                not record_timing, per_pixel_sort, max_layers, for_backward=any(ctx.needs_input_grad))
             last, last_depth, status_check, fragments, hit_masks = resume
             # private to this Function: where the reverse traversal starts, and the blend order (per-pixel
             # order, max_layers <= 32) or the hit masks (tile order); the list kernels' status word, which the
             # backward pass looks at before it trusts the lists
-            extras = [t for t in (last_depth, fragments, hit_masks) if t is not None]
+            extras = [t for t in (last_depth, fragments, hit_masks, resume.order_pool) if t is not None]
             ctx.has_last_depth = last_depth is not None
             ctx.has_fragments = fragments is not None
             ctx.has_hit_masks = hit_masks is not None
+            ctx.has_order_pool = resume.order_pool is not None
             ctx.status_check = status_check
+            if not any(ctx.needs_input_grad):
+                return (image, depthmap, timings) if record_timing else (image, depthmap)
             saved = [vertices, indices, colors, opacities, sorted_ids, offsets, bary_transforms, image, depthmap, final_weights,
                      ends, last]
             ctx.save_for_backward(*saved, *extras)
@@ -82,12 +85,14 @@ class Renderer(Function):
             last_depth = extras.pop(0) if ctx.has_last_depth else None
             fragments = extras.pop(0) if ctx.has_fragments else None
             hit_masks = extras.pop(0) if ctx.has_hit_masks else None
+            resume = _C.Resume((last, last_depth, ctx.status_check, fragments, hit_masks))
+            resume.order_pool = extras.pop(0) if ctx.has_order_pool else None
             width, height, tile_width, tile_height, threshold, per_pixel_sort, max_layers = ctx.render_args
             if grad_image is None:
                 grad_image = torch.zeros_like(saved[7])
             grad_vertices, grad_colors, grad_opacities = _C.render_backward(
                 grad_image, grad_depthmap, *saved[:11], width, height, tile_width, tile_height, threshold, per_pixel_sort,
-                max_layers, resume=(last, last_depth, ctx.status_check, fragments, hit_masks))
+                max_layers, resume=resume)
         # one slot per forward argument (wrapper.py:99-112)
         return (grad_vertices, None, grad_colors, grad_opacities, None, None, None, None, None, None, None, None)
 
