@@ -380,6 +380,26 @@ int tg_render_backward_pooled(const tg_real *grad_image, const tg_real *grad_dep
 int tg_split_gradient_block(const tg_real *block, int64_t n_vertices, tg_real *grad_vertices, tg_real *grad_colors,
                             tg_real *grad_opacities, void *stream);
 
+/* ---- in front of the renderer: near-plane splitting, division by w ------------- */
+
+/* Triangles of the clip coordinates clip (V,4) against the plane z + w >= 0 (the
+ * reference's notebook, notebooks/renderer.ipynb cell 15), in two calls with a host
+ * read of the number of output triangles between them.  tg_clip_count writes, per
+ * block of triangles (tg_clip_blocks of them), how many triangles leave it: to
+ * `totals` for the second call and to `host_totals`, memory the device can write and
+ * the host read (pinned), where bit 31 marks a block with an index outside
+ * [-V, V).  tg_clip_emit writes the n_out triangles (the sum of the totals) as a soup in
+ * input order: out_clip (3 n_out, 4), out_indices (n_out, 3) = 0, 1, 2, ..., out_colors
+ * (3 n_out, color_width) and out_opacities (3 n_out, opacity_width). */
+int64_t tg_clip_blocks(int64_t n_triangles);
+int tg_clip_count(const tg_real *clip, int32_t n_vertices, const int32_t *indices, int64_t n_triangles, uint32_t *totals,
+                  uint32_t *host_totals, void *stream);
+int tg_clip_emit(const tg_real *clip, int32_t n_vertices, const int32_t *indices, int64_t n_triangles, const tg_real *colors,
+                 int32_t color_width, const tg_real *opacities, int32_t opacity_width, const uint32_t *totals, int64_t n_out,
+                 tg_real *out_clip, int32_t *out_indices, tg_real *out_colors, tg_real *out_opacities, void *stream);
+/* (x, y, z, w) -> (x/w, y/w, z/w, 1/w) (viewer.py:276-278). */
+int tg_clip_to_render(const tg_real *clip, int64_t n_vertices, tg_real *out, void *stream);
+
 /* ---- host-side component hooks ---------------------------------------------- */
 
 /* HOST pointers, run on the CPU.  The reference exports the same six functions

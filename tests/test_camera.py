@@ -201,3 +201,34 @@ def test_projected_split_mesh_renders(cuda):
         if not crosses:
             img0, depth0 = trigrad_amd.render(camera.clip_to_render(clip).contiguous(), idx.to(cuda), col.to(cuda), op.to(cuda), W, H)
             assert torch.equal(img, img0) and torch.equal(depth, depth0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n_triangles", [1, 64, 1023, 1024, 1025, 70_001])
+@pytest.mark.parametrize("color_width,opacity_shape", [(3, ()), (5, (2, 1))])
+def test_splitting_kernels_give_the_tensor_operations_numbers(n_triangles, color_width, opacity_shape, dtype, cuda):
+    """Without gradients the splitting and the division run as kernels (tiles of 1024 triangles); with them as tensor
+    operations: one rounding per operation in the same order on both routes, so every bit agrees."""
+    cv, idx, col, op = _mesh(n_triangles, 500, n_triangles)
+    rng = np.random.default_rng(n_triangles)
+    clip = torch.from_numpy(cv).to(cuda, dtype)
+    indices = torch.from_numpy(idx).to(cuda)
+    colors = torch.from_numpy(rng.uniform(size=(500, color_width))).to(cuda, dtype)
+    opacities = torch.from_numpy(rng.uniform(size=(500,) + opacity_shape)).to(cuda, dtype)
+    got = camera.split_clipped(clip, indices, colors, opacities)
+    want = camera.split_clipped(clip.clone().requires_grad_(), indices, colors, opacities)
+    assert want[0].requires_grad and not got[0].requires_grad
+    for g, w in zip(got, want):
+        assert g.shape == w.shape and g.dtype == w.dtype and torch.equal(g, w)
+    assert torch.equal(camera.clip_to_render(got[0]), camera.clip_to_render(want[0]))
+
+
+@pytest.mark.gpu
+def test_splitting_kernels_reject_a_vertex_that_is_not_there(cuda):
+    clip = torch.zeros((4, 4), device=cuda)
+    args = torch.rand((4, 3), device=cuda), torch.rand((4,), device=cuda)
+    with pytest.raises(IndexError):
+        camera.split_clipped(clip, torch.tensor([[0, 1, 4]], dtype=torch.int32, device=cuda), *args)
+    assert camera.split_clipped(clip, torch.tensor([[0, 1, -1]], dtype=torch.int32, device=cuda), *args)[0].shape == (3, 4)
+    assert camera.split_clipped(clip, torch.zeros((0, 3), dtype=torch.int32, device=cuda), *args)[0].shape == (0, 4)

@@ -63,6 +63,10 @@ SIGNATURES = {
     "tg_render_backward": (_i, [_p] * 17 + [_i, _i, _i, _i, _f, _i, _i, _p, _p, _p, _i, _i, _i, _p]),
     "tg_render_backward_pooled": (_i, [_p] * 4 + [_i32] + [_p] * 4 + [_i64] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p, _p, _p, _i, _i, _i, _p]),
     "tg_split_gradient_block": (_i, [_p, _i64, _p, _p, _p, _p]),
+    "tg_clip_blocks": (_i64, [_i64]),
+    "tg_clip_count": (_i, [_p, _i32, _p, _i64, _p, _p, _p]),
+    "tg_clip_emit": (_i, [_p, _i32, _p, _i64, _p, _i32, _p, _i32, _p, _i64, _p, _p, _p, _p, _p]),
+    "tg_clip_to_render": (_i, [_p, _i64, _p, _p]),
     "tg_barycentric": (None, [_p] * 5),
     "tg_barycentric_backward": (None, [_p] * 6),
     "tg_interpolate3_scalar": (_f, [_p, _f, _f, _f, _p]),

@@ -8,11 +8,25 @@ and, for triangles that cross the near plane, in its notebook
 operations as differentiable torch functions that run on whatever device the
 tensors live on; `split_clipped` is vectorised over triangles instead of the
 notebook's Python loop and returns the triangles in the same order with the
-same vertex order.
+same vertex order.  On the GPU, where no gradient is asked for, the splitting and
+the division by w run as kernels of the library (csrc/tg_camera.hip): the same
+numbers bit for bit, without the hundreds of launches.
 """
 import math
 
 import torch
+
+from . import _C, _lib
+
+
+def _native(*tensors):
+    """Whether the library's kernels take these: on one GPU, of one of its scalar types, no gradient wanted."""
+    first = tensors[0]
+    if first.device.type != "cuda" or first.dtype not in (torch.float32, torch.float64):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return all(t.device == first.device and t.dtype == first.dtype for t in tensors)
 
 
 def perspective(fov_degrees, width, height, near=0.1, far=100.0, dtype=torch.float32, device=None):
@@ -35,6 +49,14 @@ def to_clip(positions, matrix):
 
 def clip_to_render(clip_vertices):
     """(V,4) clip coordinates -> (V,4) render input (x/w, y/w, z/w, 1/w) (viewer.py:276-278)."""
+    if _native(clip_vertices) and clip_vertices.dim() == 2 and clip_vertices.shape[1] == 4:
+        clip = clip_vertices.contiguous()
+        out = torch.empty_like(clip)
+        bits = _C._bits(clip)
+        with _C._on_device(clip.device):
+            _lib.check(_lib.load(bits).tg_clip_to_render(clip.data_ptr(), clip.shape[0], out.data_ptr(), _C._raw_stream(clip.device)),
+                       "tg_clip_to_render", bits)
+        return out
     w = clip_vertices[:, 3:4]
     return torch.cat([clip_vertices[:, :3] / w, 1.0 / w], dim=-1)
 
@@ -42,6 +64,36 @@ def clip_to_render(clip_vertices):
 def project(positions, matrix):
     """Positions through a projection-view matrix to `render`'s vertex layout (viewer.py:271-279)."""
     return clip_to_render(to_clip(positions, matrix))
+
+
+def _split_clipped_native(clip, indices, colors, opacities):
+    """split_clipped by the library's kernels: count, read the number of output triangles, write them."""
+    dev, dtype, bits = clip.device, clip.dtype, _C._bits(clip)
+    lib = _lib.load(bits)
+    clip, indices, colors, opacities = (t.contiguous() for t in (clip, indices, colors, opacities))
+    V, M = clip.shape[0], indices.shape[0]
+    n_out = 0
+    with _C._on_device(dev):
+        stream = _C._raw_stream(dev)
+        if M > 0:
+            totals = torch.empty((int(lib.tg_clip_blocks(M)),), dtype=torch.int32, device=dev)
+            host = torch.empty_like(totals, device="cpu", pin_memory=True)
+            _lib.check(lib.tg_clip_count(clip.data_ptr(), V, indices.data_ptr(), M, totals.data_ptr(), host.data_ptr(), stream),
+                       "tg_clip_count", bits)
+            torch.cuda.current_stream(dev).synchronize()
+            if int(host.min()) < 0:
+                raise IndexError(f"split_clipped: a triangle names a vertex outside the {V} vertices")
+            n_out = int(host.sum())
+        vertices = torch.empty((3 * n_out, 4), dtype=dtype, device=dev)
+        new_indices = torch.empty((n_out, 3), dtype=torch.int32, device=dev)
+        new_colors = torch.empty((3 * n_out,) + tuple(colors.shape[1:]), dtype=dtype, device=dev)
+        new_opacities = torch.empty((3 * n_out,) + tuple(opacities.shape[1:]), dtype=dtype, device=dev)
+        if n_out > 0:
+            _lib.check(lib.tg_clip_emit(clip.data_ptr(), V, indices.data_ptr(), M, colors.data_ptr(), math.prod(colors.shape[1:]),
+                                        opacities.data_ptr(), math.prod(opacities.shape[1:]), totals.data_ptr(), n_out,
+                                        vertices.data_ptr(), new_indices.data_ptr(), new_colors.data_ptr(), new_opacities.data_ptr(),
+                                        stream), "tg_clip_emit", bits)
+    return vertices, new_indices, new_colors, new_opacities
 
 
 def split_clipped(clip_vertices, indices, vertex_colors, vertex_opacities):
@@ -58,6 +110,10 @@ def split_clipped(clip_vertices, indices, vertex_colors, vertex_opacities):
     Returns (vertices (3N,4), indices (N,3) int32 = arange, colors (3N,C),
     opacities (3N,...)) as a triangle soup in input order.
     """
+    if (_native(clip_vertices, vertex_colors, vertex_opacities) and indices.dtype == torch.int32 and indices.device == clip_vertices.device
+            and indices.dim() == 2 and indices.shape[1] == 3 and clip_vertices.dim() == 2 and clip_vertices.shape[1] == 4
+            and vertex_colors.shape[:1] == vertex_opacities.shape[:1] == clip_vertices.shape[:1]):
+        return _split_clipped_native(clip_vertices, indices, vertex_colors, vertex_opacities)
     idx = indices.long()
     dev = clip_vertices.device
     d_all = clip_vertices[:, 2] + clip_vertices[:, 3]
