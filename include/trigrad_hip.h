@@ -9,7 +9,8 @@
  *     tg_scan_exclusive_u32_noalloc, works in a device array of its own
  *     instead of a workspace);
  *   - `stream` is a hipStream_t passed as void* (NULL = the null stream); all
- *     work is enqueued on it and no entry point synchronises;
+ *     work is enqueued on it and no entry point synchronises (tg_frame_forward
+ *     with TG_FRAME_WAIT and tg_frame_wait wait for a word in host memory);
  *   - the return value is 0 on success, a negative TG_E_* code for rejected
  *     arguments, or a positive hipError_t; tg_last_error() describes the last
  *     failure on the calling thread;
@@ -379,6 +380,80 @@ int tg_render_backward_pooled(const tg_real *grad_image, const tg_real *grad_dep
  * (V)): scalars 0..3 of a vertex's row, 4..6 and 7.  One pass over the block. */
 int tg_split_gradient_block(const tg_real *block, int64_t n_vertices, tg_real *grad_vertices, tg_real *grad_colors,
                             tg_real *grad_opacities, void *stream);
+
+/* ---- a whole frame ------------------------------------------------------------- */
+
+/* The forward pass of a frame (binning, lists, bary matrices, blending) in one call, and its backward pass in another
+ * (float build, at most 256 tile columns and rows: tg_frame_supported).  The key buffers are made for `key_capacity` keys;
+ * the kernels read the number of keys on the device.  If the frame has more, its lists are empty and n_keys tells
+ * how many it has: the caller comes again with larger buffers.  Every field is eight bytes wide.
+ *
+ * kept, scratch: device memory, 256-byte aligned, of the sizes and with the contents that tg_frame_layout reports
+ * (bytes of kept, of scratch and of the frame state; then the places inside kept of: the status word of the list
+ * kernels, sorted ids, tile offsets, bary matrices, final weights, ends, last, last_depth, the saved blend order, the hit
+ * masks).  scratch is free again when the forward kernels are done, kept is what the backward pass reads.
+ * frame, frame_bytes, epoch: as in tg_bin_frame; the 8 bytes behind frame_bytes take K and the scan's status.
+ * host: four words of memory that the device writes and the host reads (pinned): [0] K, [1] TG_FRAME_COUNTED or
+ * TG_FRAME_EXPIRED once K is there, [2] the list kernels' status once it is known (TG_FRAME_PENDING before).
+ * phases: which parts of the forward pass to launch; TG_FRAME_WAIT then waits for K (the one wait of the call) and
+ * sets n_keys and counted.
+ * gradients: (V,4), (V,3) and (V,) behind each other; block: (V,8) of scratch with per_pixel_sort. */
+typedef struct tg_frame {
+    const tg_real *vertices;
+    const int32_t *indices;
+    const tg_real *colors;
+    const tg_real *opacities;
+    tg_real *image;
+    tg_real *depthmap;
+    void *kept;
+    void *scratch;
+    void *frame;
+    uint32_t *host;
+    void *stream;
+    int64_t epoch;
+    int64_t frame_bytes;
+    int64_t phases;
+    const tg_real *grad_image;
+    const tg_real *grad_depthmap;
+    tg_real *gradients;
+    tg_real *block;
+    int64_t n_keys;  /* out */
+    int64_t counted; /* out */
+    int64_t n_vertices;
+    int64_t n_triangles;
+    int64_t width;
+    int64_t height;
+    int64_t tile_w;
+    int64_t tile_h;
+    int64_t per_pixel_sort;
+    int64_t max_layers;
+    int64_t key_capacity;
+    int64_t flags;
+    int64_t kept_bytes;
+    int64_t scratch_bytes;
+    double early_stopping_threshold;
+} tg_frame;
+
+#define TG_FRAME_BACKWARD 1     /* flags: a backward pass will follow: save what it needs */
+#define TG_FRAME_ORDER_PLANES 2 /*   ... the blend order in planes (per_pixel_sort, max_layers <= TG_MAX_SAVED_LAYERS) */
+#define TG_FRAME_ORDER_POOL 4   /*   ... the blend order in a pool (tg_order_pool_words) */
+#define TG_FRAME_HIT_MASKS 8    /*   ... the hit masks (tile order) */
+#define TG_FRAME_LIST_BOUNDS 16 /*   depth bounds of the lists (tg_list_bounds) for the per-pixel selection */
+#define TG_FRAME_BIN 1          /* phases */
+#define TG_FRAME_LISTS 2
+#define TG_FRAME_RASTER 4
+#define TG_FRAME_WAIT 8
+#define TG_FRAME_COUNTED 1u     /* host[1] */
+#define TG_FRAME_EXPIRED 2u
+#define TG_FRAME_PENDING 0xffffffffu
+#define TG_FRAME_LAYOUT_WORDS 13
+
+int tg_frame_supported(int width, int height, int tile_w, int tile_h);
+int tg_frame_layout(const tg_frame *f, int64_t *out);
+int tg_frame_forward(tg_frame *f);
+int tg_frame_backward(const tg_frame *f);
+/* Waits (on the host) until host[word] differs from `pending`. */
+int tg_frame_wait(const uint32_t *host, int word, uint32_t pending, void *stream);
 
 /* ---- in front of the renderer: near-plane splitting, division by w ------------- */
 

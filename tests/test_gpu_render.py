@@ -607,3 +607,44 @@ def test_scene_without_a_single_key(mode, cuda):
     (image.sum() + torch.where(torch.isinf(depthmap), torch.zeros_like(depthmap), depthmap).sum()).backward()
     for g in (v.grad, c.grad, o.grad):
         assert float(g.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
+@pytest.mark.parametrize("n_triangles,size,tile", [(1, 16, 16), (2048, 16, 16), (2049, 16, 16), (4097, 40, 16), (900, 256, 1), (900, 257, 1)])
+def test_frame_in_one_call_is_the_frame_stage_by_stage(n_triangles, size, tile, mode, cuda, monkeypatch):
+    """The one-call route against the stages with K on the host, at the edges of its rules: one triangle, one list of 2048 and
+    2049 entries (what the small segment sort takes), more than one sort tile, 256 and 257 tile columns (the staged route's).
+    The second run has key buffers that are far too small: empty lists first, then the frame again."""
+    import torch
+    import trigrad_amd
+    from trigrad_amd import _C
+    import scenes as S
+    scene = S.random_soup(n_triangles, size, size, seed=n_triangles, sigma_px=6.0, varying_w=True)
+    d = to_device(scene, cuda)
+    m = MODES[mode]
+    key = (cuda.index, n_triangles, size, size, tile, tile)
+    gi = torch.from_numpy(np.random.default_rng(1).standard_normal((size, size, 4)).astype(np.float32)).to(cuda)
+
+    def run():
+        leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+        image, depth = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], size, size, tile, tile, 1 / 256, False,
+                                          m["per_pixel_sort"], m["max_layers"])
+        return [image.detach(), depth.detach(), *torch.autograd.grad((image,), leaves, (gi,))]
+
+    _C._frame_key_hints.pop(key, None)
+    got = [run()]
+    supported = _C.frame_supported(d["vertices"], size, size, tile, tile)
+    assert supported == (size // tile <= 256) and (key in _C._frame_key_hints) == supported
+    if supported:
+        K = _C._frame_key_hints[key]
+        _C._frame_key_hints[key] = 0
+        monkeypatch.setattr(_C, "_round_capacity", lambda n: max(n, 1))
+        got.append(run())
+        assert _C._frame_key_hints[key] == K
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = run()
+    for one in got:
+        assert torch.equal(one[0], want[0]) and torch.equal(one[1], want[1])
+        for a, b in zip(one[2:], want[2:]):
+            # sums of float32 terms in another order: two rounding steps of the largest sum
+            assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()) + 1e-6

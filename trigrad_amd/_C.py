@@ -3,19 +3,21 @@ pybind module (src/trigrad/module.cu:8-21, render.h) with the same names and
 argument order, implemented by calling the C ABI of libtrigrad_hip.so on the
 current torch stream.  torch is used for device memory and streams only.
 
-`render_forward` runs the frame's route:
+A frame is one call forward (`frame_forward`: binning, lists and blending, launched for the capacity of the key buffers
+while the kernels read K on the device) and one call backward (`frame_backward`).  Frames with more than 256 tile columns or
+rows run stage by stage:
     bin_frame (count + scan, then key emission that reads K on the device) -> (K to the host, bary matrices meanwhile)
-    -> build_frame_lists (two passes over the tile bits through memory, depth bits and tile ranges per tile)
+    -> build_frame_lists (passes over the tile bits through memory, depth bits and tile ranges per tile)
     -> forward kernel
 The double build and frames with more than 2^21 tiles go through bin_setup + build_tile_lists, and the single stages
 (bin_count, scan_exclusive, bin_emit, sort_pairs, tile_ranges) are exposed as functions for tests and benchmarks.
 """
 import ctypes as C
+import os
+import struct
 import threading
 
 import torch
-
-import os
 
 from . import _lib
 
@@ -105,6 +107,9 @@ SAVE_HIT_MASKS = True
 # With per_pixel_sort and tile lists of at least this many entries on average, depth bounds of the lists are
 # computed (one more pass over the keys) so that the selection can stop before the end of a list.
 EARLY_STOP_MIN_AVG_LIST = 512
+# A frame's forward and backward pass in one call each where the library takes the frame (tg_frame_supported); False: the
+# stages one by one.
+ONE_CALL_FRAME = True
 # Binning (count, scan, key emission) in one launch where the library takes the frame (tg_bin_frame_supported);
 # False: tg_bin_setup + tg_build_tile_lists, the route of the double build and of frames with more than 2^21 tiles.
 FUSED_BINNING = True
@@ -549,6 +554,29 @@ class StatusCheck:
                                "invalid and its image is NaN.  Later frames number their tiles by ticket.")
 
 
+class FrameStatus(StatusCheck):
+    """The status word of a frame's list kernels where the frame's first blending workgroup leaves it: in pinned host memory
+    (words: K, whether it is there, the status), so there is no copy and no event to wait for."""
+
+    def __init__(self, stream, frame=None):
+        self.what = "tg_frame_forward"
+        self.frame = frame
+        self.checked = False
+        self.host = torch.empty((4,), dtype=torch.int32, pin_memory=True)
+        self.address = self.host.data_ptr()
+        self.word = C.c_uint32.from_address(self.address + 8)
+        self.stream = stream
+
+    def ready(self):
+        return self.word.value != _FRAME_PENDING
+
+    def failed(self):
+        if self.word.value == _FRAME_PENDING:
+            _lib.check(_lib.load(32).tg_frame_wait(self.address, 2, _FRAME_PENDING, self.stream), "tg_frame_wait")
+        self.checked = True
+        return self.word.value != 0
+
+
 _pending_checks = []  # status words of earlier frames that nobody has looked at yet
 _pending_lock = threading.Lock()
 
@@ -579,13 +607,15 @@ def verify_frames(wait=True):
 
 def verify_finished_frames():
     """verify_frames(wait=False): never waits."""
-    verify_frames(wait=False)
+    if _pending_checks:
+        verify_frames(wait=False)
 
 
 class Resume(tuple):
     """(last, last_depth, status_check, fragments, hit_masks), and as an attribute the pool with the blend order of a
     pass with more than MAX_SAVED_LAYERS layers (None: no such order was saved)."""
     order_pool = None
+    pool_keys = None  # list entries the pool was made for (None: as many as there are)
 
 
 def _order_pool(n_keys, n_triangles, tile_width, tile_height, device):
@@ -596,6 +626,230 @@ def _order_pool(n_keys, n_triangles, tile_width, tile_height, device):
         return None
     step = 1 << max(words.bit_length() - 4, 10)
     return torch.empty((-(-words // step) * step,), dtype=torch.int16, device=device)
+
+
+# ---- a frame in one call ----------------------------------------------------------------------------------
+
+_FRAME_PENDING = 0xFFFFFFFF
+_FRAME_BACKWARD, _FRAME_ORDER_PLANES, _FRAME_ORDER_POOL, _FRAME_HIT_MASKS, _FRAME_LIST_BOUNDS = 1, 2, 4, 8, 16
+_FRAME_BIN, _FRAME_LISTS, _FRAME_RASTER, _FRAME_WAIT = 1, 2, 4, 8
+# struct tg_frame of the C header: what changes from call to call in front, then the results, then the frame's kind
+_FRAME_CALL = struct.Struct("<11Q3q4Q")
+_FRAME_RESULT = struct.Struct("<2q")
+_FRAME_KIND = struct.Struct("<12qd")
+_FRAME_BYTES = _FRAME_CALL.size + _FRAME_RESULT.size + _FRAME_KIND.size
+
+_frame_plans = {}  # frame kind -> _FramePlan
+_frame_key_hints = {}  # (device index, triangles, image and tile size) -> K of the last such frame
+_MAX_REMEMBERED = 256  # entries either of them holds before it starts anew
+
+
+class _FramePlan:
+    """What frames of one kind (sizes, options, key capacity) have in common: the constant part of the call, the sizes of
+    its buffers and where things lie in the kept one."""
+    __slots__ = ("kind", "capacity", "flags", "per_pixel_sort", "kept_bytes", "scratch_bytes", "frame_bytes", "at")
+
+    def __init__(self, n_vertices, n_triangles, width, height, tile_width, tile_height, per_pixel_sort, max_layers, capacity, flags,
+                 threshold):
+        lib = _lib.load(32)
+        self.capacity = capacity
+
+        def pack(kept, scratch):
+            return _FRAME_KIND.pack(n_vertices, n_triangles, width, height, tile_width, tile_height, per_pixel_sort, max_layers,
+                                    capacity, self.flags, kept, scratch, threshold)
+
+        if flags & _FRAME_ORDER_POOL:
+            words = int(lib.tg_order_pool_words(capacity, n_triangles, tile_width, tile_height))
+            if words == 0 or words * 2 > ORDER_POOL_MAX_BYTES:
+                flags &= ~_FRAME_ORDER_POOL
+        self.flags, self.per_pixel_sort = flags, bool(per_pixel_sort)
+        layout = (C.c_int64 * 13)()
+        call = bytes(_FRAME_CALL.size + _FRAME_RESULT.size) + pack(0, 0)
+        _lib.check(lib.tg_frame_layout(call, layout), "tg_frame_layout")
+        self.kept_bytes, self.scratch_bytes, self.frame_bytes = layout[0], layout[1], layout[2]
+        self.at = dict(zip(("status", "ids", "offsets", "bary", "weights", "ends", "last", "last_depth", "order", "masks"), layout[3:]))
+        self.kind = pack(self.kept_bytes, self.scratch_bytes)
+
+
+def _remember(table, key, value):
+    if len(table) >= _MAX_REMEMBERED and key not in table:
+        table.clear()
+    table[key] = value
+
+
+def _round_capacity(n):
+    """n keys, an eighth more and up to a multiple of a sixteenth of a power of two: a scene whose K drifts from frame to frame
+    keeps its buffers' sizes."""
+    n += n // 8 + 1024
+    step = 1 << max(n.bit_length() - 5, 10)
+    return min(-(-n // step) * step, (1 << 30) - 1)
+
+
+class Frame:
+    """A frame rendered by frame_forward: its plan, the status of its lists and (K) the keys it has."""
+    __slots__ = ("plan", "status", "n_keys")
+
+
+def frame_supported(vertices, width, height, tile_width, tile_height):
+    """Whether frame_forward takes this frame (float build, at most 256 tile columns and rows)."""
+    return (ONE_CALL_FRAME and FUSED_BINNING and vertices.dtype == torch.float32
+            and bool(_lib.load(32).tg_frame_supported(width, height, tile_width, tile_height)))
+
+
+def frame_forward(vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
+                  per_pixel_sort, max_layers, for_backward=True, timer=None):
+    """-> (image, depthmap, kept, frame): `kept` is the block that holds what the backward pass reads.
+
+    The call launches everything and waits for K only then; a frame with more keys than its buffers were made for (K of the
+    last frame of its kind and an eighth more, or three per triangle) is rendered again into larger ones."""
+    global _frame_counter
+    lib = _lib.load(32)
+    dev = vertices.device
+    with _on_device(dev):
+        if timer is not None:
+            timer.start("init")
+        vertices, indices, colors, opacities = vertices.contiguous(), indices.contiguous(), colors.contiguous(), opacities.contiguous()
+        n_triangles, n_vertices = indices.shape[0], vertices.shape[0]
+        flags = 0
+        if for_backward:
+            flags = _FRAME_BACKWARD
+            if not per_pixel_sort:
+                flags |= _FRAME_HIT_MASKS if SAVE_HIT_MASKS else 0
+            elif SAVE_BLEND_ORDER:
+                flags |= _FRAME_ORDER_PLANES if max_layers <= MAX_SAVED_LAYERS else _FRAME_ORDER_POOL
+        hint_key = (dev.index, n_triangles, width, height, tile_width, tile_height)
+        expected = _frame_key_hints.get(hint_key)
+        if expected is None:
+            expected, capacity = 2 * n_triangles, min(3 * n_triangles + 65536, (1 << 30) - 1)
+        else:
+            capacity = _round_capacity(expected)
+        # long lists: depth bounds let the selection leave a list before its end
+        if per_pixel_sort and expected >= EARLY_STOP_MIN_AVG_LIST * (-(-width // tile_width) * -(-height // tile_height)):
+            flags |= _FRAME_LIST_BOUNDS
+        image = torch.empty((height, width, 4), dtype=torch.float32, device=dev)
+        depthmap = torch.empty((height, width), dtype=torch.float32, device=dev)
+        stream = _raw_stream(dev)
+        frame = Frame()
+        while True:
+            kind = (n_vertices, n_triangles, width, height, tile_width, tile_height, 1 if per_pixel_sort else 0, max_layers, capacity,
+                    flags, float(early_stopping_threshold))
+            plan = _frame_plans.get(kind)
+            if plan is None:
+                plan = _FramePlan(*kind)
+                _remember(_frame_plans, kind, plan)
+            kept = torch.empty((plan.kept_bytes,), dtype=torch.uint8, device=dev)
+            scratch = torch.empty((plan.scratch_bytes,), dtype=torch.uint8, device=dev)
+            _frame_counter += 1
+            status = FrameStatus(stream, _frame_counter)
+            call = bytearray(_FRAME_BYTES)
+            call[-_FRAME_KIND.size:] = plan.kind
+            c_call = (C.c_char * _FRAME_BYTES).from_buffer(call)
+            with _frame_launches(dev.index, stream):  # one frame at a time on a stream's state
+                state, state_bytes, epoch = _next_frame_state(dev, plan.frame_bytes)
+                for phases, stage in _FRAME_UNTIMED if timer is None else _FRAME_TIMED:
+                    if timer is not None:
+                        timer.start(stage)
+                    _FRAME_CALL.pack_into(call, 0, vertices.data_ptr(), indices.data_ptr(), colors.data_ptr(), opacities.data_ptr(),
+                                          image.data_ptr(), depthmap.data_ptr(), kept.data_ptr(), scratch.data_ptr(),
+                                          state.data_ptr(), status.address, stream, epoch, state_bytes, phases, 0, 0, 0, 0)
+                    code = lib.tg_frame_forward(c_call)
+                    if code:
+                        _lib.check(code, "tg_frame_forward")
+            n_keys, counted = _FRAME_RESULT.unpack_from(call, _FRAME_CALL.size)
+            if counted == 1 and n_keys <= capacity:
+                break
+            torch.cuda.current_stream(dev).synchronize()  # the kernels are done with the status words
+            if counted != 1:
+                # a workgroup gave up waiting for another (other work on the device): once more, with tickets
+                if _tickets_forced:
+                    raise RuntimeError("tg_frame_forward: wait for another workgroup timed out")
+                force_tickets(True)
+            else:
+                if n_keys >= 1 << 30:
+                    raise RuntimeError(f"tg_frame_forward: {n_keys} (tile, triangle) pairs, the sort takes 2^30 - 1")
+                capacity = _round_capacity(n_keys)
+        if hint_key in _frame_key_hints:
+            _frame_key_hints[hint_key] = n_keys
+        else:
+            _remember(_frame_key_hints, hint_key, n_keys)
+        _key_count_hint[dev.index] = n_keys
+        with _pending_lock:
+            _pending_checks.append(status)
+    frame.plan, frame.status, frame.n_keys = plan, status, n_keys
+    return image, depthmap, kept, frame
+
+
+_FRAME_UNTIMED = ((_FRAME_BIN | _FRAME_LISTS | _FRAME_RASTER | _FRAME_WAIT, None),)
+# the bary matrices are made where the triangles are read anyway, by the binning
+_FRAME_TIMED = ((_FRAME_BIN, "per_tile_lists"), (_FRAME_LISTS, "sorting"), (0, "bary_transforms"), (_FRAME_RASTER | _FRAME_WAIT, "rasterization"))
+
+_launch_locks = {}  # (device index, stream) -> lock
+
+
+def _frame_launches(index, stream):
+    lock = _launch_locks.get((index, stream))
+    if lock is None:
+        with _frame_lock:
+            lock = _launch_locks.setdefault((index, stream), threading.Lock())
+    return lock
+
+
+def frame_backward(frame, grad_image, grad_depthmap, vertices, indices, colors, opacities, image, depthmap, kept):
+    """frame_forward's results and inputs -> (grad_vertices, grad_colors, grad_opacities); grad_depthmap may be None.  The status
+    of the frame's lists is looked at when everything is launched (the kernels look at it too): RuntimeError if invalid."""
+    lib = _lib.load(32)
+    dev = vertices.device
+    plan = frame.plan
+    n_vertices = vertices.shape[0]
+    with _on_device(dev):
+        vertices, indices, colors, opacities = vertices.contiguous(), indices.contiguous(), colors.contiguous(), opacities.contiguous()
+        grad_image = grad_image.contiguous()
+        if grad_depthmap is not None:
+            grad_depthmap = grad_depthmap.contiguous()
+        gradients = torch.empty((8 * n_vertices,), dtype=torch.float32, device=dev)
+        block = torch.empty_like(gradients) if plan.per_pixel_sort else None
+        call = bytearray(_FRAME_BYTES)
+        call[-_FRAME_KIND.size:] = plan.kind
+        _FRAME_CALL.pack_into(call, 0, vertices.data_ptr(), indices.data_ptr(), colors.data_ptr(), opacities.data_ptr(), image.data_ptr(),
+                              depthmap.data_ptr(), kept.data_ptr(), 0, 0, 0, _raw_stream(dev), 0, 0, 0, grad_image.data_ptr(),
+                              0 if grad_depthmap is None else grad_depthmap.data_ptr(), gradients.data_ptr(),
+                              0 if block is None else block.data_ptr())
+        code = lib.tg_frame_backward((C.c_char * _FRAME_BYTES).from_buffer(call))
+        if code:
+            _lib.check(code, "tg_frame_backward")
+        frame.status.verify()
+        # (V,4) | (V,3) | (V,) behind each other
+        grad_vertices, grad_colors, grad_opacities = gradients.split_with_sizes((4 * n_vertices, 3 * n_vertices, n_vertices))
+    return grad_vertices.view(n_vertices, 4), grad_colors.view(n_vertices, 3), grad_opacities
+
+
+def _frame_results(image, depthmap, kept, frame, width, height, tile_width, tile_height, per_pixel_sort, max_layers, n_triangles):
+    """The results of _forward_full (without timings) as views into frame_forward's kept block."""
+    plan, K = frame.plan, frame.n_keys
+    pixels = width * height
+
+    def view(name, n, dtype, *shape):
+        size = torch.empty((), dtype=dtype).element_size()
+        return kept[plan.at[name]:plan.at[name] + n * size].view(dtype).view(*shape)
+
+    flags = plan.flags
+    T = num_tiles(width, height, tile_width, tile_height)
+    last = view("last", pixels, torch.int32, height, width) if flags & _FRAME_BACKWARD else None
+    last_depth = view("last_depth", pixels, torch.float32, height, width) if flags & _FRAME_BACKWARD and per_pixel_sort else None
+    fragments = view("order", 2 * max_layers * pixels, torch.int16, 2 * max_layers, height, width) if flags & _FRAME_ORDER_PLANES else None
+    masks = order_pool = None
+    lib = _lib.load(32)
+    if flags & _FRAME_HIT_MASKS:
+        words = int(lib.tg_hit_mask_words(plan.capacity, width, height, tile_width, tile_height))
+        masks = view("masks", words, torch.int64, words)
+    if flags & _FRAME_ORDER_POOL:
+        words = int(lib.tg_order_pool_words(plan.capacity, n_triangles, tile_width, tile_height))
+        order_pool = view("order", words, torch.int16, words)
+    resume = Resume((last, last_depth, frame.status, fragments, masks))
+    resume.order_pool, resume.pool_keys = order_pool, plan.capacity
+    return (image, depthmap, view("weights", pixels, torch.float32, height, width), view("ids", K, torch.int32, K),
+            view("offsets", T + 1, torch.int32, T + 1), view("bary", 9 * n_triangles, torch.float32, n_triangles, 3, 3),
+            view("ends", pixels, torch.int32, height, width), resume)
 
 
 def _forward_full(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
@@ -611,6 +865,22 @@ def _forward_full(vertices, indices, colors, opacities, width, height, tile_widt
     real = vertices.dtype
     timer = _StageTimer(disable_timing)
     dev = vertices.device
+    if frame_supported(vertices, width, height, tile_width, tile_height):
+        image, depthmap, kept, frame = frame_forward(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
+                                                     early_stopping_threshold, per_pixel_sort, int(max_layers), for_backward,
+                                                     None if disable_timing else timer)
+        timings = timer.stop()
+        if not disable_timing:  # the timer has waited for the stream anyway
+            if frame.status.failed() and not _tickets_forced:
+                # the lists are invalid (and the image NaN): the whole frame once more, its tiles numbered by ticket
+                force_tickets(True)
+                return _forward_full(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
+                                     early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward)
+            frame.status.checked = False
+            frame.status.verify()
+        *results, resume = _frame_results(image, depthmap, kept, frame, width, height, tile_width, tile_height, per_pixel_sort,
+                                          int(max_layers), indices.shape[0])
+        return (*results, timings, resume)
     with _on_device(dev):
         timer.start("init")
         vertices = vertices.contiguous()
@@ -811,7 +1081,7 @@ def render_backward(grad_output, grad_depthmap, vertices, indices, colors, opaci
         if order_pool is not None:
             p = [_ptr(t) for t in tensors]
             _lib.check(lib.tg_render_backward_pooled(
-                *p[:4], indices.shape[0], *p[4:8], sorted_ids.numel(), *p[8:], _ptr(order_pool), width, height, tile_width, tile_height,
+                *p[:4], indices.shape[0], *p[4:8], resume.pool_keys or sorted_ids.numel(), *p[8:], _ptr(order_pool), width, height, tile_width, tile_height,
                 float(early_stopping_threshold), int(max_layers), _ptr(grad_vertices), _ptr(grad_colors), _ptr(grad_opacities), *strides,
                 _stream(vertices)), "tg_render_backward_pooled", bits)
         else:

@@ -63,6 +63,11 @@ SIGNATURES = {
     "tg_render_backward": (_i, [_p] * 17 + [_i, _i, _i, _i, _f, _i, _i, _p, _p, _p, _i, _i, _i, _p]),
     "tg_render_backward_pooled": (_i, [_p] * 4 + [_i32] + [_p] * 4 + [_i64] + [_p] * 7 + [_i, _i, _i, _i, _f, _i, _p, _p, _p, _i, _i, _i, _p]),
     "tg_split_gradient_block": (_i, [_p, _i64, _p, _p, _p, _p]),
+    "tg_frame_supported": (_i, [_i, _i, _i, _i]),
+    "tg_frame_layout": (_i, [_p, _p]),
+    "tg_frame_forward": (_i, [_p]),
+    "tg_frame_backward": (_i, [_p]),
+    "tg_frame_wait": (_i, [_p, _i, C.c_uint32, _p]),
     "tg_clip_blocks": (_i64, [_i64]),
     "tg_clip_count": (_i, [_p, _i32, _p, _i64, _p, _p, _p]),
     "tg_clip_emit": (_i, [_p, _i32, _p, _i64, _p, _i32, _p, _i32, _p, _i64, _p, _p, _p, _p, _p]),

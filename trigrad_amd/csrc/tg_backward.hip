@@ -18,6 +18,7 @@
 // per_pixel_sort = 1, max_layers > 32 (backward_pixel_order_kernel): the pixel
 //   re-selects its fragments from the far end (32 at a time, below the (depth,
 //   position) of the last blended fragment saved by the forward pass).
+#include "tg_frame.hpp"
 #include "tg_raster.hpp"
 
 namespace tg {
@@ -37,7 +38,11 @@ struct BackwardArgs {
     real *grad_colors;
     real *grad_opacities;
     int vertex_stride, color_stride, opacity_stride;  // scalars from one vertex to the next in the three arrays
+    const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
 };
+
+// Lists whose sort gave up a wait are not to be read; the host finds the word and raises.
+__device__ __forceinline__ bool lists_invalid(const BackwardArgs &g) { return g.list_status && *g.list_status != TG_STATUS_OK; }
 
 // process_backward's inputs for one list entry.
 struct alignas(16) BackRecord {
@@ -469,6 +474,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
     __shared__ uint8_t s_touch[kBackBatch];
     __shared__ WaveRect s_rects[kMaxTileWaves];
     __shared__ int s_last;
+    if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
@@ -690,6 +696,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
 
     __shared__ uint8_t s_touch[kBatch];
     __shared__ WaveRect s_rects[kMaxTileWaves];
+    if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
@@ -813,6 +820,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
     __shared__ int s_tag[kMaxWaves][kWave];         // the same by column of the term matrix
     __shared__ int s_vertex[kMaxWaves][3 * kWave];  // the three vertex ids of a column's entry
     __shared__ uint8_t s_src[kMaxWaves][kWave];     // the pixel (lane) of a slot
+    if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
@@ -1008,7 +1016,7 @@ size_t backward_pixel_order_lds_bytes(int n_threads) { return pixel_order_lds_by
 
 using namespace tg;
 
-static int render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices,
+int tg::render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices,
                                   const int32_t *indices, const real *colors, const real *opacities,
                                   const int32_t *sorted_ids, const int32_t *offsets, const real *bary, const real *image,
                                   const real *depthmap, const real *final_weights, const int32_t *ends, const int32_t *last,
@@ -1016,7 +1024,7 @@ static int render_backward(const real *grad_image, const real *grad_depthmap, co
                                   int height, int tile_w,
                                   int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers, real *grad_vertices,
                                   real *grad_colors, real *grad_opacities, int vertex_stride, int color_stride,
-                                  int opacity_stride, void *stream) {
+                                  int opacity_stride, const uint32_t *list_status, void *stream) {
     if (int e = check_raster_args("tg_render_backward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!grad_image || !vertices || !indices || !colors || !opacities || !offsets || !bary || !image ||
         !depthmap || !final_weights || !ends || !last || !grad_vertices || !grad_colors || !grad_opacities ||
@@ -1036,7 +1044,7 @@ static int render_backward(const real *grad_image, const real *grad_depthmap, co
                  width, height, tile_w, tile_h, early_stopping_threshold, max_layers};
     BackwardArgs g{(const real4 *)grad_image, grad_depthmap, (const real4 *)image, depthmap, final_weights, ends, last,
                    last_depth, order, per_pixel_sort ? nullptr : hit_masks, grad_vertices, grad_colors, grad_opacities,
-                   vertex_stride, color_stride, opacity_stride};
+                   vertex_stride, color_stride, opacity_stride, list_status};
     hipStream_t s = (hipStream_t)stream;
     const int layout = (vertex_stride == 4 && color_stride == 3 && opacity_stride == 1)   ? kGradDense
                        : (vertex_stride == 8 && color_stride == 8 && opacity_stride == 8) ? kGradBlock8
@@ -1085,7 +1093,7 @@ extern "C" int tg_render_backward(const real *grad_image, const real *grad_depth
     return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
                            final_weights, ends, last, last_depth, order, hit_masks, width, height, tile_w, tile_h,
                            early_stopping_threshold, per_pixel_sort, max_layers, grad_vertices, grad_colors, grad_opacities,
-                           vertex_stride, color_stride, opacity_stride, stream);
+                           vertex_stride, color_stride, opacity_stride, nullptr, stream);
 }
 
 extern "C" int tg_render_backward_pooled(const real *grad_image, const real *grad_depthmap, const real *vertices,
@@ -1103,7 +1111,7 @@ extern "C" int tg_render_backward_pooled(const real *grad_image, const real *gra
     const OrderStore order{const_cast<uint16_t *>(order_pool), n_triangles > kShortList ? n_keys * pixels : 0, pixels};
     return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
                            final_weights, ends, last, nullptr, order, nullptr, width, height, tile_w, tile_h, early_stopping_threshold,
-                           1, max_layers, grad_vertices, grad_colors, grad_opacities, vertex_stride, color_stride, opacity_stride, stream);
+                           1, max_layers, grad_vertices, grad_colors, grad_opacities, vertex_stride, color_stride, opacity_stride, nullptr, stream);
 }
 
 extern "C" int tg_split_gradient_block(const real *block, int64_t n_vertices, real *grad_vertices, real *grad_colors,

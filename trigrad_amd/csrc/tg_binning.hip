@@ -11,6 +11,7 @@
 //                    the clip passes run that a key needs
 // The count + scan kernels and bary_kernel (60 B read, 36 B written per triangle) are bound by memory traffic, the
 // emission kernels by the vector instructions of the clipping.
+#include "tg_frame.hpp"
 #include "tg_raster.hpp"
 #include "tg_scan.hpp"
 #include "tg_sort_plan.hpp"
@@ -576,6 +577,21 @@ __device__ __forceinline__ uint32_t frame_tile_prefix(uint64_t *states, int tile
     return prefix;
 }
 
+// render.cu:310-337 cartesian_to_bary_kernel: the nine scalars of one triangle's matrix.
+__device__ __forceinline__ void write_bary(const TriXYZ &p, real *__restrict__ m) {
+    real denom = p.ax * (p.by - p.cy) + p.bx * (p.cy - p.ay) + p.cx * (p.ay - p.by);
+    if (abs_real(denom) < kEffZero) denom = 1.0f;
+    m[0] = (p.by - p.cy) / denom;
+    m[1] = (p.cx - p.bx) / denom;
+    m[2] = (p.bx * p.cy - p.cx * p.by) / denom;
+    m[3] = (p.cy - p.ay) / denom;
+    m[4] = (p.ax - p.cx) / denom;
+    m[5] = (p.cx * p.ay - p.ax * p.cy) / denom;
+    m[6] = (p.ay - p.by) / denom;
+    m[7] = (p.bx - p.ax) / denom;
+    m[8] = (p.ax * p.by - p.bx * p.ay) / denom;
+}
+
 __global__ __launch_bounds__(kScanThreads) void frame_scan_kernel(const real4 *__restrict__ vertices, int n_vertices,
                                                                   const int32_t *__restrict__ indices, int n_triangles, int W, int H,
                                                                   int tw, int th, int tiles_x, int tiles_y, uint32_t epoch,
@@ -584,7 +600,7 @@ __global__ __launch_bounds__(kScanThreads) void frame_scan_kernel(const real4 *_
                                                                   int n_scan_tiles, uint32_t head_capacity, uint32_t *__restrict__ heads,
                                                                   uint32_t *totals, uint32_t *totals_next,
                                                                   real *__restrict__ edges, uint32_t *zero, size_t zero_words,
-                                                                  uint32_t *clear_word) {
+                                                                  uint32_t *clear_word, real *__restrict__ bary) {
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_wave_total[kScanThreads / kWave];
     __shared__ uint32_t s_tile_prefix;
@@ -640,6 +656,7 @@ __global__ __launch_bounds__(kScanThreads) void frame_scan_kernel(const real4 *_
             records[t] = make_real4(A, B, C, int_in_real(r.x0));
             records[(int64_t)n_triangles + t] = make_real4(p.ax, p.ay, p.bx, p.by);
             records[2 * (int64_t)n_triangles + t] = make_real4(p.cx, p.cy, int_in_real(r.y0), int_in_real(r.y1 - r.y0 + 1));
+            if (bary) write_bary(p, bary + 9 * t);
             rect = r;
         }
         s_count[k * kScanThreads + tid] = count;
@@ -762,12 +779,16 @@ __global__ __launch_bounds__(kEmitThreads) void frame_emit_kernel(const real4 *_
                                                                   uint32_t key_capacity, const uint32_t *__restrict__ heads,
                                                                   uint32_t head_capacity, const real *__restrict__ edges, int tiles_x,
                                                                   int column_bits, uint64_t *__restrict__ keys,
-                                                                  uint32_t *__restrict__ payload) {
+                                                                  uint32_t *__restrict__ payload, uint32_t epoch, uint64_t *host_total) {
     __shared__ EmitLds L;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
     const uint32_t total = total_and_status[0];
+    if (host_total && blockIdx.x == 0 && tid == 0)
+        // K and whether a wait of the scan expired, straight to where the host looks for them
+        __hip_atomic_store(host_total, ((uint64_t)(total_and_status[1] == epoch ? TG_FRAME_EXPIRED : TG_FRAME_COUNTED) << 32) | total,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const uint32_t n_keys = total < key_capacity ? total : key_capacity;  // keys beyond the buffers are left out
     const uint32_t k0 = blockIdx.x * (uint32_t)kEmitChunk;
     if (k0 >= n_keys) return;
@@ -984,25 +1005,12 @@ __global__ __launch_bounds__(kBoundThreads) void list_bounds_kernel(const real *
     if (lane == 0) far_start[tile] = s_far;
 }
 
-// render.cu:310-337 cartesian_to_bary_kernel.
 __global__ __launch_bounds__(kBinThreads) void bary_kernel(const real4 *__restrict__ vertices, int n_vertices,
                                                            const int32_t *__restrict__ indices, int n_triangles,
                                                            real *__restrict__ out) {
     const int t = blockIdx.x * kBinThreads + threadIdx.x;
     if (t >= n_triangles) return;
-    const TriXYZ p = load_triangle(vertices, n_vertices, indices, t);
-    real denom = p.ax * (p.by - p.cy) + p.bx * (p.cy - p.ay) + p.cx * (p.ay - p.by);
-    if (abs_real(denom) < kEffZero) denom = 1.0f;
-    real *m = out + 9 * (int64_t)t;
-    m[0] = (p.by - p.cy) / denom;
-    m[1] = (p.cx - p.bx) / denom;
-    m[2] = (p.bx * p.cy - p.cx * p.by) / denom;
-    m[3] = (p.cy - p.ay) / denom;
-    m[4] = (p.ax - p.cx) / denom;
-    m[5] = (p.cx * p.ay - p.ax * p.cy) / denom;
-    m[6] = (p.ay - p.by) / denom;
-    m[7] = (p.bx - p.ax) / denom;
-    m[8] = (p.ax * p.by - p.bx * p.ay) / denom;
+    write_bary(load_triangle(vertices, n_vertices, indices, t), out + 9 * (int64_t)t);
 }
 
 static int check_geometry(const char *fn, const void *vertices, int n_vertices, const void *indices, int n_triangles, int W, int H,
@@ -1170,10 +1178,10 @@ extern "C" size_t tg_bin_frame_workspace_bytes(int32_t n_triangles, int64_t key_
     return fused_frame(nullptr, n_triangles, key_capacity, ceil_div(width, tile_w), ceil_div(height, tile_h)).bytes;
 }
 
-extern "C" int tg_bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indices, int32_t n_triangles, int width,
-                            int height, int tile_w, int tile_h, uint64_t *keys, uint32_t *values, int64_t key_capacity,
-                            uint32_t *total_and_status, void *frame, size_t frame_bytes, uint32_t epoch, void *zero,
-                            size_t zero_bytes, uint32_t *clear_word, void *stream) {
+int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indices, int32_t n_triangles, int width, int height,
+                  int tile_w, int tile_h, uint64_t *keys, uint32_t *values, int64_t key_capacity, uint32_t *total_and_status,
+                  void *frame, size_t frame_bytes, uint32_t epoch, void *zero, size_t zero_bytes, uint32_t *clear_word, real *bary,
+                  uint64_t *host_total, void *stream) {
 #ifdef TG_DOUBLE_PRECISION
     set_error("tg_bin_frame: the double build's depth keys take all 64 key bits; use tg_bin_setup and tg_build_tile_lists");
     return TG_E_ARG;
@@ -1208,15 +1216,23 @@ extern "C" int tg_bin_frame(const real *vertices, int32_t n_vertices, const int3
     TG_LAUNCH(frame_scan_kernel, dim3(n_scan_tiles), dim3(kScanThreads), 0, s, (const real4 *)vertices, n_vertices, indices, n_triangles,
               width, height, tile_w, tile_h, tiles_x, tiles_y, epoch, f.tri_offsets, f.records, total_and_status, ticket, f.states,
               n_scan_tiles, f.head_capacity, f.heads, grid.on ? fused_frame_totals(frame, epoch) : (uint32_t *)nullptr,
-              fused_frame_totals(frame, epoch + 1), f.edges, (uint32_t *)zero, zero_bytes / 4, clear_word);
+              fused_frame_totals(frame, epoch + 1), f.edges, (uint32_t *)zero, zero_bytes / 4, clear_word, bary);
     if (int e = check_launch("frame_scan_kernel")) return e;
     if (key_capacity == 0) return 0;
     // for every key position the buffers hold: the kernel reads K and the workgroups behind it leave at once
     TG_LAUNCH(frame_emit_kernel, dim3((unsigned)ceil_div64(key_capacity, kEmitChunk)), dim3(kEmitThreads), 0, s, f.records, f.tri_offsets,
               n_triangles, total_and_status, (uint32_t)key_capacity, f.heads, f.head_capacity, f.edges, tiles_x,
-              grid.on ? grid.column_bits : 0, keys, values);
+              grid.on ? grid.column_bits : 0, keys, values, epoch, host_total);
     return check_launch("frame_emit_kernel");
 #endif
+}
+
+extern "C" int tg_bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indices, int32_t n_triangles, int width,
+                            int height, int tile_w, int tile_h, uint64_t *keys, uint32_t *values, int64_t key_capacity,
+                            uint32_t *total_and_status, void *frame, size_t frame_bytes, uint32_t epoch, void *zero,
+                            size_t zero_bytes, uint32_t *clear_word, void *stream) {
+    return bin_frame(vertices, n_vertices, indices, n_triangles, width, height, tile_w, tile_h, keys, values, key_capacity,
+                     total_and_status, frame, frame_bytes, epoch, zero, zero_bytes, clear_word, nullptr, nullptr, stream);
 }
 
 namespace tg {

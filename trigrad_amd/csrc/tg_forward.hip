@@ -12,6 +12,7 @@
 //
 // Not HBM-bound: per (pixel, entry) pair ~12 VALU operations and three
 // broadcast LDS reads against 148 B of gathered data per ENTRY.
+#include "tg_frame.hpp"
 #include "tg_raster.hpp"
 
 namespace tg {
@@ -26,11 +27,18 @@ struct ForwardOut {
     OrderStore order;    // blend order: list positions relative to the tile's start
     uint64_t *hit_masks; // tile order: which list entries cover which pixel, 64 entries per word (see hit_mask_chunk); may be null
     const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
+    uint32_t *host_status;        // where the host looks for that word (memory of its own); may be null
 };
 
 // Lists whose sort gave up a wait are not to be read (unwritten entries may name anything): the frame's pixels
 // are marked instead, so that the caller sees it in the image itself.
-__device__ __forceinline__ bool lists_invalid(const ForwardOut &o) { return o.list_status && *o.list_status != TG_STATUS_OK; }
+__device__ __forceinline__ bool lists_invalid(const ForwardOut &o) {
+    if (!o.list_status) return false;
+    const uint32_t status = *o.list_status;
+    if (o.host_status && (blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0)
+        __hip_atomic_store(o.host_status, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return status != TG_STATUS_OK;
+}
 __device__ __forceinline__ void mark_pixel_invalid(const ForwardOut &o, const PixelCoord &p) {
     if (!p.valid) return;
     const real nan = std::numeric_limits<real>::quiet_NaN();
@@ -334,7 +342,7 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
     __shared__ uint8_t s_touch[kSelectBatch];
     __shared__ WaveRect s_rects[kMaxTileWaves];
     __shared__ uint64_t s_votes[kMaxTileWaves];
-    if (lists_invalid(out)) return;  // the launch before this one has marked every pixel
+    if (out.list_status && *out.list_status != TG_STATUS_OK) return;  // the launch before this one has marked every pixel
     const int tiles = tiles_x * tiles_y;
     const int share = (tiles + (int)gridDim.x - 1) / (int)gridDim.x;
     const int first = blockIdx.x * share, past = min(first + share, tiles);
@@ -419,12 +427,13 @@ extern "C" size_t tg_hit_mask_words(int64_t n_keys, int width, int height, int t
     return (size_t)(tiles * tl.grid.z + (n_keys / kWave + tiles + 1) * (int64_t)tl.grid.z * tl.threads);
 }
 
-static int render_forward(const real *vertices, const int32_t *indices, const real *colors, const real *opacities,
+int tg::render_forward(const real *vertices, const int32_t *indices, const real *colors, const real *opacities,
                                  const int32_t *sorted_ids, const int32_t *offsets, const real *bary, int width, int height,
                                  int tile_w, int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers,
                                  real *image, real *depthmap, real *final_weights, int32_t *ends, int32_t *last,
                                  real *last_depth, const OrderStore &order, uint64_t *hit_masks, const real *batch_bounds,
-                                 const int32_t *far_start, const uint32_t *list_status, void *stream) {
+                                 const int32_t *far_start, const uint32_t *list_status, uint32_t *host_status, int64_t longest,
+                                 void *stream) {
     if (int e = check_raster_args("tg_render_forward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!vertices || !indices || !colors || !opacities || !offsets || !bary || !image || !depthmap || !final_weights || !ends) {
         set_error("tg_render_forward: null pointer");
@@ -442,7 +451,7 @@ static int render_forward(const real *vertices, const int32_t *indices, const re
         return TG_E_ARG;
     }
     ForwardOut o{(real4 *)image, depthmap, final_weights, ends, last, last_depth, order, per_pixel_sort ? nullptr : hit_masks,
-                 list_status};
+                 list_status, host_status};
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
     const dim3 grid = tl.grid;
     const int n_threads = tl.threads;
@@ -468,6 +477,7 @@ static int render_forward(const real *vertices, const int32_t *indices, const re
     TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatchShort, uint16_t>), grid, dim3(n_threads),
                  lds_short, s, a, o);
     if (int e = check_launch("forward_pixel_order_kernel")) return e;
+    if (longest <= kShortList) return 0;  // no list is too long for 16-bit positions
     if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;
     const int tiles = (int)(grid.x * grid.y);
     TG_LAUNCH(forward_pixel_order_long_lists_kernel, dim3(min(tiles, kLongListGroups), 1, grid.z), dim3(n_threads), lds, s, a, o,
@@ -488,7 +498,7 @@ extern "C" int tg_render_forward(const real *vertices, const int32_t *indices, c
     const OrderStore order{fragments, (int64_t)max_layers * width * height, 0};
     return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
                           early_stopping_threshold, per_pixel_sort, max_layers, image, depthmap, final_weights, ends, last, last_depth,
-                          order, hit_masks, batch_bounds, far_start, list_status, stream);
+                          order, hit_masks, batch_bounds, far_start, list_status, nullptr, std::numeric_limits<int64_t>::max(), stream);
 }
 
 extern "C" int64_t tg_order_pool_words(int64_t n_keys, int64_t n_triangles, int tile_w, int tile_h) {
@@ -511,5 +521,5 @@ extern "C" int tg_render_forward_pooled(const real *vertices, const int32_t *ind
     const OrderStore order{order_pool, n_triangles > kShortList ? n_keys * pixels : 0, pixels};
     return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
                           early_stopping_threshold, 1, max_layers, image, depthmap, final_weights, ends, last, last_depth, order, nullptr,
-                          batch_bounds, far_start, list_status, stream);
+                          batch_bounds, far_start, list_status, nullptr, n_keys, stream);
 }

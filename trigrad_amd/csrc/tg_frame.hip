@@ -1,0 +1,251 @@
+// tg_frame.hip -- a frame's forward pass, and its backward pass, in one call each.
+//
+// Small frames are bound by the host: a frame of 20 triangles keeps the GPU busy for 70 us and took 310 us when every stage
+// was a call of its own with its own buffers and the host waited for K (the number of keys) half way, to size the rest.
+// Here the host launches the whole chain for the capacity of the key buffers, the kernels read K on the device, and the
+// host waits for K only when everything is under way: it then knows whether the buffers were large enough (if not, the
+// kernels have made empty lists and the caller comes again with larger ones).  K and the list kernels' status word are
+// written by the kernels into pinned host memory and found there by looking, so a frame has no copies and no events.
+#include <hip/hip_runtime.h>
+#include <immintrin.h>
+
+#include <atomic>
+#include <chrono>
+
+#include "tg_frame.hpp"
+
+namespace tg {
+
+#ifndef TG_DOUBLE_PRECISION
+struct FrameLayout {
+    // kept: what the backward pass and the caller look at later
+    size_t status, ids, offsets, bary, weights, ends, last, last_depth, order, masks, kept_bytes;
+    // scratch: dead when the forward pass is done
+    size_t keys, keys_alt, values_alt, sort, bounds, far_start, low, scratch_bytes;
+    size_t sort_bytes;
+};
+
+static FrameLayout frame_layout(const tg_frame &f) {
+    FrameLayout L = {};
+    const int tiles_x = (int)ceil_div64(f.width, f.tile_w), tiles_y = (int)ceil_div64(f.height, f.tile_h), tiles = tiles_x * tiles_y;
+    const int64_t pixels = f.width * f.height;
+    size_t o = 0;
+    const auto take = [&](size_t bytes) { const size_t at = o; o = (o + bytes + 255) & ~(size_t)255; return at; };
+    const bool backward = f.flags & TG_FRAME_BACKWARD;
+    L.status = take(4);  // of the sort
+    L.ids = take((size_t)f.key_capacity * 4);
+    L.offsets = take((size_t)(tiles + 1) * 4);
+    L.bary = take((size_t)f.n_triangles * 9 * sizeof(real));
+    L.weights = take((size_t)pixels * sizeof(real));
+    L.ends = take((size_t)pixels * 4);
+    if (backward) {
+        L.last = take((size_t)pixels * 4);
+        if (f.per_pixel_sort) L.last_depth = take((size_t)pixels * sizeof(real));
+        if (f.flags & TG_FRAME_ORDER_PLANES) L.order = take((size_t)(2 * f.max_layers * pixels) * 2);
+        if (f.flags & TG_FRAME_ORDER_POOL)
+            L.order = take((size_t)tg_order_pool_words(f.key_capacity, f.n_triangles, (int)f.tile_w, (int)f.tile_h) * 2);
+        if (f.flags & TG_FRAME_HIT_MASKS)
+            L.masks = take(tg_hit_mask_words(f.key_capacity, (int)f.width, (int)f.height, (int)f.tile_w, (int)f.tile_h) * 8);
+    }
+    L.kept_bytes = o;
+    o = 0;
+    L.keys = take((size_t)f.key_capacity * 8);
+    L.keys_alt = take((size_t)f.key_capacity * 8);
+    L.values_alt = take((size_t)f.key_capacity * 4);
+    L.sort_bytes = tg_build_frame_lists_workspace_bytes(f.key_capacity, tiles_x, tiles_y);
+    L.sort = take(L.sort_bytes);
+    if (f.flags & TG_FRAME_LIST_BOUNDS) {
+        L.bounds = take(tg_list_bound_words(f.key_capacity, tiles) * sizeof(real));
+        L.far_start = take((size_t)tiles * 4);
+        L.low = take((size_t)f.n_triangles * sizeof(real));
+    }
+    L.scratch_bytes = o;
+    return L;
+}
+
+static int check_frame(const char *fn, const tg_frame *f) {
+    if (!f || f->n_vertices < 0 || f->n_vertices > 0x7fffffff || f->n_triangles <= 0 || f->n_triangles > 0x7fffffff || f->width <= 0 ||
+        f->height <= 0 || f->width > 0x7fffffff || f->height > 0x7fffffff || f->tile_w <= 0 || f->tile_h <= 0 ||
+        f->tile_w > kMaxTilePixels || f->tile_h > kMaxTilePixels || f->key_capacity <= 0 || f->key_capacity >= (1ll << 30)) {
+        set_error("%s: null frame, or a size out of range", fn);
+        return TG_E_ARG;
+    }
+    if (int e = check_raster_args(fn, (int)f->width, (int)f->height, (int)f->tile_w, (int)f->tile_h, (int)f->max_layers)) return e;
+    if (!tg_frame_supported((int)f->width, (int)f->height, (int)f->tile_w, (int)f->tile_h)) {
+        set_error("%s: more than 256 tile columns or rows", fn);
+        return TG_E_ARG;
+    }
+    return 0;
+}
+
+// Zeroes the gradients, 16 bytes a thread.
+__global__ __launch_bounds__(256) void zero_gradients_kernel(real4 *p, int64_t n4) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n4) p[i] = make_real4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+static OrderStore frame_order(const tg_frame &f, const FrameLayout &L, char *kept) {
+    if (f.flags & TG_FRAME_ORDER_PLANES) return OrderStore{(uint16_t *)(kept + L.order), f.max_layers * f.width * f.height, 0};
+    if (f.flags & TG_FRAME_ORDER_POOL) {
+        const int pixels = order_pool_pixels((int)f.tile_w, (int)f.tile_h);
+        return OrderStore{(uint16_t *)(kept + L.order), f.n_triangles > kShortList ? f.key_capacity * pixels : 0, pixels};
+    }
+    return OrderStore{nullptr, 0, 0};
+}
+#endif
+
+}  // namespace tg
+
+using namespace tg;
+
+extern "C" int tg_frame_supported(int width, int height, int tile_w, int tile_h) {
+    if (!tg_bin_frame_supported(width, height, tile_w, tile_h)) return 0;
+    return frame_grid_fits(ceil_div(width, tile_w), ceil_div(height, tile_h)) ? 1 : 0;
+}
+
+#ifdef TG_DOUBLE_PRECISION
+static int no_frame(const char *fn) {
+    set_error("%s: float build only", fn);
+    return TG_E_ARG;
+}
+extern "C" int tg_frame_layout(const tg_frame *, int64_t *) { return no_frame("tg_frame_layout"); }
+extern "C" int tg_frame_forward(tg_frame *) { return no_frame("tg_frame_forward"); }
+extern "C" int tg_frame_backward(const tg_frame *) { return no_frame("tg_frame_backward"); }
+#else
+extern "C" int tg_frame_layout(const tg_frame *f, int64_t *out) {
+    if (int e = check_frame("tg_frame_layout", f)) return e;
+    if (!out) { set_error("tg_frame_layout: null pointer"); return TG_E_ARG; }
+    const FrameLayout L = frame_layout(*f);
+    const int64_t words[TG_FRAME_LAYOUT_WORDS] = {
+        (int64_t)L.kept_bytes, (int64_t)L.scratch_bytes,
+        (int64_t)tg_bin_frame_workspace_bytes((int32_t)f->n_triangles, f->key_capacity, (int)f->width, (int)f->height, (int)f->tile_w, (int)f->tile_h),
+        (int64_t)L.status, (int64_t)L.ids, (int64_t)L.offsets, (int64_t)L.bary, (int64_t)L.weights, (int64_t)L.ends, (int64_t)L.last,
+        (int64_t)L.last_depth, (int64_t)L.order, (int64_t)L.masks};
+    for (int i = 0; i < TG_FRAME_LAYOUT_WORDS; i++) out[i] = words[i];
+    return 0;
+}
+
+extern "C" int tg_frame_forward(tg_frame *f) {
+    if (int e = check_frame("tg_frame_forward", f)) return e;
+    const FrameLayout L = frame_layout(*f);
+    if (f->kept_bytes < (int64_t)L.kept_bytes || f->scratch_bytes < (int64_t)L.scratch_bytes) {
+        set_error("tg_frame_forward: buffers of %lld and %lld bytes, need %zu and %zu", (long long)f->kept_bytes,
+                  (long long)f->scratch_bytes, L.kept_bytes, L.scratch_bytes);
+        return TG_E_WORKSPACE;
+    }
+    if (!f->kept || !f->scratch || !f->host || !f->frame || (f->frame_bytes & 7) || ((uintptr_t)f->kept & 255) || ((uintptr_t)f->scratch & 255) || ((uintptr_t)f->host & 7)) {
+        set_error("tg_frame_forward: null or misaligned buffer");
+        return TG_E_ARG;
+    }
+    char *kept = (char *)f->kept, *scratch = (char *)f->scratch;
+    const int W = (int)f->width, H = (int)f->height, tw = (int)f->tile_w, th = (int)f->tile_h;
+    const int tiles_x = ceil_div(W, tw), tiles_y = ceil_div(H, th), tiles = tiles_x * tiles_y;
+    const int32_t V = (int32_t)f->n_vertices, M = (int32_t)f->n_triangles;
+    uint32_t *status = (uint32_t *)(kept + L.status);
+    uint32_t *total_and_status = (uint32_t *)((char *)f->frame + f->frame_bytes);
+    uint64_t *keys = (uint64_t *)(scratch + L.keys);
+    uint32_t *ids = (uint32_t *)(kept + L.ids);
+    int32_t *offsets = (int32_t *)(kept + L.offsets);
+    real *bary = (real *)(kept + L.bary);
+    volatile uint32_t *host = f->host;
+    const int64_t longest = f->key_capacity < f->n_triangles ? f->key_capacity : f->n_triangles;  // a triangle is in a list once
+    if (f->phases & TG_FRAME_BIN) {
+        host[1] = 0;
+        host[2] = TG_FRAME_PENDING;
+        if (int e = bin_frame(f->vertices, V, f->indices, M, W, H, tw, th, keys, ids, f->key_capacity, total_and_status, f->frame,
+                              (size_t)f->frame_bytes, (uint32_t)f->epoch, scratch + L.sort, L.sort_bytes, status, bary,
+                              (uint64_t *)f->host, f->stream))
+            return e;
+    }
+    if (f->phases & TG_FRAME_LISTS) {
+        int in_alt = 0;  // two passes: the pairs are back where they started
+        if (int e = build_frame_lists(f->frame, (uint32_t)f->epoch, f->key_capacity, total_and_status, longest, tiles_x, tiles_y, keys,
+                                      ids, (uint64_t *)(scratch + L.keys_alt), (uint32_t *)(scratch + L.values_alt), offsets,
+                                      scratch + L.sort, L.sort_bytes, status, &in_alt, f->stream))
+            return e;
+    }
+    if (f->phases & TG_FRAME_RASTER) {
+        real *bounds = nullptr;
+        int32_t *far_start = nullptr;
+        if (f->flags & TG_FRAME_LIST_BOUNDS) {
+            bounds = (real *)(scratch + L.bounds);
+            far_start = (int32_t *)(scratch + L.far_start);
+            if (int e = tg_list_bounds(f->vertices, V, f->indices, M, keys, (const int32_t *)ids, offsets, tiles,
+                                       (real *)(scratch + L.low), bounds, far_start, f->stream))
+                return e;
+        }
+        const bool backward = f->flags & TG_FRAME_BACKWARD;
+        if (int e = render_forward(f->vertices, f->indices, f->colors, f->opacities, (const int32_t *)ids, offsets, bary, W, H, tw, th,
+                                   (real)f->early_stopping_threshold, (int)f->per_pixel_sort, (int)f->max_layers, f->image, f->depthmap,
+                                   (real *)(kept + L.weights), (int32_t *)(kept + L.ends), backward ? (int32_t *)(kept + L.last) : nullptr,
+                                   backward && f->per_pixel_sort ? (real *)(kept + L.last_depth) : nullptr, frame_order(*f, L, kept),
+                                   (f->flags & TG_FRAME_HIT_MASKS) ? (uint64_t *)(kept + L.masks) : nullptr, bounds, far_start, status,
+                                   (uint32_t *)f->host + 2, longest, f->stream))
+            return e;
+    }
+    if (f->phases & TG_FRAME_WAIT) {
+        if (int e = tg_frame_wait(f->host, 1, 0, f->stream)) return e;
+        f->n_keys = host[0];
+        f->counted = host[1];
+    }
+    return 0;
+}
+
+extern "C" int tg_frame_backward(const tg_frame *f) {
+    if (int e = check_frame("tg_frame_backward", f)) return e;
+    const FrameLayout L = frame_layout(*f);
+    if (!f->kept || f->kept_bytes < (int64_t)L.kept_bytes || !(f->flags & TG_FRAME_BACKWARD) || !f->gradients ||
+        ((uintptr_t)f->gradients & 15) || ((uintptr_t)f->kept & 255) || (f->per_pixel_sort && (!f->block || ((uintptr_t)f->block & 15)))) {
+        set_error("tg_frame_backward: null, small or misaligned buffer, or a frame rendered without TG_FRAME_BACKWARD");
+        return TG_E_ARG;
+    }
+    char *kept = (char *)f->kept;
+    const int64_t V = f->n_vertices;
+    if (V == 0) return 0;
+    // one zero fill for the three gradients.  Tile order: (V,4) | (V,3) | (V,) behind each other.  Per-pixel order issues
+    // five times as many atomics; there the eight gradients of a vertex share a 32-byte sector of a (V,8) block while
+    // the kernel runs, and the three arrays are copied out afterwards.
+    real *sums = f->per_pixel_sort ? f->block : f->gradients;
+    TG_LAUNCH(zero_gradients_kernel, dim3((unsigned)ceil_div64(2 * V, 256)), dim3(256), 0, (hipStream_t)f->stream, (real4 *)sums, 2 * V);
+    if (int e = check_launch("zero_gradients_kernel")) return e;
+    const int stride = f->per_pixel_sort ? 8 : 0;
+    if (int e = render_backward(f->grad_image, f->grad_depthmap, f->vertices, f->indices, f->colors, f->opacities,
+                                (const int32_t *)(kept + L.ids), (const int32_t *)(kept + L.offsets), (const real *)(kept + L.bary), f->image,
+                                f->depthmap, (const real *)(kept + L.weights), (const int32_t *)(kept + L.ends),
+                                (const int32_t *)(kept + L.last), f->per_pixel_sort ? (const real *)(kept + L.last_depth) : nullptr,
+                                frame_order(*f, L, kept), (f->flags & TG_FRAME_HIT_MASKS) ? (const uint64_t *)(kept + L.masks) : nullptr,
+                                (int)f->width, (int)f->height, (int)f->tile_w, (int)f->tile_h, (real)f->early_stopping_threshold,
+                                (int)f->per_pixel_sort, (int)f->max_layers, sums, stride ? sums + 4 : sums + 4 * V,
+                                stride ? sums + 7 : sums + 7 * V, stride ? stride : 4, stride ? stride : 3, stride ? stride : 1,
+                                (const uint32_t *)(kept + L.status), f->stream))
+        return e;
+    if (!f->per_pixel_sort) return 0;
+    return tg_split_gradient_block(f->block, V, f->gradients, f->gradients + 4 * V, f->gradients + 7 * V, f->stream);
+}
+#endif
+
+extern "C" int tg_frame_wait(const uint32_t *host, int word, uint32_t pending, void *stream) {
+    if (!host || word < 0 || word > 3) {
+        set_error("tg_frame_wait: null pointer or no such word");
+        return TG_E_ARG;
+    }
+    const volatile uint32_t *at = host + word;
+    // the word is written early in a kernel; looking for it costs neither an event nor the wake-up of a sleeping thread.
+    // A stream busy with something long, or a frame whose kernels failed, ends the looking and waits for the stream.
+    const auto start = std::chrono::steady_clock::now();
+    for (int looks = 0; *at == pending; looks++) {
+        _mm_pause();
+        if ((looks & 63) == 63 && std::chrono::steady_clock::now() - start > std::chrono::milliseconds(50)) {
+            const hipError_t e = hipStreamSynchronize((hipStream_t)stream);
+            if (e != hipSuccess) {
+                set_error("tg_frame_wait: %s", hipGetErrorString(e));
+                return (int)e;
+            }
+            if (*at != pending) break;
+            set_error("tg_frame_wait: the stream is done and the word is not there");
+            return TG_E_ARG;
+        }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return 0;
+}

@@ -29,6 +29,7 @@
 // (then no workgroup has to finish for another to start), by the workgroup ids,
 // which saves the serialised same-address atomics.  Waits are bounded
 // (TG_STATUS_LOOKBACK_TIMEOUT).
+#include "tg_frame.hpp"
 #include "tg_scan.hpp"
 #include "tg_sort_plan.hpp"
 
@@ -203,7 +204,8 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
                                                                   int64_t n, int shift, uint32_t mask,
                                                                   const uint32_t *__restrict__ bases, int totals_given,
                                                                   uint32_t *lookback, uint32_t *ticket, uint32_t *status,
-                                                                  int unpad_bits, int tiles_x, uint32_t *tile_count) {
+                                                                  int unpad_bits, int tiles_x, uint32_t *tile_count,
+                                                                  FrameCount frame_count) {
     constexpr int kDigits = 1 << BITS;
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_global_delta[kRadix];
@@ -243,6 +245,10 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
     }
     const int tile = (int)s_tile;
     const int64_t tile_base = (int64_t)tile * kSortTile;
+    // with the number of pairs on the device the grid is made for the buffers' capacity: the rest has nothing to do
+    n = frame_count.pairs(n);
+    const int n_tiles = frame_count.word ? (int)((n + kSortTile - 1) / kSortTile) : (int)gridDim.x;
+    if (tile >= n_tiles) return;
     const int n_valid = (int)((n - tile_base) < kSortTile ? (n - tile_base) : kSortTile);
 
     // Wave-striped loads keep memory order = (wave, item, lane) order.
@@ -333,7 +339,7 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
                 in_group += word & kLbValueMask;
             }
         }
-        const bool closes_group = tile == group_first + kLookGroup - 1 || tile == (int)gridDim.x - 1;
+        const bool closes_group = tile == group_first + kLookGroup - 1 || tile == n_tiles - 1;
         if (closes_group)
             __hip_atomic_store(group_words + (size_t)group * kDigits, (group == 0 ? kLbInclusive : kLbAggregate) | ((in_group + published) & kLbValueMask),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -631,7 +637,10 @@ struct MediumSegLds {
 __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64_t *keys, uint32_t *vals, int32_t *offsets,
                                                                           int n_segments, const uint32_t *__restrict__ tile_count,
                                                                           const uint32_t *__restrict__ row_totals, int tiles_x,
-                                                                          uint32_t n_pairs) {
+                                                                          uint32_t n_pairs, FrameCount frame_count, uint32_t *status) {
+    n_pairs = (uint32_t)frame_count.pairs(n_pairs);
+    // lists made from a scan whose wait expired are as invalid as those of a sort whose wait did
+    if (frame_count.word && blockIdx.x == 0 && threadIdx.x == 0 && frame_count.word[1] == frame_count.epoch) *status = TG_STATUS_LOOKBACK_TIMEOUT;
     __shared__ union SmallLds {
         WaveSegLds wave[kSortWaves];
         MediumSegLds medium;
@@ -831,9 +840,10 @@ __global__ __launch_bounds__(kSortThreads) void tile_ranges_kernel(const uint64_
 template <int BITS>
 static void launch_sweep(dim3 grid, hipStream_t s, const uint64_t *kin, const uint32_t *vin, uint64_t *kout, uint32_t *vout,
                          int64_t n, int shift, uint32_t mask, const uint32_t *bases, int totals_given, uint32_t *lookback,
-                         uint32_t *ticket, uint32_t *status, int unpad_bits, int tiles_x, uint32_t *tile_count) {
+                         uint32_t *ticket, uint32_t *status, int unpad_bits, int tiles_x, uint32_t *tile_count,
+                         FrameCount frame_count) {
     hipLaunchKernelGGL(sort_sweep_kernel<BITS>, grid, dim3(kSweepThreads), 0, s, kin, vin, kout, vout, n, shift, mask, bases,
-                       totals_given, lookback, ticket, status, unpad_bits, tiles_x, tile_count);
+                       totals_given, lookback, ticket, status, unpad_bits, tiles_x, tile_count, frame_count);
 }
 
 // The sweeps of `plan` over (keys, values) <-> (keys_alt, values_alt).  bases: per pass kRadix words, the
@@ -843,7 +853,7 @@ static void launch_sweep(dim3 grid, hipStream_t s, const uint64_t *kin, const ui
 static int run_sweeps(const char *fn, const PassPlan &plan, int n_sort_tiles, const uint32_t *bases, int totals_given,
                       uint32_t *lookback, uint32_t *tickets, uint64_t *keys, uint32_t *values, uint64_t *keys_alt,
                       uint32_t *values_alt, int64_t n, uint32_t *status, hipStream_t s, int unpad_bits = 0, int tiles_x = 0,
-                      uint32_t *tile_count = nullptr) {
+                      uint32_t *tile_count = nullptr, FrameCount frame_count = FrameCount()) {
     uint64_t *kin = keys, *kout = keys_alt;
     uint32_t *vin = values, *vout = values_alt;
     // 534 same-address ticket atomics cost 6 us per pass; a grid that fits the device whole takes its
@@ -863,11 +873,11 @@ static int run_sweeps(const char *fn, const PassPlan &plan, int n_sort_tiles, co
         const int ub = last ? unpad_bits : 0;
         uint32_t *tc = last ? tile_count : (uint32_t *)nullptr;
         switch (plan.bits[p]) {
-        case 8: launch_sweep<8>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc); break;
-        case 7: launch_sweep<7>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc); break;
-        case 6: launch_sweep<6>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc); break;
-        case 5: launch_sweep<5>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc); break;
-        default: launch_sweep<4>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc); break;
+        case 8: launch_sweep<8>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        case 7: launch_sweep<7>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        case 6: launch_sweep<6>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        case 5: launch_sweep<5>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        default: launch_sweep<4>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
         }
         if (int e = check_launch(fn)) return e;
         uint64_t *tk = kin; kin = kout; kout = tk;
@@ -895,14 +905,16 @@ static int run_passes(const char *fn, const PassPlan &plan, const SortLayout &L,
 // With tile_count (the last sweep counted every tile's pairs) the ranges come from the counts, inside the segment kernel.
 static int ranges_and_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint32_t *v_other, int64_t n, int n_tiles,
                                int32_t *offsets, hipStream_t s, const uint32_t *tile_count = nullptr,
-                               const uint32_t *row_totals = nullptr, int tiles_x = 0) {
+                               const uint32_t *row_totals = nullptr, int tiles_x = 0, FrameCount frame_count = FrameCount(),
+                               uint32_t *status = nullptr, int64_t longest = std::numeric_limits<int64_t>::max()) {
     if (!tile_count) {
         TG_LAUNCH(tile_ranges_kernel, dim3((unsigned)ceil_div64(n + 1, kSortThreads)), dim3(kSortThreads), 0, s, k, n, n_tiles, offsets);
         if (int e = check_launch("tile_ranges_kernel")) return e;
     }
     TG_LAUNCH(segment_sort_small_kernel, dim3(ceil_div(n_tiles, kSortWaves)), dim3(kSortThreads), 0, s, k, v, offsets, n_tiles,
-              tile_count, row_totals, tiles_x, (uint32_t)n);
+              tile_count, row_totals, tiles_x, (uint32_t)n, frame_count, status);
     if (int e = check_launch("segment_sort_small_kernel")) return e;
+    if (longest <= kSegMediumCap) return 0;  // no list can be longer than what the kernel above sorts
     TG_LAUNCH(segment_sort_large_kernel, dim3(n_tiles < kSegLargeGrid ? n_tiles : kSegLargeGrid), dim3(kSortThreads), 0, s, k, v,
               k_other, v_other, offsets, n_tiles);
     return check_launch("segment_sort_large_kernel");
@@ -1105,9 +1117,13 @@ extern "C" size_t tg_build_frame_lists_workspace_bytes(int64_t n_keys, int tiles
     return kFrameSortHeadBytes + 2 * lookback_words_per_pass(ceil_div64(n_keys > 0 ? n_keys : 1, kSortTile)) * 4 + (size_t)(n_tiles + 1) * 4;
 }
 
-extern "C" int tg_build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, int tiles_x, int tiles_y, uint64_t *keys,
-                                    uint32_t *values, uint64_t *keys_alt, uint32_t *values_alt, int32_t *offsets, void *workspace,
-                                    size_t workspace_bytes, uint32_t *status, int *result_in_alt, void *stream) {
+bool tg::frame_grid_fits(int tiles_x, int tiles_y) { return grid_plan(tiles_x, tiles_y).on; }
+
+// total_and_status: null, or tg_bin_frame's pair on the device; n_keys is then the capacity of the buffers, a frame with
+// more keys than that gets empty lists, and no list holds more than `longest` keys.
+int tg::build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, const uint32_t *total_and_status, int64_t longest, int tiles_x,
+                          int tiles_y, uint64_t *keys, uint32_t *values, uint64_t *keys_alt, uint32_t *values_alt, int32_t *offsets,
+                          void *workspace, size_t workspace_bytes, uint32_t *status, int *result_in_alt, void *stream) {
     if (n_keys < 0 || n_keys > kSortMaxN || tiles_x <= 0 || tiles_y <= 0 || (int64_t)tiles_x * tiles_y > 0x7fffffff || !frame ||
         !result_in_alt || !offsets) {
         set_error("tg_build_frame_lists: n_keys must be in [0, 2^30), tile counts positive, frame state, offsets and result_in_alt given");
@@ -1125,6 +1141,10 @@ extern "C" int tg_build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys,
         return check_launch("tile_ranges_kernel");
     }
     const GridPlan grid = grid_plan(tiles_x, tiles_y);
+    if (!grid.on && total_and_status) {
+        set_error("tg_build_frame_lists: the number of keys has to be known with more than 256 tile columns or rows");
+        return TG_E_ARG;
+    }
     if (!grid.on)
         return sort_tile_lists_run("tg_build_frame_lists", keys, values, keys_alt, values_alt, n_keys, n_tiles, offsets, workspace,
                                    workspace_bytes, status, result_in_alt, s);
@@ -1140,9 +1160,18 @@ extern "C" int tg_build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys,
     uint32_t *lookback = (uint32_t *)((char *)workspace + kFrameSortHeadBytes);
     uint32_t *tile_count = (uint32_t *)((char *)workspace + kFrameSortHeadBytes + lookback_bytes);
     const uint32_t *totals = fused_frame_totals(frame, epoch);
+    const FrameCount count{total_and_status, (uint32_t)n_keys, epoch};
     if (int e = run_sweeps("tg_build_frame_lists", grid.plan, n_sort_tiles, totals, 1, lookback, tickets, keys, values, keys_alt,
-                           values_alt, n_keys, status, s, grid.column_bits, tiles_x, tile_count))
+                           values_alt, n_keys, status, s, grid.column_bits, tiles_x, tile_count, count))
         return e;
     // two passes: the sorted pairs are back in (keys, values)
-    return ranges_and_segments(keys, values, keys_alt, values_alt, n_keys, n_tiles, offsets, s, tile_count, totals + kRadix, tiles_x);
+    return ranges_and_segments(keys, values, keys_alt, values_alt, n_keys, n_tiles, offsets, s, tile_count, totals + kRadix, tiles_x,
+                               count, status, longest);
+}
+
+extern "C" int tg_build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, int tiles_x, int tiles_y, uint64_t *keys,
+                                    uint32_t *values, uint64_t *keys_alt, uint32_t *values_alt, int32_t *offsets, void *workspace,
+                                    size_t workspace_bytes, uint32_t *status, int *result_in_alt, void *stream) {
+    return build_frame_lists(frame, epoch, n_keys, nullptr, n_keys, tiles_x, tiles_y, keys, values, keys_alt, values_alt, offsets,
+                             workspace, workspace_bytes, status, result_in_alt, stream);
 }

@@ -48,8 +48,20 @@ class Renderer(Function):
             depthmap = torch.full((height, width), float("inf"), dtype=colors.dtype, device=colors.device)
             timings = None
             ctx.save_for_backward(vertices, indices, colors, opacities)
+        elif not record_timing and _C.frame_supported(vertices, width, height, tile_width, tile_height):
+            ctx.skipped = False
+            for_backward = any(ctx.needs_input_grad)
+            _C.verify_finished_frames()
+            image, depthmap, kept, frame = _C.frame_forward(
+                vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
+                per_pixel_sort, max_layers, for_backward)
+            if for_backward:
+                ctx.frame = frame
+                ctx.save_for_backward(vertices, indices, colors, opacities, image, depthmap, kept)
+            return image, depthmap
         else:
             ctx.skipped = False
+            ctx.frame = None
             (image, depthmap, final_weights, sorted_ids, offsets, bary_transforms, ends, timings, resume) = _C._forward_full(
                 vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
                 not record_timing, per_pixel_sort, max_layers, for_backward=any(ctx.needs_input_grad))
@@ -61,7 +73,7 @@ class Renderer(Function):
             ctx.has_last_depth = last_depth is not None
             ctx.has_fragments = fragments is not None
             ctx.has_hit_masks = hit_masks is not None
-            ctx.has_order_pool = resume.order_pool is not None
+            ctx.has_order_pool, ctx.pool_keys = resume.order_pool is not None, resume.pool_keys
             ctx.status_check = status_check
             if not any(ctx.needs_input_grad):
                 return (image, depthmap, timings) if record_timing else (image, depthmap)
@@ -78,6 +90,11 @@ class Renderer(Function):
             grad_vertices = torch.zeros_like(ctx.saved_tensors[0])
             grad_colors = torch.zeros_like(ctx.saved_tensors[2])
             grad_opacities = torch.zeros_like(ctx.saved_tensors[3])
+        elif ctx.frame is not None:
+            saved = ctx.saved_tensors
+            if grad_image is None:
+                grad_image = torch.zeros_like(saved[4])
+            grad_vertices, grad_colors, grad_opacities = _C.frame_backward(ctx.frame, grad_image, grad_depthmap, *saved)
         else:
             saved = ctx.saved_tensors
             last = saved[11]
@@ -86,7 +103,7 @@ class Renderer(Function):
             fragments = extras.pop(0) if ctx.has_fragments else None
             hit_masks = extras.pop(0) if ctx.has_hit_masks else None
             resume = _C.Resume((last, last_depth, ctx.status_check, fragments, hit_masks))
-            resume.order_pool = extras.pop(0) if ctx.has_order_pool else None
+            resume.order_pool, resume.pool_keys = extras.pop(0) if ctx.has_order_pool else None, ctx.pool_keys
             width, height, tile_width, tile_height, threshold, per_pixel_sort, max_layers = ctx.render_args
             if grad_image is None:
                 grad_image = torch.zeros_like(saved[7])
