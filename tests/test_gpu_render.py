@@ -614,7 +614,8 @@ def test_scene_without_a_single_key(mode, cuda):
 def test_frame_in_one_call_is_the_frame_stage_by_stage(n_triangles, size, tile, mode, cuda, monkeypatch):
     """The one-call route against the stages with K on the host, at the edges of its rules: one triangle, one list of 2048 and
     2049 entries (what the small segment sort takes), more than one sort tile, 256 and 257 tile columns (the staged route's).
-    The second run has key buffers that are far too small: empty lists first, then the frame again."""
+    The second run is the torch module's, the third has key buffers that are far too small: empty lists first, then the frame
+    again."""
     import torch
     import trigrad_amd
     from trigrad_amd import _C
@@ -637,7 +638,9 @@ def test_frame_in_one_call_is_the_frame_stage_by_stage(n_triangles, size, tile, 
     assert supported == (size // tile <= 256) and (key in _C._frame_key_hints) == supported
     if supported:
         K = _C._frame_key_hints[key]
+        got.append(run())  # by the torch module
         _C._frame_key_hints[key] = 0
+        _C._module().forget()
         monkeypatch.setattr(_C, "_round_capacity", lambda n: max(n, 1))
         got.append(run())
         assert _C._frame_key_hints[key] == K

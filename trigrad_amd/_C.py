@@ -4,7 +4,8 @@ argument order, implemented by calling the C ABI of libtrigrad_hip.so on the
 current torch stream.  torch is used for device memory and streams only.
 
 A frame is one call forward (`frame_forward`: binning, lists and blending, launched for the capacity of the key buffers
-while the kernels read K on the device) and one call backward (`frame_backward`).  Frames with more than 256 tile columns or
+while the kernels read K on the device) and one call backward (`frame_backward`).  The first frame of a kind runs here and
+leaves its plan with the torch module (csrc/tg_torch.cpp), which renders the following ones.  Frames with more than 256 tile columns or
 rows run stage by stage:
     bin_frame (count + scan, then key emission that reads K on the device) -> (K to the host, bary matrices meanwhile)
     -> build_frame_lists (passes over the tile bits through memory, depth bits and tile ranges per tile)
@@ -354,11 +355,15 @@ def _next_frame_state(dev, need):
     with _frame_lock:
         st = _frame_states.get(key)
         if st is None or st["bytes"] < need or st["epoch"] >= 0x3FFFFFF0:
-            size = need + need // 4
+            size = _state_size(need)
             st = dict(frame=torch.zeros((size + _FRAME_TAIL,), dtype=torch.uint8, device=dev), epoch=0, bytes=size)
             _frame_states[key] = st
         st["epoch"] += 1
         return st["frame"], st["bytes"], st["epoch"]
+
+
+def _state_size(need):
+    return -(-(need + need // 4) // 256) * 256
 
 
 def bin_frame(vertices, indices, width, height, tile_width, tile_height, capacity=None):
@@ -587,6 +592,8 @@ def verify_frames(wait=True):
     after it returns every frame rendered so far on this process is known to be good: what a caller who only
     renders forward (no backward pass, whose first step is this check) calls before it trusts a frame.
     wait=False looks only at the words that have arrived."""
+    if _lib._torch_module is not None:
+        _lib._torch_module.verify(wait)
     with _pending_lock:
         checks = list(_pending_checks)
         del _pending_checks[:]
@@ -671,6 +678,14 @@ class _FramePlan:
         self.kind = pack(self.kept_bytes, self.scratch_bytes)
 
 
+def _plan_for(kind):
+    plan = _frame_plans.get(kind)
+    if plan is None:
+        plan = _FramePlan(*kind)
+        _remember(_frame_plans, kind, plan)
+    return plan
+
+
 def _remember(table, key, value):
     if len(table) >= _MAX_REMEMBERED and key not in table:
         table.clear()
@@ -688,6 +703,49 @@ def _round_capacity(n):
 class Frame:
     """A frame rendered by frame_forward: its plan, the status of its lists and (K) the keys it has."""
     __slots__ = ("plan", "status", "n_keys")
+
+
+def render_by_torch_module(vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
+                           record_timing, per_pixel_sort, max_layers):
+    """(image, depthmap) of a frame whose kind was seen before, with its autograd node, or None: for the route through Python."""
+    global _module_settings
+    settings = (ONE_CALL_FRAME, FUSED_BINNING, SAVE_BLEND_ORDER, SAVE_HIT_MASKS, EARLY_STOP_MIN_AVG_LIST, ORDER_POOL_MAX_BYTES, precision)
+    if settings != _module_settings:
+        _module().forget()
+        _module_settings = settings
+    if not ONE_CALL_FRAME or precision is not torch.float32:
+        return None
+    if _pending_checks:
+        verify_frames(wait=False)
+    return _lib._torch_module.render(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
+                                     early_stopping_threshold, record_timing, per_pixel_sort, max_layers)
+
+
+_module_settings = None  # what the module's plans were made for
+
+
+def _module():
+    return _lib.torch_module(_key_count_hint)
+
+
+def _leave_plan(plan, kind, for_backward, dev, stream):
+    """Hands the plan of the frames to come (and a frame state for the stream) to the torch module."""
+    n_vertices, n_triangles, width, height, tile_width, tile_height, per_pixel_sort, max_layers, capacity, flags, threshold = kind
+    low, high = capacity // 4 if capacity > 1 << 18 else 0, 1 << 30
+    if per_pixel_sort:
+        # the depth bounds are for lists of a length; a scene that hovers around it keeps what it has
+        long_lists = EARLY_STOP_MIN_AVG_LIST * (-(-width // tile_width) * -(-height // tile_height))
+        if flags & _FRAME_LIST_BOUNDS:
+            low = max(low, long_lists - long_lists // 4)
+        else:
+            high = min(high, long_lists + long_lists // 4)
+    module = _module()
+    key = (dev.index, n_vertices, n_triangles, width, height, tile_width, tile_height,
+           struct.unpack("<q", struct.pack("<d", threshold))[0], per_pixel_sort, max_layers, 1 if for_backward else 0)
+    module.remember(key, plan.kind, plan.frame_bytes, low, high)
+    if module.state_bytes(dev.index, stream) < plan.frame_bytes:
+        size = _state_size(plan.frame_bytes)
+        module.add_state(dev.index, stream, torch.zeros((size + _FRAME_TAIL,), dtype=torch.uint8, device=dev), size)
 
 
 def frame_supported(vertices, width, height, tile_width, tile_height):
@@ -718,25 +776,24 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
             elif SAVE_BLEND_ORDER:
                 flags |= _FRAME_ORDER_PLANES if max_layers <= MAX_SAVED_LAYERS else _FRAME_ORDER_POOL
         hint_key = (dev.index, n_triangles, width, height, tile_width, tile_height)
+
+        def kind_for(expected, capacity):
+            # long lists: depth bounds let the selection leave a list before its end
+            bounds = per_pixel_sort and expected >= EARLY_STOP_MIN_AVG_LIST * (-(-width // tile_width) * -(-height // tile_height))
+            return (n_vertices, n_triangles, width, height, tile_width, tile_height, 1 if per_pixel_sort else 0, max_layers, capacity,
+                    flags | _FRAME_LIST_BOUNDS if bounds else flags, float(early_stopping_threshold))
+
         expected = _frame_key_hints.get(hint_key)
         if expected is None:
             expected, capacity = 2 * n_triangles, min(3 * n_triangles + 65536, (1 << 30) - 1)
         else:
             capacity = _round_capacity(expected)
-        # long lists: depth bounds let the selection leave a list before its end
-        if per_pixel_sort and expected >= EARLY_STOP_MIN_AVG_LIST * (-(-width // tile_width) * -(-height // tile_height)):
-            flags |= _FRAME_LIST_BOUNDS
         image = torch.empty((height, width, 4), dtype=torch.float32, device=dev)
         depthmap = torch.empty((height, width), dtype=torch.float32, device=dev)
         stream = _raw_stream(dev)
         frame = Frame()
         while True:
-            kind = (n_vertices, n_triangles, width, height, tile_width, tile_height, 1 if per_pixel_sort else 0, max_layers, capacity,
-                    flags, float(early_stopping_threshold))
-            plan = _frame_plans.get(kind)
-            if plan is None:
-                plan = _FramePlan(*kind)
-                _remember(_frame_plans, kind, plan)
+            plan = _plan_for(kind_for(expected, capacity))
             kept = torch.empty((plan.kept_bytes,), dtype=torch.uint8, device=dev)
             scratch = torch.empty((plan.scratch_bytes,), dtype=torch.uint8, device=dev)
             _frame_counter += 1
@@ -775,6 +832,9 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
         _key_count_hint[dev.index] = n_keys
         with _pending_lock:
             _pending_checks.append(status)
+        if timer is None:
+            kind = kind_for(n_keys, _round_capacity(n_keys))
+            _leave_plan(_plan_for(kind), kind, for_backward, dev, stream)
     frame.plan, frame.status, frame.n_keys = plan, status, n_keys
     return image, depthmap, kept, frame
 

@@ -109,3 +109,25 @@ def check(code, what, bits=32):
     if code != 0:
         msg = load(bits).tg_last_error()
         raise RuntimeError(f"{what} failed with code {code}: {msg.decode() if msg else ''}")
+
+
+_torch_module = None
+
+
+def torch_module(key_counts):
+    """trigrad_torch.so (csrc/tg_torch.cpp), bound to the float library.  key_counts: the dict it notes every frame's K in."""
+    global _torch_module
+    if _torch_module is None:
+        import importlib.machinery
+        import importlib.util
+        path = os.path.join(_HERE, "lib", "trigrad_torch.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `python -m trigrad_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("trigrad_torch", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("trigrad_torch", loader))
+        loader.exec_module(module)
+        lib = load(32)
+        module.bind(*[C.cast(getattr(lib, name), C.c_void_p).value for name in (
+            "tg_frame_forward", "tg_frame_backward", "tg_frame_wait", "tg_force_tickets", "tg_last_error")], key_counts)
+        _torch_module = module
+    return _torch_module

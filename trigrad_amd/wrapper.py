@@ -144,5 +144,9 @@ def render(
     """
     if tile_width * tile_height > 1024:
         raise ValueError("tile_width * tile_height must be <= 1024")
+    frame = _C.render_by_torch_module(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
+                                      early_stopping_threshold, record_timing, per_pixel_sort, max_layers)
+    if frame is not None:
+        return frame
     return Renderer.apply(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
                           early_stopping_threshold, record_timing, per_pixel_sort, max_layers)
