@@ -127,6 +127,36 @@ def test_tile_list_longer_than_16_bit_positions(mode, tile, cuda, oracle):
         assert_gradients_close(f"long list/{mode}: {label}", g.cpu().numpy(), w, mag)
 
 
+def _crowded_scene(n, width, height):
+    """Triangles of a pixel or two, most of them in one corner (a list far longer than the mean), a few large ones, and some
+    whose vertices are infinite or NaN or whose 1/w is zero."""
+    import scenes as S
+    soup = S.random_soup(n, width, height, seed=21, sigma_px=0.8, opacity=(0.1, 0.9), varying_w=True)
+    v = soup["vertices"].copy().reshape(n, 3, 4)
+    corner = np.random.default_rng(5).random(n) < 0.7
+    v[corner, :, :2] = (v[corner, :, :2] + 1.0) * 0.12 - 1.0
+    big = np.arange(n) % 97 == 0
+    centre = v[big, :, :2].mean(axis=1, keepdims=True)
+    v[big, :, :2] = centre + (v[big, :, :2] - centre) * 15.0
+    v[5::501, 1, 0], v[7::503, 2, 1], v[9::499, 0, 3] = np.inf, np.nan, 0.0
+    return dict(soup, vertices=v.reshape(-1, 4))
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
+@pytest.mark.parametrize("n,width,height,tw,th", [
+    (12000, 70, 45, 16, 16),   # partial tiles on both sides
+    (1500, 70, 45, 8, 8),      # one wave to a workgroup
+    (12000, 70, 45, 24, 16),   # six squares of 8 x 8 pixels, two workgroups
+    (12000, 64, 64, 32, 32),
+    (6000, 70, 45, 12, 6),     # a wave's pixels are no square
+    (40000, 400, 300, 16, 16),
+])
+def test_crowds_of_small_triangles_match_oracle(n, width, height, tw, th, mode, cuda, oracle):
+    scene = _crowded_scene(n, width, height)
+    _, want, got, _ = _forward_both(scene, tw, th, MODES[mode], cuda, oracle)
+    _check_forward(f"crowd {n}/{tw}x{th}/{mode}", want, got, (th, tw))
+
+
 def _grad_inputs(scene, seed, with_depth):
     rng = np.random.default_rng(seed)
     H, W = scene["height"], scene["width"]

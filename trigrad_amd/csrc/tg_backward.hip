@@ -417,22 +417,6 @@ __device__ __forceinline__ void add_run_sums(real *terms, int n, uint64_t heads,
 
 __device__ __forceinline__ int top_bit(uint64_t m) { return 63 - __builtin_clzll(m); }
 
-// Transposes the 64 x 64 bit matrix whose row i is the word x of lane i: afterwards bit i of
-// lane b's word is what bit b of lane i's word was.  Six exchange steps between lanes 32, 16, ... 1
-// apart, each swapping the off-diagonal blocks of that size.
-__device__ __forceinline__ uint64_t transpose_bits(uint64_t x, int lane) {
-    constexpr uint64_t kHigh[6] = {0xFFFFFFFF00000000ull, 0xFFFF0000FFFF0000ull, 0xFF00FF00FF00FF00ull,
-                                   0xF0F0F0F0F0F0F0F0ull, 0xCCCCCCCCCCCCCCCCull, 0xAAAAAAAAAAAAAAAAull};
-#pragma unroll
-    for (int s = 0; s < 6; s++) {
-        const int j = 32 >> s;
-        const uint32_t lo = __shfl_xor((uint32_t)x, j, kWave), hi = __shfl_xor((uint32_t)(x >> 32), j, kWave);
-        const uint64_t y = ((uint64_t)hi << 32) | lo;
-        x = (lane & j) ? (x & kHigh[s]) | ((y >> j) & ~kHigh[s]) : (x & ~kHigh[s]) | ((y << j) & kHigh[s]);
-    }
-    return x;
-}
-
 __device__ __forceinline__ int wave_max_i32(int v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, kWave));
@@ -479,7 +463,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward>();
+    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkBackward>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile];
     const PixelCoord p = pixel_of_thread(a, tile_id);
@@ -700,7 +684,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward>();
+    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkBackward>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);
@@ -729,11 +713,11 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
             __syncthreads();
             for (int e = tid; e < nb; e += blockDim.x) {
                 gather_depth(a, batch + e, s_rec[e]);
-                s_touch[e] = (uint8_t)waves_touched(s_rec[e].m, s_rects, n_waves);
+                s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent));
             }
             __syncthreads();
             uint64_t m[kBatch / kWave];
-            batch_hit_mask<kBatch / kWave>(s_rec, s_touch, nb, wave, p.px, p.py, m);
+            batch_hit_mask<kBatch / kWave>(a, s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
             if (!want) {
 #pragma unroll
                 for (int wd = 0; wd < kBatch / kWave; wd++) m[wd] = 0;
@@ -824,7 +808,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward>();
+    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkBackward>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);

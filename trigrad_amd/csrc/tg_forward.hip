@@ -67,14 +67,16 @@ __device__ __forceinline__ void write_pixel(const ForwardOut &o, const PixelCoor
     o.image[p.index] = make_real4(s.c0, s.c1, s.c2, s.alpha);
 }
 
-__global__ __launch_bounds__(kTileThreads) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
+// Eight waves per SIMD (64 registers, a few of the loop's constants in scratch memory): 212 -> 194 us against the 73 registers
+// it would take (10^6 triangles, 1920 x 1080).
+__global__ __launch_bounds__(kTileThreads, 8) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
     __shared__ BlendRecord s_rec[kBatch];
     __shared__ uint8_t s_touch[kBatch];
     __shared__ WaveRect s_rects[kMaxTileWaves];
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandForward>();
+    const TileId tile_id = tile_of_workgroup<kTileBandForward, kChunkForward>();
     const int tile = tile_id.index;
     const PixelCoord p = pixel_of_thread(a, tile_id);
     if (lists_invalid(out)) {  // the same for the whole launch
@@ -93,12 +95,12 @@ __global__ __launch_bounds__(kTileThreads) void forward_tile_order_kernel(Raster
         const int nb = min(kBatch, end - batch);
         for (int e = tid; e < nb; e += blockDim.x) {
             gather_blend(a, batch + e, s_rec[e]);
-            s_touch[e] = (uint8_t)waves_touched(s_rec[e].m, s_rects, n_waves);
+            s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent));
         }
         __syncthreads();
         // 1. inside tests; a lane keeps its hits as a 256-bit mask
         uint64_t m[kBatch / kWave];
-        batch_hit_mask<kBatch / kWave>(s_rec, s_touch, nb, wave, p.px, p.py, m);
+        batch_hit_mask<kBatch / kWave>(a, s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
         if (!running) {
 #pragma unroll
             for (int wd = 0; wd < kBatch / kWave; wd++) m[wd] = 0;
@@ -164,7 +166,7 @@ constexpr int kLongListGroups = 256;    // workgroups that look for the tiles wi
 // The per-pixel-order forward pass of one tile.  Pos: how a candidate's list position (from the tile's
 // start) is kept.  With uint16_t the candidate lists of a 16x16 tile take 48 KB instead of 64 KB, which
 // together with 64 staged entries lets a CU hold three workgroups instead of two.
-template <int kStage, typename Pos>  // kStage: list entries staged per batch
+template <int kStage, typename Pos, bool kInTurn>  // kStage: list entries staged per batch
 __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const ForwardOut &out, int tile_x, int tile_y, int tiles_x,
                                                  unsigned char *s_dyn, uint8_t *s_touch, WaveRect *s_rects) {
     const int n_threads = blockDim.x;
@@ -193,16 +195,30 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
         if (!__syncthreads_or(want)) break;
         const int cap = want ? min(kLayers, a.max_layers - s.blended) : 0;
         int found = 0;
-        // The records of the next batch are fetched into registers while this batch is worked on: the
-        // chain of dependent loads (list -> indices -> vertices, matrix) of a batch takes as long as its
-        // inside tests, and with two workgroups per CU nothing else would cover it.  (Not with depth
-        // bounds, which make the batches jump.)
-        const bool ahead = !a.batch_bounds && (int)blockDim.x >= kStage;
-        DepthRecord fetched;
-        if (ahead && tid < min(kStage, end - start)) gather_depth(a, start + tid, fetched);
-        for (int batch = start; batch < end; batch += kStage) {
+        // Without depth bounds (which make the batches jump) the records of coming batches are fetched into registers while
+        // this batch is worked on.  A wave that asks for an entry's vertices has to have its vertex numbers, and for those its
+        // triangle number: three memory latencies in a row, and whoever asks waits for the first two.  So the four waves
+        // of a tile take the batches of 64 in turn (kInTurn), and a wave's links are asked for two batches apart (its own
+        // turn comes every fourth batch); each has arrived when the next one needs it.  A frame with a list of 8400
+        // entries in one tile: 241 -> 154 us; lists of 268 everywhere: 680 -> 669.
+        const int lane = tid & (kWave - 1);
+        const bool ahead = !kInTurn && !a.batch_bounds && (int)blockDim.x >= kStage;
+        DepthParts next;
+        if constexpr (kInTurn) {
+            const int j = min(start + tid, end - 1);
+            next.fetch_triangle(a, j);
+            next.fetch_matrix(a);
+            next.fetch_triangle(a, min(j + kTileThreads, end - 1));
+            next.fetch_vertices(a);
+        } else if (ahead && tid < min(kStage, end - start)) {
+            next.fetch_triangle(a, start + tid);
+            next.fetch_matrix(a);
+            next.fetch_vertices(a);
+        }
+        int turn = 0;
+        for (int batch = start; batch < end; batch += kStage, turn = (turn + 1) & 3) {
             const int nb = min(kStage, end - batch);
-            if (a.batch_bounds) {
+            if (!kInTurn && a.batch_bounds) {
                 // a lane needs nothing from here on when its list is full and its worst candidate is nearer than
                 // every fragment the rest of the tile's list can produce (a full list rejects depths >= its worst)
                 const real rest = a.batch_bounds[batch_bound_index(start, tile, batch - start)];
@@ -217,23 +233,37 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 }
             }
             __syncthreads();
-            if (ahead) {
-                if (tid < nb) {
-                    s_rec[tid] = fetched;
-                    s_touch[tid] = (uint8_t)waves_touched(fetched.m, s_rects, n_waves);
-                }
-            } else {
+            if (kInTurn ? wave == turn && lane < nb : ahead && tid < nb) {
+                const int e = kInTurn ? lane : tid;
+                const DepthRecord r = next.record();
+                s_rec[e] = r;
+                s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves) | small_entry(a, r.extent));
+            }
+            if (!kInTurn && !ahead) {
                 for (int e = tid; e < nb; e += blockDim.x) {
                     gather_depth(a, batch + e, s_rec[e]);
-                    s_touch[e] = (uint8_t)waves_touched(s_rec[e].m, s_rects, n_waves);
+                    s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent));
                 }
             }
             __syncthreads();
-            if (ahead && batch + kStage < end && tid < min(kStage, end - batch - kStage)) gather_depth(a, batch + kStage + tid, fetched);
+            if constexpr (kInTurn) {
+                if (wave == turn) {
+                    // my next batch: its triangle numbers are here; ask for vertex numbers and matrices, and for the triangle
+                    // numbers of the batch after it (past the list's end: its last entry again, which nobody looks at)
+                    next.fetch_matrix(a);
+                    next.fetch_triangle(a, min(batch + 8 * kWave + lane, end - 1));
+                } else if (wave == (turn ^ 2)) {
+                    next.fetch_vertices(a);
+                }
+            } else if (ahead && batch + kStage < end && tid < min(kStage, end - batch - kStage)) {
+                next.fetch_triangle(a, batch + kStage + tid);
+                next.fetch_matrix(a);
+                next.fetch_vertices(a);
+            }
             // inside tests into a per-lane mask, then every lane visits its own hits in
             // list order (the order insert_sorted_topk sees them in the reference)
             uint64_t m[kStage / kWave];
-            batch_hit_mask<kStage / kWave>(s_rec, s_touch, nb, wave, p.px, p.py, m);
+            batch_hit_mask<kStage / kWave>(a, s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
             if (!want) {
 #pragma unroll
                 for (int wd = 0; wd < kStage / kWave; wd++) m[wd] = 0;
@@ -319,18 +349,19 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
 
 // One workgroup per tile.  With 16-bit positions the tiles whose lists are too long for them are left to
 // forward_pixel_order_long_lists_kernel.
-template <int kStage, typename Pos>
-__global__ __launch_bounds__(kTileThreads) void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
+// kInTurn: kStage is 64 and the workgroup has four waves.
+template <int kStage, typename Pos, bool kInTurn>
+__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 && kStage == kSelectBatchShort ? 3 : 2) void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ uint8_t s_touch[kStage];
     __shared__ WaveRect s_rects[kMaxTileWaves];
-    const TileId tile = tile_of_workgroup<kTileBandForward>();
+    const TileId tile = tile_of_workgroup<kTileBandForward, kChunkForward>();
     if (lists_invalid(out)) {  // the same for the whole launch
         mark_pixel_invalid(out, pixel_of_thread(a, tile));
         return;
     }
     if (sizeof(Pos) < sizeof(int) && a.offsets[tile.index + 1] - a.offsets[tile.index] > kShortList) return;
-    pixel_order_tile<kStage, Pos>(a, out, tile.x, tile.y, gridDim.x, s_dyn, s_touch, s_rects);
+    pixel_order_tile<kStage, Pos, kInTurn>(a, out, tile.x, tile.y, gridDim.x, s_dyn, s_touch, s_rects);
 }
 
 // The tiles whose lists are longer than kShortList, with int positions: few or none, so a small grid
@@ -360,7 +391,7 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
                 const int tile = base + w * kWave + __builtin_ctzll(todo);
                 todo &= todo - 1;
                 __syncthreads();  // the tile before is done with the LDS
-                pixel_order_tile<kSelectBatch, int>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, s_dyn, s_touch, s_rects);
+                pixel_order_tile<kSelectBatch, int, false>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, s_dyn, s_touch, s_rects);
             }
         }
     }
@@ -465,17 +496,22 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     const bool split = !a.batch_bounds && n_threads >= kSelectBatchShort;
     static size_t lds_reserved[kMaxDevices] = {0}, lds_reserved_long[kMaxDevices] = {0};
     if (!split) {
-        if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_kernel<kSelectBatch, int>, lds, lds_reserved)) return e;
-        TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatch, int>), grid, dim3(n_threads), lds, s, a, o);
+        if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_kernel<kSelectBatch, int, false>, lds, lds_reserved)) return e;
+        TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatch, int, false>), grid, dim3(n_threads), lds, s, a, o);
         return check_launch("forward_pixel_order_kernel");
     }
     const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t));
-    static size_t lds_reserved_short[kMaxDevices] = {0};
-    if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_kernel<kSelectBatchShort, uint16_t>, lds_short,
-                            lds_reserved_short))
-        return e;
-    TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatchShort, uint16_t>), grid, dim3(n_threads),
-                 lds_short, s, a, o);
+    static size_t lds_reserved_short[2][kMaxDevices] = {{0}};
+    const bool in_turn = n_threads == kTileThreads;
+    const void *kernel = in_turn ? (const void *)forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true>
+                                 : (const void *)forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false>;
+    if (int e = reserve_lds("tg_render_forward", kernel, lds_short, lds_reserved_short[in_turn])) return e;
+    if (in_turn)
+        TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true>), grid, dim3(n_threads),
+                     lds_short, s, a, o);
+    else
+        TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false>), grid, dim3(n_threads),
+                     lds_short, s, a, o);
     if (int e = check_launch("forward_pixel_order_kernel")) return e;
     if (longest <= kShortList) return 0;  // no list is too long for 16-bit positions
     if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;

@@ -69,8 +69,13 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
 // turn in the order of their linear index, and every XCD has an L2 of its own; neighbouring tiles share list
 // entries (a triangle that covers two tiles is in both lists), vertices and matrices.  So the workgroups
 // that reach one XCD take consecutive tiles of an order that keeps neighbours together: bands of kTileBand
-// tile rows, column by column inside a band.  XCD k gets the k-th eighth of that order, and the workgroups that
-// run there at one time cover a compact block of the image.
+// tile rows, column by column inside a band.  The workgroups that run on an XCD at one time cover a compact block of the
+// image.  Backward, XCD k gets the k-th eighth of that order.  Forward, the order is dealt out in chunks of kChunkForward tiles:
+// where a mesh covers part of the image an eighth can be empty and another one full (1.3 million triangles of a torus,
+// 1920 x 1080: two XCDs had 45 % of the list entries, the last one none; 800 -> 680 us of kernel time), and where every tile
+// has the same work nothing is lost (10^6 triangles: 677 -> 668; chunks of 16 to 128 within 1 %).  The backward kernels lose
+// by it what the forward ones gain (10^6 triangles, saved order: 1250 -> 1275): the tiles of a chunk's border then meet in
+// their vertices' gradients on two XCDs.
 #ifndef TG_XCD_TILES
 #define TG_XCD_TILES 1
 #endif
@@ -80,18 +85,32 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
 #ifndef TG_TILE_BAND_BACKWARD
 #define TG_TILE_BAND_BACKWARD 1
 #endif
+#ifndef TG_XCD_CHUNK_FORWARD
+#define TG_XCD_CHUNK_FORWARD 0
+#endif
 constexpr int kXcds = 8;
 constexpr int kTileBandForward = TG_TILE_BAND_FORWARD, kTileBandBackward = TG_TILE_BAND_BACKWARD;
+constexpr int kChunkForward = TG_XCD_CHUNK_FORWARD, kChunkBackward = 0;  // 0: an eighth of the tiles
 struct TileId { int x, y, index; };
-template <int kTileBand>
+template <int kTileBand, int kChunk>
 __device__ __forceinline__ TileId tile_of_workgroup() {
     const int tiles_x = (int)gridDim.x, tiles_y = (int)gridDim.y, n = tiles_x * tiles_y;
     const int linear = (int)(blockIdx.y * gridDim.x + blockIdx.x);
     TileId t;
 #if TG_XCD_TILES
-    const int per = n / kXcds, rest = n % kXcds;
     const int xcd = linear % kXcds, turn = linear / kXcds;
-    const int place = xcd < rest ? xcd * (per + 1) + turn : rest * (per + 1) + (xcd - rest) * per + turn;
+    int place, first = 0, left = turn;  // first: what the rounds of whole chunks take; left: turns after them
+    if (kChunk) {
+        const int round = turn / kChunk;
+        first = round * kXcds * kChunk;
+        left -= round * kChunk;
+    }
+    if (kChunk && first + kXcds * kChunk <= n) {
+        place = first + xcd * kChunk + left;
+    } else {
+        const int per = (n - first) / kXcds, rest = (n - first) % kXcds;
+        place = first + (xcd < rest ? xcd * (per + 1) + left : rest * (per + 1) + (xcd - rest) * per + left);
+    }
     const int band = place / (kTileBand * tiles_x), within = place - band * (kTileBand * tiles_x);
     const int rows = min(kTileBand, tiles_y - band * kTileBand);
     t.x = within / rows;
@@ -112,7 +131,7 @@ struct alignas(16) BlendRecord {
     real iw[3];   // 1/w per vertex (render.cu:444)
     real op[3];
     real col[9];  // vertex a rgb, vertex b rgb, vertex c rgb
-    real pad;
+    real extent;  // of the vertices in y (see small_entry)
 };
 static_assert(sizeof(BlendRecord) == 28 * sizeof(real), "BlendRecord layout");
 constexpr int kBlendWords = 27;  // scalars of a BlendRecord without its padding; odd
@@ -122,7 +141,7 @@ struct alignas(16) DepthRecord {
     real m[9];
     real z[3];
     real w[3];
-    real pad;
+    real extent;
 };
 static_assert(sizeof(DepthRecord) == 16 * sizeof(real), "DepthRecord layout");
 
@@ -142,7 +161,9 @@ __device__ __forceinline__ void gather_blend(const RasterArgs &a, int j, BlendRe
     const real *m = a.bary + 9 * (int64_t)t.tri;
 #pragma unroll
     for (int k = 0; k < 9; k++) r.m[k] = m[k];
-    const real wa = a.vertices[t.ia].w, wb = a.vertices[t.ib].w, wc = a.vertices[t.ic].w;
+    const real4 va = a.vertices[t.ia], vb = a.vertices[t.ib], vc = a.vertices[t.ic];
+    const real wa = va.w, wb = vb.w, wc = vc.w;
+    r.extent = max3(va.y, vb.y, vc.y) - min3(va.y, vb.y, vc.y);
     r.w[0] = wa; r.w[1] = wb; r.w[2] = wc;
     r.iw[0] = 1.0f / wa; r.iw[1] = 1.0f / wb; r.iw[2] = 1.0f / wc;
     r.op[0] = a.opacities[t.ia]; r.op[1] = a.opacities[t.ib]; r.op[2] = a.opacities[t.ic];
@@ -162,7 +183,50 @@ __device__ __forceinline__ void gather_depth(const RasterArgs &a, int j, DepthRe
     const real4 va = a.vertices[t.ia], vb = a.vertices[t.ib], vc = a.vertices[t.ic];
     r.z[0] = va.z; r.z[1] = vb.z; r.z[2] = vc.z;
     r.w[0] = va.w; r.w[1] = vb.w; r.w[2] = vc.w;
+    r.extent = max3(va.y, vb.y, vc.y) - min3(va.y, vb.y, vc.y);
 }
+
+// gather_depth in steps, for a caller that asks for a record's parts before it needs them.  The parts stay as they were
+// loaded (whole vectors, put together by `record` only): a copy into another register would wait for the load.
+typedef real real3v __attribute__((ext_vector_type(3)));
+typedef real real4v __attribute__((ext_vector_type(4)));
+typedef int int3v __attribute__((ext_vector_type(3)));
+struct __attribute__((packed, aligned(4))) TriIndices { int3v id; };
+struct __attribute__((packed, aligned(4))) Matrix9 { real4v a, b; real c; };
+struct DepthParts {
+    int tri;
+    int3v id;
+    real4v m0, m1;
+    real m2;
+    real3v va, vb, vc;  // y, z, w of the vertices
+
+    __device__ __forceinline__ void fetch_triangle(const RasterArgs &a, int j) { tri = a.sorted_ids[j]; }
+    // the triangle's vertex numbers and matrix
+    __device__ __forceinline__ void fetch_matrix(const RasterArgs &a) {
+        const int64_t t = tri;
+        id = reinterpret_cast<const TriIndices *>(a.indices + 3 * t)->id;
+        const Matrix9 *m = reinterpret_cast<const Matrix9 *>(a.bary + 9 * t);
+        m0 = m->a;
+        m1 = m->b;
+        m2 = m->c;
+    }
+    __device__ __forceinline__ void fetch_vertices(const RasterArgs &a) {
+        const real *v = reinterpret_cast<const real *>(a.vertices) + 1;
+        va = *reinterpret_cast<const real3v *>(v + 4 * (int64_t)id.x);
+        vb = *reinterpret_cast<const real3v *>(v + 4 * (int64_t)id.y);
+        vc = *reinterpret_cast<const real3v *>(v + 4 * (int64_t)id.z);
+    }
+    __device__ __forceinline__ DepthRecord record() const {
+        DepthRecord r;
+#pragma unroll
+        for (int k = 0; k < 4; k++) { r.m[k] = m0[k]; r.m[4 + k] = m1[k]; }
+        r.m[8] = m2;
+        r.z[0] = va[1]; r.z[1] = vb[1]; r.z[2] = vc[1];
+        r.w[0] = va[2]; r.w[1] = vb[2]; r.w[2] = vc[2];
+        r.extent = max3(va[0], vb[0], vc[0]) - min3(va[0], vb[0], vc[0]);
+        return r;
+    }
+};
 
 // Saved hit masks (tile order).  The buffer starts with one word per workgroup of the tile launch
 // (index hit_mask_head_index()): the largest `last` among the workgroup's pixels, i.e. how much of the
@@ -307,18 +371,153 @@ __device__ __forceinline__ uint64_t wave_candidates(const uint8_t *s_touch, int 
     return __builtin_amdgcn_ballot_w64(mine);
 }
 
+// Entries whose vertices span less than this many pixel rows are small, and are tested the other way round (lane = entry,
+// small_entry_hits) where a wave's 64 entries hold at least TG_SMALL_MIN of them.  That costs about as much as 20 tests by
+// broadcast whatever their number; below it the broadcast wins, and with 10 instead of 20 a frame of mixed sizes (10^6
+// triangles, mean edge 4 pixels) loses 10 % in per-pixel order and 30 % in tile order.  Entries of 6 or 12 rows make
+// the tallest lane's rows the whole wave's time (tile order, the same frame: 213 -> 218 -> 249 us).
+#ifndef TG_SMALL_ROWS
+#define TG_SMALL_ROWS 4.0f
+#endif
+#ifndef TG_SMALL_MIN
+#define TG_SMALL_MIN 20
+#endif
+constexpr int kSmallMin = TG_SMALL_MIN;
+constexpr uint32_t kSmallEntry = 0x80;  // flag in an entry's s_touch byte, next to the waves it touches
+__device__ __forceinline__ uint32_t small_entry(const RasterArgs &a, real extent) {
+    return extent * (real)a.H < (real)(2.0f * TG_SMALL_ROWS) ? kSmallEntry : 0u;  // NaN: not small
+}
+
+// bary_inside in two operations: a minimum passes NaNs by, as the three comparisons there do.
+__device__ __forceinline__ float min_number(float a, float b, float c) { return __builtin_fminf(__builtin_fminf(a, b), c); }
+__device__ __forceinline__ double min_number(double a, double b, double c) { return __builtin_fmin(__builtin_fmin(a, b), c); }
+__device__ __forceinline__ bool all_inside(real b0, real b1, real b2) { return !(min_number(b0, b1, b2) < kEffZero); }
+
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, true);
+}
+// A step of transpose_bits: two lanes (their words are `v` and `other`) swap the off-diagonal blocks.
+// keep: the bits a lane keeps; turn: how far the other lane's word is rotated to the right.
+__device__ __forceinline__ uint32_t exchange_blocks(uint32_t v, uint32_t other, uint32_t keep, uint32_t turn) {
+    return (v & keep) | (__builtin_amdgcn_alignbit(other, other, turn) & ~keep);
+}
+// All ones where bit `bit` of the lane is set: a mask of a step is then one literal and one operation, where a choice between
+// two literals is kept in registers by the loop around the call.
+__device__ __forceinline__ uint32_t lane_bit_mask(int lane, int bit) { return (uint32_t)__builtin_amdgcn_sbfe(lane, bit, 1); }
+// Transposes the 64 x 64 bit matrix whose row i is the word x of lane i: afterwards bit i of lane b's word is what bit b of
+// lane i's word was.  Six exchange steps between lanes 32, 16, ... 1 apart, each swapping the off-diagonal blocks of that
+// size: the first one is a single v_permlane32_swap, the others one lane move, one rotation and one bit selection per half
+// (lane moves in registers; the same steps by __shfl_xor are twelve LDS round trips).
+__device__ __forceinline__ uint64_t transpose_bits(uint64_t x, int lane) {
+    asm volatile("" : "+v"(lane));  // the masks are made here, not kept by the loop around the call
+    const auto halves = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)(x >> 32), false, false);
+    uint32_t a = halves[0], b = halves[1];
+    {
+        const auto rows_a = __builtin_amdgcn_permlane16_swap(a, a, false, false), rows_b = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+        const bool upper = lane & 16;
+        const uint32_t keep = 0x0000FFFFu ^ lane_bit_mask(lane, 4);
+        a = exchange_blocks(a, upper ? rows_a[0] : rows_a[1], keep, 16);
+        b = exchange_blocks(b, upper ? rows_b[0] : rows_b[1], keep, 16);
+    }
+    {
+        const uint32_t upper = lane_bit_mask(lane, 3), keep = 0x00FF00FFu ^ upper, turn = 24 ^ (upper & 16);  // 24 or 8
+        a = exchange_blocks(a, dpp_u32<0x128>(a), keep, turn);  // row_ror:8
+        b = exchange_blocks(b, dpp_u32<0x128>(b), keep, turn);
+    }
+    {
+        const uint32_t upper = lane_bit_mask(lane, 2), keep = 0x0F0F0F0Fu ^ upper, turn = 28 ^ (upper & 24);  // 28 or 4
+        a = exchange_blocks(a, dpp_u32<0x1B>(dpp_u32<0x141>(a)), keep, turn);  // mirrored inside eight lanes, then inside four
+        b = exchange_blocks(b, dpp_u32<0x1B>(dpp_u32<0x141>(b)), keep, turn);
+    }
+    {
+        const uint32_t upper = lane_bit_mask(lane, 1), keep = 0x33333333u ^ upper, turn = 30 ^ (upper & 28);  // 30 or 2
+        a = exchange_blocks(a, dpp_u32<0x4E>(a), keep, turn);
+        b = exchange_blocks(b, dpp_u32<0x4E>(b), keep, turn);
+    }
+    {
+        const uint32_t upper = lane_bit_mask(lane, 0), keep = 0x55555555u ^ upper, turn = 31 ^ (upper & 30);  // 31 or 1
+        a = exchange_blocks(a, dpp_u32<0xB1>(a), keep, turn);
+        b = exchange_blocks(b, dpp_u32<0xB1>(b), keep, turn);
+    }
+    return ((uint64_t)b << 32) | a;
+}
+
+__device__ __forceinline__ float lane_value(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane), hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double((long long)((hi << 32) | lo));
+}
+
+// Inside tests the other way round, for the 64 records at s_rec and a wave that owns a square of 8 x 8 pixels: lane = entry.
+// A lane (mine: its entry is to be tested) first finds the pixel rows its entry can reach, by the same monotone bound as
+// may_touch on a strip of one row, and then tests the eight pixels of those rows with the arithmetic of the test itself, so
+// the result is that of 64 tests per entry.  -> bit e: entry e covers the calling lane's pixel.
+// A test by broadcast costs about 20 vector instructions per entry for all 64 pixels and waits for its LDS reads (200
+// clocks where a long list leaves its tile alone on the CU); here 64 entries cost 250 instructions and 110 per row of the
+// tallest, all from registers.  500 000 triangles of a mesh, 500 x 500, tile order (longest list 5500 entries): 505 -> 378 us.
+template <typename Rec>
+__device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine, const WaveRect &rect, real px, real py) {
+    const int lane = threadIdx.x & (kWave - 1);
+    real m[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) m[k] = s_rec[lane].m[k];
+    uint32_t rows = 0;
+    {
+        real mx[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) mx[k] = m[3 * k] * (m[3 * k] >= 0.0f ? rect.x_hi : rect.x_lo);
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const real y = lane_value(py, 8 * r);
+            const bool reached = all_inside(mx[0] + m[1] * y + m[2], mx[1] + m[4] * y + m[5], mx[2] + m[7] * y + m[8]);
+            rows |= reached ? 1u << r : 0u;
+        }
+        if (!mine) rows = 0;
+    }
+    uint64_t covered = 0;  // of my entry: bit 8 * row + column
+    while (__builtin_amdgcn_ballot_w64(rows != 0)) {  // wave-uniform
+        const int r = rows ? __builtin_ctz(rows) : 0;
+        const real y = __shfl(py, 8 * r, kWave);
+        const real y0 = m[1] * y, y1 = m[4] * y, y2 = m[7] * y;
+        uint32_t bits = 0;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const real x = lane_value(px, c);
+            bits |= all_inside(m[0] * x + y0 + m[2], m[3] * x + y1 + m[5], m[6] * x + y2 + m[8]) ? 1u << c : 0u;
+        }
+        if (rows) covered |= (uint64_t)bits << (8 * r);
+        rows &= rows - 1;
+    }
+    return transpose_bits(covered, lane);
+}
+
 // Inside tests of one staged batch for the calling lane's pixel: bit e of the
-// result (word e / 64) is set when record e covers the pixel.  All lanes of the
-// wave read the same record at the same time (LDS broadcast); only records that
-// can touch the wave's pixels are looked at.  Rec must have a member m[9].
+// result (word e / 64) is set when record e covers the pixel.  Only records that
+// can touch the wave's pixels are looked at: all lanes of the wave read the same
+// record at the same time (LDS broadcast), or, where 20 or more of 64 entries are
+// small and the wave's pixels are a square, those are tested lane by lane.
+// Rec must have a member m[9].
 template <int kWords, typename Rec>
-__device__ __forceinline__ void batch_hit_mask(const Rec *s_rec, const uint8_t *s_touch, int nb, int wave, real px, real py,
-                                               uint64_t m[kWords]) {
+__device__ __forceinline__ void batch_hit_mask(const RasterArgs &a, const Rec *s_rec, const uint8_t *s_touch, const WaveRect *s_rects, int nb,
+                                               int wave, real px, real py, uint64_t m[kWords]) {
+    const bool square = ((a.tw | a.th) & 7) == 0;
 #pragma unroll
     for (int wd = 0; wd < kWords; wd++) {
-        const uint64_t todo = wave_candidates(s_touch, wd * kWave, nb, wave);
+        const int e = wd * kWave + (threadIdx.x & (kWave - 1));
+        const uint32_t touch = e < nb ? s_touch[e] : 0u;
+        const bool candidate = (touch >> wave) & 1u;
+        uint64_t todo = __builtin_amdgcn_ballot_w64(candidate);
+        uint64_t hits = 0;
+        const bool is_small = candidate && (touch & kSmallEntry);
+        const uint64_t small = __builtin_amdgcn_ballot_w64(is_small);
+        if (square && __builtin_popcountll(small) >= kSmallMin) {  // wave-uniform
+            hits = small_entry_hits(s_rec + wd * kWave, is_small, s_rects[wave], px, py);
+            todo &= ~small;
+        }
         // the lane's mask is built in 32-bit halves: a set bit then costs three vector operations, not six
-        uint32_t half[2] = {0u, 0u};
+        uint32_t half[2] = {(uint32_t)hits, (uint32_t)(hits >> 32)};
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             uint32_t left = (uint32_t)(todo >> (32 * h));
@@ -327,7 +526,7 @@ __device__ __forceinline__ void batch_hit_mask(const Rec *s_rec, const uint8_t *
                 left &= left - 1;
                 real b0, b1, b2;
                 bary_apply(s_rec[wd * kWave + 32 * h + bit].m, px, py, b0, b1, b2);
-                if (bary_inside(b0, b1, b2)) half[h] |= 1u << bit;
+                if (all_inside(b0, b1, b2)) half[h] |= 1u << bit;
             }
         }
         m[wd] = ((uint64_t)half[1] << 32) | half[0];
