@@ -86,7 +86,7 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
 #define TG_TILE_BAND_BACKWARD 1
 #endif
 #ifndef TG_XCD_CHUNK_FORWARD
-#define TG_XCD_CHUNK_FORWARD 0
+#define TG_XCD_CHUNK_FORWARD 32
 #endif
 constexpr int kXcds = 8;
 constexpr int kTileBandForward = TG_TILE_BAND_FORWARD, kTileBandBackward = TG_TILE_BAND_BACKWARD;
