@@ -264,6 +264,23 @@ def test_sort_tile_lists_matches_stable_sort(n, n_tiles, depth_pool, skew, cuda)
     np.testing.assert_array_equal(offsets.cpu().numpy(), np.searchsorted(keys[order] >> np.uint64(32), np.arange(n_tiles + 1)))
 
 
+@pytest.mark.parametrize("longest", [512, 513, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 10240, 10241, 16385])
+def test_sort_tile_lists_at_the_edges_of_its_rules(longest, cuda):
+    """One list of exactly `longest` pairs between lists of one pair fewer, one pair, and none."""
+    import torch
+    from trigrad_amd import _C
+    rng = np.random.default_rng(longest)
+    tile = np.repeat(np.arange(5, dtype=np.uint64), [longest - 1, 1, longest, 0, 3])
+    keys = (rng.permutation(tile) << np.uint64(32)) | rng.integers(0, 1 << 32, size=tile.size, dtype=np.uint64)
+    keys[::7] &= ~np.uint64(0xFFFFFF)  # equal depths now and then
+    order = np.argsort(keys, kind="stable")
+    sk, sv, status, offsets = _C.sort_tile_lists(torch.from_numpy(keys.view(np.int64).copy()).to(cuda),
+                                                 torch.arange(keys.size, dtype=torch.int32, device=cuda), 5)
+    assert int(status.item()) == 0
+    np.testing.assert_array_equal(u64(sk), keys[order])
+    np.testing.assert_array_equal(sv.cpu().numpy(), order.astype(np.int32))
+
+
 def test_sort_tile_lists_uniform_digits_and_empty(cuda):
     """Depth words that differ in one byte only (three of the four passes are left out), equal keys, no keys."""
     import torch

@@ -432,15 +432,22 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
 
 constexpr int kSegWaveItemsMax = 8;                                // segments up to 512 pairs: one wave each, no barriers
 constexpr int kSegWaveCap = kWave * kSegWaveItemsMax;
-constexpr int kSegLargeItems = 32;                                 // up to 8192 pairs in LDS (64 KB: two workgroups per CU)
-constexpr int kSegLargeCap = kSortThreads * kSegLargeItems;
+// Lists that are too long for one wave or four: one workgroup of 16 waves, up to 10240 pairs in LDS (99 KB, one workgroup per
+// CU).  A long list is mostly alone in its frame and its sort one chain of passes, so what counts is how many waves share
+// it.  With four waves and up to 8192 pairs (64 KB, two workgroups per CU), and now: one list of 8400 among short ones 120 ->
+// 38 us, some of up to 5500 47 -> 33, a thousand of 3700 108 -> 105 (there it is bound by the matching's instructions either
+// way), none at all 6.4 -> 6.1.  16 pairs per thread spill, and a kernel that has scratch memory takes 4 us more to launch.
+constexpr int kSegLargeThreads = 1024;
+constexpr int kSegLargeItems = 10;
+constexpr int kSegLargeCap = kSegLargeThreads * kSegLargeItems;
 constexpr int kSegStreamItems = 8;                                 // chunk of the pass through memory
-constexpr int kSegLargeGrid = 512;
+constexpr int kSegLargeGrid = 256;
 
+template <int THREADS>
 struct SegLds {
-    uint32_t count[kSortWaves][kRadix];
+    uint32_t count[THREADS / kWave][kRadix];
     uint32_t start[kRadix];
-    uint32_t wave_total[kSortWaves];
+    uint32_t wave_total[kRadix / kWave];
     uint32_t varying;
 };
 
@@ -450,36 +457,50 @@ __device__ __forceinline__ uint32_t wave_or_u32(uint32_t v) {
     return v;
 }
 
-// Ranks the workgroup's 256 * ITEMS digits (wave-striped order: wave, item, lane) and leaves in place[i]
+// Orders the LDS traffic of one wave: LDS serves a wave's instructions in order, so a lane sees what another
+// lane of its wave wrote by an earlier instruction; this keeps the compiler from moving accesses across.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Ranks the workgroup's THREADS * ITEMS digits (wave-striped order: wave, item, lane) and leaves in place[i]
 // the position of item i in digit order.  Barriers inside; the caller separates calls by one more.
-template <int ITEMS>
-__device__ __forceinline__ void workgroup_digit_places(const uint32_t (&digit)[ITEMS], SegLds &lds, uint32_t (&place)[ITEMS]) {
+template <int THREADS, int ITEMS>
+__device__ __forceinline__ void workgroup_digit_places(const uint32_t (&digit)[ITEMS], SegLds<THREADS> &lds, uint32_t (&place)[ITEMS]) {
+    static_assert(THREADS >= kRadix && THREADS % kWave == 0, "a thread for every digit");
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    for (int w = 0; w < kSortWaves; w++) lds.count[w][tid] = 0;
-    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kRadix / kWave; k++) lds.count[wave][k * kWave + lane] = 0;
+    wave_lds_sync();  // a wave's counters are its own
     wave_match_rank_ballots<kRadixBits, ITEMS>(digit, lds.count[wave], place);
     __syncthreads();
-    uint32_t run = 0;
+    uint32_t run = 0, incl = 0;
+    if (tid < kRadix) {  // whole waves
 #pragma unroll
-    for (int w = 0; w < kSortWaves; w++) {
-        const uint32_t c = lds.count[w][tid];
-        lds.count[w][tid] = run;
-        run += c;
+        for (int w = 0; w < THREADS / kWave; w++) {
+            const uint32_t c = lds.count[w][tid];
+            lds.count[w][tid] = run;
+            run += c;
+        }
+        incl = wave_inclusive_scan_u32(run);
+        if (lane == kWave - 1) lds.wave_total[wave] = incl;
     }
-    const uint32_t incl = wave_inclusive_scan_u32(run);
-    if (lane == kWave - 1) lds.wave_total[wave] = incl;
     __syncthreads();
-    uint32_t wave_prefix = 0;
-    for (int w = 0; w < wave; w++) wave_prefix += lds.wave_total[w];
-    lds.start[tid] = wave_prefix + incl - run;
+    if (tid < kRadix) {
+        uint32_t wave_prefix = 0;
+        for (int w = 0; w < wave; w++) wave_prefix += lds.wave_total[w];
+        lds.start[tid] = wave_prefix + incl - run;
+    }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < ITEMS; i++) place[i] += lds.start[digit[i]] + lds.count[wave][digit[i]];
 }
 
-// Sorts keys[start, start + n) / vals by the low key word, in place; n <= 256 * ITEMS.
-template <int ITEMS>
-__device__ __forceinline__ void segment_sort_in_lds(uint64_t *keys, uint32_t *vals, int64_t start, int n, SegLds &lds,
+// Sorts keys[start, start + n) / vals by the low key word, in place; n <= THREADS * ITEMS.
+template <int THREADS, int ITEMS>
+__device__ __forceinline__ void segment_sort_in_lds(uint64_t *keys, uint32_t *vals, int64_t start, int n, SegLds<THREADS> &lds,
                                                     uint32_t *ex_keys, uint32_t *ex_vals) {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     constexpr int kWaveSpan = kWave * ITEMS;
@@ -513,7 +534,7 @@ __device__ __forceinline__ void segment_sort_in_lds(uint64_t *keys, uint32_t *va
         uint32_t digit[ITEMS], place[ITEMS];
 #pragma unroll
         for (int i = 0; i < ITEMS; i++) digit[i] = (key[i] >> shift) & (kRadix - 1);
-        workgroup_digit_places<ITEMS>(digit, lds, place);
+        workgroup_digit_places<THREADS, ITEMS>(digit, lds, place);
 #pragma unroll
         for (int i = 0; i < ITEMS; i++) {
             ex_keys[place[i]] = key[i];
@@ -530,7 +551,7 @@ __device__ __forceinline__ void segment_sort_in_lds(uint64_t *keys, uint32_t *va
         __syncthreads();  // everything is read before the next pass writes the exchange buffer
     }
     const uint64_t high = first & 0xffffffff00000000ull;
-    for (int pos = tid; pos < n; pos += kSortThreads) {
+    for (int pos = tid; pos < n; pos += THREADS) {
         keys[start + pos] = high | ex_keys[pos];
         vals[start + pos] = ex_vals[pos];
     }
@@ -541,14 +562,6 @@ struct WaveSegLds {
     uint32_t count[kRadix];
     uint32_t ex_keys[kSegWaveCap], ex_vals[kSegWaveCap];
 };
-
-// Orders the LDS traffic of one wave: LDS serves a wave's instructions in order, so a lane sees what another
-// lane of its wave wrote by an earlier instruction; this keeps the compiler from moving accesses across.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The calling wave sorts keys[start, start + n) / vals by the low key word, in place; n <= 64 * ITEMS.
 template <int ITEMS>
@@ -622,12 +635,14 @@ __device__ __forceinline__ void segment_sort_in_wave(uint64_t *keys, uint32_t *v
 }
 
 // One workgroup per four segments.  A segment of up to kSegWaveCap pairs is sorted by one wave of its own;
-// then the workgroup takes those of up to kSegMediumCap pairs together, one after the other.  Longer ones are
-// left to segment_sort_large_kernel.
+// then the workgroup takes those of up to medium_cap pairs together, one after the other.  Longer ones are
+// left to segment_sort_large_kernel.  medium_cap is kSegMediumCap where no list can be longer (and that kernel is not
+// launched at all), else half of it: sixteen waves have a list of 2048 pairs sorted sooner than four, and its three
+// neighbours do not wait for it (1.3 million triangles of a mesh: both kernels together 111 -> 102 us, half a million: 88 -> 80).
 constexpr int kSegMediumItems = 8;
 constexpr int kSegMediumCap = kSortThreads * kSegMediumItems;  // 2048 pairs: as much LDS as the four waves' own buffers
 struct MediumSegLds {
-    SegLds lds;
+    SegLds<kSortThreads> lds;
     uint32_t ex_keys[kSegMediumCap], ex_vals[kSegMediumCap];
 };
 // Where the segments lie: either `offsets` holds their bounds (tile_ranges_kernel wrote them), or -- tile_count given --
@@ -637,7 +652,8 @@ struct MediumSegLds {
 __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64_t *keys, uint32_t *vals, int32_t *offsets,
                                                                           int n_segments, const uint32_t *__restrict__ tile_count,
                                                                           const uint32_t *__restrict__ row_totals, int tiles_x,
-                                                                          uint32_t n_pairs, FrameCount frame_count, uint32_t *status) {
+                                                                          uint32_t n_pairs, FrameCount frame_count, uint32_t *status,
+                                                                          int medium_cap) {
     n_pairs = (uint32_t)frame_count.pairs(n_pairs);
     // lists made from a scan whose wait expired are as invalid as those of a sort whose wait did
     if (frame_count.word && blockIdx.x == 0 && threadIdx.x == 0 && frame_count.word[1] == frame_count.epoch) *status = TG_STATUS_LOOKBACK_TIMEOUT;
@@ -682,7 +698,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
 #pragma unroll
     for (int w = 0; w < kSortWaves; w++) {
         const int len = bounds[w + 1] - bounds[w];
-        any_medium = any_medium || (len > kSegWaveCap && len <= kSegMediumCap);
+        any_medium = any_medium || (len > kSegWaveCap && len <= medium_cap);
         if (w == wave) { start = bounds[w]; n = len; }
     }
     if (n > 1 && n <= kSegWaveCap) {
@@ -701,12 +717,12 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
 #pragma unroll 1
     for (int w = 0; w < kSortWaves; w++) {
         const int len = bounds[w + 1] - bounds[w];
-        if (len <= kSegWaveCap || len > kSegMediumCap) continue;
+        if (len <= kSegWaveCap || len > medium_cap) continue;
         __syncthreads();  // the waves are done with their own buffers, the previous segment with the shared one
         if (len <= kSortThreads * 4)
-            segment_sort_in_lds<4>(keys, vals, bounds[w], len, s.medium.lds, s.medium.ex_keys, s.medium.ex_vals);
+            segment_sort_in_lds<kSortThreads, 4>(keys, vals, bounds[w], len, s.medium.lds, s.medium.ex_keys, s.medium.ex_vals);
         else
-            segment_sort_in_lds<kSegMediumItems>(keys, vals, bounds[w], len, s.medium.lds, s.medium.ex_keys, s.medium.ex_vals);
+            segment_sort_in_lds<kSortThreads, kSegMediumItems>(keys, vals, bounds[w], len, s.medium.lds, s.medium.ex_keys, s.medium.ex_vals);
     }
 }
 
@@ -714,29 +730,31 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
 // of the segment, then its chunks in order, every pair written to its final place of the pass in the other
 // buffer pair.  The sorted segment ends in (keys, vals).
 __device__ void segment_sort_through_memory(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt, uint32_t *vals_alt, int64_t start,
-                                            int n, SegLds &lds, uint32_t *hist /* [kRadix] */, uint32_t *next /* [kRadix] */) {
+                                            int n, SegLds<kSegLargeThreads> &lds, uint32_t *hist /* [kRadix] */, uint32_t *next /* [kRadix] */) {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    constexpr int kChunk = kSortThreads * kSegStreamItems;
+    constexpr int kChunk = kSegLargeThreads * kSegStreamItems;
     constexpr int kWaveSpan = kWave * kSegStreamItems;
     uint64_t *src_k = keys, *dst_k = keys_alt;
     uint32_t *src_v = vals, *dst_v = vals_alt;
 #pragma unroll 1
     for (int p = 0; p < 4; p++) {
         const int shift = p * kRadixBits;
-        hist[tid] = 0;
+        if (tid < kRadix) hist[tid] = 0;
         __syncthreads();
-        for (int i = tid; i < n; i += kSortThreads) atomicAdd(&hist[(uint32_t)(src_k[start + i] >> shift) & (kRadix - 1)], 1u);
+        for (int i = tid; i < n; i += kSegLargeThreads) atomicAdd(&hist[(uint32_t)(src_k[start + i] >> shift) & (kRadix - 1)], 1u);
         __syncthreads();
-        const uint32_t mine = hist[tid];
+        const uint32_t mine = tid < kRadix ? hist[tid] : 0u;
         const bool uniform = __syncthreads_or(mine == (uint32_t)n);
         if (uniform) continue;  // one digit holds the whole segment: the pass would change nothing
         {
             const uint32_t incl = wave_inclusive_scan_u32(mine);
-            if (lane == kWave - 1) lds.wave_total[wave] = incl;
+            if (lane == kWave - 1 && tid < kRadix) lds.wave_total[wave] = incl;
             __syncthreads();
             uint32_t wave_prefix = 0;
-            for (int w = 0; w < wave; w++) wave_prefix += lds.wave_total[w];
-            next[tid] = wave_prefix + incl - mine;
+            if (tid < kRadix) {
+                for (int w = 0; w < wave; w++) wave_prefix += lds.wave_total[w];
+                next[tid] = wave_prefix + incl - mine;
+            }
         }
         __syncthreads();
         for (int c0 = 0; c0 < n; c0 += kChunk) {
@@ -757,7 +775,7 @@ __device__ void segment_sort_through_memory(uint64_t *keys, uint32_t *vals, uint
                 }
             }
             n_pad = (c0 + kChunk > n) ? c0 + kChunk - n : 0;
-            workgroup_digit_places<kSegStreamItems>(digit, lds, place);
+            workgroup_digit_places<kSegLargeThreads, kSegStreamItems>(digit, lds, place);
             // place = position in the chunk's digit order; the pass position is the digit's running start plus
             // the rank among the chunk's pairs of that digit
 #pragma unroll
@@ -771,10 +789,11 @@ __device__ void segment_sort_through_memory(uint64_t *keys, uint32_t *vals, uint
             }
             __syncthreads();
             // the chunk's count of digit d = start[d + 1] - start[d]
-            const uint32_t end = (tid == kRadix - 1) ? (uint32_t)kChunk - (uint32_t)n_pad : lds.start[tid + 1];
-            const uint32_t begin = lds.start[tid];
-            __syncthreads();
-            next[tid] += (end > begin) ? end - begin : 0u;
+            if (tid < kRadix) {
+                const uint32_t end = (tid == kRadix - 1) ? (uint32_t)kChunk - (uint32_t)n_pad : lds.start[tid + 1];
+                const uint32_t begin = lds.start[tid];
+                next[tid] += (end > begin) ? end - begin : 0u;
+            }
             __syncthreads();
         }
         // the next pass reads what this one wrote
@@ -785,41 +804,51 @@ __device__ void segment_sort_through_memory(uint64_t *keys, uint32_t *vals, uint
         uint32_t *tv = src_v; src_v = dst_v; dst_v = tv;
     }
     if (src_k != keys) {
-        for (int i = tid; i < n; i += kSortThreads) {
+        for (int i = tid; i < n; i += kSegLargeThreads) {
             keys[start + i] = src_k[start + i];
             vals[start + i] = src_v[start + i];
         }
     }
 }
 
-// Segments longer than kSegMediumCap: few or none, so a workgroup looks through the lengths of its share of the
+// Segments longer than medium_cap: few or none, so a workgroup looks through the lengths of its share of the
 // segments, one segment per thread at a time, and takes the long ones in turn.
-__global__ __launch_bounds__(kSortThreads, 2) void segment_sort_large_kernel(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
+struct LargeSegLds {
+    SegLds<kSegLargeThreads> lds;
+    uint64_t votes[kSegLargeThreads / kWave];
+    uint32_t ex_keys[kSegLargeCap], ex_vals[kSegLargeCap];
+};
+__global__ __launch_bounds__(kSegLargeThreads) void segment_sort_large_kernel(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
                                                                              uint32_t *vals_alt, const int32_t *__restrict__ offsets,
-                                                                             int n_segments) {
-    __shared__ SegLds lds;
-    __shared__ uint32_t ex_keys[kSegLargeCap], ex_vals[kSegLargeCap];
-    __shared__ uint64_t s_votes[kSortWaves];
+                                                                             int n_segments, int medium_cap) {
+    extern __shared__ __align__(16) unsigned char s_large[];
+    LargeSegLds &s = *reinterpret_cast<LargeSegLds *>(s_large);
+    SegLds<kSegLargeThreads> &lds = s.lds;
+    uint32_t *const ex_keys = s.ex_keys, *const ex_vals = s.ex_vals;
     // workgroup b looks at the segments b, b + gridDim.x, ...: long segments that are neighbours go to different workgroups
     const int grid = (int)gridDim.x;
-    for (int base = 0; (int64_t)base * grid < n_segments; base += kSortThreads) {
+    for (int base = 0; (int64_t)base * grid < n_segments; base += kSegLargeThreads) {
         const int mine = (base + (int)threadIdx.x) * grid + (int)blockIdx.x;
-        const bool is_long = mine < n_segments && offsets[mine + 1] - offsets[mine] > kSegMediumCap;
+        const bool is_long = mine < n_segments && offsets[mine + 1] - offsets[mine] > medium_cap;
         const uint64_t vote = __builtin_amdgcn_ballot_w64(is_long);
         __syncthreads();  // the round before is done with the votes, the segment before with the LDS
-        if ((threadIdx.x & (kWave - 1)) == 0) s_votes[threadIdx.x / kWave] = vote;
+        if ((threadIdx.x & (kWave - 1)) == 0) s.votes[threadIdx.x / kWave] = vote;
         __syncthreads();
-        for (int w = 0; w < kSortWaves; w++) {
-            uint64_t todo = s_votes[w];
+        for (int w = 0; w < kSegLargeThreads / kWave; w++) {
+            uint64_t todo = s.votes[w];
             while (todo) {  // the same for the whole workgroup
                 const int seg = (base + w * kWave + __builtin_ctzll(todo)) * grid + (int)blockIdx.x;
                 todo &= todo - 1;
                 const int64_t start = offsets[seg];
                 const int n = offsets[seg + 1] - offsets[seg];
-                if (n <= kSortThreads * 16)
-                    segment_sort_in_lds<16>(keys, vals, start, n, lds, ex_keys, ex_vals);
+                if (n <= kSegLargeThreads * 2)
+                    segment_sort_in_lds<kSegLargeThreads, 2>(keys, vals, start, n, lds, ex_keys, ex_vals);
+                else if (n <= kSegLargeThreads * 4)
+                    segment_sort_in_lds<kSegLargeThreads, 4>(keys, vals, start, n, lds, ex_keys, ex_vals);
+                else if (n <= kSegLargeThreads * 8)
+                    segment_sort_in_lds<kSegLargeThreads, 8>(keys, vals, start, n, lds, ex_keys, ex_vals);
                 else if (n <= kSegLargeCap)
-                    segment_sort_in_lds<kSegLargeItems>(keys, vals, start, n, lds, ex_keys, ex_vals);
+                    segment_sort_in_lds<kSegLargeThreads, kSegLargeItems>(keys, vals, start, n, lds, ex_keys, ex_vals);
                 else
                     segment_sort_through_memory(keys, vals, keys_alt, vals_alt, start, n, lds, ex_keys, ex_keys + kRadix);
                 __syncthreads();  // the next segment reuses the LDS
@@ -911,12 +940,15 @@ static int ranges_and_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint
         TG_LAUNCH(tile_ranges_kernel, dim3((unsigned)ceil_div64(n + 1, kSortThreads)), dim3(kSortThreads), 0, s, k, n, n_tiles, offsets);
         if (int e = check_launch("tile_ranges_kernel")) return e;
     }
+    const int medium_cap = longest <= kSegMediumCap ? kSegMediumCap : kSegMediumCap / 2;
     TG_LAUNCH(segment_sort_small_kernel, dim3(ceil_div(n_tiles, kSortWaves)), dim3(kSortThreads), 0, s, k, v, offsets, n_tiles,
-              tile_count, row_totals, tiles_x, (uint32_t)n, frame_count, status);
+              tile_count, row_totals, tiles_x, (uint32_t)n, frame_count, status, medium_cap);
     if (int e = check_launch("segment_sort_small_kernel")) return e;
     if (longest <= kSegMediumCap) return 0;  // no list can be longer than what the kernel above sorts
-    TG_LAUNCH(segment_sort_large_kernel, dim3(n_tiles < kSegLargeGrid ? n_tiles : kSegLargeGrid), dim3(kSortThreads), 0, s, k, v,
-              k_other, v_other, offsets, n_tiles);
+    static size_t lds_reserved[kMaxDevices] = {0};
+    if (int e = reserve_lds("tg_sort_tile_lists", (const void *)segment_sort_large_kernel, sizeof(LargeSegLds), lds_reserved)) return e;
+    TG_LAUNCH(segment_sort_large_kernel, dim3(n_tiles < kSegLargeGrid ? n_tiles : kSegLargeGrid), dim3(kSegLargeThreads), sizeof(LargeSegLds),
+              s, k, v, k_other, v_other, offsets, n_tiles, medium_cap);
     return check_launch("segment_sort_large_kernel");
 }
 
