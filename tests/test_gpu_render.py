@@ -149,12 +149,37 @@ def _crowded_scene(n, width, height):
     (12000, 70, 45, 24, 16),   # six squares of 8 x 8 pixels, two workgroups
     (12000, 64, 64, 32, 32),
     (6000, 70, 45, 12, 6),     # a wave's pixels are no square
-    (40000, 400, 300, 16, 16),
+    (40000, 640, 400, 16, 16),  # more tiles than run at once: the longest lists' first
 ])
 def test_crowds_of_small_triangles_match_oracle(n, width, height, tw, th, mode, cuda, oracle):
     scene = _crowded_scene(n, width, height)
     _, want, got, _ = _forward_both(scene, tw, th, MODES[mode], cuda, oracle)
     _check_forward(f"crowd {n}/{tw}x{th}/{mode}", want, got, (th, tw))
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
+def test_more_long_tiles_than_slots(mode, cuda, monkeypatch):
+    """Some 400 tiles with long lists, of which 128 are started first: the frame is that of the stage-by-stage route, which
+    starts none first."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    n, width, height, tile = 500_000, 320, 240, 8
+    soup = S.random_soup(n, width, height, seed=8, sigma_px=0.6, opacity=(0.02, 0.3))
+    v = soup["vertices"].reshape(n, 3, 4).copy()
+    v[: n * 95 // 100, :, :2] = (v[: n * 95 // 100, :, :2] + 1.0) * 0.6 - 1.0
+    d = to_device(dict(soup, vertices=v.reshape(-1, 4)), cuda)
+    m = MODES[mode]
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, tile, tile, 1 / 256, True, m["per_pixel_sort"], ml)
+    for _ in range(3):  # the first frame's buffers are made for a guess of K, and what is long depends on them
+        got = _C.render_forward(*args)
+    lengths = got[4][1:] - got[4][:-1]
+    assert int((lengths >= max(1024, -(-2 * _C._round_capacity(got[3].numel()) // lengths.numel()))).sum()) > 128
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C.render_forward(*args)
+    for i in (0, 1, 2, 3, 4, 5, 6):
+        assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
 
 
 def _grad_inputs(scene, seed, with_depth):

@@ -28,7 +28,30 @@ struct ForwardOut {
     uint64_t *hit_masks; // tile order: which list entries cover which pixel, 64 entries per word (see hit_mask_chunk); may be null
     const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
     uint32_t *host_status;        // where the host looks for that word (memory of its own); may be null
+    LongTiles long_tiles;
+    int long_rows;                // rows of workgroups at the start of the grid, for the long tiles
 };
+
+// The tile a workgroup of a forward launch takes, and its list; false: none.  The first workgroups take the tiles with the
+// longest lists and the others, in the order of tile_of_workgroup, the rest.  Nothing here waits for a load before the next
+// one is asked for, apart from the long tiles' own: a frame without any loses 1 us by the workgroups that find none.
+__device__ __forceinline__ bool take_tile(const RasterArgs &a, const ForwardOut &o, TileId &t, int &start, int &end) {
+    if ((int)blockIdx.y < o.long_rows) {
+        const int slot = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+        if (slot >= kLongTileSlots || slot >= o.long_tiles.words[0]) return false;
+        t.index = o.long_tiles.words[1 + slot];
+        t.y = t.index / (int)gridDim.x;
+        t.x = t.index - t.y * (int)gridDim.x;
+        start = a.offsets[t.index];
+        end = a.offsets[t.index + 1];
+        return true;
+    }
+    t = tile_of_workgroup<kTileBandForward, kChunkForward>(o.long_rows);
+    start = a.offsets[t.index];
+    end = a.offsets[t.index + 1];
+    if (!o.long_rows || end - start < o.long_tiles.limit) return true;
+    return o.long_tiles.words[0] > kLongTileSlots && o.long_tiles.slot_of_tile[t.index] < 0;
+}
 
 // Lists whose sort gave up a wait are not to be read (unwritten entries may name anything): the frame's pixels
 // are marked instead, so that the caller sees it in the image itself.
@@ -39,7 +62,9 @@ __device__ __forceinline__ bool lists_invalid(const ForwardOut &o) {
         __hip_atomic_store(o.host_status, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return status != TG_STATUS_OK;
 }
-__device__ __forceinline__ void mark_pixel_invalid(const ForwardOut &o, const PixelCoord &p) {
+__device__ __forceinline__ void mark_tile_invalid(const RasterArgs &a, const ForwardOut &o) {
+    if ((int)blockIdx.y < o.long_rows) return;
+    const PixelCoord p = pixel_of_thread(a, tile_of_workgroup<kTileBandForward, kChunkForward>(o.long_rows));
     if (!p.valid) return;
     const real nan = std::numeric_limits<real>::quiet_NaN();
     o.image[p.index] = make_real4(nan, nan, nan, nan);
@@ -76,16 +101,18 @@ __global__ __launch_bounds__(kTileThreads, 8) void forward_tile_order_kernel(Ras
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandForward, kChunkForward>();
-    const int tile = tile_id.index;
-    const PixelCoord p = pixel_of_thread(a, tile_id);
+    TileId tile_id;
+    int start, end;
+    const bool mine = take_tile(a, out, tile_id, start, end);
     if (lists_invalid(out)) {  // the same for the whole launch
-        mark_pixel_invalid(out, p);
+        mark_tile_invalid(a, out);
         return;
     }
-    const int start = a.offsets[tile], end = a.offsets[tile + 1];
+    if (!mine) return;
+    const int tile = tile_id.index;
+    const PixelCoord p = pixel_of_thread(a, tile_id);
     publish_wave_rect(p, s_rects);
-    uint64_t *const masks = out.hit_masks ? out.hit_masks + hit_mask_head_words() : nullptr;
+    uint64_t *const masks = out.hit_masks ? out.hit_masks + hit_mask_head_words(out.long_rows) : nullptr;
 
     PixelState s;
     int last = 0;
@@ -355,12 +382,14 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 && kStage == kSelec
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ uint8_t s_touch[kStage];
     __shared__ WaveRect s_rects[kMaxTileWaves];
-    const TileId tile = tile_of_workgroup<kTileBandForward, kChunkForward>();
+    TileId tile;
+    int start, end;
+    const bool mine = take_tile(a, out, tile, start, end);
     if (lists_invalid(out)) {  // the same for the whole launch
-        mark_pixel_invalid(out, pixel_of_thread(a, tile));
+        mark_tile_invalid(a, out);
         return;
     }
-    if (sizeof(Pos) < sizeof(int) && a.offsets[tile.index + 1] - a.offsets[tile.index] > kShortList) return;
+    if (!mine || (sizeof(Pos) < sizeof(int) && end - start > kShortList)) return;
     pixel_order_tile<kStage, Pos, kInTurn>(a, out, tile.x, tile.y, gridDim.x, s_dyn, s_touch, s_rects);
 }
 
@@ -464,7 +493,7 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
                                  real *image, real *depthmap, real *final_weights, int32_t *ends, int32_t *last,
                                  real *last_depth, const OrderStore &order, uint64_t *hit_masks, const real *batch_bounds,
                                  const int32_t *far_start, const uint32_t *list_status, uint32_t *host_status, int64_t longest,
-                                 void *stream) {
+                                 const LongTiles &long_tiles, void *stream) {
     if (int e = check_raster_args("tg_render_forward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!vertices || !indices || !colors || !opacities || !offsets || !bary || !image || !depthmap || !final_weights || !ends) {
         set_error("tg_render_forward: null pointer");
@@ -482,9 +511,9 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
         return TG_E_ARG;
     }
     ForwardOut o{(real4 *)image, depthmap, final_weights, ends, last, last_depth, order, per_pixel_sort ? nullptr : hit_masks,
-                 list_status, host_status};
+                 list_status, host_status, long_tiles, long_tiles.words ? ceil_div(kLongTileSlots, ceil_div(width, tile_w)) : 0};
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
-    const dim3 grid = tl.grid;
+    const dim3 grid(tl.grid.x, tl.grid.y + o.long_rows, tl.grid.z);
     const int n_threads = tl.threads;
     hipStream_t s = (hipStream_t)stream;
     if (!per_pixel_sort) {
@@ -515,9 +544,9 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     if (int e = check_launch("forward_pixel_order_kernel")) return e;
     if (longest <= kShortList) return 0;  // no list is too long for 16-bit positions
     if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;
-    const int tiles = (int)(grid.x * grid.y);
+    const int tiles = (int)(tl.grid.x * tl.grid.y);
     TG_LAUNCH(forward_pixel_order_long_lists_kernel, dim3(min(tiles, kLongListGroups), 1, grid.z), dim3(n_threads), lds, s, a, o,
-              (int)grid.x, (int)grid.y);
+              (int)tl.grid.x, (int)tl.grid.y);
     return check_launch("forward_pixel_order_long_lists_kernel");
 }
 
@@ -534,7 +563,7 @@ extern "C" int tg_render_forward(const real *vertices, const int32_t *indices, c
     const OrderStore order{fragments, (int64_t)max_layers * width * height, 0};
     return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
                           early_stopping_threshold, per_pixel_sort, max_layers, image, depthmap, final_weights, ends, last, last_depth,
-                          order, hit_masks, batch_bounds, far_start, list_status, nullptr, std::numeric_limits<int64_t>::max(), stream);
+                          order, hit_masks, batch_bounds, far_start, list_status, nullptr, std::numeric_limits<int64_t>::max(), LongTiles(), stream);
 }
 
 extern "C" int64_t tg_order_pool_words(int64_t n_keys, int64_t n_triangles, int tile_w, int tile_h) {
@@ -557,5 +586,5 @@ extern "C" int tg_render_forward_pooled(const real *vertices, const int32_t *ind
     const OrderStore order{order_pool, n_triangles > kShortList ? n_keys * pixels : 0, pixels};
     return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
                           early_stopping_threshold, 1, max_layers, image, depthmap, final_weights, ends, last, last_depth, order, nullptr,
-                          batch_bounds, far_start, list_status, nullptr, n_keys, stream);
+                          batch_bounds, far_start, list_status, nullptr, n_keys, LongTiles(), stream);
 }

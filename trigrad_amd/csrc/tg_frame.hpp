@@ -17,6 +17,17 @@ struct FrameCount {
     }
 };
 
+// The tiles with the longest lists, for a kernel that starts with them: a tile's list is one workgroup's serial work, and a
+// list of thousands of entries that is started late is what the whole launch waits for.  The segment sort, which makes
+// the lists' bounds, gives every tile with `limit` entries or more a slot while there are any.  words: how many have
+// one or asked for one, then their tiles; slot_of_tile: every tile's slot, negative for none.  Null words: no such list.
+constexpr int kLongTileSlots = 128;
+struct LongTiles {
+    int32_t *words = nullptr;
+    int32_t *slot_of_tile = nullptr;
+    int limit = 0;
+};
+
 // tg_bin_frame with two outputs more: the bary matrices, and K for the host (may be null).
 int bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indices, int32_t n_triangles, int width, int height, int tile_w,
               int tile_h, uint64_t *keys, uint32_t *values, int64_t key_capacity, uint32_t *total_and_status, void *frame,
@@ -24,13 +35,14 @@ int bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indices, 
               void *stream);
 int build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, const uint32_t *total_and_status, int64_t longest, int tiles_x,
                       int tiles_y, uint64_t *keys, uint32_t *values, uint64_t *keys_alt, uint32_t *values_alt, int32_t *offsets,
-                      void *workspace, size_t workspace_bytes, uint32_t *status, int *result_in_alt, void *stream);
+                      void *workspace, size_t workspace_bytes, uint32_t *status, int *result_in_alt, const LongTiles &long_tiles,
+                      void *stream);
 // host_status: receives the list kernels' status word, in memory the host reads; longest: no list holds more entries.
 int render_forward(const real *vertices, const int32_t *indices, const real *colors, const real *opacities, const int32_t *sorted_ids,
                    const int32_t *offsets, const real *bary, int width, int height, int tile_w, int tile_h, real early_stopping_threshold,
                    int per_pixel_sort, int max_layers, real *image, real *depthmap, real *final_weights, int32_t *ends, int32_t *last,
                    real *last_depth, const OrderStore &order, uint64_t *hit_masks, const real *batch_bounds, const int32_t *far_start,
-                   const uint32_t *list_status, uint32_t *host_status, int64_t longest, void *stream);
+                   const uint32_t *list_status, uint32_t *host_status, int64_t longest, const LongTiles &long_tiles, void *stream);
 int render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices, const int32_t *indices, const real *colors,
                     const real *opacities, const int32_t *sorted_ids, const int32_t *offsets, const real *bary, const real *image,
                     const real *depthmap, const real *final_weights, const int32_t *ends, const int32_t *last, const real *last_depth,

@@ -93,9 +93,9 @@ constexpr int kTileBandForward = TG_TILE_BAND_FORWARD, kTileBandBackward = TG_TI
 constexpr int kChunkForward = TG_XCD_CHUNK_FORWARD, kChunkBackward = 0;  // 0: an eighth of the tiles
 struct TileId { int x, y, index; };
 template <int kTileBand, int kChunk>
-__device__ __forceinline__ TileId tile_of_workgroup() {
-    const int tiles_x = (int)gridDim.x, tiles_y = (int)gridDim.y, n = tiles_x * tiles_y;
-    const int linear = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+__device__ __forceinline__ TileId tile_of_workgroup(int skipped_rows = 0) {  // rows of workgroups in front that are not for tiles
+    const int tiles_x = (int)gridDim.x, tiles_y = (int)gridDim.y - skipped_rows, n = tiles_x * tiles_y;
+    const int linear = (int)((blockIdx.y - skipped_rows) * gridDim.x + blockIdx.x);
     TileId t;
 #if TG_XCD_TILES
     const int xcd = linear % kXcds, turn = linear / kXcds;
@@ -239,7 +239,7 @@ __device__ __forceinline__ int64_t hit_mask_chunk(int start, int tile, int relat
     return (int64_t)(start >> 6) + tile + (relative_position >> 6);
 }
 __device__ __forceinline__ int64_t hit_mask_head_index(int tile) { return (int64_t)tile * gridDim.z + blockIdx.z; }
-__device__ __forceinline__ int64_t hit_mask_head_words() { return (int64_t)gridDim.x * gridDim.y * gridDim.z; }
+__device__ __forceinline__ int64_t hit_mask_head_words(int skipped_rows = 0) { return (int64_t)gridDim.x * (gridDim.y - skipped_rows) * gridDim.z; }
 
 // Where the saved blend order of a pixel lies: layer l of the pixel at low[l * stride], and, in tiles whose list holds more
 // than kShortList entries, the high half of its list position at high[l * stride].  Two layouts:

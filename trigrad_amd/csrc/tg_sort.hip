@@ -653,7 +653,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
                                                                           int n_segments, const uint32_t *__restrict__ tile_count,
                                                                           const uint32_t *__restrict__ row_totals, int tiles_x,
                                                                           uint32_t n_pairs, FrameCount frame_count, uint32_t *status,
-                                                                          int medium_cap) {
+                                                                          int medium_cap, LongTiles long_tiles) {
     n_pairs = (uint32_t)frame_count.pairs(n_pairs);
     // lists made from a scan whose wait expired are as invalid as those of a sort whose wait did
     if (frame_count.word && blockIdx.x == 0 && threadIdx.x == 0 && frame_count.word[1] == frame_count.epoch) *status = TG_STATUS_LOOKBACK_TIMEOUT;
@@ -683,6 +683,14 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
                 const int end = (int)(length < n_pairs - sum ? sum + length : n_pairs);
                 if (wave == kSortWaves - 1 || t == n_segments - 1) s_bounds[wave + 1] = end;
                 if (t == n_segments - 1) offsets[n_segments] = end;
+                if (long_tiles.words) {
+                    int slot = -1;
+                    if (end - (int)sum >= long_tiles.limit) {
+                        slot = atomicAdd(long_tiles.words, 1);
+                        if (slot < kLongTileSlots) long_tiles.words[1 + slot] = t; else slot = -1;
+                    }
+                    long_tiles.slot_of_tile[t] = slot;
+                }
             }
         }
         __syncthreads();
@@ -935,14 +943,15 @@ static int run_passes(const char *fn, const PassPlan &plan, const SortLayout &L,
 static int ranges_and_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint32_t *v_other, int64_t n, int n_tiles,
                                int32_t *offsets, hipStream_t s, const uint32_t *tile_count = nullptr,
                                const uint32_t *row_totals = nullptr, int tiles_x = 0, FrameCount frame_count = FrameCount(),
-                               uint32_t *status = nullptr, int64_t longest = std::numeric_limits<int64_t>::max()) {
+                               uint32_t *status = nullptr, int64_t longest = std::numeric_limits<int64_t>::max(),
+                               const LongTiles &long_tiles = LongTiles()) {
     if (!tile_count) {
         TG_LAUNCH(tile_ranges_kernel, dim3((unsigned)ceil_div64(n + 1, kSortThreads)), dim3(kSortThreads), 0, s, k, n, n_tiles, offsets);
         if (int e = check_launch("tile_ranges_kernel")) return e;
     }
     const int medium_cap = longest <= kSegMediumCap ? kSegMediumCap : kSegMediumCap / 2;
     TG_LAUNCH(segment_sort_small_kernel, dim3(ceil_div(n_tiles, kSortWaves)), dim3(kSortThreads), 0, s, k, v, offsets, n_tiles,
-              tile_count, row_totals, tiles_x, (uint32_t)n, frame_count, status, medium_cap);
+              tile_count, row_totals, tiles_x, (uint32_t)n, frame_count, status, medium_cap, long_tiles);
     if (int e = check_launch("segment_sort_small_kernel")) return e;
     if (longest <= kSegMediumCap) return 0;  // no list can be longer than what the kernel above sorts
     static size_t lds_reserved[kMaxDevices] = {0};
@@ -1155,7 +1164,8 @@ bool tg::frame_grid_fits(int tiles_x, int tiles_y) { return grid_plan(tiles_x, t
 // more keys than that gets empty lists, and no list holds more than `longest` keys.
 int tg::build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, const uint32_t *total_and_status, int64_t longest, int tiles_x,
                           int tiles_y, uint64_t *keys, uint32_t *values, uint64_t *keys_alt, uint32_t *values_alt, int32_t *offsets,
-                          void *workspace, size_t workspace_bytes, uint32_t *status, int *result_in_alt, void *stream) {
+                          void *workspace, size_t workspace_bytes, uint32_t *status, int *result_in_alt, const LongTiles &long_tiles,
+                          void *stream) {
     if (n_keys < 0 || n_keys > kSortMaxN || tiles_x <= 0 || tiles_y <= 0 || (int64_t)tiles_x * tiles_y > 0x7fffffff || !frame ||
         !result_in_alt || !offsets) {
         set_error("tg_build_frame_lists: n_keys must be in [0, 2^30), tile counts positive, frame state, offsets and result_in_alt given");
@@ -1198,12 +1208,12 @@ int tg::build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, const uin
         return e;
     // two passes: the sorted pairs are back in (keys, values)
     return ranges_and_segments(keys, values, keys_alt, values_alt, n_keys, n_tiles, offsets, s, tile_count, totals + kRadix, tiles_x,
-                               count, status, longest);
+                               count, status, longest, long_tiles);
 }
 
 extern "C" int tg_build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, int tiles_x, int tiles_y, uint64_t *keys,
                                     uint32_t *values, uint64_t *keys_alt, uint32_t *values_alt, int32_t *offsets, void *workspace,
                                     size_t workspace_bytes, uint32_t *status, int *result_in_alt, void *stream) {
     return build_frame_lists(frame, epoch, n_keys, nullptr, n_keys, tiles_x, tiles_y, keys, values, keys_alt, values_alt, offsets,
-                             workspace, workspace_bytes, status, result_in_alt, stream);
+                             workspace, workspace_bytes, status, result_in_alt, LongTiles(), stream);
 }
