@@ -278,6 +278,24 @@ def test_render_autograd_end_to_end(cuda, oracle):
             assert_gradients_close(label, g.cpu().numpy(), w, mag)
 
 
+def test_forward_mode_is_refused_for_known_frames_too(cuda):
+    """The first frame of a kind goes through the Python function, later ones do not: a tangent is refused either way."""
+    import scenes as S
+    import torch
+    import trigrad_amd
+    from torch.autograd import forward_ad
+    d = to_device(S.random_soup(40, 48, 48, seed=2), cuda)
+    args = (d["indices"], d["colors"], d["opacities"], 48, 48)
+    for _ in range(3):
+        trigrad_amd.render(d["vertices"], *args)
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(d["vertices"], torch.ones_like(d["vertices"]))
+        with pytest.raises(RuntimeError):
+            trigrad_amd.render(dual, *args)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda v: trigrad_amd.render(v, *args)[0])(d["vertices"][None])
+
+
 def test_loss_on_depth_only(cuda, oracle):
     """Only the depth map takes part in the loss: the image's gradient arrives as None."""
     import torch

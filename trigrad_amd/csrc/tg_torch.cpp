@@ -13,9 +13,11 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/zeros_like.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include <array>
@@ -240,6 +242,10 @@ PyObject *py_render(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const at::Tensor &vertices = THPVariable_Unpack(args[0]), &indices = THPVariable_Unpack(args[1]),
                      &colors = THPVariable_Unpack(args[2]), &opacities = THPVariable_Unpack(args[3]);
     if (!vertices.is_cuda() || vertices.dim() != 2 || indices.dim() != 2) Py_RETURN_NONE;
+    // tracing, functorch transforms, dispatch modes, fake tensors and forward-mode tangents: the Python function records or refuses them
+    if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer)) Py_RETURN_NONE;
+    for (const at::Tensor *t : {&vertices, &indices, &colors, &opacities})
+        if (at::isTensorSubclassLike(*t) || t->_fw_grad(0).defined()) Py_RETURN_NONE;
     const int64_t n_vertices = vertices.size(0), n_triangles = indices.size(0);
     if (n_triangles < 1 || !fits(vertices, vertices, at::kFloat, n_vertices, 4) || !fits(indices, vertices, at::kInt, n_triangles, 3) ||
         !fits(colors, vertices, at::kFloat, n_vertices, 3) || !fits(opacities, vertices, at::kFloat, n_vertices, 0))
