@@ -232,11 +232,13 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
         const bool ahead = !kInTurn && !a.batch_bounds && (int)blockDim.x >= kStage;
         DepthParts next;
         if constexpr (kInTurn) {
-            const int j = min(start + tid, end - 1);
-            next.fetch_triangle(a, j);
-            next.fetch_matrix(a);
-            next.fetch_triangle(a, min(j + kTileThreads, end - 1));
-            next.fetch_vertices(a);
+            if (start < end) {  // an empty list has no last entry to clamp to
+                const int j = min(start + tid, end - 1);
+                next.fetch_triangle(a, j);
+                next.fetch_matrix(a);
+                next.fetch_triangle(a, min(j + kTileThreads, end - 1));
+                next.fetch_vertices(a);
+            }
         } else if (ahead && tid < min(kStage, end - start)) {
             next.fetch_triangle(a, start + tid);
             next.fetch_matrix(a);
