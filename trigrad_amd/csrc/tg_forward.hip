@@ -216,38 +216,40 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     PixelState s;
     real last_depth = -__builtin_inff();  // render.cu:585-586
     int last_j = -1;  // list positions count from the tile's start
-    bool active = p.valid;
+    bool active = p.valid && start < end;  // below, a list has a last entry
     while (true) {
         const bool want = active && s.alpha > a.thr && s.blended < a.max_layers;  // render.cu:588
         if (!__syncthreads_or(want)) break;
         const int cap = want ? min(kLayers, a.max_layers - s.blended) : 0;
         int found = 0;
-        // Without depth bounds (which make the batches jump) the records of coming batches are fetched into registers while
-        // this batch is worked on.  A wave that asks for an entry's vertices has to have its vertex numbers, and for those its
-        // triangle number: three memory latencies in a row, and whoever asks waits for the first two.  So the four waves
-        // of a tile take the batches of 64 in turn (kInTurn), and a wave's links are asked for two batches apart (its own
-        // turn comes every fourth batch); each has arrived when the next one needs it.  A frame with a list of 8400
-        // entries in one tile: 241 -> 154 us; lists of 268 everywhere: 680 -> 669.
-        const int lane = tid & (kWave - 1);
+        // The records of coming batches are fetched into registers while this batch is worked on.  A wave that asks for an
+        // entry's vertices has to have its vertex numbers, and for those its triangle number: three memory latencies in a
+        // row, and whoever asks waits for the first two.  So the four waves of a tile take the batches in turn (kInTurn;
+        // batches of 128 two waves each), and a wave's links are asked for half a turn apart; each has arrived when the next
+        // one needs it.  A frame with a list of 8400 entries in one tile: 241 -> 154 us; lists of 268 everywhere: 680 -> 669.
+        // Where depth bounds make the batches jump the turns start again (200 000 faint triangles, lists of 3700: 306 -> 292).
+        constexpr int kTurns = kTileThreads / kStage;
+        const int group = kStage == kWave ? wave : tid / kStage, mine = tid & (kStage - 1);  // in turn: whose batch, which of its entries
         const bool ahead = !kInTurn && !a.batch_bounds && (int)blockDim.x >= kStage;
         DepthParts next;
+        auto start_turns = [&](int first) {  // the records of the kTurns batches from list entry `first` on
+            const int j = min(first + tid, end - 1);
+            next.fetch_triangle(a, j);
+            next.fetch_matrix(a);
+            next.fetch_triangle(a, min(j + kTileThreads, end - 1));
+            next.fetch_vertices(a);
+        };
         if constexpr (kInTurn) {
-            if (start < end) {  // an empty list has no last entry to clamp to
-                const int j = min(start + tid, end - 1);
-                next.fetch_triangle(a, j);
-                next.fetch_matrix(a);
-                next.fetch_triangle(a, min(j + kTileThreads, end - 1));
-                next.fetch_vertices(a);
-            }
+            start_turns(start);
         } else if (ahead && tid < min(kStage, end - start)) {
             next.fetch_triangle(a, start + tid);
             next.fetch_matrix(a);
             next.fetch_vertices(a);
         }
         int turn = 0;
-        for (int batch = start; batch < end; batch += kStage, turn = (turn + 1) & 3) {
+        for (int batch = start; batch < end; batch += kStage, turn = (turn + 1) & (kTurns - 1)) {
             const int nb = min(kStage, end - batch);
-            if (!kInTurn && a.batch_bounds) {
+            if (kStage != kWave && a.batch_bounds) {  // batches of 64 go without
                 // a lane needs nothing from here on when its list is full and its worst candidate is nearer than
                 // every fragment the rest of the tile's list can produce (a full list rejects depths >= its worst)
                 const real rest = a.batch_bounds[batch_bound_index(start, tile, batch - start)];
@@ -256,14 +258,18 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                     // on to the batch that holds the first entry the bounds do not cover
                     const int resume = start + a.far_start[tile] / kStage * kStage;
                     if (resume > batch) {
+                        if (kInTurn) {
+                            start_turns(resume);
+                            turn = kTurns - 1;
+                        }
                         batch = resume - kStage;
                         continue;
                     }
                 }
             }
             __syncthreads();
-            if (kInTurn ? wave == turn && lane < nb : ahead && tid < nb) {
-                const int e = kInTurn ? lane : tid;
+            if (kInTurn ? group == turn && mine < nb : ahead && tid < nb) {
+                const int e = kInTurn ? mine : tid;
                 const DepthRecord r = next.record();
                 s_rec[e] = r;
                 s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves) | small_entry(a, r.extent));
@@ -276,12 +282,12 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
             }
             __syncthreads();
             if constexpr (kInTurn) {
-                if (wave == turn) {
+                if (group == turn) {
                     // my next batch: its triangle numbers are here; ask for vertex numbers and matrices, and for the triangle
                     // numbers of the batch after it (past the list's end: its last entry again, which nobody looks at)
                     next.fetch_matrix(a);
-                    next.fetch_triangle(a, min(batch + 8 * kWave + lane, end - 1));
-                } else if (wave == (turn ^ 2)) {
+                    next.fetch_triangle(a, min(batch + 2 * kTileThreads + mine, end - 1));
+                } else if (group == (turn ^ (kTurns / 2))) {
                     next.fetch_vertices(a);
                 }
             } else if (ahead && batch + kStage < end && tid < min(kStage, end - batch - kStage)) {
@@ -378,7 +384,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
 
 // One workgroup per tile.  With 16-bit positions the tiles whose lists are too long for them are left to
 // forward_pixel_order_long_lists_kernel.
-// kInTurn: kStage is 64 and the workgroup has four waves.
+// kInTurn: the workgroup has four waves.
 template <int kStage, typename Pos, bool kInTurn>
 __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 && kStage == kSelectBatchShort ? 3 : 2) void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
@@ -525,15 +531,20 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     const size_t lds = pixel_order_lds_bytes(n_threads, kSelectBatch);
     // Depth bounds make the batches jump in steps of kSelectBatch, so they go with the int positions.
     const bool split = !a.batch_bounds && n_threads >= kSelectBatchShort;
-    static size_t lds_reserved[kMaxDevices] = {0}, lds_reserved_long[kMaxDevices] = {0};
+    static size_t lds_reserved[2][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
+    const bool in_turn = n_threads == kTileThreads;
     if (!split) {
-        if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_kernel<kSelectBatch, int, false>, lds, lds_reserved)) return e;
-        TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatch, int, false>), grid, dim3(n_threads), lds, s, a, o);
+        const void *kernel = in_turn ? (const void *)forward_pixel_order_kernel<kSelectBatch, int, true>
+                                     : (const void *)forward_pixel_order_kernel<kSelectBatch, int, false>;
+        if (int e = reserve_lds("tg_render_forward", kernel, lds, lds_reserved[in_turn])) return e;
+        if (in_turn)
+            TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatch, int, true>), grid, dim3(n_threads), lds, s, a, o);
+        else
+            TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatch, int, false>), grid, dim3(n_threads), lds, s, a, o);
         return check_launch("forward_pixel_order_kernel");
     }
     const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t));
     static size_t lds_reserved_short[2][kMaxDevices] = {{0}};
-    const bool in_turn = n_threads == kTileThreads;
     const void *kernel = in_turn ? (const void *)forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true>
                                  : (const void *)forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false>;
     if (int e = reserve_lds("tg_render_forward", kernel, lds_short, lds_reserved_short[in_turn])) return e;
