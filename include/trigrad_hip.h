@@ -173,7 +173,7 @@ int tg_tile_ranges(const uint64_t *sorted_keys, int64_t n_keys, int n_tiles, int
  * through memory for the tile bits only (LSD passes of at most 8 bits with
  * decoupled look-back); the stable passes over the 32 depth bits then run per
  * tile inside one workgroup, pairs in registers and LDS (a tile list longer
- * than 8192 entries is sorted by its workgroup through memory instead).
+ * than 10240 entries is sorted by its workgroup through memory instead).
  * *result_in_alt (host): 0 = sorted data in (keys, values), 1 = in the _alt
  * pair.  offsets: n_tiles + 1 entries. */
 size_t tg_tile_list_sort_workspace_bytes(int64_t n, int n_tiles);

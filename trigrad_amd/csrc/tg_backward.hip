@@ -13,9 +13,9 @@
 // per_pixel_sort = 0 (backward_tile_order_kernel): all pixels of a tile share
 //   the list order, so the tile's list is walked backwards in LDS-staged
 //   batches of 64 entries.
-// per_pixel_sort = 1, max_layers <= 32 (backward_saved_order_kernel): every
+// per_pixel_sort = 1 (backward_saved_order_kernel): every
 //   pixel walks the blend order the forward pass saved for it, backwards.
-// per_pixel_sort = 1, max_layers > 32 (backward_pixel_order_kernel): the pixel
+// per_pixel_sort = 1, no saved order (backward_pixel_order_kernel): the pixel
 //   re-selects its fragments from the far end (32 at a time, below the (depth,
 //   position) of the last blended fragment saved by the forward pass).
 #include "tg_frame.hpp"
