@@ -328,12 +328,13 @@ int tg_render_forward(const tg_real *vertices, const int32_t *indices, const tg_
                       tg_real *last_depth, uint16_t *fragments, uint64_t *hit_masks,
                       const tg_real *batch_bounds, const int32_t *far_start, const uint32_t *list_status, void *stream);
 
-/* Per-pixel order with the blend order saved whatever max_layers is: a pixel blends an entry of its tile's list at
- * most once, so a tile with a list of n entries is given n rows of `order_pool`, a row holding one uint16 list position
- * per pixel of a tile (rounded up to whole waves).  tg_order_pool_words: the uint16 words of the pool (with more than
- * 65535 triangles lists can be longer than 16 bits count, and the positions' high halves take as many words again).
- * The pool is private to tg_render_forward_pooled and tg_render_backward_pooled; words of layers that are not blended
- * are never touched. */
+/* Per-pixel order with the blend order saved whatever max_layers is: where its depths are numbers a pixel blends an entry
+ * of its tile's list at most once, so a tile with a list of n entries is given n rows of `order_pool`, a row holding one
+ * uint16 list position per pixel of a tile (rounded up to whole waves).  tg_order_pool_words: the uint16 words of the pool
+ * (with more than 65535 triangles lists can be longer than 16 bits count, and the positions' high halves take as many
+ * words again).  The pool is private to tg_render_forward_pooled and tg_render_backward_pooled; words of layers that are
+ * not blended are never touched.  A NaN depth can have a pixel's list blended more than once: the layers beyond its rows
+ * count in the image but are not stored, and the backward pass walks the stored ones. */
 int64_t tg_order_pool_words(int64_t n_keys, int64_t n_triangles, int tile_w, int tile_h);
 int tg_render_forward_pooled(const tg_real *vertices, const int32_t *indices, int32_t n_triangles, const tg_real *colors,
                              const tg_real *opacities, const int32_t *sorted_ids, const int32_t *offsets, int64_t n_keys,

@@ -724,3 +724,72 @@ def test_frame_in_one_call_is_the_frame_stage_by_stage(n_triangles, size, tile, 
         for a, b in zip(one[2:], want[2:]):
             # sums of float32 terms in another order: two rounding steps of the largest sum
             assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()) + 1e-6
+
+
+def _stacks_with_a_nan_depth(with_nan):
+    """Three 16 x 16 tiles with a stack of 40 half-tile triangles each, all of one shape (a pixel is covered by
+    a whole stack or by none of it); the last one of the middle stack has a NaN depth."""
+    W, H, n = 48, 16, 40
+    vertices, tile_of = [], []
+    for tile in range(3):
+        for k in range(n - (tile == 1 and not with_nan)):
+            x = 16 * tile + np.array([1.0, 15.0, 1.0])
+            y = np.array([1.0, 1.0, 15.0])
+            z = np.full(3, np.nan if tile == 1 and k == n - 1 else 0.1 + 0.2 * k)
+            vertices.append(np.stack([2 * x / W - 1, 2 * y / H - 1, z, np.full(3, 1 / (0.1 + 0.2 * k))], axis=-1))
+            tile_of.append(tile)
+    m = len(vertices)
+    v = np.concatenate(vertices).astype(np.float32)
+    colors = np.random.default_rng(18).uniform(0, 1, (3 * 3 * n, 3)).astype(np.float32)
+    opacities = np.full(3 * 3 * n, 0.004, np.float32)
+    keep = np.arange(3 * 3 * n).reshape(-1, 3)
+    if not with_nan:
+        keep = np.delete(keep, 2 * n - 1, axis=0)
+    scene = dict(vertices=v, indices=np.arange(3 * m, dtype=np.int32).reshape(m, 3), colors=colors[keep.ravel()],
+                 opacities=opacities[keep.ravel()], width=W, height=H)
+    return scene, np.repeat(tile_of, 3)
+
+
+@pytest.mark.parametrize("max_layers", [41, 500])
+@pytest.mark.parametrize("one_call", [True, False])
+def test_nan_depth_stays_inside_its_rows_of_the_order_pool(one_call, max_layers, cuda, oracle, monkeypatch):
+    """A NaN depth has a pixel's list blended again and again: the image is the oracle's, but the order pool has one row per
+    list entry.  Nothing is written behind the pool, and the gradients of the other tiles' triangles are those of the same
+    frame without the NaN triangle."""
+    import torch
+    import trigrad_amd
+    from trigrad_amd import _C
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", one_call)
+    behind = []
+
+    def pool_and_sentinels(n_keys, n_triangles, tile_width, tile_height, device):
+        words = int(trigrad_amd._lib.load(32).tg_order_pool_words(n_keys, n_triangles, tile_width, tile_height))
+        rows = torch.full((words + (max_layers + 1) * tile_width * tile_height,), 0x5a5a, dtype=torch.int16, device=device)
+        behind.append(rows[words:])
+        return rows[:words]
+
+    monkeypatch.setattr(_C, "_order_pool", pool_and_sentinels)
+    mode = dict(per_pixel_sort=True, max_layers=max_layers)
+    scene, tile_of = _stacks_with_a_nan_depth(True)
+    _, want, got, _ = _forward_both(scene, 16, 16, mode, cuda, oracle, thr=0.0)
+    assert np.diff(want["offsets"]).tolist() == [40, 40, 40] and want["ends"].max() == max_layers > 40
+    _check_forward("NaN depth", want, got, (16, 16))
+    for sentinels in behind:
+        assert int((sentinels != 0x5a5a).sum()) == 0
+    assert bool(behind) != one_call
+
+    clean, clean_tile = _stacks_with_a_nan_depth(False)
+    W, H = scene["width"], scene["height"]
+    gi = np.random.default_rng(3).standard_normal((H, W, 4)).astype(np.float32)
+    reference = oracle.render(clean["vertices"], clean["indices"], clean["colors"], clean["opacities"], W, H, 16, 16, 0.0, True, max_layers)
+    wanted = oracle.render_backward(gi, np.zeros((H, W), np.float32), clean["vertices"], clean["indices"], clean["colors"],
+                                    clean["opacities"], reference, W, H, 16, 16, True, max_layers, magnitudes=True)
+    d = to_device(scene, cuda)
+    leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+    for _ in range(2):  # the second one is the torch module's
+        image, _ = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], W, H, 16, 16, 0.0, False, True, max_layers)
+        grads = torch.autograd.grad((image,), leaves, (torch.from_numpy(gi).to(cuda),))
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), grads, wanted[:3], wanted[3:]):
+            g = g.cpu().numpy()
+            assert np.isfinite(g).all()
+            assert_gradients_close(f"beside a NaN depth: {label}", g[tile_of != 1], w[clean_tile != 1], mag[clean_tile != 1])

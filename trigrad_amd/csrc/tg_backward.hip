@@ -823,6 +823,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
     if (p.valid) {
         st = load_back_state(g, p);
         n = min(g.ends[p.index], a.max_layers);  // render.cu:642
+        n = min(n, order_rows(g.order, a, end - start));  // fewer only where a NaN depth had the list blended more than once
     }
     const int64_t plane = order_stride(g.order, a);
     const bool long_list = end - start > kShortList;  // then the positions' high halves were saved as well

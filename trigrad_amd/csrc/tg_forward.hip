@@ -361,7 +361,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                         real b0, b1, b2;
                         bary_apply(r[u].m, p.px, p.py, b0, b1, b2);
                         if (!bary_inside(b0, b1, b2)) continue;  // cannot happen: the selection tested it
-                        if (out.order.low) {
+                        if (out.order.low && s.blended < order_rows(out.order, a, end - start)) {
                             const int64_t at = order_at + (int64_t)s.blended * order_step;
                             const int rel = tk.j(i0 + u);
                             out.order.low[at] = (uint16_t)rel;

@@ -244,10 +244,12 @@ __device__ __forceinline__ int64_t hit_mask_head_words(int skipped_rows = 0) { r
 // Where the saved blend order of a pixel lies: layer l of the pixel at low[l * stride], and, in tiles whose list holds more
 // than kShortList entries, the high half of its list position at high[l * stride].  Two layouts:
 //   planes  (max_layers <= TG_MAX_SAVED_LAYERS) one image plane per layer, the high halves in as many planes behind them
-//   pool    (any number of layers) a pixel blends an entry of its tile's list at most once, so a tile with a list of n
-//           entries is given n rows of one word per pixel: row `start + l` of the pool is layer l of the tile whose list
-//           starts at `start`, and n_keys rows hold every tile's.  Nothing has to be counted or allocated on the device, and
-//           what is never blended is never touched.
+//   pool    (any number of layers) where every depth is a number a pixel blends an entry of its tile's list at most once, so
+//           a tile with a list of n entries is given n rows of one word per pixel: row `start + l` of the pool is layer l of
+//           the tile whose list starts at `start`, and n_keys rows hold every tile's.  Nothing has to be counted or
+//           allocated on the device, and what is never blended is never touched.
+// A NaN depth breaks that bound: the last candidate of a selection, it ends the order the next one would resume from, and the
+// list is blended again and again.  Layers beyond the rows (order_rows) are neither stored nor walked backwards.
 struct OrderStore {
     uint16_t *low;      // null: no order saved
     int64_t high;       // words from a low half to its high half; 0: no list is that long
@@ -255,6 +257,10 @@ struct OrderStore {
 };
 __device__ __forceinline__ int64_t order_stride(const OrderStore &o, const RasterArgs &a) {
     return o.pool_pixels ? o.pool_pixels : (int64_t)a.W * a.H;
+}
+// Layers of a pixel there is room for; n_entries: length of its tile's list.
+__device__ __forceinline__ int order_rows(const OrderStore &o, const RasterArgs &a, int n_entries) {
+    return o.pool_pixels ? n_entries : a.max_layers;
 }
 // t: the pixel's number inside its tile
 __device__ __forceinline__ int64_t order_first(const OrderStore &o, const PixelCoord &p, int list_start, int t) {
