@@ -139,3 +139,26 @@ def test_status_word_check_raises_without_a_gpu():
         _C.verify_finished_frames()
     _C.verify_finished_frames()
     assert _C._pending_checks == []
+
+
+PAIRS_PROGRAM = r"""
+#include <cstdio>
+#include "tg_frame.hpp"
+int main() {
+    const uint32_t counted[2] = {700, 41}, expired[2] = {700, 42}, too_many[2] = {1025, 41};
+    for (const uint32_t *word : {(const uint32_t *)nullptr, counted, expired, too_many})
+        printf("%lld ", (long long)tg::FrameCount{word, 1024, 42}.pairs(33));
+}
+"""
+
+
+def test_pairs_the_sort_takes(tmp_path):
+    """How many pairs the sort's kernels take of a frame whose K is on the device, the rule compiled for the host: none where
+    a wait of the scan expired (its K is a partial sum) or the buffers are too small."""
+    import subprocess
+    from trigrad_amd import build
+    source, program = tmp_path / "pairs.hip", tmp_path / "pairs"
+    source.write_text(PAIRS_PROGRAM)
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-host-only", "-std=c++17", "-w", "-I", build.CSRC,
+                    str(source), "-o", str(program)], check=True)
+    assert subprocess.run([str(program)], check=True, capture_output=True, text=True).stdout.split() == ["33", "700", "0", "0"]

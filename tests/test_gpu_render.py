@@ -793,3 +793,44 @@ def test_nan_depth_stays_inside_its_rows_of_the_order_pool(one_call, max_layers,
             g = g.cpu().numpy()
             assert np.isfinite(g).all()
             assert_gradients_close(f"beside a NaN depth: {label}", g[tile_of != 1], w[clean_tile != 1], mag[clean_tile != 1])
+
+
+def test_pairs_of_an_expired_scan_are_not_sorted(cuda, monkeypatch):
+    """A wait of the scan that expired leaves a K that does not belong to the digit totals: the lists are empty, nothing is
+    moved, and the image is NaN.  No wait is provoked: the state word is set between the binning and the lists."""
+    import struct
+    import torch
+    from trigrad_amd import _C, _lib
+    import scenes as S
+    d = to_device(S.config(0), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], 256, 256, 16, 16, 1 / 256, True, 32)
+    lib = _lib.load(32)
+    in_phases, forged = lib.tg_frame_forward, []
+
+    def forward(call):
+        words = struct.unpack_from("<11Q3q", call)
+        state, (epoch, state_bytes, phases) = words[8], words[11:]
+        code = in_phases(call)
+        if phases == _C._FRAME_BIN:
+            memory = next(st["frame"] for st in _C._frame_states.values() if st["frame"].data_ptr() == state)
+            forged.append(memory[state_bytes + 4:state_bytes + 8].view(torch.int32).fill_(epoch))
+        return code
+
+    monkeypatch.setattr(lib, "tg_frame_forward", forward)
+    monkeypatch.setattr(_C, "_FRAME_UNTIMED", ((_C._FRAME_BIN, None), (_C._FRAME_LISTS | _C._FRAME_RASTER | _C._FRAME_WAIT, None)))
+    try:
+        image, depthmap, kept, frame = _C.frame_forward(*args)
+        with pytest.raises(RuntimeError, match="look-back wait timed out"):
+            frame.status.verify()
+    finally:
+        _C.force_tickets(False)
+        _C._module().forget()
+        for word in forged:
+            word.zero_()
+    assert len(forged) == 1 and frame.n_keys > 0
+    assert torch.isnan(image).all() and torch.isnan(depthmap).all()
+    *_, offsets, _, _, _ = _C._frame_results(image, depthmap, kept, frame, 256, 256, 16, 16, True, 32, d["indices"].shape[0])
+    assert int(offsets.abs().max()) == 0
+    ids = kept[frame.plan.at["ids"]:frame.plan.at["ids"] + 4 * frame.n_keys].view(torch.int32)
+    binned = _C.bin_frame(d["vertices"], d["indices"], 256, 256, 16, 16)
+    assert torch.equal(ids, binned["values"][:frame.n_keys])  # in emission order still

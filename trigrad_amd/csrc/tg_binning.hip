@@ -785,11 +785,13 @@ __global__ __launch_bounds__(kEmitThreads) void frame_emit_kernel(const real4 *_
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
     const uint32_t total = total_and_status[0];
+    const bool expired = total_and_status[1] == epoch;
     if (host_total && blockIdx.x == 0 && tid == 0)
         // K and whether a wait of the scan expired, straight to where the host looks for them
-        __hip_atomic_store(host_total, ((uint64_t)(total_and_status[1] == epoch ? TG_FRAME_EXPIRED : TG_FRAME_COUNTED) << 32) | total,
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    const uint32_t n_keys = total < key_capacity ? total : key_capacity;  // keys beyond the buffers are left out
+        __hip_atomic_store(host_total, ((uint64_t)(expired ? TG_FRAME_EXPIRED : TG_FRAME_COUNTED) << 32) | total, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    // keys beyond the buffers are left out; after an expired wait the heads and offsets may be another call's, so no key is made
+    const uint32_t n_keys = expired ? 0u : total < key_capacity ? total : key_capacity;
     const uint32_t k0 = blockIdx.x * (uint32_t)kEmitChunk;
     if (k0 >= n_keys) return;
     // The owners of the chunk's keys lie between the owner of its first key and the owner of the next chunk's

@@ -6,14 +6,17 @@
 namespace tg {
 
 // A number of pairs that is known on the device only: `word` points at tg_bin_frame's pair (K, epoch of an expired wait),
-// `capacity` is what the buffers hold.  With a null `word` the number is the one the host passed.
+// `capacity` is what the buffers hold.  With a null `word` the number is the one the host passed.  No pairs, so empty lists,
+// where the host runs the frame again: more keys than the buffers hold, or a wait of the scan that expired, whose K is the
+// sum of what it had and does not belong to the digit totals that the sort's bases are made from.
 struct FrameCount {
     const uint32_t *word = nullptr;
     uint32_t capacity = 0, epoch = 0;
-    __device__ __forceinline__ int64_t pairs(int64_t given) const {
+    __host__ __device__ __forceinline__ bool expired() const { return word && word[1] == epoch; }
+    __host__ __device__ __forceinline__ int64_t pairs(int64_t given) const {
         if (!word) return given;
-        const uint32_t n = *word;
-        return n <= capacity ? n : 0;  // more keys than the buffers hold: empty lists, and the host runs the frame again
+        const uint32_t n = word[0];
+        return !expired() && n <= capacity ? n : 0;
     }
 };
 

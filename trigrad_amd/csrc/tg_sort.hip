@@ -656,7 +656,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
                                                                           int medium_cap, LongTiles long_tiles) {
     n_pairs = (uint32_t)frame_count.pairs(n_pairs);
     // lists made from a scan whose wait expired are as invalid as those of a sort whose wait did
-    if (frame_count.word && blockIdx.x == 0 && threadIdx.x == 0 && frame_count.word[1] == frame_count.epoch) *status = TG_STATUS_LOOKBACK_TIMEOUT;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && frame_count.expired()) *status = TG_STATUS_LOOKBACK_TIMEOUT;
     __shared__ union SmallLds {
         WaveSegLds wave[kSortWaves];
         MediumSegLds medium;
