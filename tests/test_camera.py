@@ -232,3 +232,66 @@ def test_splitting_kernels_reject_a_vertex_that_is_not_there(cuda):
         camera.split_clipped(clip, torch.tensor([[0, 1, 4]], dtype=torch.int32, device=cuda), *args)
     assert camera.split_clipped(clip, torch.tensor([[0, 1, -1]], dtype=torch.int32, device=cuda), *args)[0].shape == (3, 4)
     assert camera.split_clipped(clip, torch.zeros((0, 3), dtype=torch.int32, device=cuda), *args)[0].shape == (0, 4)
+
+
+def test_camera_functions_are_recorded_as_tensor_operations():
+    """torch.jit.script and torch.fx take the projection: nothing in it is bound to the tensors of one call."""
+    x, m = torch.rand(7, 4) + 1.0, camera.perspective(50.0, 4, 3)
+    want = camera.clip_to_render(x), camera.project(x[:, :3], m)
+    assert torch.equal(torch.jit.script(camera.clip_to_render)(x), want[0])
+    assert torch.equal(torch.jit.script(camera.project)(x[:, :3], m), want[1])
+    assert torch.equal(torch.fx.symbolic_trace(camera.clip_to_render)(x), want[0])
+
+
+@pytest.mark.gpu
+def test_camera_functions_keep_tangents(cuda):
+    """Forward-mode tangents pass through projection and splitting on the GPU as they do on the CPU."""
+    from torch.autograd import forward_ad
+    cv, idx, col, op = _mesh(5)
+    m = camera.perspective(50.0, 4, 3, dtype=torch.float64)
+    rng = np.random.default_rng(5)
+    tangents = [torch.from_numpy(rng.standard_normal(a.shape)) for a in (cv, col, op)]
+
+    def run(device):
+        with forward_ad.dual_level():
+            clip, colors, opacities = (forward_ad.make_dual(torch.from_numpy(a).to(device), t.to(device))
+                                       for a, t in zip((cv, col, op), tangents))
+            indices = torch.from_numpy(idx).to(device)
+            v, i, c, o = camera.split_clipped(clip, indices, colors, opacities)
+            plain = [forward_ad.unpack_dual(t).primal for t in (clip, opacities)]
+            only_colors = camera.split_clipped(plain[0], indices, colors, plain[1])[2]
+            out = [v, c, o, only_colors, camera.clip_to_render(v), camera.project(clip, m)]
+            return [forward_ad.unpack_dual(t).tangent.cpu() for t in out]
+
+    for got, want in zip(run(cuda), run("cpu")):
+        torch.testing.assert_close(got, want, rtol=1e-10, atol=1e-10)
+    x, t = (torch.from_numpy(a).to(cuda) for a in (cv, rng.standard_normal(cv.shape)))
+    torch.testing.assert_close(torch.func.jvp(lambda p: camera.project(p, m), (x,), (t,))[1].cpu(),
+                               torch.func.jvp(lambda p: camera.project(p, m), (x.cpu(),), (t.cpu(),))[1], rtol=1e-10, atol=1e-10)
+
+
+@pytest.mark.gpu
+def test_camera_functions_under_vmap_tracing_and_dispatch_modes(cuda):
+    from torch.fx.experimental.proxy_tensor import make_fx
+    g = torch.Generator().manual_seed(2)
+    batch, other = torch.rand((3, 11, 4), generator=g).to(cuda) + 1.0, torch.rand((11, 4), generator=g).to(cuda) + 1.0
+    assert torch.equal(torch.func.vmap(camera.clip_to_render)(batch), torch.stack([camera.clip_to_render(x) for x in batch]))
+    for record in (lambda f: torch.jit.trace(f, batch[0]), lambda f: make_fx(f)(batch[0])):
+        assert torch.equal(record(camera.clip_to_render)(other), camera.clip_to_render(other))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_camera_functions_take_rows_off_a_16_byte_boundary(dtype, cuda):
+    cv, idx, col, op = _mesh(4)
+    n = cv.shape[0]
+    clip = torch.from_numpy(cv).to(cuda, dtype)
+    store = torch.empty((4 * n + 1,), dtype=dtype, device=cuda)
+    shifted = store[1:].view(n, 4).copy_(clip)
+    assert shifted.is_contiguous() and shifted.data_ptr() % 16 != 0 and clip.data_ptr() % 16 == 0
+    rest = torch.from_numpy(idx).to(cuda), torch.from_numpy(col).to(cuda, dtype), torch.from_numpy(op).to(cuda, dtype)
+    assert torch.equal(camera.clip_to_render(shifted), camera.clip_to_render(clip))
+    for got, want in zip(camera.split_clipped(shifted, *rest), camera.split_clipped(clip, *rest)):
+        assert torch.equal(got, want)
+    every_other = store[:4 * (n // 2)].view(n // 2, 4)[:, [3, 2, 1, 0]].T.contiguous().T  # strided rows are copied
+    assert torch.equal(camera.clip_to_render(every_other), camera.clip_to_render(every_other.clone(memory_format=torch.contiguous_format)))

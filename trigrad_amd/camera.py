@@ -19,14 +19,33 @@ import torch
 from . import _C, _lib
 
 
-def _native(*tensors):
-    """Whether the library's kernels take these: on one GPU, of one of its scalar types, no gradient wanted."""
-    first = tensors[0]
-    if first.device.type != "cuda" or first.dtype not in (torch.float32, torch.float64):
+def _plain(t):
+    """Whether `t` is memory of a GPU that a kernel can read as it stands: no subclass, proxy or functorch wrapper, no
+    forward-mode tangent, no lazy negation or zero."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and t.device.type == "cuda" and t.layout is torch.strided and not t.is_neg() and not t._is_zerotensor()
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
+
+
+def _native(scalars, others=()):
+    """Whether the library's kernels take these tensors: on one GPU, `scalars` of one of its scalar types, no gradient wanted.
+    What records or transforms tensor operations (tracing, dispatch modes, vmap, jvp) gets tensor operations."""
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    tensors = (*scalars, *others)
+    if not all(_plain(t) for t in tensors):
+        return False
+    first = scalars[0]
+    if first.dtype not in (torch.float32, torch.float64) or any(t.dtype != first.dtype for t in scalars):
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
-    return all(t.device == first.device and t.dtype == first.dtype for t in tensors)
+    return all(t.device == first.device for t in tensors)
+
+
+def _native_rows(clip):
+    """Whether these clip coordinates are rows the kernels read whole: (V,4), contiguous from a 16-byte boundary (or copied)."""
+    return clip.dim() == 2 and clip.shape[1] == 4 and (not clip.is_contiguous() or clip.data_ptr() % 16 == 0)
 
 
 def perspective(fov_degrees, width, height, near=0.1, far=100.0, dtype=torch.float32, device=None):
@@ -47,16 +66,22 @@ def to_clip(positions, matrix):
     return torch.cat([xyz, ones], dim=-1) @ matrix.to(xyz.dtype).to(xyz.device).T
 
 
+def _clip_to_render_native(clip_vertices):
+    """clip_to_render by the library's kernel."""
+    clip = clip_vertices.contiguous()
+    out = torch.empty_like(clip)
+    bits = _C._bits(clip)
+    with _C._on_device(clip.device):
+        _lib.check(_lib.load(bits).tg_clip_to_render(clip.data_ptr(), clip.shape[0], out.data_ptr(), _C._raw_stream(clip.device)),
+                   "tg_clip_to_render", bits)
+    return out
+
+
 def clip_to_render(clip_vertices):
     """(V,4) clip coordinates -> (V,4) render input (x/w, y/w, z/w, 1/w) (viewer.py:276-278)."""
-    if _native(clip_vertices) and clip_vertices.dim() == 2 and clip_vertices.shape[1] == 4:
-        clip = clip_vertices.contiguous()
-        out = torch.empty_like(clip)
-        bits = _C._bits(clip)
-        with _C._on_device(clip.device):
-            _lib.check(_lib.load(bits).tg_clip_to_render(clip.data_ptr(), clip.shape[0], out.data_ptr(), _C._raw_stream(clip.device)),
-                       "tg_clip_to_render", bits)
-        return out
+    if not torch.jit.is_scripting():
+        if _native((clip_vertices,)) and _native_rows(clip_vertices):
+            return _clip_to_render_native(clip_vertices)
     w = clip_vertices[:, 3:4]
     return torch.cat([clip_vertices[:, :3] / w, 1.0 / w], dim=-1)
 
@@ -110,8 +135,8 @@ def split_clipped(clip_vertices, indices, vertex_colors, vertex_opacities):
     Returns (vertices (3N,4), indices (N,3) int32 = arange, colors (3N,C),
     opacities (3N,...)) as a triangle soup in input order.
     """
-    if (_native(clip_vertices, vertex_colors, vertex_opacities) and indices.dtype == torch.int32 and indices.device == clip_vertices.device
-            and indices.dim() == 2 and indices.shape[1] == 3 and clip_vertices.dim() == 2 and clip_vertices.shape[1] == 4
+    if (_native((clip_vertices, vertex_colors, vertex_opacities), (indices,)) and indices.dtype == torch.int32
+            and indices.dim() == 2 and indices.shape[1] == 3 and _native_rows(clip_vertices)
             and vertex_colors.shape[:1] == vertex_opacities.shape[:1] == clip_vertices.shape[:1]):
         return _split_clipped_native(clip_vertices, indices, vertex_colors, vertex_opacities)
     idx = indices.long()
