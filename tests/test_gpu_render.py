@@ -834,3 +834,39 @@ def test_pairs_of_an_expired_scan_are_not_sorted(cuda, monkeypatch):
     ids = kept[frame.plan.at["ids"]:frame.plan.at["ids"] + 4 * frame.n_keys].view(torch.int32)
     binned = _C.bin_frame(d["vertices"], d["indices"], 256, 256, 16, 16)
     assert torch.equal(ids, binned["values"][:frame.n_keys])  # in emission order still
+
+
+def test_exceptions_of_a_known_frame_keep_their_type(cuda):
+    """What fails inside a frame that the torch module renders arrives as it does from the Python function: an allocation as
+    OutOfMemoryError, a saved-tensor hook's own exception as itself.  The frame after it is rendered as ever."""
+    import torch
+    import trigrad_amd
+    import scenes as S
+    d = to_device(S.random_soup(50, 700, 600, seed=2), cuda)
+    leaf = d["vertices"].clone().requires_grad_()
+
+    def frame():
+        return trigrad_amd.render(leaf, d["indices"], d["colors"], d["opacities"], 700, 600)
+
+    want = [frame()[0].detach() for _ in range(2)][-1]  # the module knows the kind now
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    allowed = (torch.cuda.memory_reserved() + (1 << 20)) / torch.cuda.get_device_properties(cuda).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction(allowed)
+        with pytest.raises(torch.OutOfMemoryError):
+            frame()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(frame()[0].detach(), want)
+
+    class Refused(Exception):
+        pass
+
+    def pack(t):
+        raise Refused("not this one")
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        with pytest.raises(Refused, match="not this one"):
+            frame()
+    assert torch.equal(frame()[0].detach(), want)

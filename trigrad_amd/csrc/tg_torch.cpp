@@ -10,6 +10,7 @@
 // Plans and frame states (what tg_bin_frame keeps between calls) are per kind of frame and per device and stream, are made
 // by the Python route and handed over, and are bounded in number there.
 #define PY_SSIZE_T_CLEAN
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -221,18 +222,10 @@ bool fits(const at::Tensor &t, const at::Tensor &with, at::ScalarType type, int6
            (!columns || t.size(1) == columns);
 }
 
-#define TG_NATIVE_BEGIN try {
-#define TG_NATIVE_END                                                \
-    }                                                                \
-    catch (const std::exception &e) {                                \
-        PyErr_SetString(PyExc_RuntimeError, e.what());               \
-        return nullptr;                                              \
-    }
-
 // render(vertices, indices, colors, opacities, width, height, tile_width, tile_height, threshold, record_timing, per_pixel_sort,
 // max_layers) -> (image, depthmap), or None for the Python route.
 PyObject *py_render(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    TG_NATIVE_BEGIN
+    HANDLE_TH_ERRORS  // torch's own exception types: OutOfMemoryError, and what a saved-tensor hook raised
     if (n != 12) Py_RETURN_NONE;
     for (int k = 0; k < 4; k++)
         if (!THPVariable_Check(args[k])) Py_RETURN_NONE;
@@ -313,7 +306,7 @@ PyObject *py_render(PyObject *, PyObject *const *args, Py_ssize_t n) {
     PyTuple_SET_ITEM(result, 0, THPVariable_Wrap(std::move(out[0])));
     PyTuple_SET_ITEM(result, 1, THPVariable_Wrap(std::move(out[1])));
     return result;
-    TG_NATIVE_END
+    END_HANDLE_TH_ERRORS
 }
 
 // bind(addresses of tg_frame_forward, tg_frame_backward, tg_frame_wait, tg_force_tickets, tg_last_error; dict of key counts)
@@ -394,7 +387,7 @@ PyObject *py_forget(PyObject *, PyObject *) {
 }
 
 PyObject *py_verify(PyObject *, PyObject *wait) {
-    TG_NATIVE_BEGIN
+    HANDLE_TH_ERRORS
     const bool waits = wait == Py_True;
     PyThreadState *unlocked = PyEval_SaveThread();
     try {
@@ -405,7 +398,7 @@ PyObject *py_verify(PyObject *, PyObject *wait) {
     }
     PyEval_RestoreThread(unlocked);
     Py_RETURN_NONE;
-    TG_NATIVE_END
+    END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef methods[] = {{"render", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_render)), METH_FASTCALL, nullptr},
