@@ -870,3 +870,49 @@ def test_exceptions_of_a_known_frame_keep_their_type(cuda):
         with pytest.raises(Refused, match="not this one"):
             frame()
     assert torch.equal(frame()[0].detach(), want)
+
+
+@pytest.mark.parametrize("by_module", [True, False])
+def test_status_words_of_a_failed_call_outlive_its_kernels(by_module, cuda):
+    """A call that fails when its kernels are launched already: the words they write in pinned memory are given back only
+    when the stream is done with them.  The failure is the test's: the library's call is made, then its code replaced."""
+    import ctypes as C
+    import torch
+    from trigrad_amd import _C, _lib
+    import trigrad_amd
+    import scenes as S
+    d = to_device(S.random_soup(60, 80, 64, seed=2), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], 80, 64)
+    want = [trigrad_amd.render(*args)[0] for _ in range(2)][-1]
+    lib = _lib.load(32)
+    real, stream, busy = lib.tg_frame_forward, torch.cuda.current_stream(), []
+    address = lambda f: C.cast(f, C.c_void_p).value
+
+    def bind(forward):
+        _C._module().bind(address(forward), *[address(getattr(lib, name)) for name in (
+            "tg_frame_backward", "tg_frame_wait", "tg_force_tickets", "tg_last_error")], _C._key_count_hint)
+
+    @C.CFUNCTYPE(C.c_int, C.c_void_p)
+    def failing(call):
+        phases = C.c_int64.from_address(call + 104)
+        phases.value &= ~_C._FRAME_WAIT
+        torch.cuda._sleep(200_000_000)  # about a tenth of a second in front of the kernels
+        real(call)
+        busy.append(not stream.query())
+        return -1
+
+    try:
+        if by_module:
+            bind(failing)
+        else:
+            _C._module().forget()
+            lib.tg_frame_forward = lambda call: failing(C.addressof(call))
+        with pytest.raises(RuntimeError, match="tg_frame_forward failed with code -1"):
+            trigrad_amd.render(*args)
+        assert busy == [True] and stream.query()
+    finally:
+        lib.tg_frame_forward = real
+        bind(real)
+        torch.cuda.synchronize()
+    for _ in range(2):
+        assert torch.equal(trigrad_amd.render(*args)[0], want)

@@ -575,6 +575,13 @@ class FrameStatus(StatusCheck):
     def ready(self):
         return self.word.value != _FRAME_PENDING
 
+    def keep_until_idle(self, dev):
+        """For a call that failed: kernels launched before the failure may still write the words."""
+        try:
+            torch.cuda.current_stream(dev).synchronize()
+        except RuntimeError:
+            _kept_words.append(self.host)  # never given back: nobody knows when the kernels end
+
     def failed(self):
         if self.word.value == _FRAME_PENDING:
             _lib.check(_lib.load(32).tg_frame_wait(self.address, 2, _FRAME_PENDING, self.stream), "tg_frame_wait")
@@ -582,6 +589,7 @@ class FrameStatus(StatusCheck):
         return self.word.value != 0
 
 
+_kept_words = []
 _pending_checks = []  # status words of earlier frames that nobody has looked at yet
 _pending_lock = threading.Lock()
 
@@ -811,6 +819,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
                                           state.data_ptr(), status.address, stream, epoch, state_bytes, phases, 0, 0, 0, 0)
                     code = lib.tg_frame_forward(c_call)
                     if code:
+                        status.keep_until_idle(dev)
                         _lib.check(code, "tg_frame_forward")
             n_keys, counted = _FRAME_RESULT.unpack_from(call, _FRAME_CALL.size)
             if counted == 1 and n_keys <= capacity:

@@ -113,6 +113,16 @@ void verify_pending(bool wait) {
     }
 }
 
+// The status words of a call that failed: kernels launched before the failure may still write them.
+void keep_until_idle(const std::shared_ptr<Status> &status) {
+    if (hipStreamSynchronize(static_cast<hipStream_t>(status->stream)) == hipSuccess) return;
+    (void)hipGetLastError();
+    static auto *kept = new std::deque<std::shared_ptr<Status>>;  // never given back: nobody knows when the kernels end
+    static std::mutex mutex;
+    std::lock_guard<std::mutex> lock(mutex);
+    kept->push_back(status);
+}
+
 struct Frame : torch::CustomClassHolder {
     std::shared_ptr<const Plan> plan;
     std::shared_ptr<Status> status;
@@ -153,7 +163,14 @@ bool render(Frame &frame, const std::shared_ptr<State> &state, void *stream, con
         f.frame = state->memory.data_ptr();
         f.frame_bytes = state->bytes;
         f.epoch = ++state->epoch;
-        check(lib.forward(&f), "tg_frame_forward");
+        if (const int code = lib.forward(&f)) {
+            try {
+                check(code, "tg_frame_forward");
+            } catch (...) {
+                keep_until_idle(status);
+                throw;
+            }
+        }
     }
     frame.n_keys = f.n_keys;
     if (f.counted != TG_FRAME_COUNTED || f.n_keys > f.key_capacity) {
