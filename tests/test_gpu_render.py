@@ -916,3 +916,35 @@ def test_status_words_of_a_failed_call_outlive_its_kernels(by_module, cuda):
         torch.cuda.synchronize()
     for _ in range(2):
         assert torch.equal(trigrad_amd.render(*args)[0], want)
+
+
+@pytest.mark.parametrize("route", ["module", "one call", "staged"])
+def test_frames_after_a_refused_one(route, cuda, monkeypatch):
+    """Vertices off a 16-byte boundary are refused before the binning's scan runs; the state it keeps from call to call is
+    in step again for the frames that follow."""
+    import torch
+    import trigrad_amd
+    from trigrad_amd import _C
+    import scenes as S
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", route != "staged")
+    scene = S.random_soup(900, 200, 150, seed=2)
+    d = to_device(scene, cuda)
+    n = d["vertices"].shape[0]
+    shifted = torch.empty((4 * n + 1,), device=cuda)[1:].view(n, 4).copy_(d["vertices"])
+
+    def frame(vertices):
+        if route == "one call":
+            _C._module().forget()
+        return trigrad_amd.render(vertices, d["indices"], d["colors"], d["opacities"], 200, 150)[0]
+
+    want = [frame(d["vertices"]) for _ in range(3)][-1]
+    for _ in range(2):  # either parity of the calls so far
+        frame(d["vertices"])
+        with pytest.raises(RuntimeError, match="16-byte aligned"):
+            frame(shifted)
+        state = [st["frame"] for st in _C._frame_states.values()]
+        if route != "module":
+            assert any(int(memory.abs().max()) == 0 for memory in state)
+        for _ in range(3):
+            assert torch.equal(frame(d["vertices"]), want)
+    trigrad_amd.verify_frames()

@@ -350,7 +350,9 @@ def bin_frame_supported(vertices, width, height, tile_width, tile_height):
 def _next_frame_state(dev, need):
     """The frame state of at least `need` bytes of the device's current stream, zeroed when it is made, and the epoch of
     the call about to use it (they count up by one; a state whose epochs run out is replaced by a fresh one).  A state
-    per stream: frames on one stream follow each other, frames on two streams may run at the same time."""
+    per stream: frames on one stream follow each other, frames on two streams may run at the same time.  A call counts
+    its digits into one set of totals and clears the other one for the next call; a call that failed may have done neither,
+    so its state has to be zeroed."""
     key = (dev.index, _raw_stream(dev))
     with _frame_lock:
         st = _frame_states.get(key)
@@ -397,10 +399,12 @@ def bin_frame(vertices, indices, width, height, tile_width, tile_height, capacit
     # the sort's own histogram route (more than 256 tile columns or rows) clears its workspace itself
     zero_bytes = ws_bytes if max(tiles) <= 256 else 0
     with _on_device(dev):
-        _lib.check(lib.tg_bin_frame(_ptr(vertices), vertices.shape[0], _ptr(indices), M, width, height, tile_width, tile_height,
-                                    _ptr(b["keys"]), _ptr(b["values"]), capacity, _ptr(pair), _ptr(frame),
-                                    frame_bytes, epoch, _ptr(b["ws"]), zero_bytes, _ptr(b["status"]), _stream(vertices)),
-                   "tg_bin_frame")
+        code = lib.tg_bin_frame(_ptr(vertices), vertices.shape[0], _ptr(indices), M, width, height, tile_width, tile_height,
+                                _ptr(b["keys"]), _ptr(b["values"]), capacity, _ptr(pair), _ptr(frame),
+                                frame_bytes, epoch, _ptr(b["ws"]), zero_bytes, _ptr(b["status"]), _stream(vertices))
+        if code:
+            frame.zero_()  # see _next_frame_state
+            _lib.check(code, "tg_bin_frame")
     return b
 
 
@@ -819,6 +823,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
                                           state.data_ptr(), status.address, stream, epoch, state_bytes, phases, 0, 0, 0, 0)
                     code = lib.tg_frame_forward(c_call)
                     if code:
+                        state.zero_()
                         status.keep_until_idle(dev)
                         _lib.check(code, "tg_frame_forward")
             n_keys, counted = _FRAME_RESULT.unpack_from(call, _FRAME_CALL.size)

@@ -167,6 +167,8 @@ bool render(Frame &frame, const std::shared_ptr<State> &state, void *stream, con
             try {
                 check(code, "tg_frame_forward");
             } catch (...) {
+                // whether the call's scan ran is not known: the digit totals and epochs start anew, as in a fresh state
+                state->memory.zero_();
                 keep_until_idle(status);
                 throw;
             }
