@@ -118,6 +118,27 @@ def test_double_build_matches_oracle(name, mode, cuda, oracle):
             np.testing.assert_allclose(g.cpu().numpy(), w, rtol=1e-9, atol=1e-12 + 1e-12 * scale, err_msg=f"{name}/{mode}: {label}")
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["A", "A_40", "B"])
+@pytest.mark.parametrize("n,tw,th", [(12000, 16, 16), (1500, 8, 8), (6000, 12, 6), (400, 16, 16)])
+def test_double_build_of_crowds_matches_oracle(n, tw, th, mode, cuda, oracle):
+    """The forward kernels' tests of small triangles, lane by lane, and their batches in turn, with lists long enough for the
+    depth bounds and without: bit-identical to the oracle's float64 instantiation."""
+    from test_gpu_render import _crowded_scene
+    from trigrad_amd import _C
+    W, H = 70, 45
+    scene = _as_double(_crowded_scene(n, W, H))
+    m = DOUBLE_MODES[mode]
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    d = to_device(scene, cuda)
+    arrays = [scene[k] for k in ("vertices", "indices", "colors", "opacities")]
+    want = oracle.render(*arrays, W, H, tw, th, 1 / 256, m["per_pixel_sort"], ml)
+    got = _C._forward_full(*(d[k] for k in ("vertices", "indices", "colors", "opacities")), W, H, tw, th, 1 / 256, True,
+                           m["per_pixel_sort"], ml)
+    for g, name in ((got[0], "image"), (got[3], "sorted_ids"), (got[4], "offsets"), (got[6], "ends")):
+        np.testing.assert_array_equal(g.cpu().numpy(), want[name], err_msg=name)
+
+
 def _reference_case(S, which, cuda):
     """Scenes and arguments of the reference's tests/test_render_gradients.py (opacity 0.99 everywhere)."""
     scene = S.overlapping_squares(10) if which == "squares" else S.large_triangles(3, r=4)

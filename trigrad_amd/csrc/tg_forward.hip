@@ -92,9 +92,10 @@ __device__ __forceinline__ void write_pixel(const ForwardOut &o, const PixelCoor
     o.image[p.index] = make_real4(s.c0, s.c1, s.c2, s.alpha);
 }
 
-// Eight waves per SIMD (64 registers, a few of the loop's constants in scratch memory): 212 -> 194 us against the 73 registers
-// it would take (10^6 triangles, 1920 x 1080).
-__global__ __launch_bounds__(kTileThreads, 8) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
+// Eight waves per SIMD (63 registers, nothing in scratch memory): 212 -> 194 us against the 73 registers it would take
+// (10^6 triangles, 1920 x 1080).  No bound in double precision: held to the five waves that the LDS allows it spills (8 x 8
+// tiles: 112 -> 123 us).
+__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
     __shared__ BlendRecord s_rec[kBatch];
     __shared__ uint8_t s_touch[kBatch];
     __shared__ WaveRect s_rects[kMaxTileWaves];
@@ -340,12 +341,15 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
             if (found == 0) {
                 active = false;  // render.cu:594
             } else {
-                // kGatherAhead records are fetched together: the chains of dependent loads
-                // (list -> indices -> vertices) of those that come from memory overlap
-                for (int i0 = 0; i0 < todo; i0 += kGatherAhead) {
-                    BlendRecord r[kGatherAhead];
+                // kTogether records are fetched together: the chains of dependent loads (list -> indices -> vertices) of those
+                // that come from memory overlap.  They are the kernel's peak of registers: where a wave's batches are fetched
+                // a whole batch ahead a fourth record would spill (8 x 8 tiles: 87 -> 86 us; two together: lists of
+                // hundreds 220 -> 226)
+                constexpr int kTogether = kInTurn ? 4 : 3;
+                for (int i0 = 0; i0 < todo; i0 += kTogether) {
+                    BlendRecord r[kTogether];
 #pragma unroll
-                    for (int u = 0; u < kGatherAhead; u++) {
+                    for (int u = 0; u < kTogether; u++) {
                         const int rel = tk.j(min(i0 + u, todo - 1));
                         if (rel < n_rows) {
                             real *w = reinterpret_cast<real *>(&r[u]);
@@ -356,7 +360,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                         }
                     }
 #pragma unroll
-                    for (int u = 0; u < kGatherAhead; u++) {
+                    for (int u = 0; u < kTogether; u++) {
                         if (i0 + u >= todo) break;
                         real b0, b1, b2;
                         bary_apply(r[u].m, p.px, p.py, b0, b1, b2);
@@ -385,8 +389,11 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
 // One workgroup per tile.  With 16-bit positions the tiles whose lists are too long for them are left to
 // forward_pixel_order_long_lists_kernel.
 // kInTurn: the workgroup has four waves.
+// Workgroups a CU: what their LDS allows.  No bound in double precision: held to two workgroups every instance spills (10^5
+// triangles, 1024 x 1024: 229 us instead of 223, tiles of 8 x 8 190 instead of 168).
 template <int kStage, typename Pos, bool kInTurn>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 && kStage == kSelectBatchShort ? 3 : 2) void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage == kSelectBatchShort ? 3 : 2)
+void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ uint8_t s_touch[kStage];
     __shared__ WaveRect s_rects[kMaxTileWaves];

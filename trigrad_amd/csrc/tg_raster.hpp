@@ -19,7 +19,6 @@ constexpr int kLayers = 32;         // per-pixel selection batch (render.cu:570,
 constexpr int kMaxTilePixels = 1024;  // tile_w * tile_h limit of the API (wrapper.py:143)
 constexpr int kTileThreads = 256;     // workgroup size limit
 constexpr int kShortList = 0xffff;    // longest tile list whose positions fit 16 bits
-constexpr int kGatherAhead = 4;       // records a lane of a per-pixel-order kernel fetches together
 
 struct RasterArgs {
     const real4 *vertices;
