@@ -164,17 +164,36 @@ def test_pairs_the_sort_takes(tmp_path):
     assert subprocess.run([str(program)], check=True, capture_output=True, text=True).stdout.split() == ["33", "700", "0", "0"]
 
 
+def _device_compile(source, *flags):
+    """Compiles one kernel file for the device with the build's flags; returns what the compiler said."""
+    import subprocess
+    from trigrad_amd import build
+    return subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), *[f for f in build.FLAGS if f != "-shared"],
+                           "--offload-device-only", *flags, os.path.join(build.CSRC, source)], check=True, capture_output=True, text=True).stderr
+
+
 @pytest.mark.parametrize("flags", [(), ("-DTG_DOUBLE_PRECISION",)])
 def test_forward_kernels_need_no_scratch_memory(flags, tmp_path):
     """Scratch memory costs every launch of a kernel some microseconds: no instance of the forward kernels spills a register
     to it, in neither precision, by the compiler's own report."""
-    import subprocess
-    from trigrad_amd import build
-    report = subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), *[f for f in build.FLAGS if f != "-shared"], *flags,
-                             "-Rpass-analysis=kernel-resource-usage", "--offload-device-only", "-c",
-                             os.path.join(build.CSRC, "tg_forward.hip"), "-o", str(tmp_path / "forward.o")],
-                            check=True, capture_output=True, text=True).stderr
+    report = _device_compile("tg_forward.hip", *flags, "-Rpass-analysis=kernel-resource-usage", "-c", "-o", str(tmp_path / "forward.o"))
     names = re.findall(r"Function Name: (\S+)", report)
     scratch = re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", report)
     assert len(names) == 6 == len(scratch)
     assert dict(zip(names, scratch)) == dict.fromkeys(names, "0")
+
+
+@pytest.mark.parametrize("flags,scalar", [((), "float"), (("-DTG_DOUBLE_PRECISION",), "double")])
+def test_record_parts_are_read_with_the_alignment_they_have(flags, scalar, tmp_path):
+    """The parts of a record lie on scalar boundaries (y, z, w of a vertex; a triangle's indices and matrix): as written,
+    before the optimiser narrows anything, no read of them promises more or goes beyond them."""
+    _device_compile("tg_forward.hip", *flags, "-Xclang", "-disable-llvm-passes", "-emit-llvm", "-S", "-o", str(tmp_path / "forward.ll"))
+    text = (tmp_path / "forward.ll").read_text()
+    body = {name: re.search(r"define [^\n]*%s[^\n]*\n(.*?)\n}" % name, text, re.S).group(1)
+            for name in ("DepthParts14fetch_vertices", "DepthParts12fetch_matrix")}
+    reads = re.findall(r"load <(\d) x %s>, ptr \S+, align (\d+)" % scalar, "\n".join(body.values()))
+    assert set(reads) <= {("4", "4")}  # the matrix: two fours and a scalar, packed
+    assert body["DepthParts14fetch_vertices"].count("read_three") == 3 and body["DepthParts12fetch_matrix"].count("read_three") == 1
+    copies = re.findall(r"define [^\n]*read_three[^\n]*\n.*?memcpy[^\n]* align (\d+) \S+ i64 (\d+)", text, re.S)
+    size = 4 if scalar == "float" else 8
+    assert sorted(copies) == sorted([("4", "12"), (str(size), str(3 * size))])

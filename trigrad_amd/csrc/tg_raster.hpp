@@ -186,12 +186,18 @@ __device__ __forceinline__ void gather_depth(const RasterArgs &a, int j, DepthRe
 }
 
 // gather_depth in steps, for a caller that asks for a record's parts before it needs them.  The parts stay as they were
-// loaded (whole vectors, put together by `record` only): a copy into another register would wait for the load.
+// loaded (whole vectors, put together by `record` only): a copy into another register would wait for the load.  A vector of
+// three is read as the bytes it holds: through a pointer of its own type it would be read as four and from a 16-byte boundary.
 typedef real real3v __attribute__((ext_vector_type(3)));
 typedef real real4v __attribute__((ext_vector_type(4)));
 typedef int int3v __attribute__((ext_vector_type(3)));
-struct __attribute__((packed, aligned(4))) TriIndices { int3v id; };
 struct __attribute__((packed, aligned(4))) Matrix9 { real4v a, b; real c; };
+template <typename V, typename T>
+__device__ __forceinline__ V read_three(const T *p) {
+    V v;
+    __builtin_memcpy(&v, p, 3 * sizeof(T));
+    return v;
+}
 struct DepthParts {
     int tri;
     int3v id;
@@ -203,7 +209,7 @@ struct DepthParts {
     // the triangle's vertex numbers and matrix
     __device__ __forceinline__ void fetch_matrix(const RasterArgs &a) {
         const int64_t t = tri;
-        id = reinterpret_cast<const TriIndices *>(a.indices + 3 * t)->id;
+        id = read_three<int3v>(a.indices + 3 * t);
         const Matrix9 *m = reinterpret_cast<const Matrix9 *>(a.bary + 9 * t);
         m0 = m->a;
         m1 = m->b;
@@ -211,9 +217,9 @@ struct DepthParts {
     }
     __device__ __forceinline__ void fetch_vertices(const RasterArgs &a) {
         const real *v = reinterpret_cast<const real *>(a.vertices) + 1;
-        va = *reinterpret_cast<const real3v *>(v + 4 * (int64_t)id.x);
-        vb = *reinterpret_cast<const real3v *>(v + 4 * (int64_t)id.y);
-        vc = *reinterpret_cast<const real3v *>(v + 4 * (int64_t)id.z);
+        va = read_three<real3v>(v + 4 * (int64_t)id.x);
+        vb = read_three<real3v>(v + 4 * (int64_t)id.y);
+        vc = read_three<real3v>(v + 4 * (int64_t)id.z);
     }
     __device__ __forceinline__ DepthRecord record() const {
         DepthRecord r;
