@@ -197,3 +197,20 @@ def test_record_parts_are_read_with_the_alignment_they_have(flags, scalar, tmp_p
     copies = re.findall(r"define [^\n]*read_three[^\n]*\n.*?memcpy[^\n]* align (\d+) \S+ i64 (\d+)", text, re.S)
     size = 4 if scalar == "float" else 8
     assert sorted(copies) == sorted([("4", "12"), (str(size), str(3 * size))])
+
+
+@pytest.mark.parametrize("columns,rows,slots_by_order", [(32, 24, (False, False)), (32, 32, (True, False)), (64, 32, (True, False)),
+                                                         (65, 32, (True, True))])
+def test_long_tiles_are_started_first_where_not_all_fit_at_once(columns, rows, slots_by_order):
+    """768 workgroups of a per-pixel-order frame run at one time, 2048 of a tile-order one: only frames with more tiles keep
+    slots for the tiles with long lists, 129 words and one a tile."""
+    from trigrad_amd import _C
+    tiles, counts = columns * rows, (3_000_000, 1_000_000)
+
+    def scratch(pixel_order, n_triangles):
+        return _C._FramePlan(counts[0], n_triangles, 16 * columns, 16 * rows, 16, 16, pixel_order, 32, 2_000_000, 0, 0.0).scratch_bytes
+
+    slots = 768 + 256 * -(-4 * tiles // 256)
+    for pixel_order, expected in zip((1, 0), slots_by_order):
+        short = scratch(pixel_order, 1000)  # no list can be a long one
+        assert scratch(pixel_order, counts[1]) - short == (slots if expected else 0)

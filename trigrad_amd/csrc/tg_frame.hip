@@ -57,13 +57,15 @@ static FrameLayout frame_layout(const tg_frame &f) {
     L.sort_bytes = tg_build_frame_lists_workspace_bytes(f.key_capacity, tiles_x, tiles_y);
     L.sort = take(L.sort_bytes);
     L.zero_bytes = L.sort_bytes;
-    // Where all tiles' workgroups fit the device at once (three a CU in per-pixel order) it does not matter which one starts
-    // first.  Long: 1024 entries, and twice the mean.  Forward kernel, before and after the long tiles come first: 1.3 million
-    // triangles of a mesh, 1920 x 1080 (longest list 5200) 677 -> 610 us, 200000 around the camera (8400) 184 -> 153; frames
-    // without a long list pay 1 to 2 us for the workgroups that find none.
+    // Where all tiles' workgroups fit the device at once it does not matter which one starts first: three of a 16 x 16 tile a
+    // CU in per-pixel order, eight in tile order (there, 1024 tiles of a mesh: kernel 382 us with the long ones first, 378
+    // without; 1900 tiles: 732 and 728).  Long: 1024 entries, and twice the mean.  Forward kernel, before and after the long
+    // tiles come first, per-pixel order: 1.3 million triangles of a mesh, 1920 x 1080 (longest list 5200) 677 -> 610 us,
+    // 200000 around the camera (8400) 184 -> 153; frames without a long list pay 1 to 2 us for the workgroups that find none.
     const int64_t longest = f.key_capacity < f.n_triangles ? f.key_capacity : f.n_triangles;
     const int64_t limit = std::max<int64_t>(1024, ceil_div64(2 * f.key_capacity, tiles));
-    if (tiles > 768 && longest >= limit) {
+    const int at_once = 256 * (f.per_pixel_sort ? 3 : 8);
+    if (tiles > at_once && longest >= limit) {
         L.long_limit = (int)limit;
         L.long_tiles = take((1 + kLongTileSlots) * 4);
         L.slots = take((size_t)tiles * 4);
