@@ -111,6 +111,32 @@ def test_python_entry_point_errors_without_gpu():
     chk(o, "o", 3)  # a bare int is promoted to a 1-tuple
 
 
+def test_argument_errors_and_double_precision_do_not_need_the_torch_module(monkeypatch):
+    """The C++ module for known frames is the float build's and the GPU's: what is refused for another reason says so where the
+    module is not there, and double precision does without."""
+    import torch
+    import trigrad_amd
+    from trigrad_amd import _C, _lib
+
+    def missing(key_counts):
+        raise AssertionError("the torch module was asked for")
+
+    monkeypatch.setattr(_lib, "_torch_module", None)
+    monkeypatch.setattr(_lib, "torch_module", missing)
+    monkeypatch.setattr(_C, "_module_settings", None)
+    v, i, c, o = torch.zeros((3, 4)), torch.zeros((1, 3), dtype=torch.int32), torch.zeros((3, 3)), torch.zeros(3)
+    with pytest.raises(TypeError, match="vertices must be on cuda"):
+        trigrad_amd.render(v, i, c, o, 16, 16)
+    with pytest.raises(AttributeError):
+        trigrad_amd.render([[0.0] * 4], i, c, o, 16, 16)
+    _C.set_precision(torch.float64)
+    try:
+        with pytest.raises(TypeError, match="vertices must be on cuda"):
+            trigrad_amd.render(v.double(), i, c.double(), o.double(), 16, 16)
+    finally:
+        _C.set_precision(torch.float32)
+
+
 def test_product_does_not_reach_into_the_oracle():
     """Nothing under trigrad_amd/ may import, include or load the oracle."""
     for dirpath, _, files in os.walk(os.path.join(ROOT, "trigrad_amd")):

@@ -721,12 +721,12 @@ def render_by_torch_module(vertices, indices, colors, opacities, width, height, 
                            record_timing, per_pixel_sort, max_layers):
     """(image, depthmap) of a frame whose kind was seen before, with its autograd node, or None: for the route through Python."""
     global _module_settings
-    settings = (ONE_CALL_FRAME, FUSED_BINNING, SAVE_BLEND_ORDER, SAVE_HIT_MASKS, EARLY_STOP_MIN_AVG_LIST, ORDER_POOL_MAX_BYTES, precision)
+    if not ONE_CALL_FRAME or precision is not torch.float32 or not isinstance(vertices, torch.Tensor) or not vertices.is_cuda:
+        return None  # nothing of this is the module's: it need not be there
+    settings = (FUSED_BINNING, SAVE_BLEND_ORDER, SAVE_HIT_MASKS, EARLY_STOP_MIN_AVG_LIST, ORDER_POOL_MAX_BYTES)
     if settings != _module_settings:
         _module().forget()
         _module_settings = settings
-    if not ONE_CALL_FRAME or precision is not torch.float32:
-        return None
     if _pending_checks:
         verify_frames(wait=False)
     return _lib._torch_module.render(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
