@@ -182,6 +182,29 @@ def test_more_long_tiles_than_slots(mode, cuda, monkeypatch):
         assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
 
 
+def test_more_long_tiles_than_slots_in_tile_order(cuda, monkeypatch):
+    """The same in tile order, where tiles are started out of turn in frames with more than 2048 of them: 4800 tiles, some 240
+    of them with lists beyond 1024 entries."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    n, width, height, tile = 500_000, 640, 480, 8
+    soup = S.random_soup(n, width, height, seed=8, sigma_px=0.6, opacity=(0.02, 0.3))
+    v = soup["vertices"].reshape(n, 3, 4).copy()
+    v[: n * 95 // 100, :, :2] = (v[: n * 95 // 100, :, :2] + 1.0) * 0.225 - 1.0
+    d = to_device(dict(soup, vertices=v.reshape(-1, 4)), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, tile, tile, 1 / 256, True, False, n + 1)
+    for _ in range(3):
+        got = _C.render_forward(*args)
+    lengths = got[4][1:] - got[4][:-1]
+    assert lengths.numel() > 2048
+    assert int((lengths >= max(1024, -(-2 * _C._round_capacity(got[3].numel()) // lengths.numel()))).sum()) > 128
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C.render_forward(*args)
+    for i in (0, 1, 2, 3, 4, 5, 6):
+        assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
+
+
 def _grad_inputs(scene, seed, with_depth):
     rng = np.random.default_rng(seed)
     H, W = scene["height"], scene["width"]
