@@ -240,3 +240,19 @@ def test_long_tiles_are_started_first_where_not_all_fit_at_once(columns, rows, s
     for pixel_order, expected in zip((1, 0), slots_by_order):
         short = scratch(pixel_order, 1000)  # no list can be a long one
         assert scratch(pixel_order, counts[1]) - short == (slots if expected else 0)
+
+
+@pytest.mark.parametrize("flags", [0, 1 | 4, 1 | 8, 1 | 4 | 16])
+def test_buffers_for_a_rounded_number_of_triangles_serve_every_smaller_one(flags):
+    """What frames with different numbers of triangles share is sized for the rounded number: nothing a frame needs is larger
+    for a smaller one."""
+    from trigrad_amd import _C
+    assert [_C._round_count(n) for n in (1, 31, 32, 33, 1000, 65535, 65536, 65537, 2 ** 31 - 1)] == [
+        1, 31, 32, 34, 1024, 65536, 65536, 69632, 2 ** 31 - 1]
+    for n in (33, 500, 1023, 2047, 33_000, 65_000, 65_535, 65_537, 1_000_000):
+        assert n <= _C._round_count(n) <= n + n // 16 + 1 and _C._round_count(_C._round_count(n)) == _C._round_count(n)
+        for width, height, pixel_order in ((500, 400, 1), (1920, 1080, 1), (1920, 1080, 0)):
+            sizes = [_C._FramePlan(0, k, width, height, 16, 16, pixel_order, k + 1, 300_000, flags, 0.0)
+                     for k in (n, _C._round_count(n))]
+            for field in ("kept_bytes", "scratch_bytes", "frame_bytes"):
+                assert getattr(sizes[0], field) <= getattr(sizes[1], field)

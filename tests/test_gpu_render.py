@@ -971,3 +971,60 @@ def test_frames_after_a_refused_one(route, cuda, monkeypatch):
         for _ in range(3):
             assert torch.equal(frame(d["vertices"]), want)
     trigrad_amd.verify_frames()
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_unlimited", "B_unlimited"])
+@pytest.mark.parametrize("around", [29, 2030, 65530])
+def test_frames_whose_number_of_triangles_changes_share_plans(around, mode, cuda, monkeypatch):
+    """A camera that moves through a split scene has another number of triangles in every frame: such frames share plans (up
+    to a sixteenth more triangles), so all but the first of a bucket are the torch module's; every frame is the staged
+    route's.  The counts pass the edges of buckets, of 32 triangles and of 16-bit list positions."""
+    import torch
+    import trigrad_amd
+    from trigrad_amd import _C
+    import scenes as S
+    W, H, m = 150, 100, MODES[mode]
+    d = to_device(S.random_soup(around + 40, W, H, seed=3, sigma_px=3.0), cuda)
+    gi = torch.from_numpy(np.random.default_rng(1).standard_normal((H, W, 4)).astype(np.float32)).to(cuda)
+    counts = [around + k for k in (7, 0, 3, 20, 6, 11, 1, 9, 5, 33, 4, 2)]
+
+    def run(n):
+        leaves = [d[k][:3 * n].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+        image, depth = trigrad_amd.render(leaves[0], d["indices"][:n], *leaves[1:], W, H, 16, 16, 1 / 256, False, m["per_pixel_sort"],
+                                          m["max_layers"])
+        return [image.detach(), depth.detach(), *torch.autograd.grad((image,), leaves, (gi,))]
+
+    _C._module().forget()
+    by_python, in_python = [], _C.frame_forward
+    monkeypatch.setattr(_C, "frame_forward", lambda *a, **k: by_python.append(a[1].shape[0]) or in_python(*a, **k))
+    got = [run(n) for n in counts]
+    buckets = {_C._round_count(n) for n in counts}
+    assert len(by_python) == len(buckets) and {_C._round_count(n) for n in by_python} == buckets
+    assert len(buckets) < len(counts) or around < 32
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    for n, one in zip(counts, got):
+        want = run(n)
+        assert torch.equal(one[0], want[0]) and torch.equal(one[1], want[1])
+        for a, b in zip(one[2:], want[2:]):
+            # sums of float32 terms in another order: two rounding steps of the largest sum
+            assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max()) + 1e-6
+
+
+def test_key_buffers_of_a_size_seen_before(cuda):
+    """A number of triangles not seen before takes its key buffers from the last frame of the image and tile size, not from a
+    guess, and the tables of such numbers stay bounded."""
+    import trigrad_amd
+    from trigrad_amd import _C
+    import scenes as S
+    W, H = 410, 300
+    d = to_device(S.random_soup(5000, W, H, seed=3, sigma_px=1.0), cuda)
+    made = []
+    for n in range(4000, 5000, 3):
+        image, depth, kept, frame = _C.frame_forward(d["vertices"], d["indices"][:n], d["colors"], d["opacities"], W, H, 16, 16, 1 / 256,
+                                                     True, 32)
+        made.append((frame.n_keys, frame.plan.capacity))
+    assert made[0][1] == 3 * 4000 + 65536
+    assert all(keys <= capacity <= 1.3 * keys + 2048 for keys, capacity in made[1:])
+    for table in (_C._frame_key_hints, _C._frame_size_hints, _C._frame_plans):
+        assert len(table) <= _C._MAX_REMEMBERED
+    trigrad_amd.verify_frames()

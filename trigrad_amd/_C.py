@@ -660,7 +660,8 @@ _FRAME_BYTES = _FRAME_CALL.size + _FRAME_RESULT.size + _FRAME_KIND.size
 
 _frame_plans = {}  # frame kind -> _FramePlan
 _frame_key_hints = {}  # (device index, triangles, image and tile size) -> K of the last such frame
-_MAX_REMEMBERED = 256  # entries either of them holds before it starts anew
+_frame_size_hints = {}  # (device index, image and tile size) -> (K, triangles) of the last such frame
+_MAX_REMEMBERED = 256  # entries each of them holds before the oldest one goes
 
 
 class _FramePlan:
@@ -700,8 +701,15 @@ def _plan_for(kind):
 
 def _remember(table, key, value):
     if len(table) >= _MAX_REMEMBERED and key not in table:
-        table.clear()
+        table.pop(next(iter(table)), None)
     table[key] = value
+
+
+def _round_count(n):
+    """A number of triangles up to the next one that frames share a plan for: itself below 32, else at most a sixteenth more.
+    A moving camera's split scene, or one that is being refined, has another number in every frame."""
+    step = 1 << max(n.bit_length() - 5, 0)
+    return min(-(-n // step) * step, 0x7fffffff)
 
 
 def _round_capacity(n):
@@ -740,9 +748,14 @@ def _module():
     return _lib.torch_module(_key_count_hint)
 
 
-def _leave_plan(plan, kind, for_backward, dev, stream):
-    """Hands the plan of the frames to come (and a frame state for the stream) to the torch module."""
-    n_vertices, n_triangles, width, height, tile_width, tile_height, per_pixel_sort, max_layers, capacity, flags, threshold = kind
+def _leave_plan(kind, for_backward, dev, stream):
+    """Hands a plan for the frames to come (and a frame state for the stream) to the torch module: for all numbers of vertices,
+    and of triangles up to the rounded one."""
+    _, n_triangles, width, height, tile_width, tile_height, per_pixel_sort, max_layers, capacity, flags, threshold = kind
+    limit = 0 if max_layers == n_triangles + 1 else max_layers  # 0: none
+    n_triangles = _round_count(n_triangles)
+    plan = _plan_for((0, n_triangles, width, height, tile_width, tile_height, per_pixel_sort,
+                      limit or min(n_triangles + 1, 0x7fffffff), capacity, flags, threshold))
     low, high = capacity // 4 if capacity > 1 << 18 else 0, 1 << 30
     if per_pixel_sort:
         # the depth bounds are for lists of a length; a scene that hovers around it keeps what it has
@@ -752,8 +765,8 @@ def _leave_plan(plan, kind, for_backward, dev, stream):
         else:
             high = min(high, long_lists + long_lists // 4)
     module = _module()
-    key = (dev.index, n_vertices, n_triangles, width, height, tile_width, tile_height,
-           struct.unpack("<q", struct.pack("<d", threshold))[0], per_pixel_sort, max_layers, 1 if for_backward else 0)
+    key = (dev.index, n_triangles, width, height, tile_width, tile_height,
+           struct.unpack("<q", struct.pack("<d", threshold))[0], per_pixel_sort, limit, 1 if for_backward else 0)
     module.remember(key, plan.kind, plan.frame_bytes, low, high)
     if module.state_bytes(dev.index, stream) < plan.frame_bytes:
         size = _state_size(plan.frame_bytes)
@@ -771,7 +784,8 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
     """-> (image, depthmap, kept, frame): `kept` is the block that holds what the backward pass reads.
 
     The call launches everything and waits for K only then; a frame with more keys than its buffers were made for (K of the
-    last frame of its kind and an eighth more, or three per triangle) is rendered again into larger ones."""
+    last frame of its kind, or of its size by the number of triangles, and an eighth more; else three per triangle) is
+    rendered again into larger ones."""
     global _frame_counter
     lib = _lib.load(32)
     dev = vertices.device
@@ -788,6 +802,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
             elif SAVE_BLEND_ORDER:
                 flags |= _FRAME_ORDER_PLANES if max_layers <= MAX_SAVED_LAYERS else _FRAME_ORDER_POOL
         hint_key = (dev.index, n_triangles, width, height, tile_width, tile_height)
+        size_key = (dev.index, width, height, tile_width, tile_height)
 
         def kind_for(expected, capacity):
             # long lists: depth bounds let the selection leave a list before its end
@@ -796,6 +811,9 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
                     flags | _FRAME_LIST_BOUNDS if bounds else flags, float(early_stopping_threshold))
 
         expected = _frame_key_hints.get(hint_key)
+        if expected is None and size_key in _frame_size_hints:
+            keys, triangles = _frame_size_hints[size_key]  # another number of triangles: about as many keys each
+            expected = -(-keys * n_triangles // triangles)
         if expected is None:
             expected, capacity = 2 * n_triangles, min(3 * n_triangles + 65536, (1 << 30) - 1)
         else:
@@ -843,12 +861,12 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
             _frame_key_hints[hint_key] = n_keys
         else:
             _remember(_frame_key_hints, hint_key, n_keys)
+        _remember(_frame_size_hints, size_key, (n_keys, n_triangles))
         _key_count_hint[dev.index] = n_keys
         with _pending_lock:
             _pending_checks.append(status)
         if timer is None:
-            kind = kind_for(n_keys, _round_capacity(n_keys))
-            _leave_plan(_plan_for(kind), kind, for_backward, dev, stream)
+            _leave_plan(kind_for(n_keys, _round_capacity(n_keys)), for_backward, dev, stream)
     frame.plan, frame.status, frame.n_keys = plan, status, n_keys
     return image, depthmap, kept, frame
 

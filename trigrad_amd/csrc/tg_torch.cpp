@@ -21,6 +21,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <array>
 #include <cstring>
 #include <deque>
@@ -49,17 +50,30 @@ void check(int code, const char *what) {
     throw std::runtime_error(std::string(what) + " failed with code " + std::to_string(code) + ": " + (text ? text : ""));
 }
 
-// The constant part of a call: struct tg_frame from n_vertices on.
+// The part of a call that a plan holds: struct tg_frame from n_vertices on.  The counts come with the frame: a viewer that
+// moves through a split scene, or a training loop that adds triangles, has others in every frame.  A plan's sizes are made
+// for the number of triangles rounded up (round_count), and no size a frame needs grows when its count gets smaller.
 constexpr size_t kKindBytes = sizeof(tg_frame) - offsetof(tg_frame, n_vertices);
 struct Plan {
     std::array<char, kKindBytes> kind;
     int64_t frame_bytes = 0, keys_low = 0, keys_high = 0;  // K outside [low, high]: the next frame's plan is made anew
-    void fill(tg_frame &f) const {
+    void fill(tg_frame &f, int64_t n_vertices, int64_t n_triangles, int64_t max_layers) const {
         std::memset(&f, 0, sizeof f);
         std::memcpy(reinterpret_cast<char *>(&f) + offsetof(tg_frame, n_vertices), kind.data(), kKindBytes);
+        f.n_vertices = n_vertices;
+        f.n_triangles = n_triangles;
+        f.max_layers = max_layers;
     }
 };
-using PlanKey = std::array<int64_t, 12>;
+using PlanKey = std::array<int64_t, 10>;
+
+// As _round_count of the Python side: itself below 32, else up to a multiple of a sixteenth to a thirty-second of itself.
+int64_t round_count(int64_t n) {
+    int bits = 0;
+    for (int64_t m = n; m; m >>= 1) bits++;
+    const int64_t step = (int64_t)1 << std::max(bits - 5, 0);
+    return std::min<int64_t>((n + step - 1) / step * step, 0x7fffffff);
+}
 
 struct State {
     at::Tensor memory;
@@ -127,7 +141,7 @@ struct Frame : torch::CustomClassHolder {
     std::shared_ptr<const Plan> plan;
     std::shared_ptr<Status> status;
     at::Tensor image, depthmap, kept;
-    int64_t n_keys = 0;
+    int64_t n_keys = 0, max_layers = 0;
 };
 
 at::TensorOptions on(const at::Tensor &like, at::ScalarType type) { return at::TensorOptions().device(like.device()).dtype(type); }
@@ -137,7 +151,7 @@ bool render(Frame &frame, const std::shared_ptr<State> &state, void *stream, con
             const at::Tensor &colors, const at::Tensor &opacities) {
     Registry &r = registry();
     tg_frame f;
-    frame.plan->fill(f);
+    frame.plan->fill(f, vertices.size(0), indices.size(0), frame.max_layers);
     frame.image = at::empty({f.height, f.width, 4}, on(vertices, at::kFloat));
     frame.depthmap = at::empty({f.height, f.width}, on(vertices, at::kFloat));
     frame.kept = at::empty({f.kept_bytes}, on(vertices, at::kByte));
@@ -212,7 +226,7 @@ struct Render : torch::autograd::Function<Render> {
         const int64_t n = v.size(0);
         const at::Tensor gradients = at::empty({8 * n}, on(v, at::kFloat));  // (V,4) | (V,3) | (V,) behind each other
         tg_frame f;
-        frame.plan->fill(f);
+        frame.plan->fill(f, n, i.size(0), frame.max_layers);
         at::Tensor block;
         if (f.per_pixel_sort) block = at::empty({8 * n}, on(v, at::kFloat));
         f.vertices = v.data_ptr<float>();
@@ -268,9 +282,10 @@ PyObject *py_render(PyObject *, PyObject *const *args, Py_ssize_t n) {
     int64_t threshold_bits;
     std::memcpy(&threshold_bits, &threshold, sizeof threshold_bits);
     int64_t layers = PyLong_AsLongLong(args[11]);
-    const PlanKey key = {vertices.device().index(), n_vertices, n_triangles, PyLong_AsLongLong(args[4]), PyLong_AsLongLong(args[5]),
+    if (layers <= 0) layers = n_triangles + 1;  // no limit
+    const PlanKey key = {vertices.device().index(), round_count(n_triangles), PyLong_AsLongLong(args[4]), PyLong_AsLongLong(args[5]),
                          PyLong_AsLongLong(args[6]), PyLong_AsLongLong(args[7]), threshold_bits, args[10] == Py_True,
-                         layers <= 0 ? n_triangles + 1 : layers, backward, 0};
+                         layers == n_triangles + 1 ? 0 : layers, backward};
     if (PyErr_Occurred()) {  // an integer beyond 64 bits
         PyErr_Clear();
         Py_RETURN_NONE;
@@ -278,6 +293,7 @@ PyObject *py_render(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const c10::DeviceGuard guard(vertices.device());
     void *stream = c10::hip::getCurrentHIPStream(vertices.device().index()).stream();
     auto frame = c10::make_intrusive<Frame>();
+    frame->max_layers = layers;
     std::shared_ptr<State> state;
     {
         Registry &r = registry();
@@ -344,20 +360,20 @@ PyObject *py_bind(PyObject *, PyObject *args) {
     Py_RETURN_NONE;
 }
 
-// remember(key of eleven integers, plan bytes, frame bytes, keys_low, keys_high): a plan for frames of this kind
+// remember(key of ten integers, plan bytes, frame bytes, keys_low, keys_high): a plan for frames of this kind
 PyObject *py_remember(PyObject *, PyObject *args) {
     PlanKey key = {};
-    long long k[11], frame_bytes, low, high;
+    long long k[10], frame_bytes, low, high;
     const char *bytes;
     Py_ssize_t size;
-    if (!PyArg_ParseTuple(args, "(LLLLLLLLLLL)y#LLL", &k[0], &k[1], &k[2], &k[3], &k[4], &k[5], &k[6], &k[7], &k[8], &k[9], &k[10], &bytes,
-                          &size, &frame_bytes, &low, &high))
+    if (!PyArg_ParseTuple(args, "(LLLLLLLLLL)y#LLL", &k[0], &k[1], &k[2], &k[3], &k[4], &k[5], &k[6], &k[7], &k[8], &k[9], &bytes, &size,
+                          &frame_bytes, &low, &high))
         return nullptr;
     if ((size_t)size != kKindBytes) {
         PyErr_SetString(PyExc_ValueError, "the plan's constant part has another size");
         return nullptr;
     }
-    for (int j = 0; j < 11; j++) key[j] = k[j];
+    for (int j = 0; j < 10; j++) key[j] = k[j];
     auto plan = std::make_shared<Plan>();
     std::memcpy(plan->kind.data(), bytes, kKindBytes);
     plan->frame_bytes = frame_bytes;
