@@ -15,37 +15,44 @@ numbers bit for bit, without the hundreds of launches.
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _C, _lib
 
 
+_is_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+
+
 def _plain(t):
-    """Whether `t` is memory of a GPU that a kernel can read as it stands: no subclass, proxy or functorch wrapper, no
-    forward-mode tangent, no lazy negation or zero."""
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-            and t.device.type == "cuda" and t.layout is torch.strided and not t.is_neg() and not t._is_zerotensor()
-            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
+    """Whether `t` is memory of a GPU that a kernel can read as it stands: no subclass, proxy or functorch wrapper, no lazy
+    negation or zero, no forward-mode tangent."""
+    kind = type(t)
+    return ((kind is torch.Tensor or kind is torch.nn.Parameter) and t.is_cuda and not _is_wrapped(t) and t.layout is torch.strided
+            and not t.is_neg() and not t._is_zerotensor()
+            and (forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None))
 
 
 def _native(scalars, others=()):
     """Whether the library's kernels take these tensors: on one GPU, `scalars` of one of its scalar types, no gradient wanted.
     What records or transforms tensor operations (tracing, dispatch modes, vmap, jvp) gets tensor operations."""
-    if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0:
+    if torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() > 0:
         return False
-    tensors = (*scalars, *others)
-    if not all(_plain(t) for t in tensors):
-        return False
+    for t in (*scalars, *others):
+        if not _plain(t):
+            return False
     first = scalars[0]
-    if first.dtype not in (torch.float32, torch.float64) or any(t.dtype != first.dtype for t in scalars):
+    dtype, index, grad = first.dtype, first.get_device(), torch.is_grad_enabled()
+    if dtype is not torch.float32 and dtype is not torch.float64:
         return False
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-        return False
-    return all(t.device == first.device for t in tensors)
+    for t in scalars:
+        if t.dtype is not dtype or t.get_device() != index or (grad and t.requires_grad):
+            return False
+    return all(t.get_device() == index for t in others)
 
 
 def _native_rows(clip):
     """Whether these clip coordinates are rows the kernels read whole: (V,4), contiguous from a 16-byte boundary (or copied)."""
-    return clip.dim() == 2 and clip.shape[1] == 4 and (not clip.is_contiguous() or clip.data_ptr() % 16 == 0)
+    return clip.dim() == 2 and clip.size(1) == 4 and (clip.data_ptr() % 16 == 0 or not clip.is_contiguous())
 
 
 def perspective(fov_degrees, width, height, near=0.1, far=100.0, dtype=torch.float32, device=None):
