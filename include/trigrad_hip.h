@@ -233,7 +233,8 @@ int tg_build_tile_lists(const tg_real *records, const uint32_t *tri_offsets, int
  * the rest).
  *
  * frame: tg_bin_frame_workspace_bytes() bytes, 256-byte aligned, ZERO before the
- * first call that uses it; every call leaves it ready for the next.  It holds
+ * first call that uses it, and again after a call that returned an error; every
+ * call that did not leaves it ready for the next.  It holds
  * what the two launches hand each other (per-triangle records as tg_bin_setup
  * makes them) and what calls share.  epoch: its low 30 bits must not be 0,
  * must differ from those of every earlier call on this frame state since it

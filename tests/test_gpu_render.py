@@ -1028,3 +1028,38 @@ def test_key_buffers_of_a_size_seen_before(cuda):
     for table in (_C._frame_key_hints, _C._frame_size_hints, _C._frame_plans):
         assert len(table) <= _C._MAX_REMEMBERED
     trigrad_amd.verify_frames()
+
+
+@pytest.mark.parametrize("keep", [True, False])
+@pytest.mark.parametrize("n_triangles", [40, 3000])
+def test_order_pool_of_a_first_frame_is_made_for_its_keys(n_triangles, keep, cuda, oracle, monkeypatch):
+    """A frame without a layer limit keeps a row of a tile's pixels per key.  The first one of its kind and size counts its
+    keys before it takes the memory; ORDER_POOL_MAX_BYTES = 0 keeps nothing and gives the same gradients."""
+    import torch
+    import trigrad_amd
+    from trigrad_amd import _C
+    import scenes as S
+    W, H = 223, 117 + n_triangles % 7  # of no other test
+    scene = S.random_soup(n_triangles, W, H, seed=4, sigma_px=7.0, opacity=(0.02, 0.2))
+    d = to_device(scene, cuda)
+    if not keep:
+        monkeypatch.setattr(_C, "ORDER_POOL_MAX_BYTES", 0)
+    for table in (_C._frame_key_hints, _C._frame_size_hints):
+        for key in [k for k in table if k[-4:-2] == (W, H)]:
+            del table[key]
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], W, H, 16, 16, 1 / 256, True, n_triangles + 1)
+    image, depthmap, kept, frame = _C.frame_forward(*args)
+    pool = _C._round_capacity(frame.n_keys) * 256 * 2
+    assert frame.plan.capacity == (_C._round_capacity(frame.n_keys) if keep else 3 * n_triangles + 65536)
+    assert pool < kept.numel() < pool + 400_000 + 44 * n_triangles + 28 * W * H if keep else kept.numel() < pool + 700_000
+    want = oracle.render(*(scene[k] for k in ("vertices", "indices", "colors", "opacities")), W, H, 16, 16, 1 / 256, True, n_triangles + 1)
+    assert np.array_equal(image.cpu().numpy(), want["image"])
+    gi, gd = _grad_inputs(scene, 5, False)
+    wanted = oracle.render_backward(gi, gd, *(scene[k] for k in ("vertices", "indices", "colors", "opacities")), want, W, H, 16, 16, True,
+                                    n_triangles + 1, magnitudes=True)
+    leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+    for _ in range(2):
+        image, _ = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], W, H, max_layers=-1)
+        grads = torch.autograd.grad((image,), leaves, (torch.from_numpy(gi).to(cuda),))
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), grads, wanted[:3], wanted[3:]):
+            assert_gradients_close(f"pool of a first frame: {label}", g.cpu().numpy(), w, mag)

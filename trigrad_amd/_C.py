@@ -100,7 +100,7 @@ MAX_SAVED_LAYERS = 32  # TG_MAX_SAVED_LAYERS of the C header
 # selecting the fragments again.  False trades the memory for the re-selection.
 SAVE_BLEND_ORDER = True
 # With more layers than that the order goes to a pool that holds one word per (pixel, entry of its tile's list)
-# (tg_order_pool_words), as long as the pool takes no more bytes than this; else the backward pass selects again.
+# (tg_order_pool_words), as long as the pool takes no more bytes than this; else (0: always) the backward pass selects again.
 ORDER_POOL_MAX_BYTES = 4 << 30
 # Without per_pixel_sort the forward pass saves which list entries cover which pixel (one bit per pair it
 # looked at) and the backward pass reads that back instead of repeating the inside tests.
@@ -800,7 +800,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
             if not per_pixel_sort:
                 flags |= _FRAME_HIT_MASKS if SAVE_HIT_MASKS else 0
             elif SAVE_BLEND_ORDER:
-                flags |= _FRAME_ORDER_PLANES if max_layers <= MAX_SAVED_LAYERS else _FRAME_ORDER_POOL
+                flags |= _FRAME_ORDER_PLANES if max_layers <= MAX_SAVED_LAYERS else _FRAME_ORDER_POOL if ORDER_POOL_MAX_BYTES > 0 else 0
         hint_key = (dev.index, n_triangles, width, height, tile_width, tile_height)
         size_key = (dev.index, width, height, tile_width, tile_height)
 
@@ -814,6 +814,9 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
         if expected is None and size_key in _frame_size_hints:
             keys, triangles = _frame_size_hints[size_key]  # another number of triangles: about as many keys each
             expected = -(-keys * n_triangles // triangles)
+        # An order pool takes a row of a tile's pixels per key: it is made for counted keys, not for a guess.  The first
+        # frame of its kind and size counts them in a binning of its own.
+        counting = expected is None and bool(flags & _FRAME_ORDER_POOL)
         if expected is None:
             expected, capacity = 2 * n_triangles, min(3 * n_triangles + 65536, (1 << 30) - 1)
         else:
@@ -823,7 +826,10 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
         stream = _raw_stream(dev)
         frame = Frame()
         while True:
-            plan = _plan_for(kind_for(expected, capacity))
+            kind = kind_for(expected, capacity)
+            if counting:
+                kind = (*kind[:9], kind[9] & ~_FRAME_ORDER_POOL, kind[10])
+            plan = _plan_for(kind)
             kept = torch.empty((plan.kept_bytes,), dtype=torch.uint8, device=dev)
             scratch = torch.empty((plan.scratch_bytes,), dtype=torch.uint8, device=dev)
             _frame_counter += 1
@@ -833,8 +839,8 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
             c_call = (C.c_char * _FRAME_BYTES).from_buffer(call)
             with _frame_launches(dev.index, stream):  # one frame at a time on a stream's state
                 state, state_bytes, epoch = _next_frame_state(dev, plan.frame_bytes)
-                for phases, stage in _FRAME_UNTIMED if timer is None else _FRAME_TIMED:
-                    if timer is not None:
+                for phases, stage in _FRAME_COUNTING if counting else _FRAME_UNTIMED if timer is None else _FRAME_TIMED:
+                    if timer is not None and not counting:
                         timer.start(stage)
                     _FRAME_CALL.pack_into(call, 0, vertices.data_ptr(), indices.data_ptr(), colors.data_ptr(), opacities.data_ptr(),
                                           image.data_ptr(), depthmap.data_ptr(), kept.data_ptr(), scratch.data_ptr(),
@@ -845,7 +851,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
                         status.keep_until_idle(dev)
                         _lib.check(code, "tg_frame_forward")
             n_keys, counted = _FRAME_RESULT.unpack_from(call, _FRAME_CALL.size)
-            if counted == 1 and n_keys <= capacity:
+            if counted == 1 and n_keys <= capacity and not counting:
                 break
             torch.cuda.current_stream(dev).synchronize()  # the kernels are done with the status words
             if counted != 1:
@@ -856,7 +862,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
             else:
                 if n_keys >= 1 << 30:
                     raise RuntimeError(f"tg_frame_forward: {n_keys} (tile, triangle) pairs, the sort takes 2^30 - 1")
-                capacity = _round_capacity(n_keys)
+                counting, expected, capacity = False, n_keys, _round_capacity(n_keys)
         if hint_key in _frame_key_hints:
             _frame_key_hints[hint_key] = n_keys
         else:
@@ -872,6 +878,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
 
 
 _FRAME_UNTIMED = ((_FRAME_BIN | _FRAME_LISTS | _FRAME_RASTER | _FRAME_WAIT, None),)
+_FRAME_COUNTING = ((_FRAME_BIN | _FRAME_WAIT, None),)
 # the bary matrices are made where the triangles are read anyway, by the binning
 _FRAME_TIMED = ((_FRAME_BIN, "per_tile_lists"), (_FRAME_LISTS, "sorting"), (0, "bary_transforms"), (_FRAME_RASTER | _FRAME_WAIT, "rasterization"))
 

@@ -136,6 +136,11 @@ def render(
         opacities : (N,) vertex opacities
         per_pixel_sort : order fragments per pixel (True) or per tile (False)
         max_layers : maximum number of fragments composited per pixel, <= 0 for no limit
+            With per_pixel_sort and more than 32 layers (or no limit) a frame that is differentiated keeps its blend order
+            until the backward pass: 2 bytes (4 with more than 65535 triangles) per (tile, triangle) pair and pixel of a
+            tile, where the pairs are those of the last such frame and an eighth more.  What would take more than
+            trigrad_amd._C.ORDER_POOL_MAX_BYTES (4 GiB; 0: keep none) is not kept, and the backward pass selects the
+            fragments again, several times slower.
 
     Returns:
         image : (height, width, 4); channel 3 holds the remaining transmittance, not opacity
