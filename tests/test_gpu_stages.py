@@ -385,3 +385,24 @@ def test_key_buffers_smaller_than_the_frame_needs(cuda, oracle):
     again = trigrad_amd.render(d["vertices"], d["indices"], d["colors"], d["opacities"], W, H, tw, th, 1 / 256, False, False, -1)[0]
     assert torch.equal(good, again)
     assert _C._key_count_hint[cuda.index] == K
+
+
+def test_frame_without_triangles_leaves_the_state_ready(cuda, oracle):
+    """A binning call without triangles between others: the digit totals it has to clear for the next one are cleared."""
+    import torch
+    from trigrad_amd import _C
+    scene, tw, th = SCENES["soup_varying_w"]()
+    W, H = scene["width"], scene["height"]
+    d = to_device(scene, cuda)
+    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], W, H, tw, th, 1 / 256, True, 1)
+    no_triangles = torch.empty((0, 3), dtype=torch.int32, device=cuda)
+    for empty_calls in (0, 1, 0, 2, 1, 0):
+        for _ in range(empty_calls):
+            b = _C.bin_frame(d["vertices"], no_triangles, W, H, tw, th)
+            assert b["total_and_status"].tolist()[0] == 0
+        b = _C.bin_frame(d["vertices"], d["indices"], W, H, tw, th, capacity=100_000)
+        K = int(b["total_and_status"][0].item())
+        keys, ids, status, offsets = _C.build_frame_lists(b, K)
+        assert int(status.item()) == 0
+        np.testing.assert_array_equal(ids.cpu().numpy(), want["sorted_ids"])
+        np.testing.assert_array_equal(offsets.cpu().numpy(), want["offsets"])

@@ -1161,7 +1161,9 @@ static FusedFrame fused_frame(void *base, int64_t n_triangles, int64_t key_capac
 }
 uint32_t *fused_frame_totals(void *frame, uint32_t epoch) { return (uint32_t *)frame + (epoch & 1u) * (kEmitDigitPasses * kRadix); }
 
-__global__ void bin_frame_empty_kernel(uint32_t *total_and_status, uint32_t *clear_word) {
+// A frame without triangles: K = 0, and the other set of digit totals is cleared for the next call as frame_scan_kernel does.
+__global__ void bin_frame_empty_kernel(uint32_t *total_and_status, uint32_t *totals_next, uint32_t *clear_word) {
+    for (int i = threadIdx.x; i < kEmitDigitPasses * kRadix; i += blockDim.x) totals_next[i] = 0;
     if (threadIdx.x == 0) {
         total_and_status[0] = 0;
         if (clear_word) *clear_word = 0;
@@ -1207,7 +1209,7 @@ int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indic
     }
     hipStream_t s = (hipStream_t)stream;
     if (n_triangles == 0) {
-        TG_LAUNCH(bin_frame_empty_kernel, dim3(1), dim3(64), 0, s, total_and_status, clear_word);
+        TG_LAUNCH(bin_frame_empty_kernel, dim3(1), dim3(64), 0, s, total_and_status, fused_frame_totals(frame, epoch + 1), clear_word);
         return check_launch("bin_frame_empty_kernel");
     }
     const int n_scan_tiles = (int)ceil_div64(n_triangles, kScanTile);
