@@ -256,3 +256,14 @@ def test_buffers_for_a_rounded_number_of_triangles_serve_every_smaller_one(flags
                      for k in (n, _C._round_count(n))]
             for field in ("kept_bytes", "scratch_bytes", "frame_bytes"):
                 assert getattr(sizes[0], field) <= getattr(sizes[1], field)
+
+
+@pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
+def test_state_words_of_the_frame_scan_keep_their_place(few, many):
+    """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more
+    triangles the state grows by what a triangle takes behind it (4 bytes of offset, 48 of record), and by nothing else."""
+    from trigrad_amd import _lib
+    lib = _lib.load(32)
+    grown = lib.tg_bin_frame_workspace_bytes(many, 1000, 640, 480, 16, 16) - lib.tg_bin_frame_workspace_bytes(few, 1000, 640, 480, 16, 16)
+    up = lambda n: -(-n // 256) * 256
+    assert grown == up(4 * many) - up(4 * few) + up(48 * many) - up(48 * few)

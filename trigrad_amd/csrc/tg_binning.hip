@@ -1150,7 +1150,10 @@ static FusedFrame fused_frame(void *base, int64_t n_triangles, int64_t key_capac
     const auto take = [&](size_t bytes) { char *at = p + o; o = (o + bytes + 255) & ~(size_t)255; return at; };
     f.totals = (uint32_t *)take((size_t)kFrameTotalsWords * 4);
     f.ticket = (uint32_t *)take(4);
-    f.states = (uint64_t *)take((size_t)(ceil_div64(n_triangles, kScanTile) + 1) * 8);
+    // The scan's state words are told from an earlier call's by their stamp, so nothing else may ever lie where they do: their
+    // place must not depend on the number of triangles, which differs from call to call.  Room for 2^24 triangles (64 KB), or
+    // for any number where there are more.
+    f.states = (uint64_t *)take((size_t)((n_triangles <= 1 << 24 ? 1 << 24 : 1ll << 31) / kScanTile + 1) * 8);
     f.edges = (real *)take((size_t)(tiles_x + tiles_y + 2) * sizeof(real));
     f.head_capacity = (uint32_t)(key_capacity / kEmitChunk + 2);
     f.heads = (uint32_t *)take((size_t)f.head_capacity * 4);
