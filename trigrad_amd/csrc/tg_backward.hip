@@ -822,8 +822,8 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
     int n = 0;
     if (p.valid) {
         st = load_back_state(g, p);
-        n = min(g.ends[p.index], a.max_layers);  // render.cu:642
-        n = min(n, order_rows(g.order, a, end - start));  // fewer only where a NaN depth had the list blended more than once
+        // render.cu:642; fewer than were blended only where a NaN depth had the list blended more than once
+        n = min(g.ends[p.index], min(a.max_layers, order_rows(g.order, a, end - start)));
     }
     const int64_t plane = order_stride(g.order, a);
     const bool long_list = end - start > kShortList;  // then the positions' high halves were saved as well

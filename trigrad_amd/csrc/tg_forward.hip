@@ -214,6 +214,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     const int64_t order_step = order_stride(out.order, a);
     const int64_t order_at = order_first(out.order, p, start, blockIdx.z * blockDim.x + threadIdx.x);
 
+    const int rows_kept = out.order.low ? order_rows(out.order, a, end - start) : 0;
     PixelState s;
     real last_depth = -__builtin_inff();  // render.cu:585-586
     int last_j = -1;  // list positions count from the tile's start
@@ -365,7 +366,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                         real b0, b1, b2;
                         bary_apply(r[u].m, p.px, p.py, b0, b1, b2);
                         if (!bary_inside(b0, b1, b2)) continue;  // cannot happen: the selection tested it
-                        if (out.order.low && s.blended < order_rows(out.order, a, end - start)) {
+                        if (s.blended < rows_kept) {
                             const int64_t at = order_at + (int64_t)s.blended * order_step;
                             const int rel = tk.j(i0 + u);
                             out.order.low[at] = (uint16_t)rel;
