@@ -157,6 +157,18 @@ def test_crowds_of_small_triangles_match_oracle(n, width, height, tw, th, mode, 
     _check_forward(f"crowd {n}/{tw}x{th}/{mode}", want, got, (th, tw))
 
 
+@pytest.mark.parametrize("mode", ["A_default", "B_unlimited"])
+@pytest.mark.parametrize("n", [1023, 1024, 1025])
+def test_small_triangles_in_lists_around_1024_entries(n, mode, cuda, oracle):
+    """Lists of 1024 entries and more have their small triangles tested lane by lane, shorter ones by broadcast."""
+    import scenes as S
+    scene = S.random_soup(n, 16, 16, seed=n, sigma_px=0.7, opacity=(0.02, 0.2), varying_w=True)
+    scene["vertices"][:, :2] *= 0.6
+    _, want, got, _ = _forward_both(scene, 16, 16, MODES[mode], cuda, oracle)
+    assert np.diff(want["offsets"]).tolist() == [n]
+    _check_forward(f"list of {n}/{mode}", want, got, (16, 16))
+
+
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
 def test_more_long_tiles_than_slots(mode, cuda, monkeypatch):
     """Some 400 tiles with long lists, of which 128 are started first: the frame is that of the stage-by-stage route, which

@@ -713,11 +713,11 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
             __syncthreads();
             for (int e = tid; e < nb; e += blockDim.x) {
                 gather_depth(a, batch + e, s_rec[e]);
-                s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent));
+                s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, end - start));
             }
             __syncthreads();
             uint64_t m[kBatch / kWave];
-            batch_hit_mask<kBatch / kWave>(a, s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
+            batch_hit_mask<kBatch / kWave>(s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
             if (!want) {
 #pragma unroll
                 for (int wd = 0; wd < kBatch / kWave; wd++) m[wd] = 0;

@@ -123,12 +123,12 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forwa
         const int nb = min(kBatch, end - batch);
         for (int e = tid; e < nb; e += blockDim.x) {
             gather_blend(a, batch + e, s_rec[e]);
-            s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent));
+            s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, end - start));
         }
         __syncthreads();
         // 1. inside tests; a lane keeps its hits as a 256-bit mask
         uint64_t m[kBatch / kWave];
-        batch_hit_mask<kBatch / kWave>(a, s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
+        batch_hit_mask<kBatch / kWave>(s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
         if (!running) {
 #pragma unroll
             for (int wd = 0; wd < kBatch / kWave; wd++) m[wd] = 0;
@@ -274,12 +274,12 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 const int e = kInTurn ? mine : tid;
                 const DepthRecord r = next.record();
                 s_rec[e] = r;
-                s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves) | small_entry(a, r.extent));
+                s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves) | small_entry(a, r.extent, end - start));
             }
             if (!kInTurn && !ahead) {
                 for (int e = tid; e < nb; e += blockDim.x) {
                     gather_depth(a, batch + e, s_rec[e]);
-                    s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent));
+                    s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, end - start));
                 }
             }
             __syncthreads();
@@ -300,7 +300,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
             // inside tests into a per-lane mask, then every lane visits its own hits in
             // list order (the order insert_sorted_topk sees them in the reference)
             uint64_t m[kStage / kWave];
-            batch_hit_mask<kStage / kWave>(a, s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
+            batch_hit_mask<kStage / kWave>(s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
             if (!want) {
 #pragma unroll
                 for (int wd = 0; wd < kStage / kWave; wd++) m[wd] = 0;

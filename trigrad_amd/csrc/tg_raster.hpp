@@ -383,20 +383,28 @@ __device__ __forceinline__ uint64_t wave_candidates(const uint8_t *s_touch, int 
 }
 
 // Entries whose vertices span less than this many pixel rows are small, and are tested the other way round (lane = entry,
-// small_entry_hits) where a wave's 64 entries hold at least TG_SMALL_MIN of them.  That costs about as much as 20 tests by
-// broadcast whatever their number; below it the broadcast wins, and with 10 instead of 20 a frame of mixed sizes (10^6
-// triangles, mean edge 4 pixels) loses 10 % in per-pixel order and 30 % in tile order.  Entries of 6 or 12 rows make
-// the tallest lane's rows the whole wave's time (tile order, the same frame: 213 -> 218 -> 249 us).
+// small_entry_hits) where the tile's list has TG_SMALL_LIST entries or more, a wave's pixels are a square of 8 x 8, and 64
+// entries hold at least TG_SMALL_MIN of them.  That costs about as much as 20 tests by broadcast whatever their number; below
+// it the broadcast wins, and with 10 instead of 20 a frame of mixed sizes (10^6 triangles, mean edge 4 pixels) loses 10 % in
+// per-pixel order and 30 % in tile order.  Entries of 6 or 12 rows make the tallest lane's rows the whole wave's time (tile
+// order, the same frame: 213 -> 218 -> 249 us).
+// What is gained is time that a tile with a long list spends alone on its CU, waiting for LDS reads.  A list of hundreds runs
+// among others on a chip full of instructions and loses: tile order, with and without, 10^6 triangles of 1.5 pixels 172 and
+// 140 us, an icosphere of 1.3 million at 1920 x 1080 325 and 262; a mesh with a list of 5500 367 and 529.  From 256 or 512
+// entries on: 10 to 25 % slower on the icosphere; from 2048 on: 5 % there in per-pixel order.
 #ifndef TG_SMALL_ROWS
 #define TG_SMALL_ROWS 4.0f
 #endif
 #ifndef TG_SMALL_MIN
 #define TG_SMALL_MIN 20
 #endif
-constexpr int kSmallMin = TG_SMALL_MIN;
-constexpr uint32_t kSmallEntry = 0x80;  // flag in an entry's s_touch byte, next to the waves it touches
-__device__ __forceinline__ uint32_t small_entry(const RasterArgs &a, real extent) {
-    return extent * (real)a.H < (real)(2.0f * TG_SMALL_ROWS) ? kSmallEntry : 0u;  // NaN: not small
+#ifndef TG_SMALL_LIST
+#define TG_SMALL_LIST 1024
+#endif
+constexpr int kSmallMin = TG_SMALL_MIN, kSmallList = TG_SMALL_LIST;
+constexpr uint32_t kSmallEntry = 0x80;  // flag in an entry's s_touch byte, next to the waves it touches: to be tested lane by lane
+__device__ __forceinline__ uint32_t small_entry(const RasterArgs &a, real extent, int list_length) {
+    return ((a.tw | a.th) & 7) == 0 && list_length >= kSmallList && extent * (real)a.H < (real)(2.0f * TG_SMALL_ROWS) ? kSmallEntry : 0u;  // NaN: not small
 }
 
 // bary_inside in two operations: a minimum passes NaNs by, as the three comparisons there do.
@@ -467,7 +475,7 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
 // the result is that of 64 tests per entry.  -> bit e: entry e covers the calling lane's pixel.
 // A test by broadcast costs about 20 vector instructions per entry for all 64 pixels and waits for its LDS reads (200
 // clocks where a long list leaves its tile alone on the CU); here 64 entries cost 250 instructions and 110 per row of the
-// tallest, all from registers.  500 000 triangles of a mesh, 500 x 500, tile order (longest list 5500 entries): 505 -> 378 us.
+// tallest, all from registers.  500 000 triangles of a mesh, 500 x 500, tile order (longest list 5500 entries): 529 -> 367 us.
 template <typename Rec>
 __device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine, const WaveRect &rect, real px, real py) {
     const int lane = threadIdx.x & (kWave - 1);
@@ -508,12 +516,11 @@ __device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine
 // result (word e / 64) is set when record e covers the pixel.  Only records that
 // can touch the wave's pixels are looked at: all lanes of the wave read the same
 // record at the same time (LDS broadcast), or, where 20 or more of 64 entries are
-// small and the wave's pixels are a square, those are tested lane by lane.
+// marked as small, those are tested lane by lane.
 // Rec must have a member m[9].
 template <int kWords, typename Rec>
-__device__ __forceinline__ void batch_hit_mask(const RasterArgs &a, const Rec *s_rec, const uint8_t *s_touch, const WaveRect *s_rects, int nb,
-                                               int wave, real px, real py, uint64_t m[kWords]) {
-    const bool square = ((a.tw | a.th) & 7) == 0;
+__device__ __forceinline__ void batch_hit_mask(const Rec *s_rec, const uint8_t *s_touch, const WaveRect *s_rects, int nb, int wave,
+                                               real px, real py, uint64_t m[kWords]) {
 #pragma unroll
     for (int wd = 0; wd < kWords; wd++) {
         const int e = wd * kWave + (threadIdx.x & (kWave - 1));
@@ -523,7 +530,8 @@ __device__ __forceinline__ void batch_hit_mask(const RasterArgs &a, const Rec *s
         uint64_t hits = 0;
         const bool is_small = candidate && (touch & kSmallEntry);
         const uint64_t small = __builtin_amdgcn_ballot_w64(is_small);
-        if (square && __builtin_popcountll(small) >= kSmallMin) {  // wave-uniform
+        // wave-uniform; `likely` lays the tests out in line, which long lists in tile order feel (a list of 5500: 382 -> 367 us)
+        if (__builtin_expect(__builtin_popcountll(small) >= kSmallMin, 1)) {
             hits = small_entry_hits(s_rec + wd * kWave, is_small, s_rects[wave], px, py);
             todo &= ~small;
         }
