@@ -158,15 +158,25 @@ def test_crowds_of_small_triangles_match_oracle(n, width, height, tw, th, mode, 
 
 
 @pytest.mark.parametrize("mode", ["A_default", "B_unlimited"])
-@pytest.mark.parametrize("n", [1023, 1024, 1025])
-def test_small_triangles_in_lists_around_1024_entries(n, mode, cuda, oracle):
-    """Lists of 1024 entries and more have their small triangles tested lane by lane, shorter ones by broadcast."""
+@pytest.mark.parametrize("n,others,width,lane_by_lane", [(255, 0, 272, False), (256, 0, 272, True), (400, 28_000, 272, False),
+                                                         (1023, 70_000, 272, False), (1024, 70_000, 272, True), (90, 0, 16, True),
+                                                         (90, 15_000, 256, True)])
+def test_small_triangles_around_the_edges_of_their_rule(n, others, width, lane_by_lane, mode, cuda, oracle):
+    """Which lists have their small triangles tested lane by lane: of 1024 entries, or of 256 and four times the mean, in frames
+    with more than 256 tiles (here 272), and every list in others.  One tile with a list of n, the rest spread evenly."""
     import scenes as S
-    scene = S.random_soup(n, 16, 16, seed=n, sigma_px=0.7, opacity=(0.02, 0.2), varying_w=True)
-    scene["vertices"][:, :2] *= 0.6
+    height = 16 if width == 16 else 256
+    scene = S.random_soup(n + others, width, height, seed=n, sigma_px=0.7, opacity=(0.02, 0.2), varying_w=True)
+    v = scene["vertices"].reshape(n + others, 3, 4)
+    v[:n, :, 0] = (v[:n, :, 0] * 0.4 + 1.0) * 16 / width - 1.0
+    v[:n, :, 1] = (v[:n, :, 1] * 0.4 + 1.0) * 16 / height - 1.0
+    if others:  # none in the first column of tiles
+        v[n:, :, 0] = np.where(v[n:, :, 0] < 33 / width * 2 - 1, v[n:, :, 0] * 0.5 + 0.4, v[n:, :, 0])
     _, want, got, _ = _forward_both(scene, 16, 16, MODES[mode], cuda, oracle)
-    assert np.diff(want["offsets"]).tolist() == [n]
-    _check_forward(f"list of {n}/{mode}", want, got, (16, 16))
+    lengths = np.diff(want["offsets"])
+    assert lengths[0] == n and lengths.size == (1 if width == 16 else width // 16 * 16)
+    assert (lengths.size <= 256 or n >= 1024 or (n >= 256 and n >= 4 * lengths.mean())) == lane_by_lane
+    _check_forward(f"{n} small of {others}/{mode}", want, got, (16, 16))
 
 
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])

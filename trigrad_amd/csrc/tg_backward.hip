@@ -689,6 +689,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);
     publish_wave_rect(p, s_rects);
+    const bool tests_small = tests_small_entries(a, end - start, (int)(gridDim.x * gridDim.y));
     const int n_acc = min(end - start, kAccWindow);
     for (int i = tid; i < n_acc * kTerms; i += blockDim.x) s_acc[i] = 0.0f;
 
@@ -713,7 +714,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
             __syncthreads();
             for (int e = tid; e < nb; e += blockDim.x) {
                 gather_depth(a, batch + e, s_rec[e]);
-                s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, end - start));
+                s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, tests_small));
             }
             __syncthreads();
             uint64_t m[kBatch / kWave];

@@ -113,6 +113,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forwa
     const int tile = tile_id.index;
     const PixelCoord p = pixel_of_thread(a, tile_id);
     publish_wave_rect(p, s_rects);
+    const bool tests_small = tests_small_entries(a, end - start, (int)(gridDim.x * (gridDim.y - out.long_rows)));
     uint64_t *const masks = out.hit_masks ? out.hit_masks + hit_mask_head_words(out.long_rows) : nullptr;
 
     PixelState s;
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forwa
         const int nb = min(kBatch, end - batch);
         for (int e = tid; e < nb; e += blockDim.x) {
             gather_blend(a, batch + e, s_rec[e]);
-            s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, end - start));
+            s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, tests_small));
         }
         __syncthreads();
         // 1. inside tests; a lane keeps its hits as a 256-bit mask
@@ -195,7 +196,7 @@ constexpr int kLongListGroups = 256;    // workgroups that look for the tiles wi
 // start) is kept.  With uint16_t the candidate lists of a 16x16 tile take 48 KB instead of 64 KB, which
 // together with 64 staged entries lets a CU hold three workgroups instead of two.
 template <int kStage, typename Pos, bool kInTurn>  // kStage: list entries staged per batch
-__device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const ForwardOut &out, int tile_x, int tile_y, int tiles_x,
+__device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const ForwardOut &out, int tile_x, int tile_y, int tiles_x, int n_tiles,
                                                  unsigned char *s_dyn, uint8_t *s_touch, WaveRect *s_rects) {
     const int n_threads = blockDim.x;
     DepthRecord *s_rec = reinterpret_cast<DepthRecord *>(s_dyn);
@@ -211,6 +212,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_x, tile_y);
     publish_wave_rect(p, s_rects);
+    const bool tests_small = tests_small_entries(a, end - start, n_tiles);
     const int64_t order_step = order_stride(out.order, a);
     const int64_t order_at = order_first(out.order, p, start, blockIdx.z * blockDim.x + threadIdx.x);
 
@@ -274,12 +276,12 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 const int e = kInTurn ? mine : tid;
                 const DepthRecord r = next.record();
                 s_rec[e] = r;
-                s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves) | small_entry(a, r.extent, end - start));
+                s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves) | small_entry(a, r.extent, tests_small));
             }
             if (!kInTurn && !ahead) {
                 for (int e = tid; e < nb; e += blockDim.x) {
                     gather_depth(a, batch + e, s_rec[e]);
-                    s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, end - start));
+                    s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, tests_small));
                 }
             }
             __syncthreads();
@@ -406,7 +408,7 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
         return;
     }
     if (!mine || (sizeof(Pos) < sizeof(int) && end - start > kShortList)) return;
-    pixel_order_tile<kStage, Pos, kInTurn>(a, out, tile.x, tile.y, gridDim.x, s_dyn, s_touch, s_rects);
+    pixel_order_tile<kStage, Pos, kInTurn>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
 }
 
 // The tiles whose lists are longer than kShortList, with int positions: few or none, so a small grid
@@ -436,7 +438,7 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
                 const int tile = base + w * kWave + __builtin_ctzll(todo);
                 todo &= todo - 1;
                 __syncthreads();  // the tile before is done with the LDS
-                pixel_order_tile<kSelectBatch, int, false>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, s_dyn, s_touch, s_rects);
+                pixel_order_tile<kSelectBatch, int, false>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, tiles, s_dyn, s_touch, s_rects);
             }
         }
     }

@@ -383,28 +383,32 @@ __device__ __forceinline__ uint64_t wave_candidates(const uint8_t *s_touch, int 
 }
 
 // Entries whose vertices span less than this many pixel rows are small, and are tested the other way round (lane = entry,
-// small_entry_hits) where the tile's list has TG_SMALL_LIST entries or more, a wave's pixels are a square of 8 x 8, and 64
-// entries hold at least TG_SMALL_MIN of them.  That costs about as much as 20 tests by broadcast whatever their number; below
-// it the broadcast wins, and with 10 instead of 20 a frame of mixed sizes (10^6 triangles, mean edge 4 pixels) loses 10 % in
-// per-pixel order and 30 % in tile order.  Entries of 6 or 12 rows make the tallest lane's rows the whole wave's time (tile
-// order, the same frame: 213 -> 218 -> 249 us).
-// What is gained is time that a tile with a long list spends alone on its CU, waiting for LDS reads.  A list of hundreds runs
-// among others on a chip full of instructions and loses: tile order, with and without, 10^6 triangles of 1.5 pixels 172 and
-// 140 us, an icosphere of 1.3 million at 1920 x 1080 325 and 262; a mesh with a list of 5500 367 and 529.  From 256 or 512
-// entries on: 10 to 25 % slower on the icosphere; from 2048 on: 5 % there in per-pixel order.
+// small_entry_hits) in a tile whose list is long (tests_small_entries), where 64 entries hold at least TG_SMALL_MIN of them.
+// That costs about as much as 20 tests by broadcast whatever their number; below it the broadcast wins, and with 10 instead of
+// 20 a frame of mixed sizes (10^6 triangles, mean edge 4 pixels) loses 10 % in per-pixel order and 30 % in tile order.  Entries
+// of 6 or 12 rows make the tallest lane's rows the whole wave's time (tile order, the same frame: 213 -> 218 -> 249 us).
 #ifndef TG_SMALL_ROWS
 #define TG_SMALL_ROWS 4.0f
 #endif
 #ifndef TG_SMALL_MIN
 #define TG_SMALL_MIN 20
 #endif
-#ifndef TG_SMALL_LIST
-#define TG_SMALL_LIST 1024
-#endif
-constexpr int kSmallMin = TG_SMALL_MIN, kSmallList = TG_SMALL_LIST;
+constexpr int kSmallMin = TG_SMALL_MIN;
 constexpr uint32_t kSmallEntry = 0x80;  // flag in an entry's s_touch byte, next to the waves it touches: to be tested lane by lane
-__device__ __forceinline__ uint32_t small_entry(const RasterArgs &a, real extent, int list_length) {
-    return ((a.tw | a.th) & 7) == 0 && list_length >= kSmallList && extent * (real)a.H < (real)(2.0f * TG_SMALL_ROWS) ? kSmallEntry : 0u;  // NaN: not small
+// Whether a tile's small entries are tested lane by lane.  What that gains is the time of a list that the launch waits for,
+// alone on its CU with the latency of its LDS reads; a list like all others runs among them on a chip full of instructions,
+// and loses.  So: a wave's pixels are a square of 8 x 8, and the frame has no more tiles than CUs (a list of 550 on 64 tiles:
+// 47 us with, 65 without), or the list has 1024 entries (5500 on 1024 tiles, tile order: 367 and 529), or 256 and four times
+// the mean (650 on 384 tiles with a mean of 85: 60 and 84).  Without the last two conditions, and with them, in tile order: 10^6
+// triangles of 1.5 pixels 172 and 140 us, an icosphere of 1.3 million at 1920 x 1080 325 and 270 (three times the mean 283).
+constexpr int kFewTiles = 256, kLongSmallList = 1024, kShortSmallList = 256, kSmallListMeans = 4;
+__device__ __forceinline__ bool tests_small_entries(const RasterArgs &a, int list_length, int n_tiles) {
+    if ((a.tw | a.th) & 7) return false;
+    if (n_tiles <= kFewTiles || list_length >= kLongSmallList) return true;
+    return list_length >= kShortSmallList && (int64_t)list_length * n_tiles >= (int64_t)kSmallListMeans * a.offsets[n_tiles];
+}
+__device__ __forceinline__ uint32_t small_entry(const RasterArgs &a, real extent, bool tests_small) {
+    return tests_small && extent * (real)a.H < (real)(2.0f * TG_SMALL_ROWS) ? kSmallEntry : 0u;  // NaN: not small
 }
 
 // bary_inside in two operations: a minimum passes NaNs by, as the three comparisons there do.
