@@ -281,6 +281,25 @@ def test_sort_tile_lists_at_the_edges_of_its_rules(longest, cuda):
     np.testing.assert_array_equal(sv.cpu().numpy(), order.astype(np.int32))
 
 
+@pytest.mark.parametrize("n_tiles,typical", [(2049, 1100), (2048, 1100), (2049, 500), (2049, 2060)])
+def test_sort_of_many_lists_around_the_workgroups_two_sizes(n_tiles, typical, cuda):
+    """Most lists of 512 to 2048 pairs, in more than 2048 tiles: sorted by the small kernel up to 2048; else up to 1024."""
+    from trigrad_amd import _C
+    import torch
+    rng = np.random.default_rng(n_tiles + typical)
+    lengths = rng.integers(typical - 20, typical + 20, n_tiles)
+    lengths[rng.choice(n_tiles, 60, replace=False)] = np.repeat([0, 1, 512, 513, 1024, 1025, 2047, 2048, 2049, 4000], 6)
+    tiles = rng.permutation(np.repeat(np.arange(n_tiles, dtype=np.uint64), lengths))
+    keys = (tiles << np.uint64(32)) | rng.integers(0, 1 << 32, tiles.size, dtype=np.uint64)
+    values = np.arange(tiles.size, dtype=np.int32)
+    k, v, status, offsets = _C.sort_tile_lists(torch.from_numpy(keys.view(np.int64)).to(cuda), torch.from_numpy(values).to(cuda), n_tiles)
+    assert int(status.item()) == 0
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(u64(k), keys[order])
+    np.testing.assert_array_equal(v.cpu().numpy(), values[order])
+    np.testing.assert_array_equal(offsets.cpu().numpy(), np.concatenate([[0], np.cumsum(lengths)]))
+
+
 def test_sort_tile_lists_uniform_digits_and_empty(cuda):
     """Depth words that differ in one byte only (three of the four passes are left out), equal keys, no keys."""
     import torch

@@ -636,11 +636,18 @@ __device__ __forceinline__ void segment_sort_in_wave(uint64_t *keys, uint32_t *v
 
 // One workgroup per four segments.  A segment of up to kSegWaveCap pairs is sorted by one wave of its own;
 // then the workgroup takes those of up to medium_cap pairs together, one after the other.  Longer ones are
-// left to segment_sort_large_kernel.  medium_cap is kSegMediumCap where no list can be longer (and that kernel is not
-// launched at all), else half of it: sixteen waves have a list of 2048 pairs sorted sooner than four, and its three
-// neighbours do not wait for it (1.3 million triangles of a mesh: both kernels together 111 -> 102 us, half a million: 88 -> 80).
+// left to segment_sort_large_kernel.  medium_cap (medium_segments) is kSegMediumCap where no list can be longer (and that kernel
+// is not launched at all), else half of it: sixteen waves have a list of 2048 pairs sorted sooner than four, and its three
+// neighbours do not wait for it (both kernels together, 1.3 million triangles of a torus: 110 -> 102 us, half a million on 1024
+// tiles 89 -> 81, 200 000 faint ones with lists of 3700 134 -> 110; an icosphere the other way, 85 -> 102).  Where most lists
+// are that long, though, one of the large kernel's 256 workgroups sorts many of them in turn: kSegMediumCap again (8160 lists of
+// 1100 to 1800 pairs: 340 -> 190 us, 3600: 165 -> 115; 1024 lists: 56 and 65, and lists of 1500 to 3000 300 and 360).
 constexpr int kSegMediumItems = 8;
 constexpr int kSegMediumCap = kSortThreads * kSegMediumItems;  // 2048 pairs: as much LDS as the four waves' own buffers
+static int medium_segments(int64_t longest, int64_t n, int n_tiles) {
+    const bool most = n_tiles > 2048 && n >= (int64_t)(kSegMediumCap / 4) * n_tiles && n < (int64_t)kSegMediumCap * n_tiles;
+    return longest <= kSegMediumCap || most ? kSegMediumCap : kSegMediumCap / 2;
+}
 struct MediumSegLds {
     SegLds<kSortThreads> lds;
     uint32_t ex_keys[kSegMediumCap], ex_vals[kSegMediumCap];
@@ -949,7 +956,7 @@ static int ranges_and_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint
         TG_LAUNCH(tile_ranges_kernel, dim3((unsigned)ceil_div64(n + 1, kSortThreads)), dim3(kSortThreads), 0, s, k, n, n_tiles, offsets);
         if (int e = check_launch("tile_ranges_kernel")) return e;
     }
-    const int medium_cap = longest <= kSegMediumCap ? kSegMediumCap : kSegMediumCap / 2;
+    const int medium_cap = medium_segments(longest, n, n_tiles);
     TG_LAUNCH(segment_sort_small_kernel, dim3(ceil_div(n_tiles, kSortWaves)), dim3(kSortThreads), 0, s, k, v, offsets, n_tiles,
               tile_count, row_totals, tiles_x, (uint32_t)n, frame_count, status, medium_cap, long_tiles);
     if (int e = check_launch("segment_sort_small_kernel")) return e;
