@@ -27,6 +27,7 @@ struct FrameLayout {
     int long_limit;                 // list entries that make a tile a long one; 0: the frame has no use for them
 };
 
+// No size is larger for a smaller number of triangles, all else equal: callers size buffers for a rounded one.
 static FrameLayout frame_layout(const tg_frame &f) {
     FrameLayout L = {};
     const int tiles_x = (int)ceil_div64(f.width, f.tile_w), tiles_y = (int)ceil_div64(f.height, f.tile_h), tiles = tiles_x * tiles_y;

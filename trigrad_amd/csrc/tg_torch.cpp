@@ -7,8 +7,8 @@
 // by returning None: a kind of frame not seen before on this stream, a scene whose number of keys has left the range its
 // plan was made for, a wait of the kernels that expired, arguments the checks there have an error for.
 //
-// Plans and frame states (what tg_bin_frame keeps between calls) are per kind of frame and per device and stream, are made
-// by the Python route and handed over, and are bounded in number there.
+// Plans are per kind of frame (sizes, options, a rounded number of triangles), frame states (what tg_bin_frame keeps between
+// calls) per device and stream; both are made by the Python route, handed over, and bounded in number.
 #define PY_SSIZE_T_CLEAN
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
