@@ -1046,6 +1046,8 @@ def test_key_buffers_of_a_size_seen_before(cuda):
                                                      True, 32)
         made.append((frame.n_keys, frame.plan.capacity))
     assert made[0][1] == 3 * 4000 + 65536
+    few = _C.frame_forward(d["vertices"], d["indices"][:1200], d["colors"], d["opacities"], W, H, 16, 16, 1 / 256, True, 32)[3]
+    assert few.plan.capacity == 3 * 1200 + 65536  # another scene: its keys per triangle say nothing
     assert all(keys <= capacity <= 1.3 * keys + 2048 for keys, capacity in made[1:])
     for table in (_C._frame_key_hints, _C._frame_size_hints, _C._frame_plans):
         assert len(table) <= _C._MAX_REMEMBERED

@@ -700,9 +700,13 @@ def _plan_for(kind):
 
 
 def _remember(table, key, value):
-    if len(table) >= _MAX_REMEMBERED and key not in table:
-        table.pop(next(iter(table)), None)
-    table[key] = value
+    with _table_lock:
+        if len(table) >= _MAX_REMEMBERED and key not in table:
+            del table[next(iter(table))]
+        table[key] = value
+
+
+_table_lock = threading.Lock()
 
 
 def _round_count(n):
@@ -811,9 +815,10 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
                     flags | _FRAME_LIST_BOUNDS if bounds else flags, float(early_stopping_threshold))
 
         expected = _frame_key_hints.get(hint_key)
-        if expected is None and size_key in _frame_size_hints:
-            keys, triangles = _frame_size_hints[size_key]  # another number of triangles: about as many keys each
-            expected = -(-keys * n_triangles // triangles)
+        if expected is None:
+            keys, triangles = _frame_size_hints.get(size_key, (0, 0))
+            if triangles <= 2 * n_triangles and n_triangles <= 2 * triangles:
+                expected = -(-keys * n_triangles // triangles)  # the same scene with a few triangles more or fewer
         # An order pool takes a row of a tile's pixels per key: it is made for counted keys, not for a guess.  The first
         # frame of its kind and size counts them in a binning of its own.
         counting = expected is None and bool(flags & _FRAME_ORDER_POOL)
