@@ -243,7 +243,7 @@ int tg_build_tile_lists(const tg_real *records, const uint32_t *tri_offsets, int
  * cleared between calls.  One call at a time per frame state.  A wait for
  * another workgroup that expires (see TG_STATUS_*) writes `epoch` to
  * total_and_status[1], which is not written otherwise: pass a word that holds
- * something else.
+ * something else.  No key is written then, and K means nothing.
  *
  * On the side the first launch zeroes zero_bytes bytes at `zero` (pass the
  * workspace of the tg_build_frame_lists call that follows, sized for
