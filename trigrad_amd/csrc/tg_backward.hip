@@ -361,15 +361,6 @@ __device__ __forceinline__ TermLane term_lane(const BackwardArgs &g, int lane) {
     return t;
 }
 
-// Orders the LDS traffic of one wave: what lanes wrote before is visible to the
-// lanes that read after (LDS serves a wave's instructions in order; this keeps
-// the compiler from moving accesses across the point).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Adds up the runs of equal list entry among the first n slots of a wave's term matrix (row q = term
 // q, rows kTermStride apart; slots of one entry are neighbours) and adds every non-zero run sum to the
 // gradient arrays.  Bit c of `heads` is set where slot c starts a run.  Lane (group, q) owns a fixed third of
@@ -421,10 +412,6 @@ __device__ __forceinline__ int wave_max_i32(int v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, kWave));
     return v;
-}
-
-__device__ __forceinline__ uint32_t lanes_below_mask(uint64_t mask) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
 // Tile-order backward.  LDS floating-point atomics cost about three cycles per lane on
@@ -481,12 +468,10 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
     const int my_last = p.valid ? g.last[p.index] : 0;  // entries [0, my_last) of the list may hold my fragments
     BackState st;
     if (p.valid) st = load_back_state(g, p);
-    int tile_last;
-    if (saved_masks) {
-        tile_last = (int)g.hit_masks[hit_mask_head_index(tile)];
-    } else {
+    int tile_last = saved_masks ? (int)(int64_t)g.hit_masks[hit_mask_head_index(tile)] : -1;
+    if (tile_last < 0) {  // the same for the workgroup: no masks, or its pixels were rendered by several workgroups
         if (tid == 0) s_last = 0;
-        publish_wave_rect(p, s_rects);  // only the repeated inside tests cull by wave rectangle
+        if (!saved_masks) publish_wave_rect(p, s_rects);  // only the repeated inside tests cull by wave rectangle
         __syncthreads();
         if (my_last > 0) atomicMax(&s_last, my_last);
         __syncthreads();

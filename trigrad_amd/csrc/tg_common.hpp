@@ -162,6 +162,15 @@ __device__ __forceinline__ real pixel_ndc(int i, int extent) {
     return (real)(((double)(real)i + 0.5) / (double)(real)extent * 2.0 - 1.0);
 }
 
+// Orders the LDS traffic of one wave: what lanes wrote before is visible to the
+// lanes that read after (LDS serves a wave's instructions in order; this keeps
+// the compiler from moving accesses across the point).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- wave64 DPP scan -----------------------------------------------------------
 template <int kCtrl, int kRowMask>
 __device__ __forceinline__ uint32_t dpp_add_u32(uint32_t v) {

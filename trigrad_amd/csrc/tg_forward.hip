@@ -12,6 +12,8 @@
 //
 // Not HBM-bound: per (pixel, entry) pair ~12 VALU operations and three
 // broadcast LDS reads against 148 B of gathered data per ENTRY.
+#include <algorithm>
+
 #include "tg_frame.hpp"
 #include "tg_raster.hpp"
 
@@ -32,25 +34,19 @@ struct ForwardOut {
     int long_rows;                // rows of workgroups at the start of the grid, for the long tiles
 };
 
-// The tile a workgroup of a forward launch takes, and its list; false: none.  The first workgroups take the tiles with the
-// longest lists and the others, in the order of tile_of_workgroup, the rest.  Nothing here waits for a load before the next
-// one is asked for, apart from the long tiles' own: a frame without any loses 1 us by the workgroups that find none.
-__device__ __forceinline__ bool take_tile(const RasterArgs &a, const ForwardOut &o, TileId &t, int &start, int &end) {
-    if ((int)blockIdx.y < o.long_rows) {
-        const int slot = (int)(blockIdx.y * gridDim.x + blockIdx.x);
-        if (slot >= kLongTileSlots || slot >= o.long_tiles.words[0]) return false;
-        t.index = o.long_tiles.words[1 + slot];
-        t.y = t.index / (int)gridDim.x;
-        t.x = t.index - t.y * (int)gridDim.x;
-        start = a.offsets[t.index];
-        end = a.offsets[t.index + 1];
-        return true;
-    }
-    t = tile_of_workgroup<kTileBandForward, kChunkForward>(o.long_rows);
-    start = a.offsets[t.index];
-    end = a.offsets[t.index + 1];
-    if (!o.long_rows || end - start < o.long_tiles.limit) return true;
-    return o.long_tiles.words[0] > kLongTileSlots && o.long_tiles.slot_of_tile[t.index] < 0;
+// The workgroups in the first long_rows rows of a forward launch take the tiles with the longest lists (LongTiles), the others
+// the rest in the order of tile_of_workgroup.  A frame without a long tile loses 1 us by the workgroups that find none.
+__device__ __forceinline__ int long_tiles(const ForwardOut &o) { return min(o.long_tiles.words[0], kLongTileSlots); }
+__device__ __forceinline__ TileId long_tile(const ForwardOut &o, int slot) {
+    TileId t;
+    t.index = o.long_tiles.words[1 + slot];
+    t.y = t.index / (int)gridDim.x;
+    t.x = t.index - t.y * (int)gridDim.x;
+    return t;
+}
+// Whether a tile is one of those, of which the first `taken` slots are.
+__device__ __forceinline__ bool is_long_tile(const ForwardOut &o, int tile, int n_entries, int taken) {
+    return o.long_rows && n_entries >= o.long_tiles.limit && (uint32_t)o.long_tiles.slot_of_tile[tile] < (uint32_t)taken;
 }
 
 // Lists whose sort gave up a wait are not to be read (unwritten entries may name anything): the frame's pixels
@@ -92,25 +88,129 @@ __device__ __forceinline__ void write_pixel(const ForwardOut &o, const PixelCoor
     o.image[p.index] = make_real4(s.c0, s.c1, s.c2, s.alpha);
 }
 
-// Eight waves per SIMD (63 registers, nothing in scratch memory): 212 -> 194 us against the 73 registers it would take
+// A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup, in
+// tile order: each tests 64 of 256 entries, lane = entry, from registers; the records of those that are hit go to LDS, and the
+// first wave composites them in list order.  500 000 triangles of a mesh, 500 x 500 (longest list 5500, a tile one workgroup's
+// chain before): 367 -> 127 us.  s_hits: per wave, which of its 64 entries cover a pixel, then which of them cover any, then which
+// of those are staged.
+__device__ __forceinline__ void long_tile_part(const RasterArgs &a, const ForwardOut &out, const TileId &tile, int part, BlendRecord *s_rec,
+                                               uint64_t (*s_hits)[kWave + 2]) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // what depends on it is made here, not kept in registers by the loop around the call
+    const int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
+    const int slot = (blockIdx.z * kMaxTileWaves + part) * kWave + lane;
+    const PixelCoord p = pixel_of_slot(a, tile.x, tile.y, slot);
+    const WaveRect rect = wave_rect(p);
+    const bool squares = ((a.tw | a.th) & 7) == 0;
+    PixelState s;  // of the first wave
+    int last = 0;
+    // an entry's matrix and vertex numbers are asked for while the entries before it are composited, its triangle's number
+    // before that; what only the entries that are hit need is read when it is known which they are
+    DepthParts next;
+    const auto entry = [&](int first) { return min(first + tid, end - 1); };
+    next.fetch_triangle(a, entry(start));
+    next.fetch_matrix(a);
+    next.fetch_triangle(a, entry(start + kTileThreads));
+    for (int first = start; first < end; first += kTileThreads) {
+        const bool running = wave == 0 && p.valid && s.alpha > a.thr && s.blended < a.max_layers;
+        if (!__syncthreads_or(running)) break;
+        const real matrix[9] = {next.m0[0], next.m0[1], next.m0[2], next.m0[3], next.m1[0], next.m1[1], next.m1[2], next.m1[3], next.m2};
+        const int3v id = next.id;
+        next.fetch_matrix(a);
+        next.fetch_triangle(a, entry(first + 2 * kTileThreads));
+        uint64_t hit;
+        const uint64_t m = wave_hits(matrix, first + tid < end, squares, rect, p.px, p.py, hit);
+        s_hits[wave][lane] = m;
+        if (lane == 0) s_hits[wave][kWave] = hit;
+        if (out.hit_masks && first + wave * kWave < end) {
+            const int64_t chunk = hit_mask_chunk(start, tile.index, first + wave * kWave - start);
+            out.hit_masks[hit_mask_head_words(out.long_rows) + chunk * ((int64_t)gridDim.z * kTileThreads) + slot] = m;
+        }
+        __syncthreads();
+        int before = 0, total = 0;
+#pragma unroll
+        for (int w = 0; w < kMaxTileWaves; w++) {
+            const int count = __builtin_popcountll(s_hits[w][kWave]);
+            if (w < wave) before += count;
+            total += count;
+        }
+        const int rank = before + (int)lanes_below_mask(hit);
+        for (int round = 0; round < total; round += kBatch) {  // the same for the workgroup
+            const bool staged = ((hit >> lane) & 1) && rank >= round && rank < round + kBatch;
+            const uint64_t group = __builtin_amdgcn_ballot_w64(staged);
+            if (lane == 0) s_hits[wave][kWave + 1] = group;
+            if (staged) gather_record(a, matrix, id, s_rec[rank - round]);
+            __syncthreads();
+            if (wave == 0) {
+                int base = 0;
+                for (int w = 0; w < kMaxTileWaves; w++) {
+                    const uint64_t there = s_hits[w][kWave + 1];
+                    uint64_t bits = s_hits[w][lane] & there;
+                    while (true) {
+                        const bool more = bits && p.valid && s.alpha > a.thr && s.blended < a.max_layers;  // render.cu:578, tested before every fragment
+                        if (__builtin_amdgcn_ballot_w64(more) == 0) break;  // wave-uniform
+                        if (!more) continue;
+                        const int e = __builtin_ctzll(bits);
+                        bits &= bits - 1;
+                        const BlendRecord &b = s_rec[base + __builtin_popcountll(there & ((1ull << e) - 1))];
+                        real b0, b1, b2;
+                        bary_apply(b.m, p.px, p.py, b0, b1, b2);
+                        blend_fragment(s, b, b0, b1, b2);
+                        last = first - start + w * kWave + e + 1;
+                    }
+                    base += __builtin_popcountll(there);
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (wave == 0 && p.valid) write_pixel(out, p, s, last, 0.0f);
+    // the tile's pixels are four workgroups': the backward pass finds out for itself how far they got
+    if (out.hit_masks && tid == 0) out.hit_masks[hit_mask_head_index(tile.index)] = ~0ull;
+}
+
+// kSplit: the long tiles' work is shared out to four waves (long_tile_part), which takes 121 registers, four waves per SIMD.
+// That is what up to 1024 workgroups fill, so only a launch of more goes without (its long tiles come first, that is all):
+// eight waves per SIMD there (63 registers, nothing in scratch memory): 212 -> 194 us against the 73 registers it would take
 // (10^6 triangles, 1920 x 1080).  No bound in double precision: held to the five waves that the LDS allows it spills (8 x 8
 // tiles: 112 -> 123 us).
-__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
+constexpr int kFewTileGroups = 1024;
+// Workgroups for the long tiles, at most: more find nothing to do at 1 us for 128 (per-pixel order: 128 to 1024 within 1 % on
+// the mesh of 1.3 million triangles, 10^5 triangles without a long tile 92 -> 93 us), unless the others leave room: in tile
+// order with few tiles (500 000 triangles of a mesh: 128 groups 230 us, 512 190, 1024 175), and wherever there are no more
+// tiles than CUs.
+constexpr int kLongGroups = 128, kLongGroupsFewTiles = 1024;
+template <bool kSplit>
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kSplit ? 4 : 8) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
     __shared__ BlendRecord s_rec[kBatch];
     __shared__ uint8_t s_touch[kBatch];
     __shared__ WaveRect s_rects[kMaxTileWaves];
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
-    TileId tile_id;
-    int start, end;
-    const bool mine = take_tile(a, out, tile_id, start, end);
     if (lists_invalid(out)) {  // the same for the whole launch
         mark_tile_invalid(a, out);
         return;
     }
-    if (!mine) return;
+    TileId tile_id;
+    if ((int)blockIdx.y < out.long_rows) {
+        const int group = (int)(blockIdx.y * gridDim.x + blockIdx.x), groups = out.long_rows * (int)gridDim.x;
+        if constexpr (kSplit) {
+            __shared__ uint64_t s_hits[kMaxTileWaves][kWave + 2];
+            const int n_items = kMaxTileWaves * long_tiles(out);
+            for (int item = group; item < n_items; item += groups) long_tile_part(a, out, long_tile(out, item / kMaxTileWaves), item % kMaxTileWaves, s_rec, s_hits);
+            return;
+        } else {
+            if (group >= long_tiles(out)) return;
+            tile_id = long_tile(out, group);
+        }
+    } else {
+        tile_id = tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
+    }
     const int tile = tile_id.index;
+    const int start = a.offsets[tile], end = a.offsets[tile + 1];
+    if ((int)blockIdx.y >= out.long_rows && is_long_tile(out, tile, end - start, kSplit ? kLongTileSlots : out.long_rows * (int)gridDim.x)) return;
     const PixelCoord p = pixel_of_thread(a, tile_id);
     publish_wave_rect(p, s_rects);
     const bool tests_small = tests_small_entries(a, end - start, (int)(gridDim.x * (gridDim.y - out.long_rows)));
@@ -389,6 +489,185 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     if (p.valid) write_pixel(out, p, s, last_j + 1, last_depth);
 }
 
+// A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup: each
+// takes every fourth block of 64 entries and keeps candidate lists of its own, without a barrier, and the first wave merges the
+// four sorted lists of a pixel, by depth and list position, while it blends.  A list was one workgroup's serial chain before,
+// 7 us for every 64 entries with most of the CU empty; it is a quarter as long now, and a tile's four squares run beside
+// each other.  What a wave tests it holds in registers, lane = entry, so only the entries that are hit go through LDS, kStage / 4
+// at a time: the candidate lists leave no more (64 at a time, with fewer candidates kept, is no faster).
+// 1.3 million triangles of a mesh, 1920 x 1080 (longest list 5200, 221 of at least 1024): 604 -> 332 us; 200 000 around the
+// camera (one list of 8400): 152 -> 117; 81 tiles with lists of some 2600, where depth bounds end the looking early: 105 -> 91.
+// s_quarter: a depth for every thread, with depth bounds; else null.
+template <int kStage, typename Pos>
+__device__ __forceinline__ void long_tile_part(const RasterArgs &a, const ForwardOut &out, const TileId &tile, int part, unsigned char *s_dyn,
+                                               volatile real *s_quarter) {
+    constexpr int kStaged = kStage / kMaxTileWaves;  // records of a wave in LDS at a time
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1], n = end - start;
+    if (sizeof(Pos) < sizeof(int) && n > kShortList) return;  // left to forward_pixel_order_long_lists_kernel
+    DepthRecord *s_rec = reinterpret_cast<DepthRecord *>(s_dyn) + wave * kStaged;
+    TopKOf<Pos> tk;
+    tk.depth = reinterpret_cast<real *>(s_dyn + sizeof(DepthRecord) * kStage);
+    tk.pos = reinterpret_cast<Pos *>(tk.depth + kLayers * kTileThreads);
+    tk.n_threads = kTileThreads;
+    // between two selections the place of the staged records holds what the waves tell each other
+    struct Shared { int found[kTileThreads], cap[kWave], last_j[kWave], nan[kMaxTileWaves]; real last_depth[kWave]; };
+    static_assert(sizeof(Shared) <= sizeof(DepthRecord) * kStage, "the waves' exchange fits the staging area");
+    Shared *shared = reinterpret_cast<Shared *>(s_dyn);
+
+    const int slot = (blockIdx.z * kMaxTileWaves + part) * kWave + lane;
+    const PixelCoord p = pixel_of_slot(a, tile.x, tile.y, slot);
+    const WaveRect rect = wave_rect(p);
+    const bool squares = ((a.tw | a.th) & 7) == 0;
+    const int64_t order_step = order_stride(out.order, a);
+    const int64_t order_at = order_first(out.order, p, start, slot);
+    const int rows_kept = out.order.low ? order_rows(out.order, a, n) : 0;
+
+    PixelState s;  // of the first wave
+    real last_depth = -__builtin_inff();
+    int last_j = -1;
+    bool active = p.valid && n > 0;
+    while (true) {
+        const int wanted = active && s.alpha > a.thr && s.blended < a.max_layers ? min(kLayers, a.max_layers - s.blended) : 0;
+        __syncthreads();
+        if (wave == 0) {
+            shared->cap[lane] = wanted;
+            shared->last_depth[lane] = last_depth;
+            shared->last_j[lane] = last_j;
+        }
+        if (s_quarter) s_quarter[tid] = __builtin_inff();
+        __syncthreads();
+        const int cap = shared->cap[lane];
+        last_depth = shared->last_depth[lane];
+        last_j = shared->last_j[lane];
+        if (__builtin_amdgcn_ballot_w64(cap > 0) == 0) break;  // the same for all waves
+        __syncthreads();
+        // The waves take the list's blocks of 64 entries in turn, each with candidate lists of its own.  A NaN depth ends a
+        // candidate list wherever it comes (topk_insert), so which candidates stay depends on what came before it: where one is
+        // met the first wave does the selection alone.
+        int found = 0;
+        for (int waves = kMaxTileWaves; ; waves = 1) {
+            found = 0;
+            bool met_nan = false;
+            if (wave < waves) {
+                const auto entry = [&](int block) { return min(start + block * kWave + lane, end - 1); };
+                DepthParts next;
+                const auto fetch_from = [&](int block) {
+                    next.fetch_triangle(a, entry(block));
+                    next.fetch_matrix(a);
+                    next.fetch_triangle(a, entry(block + waves));
+                    next.fetch_vertices(a);
+                };
+                fetch_from(wave);
+                for (int block = wave; block * kWave < n; block += waves) {
+                    if (kStage != kWave && a.batch_bounds) {
+                        // as in pixel_order_tile: there are enough candidates nearer than all the rest of the list.  Each wave
+                        // knows that of a quarter of them in every wave's lists; at a depth of its own the rest might come
+                        // before another wave's candidate.
+                        const real rest = a.batch_bounds[batch_bound_index(start, tile.index, block * kWave)];
+                        const int resume = a.far_start[tile.index] / kWave;
+                        bool settled = cap == 0;
+                        if (!settled && waves == 1) settled = found == cap && tk.d(cap - 1) <= rest;
+                        if (!settled && waves > 1) {
+                            settled = true;
+#pragma unroll
+                            for (int w = 0; w < kMaxTileWaves; w++) settled = settled && s_quarter[w * kWave + lane] < rest;
+                        }
+                        if (resume > block && !__builtin_amdgcn_ballot_w64(!settled)) {
+                            block = resume + (wave - resume % waves + waves) % waves;
+                            if (block * kWave >= n) break;
+                            fetch_from(block);
+                        }
+                    }
+                    const DepthRecord r = next.record();
+                    next.fetch_matrix(a);
+                    next.fetch_triangle(a, entry(block + 2 * waves));
+                    uint64_t hit;
+                    uint64_t m = wave_hits(r.m, block * kWave + lane < n, squares, rect, p.px, p.py, hit);
+                    if (cap == 0) m = 0;
+                    next.fetch_vertices(a);
+                    while (hit) {  // wave-uniform: the hit entries' records through LDS, kStaged at a time
+                        const uint32_t rank = lanes_below_mask(hit);
+                        const bool staged = ((hit >> lane) & 1) && rank < (uint32_t)kStaged;
+                        const uint64_t group = __builtin_amdgcn_ballot_w64(staged);
+                        if (staged) s_rec[rank] = r;
+                        wave_lds_sync();
+                        uint64_t mine = m & group;
+                        while (__builtin_amdgcn_ballot_w64(mine != 0)) {
+                            if (mine == 0) continue;
+                            const int e = __builtin_ctzll(mine);
+                            mine &= mine - 1;
+                            const DepthRecord &d = s_rec[__builtin_popcountll(group & ((1ull << e) - 1))];
+                            real b0, b1, b2;
+                            bary_apply(d.m, p.px, p.py, b0, b1, b2);
+                            const real pd = interp_w(b0, b1, b2, d.z[0], d.z[1], d.z[2], d.w[0], d.w[1], d.w[2]);  // render.cu:404
+                            const int j = block * kWave + e;
+                            met_nan = met_nan || pd != pd;
+                            if (pd < last_depth || (pd == last_depth && j <= last_j)) continue;
+                            topk_insert(tk, cap, found, pd, j);
+                        }
+                        hit &= ~group;
+                        wave_lds_sync();
+                    }
+                    const int quarter = (cap + kMaxTileWaves - 1) / kMaxTileWaves;
+                    if (s_quarter && waves > 1 && cap > 0 && found >= quarter) s_quarter[tid] = tk.d(quarter - 1);
+                }
+            }
+            __syncthreads();
+            shared->found[tid] = found;
+            const uint64_t nan_lanes = __builtin_amdgcn_ballot_w64(met_nan);
+            if (lane == 0) shared->nan[wave] = nan_lanes != 0;
+            __syncthreads();
+            if (waves == 1 || !(shared->nan[0] | shared->nan[1] | shared->nan[2] | shared->nan[3])) break;
+            __syncthreads();
+        }
+        if (wave == 0 && cap > 0) {
+            // the four sorted lists of this lane's pixel, nearest first; no list has a NaN, or three are empty
+            const auto depth_at = [&](int w, int i) { return tk.depth[i * kTileThreads + w * kWave + lane]; };
+            const auto pos_at = [&](int w, int i) { return (int)tk.pos[i * kTileThreads + w * kWave + lane]; };
+            int count[kMaxTileWaves], at[kMaxTileWaves], pos[kMaxTileWaves], total = 0;
+            real depth[kMaxTileWaves];
+#pragma unroll
+            for (int w = 0; w < kMaxTileWaves; w++) {
+                count[w] = shared->found[w * kWave + lane];
+                total += count[w];
+                at[w] = 0;
+                depth[w] = count[w] ? depth_at(w, 0) : 0.0f;
+                pos[w] = count[w] ? pos_at(w, 0) : 0;
+            }
+            const int todo = min(total, cap);
+            for (int i = 0; i < todo; i++) {
+                int best = -1;
+#pragma unroll
+                for (int w = 0; w < kMaxTileWaves; w++)
+                    if (at[w] < count[w] && (best < 0 || depth[w] < last_depth || (depth[w] == last_depth && pos[w] < last_j))) {
+                        best = w;
+                        last_depth = depth[w];
+                        last_j = pos[w];
+                    }
+#pragma unroll
+                for (int w = 0; w < kMaxTileWaves; w++)
+                    if (w == best && ++at[w] < count[w]) {
+                        depth[w] = depth_at(w, at[w]);
+                        pos[w] = pos_at(w, at[w]);
+                    }
+                BlendRecord r;
+                gather_blend(a, start + last_j, r);
+                if (s.blended < rows_kept) {
+                    const int64_t word = order_at + (int64_t)s.blended * order_step;
+                    out.order.low[word] = (uint16_t)last_j;
+                    if (sizeof(Pos) > sizeof(uint16_t) && n > kShortList) out.order.low[out.order.high + word] = (uint16_t)(last_j >> 16);
+                }
+                real b0, b1, b2;
+                bary_apply(r.m, p.px, p.py, b0, b1, b2);
+                blend_fragment(s, r, b0, b1, b2);
+            }
+            if (total < cap) active = false;  // the list is exhausted (render.cu:594)
+        }
+    }
+    if (wave == 0 && p.valid) write_pixel(out, p, s, last_j + 1, last_depth);
+}
+
 // One workgroup per tile.  With 16-bit positions the tiles whose lists are too long for them are left to
 // forward_pixel_order_long_lists_kernel.
 // kInTurn: the workgroup has four waves.
@@ -400,14 +679,30 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ uint8_t s_touch[kStage];
     __shared__ WaveRect s_rects[kMaxTileWaves];
-    TileId tile;
-    int start, end;
-    const bool mine = take_tile(a, out, tile, start, end);
     if (lists_invalid(out)) {  // the same for the whole launch
         mark_tile_invalid(a, out);
         return;
     }
-    if (!mine || (sizeof(Pos) < sizeof(int) && end - start > kShortList)) return;
+    TileId tile;
+    if ((int)blockIdx.y < out.long_rows) {
+        const int group = (int)(blockIdx.y * gridDim.x + blockIdx.x), groups = out.long_rows * (int)gridDim.x;
+        if constexpr (kInTurn) {
+            __shared__ real s_quarter[kStage != kWave ? kTileThreads : 1];  // with depth bounds; batches of 64 go without
+            const int n_items = kMaxTileWaves * long_tiles(out);
+            for (int item = group; item < n_items; item += groups)
+                long_tile_part<kStage, Pos>(a, out, long_tile(out, item / kMaxTileWaves), item % kMaxTileWaves, s_dyn,
+                                            kStage != kWave ? s_quarter : nullptr);
+            return;
+        } else {
+            if (group >= long_tiles(out)) return;
+            tile = long_tile(out, group);
+        }
+    } else {
+        tile = tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
+    }
+    const int n_entries = a.offsets[tile.index + 1] - a.offsets[tile.index];
+    if (sizeof(Pos) < sizeof(int) && n_entries > kShortList) return;
+    if ((int)blockIdx.y >= out.long_rows && is_long_tile(out, tile.index, n_entries, kInTurn ? kLongTileSlots : out.long_rows * (int)gridDim.x)) return;
     pixel_order_tile<kStage, Pos, kInTurn>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
 }
 
@@ -529,13 +824,20 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
         return TG_E_ARG;
     }
     ForwardOut o{(real4 *)image, depthmap, final_weights, ends, last, last_depth, order, per_pixel_sort ? nullptr : hit_masks,
-                 list_status, host_status, long_tiles, long_tiles.words ? ceil_div(kLongTileSlots, ceil_div(width, tile_w)) : 0};
+                 list_status, host_status, long_tiles, 0};
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
+    const bool split_tiles = !per_pixel_sort && tl.threads == kTileThreads && (int64_t)tl.grid.x * tl.grid.y * tl.grid.z <= kFewTileGroups;
+    if (long_tiles.words)
+        o.long_rows = ceil_div((int)std::min<int64_t>(split_tiles || (int64_t)tl.grid.x * tl.grid.y <= kFewTiles ? kLongGroupsFewTiles : kLongGroups,
+                                                      kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
     const dim3 grid(tl.grid.x, tl.grid.y + o.long_rows, tl.grid.z);
     const int n_threads = tl.threads;
     hipStream_t s = (hipStream_t)stream;
     if (!per_pixel_sort) {
-        TG_LAUNCH(forward_tile_order_kernel, grid, dim3(n_threads), 0, s, a, o);
+        if (split_tiles)
+            TG_LAUNCH_AS("forward_tile_order_kernel", forward_tile_order_kernel<true>, grid, dim3(n_threads), 0, s, a, o);
+        else
+            TG_LAUNCH_AS("forward_tile_order_kernel", forward_tile_order_kernel<false>, grid, dim3(n_threads), 0, s, a, o);
         return check_launch("forward_tile_order_kernel");
     }
     const size_t lds = pixel_order_lds_bytes(n_threads, kSelectBatch);

@@ -58,15 +58,14 @@ static FrameLayout frame_layout(const tg_frame &f) {
     L.sort_bytes = tg_build_frame_lists_workspace_bytes(f.key_capacity, tiles_x, tiles_y);
     L.sort = take(L.sort_bytes);
     L.zero_bytes = L.sort_bytes;
-    // Where all tiles' workgroups fit the device at once it does not matter which one starts first: three of a 16 x 16 tile a
-    // CU in per-pixel order, eight in tile order (there, 1024 tiles of a mesh: kernel 382 us with the long ones first, 378
-    // without; 1900 tiles: 732 and 728).  Long: 1024 entries, and twice the mean.  Forward kernel, before and after the long
-    // tiles come first, per-pixel order: 1.3 million triangles of a mesh, 1920 x 1080 (longest list 5200) 677 -> 610 us,
-    // 200000 around the camera (8400) 184 -> 153; frames without a long list pay 1 to 2 us for the workgroups that find none.
+    // Long: 1024 entries, and twice what a tile has on average, or twice what one of the workgroups that run at once (three of a
+    // 16 x 16 tile a CU in per-pixel order, eight in tile order) has where there are fewer tiles than that.  Shorter ones are
+    // served as well by the others' way (mesh of 1.3 million triangles, per-pixel order: 1024 entries 333 us, 768 336, 1400
+    // 350; mesh of 500 000, 1024 tiles, tile order: 127, 142, 126).
     const int64_t longest = f.key_capacity < f.n_triangles ? f.key_capacity : f.n_triangles;
-    const int64_t limit = std::max<int64_t>(1024, ceil_div64(2 * f.key_capacity, tiles));
-    const int at_once = 256 * (f.per_pixel_sort ? 3 : 8);
-    if (tiles > at_once && longest >= limit) {
+    const int64_t at_once = 256 * (f.per_pixel_sort ? 3 : 8);
+    const int64_t limit = std::max<int64_t>(1024, ceil_div64(2 * f.key_capacity, std::max<int64_t>(tiles, 2 * at_once)));
+    if (longest >= limit) {
         L.long_limit = (int)limit;
         L.long_tiles = take((1 + kLongTileSlots) * 4);
         L.slots = take((size_t)tiles * 4);
@@ -168,7 +167,7 @@ extern "C" int tg_frame_forward(tg_frame *f) {
     volatile uint32_t *host = f->host;
     const int64_t longest = f->key_capacity < f->n_triangles ? f->key_capacity : f->n_triangles;  // a triangle is in a list once
     LongTiles long_tiles;
-    if (L.long_limit) long_tiles = LongTiles{(int32_t *)(scratch + L.long_tiles), (int32_t *)(scratch + L.slots), L.long_limit};
+    if (L.long_limit) long_tiles = LongTiles{(int32_t *)(scratch + L.long_tiles), (int32_t *)(scratch + L.slots), L.long_limit, std::min<int64_t>(tiles, f->key_capacity / L.long_limit)};
     if (f->phases & TG_FRAME_BIN) {
         host[1] = 0;
         host[2] = TG_FRAME_PENDING;

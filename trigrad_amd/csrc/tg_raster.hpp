@@ -41,9 +41,9 @@ struct PixelCoord {
     real px, py;
 };
 
-__device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int tile_x, int tile_y) {
+// The pixel in slot t of a tile.
+__device__ __forceinline__ PixelCoord pixel_of_slot(const RasterArgs &a, int tile_x, int tile_y, int t) {
     PixelCoord p;
-    const int t = blockIdx.z * blockDim.x + threadIdx.x;
     int lx, ly;
     if (((a.tw | a.th) & 7) == 0) {
         // a wave takes a square of 8 x 8 pixels: fewer list entries touch a square than a strip of the
@@ -62,6 +62,10 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
     p.px = pixel_ndc(p.ix, a.W);
     p.py = pixel_ndc(p.iy, a.H);
     return p;
+}
+
+__device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int tile_x, int tile_y) {
+    return pixel_of_slot(a, tile_x, tile_y, blockIdx.z * blockDim.x + threadIdx.x);
 }
 
 // The tile a workgroup of a (tiles_x, tiles_y, parts) launch takes.  Workgroups go to the eight XCDs of the device in
@@ -155,6 +159,17 @@ __device__ __forceinline__ TriIds load_ids(const RasterArgs &a, int j) {
     return t;
 }
 
+// The attributes of a record's vertices.
+__device__ __forceinline__ void gather_attributes(const RasterArgs &a, int ia, int ib, int ic, BlendRecord &r) {
+    r.op[0] = a.opacities[ia]; r.op[1] = a.opacities[ib]; r.op[2] = a.opacities[ic];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        r.col[k] = a.colors[3 * (int64_t)ia + k];
+        r.col[3 + k] = a.colors[3 * (int64_t)ib + k];
+        r.col[6 + k] = a.colors[3 * (int64_t)ic + k];
+    }
+}
+
 __device__ __forceinline__ void gather_blend(const RasterArgs &a, int j, BlendRecord &r) {
     const TriIds t = load_ids(a, j);
     const real *m = a.bary + 9 * (int64_t)t.tri;
@@ -165,13 +180,7 @@ __device__ __forceinline__ void gather_blend(const RasterArgs &a, int j, BlendRe
     r.extent = max3(va.y, vb.y, vc.y) - min3(va.y, vb.y, vc.y);
     r.w[0] = wa; r.w[1] = wb; r.w[2] = wc;
     r.iw[0] = 1.0f / wa; r.iw[1] = 1.0f / wb; r.iw[2] = 1.0f / wc;
-    r.op[0] = a.opacities[t.ia]; r.op[1] = a.opacities[t.ib]; r.op[2] = a.opacities[t.ic];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        r.col[k] = a.colors[3 * (int64_t)t.ia + k];
-        r.col[3 + k] = a.colors[3 * (int64_t)t.ib + k];
-        r.col[6 + k] = a.colors[3 * (int64_t)t.ic + k];
-    }
+    gather_attributes(a, t.ia, t.ib, t.ic, r);
 }
 
 __device__ __forceinline__ void gather_depth(const RasterArgs &a, int j, DepthRecord &r) {
@@ -183,6 +192,18 @@ __device__ __forceinline__ void gather_depth(const RasterArgs &a, int j, DepthRe
     r.z[0] = va.z; r.z[1] = vb.z; r.z[2] = vc.z;
     r.w[0] = va.w; r.w[1] = vb.w; r.w[2] = vc.w;
     r.extent = max3(va.y, vb.y, vc.y) - min3(va.y, vb.y, vc.y);
+}
+
+// A BlendRecord where the triangle's matrix and vertex numbers are known.
+template <typename Ids>
+__device__ __forceinline__ void gather_record(const RasterArgs &a, const real m[9], const Ids &id, BlendRecord &r) {
+#pragma unroll
+    for (int k = 0; k < 9; k++) r.m[k] = m[k];
+    asm volatile("" ::: "memory");  // the matrix is out of the registers before the rest is asked for
+    const real wa = a.vertices[id.x].w, wb = a.vertices[id.y].w, wc = a.vertices[id.z].w;
+    r.w[0] = wa; r.w[1] = wb; r.w[2] = wc;
+    r.iw[0] = 1.0f / wa; r.iw[1] = 1.0f / wb; r.iw[2] = 1.0f / wc;
+    gather_attributes(a, id.x, id.y, id.z, r);
 }
 
 // gather_depth in steps, for a caller that asks for a record's parts before it needs them.  The parts stay as they were
@@ -350,17 +371,31 @@ __device__ __forceinline__ real wave_max(real v) {
     return v;
 }
 
+__device__ __forceinline__ float lane_value(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane), hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double((long long)((hi << 32) | lo));
+}
+
+__device__ __forceinline__ real first_value(real v) { return lane_value(v, 0); }  // of a value that is the same in all lanes
+
 constexpr int kMaxTileWaves = kTileThreads / kWave;
 
-// Every wave publishes the rectangle of its valid pixels (an empty rectangle,
-// lo > hi, if it has none); call with all threads, followed by __syncthreads().
-__device__ __forceinline__ void publish_wave_rect(const PixelCoord &p, WaveRect *s_rects) {
+// The rectangle of a wave's valid pixels: empty (lo > hi) if it has none.
+__device__ __forceinline__ WaveRect wave_rect(const PixelCoord &p) {
     const real big = 3.0e38f;
     WaveRect r;
-    r.x_lo = wave_min(p.valid ? p.px : big);
-    r.x_hi = wave_max(p.valid ? p.px : -big);
-    r.y_lo = wave_min(p.valid ? p.py : big);
-    r.y_hi = wave_max(p.valid ? p.py : -big);
+    r.x_lo = first_value(wave_min(p.valid ? p.px : big));
+    r.x_hi = first_value(wave_max(p.valid ? p.px : -big));
+    r.y_lo = first_value(wave_min(p.valid ? p.py : big));
+    r.y_hi = first_value(wave_max(p.valid ? p.py : -big));
+    return r;
+}
+
+// Every wave publishes its rectangle; call with all threads, followed by __syncthreads().
+__device__ __forceinline__ void publish_wave_rect(const PixelCoord &p, WaveRect *s_rects) {
+    const WaveRect r = wave_rect(p);
     if ((threadIdx.x & (kWave - 1)) == 0) s_rects[threadIdx.x / kWave] = r;
 }
 
@@ -466,40 +501,29 @@ __device__ __forceinline__ uint64_t transpose_bits(uint64_t x, int lane) {
     return ((uint64_t)b << 32) | a;
 }
 
-__device__ __forceinline__ float lane_value(float v, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane)); }
-__device__ __forceinline__ double lane_value(double v, int lane) {
-    const uint64_t b = (uint64_t)__double_as_longlong(v);
-    const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane), hi = (uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double((long long)((hi << 32) | lo));
-}
-
-// Inside tests the other way round, for the 64 records at s_rec and a wave that owns a square of 8 x 8 pixels: lane = entry.
+// Inside tests the other way round, for 64 entries and a wave that owns a square of 8 x 8 pixels: lane = entry (m: its matrix).
 // A lane (mine: its entry is to be tested) first finds the pixel rows its entry can reach, by the same monotone bound as
 // may_touch on a strip of one row, and then tests the eight pixels of those rows with the arithmetic of the test itself, so
-// the result is that of 64 tests per entry.  -> bit e: entry e covers the calling lane's pixel.
+// the result is that of 64 tests per entry.  -> bit 8 * row + column: the calling lane's entry covers that pixel.
 // A test by broadcast costs about 20 vector instructions per entry for all 64 pixels and waits for its LDS reads (200
 // clocks where a long list leaves its tile alone on the CU); here 64 entries cost 250 instructions and 110 per row of the
 // tallest, all from registers.  500 000 triangles of a mesh, 500 x 500, tile order (longest list 5500 entries): 529 -> 367 us.
-template <typename Rec>
-__device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine, const WaveRect &rect, real px, real py) {
-    const int lane = threadIdx.x & (kWave - 1);
-    real m[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++) m[k] = s_rec[lane].m[k];
+__device__ __forceinline__ uint32_t reached_rows(const real m[9], const WaveRect &rect, real py) {
     uint32_t rows = 0;
-    {
-        real mx[3];
+    real mx[3];
 #pragma unroll
-        for (int k = 0; k < 3; k++) mx[k] = m[3 * k] * (m[3 * k] >= 0.0f ? rect.x_hi : rect.x_lo);
+    for (int k = 0; k < 3; k++) mx[k] = m[3 * k] * (m[3 * k] >= 0.0f ? rect.x_hi : rect.x_lo);
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const real y = lane_value(py, 8 * r);
-            const bool reached = all_inside(mx[0] + m[1] * y + m[2], mx[1] + m[4] * y + m[5], mx[2] + m[7] * y + m[8]);
-            rows |= reached ? 1u << r : 0u;
-        }
-        if (!mine) rows = 0;
+    for (int r = 0; r < 8; r++) {
+        const real y = lane_value(py, 8 * r);
+        const bool reached = all_inside(mx[0] + m[1] * y + m[2], mx[1] + m[4] * y + m[5], mx[2] + m[7] * y + m[8]);
+        rows |= reached ? 1u << r : 0u;
     }
-    uint64_t covered = 0;  // of my entry: bit 8 * row + column
+    return rows;
+}
+// rows: the pixel rows to test.
+__device__ __forceinline__ uint64_t covered_pixels(const real m[9], uint32_t rows, real px, real py) {
+    uint64_t covered = 0;
     while (__builtin_amdgcn_ballot_w64(rows != 0)) {  // wave-uniform
         const int r = rows ? __builtin_ctz(rows) : 0;
         const real y = __shfl(py, 8 * r, kWave);
@@ -513,7 +537,45 @@ __device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine
         if (rows) covered |= (uint64_t)bits << (8 * r);
         rows &= rows - 1;
     }
-    return transpose_bits(covered, lane);
+    return covered;
+}
+// The same for the 64 records at s_rec -> bit e: entry e covers the calling lane's pixel.
+template <typename Rec>
+__device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine, const WaveRect &rect, real px, real py) {
+    const int lane = threadIdx.x & (kWave - 1);
+    real m[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) m[k] = s_rec[lane].m[k];
+    return transpose_bits(covered_pixels(m, mine ? reached_rows(m, rect, py) : 0u, px, py), lane);
+}
+
+// The inside tests of 64 entries against a wave's pixels where every lane holds an entry's matrix and nothing is in LDS (mine:
+// there is one): 20 or more that can touch the pixels as above, fewer one by one, their matrices read from the lane that has
+// them.  -> bit e: entry e covers the calling lane's pixel; hit: the entries that cover any of the pixels.
+__device__ __forceinline__ uint64_t wave_hits(const real m[9], bool mine, bool by_lane, const WaveRect &rect, real px, real py,
+                                              uint64_t &hit) {
+    int lane = threadIdx.x & (kWave - 1);
+    asm volatile("" : "+v"(lane), "+v"(px), "+v"(py));  // the pixels' coordinates by row and column are made here, not kept by the loop around the call
+    const bool candidate = mine && rect.x_lo <= rect.x_hi && may_touch(m, rect);
+    uint64_t todo = __builtin_amdgcn_ballot_w64(candidate), hits = 0;
+    hit = 0;
+    if (by_lane && __builtin_popcountll(todo) >= kSmallMin) {  // wave-uniform
+        const uint64_t covered = covered_pixels(m, candidate ? reached_rows(m, rect, py) : 0u, px, py);
+        hit = __builtin_amdgcn_ballot_w64(covered != 0);
+        return transpose_bits(covered, lane);
+    }
+    while (todo) {  // wave-uniform
+        const int e = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        real t[9], b0, b1, b2;
+#pragma unroll
+        for (int k = 0; k < 9; k++) t[k] = lane_value(m[k], e);
+        bary_apply(t, px, py, b0, b1, b2);
+        const bool inside = all_inside(b0, b1, b2);
+        if (inside) hits |= 1ull << e;
+        if (__builtin_amdgcn_ballot_w64(inside)) hit |= 1ull << e;
+    }
+    return hits;
 }
 
 // Inside tests of one staged batch for the calling lane's pixel: bit e of the
@@ -554,6 +616,10 @@ __device__ __forceinline__ void batch_hit_mask(const Rec *s_rec, const uint8_t *
         }
         m[wd] = ((uint64_t)half[1] << 32) | half[0];
     }
+}
+
+__device__ __forceinline__ uint32_t lanes_below_mask(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
 // Lowest set bit of a mask of kWords 64-bit words, removed from the mask; -1 if the mask is empty.

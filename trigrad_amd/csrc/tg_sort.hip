@@ -457,14 +457,6 @@ __device__ __forceinline__ uint32_t wave_or_u32(uint32_t v) {
     return v;
 }
 
-// Orders the LDS traffic of one wave: LDS serves a wave's instructions in order, so a lane sees what another
-// lane of its wave wrote by an earlier instruction; this keeps the compiler from moving accesses across.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Ranks the workgroup's THREADS * ITEMS digits (wave-striped order: wave, item, lane) and leaves in place[i]
 // the position of item i in digit order.  Barriers inside; the caller separates calls by one more.
 template <int THREADS, int ITEMS>
