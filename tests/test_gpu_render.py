@@ -268,8 +268,8 @@ def test_long_tiles_shared_out(n, sigma, tw, th, mode, cuda, oracle):
 
 @pytest.mark.parametrize("width,per_pixel_sort", [(1024, True), (1024, False), (512, False)])
 def test_long_tiles_match_the_other_route(width, per_pixel_sort, cuda, monkeypatch):
-    """Some 1100 tiles (of 4096) with lists of 1024 entries and more, where 1024 have a slot; in tile order, with 4096 tiles and
-    with 1024, where the long ones are shared out.  Some depths are NaN: in per-pixel order such a candidate ends a selection, so
+    """Some 1200 tiles (of 4096) with lists of 1024 entries and more, shared out in per-pixel order; in tile order the first of
+    them are started first, and with 1024 tiles the long ones are shared out there too.  Some depths are NaN: in per-pixel order such a candidate ends a selection, so
     what is kept depends on the order of looking.  The frame is that of the stage-by-stage route, which knows no long tile."""
     import torch
     import scenes as S

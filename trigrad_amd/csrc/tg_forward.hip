@@ -14,263 +14,26 @@
 // broadcast LDS reads against 148 B of gathered data per ENTRY.
 #include <algorithm>
 
-#include "tg_frame.hpp"
-#include "tg_raster.hpp"
+#include "tg_forward.hpp"
 
 namespace tg {
 
-struct ForwardOut {
-    real4 *image;
-    real *depthmap;
-    real *weights;
-    int32_t *ends;
-    int32_t *last;
-    real *last_depth;
-    OrderStore order;    // blend order: list positions relative to the tile's start
-    uint64_t *hit_masks; // tile order: which list entries cover which pixel, 64 entries per word (see hit_mask_chunk); may be null
-    const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
-    uint32_t *host_status;        // where the host looks for that word (memory of its own); may be null
-    LongTiles long_tiles;
-    int long_rows;                // rows of workgroups at the start of the grid, for the long tiles
-};
-
-// The workgroups in the first long_rows rows of a forward launch take the tiles with the longest lists (LongTiles), the others
-// the rest in the order of tile_of_workgroup.  A frame without a long tile loses 1 us by the workgroups that find none.
-__device__ __forceinline__ int long_tiles(const ForwardOut &o) { return min(o.long_tiles.words[0], kLongTileSlots); }
-__device__ __forceinline__ TileId long_tile(const ForwardOut &o, int slot) {
-    TileId t;
-    t.index = o.long_tiles.words[1 + slot];
-    t.y = t.index / (int)gridDim.x;
-    t.x = t.index - t.y * (int)gridDim.x;
-    return t;
-}
-// Whether a tile is one of those, of which the first `taken` slots are.
-__device__ __forceinline__ bool is_long_tile(const ForwardOut &o, int tile, int n_entries, int taken) {
-    return o.long_rows && n_entries >= o.long_tiles.limit && (uint32_t)o.long_tiles.slot_of_tile[tile] < (uint32_t)taken;
-}
-
-// Lists whose sort gave up a wait are not to be read (unwritten entries may name anything): the frame's pixels
-// are marked instead, so that the caller sees it in the image itself.
-__device__ __forceinline__ bool lists_invalid(const ForwardOut &o) {
-    if (!o.list_status) return false;
-    const uint32_t status = *o.list_status;
-    if (o.host_status && (blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) == 0)
-        __hip_atomic_store(o.host_status, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    return status != TG_STATUS_OK;
-}
-__device__ __forceinline__ void mark_tile_invalid(const RasterArgs &a, const ForwardOut &o) {
-    if ((int)blockIdx.y < o.long_rows) return;
-    const PixelCoord p = pixel_of_thread(a, tile_of_workgroup<kTileBandForward, kChunkForward>(o.long_rows));
-    if (!p.valid) return;
-    const real nan = std::numeric_limits<real>::quiet_NaN();
-    o.image[p.index] = make_real4(nan, nan, nan, nan);
-    o.depthmap[p.index] = nan;
-    o.weights[p.index] = 0.0f;
-    o.ends[p.index] = 0;
-    if (o.last) o.last[p.index] = 0;
-    if (o.last_depth) o.last_depth[p.index] = nan;
-}
-
-__device__ __forceinline__ void write_pixel(const ForwardOut &o, const PixelCoord &p, PixelState s, int last, real last_depth) {
-    // render.cu:609-618
-    real depth;
-    if (s.weight > kEffZero) {
-        depth = s.depth / s.weight;
-    } else {
-        depth = __builtin_inff();
-        s.weight = 0.0f;
-    }
-    o.depthmap[p.index] = depth;
-    o.weights[p.index] = s.weight;
-    o.ends[p.index] = s.blended;
-    if (o.last) o.last[p.index] = last;
-    if (o.last_depth) o.last_depth[p.index] = last_depth;
-    o.image[p.index] = make_real4(s.c0, s.c1, s.c2, s.alpha);
-}
-
-// A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup, in
-// tile order: each tests 64 of 256 entries, lane = entry, from registers; the records of those that are hit go to LDS, and the
-// first wave composites them in list order.  500 000 triangles of a mesh, 500 x 500 (longest list 5500, a tile one workgroup's
-// chain before): 367 -> 127 us.  s_hits: per wave, which of its 64 entries cover a pixel, then which of them cover any, then which
-// of those are staged.
-__device__ __forceinline__ void long_tile_part(const RasterArgs &a, const ForwardOut &out, const TileId &tile, int part, BlendRecord *s_rec,
-                                               uint64_t (*s_hits)[kWave + 2]) {
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));  // what depends on it is made here, not kept in registers by the loop around the call
-    const int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
-    const int slot = (blockIdx.z * kMaxTileWaves + part) * kWave + lane;
-    const PixelCoord p = pixel_of_slot(a, tile.x, tile.y, slot);
-    const WaveRect rect = wave_rect(p);
-    const bool squares = ((a.tw | a.th) & 7) == 0;
-    PixelState s;  // of the first wave
-    int last = 0;
-    // an entry's matrix and vertex numbers are asked for while the entries before it are composited, its triangle's number
-    // before that; what only the entries that are hit need is read when it is known which they are
-    DepthParts next;
-    const auto entry = [&](int first) { return min(first + tid, end - 1); };
-    next.fetch_triangle(a, entry(start));
-    next.fetch_matrix(a);
-    next.fetch_triangle(a, entry(start + kTileThreads));
-    for (int first = start; first < end; first += kTileThreads) {
-        const bool running = wave == 0 && p.valid && s.alpha > a.thr && s.blended < a.max_layers;
-        if (!__syncthreads_or(running)) break;
-        const real matrix[9] = {next.m0[0], next.m0[1], next.m0[2], next.m0[3], next.m1[0], next.m1[1], next.m1[2], next.m1[3], next.m2};
-        const int3v id = next.id;
-        next.fetch_matrix(a);
-        next.fetch_triangle(a, entry(first + 2 * kTileThreads));
-        uint64_t hit;
-        const uint64_t m = wave_hits(matrix, first + tid < end, squares, rect, p.px, p.py, hit);
-        s_hits[wave][lane] = m;
-        if (lane == 0) s_hits[wave][kWave] = hit;
-        if (out.hit_masks && first + wave * kWave < end) {
-            const int64_t chunk = hit_mask_chunk(start, tile.index, first + wave * kWave - start);
-            out.hit_masks[hit_mask_head_words(out.long_rows) + chunk * ((int64_t)gridDim.z * kTileThreads) + slot] = m;
-        }
-        __syncthreads();
-        int before = 0, total = 0;
-#pragma unroll
-        for (int w = 0; w < kMaxTileWaves; w++) {
-            const int count = __builtin_popcountll(s_hits[w][kWave]);
-            if (w < wave) before += count;
-            total += count;
-        }
-        const int rank = before + (int)lanes_below_mask(hit);
-        for (int round = 0; round < total; round += kBatch) {  // the same for the workgroup
-            const bool staged = ((hit >> lane) & 1) && rank >= round && rank < round + kBatch;
-            const uint64_t group = __builtin_amdgcn_ballot_w64(staged);
-            if (lane == 0) s_hits[wave][kWave + 1] = group;
-            if (staged) gather_record(a, matrix, id, s_rec[rank - round]);
-            __syncthreads();
-            if (wave == 0) {
-                int base = 0;
-                for (int w = 0; w < kMaxTileWaves; w++) {
-                    const uint64_t there = s_hits[w][kWave + 1];
-                    uint64_t bits = s_hits[w][lane] & there;
-                    while (true) {
-                        const bool more = bits && p.valid && s.alpha > a.thr && s.blended < a.max_layers;  // render.cu:578, tested before every fragment
-                        if (__builtin_amdgcn_ballot_w64(more) == 0) break;  // wave-uniform
-                        if (!more) continue;
-                        const int e = __builtin_ctzll(bits);
-                        bits &= bits - 1;
-                        const BlendRecord &b = s_rec[base + __builtin_popcountll(there & ((1ull << e) - 1))];
-                        real b0, b1, b2;
-                        bary_apply(b.m, p.px, p.py, b0, b1, b2);
-                        blend_fragment(s, b, b0, b1, b2);
-                        last = first - start + w * kWave + e + 1;
-                    }
-                    base += __builtin_popcountll(there);
-                }
-            }
-            __syncthreads();
-        }
-    }
-    if (wave == 0 && p.valid) write_pixel(out, p, s, last, 0.0f);
-    // the tile's pixels are four workgroups': the backward pass finds out for itself how far they got
-    if (out.hit_masks && tid == 0) out.hit_masks[hit_mask_head_index(tile.index)] = ~0ull;
-}
-
-// kSplit: the long tiles' work is shared out to four waves (long_tile_part), which takes 121 registers, four waves per SIMD.
-// That is what up to 1024 workgroups fill, so only a launch of more goes without (its long tiles come first, that is all):
-// eight waves per SIMD there (63 registers, nothing in scratch memory): 212 -> 194 us against the 73 registers it would take
+// Eight waves per SIMD (63 registers, nothing in scratch memory): 212 -> 194 us against the 73 registers it would take
 // (10^6 triangles, 1920 x 1080).  No bound in double precision: held to the five waves that the LDS allows it spills (8 x 8
-// tiles: 112 -> 123 us).
-constexpr int kFewTileGroups = 1024;
-// Workgroups for the long tiles, at most: more find nothing to do at 1 us for 128 (per-pixel order: 128 to 1024 within 1 % on
-// the mesh of 1.3 million triangles, 10^5 triangles without a long tile 92 -> 93 us), unless the others leave room: in tile
-// order with few tiles (500 000 triangles of a mesh: 128 groups 230 us, 512 190, 1024 175), and wherever there are no more
-// tiles than CUs.
-constexpr int kLongGroups = 128, kLongGroupsFewTiles = 1024;
-template <bool kSplit>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kSplit ? 4 : 8) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
-    __shared__ BlendRecord s_rec[kBatch];
-    __shared__ uint8_t s_touch[kBatch];
-    __shared__ WaveRect s_rects[kMaxTileWaves];
-    const int tid = threadIdx.x;
-    const int wave = tid / kWave;
-    const int n_waves = blockDim.x / kWave;
+// tiles: 112 -> 123 us).  The tiles with the longest lists are started first, as far as there are workgroups for them; a launch
+// of few workgroups shares their work out instead (forward_tile_order_few_kernel).
+__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
+    __shared__ TileOrderLds s;
     if (lists_invalid(out)) {  // the same for the whole launch
         mark_tile_invalid(a, out);
         return;
     }
-    TileId tile_id;
-    if ((int)blockIdx.y < out.long_rows) {
-        const int group = (int)(blockIdx.y * gridDim.x + blockIdx.x), groups = out.long_rows * (int)gridDim.x;
-        if constexpr (kSplit) {
-            __shared__ uint64_t s_hits[kMaxTileWaves][kWave + 2];
-            const int n_items = kMaxTileWaves * long_tiles(out);
-            for (int item = group; item < n_items; item += groups) long_tile_part(a, out, long_tile(out, item / kMaxTileWaves), item % kMaxTileWaves, s_rec, s_hits);
-            return;
-        } else {
-            if (group >= long_tiles(out)) return;
-            tile_id = long_tile(out, group);
-        }
-    } else {
-        tile_id = tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
-    }
-    const int tile = tile_id.index;
-    const int start = a.offsets[tile], end = a.offsets[tile + 1];
-    if ((int)blockIdx.y >= out.long_rows && is_long_tile(out, tile, end - start, kSplit ? kLongTileSlots : out.long_rows * (int)gridDim.x)) return;
-    const PixelCoord p = pixel_of_thread(a, tile_id);
-    publish_wave_rect(p, s_rects);
-    const bool tests_small = tests_small_entries(a, end - start, (int)(gridDim.x * (gridDim.y - out.long_rows)));
-    uint64_t *const masks = out.hit_masks ? out.hit_masks + hit_mask_head_words(out.long_rows) : nullptr;
-
-    PixelState s;
-    int last = 0;
-    for (int batch = start; batch < end; batch += kBatch) {
-        const bool running = p.valid && s.alpha > a.thr && s.blended < a.max_layers;
-        if (!__syncthreads_or(running)) break;
-        const int nb = min(kBatch, end - batch);
-        for (int e = tid; e < nb; e += blockDim.x) {
-            gather_blend(a, batch + e, s_rec[e]);
-            s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, tests_small));
-        }
-        __syncthreads();
-        // 1. inside tests; a lane keeps its hits as a 256-bit mask
-        uint64_t m[kBatch / kWave];
-        batch_hit_mask<kBatch / kWave>(s_rec, s_touch, s_rects, nb, wave, p.px, p.py, m);
-        if (!running) {
-#pragma unroll
-            for (int wd = 0; wd < kBatch / kWave; wd++) m[wd] = 0;
-        }
-        if (masks) {
-            // kept for the backward pass, which then has no inside test to repeat
-            const int64_t chunk = hit_mask_chunk(start, tile, batch - start);
-            const int64_t slots = (int64_t)gridDim.z * blockDim.x, slot = (int64_t)blockIdx.z * blockDim.x + tid;
-#pragma unroll
-            for (int wd = 0; wd < kBatch / kWave; wd++)
-                if (wd * kWave < nb) masks[(chunk + wd) * slots + slot] = m[wd];
-        }
-        // 2. every lane composites its own hits in list order, so the blend arithmetic
-        //    runs with as many lanes busy as there are pixels with a fragment left
-        while (true) {
-            int e = -1;
-            if (s.alpha > a.thr && s.blended < a.max_layers) e = pop_lowest<kBatch / kWave>(m);  // render.cu:578, tested before every fragment
-            if (__builtin_amdgcn_ballot_w64(e >= 0) == 0) break;  // wave-uniform
-            if (e >= 0) {
-                const BlendRecord &r = s_rec[e];
-                real b0, b1, b2;
-                bary_apply(r.m, p.px, p.py, b0, b1, b2);
-                blend_fragment(s, r, b0, b1, b2);
-                last = batch + e - start + 1;
-            }
-        }
-    }
-    if (p.valid) write_pixel(out, p, s, last, 0.0f);
-    if (out.hit_masks) {
-        // how far into the list this workgroup's pixels got
-        __shared__ int s_last;
-        __syncthreads();
-        if (tid == 0) s_last = 0;
-        __syncthreads();
-        int wave_last = p.valid ? last : 0;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) wave_last = max(wave_last, __shfl_xor(wave_last, off, kWave));
-        if ((tid & (kWave - 1)) == 0 && wave_last > 0) atomicMax(&s_last, wave_last);
-        __syncthreads();
-        if (tid == 0) out.hit_masks[hit_mask_head_index(tile)] = (uint64_t)s_last;
-    }
+    const bool first = (int)blockIdx.y < out.long_rows;
+    if (first && long_group(out) >= tiles_started_first(out)) return;
+    const TileId tile = first ? tile_of_index(out.long_tiles.words[1 + long_group(out)]) : tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
+    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
+    if (!first && is_started_first(out, tile.index, end - start)) return;
+    tile_order_tile(a, out, tile, start, end, s);
 }
 
 // render.cu:338-373 insert_sorted_topk on an LDS candidate list of capacity `cap`.
@@ -683,26 +446,23 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
         mark_tile_invalid(a, out);
         return;
     }
-    TileId tile;
-    if ((int)blockIdx.y < out.long_rows) {
-        const int group = (int)(blockIdx.y * gridDim.x + blockIdx.x), groups = out.long_rows * (int)gridDim.x;
-        if constexpr (kInTurn) {
+    const bool first = (int)blockIdx.y < out.long_rows;
+    if constexpr (kInTurn) {
+        if (first) {
             __shared__ real s_quarter[kStage != kWave ? kTileThreads : 1];  // with depth bounds; batches of 64 go without
-            const int n_items = kMaxTileWaves * long_tiles(out);
-            for (int item = group; item < n_items; item += groups)
-                long_tile_part<kStage, Pos>(a, out, long_tile(out, item / kMaxTileWaves), item % kMaxTileWaves, s_dyn,
+            const int n_items = kMaxTileWaves * out.long_tiles.words[0];
+            for (int item = long_group(out); item < n_items; item += long_groups(out))
+                long_tile_part<kStage, Pos>(a, out, tile_of_index(out.long_tiles.all[item / kMaxTileWaves]), item % kMaxTileWaves, s_dyn,
                                             kStage != kWave ? s_quarter : nullptr);
             return;
-        } else {
-            if (group >= long_tiles(out)) return;
-            tile = long_tile(out, group);
         }
     } else {
-        tile = tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
+        if (first && long_group(out) >= tiles_started_first(out)) return;
     }
+    const TileId tile = first ? tile_of_index(out.long_tiles.words[1 + long_group(out)]) : tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
     const int n_entries = a.offsets[tile.index + 1] - a.offsets[tile.index];
     if (sizeof(Pos) < sizeof(int) && n_entries > kShortList) return;
-    if ((int)blockIdx.y >= out.long_rows && is_long_tile(out, tile.index, n_entries, kInTurn ? kLongTileSlots : out.long_rows * (int)gridDim.x)) return;
+    if (kInTurn ? is_long_tile(out, n_entries) : !first && is_started_first(out, tile.index, n_entries)) return;
     pixel_order_tile<kStage, Pos, kInTurn>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
 }
 
@@ -739,6 +499,11 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
     }
 }
 
+// Workgroups for the long tiles, at most: more find nothing to do at 1 us for 128 (per-pixel order: 128 to 1024 within 1 % on
+// the mesh of 1.3 million triangles, 10^5 triangles without a long tile 92 -> 93 us), unless the others leave room: in tile
+// order with few tiles (500 000 triangles of a mesh: 128 groups 230 us, 512 190, 1024 175), and wherever there are no more
+// tiles than CUs.
+constexpr int kLongGroups = 128, kLongGroupsFewTiles = 1024;
 TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_threads) {
     TileLaunch t;
     const int pixels = tile_w * tile_h;
@@ -835,9 +600,9 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     hipStream_t s = (hipStream_t)stream;
     if (!per_pixel_sort) {
         if (split_tiles)
-            TG_LAUNCH_AS("forward_tile_order_kernel", forward_tile_order_kernel<true>, grid, dim3(n_threads), 0, s, a, o);
+            TG_LAUNCH(forward_tile_order_few_kernel, grid, dim3(n_threads), 0, s, a, o);
         else
-            TG_LAUNCH_AS("forward_tile_order_kernel", forward_tile_order_kernel<false>, grid, dim3(n_threads), 0, s, a, o);
+            TG_LAUNCH(forward_tile_order_kernel, grid, dim3(n_threads), 0, s, a, o);
         return check_launch("forward_tile_order_kernel");
     }
     const size_t lds = pixel_order_lds_bytes(n_threads, kSelectBatch);

@@ -1,0 +1,109 @@
+// tg_forward_few.hip -- the tile-order forward kernel of launches with few workgroups, which shares the long tiles' work out.
+#include "tg_forward.hpp"
+
+namespace tg {
+
+// A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup, in
+// tile order: each tests 64 of 256 entries, lane = entry, from registers; the records of those that are hit go to LDS, and the
+// first wave composites them in list order.  500 000 triangles of a mesh, 500 x 500 (longest list 5500, a tile one workgroup's
+// chain before): 367 -> 127 us.  s_hits: per wave, which of its 64 entries cover a pixel, then which of them cover any, then which
+// of those are staged.
+__device__ __forceinline__ void long_tile_part(const RasterArgs &a, const ForwardOut &out, const TileId &tile, int part, BlendRecord *s_rec,
+                                               uint64_t (*s_hits)[kWave + 2]) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // what depends on it is made here, not kept in registers by the loop around the call
+    const int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
+    const int slot = (blockIdx.z * kMaxTileWaves + part) * kWave + lane;
+    const PixelCoord p = pixel_of_slot(a, tile.x, tile.y, slot);
+    const WaveRect rect = wave_rect(p);
+    const bool squares = ((a.tw | a.th) & 7) == 0;
+    PixelState s;  // of the first wave
+    int last = 0;
+    // an entry's matrix and vertex numbers are asked for while the entries before it are composited, its triangle's number
+    // before that; what only the entries that are hit need is read when it is known which they are
+    DepthParts next;
+    const auto entry = [&](int first) { return min(first + tid, end - 1); };
+    next.fetch_triangle(a, entry(start));
+    next.fetch_matrix(a);
+    next.fetch_triangle(a, entry(start + kTileThreads));
+    for (int first = start; first < end; first += kTileThreads) {
+        const bool running = wave == 0 && p.valid && s.alpha > a.thr && s.blended < a.max_layers;
+        if (!__syncthreads_or(running)) break;
+        const real matrix[9] = {next.m0[0], next.m0[1], next.m0[2], next.m0[3], next.m1[0], next.m1[1], next.m1[2], next.m1[3], next.m2};
+        const int3v id = next.id;
+        next.fetch_matrix(a);
+        next.fetch_triangle(a, entry(first + 2 * kTileThreads));
+        uint64_t hit;
+        const uint64_t m = wave_hits(matrix, first + tid < end, squares, rect, p.px, p.py, hit);
+        s_hits[wave][lane] = m;
+        if (lane == 0) s_hits[wave][kWave] = hit;
+        if (out.hit_masks && first + wave * kWave < end) {
+            const int64_t chunk = hit_mask_chunk(start, tile.index, first + wave * kWave - start);
+            out.hit_masks[hit_mask_head_words(out.long_rows) + chunk * ((int64_t)gridDim.z * kTileThreads) + slot] = m;
+        }
+        __syncthreads();
+        int before = 0, total = 0;
+#pragma unroll
+        for (int w = 0; w < kMaxTileWaves; w++) {
+            const int count = __builtin_popcountll(s_hits[w][kWave]);
+            if (w < wave) before += count;
+            total += count;
+        }
+        const int rank = before + (int)lanes_below_mask(hit);
+        for (int round = 0; round < total; round += kBatch) {  // the same for the workgroup
+            const bool staged = ((hit >> lane) & 1) && rank >= round && rank < round + kBatch;
+            const uint64_t group = __builtin_amdgcn_ballot_w64(staged);
+            if (lane == 0) s_hits[wave][kWave + 1] = group;
+            if (staged) gather_record(a, matrix, id, s_rec[rank - round]);
+            __syncthreads();
+            if (wave == 0) {
+                int base = 0;
+                for (int w = 0; w < kMaxTileWaves; w++) {
+                    const uint64_t there = s_hits[w][kWave + 1];
+                    uint64_t bits = s_hits[w][lane] & there;
+                    while (true) {
+                        const bool more = bits && p.valid && s.alpha > a.thr && s.blended < a.max_layers;  // render.cu:578, tested before every fragment
+                        if (__builtin_amdgcn_ballot_w64(more) == 0) break;  // wave-uniform
+                        if (!more) continue;
+                        const int e = __builtin_ctzll(bits);
+                        bits &= bits - 1;
+                        const BlendRecord &b = s_rec[base + __builtin_popcountll(there & ((1ull << e) - 1))];
+                        real b0, b1, b2;
+                        bary_apply(b.m, p.px, p.py, b0, b1, b2);
+                        blend_fragment(s, b, b0, b1, b2);
+                        last = first - start + w * kWave + e + 1;
+                    }
+                    base += __builtin_popcountll(there);
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (wave == 0 && p.valid) write_pixel(out, p, s, last, 0.0f);
+    // the tile's pixels are four workgroups': the backward pass finds out for itself how far they got
+    if (out.hit_masks && tid == 0) out.hit_masks[hit_mask_head_index(tile.index)] = ~0ull;
+}
+
+// Shared out, a tile with a long list is four waves' work for each of its squares.  That takes 121 registers, four waves per
+// SIMD, which up to 1024 workgroups do not need more of; a launch of more is better off with eight (forward_tile_order_kernel).
+__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void forward_tile_order_few_kernel(RasterArgs a, ForwardOut out) {
+    __shared__ TileOrderLds s;
+    if (lists_invalid(out)) {  // the same for the whole launch
+        mark_tile_invalid(a, out);
+        return;
+    }
+    if ((int)blockIdx.y < out.long_rows) {
+        __shared__ uint64_t s_hits[kMaxTileWaves][kWave + 2];
+        const int n_items = kMaxTileWaves * out.long_tiles.words[0];
+        for (int item = long_group(out); item < n_items; item += long_groups(out))
+            long_tile_part(a, out, tile_of_index(out.long_tiles.all[item / kMaxTileWaves]), item % kMaxTileWaves, s.rec, s_hits);
+        return;
+    }
+    const TileId tile = tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
+    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
+    if (is_long_tile(out, end - start)) return;
+    tile_order_tile(a, out, tile, start, end, s);
+}
+
+}  // namespace tg

@@ -22,7 +22,7 @@ struct FrameLayout {
     // kept: what the backward pass and the caller look at later
     size_t status, ids, offsets, bary, weights, ends, last, last_depth, order, masks, kept_bytes;
     // scratch: dead when the forward pass is done
-    size_t keys, keys_alt, values_alt, sort, long_tiles, slots, bounds, far_start, low, scratch_bytes;
+    size_t keys, keys_alt, values_alt, sort, long_tiles, all_long_tiles, bounds, far_start, low, scratch_bytes;
     size_t sort_bytes, zero_bytes;  // of the sort's workspace, and what of it (and of the long tiles' count) starts at zero
     int long_limit;                 // list entries that make a tile a long one; 0: the frame has no use for them
 };
@@ -65,10 +65,10 @@ static FrameLayout frame_layout(const tg_frame &f) {
     const int64_t longest = f.key_capacity < f.n_triangles ? f.key_capacity : f.n_triangles;
     const int64_t at_once = 256 * (f.per_pixel_sort ? 3 : 8);
     const int64_t limit = std::max<int64_t>(1024, ceil_div64(2 * f.key_capacity, std::max<int64_t>(tiles, 2 * at_once)));
-    if (longest >= limit) {
-        L.long_limit = (int)limit;
+    if (longest >= limit) L.long_limit = (int)limit;
+    if (L.long_limit || tiles <= at_once) {  // where the place is small, it is there whatever the number of triangles
         L.long_tiles = take((1 + kLongTileSlots) * 4);
-        L.slots = take((size_t)tiles * 4);
+        L.all_long_tiles = take((size_t)tiles * 4);
         L.zero_bytes = L.long_tiles + 4 - L.sort;
     }
     if (f.flags & TG_FRAME_LIST_BOUNDS) {
@@ -167,7 +167,7 @@ extern "C" int tg_frame_forward(tg_frame *f) {
     volatile uint32_t *host = f->host;
     const int64_t longest = f->key_capacity < f->n_triangles ? f->key_capacity : f->n_triangles;  // a triangle is in a list once
     LongTiles long_tiles;
-    if (L.long_limit) long_tiles = LongTiles{(int32_t *)(scratch + L.long_tiles), (int32_t *)(scratch + L.slots), L.long_limit, std::min<int64_t>(tiles, f->key_capacity / L.long_limit)};
+    if (L.long_limit) long_tiles = LongTiles{(int32_t *)(scratch + L.long_tiles), (int32_t *)(scratch + L.all_long_tiles), L.long_limit, std::min<int64_t>(tiles, f->key_capacity / L.long_limit)};
     if (f->phases & TG_FRAME_BIN) {
         host[1] = 0;
         host[2] = TG_FRAME_PENDING;

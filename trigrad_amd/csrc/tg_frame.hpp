@@ -20,15 +20,14 @@ struct FrameCount {
     }
 };
 
-// The tiles with the longest lists, for a kernel that starts with them and shares their work out: a tile's list is one
+// The tiles with the longest lists, for a kernel that starts with them, or shares their work out: a tile's list is one
 // workgroup's serial work, and what the whole launch waits for is the longest.  The segment sort, which makes the lists'
-// bounds, gives every tile with `limit` entries or more a slot while there are any.  words: how many have one or asked for
-// one, then their tiles; slot_of_tile: every tile's slot, negative for none; most: no more tiles than that can have one.
-// Null words: no such list.
-constexpr int kLongTileSlots = 1024;
+// bounds, notes every tile with `limit` entries or more.  words: how many there are, then the first kLongTileSlots of them; all:
+// all of them; most: no more of them are possible.  Null words: there can be none.
+constexpr int kLongTileSlots = 128;
 struct LongTiles {
     int32_t *words = nullptr;
-    int32_t *slot_of_tile = nullptr;
+    int32_t *all = nullptr;  // room for every tile
     int limit = 0;
     int64_t most = 0;
 };

@@ -682,13 +682,10 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
                 const int end = (int)(length < n_pairs - sum ? sum + length : n_pairs);
                 if (wave == kSortWaves - 1 || t == n_segments - 1) s_bounds[wave + 1] = end;
                 if (t == n_segments - 1) offsets[n_segments] = end;
-                if (long_tiles.words) {
-                    int slot = -1;
-                    if (end - (int)sum >= long_tiles.limit) {
-                        slot = atomicAdd(long_tiles.words, 1);
-                        if (slot < kLongTileSlots) long_tiles.words[1 + slot] = t; else slot = -1;
-                    }
-                    long_tiles.slot_of_tile[t] = slot;
+                if (long_tiles.words && end - (int)sum >= long_tiles.limit) {
+                    const int slot = atomicAdd(long_tiles.words, 1);
+                    if (slot < kLongTileSlots) long_tiles.words[1 + slot] = t;
+                    long_tiles.all[slot] = t;
                 }
             }
         }
