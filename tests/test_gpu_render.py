@@ -227,71 +227,6 @@ def test_more_long_tiles_than_slots_in_tile_order(cuda, monkeypatch):
         assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
 
 
-@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "A_unlimited", "B_3_layers", "B_unlimited"])
-@pytest.mark.parametrize("n,sigma,tw,th", [
-    (1023, 0.7, 16, 16), (1024, 0.7, 16, 16),  # at the rule's edge
-    (1025, 0.7, 16, 16), (1281, 5.0, 16, 16),  # a block of one entry; triangles that cover most of the tile
-    (2500, 2.0, 32, 32), (1500, 2.0, 24, 16),  # the tile's squares are several workgroups'
-    (1100, 3.0, 20, 13),  # a wave's pixels are no square
-])
-def test_long_tiles_shared_out(n, sigma, tw, th, mode, cuda, oracle):
-    """Tiles whose lists of 1024 entries and more are four waves' work: one list of n next to short ones, forward and backward,
-    with lists that are longer than the layers a selection takes and partial tiles on both sides."""
-    import torch
-    import scenes as S
-    from trigrad_amd import _C
-    width, height = 3 * tw - 5, 2 * th - 3
-    scene = S.random_soup(n + 60, tw, th, seed=n, sigma_px=sigma, opacity=(0.02, 0.2), varying_w=True)
-    v = scene["vertices"].reshape(n + 60, 3, 4)
-    rng = np.random.default_rng(n)
-    xy = rng.uniform(-0.7, 0.7, (2 * n, 1, 2)) + rng.standard_normal((2 * n, 3, 2)) * sigma * 2.0 / np.array([tw, th])
-    xy = np.clip(xy, -0.98, 0.98)
-    edges = xy[:, 1:] - xy[:, :1]
-    xy = xy[np.abs(np.linalg.det(edges)) > 1e-3][:n]  # a triangle without an area is in no list
-    v[:n, :, :2] = (xy + 1.0) * np.array([tw / width, th / height]) - 1.0  # into the first tile
-    v[n:, :, 0] = v[n:, :, 0] * 0.3 + 0.6  # the others beside it
-    scene.update(width=width, height=height)
-    m = MODES[mode]
-    d, want, got, ml = _forward_both(scene, tw, th, m, cuda, oracle)
-    assert np.diff(want["offsets"])[0] == n and np.diff(want["offsets"])[1:].max() < 100
-    _check_forward(f"long tile {n}/{tw}x{th}/{mode}", want, got, (th, tw))
-    gi, gd = _grad_inputs(scene, 9, True)
-    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
-                                    tw, th, m["per_pixel_sort"], ml, literal=False, magnitudes=True)
-    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
-    out = _C.render_backward(torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda), d["vertices"], d["indices"], d["colors"],
-                             d["opacities"], sorted_ids, offsets, bary, image, depthmap, weights, ends, width, height, tw, th, 1 / 256,
-                             m["per_pixel_sort"], ml, resume=resume)
-    for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
-        assert_gradients_close(f"long tile {n}/{mode}: {label}", g.cpu().numpy(), w, mag)
-
-
-@pytest.mark.parametrize("width,per_pixel_sort", [(1024, True), (1024, False), (512, False)])
-def test_long_tiles_match_the_other_route(width, per_pixel_sort, cuda, monkeypatch):
-    """Some 1200 tiles (of 4096) with lists of 1024 entries and more, shared out in per-pixel order; in tile order the first of
-    them are started first, and with 1024 tiles the long ones are shared out there too.  Some depths are NaN: in per-pixel order such a candidate ends a selection, so
-    what is kept depends on the order of looking.  The frame is that of the stage-by-stage route, which knows no long tile."""
-    import torch
-    import scenes as S
-    from trigrad_amd import _C
-    side = 36 if width == 1024 else 10  # tiles to a side of the crowded corner
-    n = side * side * 1250
-    soup = S.random_soup(n, width, width, seed=8, sigma_px=0.6, opacity=(0.1, 0.6))
-    v = soup["vertices"].reshape(n, 3, 4).copy()
-    v[: n * 97 // 100, :, :2] = (v[: n * 97 // 100, :, :2] + 1.0) * (side * 16 / width) - 1.0
-    v[::5003, 1, 2] = np.nan
-    d = to_device(dict(soup, vertices=v.reshape(-1, 4)), cuda)
-    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, width, 16, 16, 1 / 256, True, per_pixel_sort, 32)
-    for _ in range(3):  # the first frame's buffers are made for a guess of K, and what is long depends on them
-        got = _C.render_forward(*args)
-    lengths = got[4][1:] - got[4][:-1]
-    assert int((lengths >= 1024).sum()) > (1024 if width == 1024 else 64)
-    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
-    want = _C.render_forward(*args)
-    for i in (0, 1, 2, 3, 4, 5, 6):
-        assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
-
-
 def _grad_inputs(scene, seed, with_depth):
     rng = np.random.default_rng(seed)
     H, W = scene["height"], scene["width"]
@@ -1152,3 +1087,68 @@ def test_order_pool_of_a_first_frame_is_made_for_its_keys(n_triangles, keep, cud
         grads = torch.autograd.grad((image,), leaves, (torch.from_numpy(gi).to(cuda),))
         for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), grads, wanted[:3], wanted[3:]):
             assert_gradients_close(f"pool of a first frame: {label}", g.cpu().numpy(), w, mag)
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "A_unlimited", "B_3_layers", "B_unlimited"])
+@pytest.mark.parametrize("n,sigma,tw,th", [
+    (1023, 0.7, 16, 16), (1024, 0.7, 16, 16),  # at the rule's edge
+    (1025, 0.7, 16, 16), (1281, 5.0, 16, 16),  # a block of one entry; triangles that cover most of the tile
+    (2500, 2.0, 32, 32), (1500, 2.0, 24, 16),  # the tile's squares are several workgroups'
+    (1100, 3.0, 20, 13),  # a wave's pixels are no square
+])
+def test_long_tiles_shared_out(n, sigma, tw, th, mode, cuda, oracle):
+    """Tiles whose lists of 1024 entries and more are four waves' work: one list of n next to short ones, forward and backward,
+    with lists that are longer than the layers a selection takes and partial tiles on both sides."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    width, height = 3 * tw - 5, 2 * th - 3
+    scene = S.random_soup(n + 60, tw, th, seed=n, sigma_px=sigma, opacity=(0.02, 0.2), varying_w=True)
+    v = scene["vertices"].reshape(n + 60, 3, 4)
+    rng = np.random.default_rng(n)
+    xy = rng.uniform(-0.7, 0.7, (2 * n, 1, 2)) + rng.standard_normal((2 * n, 3, 2)) * sigma * 2.0 / np.array([tw, th])
+    xy = np.clip(xy, -0.98, 0.98)
+    edges = xy[:, 1:] - xy[:, :1]
+    xy = xy[np.abs(np.linalg.det(edges)) > 1e-3][:n]  # a triangle without an area is in no list
+    v[:n, :, :2] = (xy + 1.0) * np.array([tw / width, th / height]) - 1.0  # into the first tile
+    v[n:, :, 0] = v[n:, :, 0] * 0.3 + 0.6  # the others beside it
+    scene.update(width=width, height=height)
+    m = MODES[mode]
+    d, want, got, ml = _forward_both(scene, tw, th, m, cuda, oracle)
+    assert np.diff(want["offsets"])[0] == n and np.diff(want["offsets"])[1:].max() < 100
+    _check_forward(f"long tile {n}/{tw}x{th}/{mode}", want, got, (th, tw))
+    gi, gd = _grad_inputs(scene, 9, True)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
+                                    tw, th, m["per_pixel_sort"], ml, literal=False, magnitudes=True)
+    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
+    out = _C.render_backward(torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda), d["vertices"], d["indices"], d["colors"],
+                             d["opacities"], sorted_ids, offsets, bary, image, depthmap, weights, ends, width, height, tw, th, 1 / 256,
+                             m["per_pixel_sort"], ml, resume=resume)
+    for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+        assert_gradients_close(f"long tile {n}/{mode}: {label}", g.cpu().numpy(), w, mag)
+
+
+@pytest.mark.parametrize("width,per_pixel_sort", [(1024, True), (1024, False), (512, False)])
+def test_long_tiles_match_the_other_route(width, per_pixel_sort, cuda, monkeypatch):
+    """Some 1200 tiles (of 4096) with lists of 1024 entries and more, shared out in per-pixel order; in tile order the first of
+    them are started first, and with 1024 tiles the long ones are shared out there too.  Some depths are NaN: in per-pixel order such a candidate ends a selection, so
+    what is kept depends on the order of looking.  The frame is that of the stage-by-stage route, which knows no long tile."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    side = 36 if width == 1024 else 10  # tiles to a side of the crowded corner
+    n = side * side * 1250
+    soup = S.random_soup(n, width, width, seed=8, sigma_px=0.6, opacity=(0.1, 0.6))
+    v = soup["vertices"].reshape(n, 3, 4).copy()
+    v[: n * 97 // 100, :, :2] = (v[: n * 97 // 100, :, :2] + 1.0) * (side * 16 / width) - 1.0
+    v[::5003, 1, 2] = np.nan
+    d = to_device(dict(soup, vertices=v.reshape(-1, 4)), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, width, 16, 16, 1 / 256, True, per_pixel_sort, 32)
+    for _ in range(3):  # the first frame's buffers are made for a guess of K, and what is long depends on them
+        got = _C.render_forward(*args)
+    lengths = got[4][1:] - got[4][:-1]
+    assert int((lengths >= 1024).sum()) > (1024 if width == 1024 else 64)
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C.render_forward(*args)
+    for i in (0, 1, 2, 3, 4, 5, 6):
+        assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i

@@ -67,17 +67,24 @@ __device__ __forceinline__ float reciprocal(float x) {
     return __builtin_amdgcn_classf(r, 0x198) ? refined : r;  // +-normal, +-denormal
 }
 __device__ __forceinline__ double reciprocal(double x) { return 1.0 / x; }
+// x / y from r = reciprocal(y): the quotient x * r put right by its exact remainder, two fused operations (Markstein's
+// correction).  What is rounded at the end is the exact quotient to within some 2^-22 units in the last place, so the result is
+// the correctly rounded one, but for a few operand pairs in millions that are as close to a tie.  Where x * r is no ordinary
+// number (an infinite x, say) the remainder is none either; then it is x / y as it is.
+__device__ __forceinline__ float quotient(float x, float y, float r) {
+    const float q = x * r;
+    const float corrected = __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
+    return __builtin_amdgcn_classf(q, 0x1f8) ? corrected : q;  // +-normal, +-denormal, +-0
+}
+__device__ __forceinline__ double quotient(double x, double y, double) { return x / y; }
 
 __device__ __forceinline__ void gather_back(const RasterArgs &a, int j, BackRecord &r) {
     const TriIds t = load_ids(a, j);
     const real *m = a.bary + 9 * (int64_t)t.tri;
+    real4v va = *reinterpret_cast<const real4v *>(a.vertices + t.ia), vb = *reinterpret_cast<const real4v *>(a.vertices + t.ib),
+           vc = *reinterpret_cast<const real4v *>(a.vertices + t.ic);
 #pragma unroll
     for (int k = 0; k < 9; k++) r.m[k] = m[k];
-    const real4 va = a.vertices[t.ia], vb = a.vertices[t.ib], vc = a.vertices[t.ic];
-    r.w[0] = va.w; r.w[1] = vb.w; r.w[2] = vc.w;
-    // gradients only: 1 / w to within one unit in the last place, and its square for 1 / (w * w)
-    r.iw[0] = reciprocal(va.w); r.iw[1] = reciprocal(vb.w); r.iw[2] = reciprocal(vc.w);
-    r.iw2[0] = r.iw[0] * r.iw[0]; r.iw2[1] = r.iw[1] * r.iw[1]; r.iw2[2] = r.iw[2] * r.iw[2];
     r.op[0] = a.opacities[t.ia]; r.op[1] = a.opacities[t.ib]; r.op[2] = a.opacities[t.ic];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -85,10 +92,16 @@ __device__ __forceinline__ void gather_back(const RasterArgs &a, int j, BackReco
         r.col[3 + k] = a.colors[3 * (int64_t)t.ib + k];
         r.col[6 + k] = a.colors[3 * (int64_t)t.ic + k];
     }
-    r.xy[0] = va.x; r.xy[1] = va.y; r.xy[2] = vb.x; r.xy[3] = vb.y; r.xy[4] = vc.x; r.xy[5] = vc.y;
+    // z is not used, and without this a vertex would be two loads, x and y, and w (14 instead of 17 loads an entry: 1 % of the
+    // saved-order kernel); here, behind all loads, because it is where they are waited for
+    asm("" : "+v"(va), "+v"(vb), "+v"(vc));
+    r.w[0] = va[3]; r.w[1] = vb[3]; r.w[2] = vc[3];
+    // gradients only: 1 / w to within one unit in the last place, and its square for 1 / (w * w)
+    r.iw[0] = reciprocal(r.w[0]); r.iw[1] = reciprocal(r.w[1]); r.iw[2] = reciprocal(r.w[2]);
+    r.iw2[0] = r.iw[0] * r.iw[0]; r.iw2[1] = r.iw[1] * r.iw[1]; r.iw2[2] = r.iw[2] * r.iw[2];
+    r.xy[0] = va[0]; r.xy[1] = va[1]; r.xy[2] = vb[0]; r.xy[3] = vb[1]; r.xy[4] = vc[0]; r.xy[5] = vc[1];
     r.id[0] = t.ia; r.id[1] = t.ib; r.id[2] = t.ic;
 }
-
 
 // Reverse-traversal state of one pixel (render.cu:647-653).
 struct BackState {
@@ -108,12 +121,12 @@ __device__ __forceinline__ void interp_backward_scalar(real g, const real b[3], 
     // around the assignments of three arrays makes the compiler keep them in scratch memory
     const bool dead = denom * denom < kEffZero;
     const real inv = reciprocal(denom);  // the reference divides nine times, by denom and by its square
-    const real inv2 = inv * inv;
+    const real inv2 = inv * inv, g_inv2 = g * inv2;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         gb[k] = dead ? 0.0f : g * ((v[k] * w[k] * denom - nom * w[k]) * inv2);
         gv[k] = dead ? 0.0f : g * b[k] * w[k] * inv;
-        gw[k] = dead ? 0.0f : g * (b[k] * v[k] * denom - nom * b[k]) * inv2;
+        gw[k] = dead ? 0.0f : g_inv2 * (b[k] * v[k] * denom - nom * b[k]);
     }
 }
 
@@ -163,7 +176,7 @@ __device__ __forceinline__ FragSeed fragment_chain_step(BackState &st, const Fra
 #pragma unroll
     for (int k = 0; k < 3; k++) t3[k] = (color[k] * st.alpha - s[k]) * inv_om * g[k];
     const real drgb_do = ((t3[0] + t3[1]) + t3[2]) + st.g3 * (-st.final_alpha * inv_om);  // :491
-    st.alpha /= om;                                                                        // :492 (state: kept exact)
+    st.alpha = quotient(st.alpha, om, inv_om);                                             // :492 (state: kept exact)
 #pragma unroll
     for (int k = 0; k < 3; k++) s[k] += color[k] * o * st.alpha;                       // :493
     st.s0 = s[0]; st.s1 = s[1]; st.s2 = s[2];
@@ -213,10 +226,10 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
             for (int k = 0; k < 3; k++) {
                 const real a = r.col[3 * v + k];
                 dfb[k] = w[v] * (a * denom - nom[k]) * inv2;
-                dfw[k] = (b[v] * a * denom - nom[k] * b[v]) * inv2;
+                dfw[k] = b[v] * a * denom - nom[k] * b[v];
             }
             gb_c[v] = dead ? 0.0f : (gc[0] * dfb[0] + gc[1] * dfb[1]) + gc[2] * dfb[2];
-            gw_c[v] = dead ? 0.0f : (gc[0] * dfw[0] + gc[1] * dfw[1]) + gc[2] * dfw[2];
+            gw_c[v] = dead ? 0.0f : ((gc[0] * dfw[0] + gc[1] * dfw[1]) + gc[2] * dfw[2]) * inv2;
             scale[v] = dead ? 0.0f : b[v] * w[v] * inv;
         }
     }
@@ -249,30 +262,31 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
         const real d = ax * (by - cy) + bx * (-ay + cy) + cx * (ay - by);
         const bool flat = abs_real(d) < kEffZero;  // util.h:421: zero (selection, not a branch: see above)
         {
-            const real inv_d = reciprocal(d);
+            const real inv_d = reciprocal(d);  // of the sum, not of its 18 numerators: 12 multiplications and as many roundings less
             real J[3][2][3];
-            J[0][0][0] = l0 * (-by + cy) * inv_d;
-            J[0][0][1] = (-cy - l1 * (by - cy) + py) * inv_d;
-            J[0][0][2] = (by - l2 * (by - cy) - py) * inv_d;
-            J[0][1][0] = l0 * (bx - cx) * inv_d;
-            J[0][1][1] = (cx + l1 * (bx - cx) - px) * inv_d;
-            J[0][1][2] = (-bx + l2 * (bx - cx) + px) * inv_d;
-            J[1][0][0] = (cy + l0 * (ay - cy) - py) * inv_d;
-            J[1][0][1] = l1 * (ay - cy) * inv_d;
-            J[1][0][2] = (-ay + l2 * (ay - cy) + py) * inv_d;
-            J[1][1][0] = (-cx - l0 * (ax - cx) + px) * inv_d;
-            J[1][1][1] = l1 * (-ax + cx) * inv_d;
-            J[1][1][2] = (ax - l2 * (ax - cx) - px) * inv_d;
-            J[2][0][0] = (-by - l0 * (ay - by) + py) * inv_d;
-            J[2][0][1] = (ay - l1 * (ay - by) - py) * inv_d;
-            J[2][0][2] = l2 * (-ay + by) * inv_d;
-            J[2][1][0] = (bx + l0 * (ax - bx) - px) * inv_d;
-            J[2][1][1] = (-ax + l1 * (ax - bx) + px) * inv_d;
-            J[2][1][2] = l2 * (ax - bx) * inv_d;
+            J[0][0][0] = l0 * (-by + cy);
+            J[0][0][1] = -cy - l1 * (by - cy) + py;
+            J[0][0][2] = by - l2 * (by - cy) - py;
+            J[0][1][0] = l0 * (bx - cx);
+            J[0][1][1] = cx + l1 * (bx - cx) - px;
+            J[0][1][2] = -bx + l2 * (bx - cx) + px;
+            J[1][0][0] = cy + l0 * (ay - cy) - py;
+            J[1][0][1] = l1 * (ay - cy);
+            J[1][0][2] = -ay + l2 * (ay - cy) + py;
+            J[1][1][0] = -cx - l0 * (ax - cx) + px;
+            J[1][1][1] = l1 * (-ax + cx);
+            J[1][1][2] = ax - l2 * (ax - cx) - px;
+            J[2][0][0] = -by - l0 * (ay - by) + py;
+            J[2][0][1] = ay - l1 * (ay - by) - py;
+            J[2][0][2] = l2 * (-ay + by);
+            J[2][1][0] = bx + l0 * (ax - bx) - px;
+            J[2][1][1] = -ax + l1 * (ax - bx) + px;
+            J[2][1][2] = l2 * (ax - bx);
 #pragma unroll
             for (int v = 0; v < 3; v++)
 #pragma unroll
-                for (int c = 0; c < 2; c++) dxy[v][c] = flat ? 0.0f : gbary[0] * J[v][c][0] + gbary[1] * J[v][c][1] + gbary[2] * J[v][c][2];
+                for (int c = 0; c < 2; c++)
+                    dxy[v][c] = flat ? 0.0f : (gbary[0] * J[v][c][0] + gbary[1] * J[v][c][1] + gbary[2] * J[v][c][2]) * inv_d;
         }
     }
 #pragma unroll
@@ -794,7 +808,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkBackward>();
+    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkSavedOrder>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);
