@@ -499,11 +499,11 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
     }
 }
 
-// Workgroups for the long tiles, at most: more find nothing to do at 1 us for 128 (per-pixel order: 128 to 1024 within 1 % on
-// the mesh of 1.3 million triangles, 10^5 triangles without a long tile 92 -> 93 us), unless the others leave room: in tile
-// order with few tiles (500 000 triangles of a mesh: 128 groups 230 us, 512 190, 1024 175), and wherever there are no more
-// tiles than CUs.
-constexpr int kLongGroups = 128, kLongGroupsFewTiles = 1024;
+// Workgroups for the long tiles, at most, by the number of the others: they cost 1 us for every 300 or so that find nothing to
+// do, and what they find may be too much for them.  Few others (a CU each): 54 tiles of 32 x 32 in tile order 110 us with 1024
+// groups, 158 with 512, 210 with 256.  As many as run at once: mesh of 500 000, 1024 tiles, 121, 121, 149; mesh of 700 000 in
+// per-pixel order, 437 tiles, 308, 310, 317.  More: mesh of 1.3 million, 8160 tiles, 128 to 1024 groups within 1 %.
+constexpr int kLongGroupsFew = 1024, kLongGroupsSome = 512, kLongGroups = 128;
 TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_threads) {
     TileLaunch t;
     const int pixels = tile_w * tile_h;
@@ -591,10 +591,12 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     ForwardOut o{(real4 *)image, depthmap, final_weights, ends, last, last_depth, order, per_pixel_sort ? nullptr : hit_masks,
                  list_status, host_status, long_tiles, 0};
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
-    const bool split_tiles = !per_pixel_sort && tl.threads == kTileThreads && (int64_t)tl.grid.x * tl.grid.y * tl.grid.z <= kFewTileGroups;
-    if (long_tiles.words)
-        o.long_rows = ceil_div((int)std::min<int64_t>(split_tiles || (int64_t)tl.grid.x * tl.grid.y <= kFewTiles ? kLongGroupsFewTiles : kLongGroups,
-                                                      kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
+    const int64_t groups = (int64_t)tl.grid.x * tl.grid.y * tl.grid.z;
+    const bool split_tiles = !per_pixel_sort && tl.threads == kTileThreads && groups <= kFewTileGroups;
+    if (long_tiles.words) {
+        const int most = groups <= 256 ? kLongGroupsFew : split_tiles || groups <= 768 ? kLongGroupsSome : kLongGroups;
+        o.long_rows = ceil_div((int)std::min<int64_t>(ceil_div(most, (int)tl.grid.z), kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
+    }
     const dim3 grid(tl.grid.x, tl.grid.y + o.long_rows, tl.grid.z);
     const int n_threads = tl.threads;
     hipStream_t s = (hipStream_t)stream;
