@@ -1152,3 +1152,24 @@ def test_long_tiles_match_the_other_route(width, per_pixel_sort, cuda, monkeypat
     want = _C.render_forward(*args)
     for i in (0, 1, 2, 3, 4, 5, 6):
         assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
+
+
+@pytest.mark.parametrize("layers", [5, 23, 24, 27, 32, 40, -1])
+@pytest.mark.parametrize("n", [22, 23, 24, 25, 31, 32, 33, 60])
+def test_candidate_lists_around_their_places_in_lds(n, layers, cuda, oracle):
+    """A pixel's first 23 candidates are kept in LDS, the others up to 32 in registers: n triangles over every pixel, tilted, so
+    that their order at a pixel is not the list's, a third of them at equal depths, and layers that end inside either part."""
+    import scenes as S
+    rng = np.random.default_rng(100 * n + layers)
+    size = 24
+    z = rng.uniform(1.0, 5.0, (n, 1)) * rng.uniform(0.5, 1.5, (n, 3))
+    z[::3] = rng.choice([2.0, 3.0], (z[::3].shape[0], 1))
+    xy = np.array([[-9.0, -9.0], [9.0, -9.0], [0.0, 16.0]]) * rng.uniform(0.9, 1.1, (n, 1, 1))
+    vertices = np.concatenate([xy, z[:, :, None], 1.0 / z[:, :, None]], axis=-1).astype(np.float32).reshape(-1, 4)
+    scene = dict(S.random_soup(n, size, size, seed=n, opacity=(0.02, 0.3)), vertices=vertices)
+    mode = dict(per_pixel_sort=True, max_layers=layers)
+    _, want, got, _ = _forward_both(scene, 16, 16, mode, cuda, oracle)
+    assert int(want["ends"].max()) == min(n, layers if layers > 0 else n)
+    _check_forward(f"{n} candidates, {layers} layers", want, got, (16, 16))
+    _, want, got, _ = _forward_both(scene, 8, 8, mode, cuda, oracle)  # one wave to a workgroup
+    _check_forward(f"{n} candidates, {layers} layers, small tiles", want, got, (8, 8))

@@ -38,9 +38,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forwa
 
 // render.cu:338-373 insert_sorted_topk on an LDS candidate list of capacity `cap`.
 template <typename Pos>
-__device__ __forceinline__ void topk_insert(const TopKOf<Pos> &tk, int cap, int &n, real d, int j) {
-    if (n == cap && d >= tk.d(cap - 1)) return;
-    int i = (n < cap) ? n : cap - 1;
+__device__ __forceinline__ void topk_insert_at(const TopKOf<Pos> &tk, int i, real d, int j) {  // place i is free
     while (i > 0 && d < tk.d(i - 1)) {
         tk.d(i) = tk.d(i - 1);
         tk.j(i) = tk.j(i - 1);
@@ -48,25 +46,113 @@ __device__ __forceinline__ void topk_insert(const TopKOf<Pos> &tk, int cap, int 
     }
     tk.d(i) = d;
     tk.j(i) = (Pos)j;
+}
+template <typename Pos>
+__device__ __forceinline__ void topk_insert(const TopKOf<Pos> &tk, int cap, int &n, real d, int j) {
+    if (n == cap && d >= tk.d(cap - 1)) return;
+    topk_insert_at(tk, (n < cap) ? n : cap - 1, d, j);
     if (n < cap) n++;
 }
 
 constexpr int kSelectBatch = 128;       // list entries staged per batch where positions take an int
 constexpr int kSelectBatchShort = 64;   // ... and where they take 16 bits
+// Places of a candidate list in LDS where positions take 16 bits; the rest is in registers (Candidates).  With 23 a workgroup of
+// 256 threads takes 39.4 KB, four a CU, and fits the 128 registers of four waves per SIMD, where 32 were three: 10^6 triangles
+// 601 -> 537 us, 10^5 92 -> 82, 20 000 large ones without a limit on the layers 431 -> 360, the mesh of 1.3 million 327 -> 297,
+// 200 000 around the camera 117 -> 100, 33 000 in tiles of 8 x 8 (a wave to a workgroup) 88 -> 84.  With 22: 548, 83, 372.
+// Lists with depth bounds keep all places in LDS and three kinds of 16-bit positions lose there: 200 000 faint triangles 288
+// us, with 29 places and three workgroups a CU 301, with 21 and four 338: every pixel has 32 candidates.
+constexpr int kShortHead = sizeof(real) == 4 ? 23 : kLayers;
 constexpr int kLongListGroups = 256;    // workgroups that look for the tiles with longer lists
+
+// The last places of a candidate list, in registers: place kPlace and those behind it.  (A structure of its own for every place:
+// of an array the compiler makes scratch memory.)
+template <int kPlace, int kPlaces>
+struct ListTail {
+    real d;
+    int j;
+    ListTail<kPlace + 1, kPlaces> rest;
+    // bit k of places: depth x belongs in place k or further to the front; all: it is less than every one of the `used` first
+    __device__ __forceinline__ void compare(real x, int used, bool &all, uint32_t &places) const {
+        rest.compare(x, used, all, places);
+        all = all && (kPlace >= used || x < d);
+        places |= all && kPlace <= used ? 1u << kPlace : 0u;
+    }
+    __device__ __forceinline__ void insert(uint32_t places, int used, real x, int xj, real front_d, int front_j) {
+        const bool shifted = kPlace > 0 && kPlace <= used && (places >> (kPlace > 0 ? kPlace - 1 : 0) & 1), here = places >> kPlace & 1;
+        const real my_d = d;
+        const int my_j = j;
+        d = shifted ? front_d : here ? x : my_d;
+        j = shifted ? front_j : here ? xj : my_j;
+        rest.insert(places, used, x, xj, my_d, my_j);
+    }
+    __device__ __forceinline__ void read(int place, real &x, int &xj) const {
+        x = place == kPlace ? d : x;
+        xj = place == kPlace ? j : xj;
+        rest.read(place, x, xj);
+    }
+};
+template <int kPlaces>
+struct ListTail<kPlaces, kPlaces> {
+    __device__ __forceinline__ void compare(real, int, bool &, uint32_t &) const {}
+    __device__ __forceinline__ void insert(uint32_t, int, real, int, real, int) {}
+    __device__ __forceinline__ void read(int, real &, int &) const {}
+};
+
+// A pixel's candidates in the per-pixel-order pass: the nearest kHead in LDS, the others (kLayers - kHead) in registers, which
+// few pixels have and which only they pay for.  Insertion is topk_insert's, place by place: from the end of the list to the
+// front, as far as the new depth is less.
+template <typename Pos, int kHead>
+struct Candidates {
+    TopKOf<Pos> head;
+    ListTail<0, kLayers - kHead> tail;
+
+    __device__ __forceinline__ void insert(int cap, int &n, real d, int j) {
+        if constexpr (kHead == kLayers) return topk_insert(head, cap, n, d, j);
+        if (n < kHead || cap <= kHead) {  // fewer than kHead: there is a place, whichever of the two ends it is
+            topk_insert(head, min(cap, kHead), n, d, j);
+            return;
+        }
+        if (n == cap && d >= depth(cap - 1)) return;
+        const int used = n == cap ? cap - 1 - kHead : n - kHead;  // a full list loses its last
+        bool all = true;
+        uint32_t places = 0;
+        tail.compare(d, used, all, places);
+        const real last_d = head.d(kHead - 1);
+        const int last_j = head.j(kHead - 1);
+        const bool to_head = all && d < last_d;  // then the tail takes the head's last one, in its first place
+        tail.insert(places, used, to_head ? last_d : d, to_head ? last_j : j, 0.0f, 0);
+        if (to_head) topk_insert_at(head, kHead - 1, d, j);
+        if (n < cap) n++;
+    }
+    __device__ __forceinline__ real depth(int i) const {
+        if constexpr (kHead == kLayers) return head.d(i);
+        real d = head.d(min(i, kHead - 1));
+        int j = 0;
+        tail.read(i - kHead, d, j);
+        return d;
+    }
+    __device__ __forceinline__ int position(int i) const {
+        if constexpr (kHead == kLayers) return head.j(i);
+        int j = head.j(min(i, kHead - 1));
+        real d = 0.0f;
+        tail.read(i - kHead, d, j);
+        return j;
+    }
+};
 
 // The per-pixel-order forward pass of one tile.  Pos: how a candidate's list position (from the tile's
 // start) is kept.  With uint16_t the candidate lists of a 16x16 tile take 48 KB instead of 64 KB, which
 // together with 64 staged entries lets a CU hold three workgroups instead of two.
-template <int kStage, typename Pos, bool kInTurn>  // kStage: list entries staged per batch
+template <int kStage, typename Pos, bool kInTurn, int kHead>  // kStage: list entries staged per batch
 __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const ForwardOut &out, int tile_x, int tile_y, int tiles_x, int n_tiles,
                                                  unsigned char *s_dyn, uint8_t *s_touch, WaveRect *s_rects) {
     const int n_threads = blockDim.x;
     DepthRecord *s_rec = reinterpret_cast<DepthRecord *>(s_dyn);
-    TopKOf<Pos> tk;
-    tk.depth = reinterpret_cast<real *>(s_dyn + sizeof(DepthRecord) * kStage);
-    tk.pos = reinterpret_cast<Pos *>(tk.depth + kLayers * n_threads);
-    tk.n_threads = n_threads;
+    Candidates<Pos, kHead> tk;
+    tk.head.depth = reinterpret_cast<real *>(s_dyn + sizeof(DepthRecord) * kStage);
+    tk.head.pos = reinterpret_cast<Pos *>(tk.head.depth + kHead * n_threads);
+    tk.head.n_threads = n_threads;
 
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
@@ -120,7 +206,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 // a lane needs nothing from here on when its list is full and its worst candidate is nearer than
                 // every fragment the rest of the tile's list can produce (a full list rejects depths >= its worst)
                 const real rest = a.batch_bounds[batch_bound_index(start, tile, batch - start)];
-                const bool settled = !want || (found == cap && tk.d(cap - 1) <= rest);
+                const bool settled = !want || (found == cap && tk.depth(cap - 1) <= rest);
                 if (__syncthreads_and(settled)) {
                     // on to the batch that holds the first entry the bounds do not cover
                     const int resume = start + a.far_start[tile] / kStage * kStage;
@@ -181,7 +267,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 const int j = batch + e - start;
                 if (pd < last_depth) continue;
                 if (pd == last_depth && j <= last_j) continue;
-                topk_insert(tk, cap, found, pd, j);
+                tk.insert(cap, found, pd, j);
             }
         }
         // Selection is over: the staging area and the depth lists are dead apart from
@@ -190,10 +276,10 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
         // apart: lanes reading different entries use different banks); entries
         // beyond it are gathered from memory.
         const int todo = (want && found > 0) ? min(found, a.max_layers - s.blended) : 0;
-        const real todo_depth = todo > 0 ? tk.d(todo - 1) : 0.0f;
+        const real todo_depth = todo > 0 ? tk.depth(todo - 1) : 0.0f;
         __syncthreads();
         real *rows = reinterpret_cast<real *>(s_dyn);
-        const int n_rows = min(end - start, (int)((sizeof(DepthRecord) * kStage + sizeof(real) * kLayers * n_threads) /
+        const int n_rows = min(end - start, (int)((sizeof(DepthRecord) * kStage + sizeof(real) * kHead * n_threads) /
                                                    (sizeof(real) * kBlendWords)));
         for (int e = tid; e < n_rows; e += blockDim.x) {
             BlendRecord r;
@@ -208,15 +294,14 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 active = false;  // render.cu:594
             } else {
                 // kTogether records are fetched together: the chains of dependent loads (list -> indices -> vertices) of those
-                // that come from memory overlap.  They are the kernel's peak of registers: where a wave's batches are fetched
-                // a whole batch ahead a fourth record would spill (8 x 8 tiles: 87 -> 86 us; two together: lists of
-                // hundreds 220 -> 226)
-                constexpr int kTogether = kInTurn ? 4 : 3;
+                // that come from memory overlap.  They are the kernel's peak of registers (two together where three would
+                // do: lists of hundreds 220 -> 226)
+                constexpr int kTogether = kHead < kLayers ? 1 : kInTurn ? 4 : 3;
                 for (int i0 = 0; i0 < todo; i0 += kTogether) {
                     BlendRecord r[kTogether];
 #pragma unroll
                     for (int u = 0; u < kTogether; u++) {
-                        const int rel = tk.j(min(i0 + u, todo - 1));
+                        const int rel = tk.position(min(i0 + u, todo - 1));
                         if (rel < n_rows) {
                             real *w = reinterpret_cast<real *>(&r[u]);
 #pragma unroll
@@ -233,7 +318,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                         if (!bary_inside(b0, b1, b2)) continue;  // cannot happen: the selection tested it
                         if (s.blended < rows_kept) {
                             const int64_t at = order_at + (int64_t)s.blended * order_step;
-                            const int rel = tk.j(i0 + u);
+                            const int rel = tk.position(i0 + u);
                             out.order.low[at] = (uint16_t)rel;
                             if (sizeof(Pos) > sizeof(uint16_t) && end - start > kShortList)
                                 out.order.low[out.order.high + at] = (uint16_t)(rel >> 16);
@@ -242,7 +327,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                     }
                 }
                 last_depth = todo_depth;
-                last_j = tk.j(todo - 1);
+                last_j = tk.position(todo - 1);
                 // fewer candidates than asked for: the list is exhausted, the next
                 // selection would return nothing (render.cu:594)
                 if (found < cap) active = false;
@@ -250,6 +335,52 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
         }
     }
     if (p.valid) write_pixel(out, p, s, last_j + 1, last_depth);
+}
+
+// Visits the nearest `cap` candidates of a lane's pixel in the four waves' sorted lists, nearest first, by depth and list
+// position: visit(i, depth, position).  short_list: a list was through before that which has dropped candidates.
+// -> how many were visited.
+template <typename Shared, typename Pos, typename Visit>
+__device__ __forceinline__ int merge_lists(const Shared *shared, const TopKOf<Pos> &tk, int lane, int cap, Visit visit, bool &short_list) {
+    const auto depth_at = [&](int w, int i) { return tk.depth[i * tk.n_threads + w * kWave + lane]; };
+    const auto pos_at = [&](int w, int i) { return (int)tk.pos[i * tk.n_threads + w * kWave + lane]; };
+    uint32_t left = 0, at = 0;  // of every list: candidates not visited yet, and the next one's place; a byte each
+    int pos[kMaxTileWaves];
+    real depth[kMaxTileWaves];
+    uint32_t dropped = 0;
+#pragma unroll
+    for (int w = 0; w < kMaxTileWaves; w++) {
+        const int count = shared->found[w * kWave + lane];
+        left |= (uint32_t)count << (8 * w);
+        dropped |= (uint32_t)shared->dropped[w * kWave + lane] << w;
+        depth[w] = count ? depth_at(w, 0) : 0.0f;
+        pos[w] = count ? pos_at(w, 0) : 0;
+    }
+    for (int i = 0; i < cap; i++) {
+        int best = -1, j = 0;
+        real d = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kMaxTileWaves; w++) {
+            if ((left >> (8 * w) & 0xff) == 0) {
+                short_list = short_list || (dropped >> w & 1);
+            } else if (best < 0 || depth[w] < d || (depth[w] == d && pos[w] < j)) {
+                best = w;
+                d = depth[w];
+                j = pos[w];
+            }
+        }
+        if (best < 0) return i;
+        visit(i, d, j);
+        left -= 1u << (8 * best);
+        at += 1u << (8 * best);
+#pragma unroll
+        for (int w = 0; w < kMaxTileWaves; w++)
+            if (w == best && (left >> (8 * w) & 0xff)) {
+                depth[w] = depth_at(w, at >> (8 * w) & 0xff);
+                pos[w] = pos_at(w, at >> (8 * w) & 0xff);
+            }
+    }
+    return cap;
 }
 
 // A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup: each
@@ -261,20 +392,22 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
 // 1.3 million triangles of a mesh, 1920 x 1080 (longest list 5200, 221 of at least 1024): 604 -> 332 us; 200 000 around the
 // camera (one list of 8400): 152 -> 117; 81 tiles with lists of some 2600, where depth bounds end the looking early: 105 -> 91.
 // s_quarter: a depth for every thread, with depth bounds; else null.
-template <int kStage, typename Pos>
+template <int kStage, typename Pos, int kHead>
 __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const ForwardOut &out, const TileId &tile, int part, unsigned char *s_dyn,
                                                volatile real *s_quarter) {
     constexpr int kStaged = kStage / kMaxTileWaves;  // records of a wave in LDS at a time
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // what depends on it is made here, not kept in registers by the loop around the call
+    const int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1], n = end - start;
     if (sizeof(Pos) < sizeof(int) && n > kShortList) return;  // left to forward_pixel_order_long_lists_kernel
     DepthRecord *s_rec = reinterpret_cast<DepthRecord *>(s_dyn) + wave * kStaged;
     TopKOf<Pos> tk;
     tk.depth = reinterpret_cast<real *>(s_dyn + sizeof(DepthRecord) * kStage);
-    tk.pos = reinterpret_cast<Pos *>(tk.depth + kLayers * kTileThreads);
-    tk.n_threads = kTileThreads;
+    tk.pos = reinterpret_cast<Pos *>(tk.depth + kHead * kTileThreads);
+    static_assert(kLayers <= kMaxTileWaves * kHead, "one wave's lists have room in the place of four");
     // between two selections the place of the staged records holds what the waves tell each other
-    struct Shared { int found[kTileThreads], cap[kWave], last_j[kWave], nan[kMaxTileWaves]; real last_depth[kWave]; };
+    struct Shared { int found[kTileThreads], cap[kWave], last_j[kWave], again[kMaxTileWaves]; real last_depth[kWave]; uint8_t dropped[kTileThreads]; };
     static_assert(sizeof(Shared) <= sizeof(DepthRecord) * kStage, "the waves' exchange fits the staging area");
     Shared *shared = reinterpret_cast<Shared *>(s_dyn);
 
@@ -282,9 +415,6 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
     const PixelCoord p = pixel_of_slot(a, tile.x, tile.y, slot);
     const WaveRect rect = wave_rect(p);
     const bool squares = ((a.tw | a.th) & 7) == 0;
-    const int64_t order_step = order_stride(out.order, a);
-    const int64_t order_at = order_first(out.order, p, start, slot);
-    const int rows_kept = out.order.low ? order_rows(out.order, a, n) : 0;
 
     PixelState s;  // of the first wave
     real last_depth = -__builtin_inff();
@@ -305,13 +435,16 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
         last_j = shared->last_j[lane];
         if (__builtin_amdgcn_ballot_w64(cap > 0) == 0) break;  // the same for all waves
         __syncthreads();
-        // The waves take the list's blocks of 64 entries in turn, each with candidate lists of its own.  A NaN depth ends a
-        // candidate list wherever it comes (topk_insert), so which candidates stay depends on what came before it: where one is
-        // met the first wave does the selection alone.
-        int found = 0;
+        // The waves take the list's blocks of 64 entries in turn, each with candidate lists of its own, of kHead places.  Where
+        // that does not do the first wave makes the selection alone, with room for all the layers: if a wave dropped a candidate
+        // that may be among the nearest (the merge comes to the end of its list); and if a depth is NaN, which ends a candidate
+        // list wherever it comes (topk_insert), so that what stays depends on what came before it.
+        int found = 0, todo = 0;
         for (int waves = kMaxTileWaves; ; waves = 1) {
+            tk.n_threads = waves == 1 ? kWave : kTileThreads;
+            const int room = min(cap, waves == 1 ? kLayers : kHead);
             found = 0;
-            bool met_nan = false;
+            bool met_nan = false, dropped = false;
             if (wave < waves) {
                 const auto entry = [&](int block) { return min(start + block * kWave + lane, end - 1); };
                 DepthParts next;
@@ -330,7 +463,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
                         const real rest = a.batch_bounds[batch_bound_index(start, tile.index, block * kWave)];
                         const int resume = a.far_start[tile.index] / kWave;
                         bool settled = cap == 0;
-                        if (!settled && waves == 1) settled = found == cap && tk.d(cap - 1) <= rest;
+                        if (!settled && waves == 1) settled = found == room && tk.d(room - 1) <= rest;
                         if (!settled && waves > 1) {
                             settled = true;
 #pragma unroll
@@ -367,7 +500,8 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
                             const int j = block * kWave + e;
                             met_nan = met_nan || pd != pd;
                             if (pd < last_depth || (pd == last_depth && j <= last_j)) continue;
-                            topk_insert(tk, cap, found, pd, j);
+                            dropped = dropped || (found == room && room < cap);
+                            topk_insert(tk, room, found, pd, j);
                         }
                         hit &= ~group;
                         wave_lds_sync();
@@ -378,54 +512,41 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
             }
             __syncthreads();
             shared->found[tid] = found;
+            shared->dropped[tid] = dropped;
             const uint64_t nan_lanes = __builtin_amdgcn_ballot_w64(met_nan);
-            if (lane == 0) shared->nan[wave] = nan_lanes != 0;
+            if (lane == 0) shared->again[wave] = waves > 1 && nan_lanes != 0;
             __syncthreads();
-            if (waves == 1 || !(shared->nan[0] | shared->nan[1] | shared->nan[2] | shared->nan[3])) break;
+            if (wave == 0 && waves > 1) {
+                bool short_list = false;
+                merge_lists(shared, tk, lane, cap, [&](int, real, int) {}, short_list);
+                const uint64_t short_lanes = __builtin_amdgcn_ballot_w64(short_list);
+                if (lane == 0 && short_lanes) shared->again[0] = 1;
+            }
             __syncthreads();
+            const int again = shared->again[0] | shared->again[1] | shared->again[2] | shared->again[3];
+            __syncthreads();
+            if (!again) break;
         }
         if (wave == 0 && cap > 0) {
-            // the four sorted lists of this lane's pixel, nearest first; no list has a NaN, or three are empty
-            const auto depth_at = [&](int w, int i) { return tk.depth[i * kTileThreads + w * kWave + lane]; };
-            const auto pos_at = [&](int w, int i) { return (int)tk.pos[i * kTileThreads + w * kWave + lane]; };
-            int count[kMaxTileWaves], at[kMaxTileWaves], pos[kMaxTileWaves], total = 0;
-            real depth[kMaxTileWaves];
-#pragma unroll
-            for (int w = 0; w < kMaxTileWaves; w++) {
-                count[w] = shared->found[w * kWave + lane];
-                total += count[w];
-                at[w] = 0;
-                depth[w] = count[w] ? depth_at(w, 0) : 0.0f;
-                pos[w] = count[w] ? pos_at(w, 0) : 0;
-            }
-            const int todo = min(total, cap);
-            for (int i = 0; i < todo; i++) {
-                int best = -1;
-#pragma unroll
-                for (int w = 0; w < kMaxTileWaves; w++)
-                    if (at[w] < count[w] && (best < 0 || depth[w] < last_depth || (depth[w] == last_depth && pos[w] < last_j))) {
-                        best = w;
-                        last_depth = depth[w];
-                        last_j = pos[w];
-                    }
-#pragma unroll
-                for (int w = 0; w < kMaxTileWaves; w++)
-                    if (w == best && ++at[w] < count[w]) {
-                        depth[w] = depth_at(w, at[w]);
-                        pos[w] = pos_at(w, at[w]);
-                    }
+            const int64_t order_step = order_stride(out.order, a);
+            const int64_t order_at = order_first(out.order, p, start, slot);
+            const int rows_kept = out.order.low ? order_rows(out.order, a, n) : 0;
+            bool short_list = false;
+            todo = merge_lists(shared, tk, lane, cap, [&](int, real d, int j) {
+                last_depth = d;
+                last_j = j;
                 BlendRecord r;
-                gather_blend(a, start + last_j, r);
+                gather_blend(a, start + j, r);
                 if (s.blended < rows_kept) {
                     const int64_t word = order_at + (int64_t)s.blended * order_step;
-                    out.order.low[word] = (uint16_t)last_j;
-                    if (sizeof(Pos) > sizeof(uint16_t) && n > kShortList) out.order.low[out.order.high + word] = (uint16_t)(last_j >> 16);
+                    out.order.low[word] = (uint16_t)j;
+                    if (sizeof(Pos) > sizeof(uint16_t) && n > kShortList) out.order.low[out.order.high + word] = (uint16_t)(j >> 16);
                 }
                 real b0, b1, b2;
                 bary_apply(r.m, p.px, p.py, b0, b1, b2);
                 blend_fragment(s, r, b0, b1, b2);
-            }
-            if (total < cap) active = false;  // the list is exhausted (render.cu:594)
+            }, short_list);
+            if (todo < cap) active = false;  // the list is exhausted (render.cu:594)
         }
     }
     if (wave == 0 && p.valid) write_pixel(out, p, s, last_j + 1, last_depth);
@@ -436,8 +557,8 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
 // kInTurn: the workgroup has four waves.
 // Workgroups a CU: what their LDS allows.  No bound in double precision: held to two workgroups every instance spills (10^5
 // triangles, 1024 x 1024: 229 us instead of 223, tiles of 8 x 8 190 instead of 168).
-template <int kStage, typename Pos, bool kInTurn>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage == kSelectBatchShort ? 3 : 2)
+template <int kStage, typename Pos, bool kInTurn, int kHead>
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage != kSelectBatchShort ? 2 : kInTurn ? 4 : 3)
 void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ uint8_t s_touch[kStage];
@@ -452,7 +573,7 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
             __shared__ real s_quarter[kStage != kWave ? kTileThreads : 1];  // with depth bounds; batches of 64 go without
             const int n_items = kMaxTileWaves * out.long_tiles.words[0];
             for (int item = long_group(out); item < n_items; item += long_groups(out))
-                long_tile_part<kStage, Pos>(a, out, tile_of_index(out.long_tiles.all[item / kMaxTileWaves]), item % kMaxTileWaves, s_dyn,
+                long_tile_part<kStage, Pos, kHead>(a, out, tile_of_index(out.long_tiles.all[item / kMaxTileWaves]), item % kMaxTileWaves, s_dyn,
                                             kStage != kWave ? s_quarter : nullptr);
             return;
         }
@@ -463,7 +584,7 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     const int n_entries = a.offsets[tile.index + 1] - a.offsets[tile.index];
     if (sizeof(Pos) < sizeof(int) && n_entries > kShortList) return;
     if (kInTurn ? is_long_tile(out, n_entries) : !first && is_started_first(out, tile.index, n_entries)) return;
-    pixel_order_tile<kStage, Pos, kInTurn>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
+    pixel_order_tile<kStage, Pos, kInTurn, kHead>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
 }
 
 // The tiles whose lists are longer than kShortList, with int positions: few or none, so a small grid
@@ -493,7 +614,7 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
                 const int tile = base + w * kWave + __builtin_ctzll(todo);
                 todo &= todo - 1;
                 __syncthreads();  // the tile before is done with the LDS
-                pixel_order_tile<kSelectBatch, int, false>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, tiles, s_dyn, s_touch, s_rects);
+                pixel_order_tile<kSelectBatch, int, false, kLayers>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, tiles, s_dyn, s_touch, s_rects);
             }
         }
     }
@@ -534,8 +655,8 @@ int pixel_order_threads(int preferred) {
     return override ? override : preferred;
 }
 
-size_t pixel_order_lds_bytes(int n_threads, int staged_entries, size_t position_bytes) {
-    return sizeof(DepthRecord) * staged_entries + (size_t)kLayers * n_threads * (sizeof(real) + position_bytes);
+size_t pixel_order_lds_bytes(int n_threads, int staged_entries, size_t position_bytes, int places) {
+    return sizeof(DepthRecord) * staged_entries + (size_t)places * n_threads * (sizeof(real) + position_bytes);
 }
 
 int check_raster_args(const char *fn, int width, int height, int tile_w, int tile_h, int max_layers) {
@@ -608,32 +729,20 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
         return check_launch("forward_tile_order_kernel");
     }
     const size_t lds = pixel_order_lds_bytes(n_threads, kSelectBatch);
-    // Depth bounds make the batches jump in steps of kSelectBatch, so they go with the int positions.
-    const bool split = !a.batch_bounds && n_threads >= kSelectBatchShort;
-    static size_t lds_reserved[2][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
+    static size_t lds_reserved[4][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
     const bool in_turn = n_threads == kTileThreads;
-    if (!split) {
-        const void *kernel = in_turn ? (const void *)forward_pixel_order_kernel<kSelectBatch, int, true>
-                                     : (const void *)forward_pixel_order_kernel<kSelectBatch, int, false>;
-        if (int e = reserve_lds("tg_render_forward", kernel, lds, lds_reserved[in_turn])) return e;
-        if (in_turn)
-            TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatch, int, true>), grid, dim3(n_threads), lds, s, a, o);
-        else
-            TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatch, int, false>), grid, dim3(n_threads), lds, s, a, o);
+    const auto launch = [&](void (*kernel)(RasterArgs, ForwardOut), size_t lds_bytes, size_t *reserved) -> int {
+        if (int e = reserve_lds("tg_render_forward", (const void *)kernel, lds_bytes, reserved)) return e;
+        TG_LAUNCH_AS("forward_pixel_order_kernel", kernel, grid, dim3(n_threads), lds_bytes, s, a, o);
         return check_launch("forward_pixel_order_kernel");
-    }
-    const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t));
-    static size_t lds_reserved_short[2][kMaxDevices] = {{0}};
-    const void *kernel = in_turn ? (const void *)forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true>
-                                 : (const void *)forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false>;
-    if (int e = reserve_lds("tg_render_forward", kernel, lds_short, lds_reserved_short[in_turn])) return e;
-    if (in_turn)
-        TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true>), grid, dim3(n_threads),
-                     lds_short, s, a, o);
-    else
-        TG_LAUNCH_AS("forward_pixel_order_kernel", (forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false>), grid, dim3(n_threads),
-                     lds_short, s, a, o);
-    if (int e = check_launch("forward_pixel_order_kernel")) return e;
+    };
+    if (a.batch_bounds)  // they make the batches jump in steps of kSelectBatch
+        return in_turn ? launch(forward_pixel_order_kernel<kSelectBatch, int, true, kLayers>, lds, lds_reserved[0])
+                       : launch(forward_pixel_order_kernel<kSelectBatch, int, false, kLayers>, lds, lds_reserved[1]);
+    const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kShortHead);
+    if (int e = in_turn ? launch(forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>, lds_short, lds_reserved[2])
+                        : launch(forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>, lds_short, lds_reserved[3]))
+        return e;
     if (longest <= kShortList) return 0;  // no list is too long for 16-bit positions
     if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;
     const int tiles = (int)(tl.grid.x * tl.grid.y);

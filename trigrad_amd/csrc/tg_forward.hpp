@@ -27,9 +27,11 @@ __device__ __forceinline__ int long_group(const ForwardOut &o) { return (int)(bl
 __device__ __forceinline__ int long_groups(const ForwardOut &o) { return o.long_rows * (int)gridDim.x; }
 __device__ __forceinline__ TileId tile_of_index(int index) {
     TileId t;
+    int columns = (int)gridDim.x;
+    asm volatile("" : "+s"(columns));  // the division's constants are made here, not kept in registers by the loop around the call
     t.index = index;
-    t.y = index / (int)gridDim.x;
-    t.x = index - t.y * (int)gridDim.x;
+    t.y = index / columns;
+    t.x = index - t.y * columns;
     return t;
 }
 // A launch that shares the long tiles' work out takes them all; one that only starts with them takes the first few, whole.

@@ -48,12 +48,16 @@ __device__ __forceinline__ PixelCoord pixel_of_slot(const RasterArgs &a, int til
     if (((a.tw | a.th) & 7) == 0) {
         // a wave takes a square of 8 x 8 pixels: fewer list entries touch a square than a strip of the
         // same area, so the waves cull more and share an entry among more lanes
-        const int squares_x = a.tw >> 3, square = t >> 6, l = t & 63;
+        int squares_x = a.tw >> 3;
+        asm volatile("" : "+s"(squares_x));  // the division's constants are made here, not kept in registers by a loop around the call
+        const int square = t >> 6, l = t & 63;
         lx = (square % squares_x) * 8 + (l & 7);
         ly = (square / squares_x) * 8 + (l >> 3);
     } else {
-        lx = t % a.tw;
-        ly = t / a.tw;
+        int columns = a.tw;
+        asm volatile("" : "+s"(columns));
+        lx = t % columns;
+        ly = t / columns;
     }
     p.ix = tile_x * a.tw + lx;
     p.iy = tile_y * a.th + ly;
@@ -334,7 +338,7 @@ __device__ __forceinline__ void blend_fragment(PixelState &s, const BlendRecord 
 struct TileLaunch { dim3 grid; int threads; };
 TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_threads);
 int pixel_order_threads(int preferred);
-size_t pixel_order_lds_bytes(int n_threads, int staged_entries, size_t position_bytes = sizeof(int));
+size_t pixel_order_lds_bytes(int n_threads, int staged_entries, size_t position_bytes = sizeof(int), int places = kLayers);
 inline int order_pool_pixels(int tile_w, int tile_h) { return ceil_div(tile_w * tile_h, kWave) * kWave; }
 int check_raster_args(const char *fn, int width, int height, int tile_w, int tile_h, int max_layers);
 
