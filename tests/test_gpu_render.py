@@ -1173,3 +1173,27 @@ def test_candidate_lists_around_their_places_in_lds(n, layers, cuda, oracle):
     _check_forward(f"{n} candidates, {layers} layers", want, got, (16, 16))
     _, want, got, _ = _forward_both(scene, 8, 8, mode, cuda, oracle)  # one wave to a workgroup
     _check_forward(f"{n} candidates, {layers} layers, small tiles", want, got, (8, 8))
+
+
+@pytest.mark.parametrize("width,height", [(16, 16), (70, 45), (1024, 1024), (1040, 1024)])
+@pytest.mark.parametrize("n", [1, 40, 700, 1020, 1030, 2040, 2060, 4090, 4100, 6200, 8200])
+def test_frames_with_few_keys_have_the_other_routes_lists(n, width, height, cuda, monkeypatch):
+    """Frames of up to some 8000 keys and 4096 tiles are sorted by one workgroup, by tile, and by depth as well up to some 900:
+    around the numbers of keys a thread takes, with equal depths (the order is then the triangles'), tiles without a key, and a
+    tile whose list is a long one.  Lists and image are those of the stage-by-stage route."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    soup = S.random_soup(n, width, height, seed=n, sigma_px=1.0, opacity=(0.1, 0.6))
+    v = soup["vertices"].reshape(n, 3, 4).copy()
+    v[::3, :, 2:] = (2.0, 0.5)
+    if n > 2000:
+        v[: n // 2, :, :2] = v[: n // 2, :, :2] * (4.0 / max(width, height)) + 0.13  # half of them in a tile or two
+    d = to_device(dict(soup, vertices=v.reshape(-1, 4)), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, 16, 16, 1 / 256, True, True, 32)
+    for _ in range(3):  # the first frame's buffers are made for a guess of K, and the route goes by them
+        got = _C.render_forward(*args)
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C.render_forward(*args)
+    for i in (0, 1, 2, 3, 4, 5, 6):
+        assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i

@@ -861,6 +861,118 @@ __global__ __launch_bounds__(kSegLargeThreads) void segment_sort_large_kernel(ui
     }
 }
 
+// ---- the lists of a frame with few keys, by one workgroup ---------------------------------------------
+//
+// Two sweeps are two launches that wait for one another, each nine microseconds of latency however little there is to sort.
+// Up to kFewKeys pairs fit the LDS of one workgroup, which sorts them by tile (one or two stable 8-bit passes) and looks the
+// tiles' bounds up in the sorted pairs; the segment sort follows as ever.  Up to kFewestKeys it sorts them by depth as well,
+// before that, and the segment sort's launch goes too.  Sweeps and segment sort, and now, us: 20 triangles (100 keys) 25 -> 12,
+// 1000 (2600) 26 -> 18, 225 large ones (4000) 27 -> 23, 2000 (4500) 28 -> 24.  By depth as well at 2600 keys: 25.
+constexpr int kFewKeys = kSegLargeThreads * 8, kFewestKeys = kSegLargeThreads * 2;
+constexpr int kFewKeysTiles = 4096;  // a tile's bound is a search of thirteen LDS reads, four of them a thread
+struct FewKeysLds {
+    SegLds<kSegLargeThreads> lds;
+    uint32_t varying_tile;
+    uint32_t depth[kFewKeys], value[kFewKeys];
+    uint16_t tile[kFewKeys];
+};
+template <int ITEMS>
+__device__ __forceinline__ void sort_few_keys(const uint64_t *keys, const uint32_t *vals, int n, bool by_depth, int column_bits, int tiles_x, FewKeysLds &s) {
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    constexpr int kWaveSpan = kWave * ITEMS;
+    uint32_t depth[ITEMS], tile[ITEMS], value[ITEMS];
+    uint32_t varying = 0, varying_tile = 0;
+    const uint32_t first_depth = (uint32_t)keys[0], first_high = (uint32_t)(keys[0] >> 32);
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) {
+        const int pos = wave * kWaveSpan + i * kWave + lane;
+        depth[i] = ~0u;  // padding: behind every real pair, and a stable sort keeps it there
+        tile[i] = 0xffff;
+        value[i] = 0;
+        if (pos < n) {
+            const uint64_t key = keys[pos];
+            const uint32_t high = (uint32_t)(key >> 32);
+            depth[i] = (uint32_t)key;
+            tile[i] = (high >> column_bits) * (uint32_t)tiles_x + (high & ((1u << column_bits) - 1));
+            value[i] = vals[pos];
+            varying |= depth[i] ^ first_depth;
+            varying_tile |= tile[i] ^ ((first_high >> column_bits) * (uint32_t)tiles_x + (first_high & ((1u << column_bits) - 1)));
+        }
+        s.depth[pos] = depth[i];
+        s.tile[pos] = (uint16_t)tile[i];
+        s.value[pos] = value[i];
+    }
+    if (tid == 0) s.lds.varying = s.varying_tile = 0;
+    __syncthreads();
+    varying = wave_or_u32(varying);
+    varying_tile = wave_or_u32(varying_tile);
+    if (lane == 0 && varying) atomicOr(&s.lds.varying, varying);
+    if (lane == 0 && varying_tile) atomicOr(&s.varying_tile, varying_tile);
+    __syncthreads();
+    varying = by_depth ? s.lds.varying : 0;
+    varying_tile = s.varying_tile;
+#pragma unroll 1
+    for (int p = 0; p < 6; p++) {  // four bytes of the depth, two of the tile
+        const int shift = (p & 3) * kRadixBits;
+        if ((((p < 4 ? varying : varying_tile) >> shift) & (kRadix - 1)) == 0) continue;  // all pairs share this digit
+        uint32_t digit[ITEMS], place[ITEMS];
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) digit[i] = ((p < 4 ? depth[i] : tile[i]) >> shift) & (kRadix - 1);
+        workgroup_digit_places<kSegLargeThreads, ITEMS>(digit, s.lds, place);
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) {
+            s.depth[place[i]] = depth[i];
+            s.tile[place[i]] = (uint16_t)tile[i];
+            s.value[place[i]] = value[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) {
+            const int pos = wave * kWaveSpan + i * kWave + lane;
+            depth[i] = s.depth[pos];
+            tile[i] = s.tile[pos];
+            value[i] = s.value[pos];
+        }
+        __syncthreads();  // everything is read before the next pass writes
+    }
+}
+__global__ __launch_bounds__(kSegLargeThreads) void sort_few_keys_kernel(uint64_t *keys, uint32_t *vals, int32_t *offsets, int n_tiles,
+                                                                         int column_bits, int tiles_x, bool by_depth, uint32_t capacity,
+                                                                         FrameCount frame_count, uint32_t *status, LongTiles long_tiles) {
+    extern __shared__ __align__(16) unsigned char s_few[];
+    FewKeysLds &s = *reinterpret_cast<FewKeysLds *>(s_few);
+    const int tid = threadIdx.x;
+    const int n = (int)frame_count.pairs(capacity);
+    if (tid == 0 && frame_count.expired()) *status = TG_STATUS_LOOKBACK_TIMEOUT;
+    if (n > 0) {  // the same for the workgroup, as what follows
+        if (n <= kSegLargeThreads) sort_few_keys<1>(keys, vals, n, by_depth, column_bits, tiles_x, s);
+        else if (n <= 2 * kSegLargeThreads) sort_few_keys<2>(keys, vals, n, by_depth, column_bits, tiles_x, s);
+        else if (n <= 4 * kSegLargeThreads) sort_few_keys<4>(keys, vals, n, by_depth, column_bits, tiles_x, s);
+        else sort_few_keys<8>(keys, vals, n, by_depth, column_bits, tiles_x, s);
+    }
+    for (int pos = tid; pos < n; pos += kSegLargeThreads) {
+        keys[pos] = (uint64_t)s.tile[pos] << 32 | s.depth[pos];
+        vals[pos] = s.value[pos];
+    }
+    const auto first_of = [&](int tile) {  // the first pair of this tile or a later one
+        int low = 0, high = n;
+        while (low < high) {
+            const int middle = (low + high) / 2;
+            if (s.tile[middle] < tile) low = middle + 1; else high = middle;
+        }
+        return low;
+    };
+    for (int t = tid; t <= n_tiles; t += kSegLargeThreads) {
+        const int first = first_of(t);
+        offsets[t] = first;
+        if (long_tiles.words && t < n_tiles && n - first >= long_tiles.limit && first_of(t + 1) - first >= long_tiles.limit) {
+            const int slot = atomicAdd(long_tiles.words, 1);
+            if (slot < kLongTileSlots) long_tiles.words[1 + slot] = t;
+            long_tiles.all[slot] = t;
+        }
+    }
+}
+
 __global__ __launch_bounds__(kSortThreads) void tile_ranges_kernel(const uint64_t *__restrict__ sorted_keys, int64_t n_keys,
                                                                    int n_tiles, int32_t *__restrict__ offsets) {
     const int64_t i = (int64_t)blockIdx.x * kSortThreads + threadIdx.x;
@@ -934,17 +1046,11 @@ static int run_passes(const char *fn, const PassPlan &plan, const SortLayout &L,
     return run_sweeps(fn, plan, L.n_tiles, bases, 0, lookback, tickets, keys, values, keys_alt, values_alt, n, status, s);
 }
 
-// Tile ranges of keys that are ordered by tile, then every tile's segment sorted by its depth bits in place.
-// With tile_count (the last sweep counted every tile's pairs) the ranges come from the counts, inside the segment kernel.
-static int ranges_and_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint32_t *v_other, int64_t n, int n_tiles,
-                               int32_t *offsets, hipStream_t s, const uint32_t *tile_count = nullptr,
-                               const uint32_t *row_totals = nullptr, int tiles_x = 0, FrameCount frame_count = FrameCount(),
-                               uint32_t *status = nullptr, int64_t longest = std::numeric_limits<int64_t>::max(),
-                               const LongTiles &long_tiles = LongTiles()) {
-    if (!tile_count) {
-        TG_LAUNCH(tile_ranges_kernel, dim3((unsigned)ceil_div64(n + 1, kSortThreads)), dim3(kSortThreads), 0, s, k, n, n_tiles, offsets);
-        if (int e = check_launch("tile_ranges_kernel")) return e;
-    }
+// Every tile's segment of keys that are ordered by tile sorted by its depth bits in place.  With tile_count (the last sweep
+// counted every tile's pairs) the segments' bounds come from the counts and are written to `offsets`, which else hold them.
+static int sort_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint32_t *v_other, int64_t n, int n_tiles, int32_t *offsets,
+                         hipStream_t s, const uint32_t *tile_count, const uint32_t *row_totals, int tiles_x, FrameCount frame_count,
+                         uint32_t *status, int64_t longest, const LongTiles &long_tiles) {
     const int medium_cap = medium_segments(longest, n, n_tiles);
     TG_LAUNCH(segment_sort_small_kernel, dim3(ceil_div(n_tiles, kSortWaves)), dim3(kSortThreads), 0, s, k, v, offsets, n_tiles,
               tile_count, row_totals, tiles_x, (uint32_t)n, frame_count, status, medium_cap, long_tiles);
@@ -955,6 +1061,19 @@ static int ranges_and_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint
     TG_LAUNCH(segment_sort_large_kernel, dim3(n_tiles < kSegLargeGrid ? n_tiles : kSegLargeGrid), dim3(kSegLargeThreads), sizeof(LargeSegLds),
               s, k, v, k_other, v_other, offsets, n_tiles, medium_cap);
     return check_launch("segment_sort_large_kernel");
+}
+
+// Tile ranges, then the segments.
+static int ranges_and_segments(uint64_t *k, uint32_t *v, uint64_t *k_other, uint32_t *v_other, int64_t n, int n_tiles,
+                               int32_t *offsets, hipStream_t s, const uint32_t *tile_count = nullptr,
+                               const uint32_t *row_totals = nullptr, int tiles_x = 0, FrameCount frame_count = FrameCount(),
+                               uint32_t *status = nullptr, int64_t longest = std::numeric_limits<int64_t>::max(),
+                               const LongTiles &long_tiles = LongTiles()) {
+    if (!tile_count) {
+        TG_LAUNCH(tile_ranges_kernel, dim3((unsigned)ceil_div64(n + 1, kSortThreads)), dim3(kSortThreads), 0, s, k, n, n_tiles, offsets);
+        if (int e = check_launch("tile_ranges_kernel")) return e;
+    }
+    return sort_segments(k, v, k_other, v_other, n, n_tiles, offsets, s, tile_count, row_totals, tiles_x, frame_count, status, longest, long_tiles);
 }
 
 static int check_sort_buffers(const char *fn, const void *keys, const void *values, const void *keys_alt, const void *values_alt,
@@ -1199,6 +1318,16 @@ int tg::build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, const uin
     uint32_t *tile_count = (uint32_t *)((char *)workspace + kFrameSortHeadBytes + lookback_bytes);
     const uint32_t *totals = fused_frame_totals(frame, epoch);
     const FrameCount count{total_and_status, (uint32_t)n_keys, epoch};
+    if (total_and_status && n_keys <= kFewKeys && n_tiles <= kFewKeysTiles) {
+        const bool by_depth = n_keys <= kFewestKeys;
+        static size_t lds_reserved[kMaxDevices] = {0};
+        if (int e = reserve_lds("tg_build_frame_lists", (const void *)sort_few_keys_kernel, sizeof(FewKeysLds), lds_reserved)) return e;
+        TG_LAUNCH(sort_few_keys_kernel, dim3(1), dim3(kSegLargeThreads), sizeof(FewKeysLds), s, keys, values, offsets, n_tiles,
+                  grid.column_bits, tiles_x, by_depth, (uint32_t)n_keys, count, status, long_tiles);
+        if (int e = check_launch("sort_few_keys_kernel")) return e;
+        return by_depth ? 0 : sort_segments(keys, values, keys_alt, values_alt, n_keys, n_tiles, offsets, s, nullptr, nullptr, 0, count,
+                                            status, longest, LongTiles());
+    }
     if (int e = run_sweeps("tg_build_frame_lists", grid.plan, n_sort_tiles, totals, 1, lookback, tickets, keys, values, keys_alt,
                            values_alt, n_keys, status, s, grid.column_bits, tiles_x, tile_count, count))
         return e;
