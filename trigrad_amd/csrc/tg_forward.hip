@@ -63,6 +63,8 @@ constexpr int kSelectBatchShort = 64;   // ... and where they take 16 bits
 // Lists with depth bounds keep all places in LDS and three kinds of 16-bit positions lose there: 200 000 faint triangles 288
 // us, with 29 places and three workgroups a CU 301, with 21 and four 338: every pixel has 32 candidates.
 constexpr int kShortHead = sizeof(real) == 4 ? 23 : kLayers;
+constexpr int kLongHead = sizeof(real) == 4 ? 17 : 24;  // the same LDS with int positions, in long_tile_part
+static_assert((sizeof(real) + sizeof(int)) * kLongHead <= (sizeof(real) + sizeof(uint16_t)) * kShortHead, "the same LDS");
 constexpr int kLongListGroups = 256;    // workgroups that look for the tiles with longer lists
 
 // The last places of a candidate list, in registers: place kPlace and those behind it.  (A structure of its own for every place:
@@ -400,7 +402,6 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
     asm volatile("" : "+v"(tid));  // what depends on it is made here, not kept in registers by the loop around the call
     const int lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1], n = end - start;
-    if (sizeof(Pos) < sizeof(int) && n > kShortList) return;  // left to forward_pixel_order_long_lists_kernel
     DepthRecord *s_rec = reinterpret_cast<DepthRecord *>(s_dyn) + wave * kStaged;
     TopKOf<Pos> tk;
     tk.depth = reinterpret_cast<real *>(s_dyn + sizeof(DepthRecord) * kStage);
@@ -552,8 +553,8 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
     if (wave == 0 && p.valid) write_pixel(out, p, s, last_j + 1, last_depth);
 }
 
-// One workgroup per tile.  With 16-bit positions the tiles whose lists are too long for them are left to
-// forward_pixel_order_long_lists_kernel.
+// One workgroup per tile.  With 16-bit positions the tiles whose lists are too long for them are shared out as long tiles, with
+// int positions, or left to forward_pixel_order_long_lists_kernel.
 // kInTurn: the workgroup has four waves.
 // Workgroups a CU: what their LDS allows.  No bound in double precision: held to two workgroups every instance spills (10^5
 // triangles, 1024 x 1024: 229 us instead of 223, tiles of 8 x 8 190 instead of 168).
@@ -572,9 +573,14 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
         if (first) {
             __shared__ real s_quarter[kStage != kWave ? kTileThreads : 1];  // with depth bounds; batches of 64 go without
             const int n_items = kMaxTileWaves * out.long_tiles.words[0];
-            for (int item = long_group(out); item < n_items; item += long_groups(out))
-                long_tile_part<kStage, Pos, kHead>(a, out, tile_of_index(out.long_tiles.all[item / kMaxTileWaves]), item % kMaxTileWaves, s_dyn,
-                                            kStage != kWave ? s_quarter : nullptr);
+            for (int item = long_group(out); item < n_items; item += long_groups(out)) {
+                const TileId tile = tile_of_index(out.long_tiles.all[item / kMaxTileWaves]);
+                const int part = item % kMaxTileWaves, n = a.offsets[tile.index + 1] - a.offsets[tile.index];
+                if (sizeof(Pos) == sizeof(int) || n <= kShortList)
+                    long_tile_part<kStage, Pos, kHead>(a, out, tile, part, s_dyn, kStage != kWave ? s_quarter : nullptr);
+                else
+                    long_tile_part<kStage, int, kLongHead>(a, out, tile, part, s_dyn, nullptr);
+            }
             return;
         }
     } else {
@@ -587,8 +593,8 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     pixel_order_tile<kStage, Pos, kInTurn, kHead>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
 }
 
-// The tiles whose lists are longer than kShortList, with int positions: few or none, so a small grid
-// looks through the tiles' list lengths (a workgroup through its share of the tiles, one tile per thread at a
+// The tiles whose lists are longer than kShortList, with int positions, where the kernel above does not share them out as long
+// tiles (their launch is saved there, 4.7 us whether there are any or not): few or none, so a small grid looks through the tiles' list lengths (a workgroup through its share of the tiles, one tile per thread at a
 // time) and takes those.
 __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_kernel(RasterArgs a, ForwardOut out, int tiles_x,
                                                                                       int tiles_y) {
@@ -603,7 +609,8 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
     const int n_waves = blockDim.x / kWave;
     for (int base = first; base < past; base += blockDim.x) {
         const int mine = base + (int)threadIdx.x;
-        const bool is_long = mine < past && a.offsets[mine + 1] - a.offsets[mine] > kShortList;
+        const int length = mine < past ? a.offsets[mine + 1] - a.offsets[mine] : 0;
+        const bool is_long = length > kShortList && !(out.long_rows && blockDim.x == kTileThreads && length >= out.long_tiles.limit);
         const uint64_t vote = __builtin_amdgcn_ballot_w64(is_long);
         __syncthreads();  // the round before is done with the votes
         if ((threadIdx.x & (kWave - 1)) == 0) s_votes[threadIdx.x / kWave] = vote;
@@ -743,7 +750,8 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     if (int e = in_turn ? launch(forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>, lds_short, lds_reserved[2])
                         : launch(forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>, lds_short, lds_reserved[3]))
         return e;
-    if (longest <= kShortList) return 0;  // no list is too long for 16-bit positions
+    // no list is too long for 16-bit positions, or those that are are long tiles, which the kernel above has shared out
+    if (longest <= kShortList || (in_turn && o.long_rows && long_tiles.limit <= kShortList)) return 0;
     if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;
     const int tiles = (int)(tl.grid.x * tl.grid.y);
     TG_LAUNCH(forward_pixel_order_long_lists_kernel, dim3(min(tiles, kLongListGroups), 1, grid.z), dim3(n_threads), lds, s, a, o,
