@@ -1156,12 +1156,13 @@ def test_long_tiles_match_the_other_route(width, per_pixel_sort, cuda, monkeypat
 
 @pytest.mark.parametrize("layers", [5, 23, 24, 27, 32, 40, -1])
 @pytest.mark.parametrize("n", [22, 23, 24, 25, 31, 32, 33, 60])
-def test_candidate_lists_around_their_places_in_lds(n, layers, cuda, oracle):
-    """A pixel's first 23 candidates are kept in LDS, the others up to 32 in registers: n triangles over every pixel, tilted, so
+@pytest.mark.parametrize("size", [24, 460])
+def test_candidate_lists_around_their_places_in_lds(size, n, layers, cuda, oracle):
+    """A pixel's first 23 candidates are kept in LDS, the others up to 32 in registers -- or all in LDS, where there are so few
+    workgroups (768 of 16 x 16 tiles, some 2500 of 8 x 8) that they run at once all the same: n triangles over every pixel, tilted, so
     that their order at a pixel is not the list's, a third of them at equal depths, and layers that end inside either part."""
     import scenes as S
     rng = np.random.default_rng(100 * n + layers)
-    size = 24
     z = rng.uniform(1.0, 5.0, (n, 1)) * rng.uniform(0.5, 1.5, (n, 3))
     z[::3] = rng.choice([2.0, 3.0], (z[::3].shape[0], 1))
     xy = np.array([[-9.0, -9.0], [9.0, -9.0], [0.0, 16.0]]) * rng.uniform(0.9, 1.1, (n, 1, 1))

@@ -559,7 +559,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
 // Workgroups a CU: what their LDS allows.  No bound in double precision: held to two workgroups every instance spills (10^5
 // triangles, 1024 x 1024: 229 us instead of 223, tiles of 8 x 8 190 instead of 168).
 template <int kStage, typename Pos, bool kInTurn, int kHead>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage != kSelectBatchShort ? 2 : kInTurn ? 4 : 3)
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage != kSelectBatchShort ? 2 : kInTurn && kHead < kLayers ? 4 : 3)
 void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ uint8_t s_touch[kStage];
@@ -594,8 +594,8 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
 }
 
 // The tiles whose lists are longer than kShortList, with int positions, where the kernel above does not share them out as long
-// tiles (their launch is saved there, 4.7 us whether there are any or not): few or none, so a small grid looks through the tiles' list lengths (a workgroup through its share of the tiles, one tile per thread at a
-// time) and takes those.
+// tiles (their launch is saved there, 4.7 us whether there are any or not): few or none, so a small grid looks through the
+// tiles' list lengths (a workgroup through its share of the tiles, one tile per thread at a time) and takes those.
 __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_kernel(RasterArgs a, ForwardOut out, int tiles_x,
                                                                                       int tiles_y) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
@@ -736,7 +736,7 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
         return check_launch("forward_tile_order_kernel");
     }
     const size_t lds = pixel_order_lds_bytes(n_threads, kSelectBatch);
-    static size_t lds_reserved[4][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
+    static size_t lds_reserved[6][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
     const bool in_turn = n_threads == kTileThreads;
     const auto launch = [&](void (*kernel)(RasterArgs, ForwardOut), size_t lds_bytes, size_t *reserved) -> int {
         if (int e = reserve_lds("tg_render_forward", (const void *)kernel, lds_bytes, reserved)) return e;
@@ -746,10 +746,19 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     if (a.batch_bounds)  // they make the batches jump in steps of kSelectBatch
         return in_turn ? launch(forward_pixel_order_kernel<kSelectBatch, int, true, kLayers>, lds, lds_reserved[0])
                        : launch(forward_pixel_order_kernel<kSelectBatch, int, false, kLayers>, lds, lds_reserved[1]);
-    const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kShortHead);
-    if (int e = in_turn ? launch(forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>, lds_short, lds_reserved[2])
-                        : launch(forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>, lds_short, lds_reserved[3]))
-        return e;
+    // Short heads are for workgroups that would wait for a place with all candidates in LDS.  Where all of them run at once
+    // anyway (three waves a SIMD, or LDS) the kernel is one chain of latencies, which the tail and its single records lengthen.
+    // Tiles of 8 x 8, us with all places and with short heads: 558 with 165 large faint triangles each 64 and 74, 323 with 240
+    // small ones 47 and 51, 943 with 7 11.6 and 12.8.  At 1024 tiles of 16 x 16 the short ones win (445 and 360).
+    const size_t lds_all = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kLayers);
+    const int64_t at_once = 256 * std::min<int64_t>(3 * kTileThreads / n_threads, 160 * 1024 / (lds_all + 512));
+    const bool all_places = groups <= at_once;
+    const size_t lds_short = all_places ? lds_all : pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kShortHead);
+    const auto short_kernel = all_places ? (in_turn ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kLayers>
+                                                    : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kLayers>)
+                                         : (in_turn ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>
+                                                    : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>);
+    if (int e = launch(short_kernel, lds_short, lds_reserved[2 + 2 * all_places + in_turn])) return e;
     // no list is too long for 16-bit positions, or those that are are long tiles, which the kernel above has shared out
     if (longest <= kShortList || (in_turn && o.long_rows && long_tiles.limit <= kShortList)) return 0;
     if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;
