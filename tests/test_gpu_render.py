@@ -1198,3 +1198,26 @@ def test_frames_with_few_keys_have_the_other_routes_lists(n, width, height, cuda
     want = _C.render_forward(*args)
     for i in (0, 1, 2, 3, 4, 5, 6):
         assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
+
+
+@pytest.mark.parametrize("layers", [15, 16])
+@pytest.mark.parametrize("columns,rows", [(1, 1), (127, 1), (128, 1), (43, 3), (19, 27)])
+def test_gradients_whichever_tiles_an_xcd_takes(columns, rows, layers, cuda, oracle):
+    """The saved-order backward kernel deals the tiles out to the XCDs in eighths of them, or in chunks of 16 from 16 layers on:
+    numbers of tiles around a round of chunks (128) and with a remainder, every tile with triangles of its own and shared ones."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    width, height = 16 * columns - 3, 16 * rows - 5
+    n = 20 * columns * rows
+    scene = S.random_soup(n, width, height, seed=n + layers, sigma_px=9.0, opacity=(0.1, 0.5), varying_w=True)
+    d, want, got, ml = _forward_both(scene, 16, 16, dict(per_pixel_sort=True, max_layers=layers), cuda, oracle)
+    gi, gd = _grad_inputs(scene, 4, True)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
+                                    16, 16, True, ml, literal=False, magnitudes=True)
+    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
+    out = _C.render_backward(torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda), d["vertices"], d["indices"], d["colors"],
+                             d["opacities"], sorted_ids, offsets, bary, image, depthmap, weights, ends, width, height, 16, 16, 1 / 256,
+                             True, ml, resume=resume)
+    for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+        assert_gradients_close(f"{columns}x{rows} tiles, {layers} layers: {label}", g.cpu().numpy(), w, mag)

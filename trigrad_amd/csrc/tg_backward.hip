@@ -808,7 +808,8 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkSavedOrder>();
+    const TileId tile_id = a.max_layers < kManyLayers ? tile_of_workgroup<kTileBandBackward, kChunkBackward>()
+                                                      : tile_of_workgroup<kTileBandBackward, kChunkSavedOrder>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);

@@ -81,10 +81,12 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
 // where a mesh covers part of the image an eighth can be empty and another one full (1.3 million triangles of a torus,
 // 1920 x 1080: two XCDs had 45 % of the list entries, the last one none; 800 -> 680 us of kernel time), and where every tile
 // has the same work nothing is lost (10^6 triangles: 677 -> 668; chunks of 16 to 128 within 1 %).  The backward kernel with the
-// saved order takes chunks of 8 tiles of a row: the mesh 224 -> 201, 20 000 large triangles on 512 x 512 665 -> 640, 33 000 in
-// tiles of 8 x 8 240 -> 234, 10^6 triangles 1247 -> 1218 to 1249; chunks of 16, or two rows high, lose up to 1 % on the last.
-// The one in tile order loses by any (618 -> 700 with chunks of 16): its gradient arrays are dense, and the tiles of a chunk's
-// border meet in their vertices' gradients on two XCDs.
+// saved order takes chunks of 16 tiles of a row: the mesh 222 -> 198, 20 000 large triangles on 512 x 512 641 -> 617, 33 000 in
+// tiles of 8 x 8 234 -> 231, 10^6 triangles 1190 -> 1152; chunks of 8 or 32 within 1 %, bands of 2 and 4 rows lose up to 6 %.
+// Gradients that tiles on two XCDs share cost more than those that stay on one.  Deep enough that does not show; with few layers
+// most of them are the nearest triangles', the large ones among which cover many tiles: 10^6 triangles with a heavy tail and 2, 8,
+// 16 layers 148, 574, 1031 us in eighths and 187, 604, 1037 in chunks.  So below kManyLayers it takes eighths, like the kernel
+// in tile order, where vertices share lines in dense gradient arrays as well (618 -> 700 with chunks of 16).
 #ifndef TG_XCD_TILES
 #define TG_XCD_TILES 1
 #endif
@@ -99,7 +101,8 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
 #endif
 constexpr int kXcds = 8;
 constexpr int kTileBandForward = TG_TILE_BAND_FORWARD, kTileBandBackward = TG_TILE_BAND_BACKWARD;
-constexpr int kChunkForward = TG_XCD_CHUNK_FORWARD, kChunkSavedOrder = 8, kChunkBackward = 0;  // 0: an eighth of the tiles
+constexpr int kChunkForward = TG_XCD_CHUNK_FORWARD, kChunkSavedOrder = 16, kChunkBackward = 0;  // 0: an eighth of the tiles
+constexpr int kManyLayers = 16;
 struct TileId { int x, y, index; };
 template <int kTileBand, int kChunk>
 __device__ __forceinline__ TileId tile_of_workgroup(int skipped_rows = 0) {  // rows of workgroups in front that are not for tiles
