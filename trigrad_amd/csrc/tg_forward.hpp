@@ -161,8 +161,11 @@ __device__ __forceinline__ void tile_order_tile(const RasterArgs &a, const Forwa
     }
 }
 
-// forward_tile_order_kernel for launches of few workgroups (tg_forward_few.hip).
+// The kernels of launches with few workgroups (tg_forward_few.hip): forward_tile_order_kernel's, and forward_pixel_order_kernel
+// with all of a candidate list's places in LDS.
 constexpr int kFewTileGroups = 1024;
 __global__ void forward_tile_order_few_kernel(RasterArgs a, ForwardOut out);
+using ForwardKernel = void (*)(RasterArgs, ForwardOut);
+ForwardKernel pixel_order_few_kernel(bool in_turn);
 
 }  // namespace tg

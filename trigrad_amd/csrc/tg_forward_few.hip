@@ -1,5 +1,6 @@
-// tg_forward_few.hip -- the tile-order forward kernel of launches with few workgroups, which shares the long tiles' work out.
-#include "tg_forward.hpp"
+// tg_forward_few.hip -- the forward kernels of launches with few workgroups: in tile order one that shares the long tiles' work
+// out, in per-pixel order the instances with all of a candidate list's places in LDS.
+#include "tg_forward_pixel.hpp"
 
 namespace tg {
 
@@ -105,5 +106,13 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void forwa
     if (is_long_tile(out, end - start)) return;
     tile_order_tile(a, out, tile, start, end, s);
 }
+
+// In double precision every launch has all places in LDS; there is no second kernel then.
+template <int kStage>
+static ForwardKernel all_places_kernel(bool in_turn) {
+    if constexpr (kShortHead == kLayers) return nullptr;
+    else return in_turn ? forward_pixel_order_kernel<kStage, uint16_t, true, kLayers> : forward_pixel_order_kernel<kStage, uint16_t, false, kLayers>;
+}
+ForwardKernel pixel_order_few_kernel(bool in_turn) { return all_places_kernel<kSelectBatchShort>(in_turn); }
 
 }  // namespace tg
