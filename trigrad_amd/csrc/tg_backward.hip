@@ -384,6 +384,16 @@ __device__ __forceinline__ TermLane term_lane(const BackwardArgs &g, int lane) {
 // then holds a sum to deliver, and every lane walks the ones of its own third.  vertex_at(c, v): vertex id v of
 // the entry in slot c.
 constexpr int kRunSpan = 22;  // slots of a third (the last one has kWave - 2 * kRunSpan = 20)
+// Bit k of x as a mask, all ones or 0.  (The compiler is not to know that: it makes a comparison and a selection of a mask, three
+// operations and a wait for one.)
+__device__ __forceinline__ int bit_mask(int x, int k) {
+    int mask = __builtin_amdgcn_sbfe(x, k, 1);
+    asm("" : "+v"(mask));
+    return mask;
+}
+// x where mask is all ones, 0 where it is 0.
+__device__ __forceinline__ float masked(float x, int mask) { return __int_as_float(__float_as_int(x) & mask); }
+__device__ __forceinline__ double masked(double x, int mask) { return mask ? x : 0.0; }
 template <typename VertexAt>
 __device__ __forceinline__ void add_run_sums(real *terms, int n, uint64_t heads, const TermLane &t, VertexAt vertex_at) {
     if (t.group >= 3) return;  // the one lane left over; nothing below synchronises the wave
@@ -391,14 +401,14 @@ __device__ __forceinline__ void add_run_sums(real *terms, int n, uint64_t heads,
     real *row = terms + t.q * kTermStride + c0;
     const bool full = t.group < 2;  // a third of kRunSpan slots
     {
-        const uint32_t mine = (uint32_t)(heads >> c0);
+        const int carries = (int)~(uint32_t)(heads >> c0);  // bit k: slot k goes on with the run of the slot before it
         real v[kRunSpan];
 #pragma unroll
         for (int k = 0; k < kRunSpan; k++) v[k] = (k < kWave - 2 * kRunSpan || full) ? row[k] : 0.0f;
         real sum = 0.0f;
 #pragma unroll
         for (int k = 0; k < kRunSpan; k++) {
-            sum = ((mine >> k) & 1) ? v[k] : sum + v[k];
+            sum = v[k] + masked(sum, bit_mask(carries, k));
             if (k < kWave - 2 * kRunSpan || full) row[k] = sum;
         }
     }
@@ -422,10 +432,20 @@ __device__ __forceinline__ void add_run_sums(real *terms, int n, uint64_t heads,
 
 __device__ __forceinline__ int top_bit(uint64_t m) { return 63 - __builtin_clzll(m); }
 
+// The largest of the wave's values that are not negative (all lanes must be active; 0 where all are negative): six operations,
+// where exchanges by LDS are six round trips, one after the other.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ int dpp_max_i32(int v) {
+    return max(v, __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, false));
+}
 __device__ __forceinline__ int wave_max_i32(int v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, kWave));
-    return v;
+    v = dpp_max_i32<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+    v = dpp_max_i32<0x112, 0xf>(v);
+    v = dpp_max_i32<0x114, 0xf>(v);
+    v = dpp_max_i32<0x118, 0xf>(v);
+    v = dpp_max_i32<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    v = dpp_max_i32<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(v, kWave - 1);
 }
 
 // Tile-order backward.  LDS floating-point atomics cost about three cycles per lane on
@@ -856,6 +876,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
         return __builtin_popcountll(first) + __builtin_popcountll(second) + __builtin_popcountll(third) + __builtin_popcountll(fourth);
     };
 
+    int span = end - start;  // list positions of the last round, from its threshold to its largest
     for (int round = 0; remaining > 0; round++) {
         // 1. the round's slots.  A round takes the wave's pending fragments from the far end of the tile's LIST, not step s
         //    of every pixel: a triangle is at another step in each pixel it covers, but at one list position, so the
@@ -863,14 +884,19 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
         //    their cache lines.  Every pixel gives a prefix of its next (at most four) steps, those at or above a
         //    threshold: the largest threshold that fills the 64 slots.  What overflows is cut off in lane order from a
         //    start lane that moves from round to round, and waits for the next round.
-        int threshold = 0, offered = slots_at(0);
+        int threshold = 0, offered = slots_at(0), match_bits = rel_bits;
         if (offered > kWave) {
-            int high = __builtin_amdgcn_readfirstlane(wave_max_i32(ahead0)) + 1;  // slots_at(threshold) >= 64 > slots_at(high) = 0
+            const int top = wave_max_i32(ahead0) + 1;
+            int high = top;  // slots_at(threshold) >= 64 > slots_at(high) = 0
+            int middle = high - 2 * span;  // first twice what the last round took, then halves
             while (high - threshold > 1) {
-                const int middle = threshold + (high - threshold) / 2;
+                if (middle <= threshold) middle = threshold + (high - threshold) / 2;
                 const int slots = slots_at(middle);
                 if (slots >= kWave) { threshold = middle; offered = slots; } else { high = middle; }
+                middle = 0;
             }
+            span = max(top - threshold, 1);
+            match_bits = 32 - __builtin_clz(span);
         }
         const bool first = ahead0 >= threshold, second = first && ahead1 >= threshold, third = second && ahead2 >= threshold,
                    fourth = third && ahead3 >= threshold;
@@ -951,11 +977,14 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
             f.gc[2] = terms[3 * kTermStride + lane];
             f.dd_dz = terms[4 * kTermStride + lane];
         }
+        // By the bits that tell positions of the round's range apart: the few positions outside it (a second step behind a
+        // first one, by depth, may come later in the list) can be taken together with others, and then make more runs, not
+        // other ones.
         uint64_t peers = __builtin_amdgcn_ballot_w64(active);
-        for (int b = 0; b < rel_bits; b++) {  // wave-uniform
-            const bool bit = (rel >> b) & 1;
-            const uint64_t vote = __builtin_amdgcn_ballot_w64(bit);
-            peers &= bit ? vote : ~vote;
+        for (int b = 0; b < match_bits; b++) {  // wave-uniform
+            const int bit = bit_mask(rel, b);
+            const uint64_t vote = __builtin_amdgcn_ballot_w64(bit != 0);
+            peers &= ~(vote ^ (uint64_t)(int64_t)bit);
         }
         const uint32_t rank = lanes_below_mask(peers);
         const bool leads = active && rank == 0;
