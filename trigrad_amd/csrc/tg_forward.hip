@@ -166,7 +166,7 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
     const int64_t groups = (int64_t)tl.grid.x * tl.grid.y * tl.grid.z;
     const bool split_tiles = !per_pixel_sort && tl.threads == kTileThreads && groups <= kFewTileGroups;
-    if (long_tiles.words) {
+    if (long_tiles.words && (per_pixel_sort || split_tiles || groups > 256 * 8)) {  // eight in tile order run on a CU at once: then none is first
         const int most = groups <= 256 ? kLongGroupsFew : split_tiles || groups <= 768 ? kLongGroupsSome : kLongGroups;
         o.long_rows = ceil_div((int)std::min<int64_t>(ceil_div(most, (int)tl.grid.z), kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
     }
@@ -191,14 +191,20 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     if (a.batch_bounds)  // they make the batches jump in steps of kSelectBatch
         return in_turn ? launch(forward_pixel_order_kernel<kSelectBatch, int, true, kLayers>, lds, lds_reserved[0])
                        : launch(forward_pixel_order_kernel<kSelectBatch, int, false, kLayers>, lds, lds_reserved[1]);
-    // Short heads are for workgroups that would wait for a place with all candidates in LDS.  Where all of them run at once
-    // anyway (three waves a SIMD, or LDS) the kernel is one chain of latencies, which the tail and its single records lengthen.
-    // Tiles of 8 x 8, us with all places and with short heads: 558 with 165 large faint triangles each 64 and 74, 323 with 240
-    // small ones 47 and 51, 943 with 7 11.6 and 12.8.  At 1024 tiles of 16 x 16 the short ones win (445 and 360).
+    // Short heads are worth it where they save a generation of workgroups (four a CU in the place of three, or eleven of a wave in
+    // the place of nine).  Where they do not, the kernel is the same number of latency chains after one another, which the tail
+    // and its single records lengthen.  Per-pixel order, frames in us with all places and with short heads: 323 tiles of 8 x 8
+    // with 240 small faint triangles each, one generation of either, kernel 47 and 51; 1224 tiles of 16 x 16, two of either, 213 and
+    // 230; 2074, three of either, 347 and 385; 3480 of 8 x 8, two of either, 250 and 275.  1000 tiles, two and one, 154 and 139;
+    // 3773, five and four, 302 and 281; 2646 of 8 x 8, two and one, 148 and 133.
     const size_t lds_all = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kLayers);
-    const int64_t at_once = 256 * std::min<int64_t>(3 * kTileThreads / n_threads, 160 * 1024 / (lds_all + 512));
-    const bool all_places = kShortHead < kLayers && groups <= at_once;
-    const size_t lds_short = all_places ? lds_all : pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kShortHead);
+    const size_t lds_heads = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kShortHead);
+    const auto generations = [&](size_t lds_bytes, int waves) {  // waves a SIMD that the registers allow; LDS comes in pieces of 1280 bytes
+        const int64_t pieces = ceil_div64((int64_t)lds_bytes + 512, 1280);
+        return ceil_div64(groups, 256 * std::min<int64_t>(waves * kTileThreads / n_threads, 128 / pieces));
+    };
+    const bool all_places = kShortHead < kLayers && generations(lds_all, 3) <= generations(lds_heads, 4);
+    const size_t lds_short = all_places ? lds_all : lds_heads;
     const auto short_kernel = all_places ? pixel_order_few_kernel(in_turn)
                               : in_turn  ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>
                                          : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>;

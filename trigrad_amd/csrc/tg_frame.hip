@@ -58,16 +58,19 @@ static FrameLayout frame_layout(const tg_frame &f) {
     L.sort_bytes = tg_build_frame_lists_workspace_bytes(f.key_capacity, tiles_x, tiles_y);
     L.sort = take(L.sort_bytes);
     L.zero_bytes = L.sort_bytes;
-    // Long: 1024 entries, and twice the mean.  In frames of so few tiles that four times as many workgroups run at once (three of
-    // a 16 x 16 tile a CU in per-pixel order, four in tile order) 1024 entries are enough, because most of the chip has nothing
-    // else to do -- unless a triangle is in more than four tiles on average: such triangles fill a pixel's layers, and depth
-    // bounds end the looking, long before the list does.  Shorter lists are served as well by the others' way.  Forward kernel,
-    // us: mesh of 1.3 million triangles, per-pixel order, 1024 entries 333, 768 336, 1400 350; 624 tiles of some 980 entries 327,
-    // shared out all the same 565; mesh of 800 000 on 42 tiles 4640, with those of twice the mean shared out 2153, with all 1118;
-    // 42 tiles with 3200 large triangles each 87, shared out 101.
+    // Long: 1024 entries, and twice the mean.  In frames with a workgroup (256 pixels) for half of the CUs at most in per-pixel
+    // order, for each CU in tile order, 1024 entries are enough, because much of the chip has nothing else to do -- unless a
+    // triangle is in more than four tiles on average: such triangles fill a pixel's layers, and depth bounds end the looking,
+    // long before the list does.  Shorter lists are served as well by the others' way.  Forward
+    // kernel, us: mesh of 1.3 million triangles, per-pixel order, 1024 entries 333, 768 336, 1400 350; mesh of 800 000 on 42 tiles
+    // 4640, with those of twice the mean shared out 2153, with all 1118; 42 tiles with 3200 large triangles each 87, shared out 101.
+    // Frames, us, all lists alike, by one workgroup each and shared out, per-pixel order: 96 workgroups with lists of 3500
+    // 492, 322; 126 with 6200 727, 406; 132 with 1700 298, 328; 182 with 1400 312, 377; 432 (tiles of 32 x 32) with 2900 314, 790.
+    // Tile order: 209 with 3500 189, 167; 238 with 1700 270, 227; 320 (32 x 32) with 3000 129, 149.
     const int64_t longest = f.key_capacity < f.n_triangles ? f.key_capacity : f.n_triangles;
     const int64_t at_once = 256 * (f.per_pixel_sort ? 3 : 8);
-    const bool few = tiles <= (f.per_pixel_sort ? 192 : 256) && f.key_capacity <= 4 * f.n_triangles;
+    const int64_t groups = (int64_t)tiles * ceil_div64(f.tile_w * f.tile_h, kTileThreads);
+    const bool few = groups <= (f.per_pixel_sort ? 128 : 256) && f.key_capacity <= 4 * f.n_triangles;
     const int64_t limit = std::max<int64_t>(1024, few ? 0 : ceil_div64(2 * f.key_capacity, tiles));
     if (longest >= limit) L.long_limit = (int)limit;
     if (L.long_limit || tiles <= at_once) {  // where the place is small, it is there whatever the number of triangles
