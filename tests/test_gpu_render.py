@@ -1200,24 +1200,27 @@ def test_frames_with_few_keys_have_the_other_routes_lists(n, width, height, cuda
         assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
 
 
-@pytest.mark.parametrize("layers", [15, 16])
-@pytest.mark.parametrize("columns,rows", [(1, 1), (127, 1), (128, 1), (43, 3), (19, 27)])
-def test_gradients_whichever_tiles_an_xcd_takes(columns, rows, layers, cuda, oracle):
-    """The saved-order backward kernel deals the tiles out to the XCDs in eighths of them, or in chunks of 16 from 16 layers on:
-    numbers of tiles around a round of chunks (128) and with a remainder, every tile with triangles of its own and shared ones."""
+@pytest.mark.parametrize("layers,tile_entries", [(15, 100), (16, 100), (16, 40)])
+@pytest.mark.parametrize("columns,rows", [(1, 1), (15, 1), (16, 1), (17, 1), (43, 3), (19, 27)])
+def test_gradients_whichever_tiles_an_xcd_takes(columns, rows, layers, tile_entries, cuda, oracle):
+    """The saved-order backward kernel deals the tiles out to the XCDs in eighths of them, or in sixteenths from either end where
+    there are 16 layers and 96 keys a tile: numbers of tiles around sixteen and with a remainder, every tile with triangles of its
+    own and shared ones."""
     import torch
     import scenes as S
-    from trigrad_amd import _C
+    import trigrad_amd
     width, height = 16 * columns - 3, 16 * rows - 5
-    n = 20 * columns * rows
-    scene = S.random_soup(n, width, height, seed=n + layers, sigma_px=9.0, opacity=(0.1, 0.5), varying_w=True)
-    d, want, got, ml = _forward_both(scene, 16, 16, dict(per_pixel_sort=True, max_layers=layers), cuda, oracle)
+    n = tile_entries * columns * rows
+    scene = S.random_soup(n, width, height, seed=n + layers, sigma_px=3.0, opacity=(0.1, 0.5), varying_w=True)
+    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, 16, 16, 1 / 256, True, layers)
+    assert (want["offsets"][-1] >= 96 * columns * rows) == (tile_entries == 100)
     gi, gd = _grad_inputs(scene, 4, True)
     wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
-                                    16, 16, True, ml, literal=False, magnitudes=True)
-    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
-    out = _C.render_backward(torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda), d["vertices"], d["indices"], d["colors"],
-                             d["opacities"], sorted_ids, offsets, bary, image, depthmap, weights, ends, width, height, 16, 16, 1 / 256,
-                             True, ml, resume=resume)
-    for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
-        assert_gradients_close(f"{columns}x{rows} tiles, {layers} layers: {label}", g.cpu().numpy(), w, mag)
+                                    16, 16, True, layers, literal=False, magnitudes=True)
+    d = to_device(scene, cuda)
+    leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+    for _ in range(2):  # a first frame, and one whose number of keys is known
+        outputs = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, max_layers=layers)
+        out = torch.autograd.grad(outputs, leaves, (torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda)))
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+            assert_gradients_close(f"{columns}x{rows} tiles, {layers} layers: {label}", g.cpu().numpy(), w, mag)

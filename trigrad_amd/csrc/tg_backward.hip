@@ -39,6 +39,7 @@ struct BackwardArgs {
     real *grad_opacities;
     int vertex_stride, color_stride, opacity_stride;  // scalars from one vertex to the next in the three arrays
     const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
+    bool deep;                    // many layers and long lists: which tiles an XCD takes (tile_of_workgroup)
 };
 
 // Lists whose sort gave up a wait are not to be read; the host finds the word and raises.
@@ -484,7 +485,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkBackward>();
+    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kEighths>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile];
     const PixelCoord p = pixel_of_thread(a, tile_id);
@@ -703,7 +704,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
     const int n_waves = blockDim.x / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kChunkBackward>();
+    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kEighths>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);
@@ -828,8 +829,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
-    const TileId tile_id = a.max_layers < kManyLayers ? tile_of_workgroup<kTileBandBackward, kChunkBackward>()
-                                                      : tile_of_workgroup<kTileBandBackward, kChunkSavedOrder>();
+    const TileId tile_id = g.deep ? tile_of_workgroup<kTileBandBackward, kSixteenths>() : tile_of_workgroup<kTileBandBackward, kEighths>();
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);
@@ -1039,7 +1039,7 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
                                   int height, int tile_w,
                                   int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers, real *grad_vertices,
                                   real *grad_colors, real *grad_opacities, int vertex_stride, int color_stride,
-                                  int opacity_stride, const uint32_t *list_status, void *stream) {
+                                  int opacity_stride, const uint32_t *list_status, int64_t n_keys, void *stream) {
     if (int e = check_raster_args("tg_render_backward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!grad_image || !vertices || !indices || !colors || !opacities || !offsets || !bary || !image ||
         !depthmap || !final_weights || !ends || !last || !grad_vertices || !grad_colors || !grad_opacities ||
@@ -1059,7 +1059,8 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
                  width, height, tile_w, tile_h, early_stopping_threshold, max_layers};
     BackwardArgs g{(const real4 *)grad_image, grad_depthmap, (const real4 *)image, depthmap, final_weights, ends, last,
                    last_depth, order, per_pixel_sort ? nullptr : hit_masks, grad_vertices, grad_colors, grad_opacities,
-                   vertex_stride, color_stride, opacity_stride, list_status};
+                   vertex_stride, color_stride, opacity_stride, list_status,
+                   max_layers >= kManyLayers && n_keys / kDeepLists >= (int64_t)ceil_div(width, tile_w) * ceil_div(height, tile_h)};
     hipStream_t s = (hipStream_t)stream;
     const int layout = (vertex_stride == 4 && color_stride == 3 && opacity_stride == 1)   ? kGradDense
                        : (vertex_stride == 8 && color_stride == 8 && opacity_stride == 8) ? kGradBlock8
@@ -1108,7 +1109,7 @@ extern "C" int tg_render_backward(const real *grad_image, const real *grad_depth
     return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
                            final_weights, ends, last, last_depth, order, hit_masks, width, height, tile_w, tile_h,
                            early_stopping_threshold, per_pixel_sort, max_layers, grad_vertices, grad_colors, grad_opacities,
-                           vertex_stride, color_stride, opacity_stride, nullptr, stream);
+                           vertex_stride, color_stride, opacity_stride, nullptr, 0, stream);
 }
 
 extern "C" int tg_render_backward_pooled(const real *grad_image, const real *grad_depthmap, const real *vertices,
@@ -1126,7 +1127,7 @@ extern "C" int tg_render_backward_pooled(const real *grad_image, const real *gra
     const OrderStore order{const_cast<uint16_t *>(order_pool), n_triangles > kShortList ? n_keys * pixels : 0, pixels};
     return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
                            final_weights, ends, last, nullptr, order, nullptr, width, height, tile_w, tile_h, early_stopping_threshold,
-                           1, max_layers, grad_vertices, grad_colors, grad_opacities, vertex_stride, color_stride, opacity_stride, nullptr, stream);
+                           1, max_layers, grad_vertices, grad_colors, grad_opacities, vertex_stride, color_stride, opacity_stride, nullptr, n_keys, stream);
 }
 
 extern "C" int tg_split_gradient_block(const real *block, int64_t n_vertices, real *grad_vertices, real *grad_colors,

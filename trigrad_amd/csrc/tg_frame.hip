@@ -243,7 +243,7 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
                                 (int)f->width, (int)f->height, (int)f->tile_w, (int)f->tile_h, (real)f->early_stopping_threshold,
                                 (int)f->per_pixel_sort, (int)f->max_layers, sums, stride ? sums + 4 : sums + 4 * V,
                                 stride ? sums + 7 : sums + 7 * V, stride ? stride : 4, stride ? stride : 3, stride ? stride : 1,
-                                (const uint32_t *)(kept + L.status), f->stream))
+                                (const uint32_t *)(kept + L.status), f->key_capacity, f->stream))
         return e;
     if (!f->per_pixel_sort) return 0;
     return tg_split_gradient_block(f->block, V, f->gradients, f->gradients + 4 * V, f->gradients + 7 * V, f->stream);

@@ -53,7 +53,7 @@ int render_backward(const real *grad_image, const real *grad_depthmap, const rea
                     const OrderStore &order, const uint64_t *hit_masks, int width, int height, int tile_w, int tile_h,
                     real early_stopping_threshold, int per_pixel_sort, int max_layers, real *grad_vertices, real *grad_colors,
                     real *grad_opacities, int vertex_stride, int color_stride, int opacity_stride, const uint32_t *list_status,
-                    void *stream);
+                    int64_t n_keys, void *stream);  // n_keys: about how many, for what does not have to be right; 0 if it is not known
 bool frame_grid_fits(int tiles_x, int tiles_y);  // at most 256 tile columns and rows: the sort passes are the tile's coordinates
 
 }  // namespace tg

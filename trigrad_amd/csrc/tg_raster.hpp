@@ -80,13 +80,16 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
 // image.  Backward, XCD k gets the k-th eighth of that order.  Forward, the order is dealt out in chunks of kChunkForward tiles:
 // where a mesh covers part of the image an eighth can be empty and another one full (1.3 million triangles of a torus,
 // 1920 x 1080: two XCDs had 45 % of the list entries, the last one none; 800 -> 680 us of kernel time), and where every tile
-// has the same work nothing is lost (10^6 triangles: 677 -> 668; chunks of 16 to 128 within 1 %).  The backward kernel with the
-// saved order takes chunks of 16 tiles of a row: the mesh 222 -> 198, 20 000 large triangles on 512 x 512 641 -> 617, 33 000 in
-// tiles of 8 x 8 234 -> 231, 10^6 triangles 1190 -> 1152; chunks of 8 or 32 within 1 %, bands of 2 and 4 rows lose up to 6 %.
+// has the same work nothing is lost (10^6 triangles: 677 -> 668; chunks of 16 to 128 within 1 %).
+// The backward kernel with the saved order takes two sixteenths, the k-th from either end: what lies in the middle, or on one side, is
+// shared by all, and neighbours stay together nearly as well.  Frames, us, in eighths and so: mesh of 1.3 million triangles 734, 721,
+// 20 000 large triangles on 512 x 512 1059, 1005, 10^6 triangles 1924, 1912 (in chunks of 16 tiles 716, 1008, 1936).
 // Gradients that tiles on two XCDs share cost more than those that stay on one.  Deep enough that does not show; with few layers
-// most of them are the nearest triangles', the large ones among which cover many tiles: 10^6 triangles with a heavy tail and 2, 8,
-// 16 layers 148, 574, 1031 us in eighths and 187, 604, 1037 in chunks.  So below kManyLayers it takes eighths, like the kernel
-// in tile order, where vertices share lines in dense gradient arrays as well (618 -> 700 with chunks of 16).
+// or short lists most of them are a few large triangles', which cover many tiles: 10^6 triangles with a heavy tail and 2, 8 layers
+// 147, 577 us in eighths and 187, 604 in chunks; 900 and 7500 triangles with a heavy tail on 1920 x 1080, lists of 12, 682, 394 in
+// eighths, 870, 485 in sixteenths.  So below kManyLayers layers or kDeepLists entries a tile (from there on 1.002 of the eighths' time
+// on average over frames of all kinds, 1.08 at worst) it takes eighths, like the kernel in tile order, where vertices share lines
+// in dense gradient arrays as well (618 -> 700 with chunks of 16).
 #ifndef TG_XCD_TILES
 #define TG_XCD_TILES 1
 #endif
@@ -101,8 +104,9 @@ __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, int t
 #endif
 constexpr int kXcds = 8;
 constexpr int kTileBandForward = TG_TILE_BAND_FORWARD, kTileBandBackward = TG_TILE_BAND_BACKWARD;
-constexpr int kChunkForward = TG_XCD_CHUNK_FORWARD, kChunkSavedOrder = 16, kChunkBackward = 0;  // 0: an eighth of the tiles
-constexpr int kManyLayers = 16;
+constexpr int kEighths = 0, kSixteenths = -1;  // in the place of a number of tiles: one eighth of them an XCD, two sixteenths
+constexpr int kChunkForward = TG_XCD_CHUNK_FORWARD;
+constexpr int kManyLayers = 16, kDeepLists = 96;
 struct TileId { int x, y, index; };
 template <int kTileBand, int kChunk>
 __device__ __forceinline__ TileId tile_of_workgroup(int skipped_rows = 0) {  // rows of workgroups in front that are not for tiles
@@ -112,12 +116,15 @@ __device__ __forceinline__ TileId tile_of_workgroup(int skipped_rows = 0) {  // 
 #if TG_XCD_TILES
     const int xcd = linear % kXcds, turn = linear / kXcds;
     int place, first = 0, left = turn;  // first: what the rounds of whole chunks take; left: turns after them
-    if (kChunk) {
+    if (kChunk > 0) {
         const int round = turn / kChunk;
         first = round * kXcds * kChunk;
         left -= round * kChunk;
     }
-    if (kChunk && first + kXcds * kChunk <= n) {
+    if (kChunk == kSixteenths) {
+        const int part = n / (2 * kXcds);  // the last tiles, fewer than 16, go as they come
+        place = turn < part ? xcd * part + turn : turn < 2 * part ? (2 * kXcds - 2 - xcd) * part + turn : linear;
+    } else if (kChunk > 0 && first + kXcds * kChunk <= n) {
         place = first + xcd * kChunk + left;
     } else {
         const int per = (n - first) / kXcds, rest = (n - first) % kXcds;
