@@ -1224,3 +1224,34 @@ def test_gradients_whichever_tiles_an_xcd_takes(columns, rows, layers, tile_entr
         out = torch.autograd.grad(outputs, leaves, (torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda)))
         for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
             assert_gradients_close(f"{columns}x{rows} tiles, {layers} layers: {label}", g.cpu().numpy(), w, mag)
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
+def test_gradients_of_a_scene_far_away(mode, cuda, oracle):
+    """w around 2e-19 (depths around 5e18): the square of an interpolation's denominator is just above the smallest normal number and its
+    reciprocal times a gradient of some hundreds is not in float32, but the w gradient is: it has the reciprocal times differences
+    of the size of w."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    scene = S.random_soup(300, 70, 45, seed=12, sigma_px=7.0, opacity=(0.2, 0.9))
+    v = scene["vertices"].copy()
+    rng = np.random.default_rng(12)
+    v[:, 2] = rng.uniform(4e18, 6e18, v.shape[0])
+    v[:, 3] = 1.0 / v[:, 2]
+    scene.update(vertices=v)
+    m = MODES[mode]
+    d, want, got, ml = _forward_both(scene, 16, 16, m, cuda, oracle)
+    _check_forward(f"far away/{mode}", want, got, (16, 16))
+    gi, gd = _grad_inputs(scene, 12, False)
+    gi = (gi * 300.0).astype(np.float32)
+    gd = np.zeros((45, 70), np.float32)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, 70, 45, 16, 16,
+                                    m["per_pixel_sort"], ml, literal=False, magnitudes=True)
+    assert all(np.isfinite(w).all() for w in wanted) and np.abs(wanted[0][:, 3]).max() > 1e19
+    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
+    out = _C.render_backward(torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda), d["vertices"], d["indices"], d["colors"],
+                             d["opacities"], sorted_ids, offsets, bary, image, depthmap, weights, ends, 70, 45, 16, 16, 1 / 256,
+                             m["per_pixel_sort"], ml, resume=resume)
+    for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+        assert_gradients_close(f"far away/{mode}: {label}", g.cpu().numpy(), w, mag)

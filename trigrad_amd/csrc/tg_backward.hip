@@ -122,12 +122,12 @@ __device__ __forceinline__ void interp_backward_scalar(real g, const real b[3], 
     // around the assignments of three arrays makes the compiler keep them in scratch memory
     const bool dead = denom * denom < kEffZero;
     const real inv = reciprocal(denom);  // the reference divides nine times, by denom and by its square
-    const real inv2 = inv * inv, g_inv2 = g * inv2;
+    const real inv2 = inv * inv;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         gb[k] = dead ? 0.0f : g * ((v[k] * w[k] * denom - nom * w[k]) * inv2);
         gv[k] = dead ? 0.0f : g * b[k] * w[k] * inv;
-        gw[k] = dead ? 0.0f : g_inv2 * (b[k] * v[k] * denom - nom * b[k]);
+        gw[k] = dead ? 0.0f : g * (b[k] * v[k] * denom - nom * b[k]) * inv2;  // g * inv2 overflows where w is around 1e-18
     }
 }
 
