@@ -1255,3 +1255,46 @@ def test_gradients_of_a_scene_far_away(mode, cuda, oracle):
                              m["per_pixel_sort"], ml, resume=resume)
     for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
         assert_gradients_close(f"far away/{mode}: {label}", g.cpu().numpy(), w, mag)
+
+
+@pytest.mark.parametrize("per_pixel_sort", [True, False])
+def test_transmittance_is_put_together_by_correctly_rounded_division(per_pixel_sort, cuda):
+    """Bit for bit, down to 2^-124 (a threshold of 0): every pixel of 32 x 32 has 52 triangles of its own, whose barycentric coordinates
+    at the pixel are 1/4, 1/4 and 1/2 exactly, so a colour gradient is a power of two times (transmittance in front of the fragment
+    * opacity), the transmittance being the image's, divided by (1 - opacity) fragment by fragment from the far end."""
+    import torch
+    from trigrad_amd import _C
+    size, layers, scale = 32, 52, np.float32(2.0 ** 60)
+    rng = np.random.default_rng(7)
+    centre = ((2 * np.arange(size) + 1) / size - 1.0).astype(np.float32)
+    h = np.float32(1.0 / 64.0)
+    corners = np.array([[-h, -h], [h, -h], [0.0, h]], np.float32)
+    v = np.zeros((layers, size, size, 3, 4), np.float32)
+    v[..., 0] = centre[None, None, :, None] + corners[:, 0]
+    v[..., 1] = centre[None, :, None, None] + corners[:, 1]
+    v[..., 2] = (1.0 + np.arange(layers))[:, None, None, None]
+    v[..., 3] = 1.0
+    opacity = rng.uniform(0.5, 0.97, (layers, size, size)).astype(np.float32)
+    n = layers * size * size
+    d = [torch.from_numpy(a).to(cuda) for a in (v.reshape(-1, 4), np.arange(3 * n, dtype=np.int32).reshape(n, 3), np.full((3 * n, 3), 0.5, np.float32),
+                                                np.repeat(opacity.reshape(-1), 3))]
+    got = _C._forward_full(*d, size, size, 16, 16, 0.0, True, per_pixel_sort, n + 1)
+    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
+    assert bool((ends == layers).all())
+    gi = torch.zeros((size, size, 4), device=cuda)
+    gi[..., :3] = float(scale)
+    out = _C.render_backward(gi, torch.zeros((size, size), device=cuda), *d, sorted_ids, offsets, bary, image, depthmap, weights, ends, size,
+                             size, 16, 16, 0.0, per_pixel_sort, n + 1, resume=resume)
+    grad = out[1].cpu().numpy().reshape(layers, size, size, 3, 3)[..., 0]
+    alpha = image.cpu().numpy()[..., 3]
+    assert 2.0 ** -124 > alpha.min() and (alpha < 2.0 ** -104).mean() > 0.5
+    compared = 0
+    for layer in range(layers - 1, -1, -1):
+        o = opacity[layer]
+        alpha = (alpha / (np.float32(1.0) - o)).astype(np.float32)
+        want = (alpha * o).astype(np.float32) * scale
+        whole = alpha > 2.0 ** -124  # below, alpha * o and the quotient itself may be denormal
+        compared += int(whole.sum())
+        differ = (grad[layer].max(-1) != (want * np.float32(0.5))) & whole
+        assert not differ.any(), f"layer {layer}: {differ.sum()} of {whole.sum()} pixels, transmittances from {alpha[differ].min():.3g}"
+    assert compared > 0.95 * n

@@ -68,14 +68,17 @@ __device__ __forceinline__ float reciprocal(float x) {
     return __builtin_amdgcn_classf(r, 0x198) ? refined : r;  // +-normal, +-denormal
 }
 __device__ __forceinline__ double reciprocal(double x) { return 1.0 / x; }
-// x / y from r = reciprocal(y): the quotient x * r put right by its exact remainder, two fused operations (Markstein's
-// correction).  What is rounded at the end is the exact quotient to within some 2^-22 units in the last place, so the result is
-// the correctly rounded one, but for a few operand pairs in millions that are as close to a tie.  Where x * r is no ordinary
-// number (an infinite x, say) the remainder is none either; then it is x / y as it is.
+// x / y, correctly rounded, for y in [1e-4, 1] and r = reciprocal(y): the quotient x * r put right by its exact remainder twice, the
+// steps of the division itself without its scaling (one of them leaves a few operand pairs in millions a unit off).  The
+// remainder is a number of float32 as long as x is above 2^-102; other x, which a pixel's transmittance is with a threshold of 0
+// only, are divided.
 __device__ __forceinline__ float quotient(float x, float y, float r) {
-    const float q = x * r;
-    const float corrected = __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
-    return __builtin_amdgcn_classf(q, 0x1f8) ? corrected : q;  // +-normal, +-denormal, +-0
+    if (__float_as_uint(x) - 0x0d800000u < 0x7f000000u - 0x0d800000u) {  // 2^-100 <= x < 2^127
+        float q = x * r;
+        q = __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
+        return __builtin_fmaf(__builtin_fmaf(-y, q, x), r, q);
+    }
+    return x / y;
 }
 __device__ __forceinline__ double quotient(double x, double y, double) { return x / y; }
 
