@@ -524,7 +524,8 @@ __device__ __forceinline__ uint64_t transpose_bits(uint64_t x, int lane) {
 // A test by broadcast costs about 20 vector instructions per entry for all 64 pixels and waits for its LDS reads (200
 // clocks where a long list leaves its tile alone on the CU); here 64 entries cost 250 instructions and 110 per row of the
 // tallest, all from registers.  500 000 triangles of a mesh, 500 x 500, tile order (longest list 5500 entries): 529 -> 367 us.
-__device__ __forceinline__ uint32_t reached_rows(const real m[9], const WaveRect &rect, real py) {
+// reached_rows reads the coordinates of eight lanes: all lanes of the wave call it, those without an entry leave the result.
+__device__ __forceinline__ uint32_t reached_rows(const real m[9], bool mine, const WaveRect &rect, real py) {
     uint32_t rows = 0;
     real mx[3];
 #pragma unroll
@@ -535,7 +536,7 @@ __device__ __forceinline__ uint32_t reached_rows(const real m[9], const WaveRect
         const bool reached = all_inside(mx[0] + m[1] * y + m[2], mx[1] + m[4] * y + m[5], mx[2] + m[7] * y + m[8]);
         rows |= reached ? 1u << r : 0u;
     }
-    return rows;
+    return mine ? rows : 0u;
 }
 // rows: the pixel rows to test.
 __device__ __forceinline__ uint64_t covered_pixels(const real m[9], uint32_t rows, real px, real py) {
@@ -562,7 +563,7 @@ __device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine
     real m[9];
 #pragma unroll
     for (int k = 0; k < 9; k++) m[k] = s_rec[lane].m[k];
-    return transpose_bits(covered_pixels(m, mine ? reached_rows(m, rect, py) : 0u, px, py), lane);
+    return transpose_bits(covered_pixels(m, reached_rows(m, mine, rect, py), px, py), lane);
 }
 
 // The inside tests of 64 entries against a wave's pixels where every lane holds an entry's matrix and nothing is in LDS (mine:
@@ -576,7 +577,7 @@ __device__ __forceinline__ uint64_t wave_hits(const real m[9], bool mine, bool b
     uint64_t todo = __builtin_amdgcn_ballot_w64(candidate), hits = 0;
     hit = 0;
     if (by_lane && __builtin_popcountll(todo) >= kSmallMin) {  // wave-uniform
-        const uint64_t covered = covered_pixels(m, candidate ? reached_rows(m, rect, py) : 0u, px, py);
+        const uint64_t covered = covered_pixels(m, reached_rows(m, candidate, rect, py), px, py);
         hit = __builtin_amdgcn_ballot_w64(covered != 0);
         return transpose_bits(covered, lane);
     }
