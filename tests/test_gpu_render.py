@@ -1298,3 +1298,49 @@ def test_transmittance_is_put_together_by_correctly_rounded_division(per_pixel_s
         differ = (grad[layer].max(-1) != (want * np.float32(0.5))) & whole
         assert not differ.any(), f"layer {layer}: {differ.sum()} of {whole.sum()} pixels, transmittances from {alpha[differ].min():.3g}"
     assert compared > 0.95 * n
+
+
+@pytest.mark.parametrize("layers", [32, 40])
+@pytest.mark.parametrize("n", [1500, 66_000])
+def test_selection_of_a_shared_out_tile_is_made_again_by_one_wave(n, layers, cuda, monkeypatch):
+    """Every fourth triangle of a tile's list is near and the others are far, so all of a pixel's nearest are candidates of one of
+    the four waves that take the list's entries in turn: more than the 23 it has places for (17 where positions take 32 bits), so
+    the merge comes to the end of its list and the selection is one wave's.  A triangle's key is its depth in one corner of the
+    tile, and its number is its place in the list.  Frame and saved order are those of the stage-by-stage route."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    size = 512  # 1024 tiles, which run at once with 23 places a candidate list and would not with all of them
+    rng = np.random.default_rng(n)
+    corner = np.float32(2.0 ** -9)  # of the tile in row 16 and column 16
+    crowd = np.ones((n, 3, 4), np.float32)
+    crowd[:, :, :2] = corner
+    crowd[:, 1, 0] = crowd[:, 2, 1] = corner + np.float32(2.0 ** -4)
+    key = 2.0 + np.arange(n) * 2.0 ** (-10 if n < 2048 else -15)
+    crowd[:, 0, 2] = key
+    crowd[:, 1:, 2] = (key + rng.integers(0, 64, n) / 64.0 + np.where(np.arange(n) % 4 == 0, 0.0, 64.0))[:, None]
+    others = S.random_soup(800, size, size, seed=n, sigma_px=4.0)
+    others["vertices"][:, 0] = others["vertices"][:, 0] * 0.4 - 0.55  # not in that tile
+    vertices = np.concatenate([crowd.reshape(-1, 4), others["vertices"]])
+    scene = dict(vertices=vertices, indices=np.arange(vertices.shape[0], dtype=np.int32).reshape(-1, 3),
+                 colors=rng.uniform(0, 1, (vertices.shape[0], 3)).astype(np.float32),
+                 opacities=rng.uniform(0.02, 0.08, vertices.shape[0]).astype(np.float32))
+    d = to_device(scene, cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], size, size, 16, 16, 1 / 256, True, True, layers)
+    for _ in range(3):  # the first frame's buffers are made for a guess of K, and what is long depends on them
+        got = _C._forward_full(*args)
+    capacity = _C._round_capacity(int(got[4][-1]))
+    assert n >= max(1024, -(-2 * capacity // 1024))  # the tile is a long one
+    tile = 16 * 32 + 16
+    assert torch.equal(got[3][int(got[4][tile]):int(got[4][tile + 1])], torch.arange(n, dtype=torch.int32, device=cuda))
+    assert int(got[6][256:272, 256:272].max()) == layers
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C._forward_full(*args)
+    for i in (0, 1, 2, 3, 4, 5, 6):
+        assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
+    if layers == 32:  # in planes
+        order = [_C.saved_blend_order(frame[8][3], frame[4], 16, 16) for frame in (got, want)]
+        taken = torch.arange(layers, device=cuda)[:, None, None] < got[6]
+        assert torch.equal(order[0][taken], order[1][taken])
+        near = order[0][:, 258, 258]
+        assert bool((near % 4 == 0).all()) and near.unique().numel() == layers

@@ -354,7 +354,7 @@ __device__ __forceinline__ int merge_lists(const Shared *shared, const TopKOf<Po
 }
 
 // A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup: each
-// takes every fourth block of 64 entries and keeps candidate lists of its own, without a barrier, and the first wave merges the
+// takes every fourth entry and keeps candidate lists of its own, without a barrier, and the first wave merges the
 // four sorted lists of a pixel, by depth and list position, while it blends.  A list was one workgroup's serial chain before,
 // 7 us for every 64 entries with most of the CU empty; it is a quarter as long now, and a tile's four squares run beside
 // each other.  What a wave tests it holds in registers, lane = entry, so only the entries that are hit go through LDS, kStage / 4
@@ -404,8 +404,10 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
         last_j = shared->last_j[lane];
         if (__builtin_amdgcn_ballot_w64(cap > 0) == 0) break;  // the same for all waves
         __syncthreads();
-        // The waves take the list's blocks of 64 entries in turn, each with candidate lists of its own, of kHead places.  Where
-        // that does not do the first wave makes the selection alone, with room for all the layers: if a wave dropped a candidate
+        // The waves take the list's entries in turn, each with candidate lists of its own, of kHead places.  (Not blocks of 64: the
+        // list is sorted by depth, so where triangles cover the square a pixel's nearest candidates are in one block, one wave's,
+        // which drops some: 30 tiles of 3000 large faint triangles among 60 000 small ones 750 us, by entries 294, one workgroup a
+        // tile 562.)  Where that does not do the first wave makes the selection alone, with room for all the layers: if a wave dropped a candidate
         // that may be among the nearest (the merge comes to the end of its list); and if a depth is NaN, which ends a candidate
         // list wherever it comes (topk_insert), so that what stays depends on what came before it.
         int found = 0, todo = 0;
@@ -415,22 +417,24 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
             found = 0;
             bool met_nan = false, dropped = false;
             if (wave < waves) {
-                const auto entry = [&](int block) { return min(start + block * kWave + lane, end - 1); };
+                // a group of the list is 64 entries for each wave
+                const int group = waves * kWave, mine = lane * waves + wave;
+                const auto entry = [&](int first) { return min(start + first + mine, end - 1); };
                 DepthParts next;
-                const auto fetch_from = [&](int block) {
-                    next.fetch_triangle(a, entry(block));
+                const auto fetch_from = [&](int first) {
+                    next.fetch_triangle(a, entry(first));
                     next.fetch_matrix(a);
-                    next.fetch_triangle(a, entry(block + waves));
+                    next.fetch_triangle(a, entry(first + group));
                     next.fetch_vertices(a);
                 };
-                fetch_from(wave);
-                for (int block = wave; block * kWave < n; block += waves) {
+                fetch_from(0);
+                for (int first = 0; first < n; first += group) {
                     if (kStage != kWave && a.batch_bounds) {
                         // as in pixel_order_tile: there are enough candidates nearer than all the rest of the list.  Each wave
                         // knows that of a quarter of them in every wave's lists; at a depth of its own the rest might come
                         // before another wave's candidate.
-                        const real rest = a.batch_bounds[batch_bound_index(start, tile.index, block * kWave)];
-                        const int resume = a.far_start[tile.index] / kWave;
+                        const real rest = a.batch_bounds[batch_bound_index(start, tile.index, first)];
+                        const int resume = a.far_start[tile.index] / group * group;
                         bool settled = cap == 0;
                         if (!settled && waves == 1) settled = found == room && tk.d(room - 1) <= rest;
                         if (!settled && waves > 1) {
@@ -438,41 +442,41 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
 #pragma unroll
                             for (int w = 0; w < kMaxTileWaves; w++) settled = settled && s_quarter[w * kWave + lane] < rest;
                         }
-                        if (resume > block && !__builtin_amdgcn_ballot_w64(!settled)) {
-                            block = resume + (wave - resume % waves + waves) % waves;
-                            if (block * kWave >= n) break;
-                            fetch_from(block);
+                        if (resume > first && !__builtin_amdgcn_ballot_w64(!settled)) {
+                            first = resume;
+                            if (first >= n) break;
+                            fetch_from(first);
                         }
                     }
                     const DepthRecord r = next.record();
                     next.fetch_matrix(a);
-                    next.fetch_triangle(a, entry(block + 2 * waves));
+                    next.fetch_triangle(a, entry(first + 2 * group));
                     uint64_t hit;
-                    uint64_t m = wave_hits(r.m, block * kWave + lane < n, squares, rect, p.px, p.py, hit);
+                    uint64_t m = wave_hits(r.m, first + mine < n, squares, rect, p.px, p.py, hit);
                     if (cap == 0) m = 0;
                     next.fetch_vertices(a);
                     while (hit) {  // wave-uniform: the hit entries' records through LDS, kStaged at a time
                         const uint32_t rank = lanes_below_mask(hit);
                         const bool staged = ((hit >> lane) & 1) && rank < (uint32_t)kStaged;
-                        const uint64_t group = __builtin_amdgcn_ballot_w64(staged);
+                        const uint64_t there = __builtin_amdgcn_ballot_w64(staged);
                         if (staged) s_rec[rank] = r;
                         wave_lds_sync();
-                        uint64_t mine = m & group;
-                        while (__builtin_amdgcn_ballot_w64(mine != 0)) {
-                            if (mine == 0) continue;
-                            const int e = __builtin_ctzll(mine);
-                            mine &= mine - 1;
-                            const DepthRecord &d = s_rec[__builtin_popcountll(group & ((1ull << e) - 1))];
+                        uint64_t todo = m & there;
+                        while (__builtin_amdgcn_ballot_w64(todo != 0)) {
+                            if (todo == 0) continue;
+                            const int e = __builtin_ctzll(todo);
+                            todo &= todo - 1;
+                            const DepthRecord &d = s_rec[__builtin_popcountll(there & ((1ull << e) - 1))];
                             real b0, b1, b2;
                             bary_apply(d.m, p.px, p.py, b0, b1, b2);
                             const real pd = interp_w(b0, b1, b2, d.z[0], d.z[1], d.z[2], d.w[0], d.w[1], d.w[2]);  // render.cu:404
-                            const int j = block * kWave + e;
+                            const int j = first + e * waves + wave;
                             met_nan = met_nan || pd != pd;
                             if (pd < last_depth || (pd == last_depth && j <= last_j)) continue;
                             dropped = dropped || (found == room && room < cap);
                             topk_insert(tk, room, found, pd, j);
                         }
-                        hit &= ~group;
+                        hit &= ~there;
                         wave_lds_sync();
                     }
                     const int quarter = (cap + kMaxTileWaves - 1) / kMaxTileWaves;
