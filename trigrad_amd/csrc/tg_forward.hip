@@ -72,11 +72,12 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
     }
 }
 
-// Workgroups for the long tiles, at most, by the number of the others: they cost 1 us for every 300 or so that find nothing to
-// do, and what they find may be too much for them.  Few others (a CU each): 54 tiles of 32 x 32 in tile order 110 us with 1024
-// groups, 158 with 512, 210 with 256.  As many as run at once: mesh of 500 000, 1024 tiles, 121, 121, 149; mesh of 700 000 in
-// per-pixel order, 437 tiles, 308, 310, 317.  More: mesh of 1.3 million, 8160 tiles, 128 to 1024 groups within 1 %.
-constexpr int kLongGroupsFew = 1024, kLongGroupsSome = 512, kLongGroups = 128;
+// Workgroups for the long tiles where they are shared out, at most: as many as run at once, four a CU; fewer may find too much
+// (1920 x 1080, 200 tiles of 1100 large faint triangles among 60 000 small ones, forward, us: 128 workgroups 630, 512 396, 1024
+// 339, one for each tile 478; without a limit on the layers 1597, 890, 637, 1048; 54 tiles of 32 x 32 in tile order, 256 210, 512
+// 158, 1024 110).  Those that find nothing cost nothing that shows: 10^6 triangles 671 with 128 and 670 with 1024, 10^5 253 and
+// 254, a mesh of 1.3 million 716 and 718.
+constexpr int kLongGroups = 1024;
 TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_threads) {
     TileLaunch t;
     const int pixels = tile_w * tile_h;
@@ -167,8 +168,9 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     const int64_t groups = (int64_t)tl.grid.x * tl.grid.y * tl.grid.z;
     const bool split_tiles = !per_pixel_sort && tl.threads == kTileThreads && groups <= kFewTileGroups;
     if (long_tiles.words && (per_pixel_sort || split_tiles || groups > 256 * 8)) {  // eight in tile order run on a CU at once: then none is first
-        const int most = groups <= 256 ? kLongGroupsFew : split_tiles || groups <= 768 ? kLongGroupsSome : kLongGroups;
-        o.long_rows = ceil_div((int)std::min<int64_t>(ceil_div(most, (int)tl.grid.z), kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
+        const bool shared_out = per_pixel_sort ? tl.threads == kTileThreads : split_tiles;
+        const int most = ceil_div(shared_out ? kLongGroups : kLongTileSlots, (int)tl.grid.z);
+        o.long_rows = ceil_div((int)std::min<int64_t>(most, kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
     }
     const dim3 grid(tl.grid.x, tl.grid.y + o.long_rows, tl.grid.z);
     const int n_threads = tl.threads;
