@@ -320,7 +320,10 @@ int tg_list_bounds(const tg_real *vertices, int32_t n_vertices, const int32_t *i
  * list_status (may be NULL): the status word of the call that made the lists.  If it
  * is not TG_STATUS_OK when the kernel runs, the lists are not read: image and depthmap
  * are filled with NaN (ends, last 0), so that an invalid frame shows in the frame itself.
- * max_layers must be > 0 (the Python layer maps <= 0 to M+1, wrapper.py:35). */
+ * max_layers must be > 0 (the Python layer maps <= 0 to M+1, wrapper.py:35).
+ * tg_candidate_places: how many of the 32 nearest candidates of a pixel a frame in per-pixel order without batch_bounds keeps
+ * in LDS (the others are in registers); which it is changes the time only. */
+int tg_candidate_places(int width, int height, int tile_w, int tile_h);
 size_t tg_hit_mask_words(int64_t n_keys, int width, int height, int tile_w, int tile_h);
 int tg_render_forward(const tg_real *vertices, const int32_t *indices, const tg_real *colors, const tg_real *opacities,
                       const int32_t *sorted_ids, const int32_t *offsets, const tg_real *bary, int width, int height,

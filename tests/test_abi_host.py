@@ -31,6 +31,28 @@ def test_library_exports_every_declared_entry_point(bits):
     assert lib.tg_precision_bits() == bits
 
 
+@pytest.mark.parametrize("tile_w,tile_h,at_once_32,at_once_23", [
+    (8, 8, 9, 11), (2, 2, 9, 11), (8, 16, 5, 7), (12, 16, 3, 5), (16, 16, 3, 4), (20, 13, 3, 4),
+])
+def test_candidate_places_save_a_generation_of_workgroups(tile_w, tile_h, at_once_32, at_once_23):
+    """at_once: workgroups a CU with 32 and with 23 places of 6 bytes a thread in LDS next to 64 staged records of 64 bytes: by
+    160 KB of LDS in pieces of 1280 bytes, and by three and four waves a SIMD, which the kernels are compiled for."""
+    from trigrad_amd import _lib
+    lib = _lib.load(32)
+    threads = -(-tile_w * tile_h // 64) * 64
+    split = -(-tile_w * tile_h // min(threads, 256))  # workgroups of a tile
+    threads = min(threads, 256)
+    for places, at_once, waves in ((32, at_once_32, 3), (23, at_once_23, 4)):
+        pieces = -(-(64 * 64 + places * threads * 6 + 512) // 1280)
+        assert at_once == min(128 // pieces, waves * 256 // threads)
+    for tiles in sorted({256 * n * k + d for n in (at_once_32, at_once_23) for k in (1, 2, 3) for d in (-1, 0, 1)}):
+        groups = split * tiles
+        generations = [-(-groups // (256 * n)) for n in (at_once_32, at_once_23)]
+        assert lib.tg_candidate_places(tile_w * tiles, tile_h, tile_w, tile_h) == (32 if generations[0] <= generations[1] else 23)
+    assert lib.tg_candidate_places(0, 16, 16, 16) == 0 and lib.tg_candidate_places(64, 64, 64, 32) == 0
+    assert _lib.load(64).tg_candidate_places(8192, 8192, 16, 16) == 32
+
+
 @pytest.mark.parametrize("bits", [32, 64])
 def test_host_side_helpers_and_argument_rejection(bits):
     from trigrad_amd import _lib

@@ -56,6 +56,7 @@ SIGNATURES = {
     "tg_bary": (_i, [_p, _i32, _p, _i32, _p, _p]),
     "tg_list_bound_words": (_sz, [_i64, _i]),
     "tg_list_bounds": (_i, [_p, _i32, _p, _i32, _p, _p, _p, _i, _p, _p, _p, _p]),
+    "tg_candidate_places": (_i, [_i, _i, _i, _i]),
     "tg_hit_mask_words": (_sz, [_i64, _i, _i, _i, _i]),
     "tg_render_forward": (_i, [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _f, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     "tg_order_pool_words": (_i64, [_i64, _i64, _i, _i]),

@@ -112,6 +112,21 @@ size_t pixel_order_lds_bytes(int n_threads, int staged_entries, size_t position_
     return sizeof(DepthRecord) * staged_entries + (size_t)places * n_threads * (sizeof(real) + position_bytes);
 }
 
+// Places of a pixel's candidate list that a launch with 16-bit positions keeps in LDS: kShortHead or all.
+// Short heads are worth it where they save a generation of workgroups (four a CU in the place of three, or eleven of a wave in
+// the place of nine).  Where they do not, the kernel is the same number of latency chains after one another, which the tail
+// and its single records lengthen.  Per-pixel order, frames in us with all places and with short heads: 323 tiles of 8 x 8
+// with 240 small faint triangles each, one generation of either, kernel 47 and 51; 1224 tiles of 16 x 16, two of either, 213 and
+// 230; 2074, three of either, 347 and 385; 3480 of 8 x 8, two of either, 250 and 275.  1000 tiles, two and one, 154 and 139;
+// 3773, five and four, 302 and 281; 2646 of 8 x 8, two and one, 148 and 133.
+static int candidate_places(int64_t groups, int n_threads) {
+    const auto generations = [&](int places) {  // LDS comes in pieces of 1280 bytes
+        const int64_t pieces = ceil_div64((int64_t)pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), places) + 512, 1280);
+        return ceil_div64(groups, 256 * std::min<int64_t>(short_list_waves(places) * kTileThreads / n_threads, 128 / pieces));
+    };
+    return generations(kLayers) <= generations(kShortHead) ? kLayers : kShortHead;
+}
+
 int check_raster_args(const char *fn, int width, int height, int tile_w, int tile_h, int max_layers) {
     if (width <= 0 || height <= 0 || tile_w <= 0 || tile_h <= 0 || tile_w * tile_h > kMaxTilePixels) {
         set_error("%s: image size must be positive and tile_w*tile_h in [1, %d]", fn, kMaxTilePixels);
@@ -131,6 +146,12 @@ int check_raster_args(const char *fn, int width, int height, int tile_w, int til
 }  // namespace tg
 
 using namespace tg;
+
+extern "C" int tg_candidate_places(int width, int height, int tile_w, int tile_h) {
+    if (width <= 0 || height <= 0 || tile_w <= 0 || tile_h <= 0 || tile_w * tile_h > kMaxTilePixels) return 0;
+    const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, pixel_order_threads(kTileThreads));
+    return candidate_places((int64_t)tl.grid.x * tl.grid.y * tl.grid.z, tl.threads);
+}
 
 extern "C" size_t tg_hit_mask_words(int64_t n_keys, int width, int height, int tile_w, int tile_h) {
     if (n_keys < 0 || width <= 0 || height <= 0 || tile_w <= 0 || tile_h <= 0 || tile_w * tile_h > kMaxTilePixels) return 0;
@@ -193,20 +214,9 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     if (a.batch_bounds)  // they make the batches jump in steps of kSelectBatch
         return in_turn ? launch(forward_pixel_order_kernel<kSelectBatch, int, true, kLayers>, lds, lds_reserved[0])
                        : launch(forward_pixel_order_kernel<kSelectBatch, int, false, kLayers>, lds, lds_reserved[1]);
-    // Short heads are worth it where they save a generation of workgroups (four a CU in the place of three, or eleven of a wave in
-    // the place of nine).  Where they do not, the kernel is the same number of latency chains after one another, which the tail
-    // and its single records lengthen.  Per-pixel order, frames in us with all places and with short heads: 323 tiles of 8 x 8
-    // with 240 small faint triangles each, one generation of either, kernel 47 and 51; 1224 tiles of 16 x 16, two of either, 213 and
-    // 230; 2074, three of either, 347 and 385; 3480 of 8 x 8, two of either, 250 and 275.  1000 tiles, two and one, 154 and 139;
-    // 3773, five and four, 302 and 281; 2646 of 8 x 8, two and one, 148 and 133.
-    const size_t lds_all = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kLayers);
-    const size_t lds_heads = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), kShortHead);
-    const auto generations = [&](size_t lds_bytes, int waves) {  // waves a SIMD that the registers allow; LDS comes in pieces of 1280 bytes
-        const int64_t pieces = ceil_div64((int64_t)lds_bytes + 512, 1280);
-        return ceil_div64(groups, 256 * std::min<int64_t>(waves * kTileThreads / n_threads, 128 / pieces));
-    };
-    const bool all_places = kShortHead < kLayers && generations(lds_all, 3) <= generations(lds_heads, 4);
-    const size_t lds_short = all_places ? lds_all : lds_heads;
+    const int places = candidate_places(groups, n_threads);
+    const bool all_places = kShortHead < kLayers && places == kLayers;
+    const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), places);
     const auto short_kernel = all_places ? pixel_order_few_kernel(in_turn)
                               : in_turn  ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>
                                          : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>;

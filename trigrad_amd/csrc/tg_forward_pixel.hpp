@@ -32,6 +32,9 @@ constexpr int kSelectBatchShort = 64;   // ... and where they take 16 bits
 // Lists with depth bounds keep all places in LDS and three kinds of 16-bit positions lose there: 200 000 faint triangles 288
 // us, with 29 places and three workgroups a CU 301, with 21 and four 338: every pixel has 32 candidates.
 constexpr int kShortHead = sizeof(real) == 4 ? 23 : kLayers;
+// Waves a SIMD that the registers of the instances with 16-bit positions are held to, by their places in LDS: what the kernel is
+// compiled with, and what the choice between them counts on (candidate_places).
+constexpr int short_list_waves(int head) { return head < kLayers ? 4 : 3; }
 constexpr int kLongHead = sizeof(real) == 4 ? 17 : 24;  // the same LDS with int positions, in long_tile_part
 static_assert((sizeof(real) + sizeof(int)) * kLongHead <= (sizeof(real) + sizeof(uint16_t)) * kShortHead, "the same LDS");
 
@@ -531,7 +534,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
 // Workgroups a CU: what their LDS allows.  No bound in double precision: held to two workgroups every instance spills (10^5
 // triangles, 1024 x 1024: 229 us instead of 223, tiles of 8 x 8 190 instead of 168).
 template <int kStage, typename Pos, bool kInTurn, int kHead>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage != kSelectBatchShort ? 2 : kInTurn && kHead < kLayers ? 4 : 3)
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage != kSelectBatchShort ? 2 : short_list_waves(kHead))
 void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ uint8_t s_touch[kStage];
