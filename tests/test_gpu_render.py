@@ -1156,12 +1156,17 @@ def test_long_tiles_match_the_other_route(width, per_pixel_sort, cuda, monkeypat
 
 @pytest.mark.parametrize("layers", [5, 23, 24, 27, 32, 40, -1])
 @pytest.mark.parametrize("n", [22, 23, 24, 25, 31, 32, 33, 60])
-@pytest.mark.parametrize("size", [24, 460])
-def test_candidate_lists_around_their_places_in_lds(size, n, layers, cuda, oracle):
-    """A pixel's first 23 candidates are kept in LDS, the others up to 32 in registers -- or all in LDS, where there are so few
-    workgroups (768 of 16 x 16 tiles, some 2500 of 8 x 8) that they run at once all the same: n triangles over every pixel, tilted, so
-    that their order at a pixel is not the list's, a third of them at equal depths, and layers that end inside either part."""
+@pytest.mark.parametrize("size,tiles,places", [
+    (24, [(16, 16), (8, 8), (8, 16)], 32),
+    (400, [(8, 8)], 23),  # one wave to a workgroup
+    (460, [(16, 16), (8, 16), (12, 16)], 23),  # four waves, two and three
+])
+def test_candidate_lists_around_their_places_in_lds(size, tiles, places, n, layers, cuda, oracle):
+    """A pixel's first 23 candidates are kept in LDS, the others up to 32 in registers -- or all in LDS, where that takes no more
+    generations of workgroups: n triangles over every pixel, tilted, so that their order at a pixel is not the list's, a third of
+    them at equal depths, and layers that end inside either part."""
     import scenes as S
+    from trigrad_amd import _lib
     rng = np.random.default_rng(100 * n + layers)
     z = rng.uniform(1.0, 5.0, (n, 1)) * rng.uniform(0.5, 1.5, (n, 3))
     z[::3] = rng.choice([2.0, 3.0], (z[::3].shape[0], 1))
@@ -1169,11 +1174,11 @@ def test_candidate_lists_around_their_places_in_lds(size, n, layers, cuda, oracl
     vertices = np.concatenate([xy, z[:, :, None], 1.0 / z[:, :, None]], axis=-1).astype(np.float32).reshape(-1, 4)
     scene = dict(S.random_soup(n, size, size, seed=n, opacity=(0.02, 0.3)), vertices=vertices)
     mode = dict(per_pixel_sort=True, max_layers=layers)
-    _, want, got, _ = _forward_both(scene, 16, 16, mode, cuda, oracle)
-    assert int(want["ends"].max()) == min(n, layers if layers > 0 else n)
-    _check_forward(f"{n} candidates, {layers} layers", want, got, (16, 16))
-    _, want, got, _ = _forward_both(scene, 8, 8, mode, cuda, oracle)  # one wave to a workgroup
-    _check_forward(f"{n} candidates, {layers} layers, small tiles", want, got, (8, 8))
+    for tw, th in tiles:
+        assert _lib.load(32).tg_candidate_places(size, size, tw, th) == places
+        _, want, got, _ = _forward_both(scene, tw, th, mode, cuda, oracle)
+        assert int(want["ends"].max()) == min(n, layers if layers > 0 else n)
+        _check_forward(f"{n} candidates, {layers} layers, tiles of {tw} x {th}", want, got, (th, tw))
 
 
 @pytest.mark.parametrize("width,height", [(16, 16), (70, 45), (1024, 1024), (1040, 1024)])
@@ -1309,8 +1314,9 @@ def test_selection_of_a_shared_out_tile_is_made_again_by_one_wave(n, layers, cud
     tile, and its number is its place in the list.  Frame and saved order are those of the stage-by-stage route."""
     import torch
     import scenes as S
-    from trigrad_amd import _C
+    from trigrad_amd import _C, _lib
     size = 512  # 1024 tiles, which run at once with 23 places a candidate list and would not with all of them
+    assert _lib.load(32).tg_candidate_places(size, size, 16, 16) == 23
     rng = np.random.default_rng(n)
     corner = np.float32(2.0 ** -9)  # of the tile in row 16 and column 16
     crowd = np.ones((n, 3, 4), np.float32)
