@@ -33,7 +33,9 @@ def _nan_equal(a, b):
     return np.array_equal(a, b, equal_nan=True)
 
 
-def _forward_both(scene, tw, th, mode, cuda, oracle, thr=1 / 256):
+def _forward_both(scene, tw, th, mode, cuda, oracle, thr=1 / 256, frames=1):
+    """frames: which frame of the scene it is; the first one's buffers are made for a guess of K, and what is a long tile, or
+    sorted by one workgroup, goes by the buffers."""
     from trigrad_amd import _C
     W, H = scene["width"], scene["height"]
     d = to_device(scene, cuda)
@@ -41,9 +43,27 @@ def _forward_both(scene, tw, th, mode, cuda, oracle, thr=1 / 256):
     ml = mode["max_layers"] if mode["max_layers"] > 0 else M + 1
     want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], W, H, tw, th, thr,
                          mode["per_pixel_sort"], ml)
-    got = _C._forward_full(d["vertices"], d["indices"], d["colors"], d["opacities"], W, H, tw, th, thr, True,
-                            mode["per_pixel_sort"], ml)
+    for _ in range(frames):
+        got = _C._forward_full(d["vertices"], d["indices"], d["colors"], d["opacities"], W, H, tw, th, thr, True,
+                               mode["per_pixel_sort"], ml)
     return d, want, got, ml
+
+
+def _long_tile_limit(scene, tw, th, per_pixel_sort, n_keys):
+    """How many list entries make a tile a long one, in a frame whose number of keys is known: 1024 and twice the mean, but in a
+    frame of few workgroups and small triangles 1024."""
+    from trigrad_amd import _C
+    capacity, n = _C._round_capacity(int(n_keys)), scene["indices"].shape[0]
+    tiles = -(-scene["width"] // tw) * -(-scene["height"] // th)
+    few = tiles * -(-tw * th // 256) <= (128 if per_pixel_sort else 256) and capacity <= 4 * n
+    return 1024 if few else max(1024, -(-2 * capacity // tiles))
+
+
+def _shared_out(got, want, tw, th):
+    """Of a frame in tile order: the tiles whose pixels were several workgroups', of which the saved hit masks do not say how far
+    they got (the words in front of them, one for each workgroup of a tile)."""
+    n_tiles, parts = want["offsets"].size - 1, -(-tw * th // 256)
+    return (got[8][4][:n_tiles * parts].view(n_tiles, parts) == -1).all(1).cpu().numpy()
 
 
 def _check_forward(name, want, got, tile_shape):
@@ -153,8 +173,15 @@ def _crowded_scene(n, width, height):
 ])
 def test_crowds_of_small_triangles_match_oracle(n, width, height, tw, th, mode, cuda, oracle):
     scene = _crowded_scene(n, width, height)
-    _, want, got, _ = _forward_both(scene, tw, th, MODES[mode], cuda, oracle)
+    _, want, got, _ = _forward_both(scene, tw, th, MODES[mode], cuda, oracle, frames=3)
     _check_forward(f"crowd {n}/{tw}x{th}/{mode}", want, got, (th, tw))
+    lengths = np.diff(want["offsets"])
+    long = lengths >= _long_tile_limit(scene, tw, th, MODES[mode]["per_pixel_sort"], lengths.sum())
+    assert long.any() == (n > 1500)
+    # with depth bounds where lists are of 512 entries on average and more, in per-pixel order
+    assert (lengths.mean() >= 512) == (n == 12000)
+    if not MODES[mode]["per_pixel_sort"]:
+        assert np.array_equal(_shared_out(got, want, tw, th), long & (-(-tw * th // 64) >= 4))
 
 
 @pytest.mark.parametrize("mode", ["A_default", "B_unlimited"])
@@ -1114,8 +1141,12 @@ def test_long_tiles_shared_out(n, sigma, tw, th, mode, cuda, oracle):
     v[n:, :, 0] = v[n:, :, 0] * 0.3 + 0.6  # the others beside it
     scene.update(width=width, height=height)
     m = MODES[mode]
-    d, want, got, ml = _forward_both(scene, tw, th, m, cuda, oracle)
-    assert np.diff(want["offsets"])[0] == n and np.diff(want["offsets"])[1:].max() < 100
+    d, want, got, ml = _forward_both(scene, tw, th, m, cuda, oracle, frames=3)
+    lengths = np.diff(want["offsets"])
+    assert lengths[0] == n and lengths[1:].max() < 100
+    assert _long_tile_limit(scene, tw, th, m["per_pixel_sort"], lengths.sum()) == 1024
+    if not m["per_pixel_sort"]:
+        assert np.array_equal(_shared_out(got, want, tw, th), lengths >= 1024)
     _check_forward(f"long tile {n}/{tw}x{th}/{mode}", want, got, (th, tw))
     gi, gd = _grad_inputs(scene, 9, True)
     wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
