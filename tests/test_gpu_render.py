@@ -1215,9 +1215,9 @@ def test_candidate_lists_around_their_places_in_lds(size, tiles, places, n, laye
 @pytest.mark.parametrize("width,height", [(16, 16), (70, 45), (1024, 1024), (1040, 1024)])
 @pytest.mark.parametrize("n", [1, 40, 700, 1020, 1030, 2040, 2060, 4090, 4100, 6200, 8200])
 def test_frames_with_few_keys_have_the_other_routes_lists(n, width, height, cuda, monkeypatch):
-    """Frames of up to some 8000 keys and 4096 tiles are sorted by one workgroup, by tile, and by depth as well up to some 900:
-    around the numbers of keys a thread takes, with equal depths (the order is then the triangles'), tiles without a key, and a
-    tile whose list is a long one.  Lists and image are those of the stage-by-stage route."""
+    """Frames whose buffers are for up to 8192 keys (6372 of the frame) and 4096 tiles are sorted by one workgroup, by tile, and by
+    depth as well up to 2048 (911): around the numbers of keys a thread takes, with equal depths (the order is then the triangles'),
+    tiles without a key, and a tile whose list is a long one.  Lists and image are those of the stage-by-stage route."""
     import torch
     import scenes as S
     from trigrad_amd import _C
@@ -1230,6 +1230,34 @@ def test_frames_with_few_keys_have_the_other_routes_lists(n, width, height, cuda
     args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, 16, 16, 1 / 256, True, True, 32)
     for _ in range(3):  # the first frame's buffers are made for a guess of K, and the route goes by them
         got = _C.render_forward(*args)
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C.render_forward(*args)
+    for i in (0, 1, 2, 3, 4, 5, 6):
+        assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
+
+
+@pytest.mark.parametrize("width,height", [(16, 16), (1024, 1024), (1040, 1024)])
+@pytest.mark.parametrize("n_keys,capacity", [(911, 2048), (912, 3072), (6372, 8192), (6373, 9216)])
+def test_frames_with_few_keys_at_the_edges_of_their_rule(n_keys, capacity, width, height, cuda, monkeypatch):
+    """Every triangle is in one tile, so the number of keys is theirs: the last and the first one on either side of a buffer of
+    2048 keys (sorted by depth by the one workgroup) and of 8192 (by tile), with 1, 4096 and 4160 tiles."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    soup = S.random_soup(n_keys, 16, 16, seed=n_keys, sigma_px=2.0, opacity=(0.02, 0.3))
+    rng = np.random.default_rng(n_keys)
+    v = soup["vertices"].reshape(n_keys, 3, 4).copy()
+    v[:, :, :2] = rng.uniform(-0.9, 0.9, (n_keys, 3, 2))  # of a tile
+    size, tiles = np.array([width, height]), np.array([width, height]) // 16
+    at = rng.integers(0, tiles, (n_keys, 1, 2)) if width > 16 else np.zeros((n_keys, 1, 2))
+    at[: n_keys // 2] = tiles // 2  # half of them in one
+    v[:, :, :2] = ((v[:, :, :2] + 1.0) * 8.0 + 16.0 * at) / size * 2.0 - 1.0
+    v[::3, :, 2:] = (2.0, 0.5)  # equal depths
+    d = to_device(dict(soup, vertices=v.astype(np.float32).reshape(-1, 4)), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, 16, 16, 1 / 256, True, True, 32)
+    for _ in range(3):  # the first frame's buffers are made for a guess of K, and the route goes by them
+        got = _C.render_forward(*args)
+    assert int(got[4][-1]) == n_keys and _C._round_capacity(n_keys) == capacity
     monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
     want = _C.render_forward(*args)
     for i in (0, 1, 2, 3, 4, 5, 6):

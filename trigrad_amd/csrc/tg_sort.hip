@@ -866,7 +866,9 @@ __global__ __launch_bounds__(kSegLargeThreads) void segment_sort_large_kernel(ui
 // Two sweeps are two launches that wait for one another, each nine microseconds of latency however little there is to sort.
 // Up to kFewKeys pairs fit the LDS of one workgroup, which sorts them by tile (one or two stable 8-bit passes) and looks the
 // tiles' bounds up in the sorted pairs; the segment sort follows as ever.  Up to kFewestKeys it sorts them by depth as well,
-// before that, and the segment sort's launch goes too.  Sweeps and segment sort, and now, us: 20 triangles (100 keys) 25 -> 12,
+// before that, and the segment sort's launch goes too.  Both are compared with the buffers' capacity, because K is known on the
+// device only; the Python layer's capacity is K, an eighth more and 1024, rounded up, so a frame of up to 6372 keys is sorted
+// here, of up to 911 by depth as well, and a first frame, whose buffers are made for a guess, is not.  Sweeps and segment sort, and now, us: 20 triangles (100 keys) 25 -> 12,
 // 1000 (2600) 26 -> 18, 225 large ones (4000) 27 -> 23, 2000 (4500) 28 -> 24.  By depth as well at 2600 keys: 25.
 constexpr int kFewKeys = kSegLargeThreads * 8, kFewestKeys = kSegLargeThreads * 2;
 constexpr int kFewKeysTiles = 4096;  // a tile's bound is a search of thirteen LDS reads, four of them a thread
