@@ -187,7 +187,7 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
                  list_status, host_status, long_tiles, 0};
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
     const int64_t groups = (int64_t)tl.grid.x * tl.grid.y * tl.grid.z;
-    const bool split_tiles = !per_pixel_sort && tl.threads == kTileThreads && groups <= kFewTileGroups;
+    const bool split_tiles = kSharesLongTiles && !per_pixel_sort && tl.threads == kTileThreads && groups <= kFewTileGroups;
     if (long_tiles.words && (per_pixel_sort || split_tiles || groups > 256 * 8)) {  // eight in tile order run on a CU at once: then none is first
         const bool shared_out = per_pixel_sort ? tl.threads == kTileThreads : split_tiles;
         const int most = ceil_div(shared_out ? kLongGroups : kLongTileSlots, (int)tl.grid.z);
@@ -198,7 +198,7 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     hipStream_t s = (hipStream_t)stream;
     if (!per_pixel_sort) {
         if (split_tiles)
-            TG_LAUNCH(forward_tile_order_few_kernel, grid, dim3(n_threads), 0, s, a, o);
+            TG_LAUNCH_AS("forward_tile_order_few_kernel", tile_order_few_kernel(), grid, dim3(n_threads), 0, s, a, o);
         else
             TG_LAUNCH(forward_tile_order_kernel, grid, dim3(n_threads), 0, s, a, o);
         return check_launch("forward_tile_order_kernel");

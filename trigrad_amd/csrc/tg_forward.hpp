@@ -162,10 +162,12 @@ __device__ __forceinline__ void tile_order_tile(const RasterArgs &a, const Forwa
 }
 
 // The kernels of launches with few workgroups (tg_forward_few.hip): forward_tile_order_kernel's, and forward_pixel_order_kernel
-// with all of a candidate list's places in LDS.
+// with all of a candidate list's places in LDS.  Null in the double build, which has neither: every launch has all places in LDS
+// there, and long tiles are noted by tg_frame_forward, a call of the float build.
 constexpr int kFewTileGroups = 1024;
-__global__ void forward_tile_order_few_kernel(RasterArgs a, ForwardOut out);
+constexpr bool kSharesLongTiles = sizeof(real) == 4;
 using ForwardKernel = void (*)(RasterArgs, ForwardOut);
+ForwardKernel tile_order_few_kernel();
 ForwardKernel pixel_order_few_kernel(bool in_turn);
 
 }  // namespace tg

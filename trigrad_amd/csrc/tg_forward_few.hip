@@ -4,6 +4,11 @@
 
 namespace tg {
 
+#ifdef TG_DOUBLE_PRECISION
+ForwardKernel tile_order_few_kernel() { return nullptr; }
+ForwardKernel pixel_order_few_kernel(bool) { return nullptr; }
+#else
+
 // A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup, in
 // tile order: each tests 64 of 256 entries, lane = entry, from registers; the records of those that are hit go to LDS, and the
 // first wave composites them in list order.  500 000 triangles of a mesh, 500 x 500 (longest list 5500, a tile one workgroup's
@@ -86,9 +91,9 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
     if (out.hit_masks && tid == 0) out.hit_masks[hit_mask_head_index(tile.index)] = ~0ull;
 }
 
-// Shared out, a tile with a long list is four waves' work for each of its squares.  That takes 121 registers, four waves per
+// Shared out, a tile with a long list is four waves' work for each of its squares.  That takes 120 registers, four waves per
 // SIMD, which up to 1024 workgroups do not need more of; a launch of more is better off with eight (forward_tile_order_kernel).
-__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void forward_tile_order_few_kernel(RasterArgs a, ForwardOut out) {
+__global__ __launch_bounds__(kTileThreads, 4) void forward_tile_order_few_kernel(RasterArgs a, ForwardOut out) {
     __shared__ TileOrderLds s;
     if (lists_invalid(out)) {  // the same for the whole launch
         mark_tile_invalid(a, out);
@@ -107,12 +112,11 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void forwa
     tile_order_tile(a, out, tile, start, end, s);
 }
 
-// In double precision every launch has all places in LDS; there is no second kernel then.
-template <int kStage>
-static ForwardKernel all_places_kernel(bool in_turn) {
-    if constexpr (kShortHead == kLayers) return nullptr;
-    else return in_turn ? forward_pixel_order_kernel<kStage, uint16_t, true, kLayers> : forward_pixel_order_kernel<kStage, uint16_t, false, kLayers>;
+ForwardKernel tile_order_few_kernel() { return forward_tile_order_few_kernel; }
+ForwardKernel pixel_order_few_kernel(bool in_turn) {
+    return in_turn ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kLayers>
+                   : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kLayers>;
 }
-ForwardKernel pixel_order_few_kernel(bool in_turn) { return all_places_kernel<kSelectBatchShort>(in_turn); }
+#endif
 
 }  // namespace tg

@@ -35,7 +35,7 @@ constexpr int kShortHead = sizeof(real) == 4 ? 23 : kLayers;
 // Waves a SIMD that the registers of the instances with 16-bit positions are held to, by their places in LDS: what the kernel is
 // compiled with, and what the choice between them counts on (candidate_places).
 constexpr int short_list_waves(int head) { return head < kLayers ? 4 : 3; }
-constexpr int kLongHead = sizeof(real) == 4 ? 17 : 24;  // the same LDS with int positions, in long_tile_part
+constexpr int kLongHead = 17;  // the same LDS with int positions, in long_tile_part
 static_assert((sizeof(real) + sizeof(int)) * kLongHead <= (sizeof(real) + sizeof(uint16_t)) * kShortHead, "the same LDS");
 
 // The last places of a candidate list, in registers: place kPlace and those behind it.  (A structure of its own for every place:
@@ -544,7 +544,7 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
         return;
     }
     const bool first = (int)blockIdx.y < out.long_rows;
-    if constexpr (kInTurn) {
+    if constexpr (kInTurn && kSharesLongTiles) {
         if (first) {
             __shared__ real s_quarter[kStage != kWave ? kTileThreads : 1];  // with depth bounds; batches of 64 go without
             const int n_items = kMaxTileWaves * out.long_tiles.words[0];
