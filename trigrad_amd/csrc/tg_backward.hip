@@ -250,9 +250,9 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
     real dxy[3][2];
     {
         // The reference divides each of the 21 numerators below by T or d (util.h:405-455).  Here the two
-        // reciprocals are formed once and multiplied in: every quotient is within two units in the last
-        // place of the reference's, and 19 of the fragment's 50 divisions go away.  The numerators keep the
-        // reference's form: its differences of screen coordinates cancel, and for a sliver that rounding
+        // reciprocals are formed once: T's is multiplied into l0..l2, each within two units in the last place of
+        // the reference's quotient, and d's into the six sums of three products, whose 18 quotients are not formed
+        // (19 of the fragment's 50 divisions go away).  The numerators keep the reference's form: its differences of screen coordinates cancel, and for a sliver that rounding
         // is larger than the tolerance of the comparison, so the shorter closed form
         // (-l_v * row k of the matrix) does not reproduce the reference's numbers.
         // Nor are they fused: a fused multiply-add moves l0..l2 by as much as the reference's own rounding

@@ -86,15 +86,13 @@ TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_th
     return t;
 }
 
-// Workgroup size of the per-pixel-sort kernels.  Their candidate lists take
-// 32 * (scalar + int) bytes of LDS per thread: 64 KB for the 256 threads of a
-// 16x16 tile.  The selection kernels are bound by latency, so what counts is
-// how many waves a CU holds: the forward kernel stages 128 list entries at a
-// time (7.5 KB), two workgroups of 256 threads fit a CU.  Measured on the five
-// configurations against 64, 192 and 256 staged entries and against tiles split
-// over two workgroups of 128 threads or four of 64 (which stage every entry two
-// or four times): 15 to 35 % faster than 256 entries and 128 threads.  The
-// re-selecting backward kernel also keeps 43 KB of gradient sums.
+// Workgroup size of the per-pixel-sort kernels: the 256 threads of a 16x16 tile.  They are bound by latency, so what counts is
+// how many waves a CU holds, and that is set by the candidate lists in LDS.  With int positions (depth bounds, longest lists,
+// and the re-selecting backward kernel, which also keeps 43 KB of gradient sums) those take 32 * (scalar + int) bytes a thread,
+// 64 KB a workgroup, two a CU next to 128 staged entries (8 KB); with 16-bit positions 48 KB, three, or 34.5 KB with 23
+// places, four (candidate_places).  Measured with int positions on frames of all sizes against 64, 192 and 256 staged entries
+// and against tiles split over two workgroups of 128 threads or four of 64 (which stage every entry two or four times): 15 to
+// 35 % faster than 256 entries and 128 threads.
 // TRIGRAD_PIXEL_ORDER_THREADS (64, 128 or 256) overrides the workgroup size.
 int pixel_order_threads(int preferred) {
     static int override = -1;
