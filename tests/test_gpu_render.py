@@ -1185,6 +1185,64 @@ def test_long_tiles_match_the_other_route(width, per_pixel_sort, cuda, monkeypat
         assert torch.equal(got[i].view(torch.int32), want[i].view(torch.int32)), i
 
 
+@pytest.mark.parametrize("tw,width,entries,layers,crowded,per_tile", [
+    *[(16, 512, 4, 32, crowded, 1100) for crowded in (1, 31, 33, 150)],  # with 23 places a candidate list
+    *[(16, 320, 4, 32, crowded, 1100) for crowded in (1, 40, 150)],  # with all of them
+    *[(16, 320, 700, 40, crowded, 4000) for crowded in (1, 40)],  # with depth bounds, where they do not help
+    *[(24, 384, 4, -1, crowded, 1100) for crowded in (1, 40, 150)],  # a tile is two workgroups
+])
+def test_tiles_that_are_done_help_with_the_long_ones(tw, width, entries, layers, crowded, per_tile, cuda, monkeypatch):
+    """Up to 1024 workgroups, of which those of short lists draw the long tiles' work by a counter that ends at zero: the raster
+    phase is run twice on the same lists, into another image each time, and both are the stage-by-stage route's.  From fewer long
+    tiles than there are workgroups in front of the others (one item for four of them) to several items for each."""
+    import ctypes as C
+    import struct
+    import torch
+    import scenes as S
+    from trigrad_amd import _C, _lib
+    columns, rows = width // tw, width // 16
+    tiles, rng = columns * rows, np.random.default_rng(crowded)
+    soup = S.random_soup(entries * tiles + crowded * per_tile, width, width, seed=crowded, sigma_px=1.5, opacity=(0.02, 0.3))
+    v = soup["vertices"].reshape(-1, 3, 4).copy()
+    at = rng.choice(tiles, crowded, replace=False)[np.arange(crowded * per_tile) % crowded]
+    corner = np.stack([at % columns * tw, at // columns * 16], axis=-1)[:, None]
+    pixels = corner + rng.uniform(0.3, 15.7, (crowded * per_tile, 3, 2))
+    v[: crowded * per_tile, :, :2] = pixels / width * 2.0 - 1.0
+    d = to_device(dict(soup, vertices=v.astype(np.float32).reshape(-1, 4)), cuda)
+    n = d["indices"].shape[0]
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, width, tw, 16, 1 / 256, True, layers if layers > 0 else n + 1)
+    for _ in range(2):  # the first frame's buffers are made for a guess of K, and what is long depends on them
+        frame = _C.frame_forward(*args)[3]
+    lib = _lib.load(32)
+    real, others = lib.tg_frame_forward, []
+
+    def forward(call):
+        other = torch.zeros((width, width, 4), device=cuda)
+        words = list(struct.unpack_from("<14Q", call))
+        struct.pack_into("<Q", call, 4 * 8, other.data_ptr())
+        struct.pack_into("<Q", call, 13 * 8, _C._FRAME_BIN | _C._FRAME_LISTS | _C._FRAME_RASTER)
+        assert real(call) == 0
+        struct.pack_into("<Q", call, 4 * 8, words[4])
+        struct.pack_into("<Q", call, 13 * 8, _C._FRAME_RASTER | _C._FRAME_WAIT)
+        others.append(other)
+        return real(call)
+
+    monkeypatch.setattr(lib, "tg_frame_forward", forward)
+    image, depthmap, kept, frame = _C.frame_forward(*args)
+    monkeypatch.setattr(lib, "tg_frame_forward", real)
+    frame.status.verify()
+    *_, offsets, _, _, _ = _C._frame_results(image, depthmap, kept, frame, width, width, tw, 16, True, args[-1], n)
+    lengths = (offsets[1:] - offsets[:-1]).cpu().numpy()
+    scene = dict(width=width, height=width, indices=d["indices"])
+    assert (lengths >= _long_tile_limit(scene, tw, 16, True, frame.n_keys)).sum() == crowded
+    assert tiles * -(-tw // 16) <= 1024 and (lengths.mean() >= 512) == (entries == 700)
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C.render_forward(*args[:9], True, True, args[-1])
+    assert len(others) == 1
+    for got in (image, others[0]):
+        assert torch.equal(got.view(torch.int32), want[0].view(torch.int32))
+
+
 @pytest.mark.parametrize("layers", [5, 23, 24, 27, 32, 40, -1])
 @pytest.mark.parametrize("n", [22, 23, 24, 25, 31, 32, 33, 60])
 @pytest.mark.parametrize("size,tiles,places", [

@@ -76,7 +76,9 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
 // (1920 x 1080, 200 tiles of 1100 large faint triangles among 60 000 small ones, forward, us: 128 workgroups 630, 512 396, 1024
 // 339, one for each tile 478; without a limit on the layers 1597, 890, 637, 1048; 54 tiles of 32 x 32 in tile order, 256 210, 512
 // 158, 1024 110).  Those that find nothing cost nothing that shows: 10^6 triangles 671 with 128 and 670 with 1024, 10^5 253 and
-// 254, a mesh of 1.3 million 716 and 718.
+// 254, a mesh of 1.3 million 716 and 718.  They do where there is one generation of workgroups, which in per-pixel order therefore
+// has the places that are left and at least 128 of them, and help from the tiles' own (forward_pixel_order_helping_kernel; depth
+// bounds, where two workgroups run on a CU, keep to the many in front: 200 000 faint triangles 845 us, with help 850).
 constexpr int kLongGroups = 1024;
 TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_threads) {
     TileLaunch t;
@@ -186,10 +188,12 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, per_pixel_sort ? pixel_order_threads(kTileThreads) : kTileThreads);
     const int64_t groups = (int64_t)tl.grid.x * tl.grid.y * tl.grid.z;
     const bool split_tiles = kSharesLongTiles && !per_pixel_sort && tl.threads == kTileThreads && groups <= kFewTileGroups;
+    bool tiles_help = false;
     if (long_tiles.words && (per_pixel_sort || split_tiles || groups > 256 * 8)) {  // eight in tile order run on a CU at once: then none is first
         const bool shared_out = per_pixel_sort ? tl.threads == kTileThreads : split_tiles;
-        const int most = ceil_div(shared_out ? kLongGroups : kLongTileSlots, (int)tl.grid.z);
-        o.long_rows = ceil_div((int)std::min<int64_t>(most, kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
+        tiles_help = kSharesLongTiles && shared_out && per_pixel_sort && !a.batch_bounds && groups <= kLongGroups;
+        const int most = tiles_help ? std::max(kLongGroups - (int)groups, kLongTileSlots) : shared_out ? kLongGroups : kLongTileSlots;
+        o.long_rows = ceil_div((int)std::min<int64_t>(ceil_div(most, (int)tl.grid.z), kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
     }
     const dim3 grid(tl.grid.x, tl.grid.y + o.long_rows, tl.grid.z);
     const int n_threads = tl.threads;
@@ -202,7 +206,7 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
         return check_launch("forward_tile_order_kernel");
     }
     const size_t lds = pixel_order_lds_bytes(n_threads, kSelectBatch);
-    static size_t lds_reserved[6][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
+    static size_t lds_reserved[8][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
     const bool in_turn = n_threads == kTileThreads;
     const auto launch = [&](void (*kernel)(RasterArgs, ForwardOut), size_t lds_bytes, size_t *reserved) -> int {
         if (int e = reserve_lds("tg_render_forward", (const void *)kernel, lds_bytes, reserved)) return e;
@@ -215,10 +219,11 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     const int places = candidate_places(groups, n_threads);
     const bool all_places = kShortHead < kLayers && places == kLayers;
     const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), places);
-    const auto short_kernel = all_places ? pixel_order_few_kernel(in_turn)
-                              : in_turn  ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>
-                                         : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>;
-    if (int e = launch(short_kernel, lds_short, lds_reserved[2 + 2 * all_places + in_turn])) return e;
+    const auto short_kernel = tiles_help   ? pixel_order_helping_kernel(all_places)
+                              : all_places ? pixel_order_few_kernel(in_turn)
+                              : in_turn    ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>
+                                           : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>;
+    if (int e = launch(short_kernel, lds_short, lds_reserved[tiles_help ? 6 + all_places : 2 + 2 * all_places + in_turn])) return e;
     // no list is too long for 16-bit positions, or those that are are long tiles, which the kernel above has shared out
     if (longest <= kShortList || (in_turn && o.long_rows && long_tiles.limit <= kShortList)) return 0;
     if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;

@@ -162,12 +162,14 @@ __device__ __forceinline__ void tile_order_tile(const RasterArgs &a, const Forwa
 }
 
 // The kernels of launches with few workgroups (tg_forward_few.hip): forward_tile_order_kernel's, and forward_pixel_order_kernel
-// with all of a candidate list's places in LDS.  Null in the double build, which has neither: every launch has all places in LDS
-// there, and long tiles are noted by tg_frame_forward, a call of the float build.
+// with all of a candidate list's places in LDS, and where the tiles' workgroups help with the long tiles.  Null in the double
+// build, which has none of them: every launch has all places in LDS there, and long tiles are noted by tg_frame_forward, a call of
+// the float build.
 constexpr int kFewTileGroups = 1024;
 constexpr bool kSharesLongTiles = sizeof(real) == 4;
 using ForwardKernel = void (*)(RasterArgs, ForwardOut);
 ForwardKernel tile_order_few_kernel();
 ForwardKernel pixel_order_few_kernel(bool in_turn);
+ForwardKernel pixel_order_helping_kernel(bool all_places);
 
 }  // namespace tg

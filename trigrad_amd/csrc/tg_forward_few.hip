@@ -1,5 +1,6 @@
 // tg_forward_few.hip -- the forward kernels of launches with few workgroups: in tile order one that shares the long tiles' work
-// out, in per-pixel order the instances with all of a candidate list's places in LDS.
+// out, in per-pixel order one whose workgroups help with the long tiles, and the instances with all of a candidate list's places
+// in LDS.
 #include "tg_forward_pixel.hpp"
 
 namespace tg {
@@ -7,6 +8,7 @@ namespace tg {
 #ifdef TG_DOUBLE_PRECISION
 ForwardKernel tile_order_few_kernel() { return nullptr; }
 ForwardKernel pixel_order_few_kernel(bool) { return nullptr; }
+ForwardKernel pixel_order_helping_kernel(bool) { return nullptr; }
 #else
 
 // A wave's share (64 pixels; the part-th of its workgroup's) of a tile with a long list, by the four waves of a workgroup, in
@@ -112,10 +114,61 @@ __global__ __launch_bounds__(kTileThreads, 4) void forward_tile_order_few_kernel
     tile_order_tile(a, out, tile, start, end, s);
 }
 
+// forward_pixel_order_kernel with 16-bit positions of a launch whose workgroups run at once: those that are done with a tile's list help with the long tiles.
+// So there need not be a workgroup in front of the others for each item (a long tile's square) that there may be, and there had
+// better not: they change which tiles meet on a CU, which a launch of one generation has no others to make up for (20 000 large
+// triangles on 1024 tiles without a limit on the layers, forward, us: 128 in front 366, 1024 387), and 128 alone find too much
+// (1024 tiles, 200 with 3000 large faint triangles, frames, us: 128 1735, 1024 772, 128 and the tiles' 793; 100 such tiles 970, 573,
+// 603; 784 tiles, 30 such 310, 310, 310).
+//
+// The first items are those of the workgroups in front, in order.  If there are more, every workgroup that is done draws the next
+// one until it draws one beyond the last: a draw for each item behind the first ones, and one more of every workgroup.  That is one
+// for each item and each tile in all; the last of them finds the counter at items + tiles - 1 and leaves it at zero, for another
+// launch.
+static_assert(kMaxTilePixels <= kLongTileCounters * kTileThreads, "a counter for each of a tile's workgroups");
+template <int kHead>
+__global__ __launch_bounds__(kTileThreads, short_list_waves(kHead)) void forward_pixel_order_helping_kernel(RasterArgs a, ForwardOut out) {
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    __shared__ uint8_t s_touch[kSelectBatchShort];
+    __shared__ WaveRect s_rects[kMaxTileWaves];
+    __shared__ int s_drawn;
+    if (lists_invalid(out)) {  // the same for the whole launch
+        mark_tile_invalid(a, out);
+        return;
+    }
+    const bool first = (int)blockIdx.y < out.long_rows;
+    if (!first) {
+        const TileId tile = tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
+        const int n = a.offsets[tile.index + 1] - a.offsets[tile.index];
+        if (!is_long_tile(out, n) && n <= kShortList)
+            pixel_order_tile<kSelectBatchShort, uint16_t, true, kHead>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
+    }
+    const auto items = [&] { return kMaxTileWaves * out.long_tiles.words[0]; };
+    const auto draw = [&] {
+        if (items() <= long_groups(out)) return items();
+        __syncthreads();  // all have read the last one
+        if (threadIdx.x == 0)
+            s_drawn = (int)atomicInc(out.long_tiles.taken + blockIdx.z, (uint32_t)items() + gridDim.x * (gridDim.y - out.long_rows) - 1);
+        __syncthreads();
+        return long_groups(out) + s_drawn;
+    };
+    for (int item = first ? long_group(out) : draw(); item < items(); item = draw()) {
+        const TileId tile = tile_of_index(out.long_tiles.all[item / kMaxTileWaves]);
+        const int part = item % kMaxTileWaves, n = a.offsets[tile.index + 1] - a.offsets[tile.index];
+        if (n <= kShortList)
+            long_tile_part<kSelectBatchShort, uint16_t, kHead>(a, out, tile, part, s_dyn, nullptr);
+        else
+            long_tile_part<kSelectBatchShort, int, kLongHead>(a, out, tile, part, s_dyn, nullptr);
+    }
+}
+
 ForwardKernel tile_order_few_kernel() { return forward_tile_order_few_kernel; }
 ForwardKernel pixel_order_few_kernel(bool in_turn) {
     return in_turn ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kLayers>
                    : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kLayers>;
+}
+ForwardKernel pixel_order_helping_kernel(bool all_places) {
+    return all_places ? forward_pixel_order_helping_kernel<kLayers> : forward_pixel_order_helping_kernel<kShortHead>;
 }
 #endif
 

@@ -74,9 +74,9 @@ static FrameLayout frame_layout(const tg_frame &f) {
     const int64_t limit = std::max<int64_t>(1024, few ? 0 : ceil_div64(2 * f.key_capacity, tiles));
     if (longest >= limit) L.long_limit = (int)limit;
     if (L.long_limit || tiles <= at_once) {  // where the place is small, it is there whatever the number of triangles
-        L.long_tiles = take((1 + kLongTileSlots) * 4);
+        L.long_tiles = take((kLongTileCounters + 1 + kLongTileSlots) * 4);
         L.all_long_tiles = take((size_t)tiles * 4);
-        L.zero_bytes = L.long_tiles + 4 - L.sort;
+        L.zero_bytes = L.long_tiles + (kLongTileCounters + 1) * 4 - L.sort;
     }
     if (f.flags & TG_FRAME_LIST_BOUNDS) {
         L.bounds = take(tg_list_bound_words(f.key_capacity, tiles) * sizeof(real));
@@ -174,7 +174,9 @@ extern "C" int tg_frame_forward(tg_frame *f) {
     volatile uint32_t *host = f->host;
     const int64_t longest = f->key_capacity < f->n_triangles ? f->key_capacity : f->n_triangles;  // a triangle is in a list once
     LongTiles long_tiles;
-    if (L.long_limit) long_tiles = LongTiles{(int32_t *)(scratch + L.long_tiles), (int32_t *)(scratch + L.all_long_tiles), L.long_limit, std::min<int64_t>(tiles, f->key_capacity / L.long_limit)};
+    if (L.long_limit)
+        long_tiles = LongTiles{(int32_t *)(scratch + L.long_tiles) + kLongTileCounters, (int32_t *)(scratch + L.all_long_tiles), L.long_limit,
+                               std::min<int64_t>(tiles, f->key_capacity / L.long_limit), (uint32_t *)(scratch + L.long_tiles)};
     if (f->phases & TG_FRAME_BIN) {
         host[1] = 0;
         host[2] = TG_FRAME_PENDING;

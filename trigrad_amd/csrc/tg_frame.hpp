@@ -24,12 +24,13 @@ struct FrameCount {
 // workgroup's serial work, and what the whole launch waits for is the longest.  The segment sort, which makes the lists'
 // bounds, notes every tile with `limit` entries or more.  words: how many there are, then the first kLongTileSlots of them; all:
 // all of them; most: no more of them are possible.  Null words: there can be none.
-constexpr int kLongTileSlots = 128;
+constexpr int kLongTileSlots = 128, kLongTileCounters = 4;
 struct LongTiles {
     int32_t *words = nullptr;
     int32_t *all = nullptr;  // room for every tile
     int limit = 0;
     int64_t most = 0;
+    uint32_t *taken = nullptr;  // a counter for each of a tile's workgroups, for a launch that shares the work out; zero between launches
 };
 
 // tg_bin_frame with two outputs more: the bary matrices, and K for the host (may be null).
