@@ -78,8 +78,10 @@ __global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_k
 // 158, 1024 110).  Those that find nothing cost nothing that shows: 10^6 triangles 671 with 128 and 670 with 1024, 10^5 253 and
 // 254, a mesh of 1.3 million 716 and 718.  They do where there is one generation of workgroups, which in per-pixel order therefore
 // has the places that are left and at least 128 of them, and help from the tiles' own (forward_pixel_order_helping_kernel; depth
-// bounds, where two workgroups run on a CU, keep to the many in front: 200 000 faint triangles 845 us, with help 850).
-constexpr int kLongGroups = 1024;
+// bounds, where two workgroups run on a CU, keep to the many in front: 200 000 faint triangles 845 us, with help 850), and in tile
+// order, from 257 workgroups on, half as many (400 tiles with lists of 1000 large faint triangles, frames, us: 246, with 1024 275; 576
+// with 350, 184 and 196; 1024 tiles, 100 of them with 3000, 497 and 496).
+constexpr int kLongGroups = 1024, kLongGroupsTileOrder = 512;
 TileLaunch tile_launch(int width, int height, int tile_w, int tile_h, int max_threads) {
     TileLaunch t;
     const int pixels = tile_w * tile_h;
@@ -192,7 +194,10 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     if (long_tiles.words && (per_pixel_sort || split_tiles || groups > 256 * 8)) {  // eight in tile order run on a CU at once: then none is first
         const bool shared_out = per_pixel_sort ? tl.threads == kTileThreads : split_tiles;
         tiles_help = kSharesLongTiles && shared_out && per_pixel_sort && !a.batch_bounds && groups <= kLongGroups;
-        const int most = tiles_help ? std::max(kLongGroups - (int)groups, kLongTileSlots) : shared_out ? kLongGroups : kLongTileSlots;
+        int most = kLongGroups;
+        if (tiles_help) most = std::max(kLongGroups - (int)groups, kLongTileSlots);
+        else if (!shared_out) most = kLongTileSlots;
+        else if (!per_pixel_sort && groups > 256) most = kLongGroupsTileOrder;
         o.long_rows = ceil_div((int)std::min<int64_t>(ceil_div(most, (int)tl.grid.z), kMaxTileWaves * long_tiles.most), (int)tl.grid.x);
     }
     const dim3 grid(tl.grid.x, tl.grid.y + o.long_rows, tl.grid.z);
