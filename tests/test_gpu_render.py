@@ -1467,3 +1467,51 @@ def test_selection_of_a_shared_out_tile_is_made_again_by_one_wave(n, layers, cud
         assert torch.equal(order[0][taken], order[1][taken])
         near = order[0][:, 258, 258]
         assert bool((near % 4 == 0).all()) and near.unique().numel() == layers
+
+
+def _with_w(scene, w):
+    v = scene["vertices"].copy()
+    v[:, 3] = w
+    v[:, 2] = 1.0 / np.where(v[:, 3] == 0.0, 1.0, v[:, 3])
+    return dict(scene, vertices=v)
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
+@pytest.mark.parametrize("w", ["soup_varying_w", "degenerate", "overlap_mesh_inf_w", "unit_square_negative_z", 0.9e-6, 1.1e-6, 0.9e6, 1.1e6,
+                               1e-20, 1e-30, 1e-38, 1e30, 0.0, "around zero", "inf"])
+def test_gradients_where_the_depth_map_has_none(w, mode, cuda):
+    """A frame whose depth map took no part in the loss has kernels of its own, which leave out what is 0 times the depth's derivatives
+    but keep the NaNs it makes where those are not finite: against the general ones with a gradient of zeros."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    from trigrad_amd._C import _forward_full
+    if w in SCENES:
+        scene, tw, th = SCENES[w]()
+    else:
+        rng = np.random.default_rng(3)
+        scene, tw, th = S.random_soup(400, 70, 45, seed=3, sigma_px=7.0, opacity=(0.2, 0.9)), 16, 16
+        n = scene["vertices"].shape[0]
+        with np.errstate(all="ignore"):
+            if w == "around zero":
+                scene = _with_w(scene, (rng.standard_normal(n) * 1e-3).astype(np.float32))
+            elif w == "inf":  # some vertices
+                scene = _with_w(scene, np.where(rng.random(n) < 0.05, np.inf, rng.uniform(0.1, 2.0, n)).astype(np.float32))
+            else:
+                scene = _with_w(scene, (w * rng.uniform(1.0, 1.0001, n)).astype(np.float32))
+    m = MODES[mode]
+    W, H = scene["width"], scene["height"]
+    d = to_device(scene, cuda)
+    ml = m["max_layers"] if m["max_layers"] > 0 else scene["indices"].shape[0] + 1
+    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = _forward_full(
+        d["vertices"], d["indices"], d["colors"], d["opacities"], W, H, tw, th, 1 / 256, True, m["per_pixel_sort"], ml)
+    gi, gd = _grad_inputs(scene, 3, False)
+    outs = [_C.render_backward(torch.from_numpy(gi).to(cuda), g, d["vertices"], d["indices"], d["colors"], d["opacities"], sorted_ids,
+                               offsets, bary, image, depthmap, weights, ends, W, H, tw, th, 1 / 256, m["per_pixel_sort"], ml, resume=resume)
+            for g in (None, torch.from_numpy(gd).to(cuda))]
+    for label, got, want in zip(("grad_vertices", "grad_colors", "grad_opacities"), *(tuple(g.cpu().numpy() for g in out) for out in outs)):
+        # the same terms, added in another order: within the rounding of a sum of some hundreds of the array's largest
+        finite = np.isfinite(want)
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want), err_msg=label)
+        largest = float(np.abs(want[finite]).max()) if finite.any() else 0.0
+        assert_close(f"{w}/{mode}: {label}", np.where(finite, got, 0), np.where(finite, want, 0), 1e-4, 300 * 2.0 ** -24 * largest + 1e-30)

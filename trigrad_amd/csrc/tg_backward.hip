@@ -45,19 +45,32 @@ struct BackwardArgs {
 // Lists whose sort gave up a wait are not to be read; the host finds the word and raises.
 __device__ __forceinline__ bool lists_invalid(const BackwardArgs &g) { return g.list_status && *g.list_status != TG_STATUS_OK; }
 
+// Most losses are of the image alone: kDepth = false is for a frame whose depth map has no gradient.  Its terms by way of the depth
+// are then zeros, a sixth of a fragment's arithmetic, and are left out, but for the cases where they are 0 times infinity: the
+// NaNs that make of a gradient are kept (depth_is_ordinary, load_back_state).  The saved-order kernel then needs 96 registers, not
+// 117, and five waves a SIMD find room: 10^6 triangles 1219 -> 1043 us, 20 000 without a limit on the layers 604 -> 541; in tile order
+// 619 -> 594.
+
 // process_backward's inputs for one list entry.
-struct alignas(16) BackRecord {
-    real m[9];
-    real w[3];
+template <bool kDepth>
+struct VertexDepths {
     real iw[3];
     real iw2[3];  // 1 / (w * w)
+};
+template <>
+struct VertexDepths<false> {};
+template <bool kDepth>
+struct alignas(16) BackRecord : VertexDepths<kDepth> {
+    real m[9];
+    real w[3];
     real op[3];
     real col[9];
     real xy[6];   // ax, ay, bx, by, cx, cy
     int id[3];
 };
-constexpr int kBackReals = 36;  // scalars in front of the ids
-static_assert(offsetof(BackRecord, id) == kBackReals * sizeof(real), "BackRecord layout");
+
+// Whether any lane of the wave meets a case that has to be put right (wave-uniform; laid out as the exception).
+__device__ __forceinline__ bool any_lane(bool x) { return __builtin_expect(__builtin_amdgcn_ballot_w64(x) != 0, 0); }
 
 // 1 / x to within one unit in the last place: the hardware estimate and one Newton step where
 // the estimate is an ordinary number (zero, infinity and NaN pass through as they are).  Used
@@ -68,12 +81,18 @@ __device__ __forceinline__ float reciprocal(float x) {
     return __builtin_amdgcn_classf(r, 0x198) ? refined : r;  // +-normal, +-denormal
 }
 __device__ __forceinline__ double reciprocal(double x) { return 1.0 / x; }
+__device__ __forceinline__ float reciprocal_of_normal(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+__device__ __forceinline__ double reciprocal_of_normal(double x) { return 1.0 / x; }
 // x / y, correctly rounded, for y in [1e-4, 1] and r = reciprocal(y): the quotient x * r put right by its exact remainder twice, the
 // steps of the division itself without its scaling (one of them leaves a few operand pairs in millions a unit off).  The
 // remainder is a number of float32 as long as x is above 2^-102; other x, which a pixel's transmittance is with a threshold of 0
 // only, are divided, with the lanes beside them.  (A branch of the wave, not of the lane, which cost the saved-order kernel 1 %, 10^6
-// triangles 1239 us, so 1218; scaled by div_fmas without a branch 1234.
-// Not expected, because else the division is made in every case: 1238.)
+// triangles 1239 us, so 1218; scaled by div_fmas without a branch 1234.  Not expected, and said so here and not in a function
+// around the condition, because else the division is made in every case: 1238.  One test for the whole walk, of the
+// smallest transmittance at its start, is three operations a fragment less and slower: 1003, 1028.)
 __device__ __forceinline__ float quotient(float x, float y, float r) {
     const bool ordinary = __float_as_uint(x) - 0x0d800000u < 0x7f000000u - 0x0d800000u;  // 2^-100 <= x < 2^127
     float q = x * r;
@@ -84,7 +103,17 @@ __device__ __forceinline__ float quotient(float x, float y, float r) {
 }
 __device__ __forceinline__ double quotient(double x, double y, double) { return x / y; }
 
-__device__ __forceinline__ void gather_back(const RasterArgs &a, int j, BackRecord &r) {
+// gradients only: 1 / w to within one unit in the last place, and its square for 1 / (w * w)
+__device__ __forceinline__ void vertex_depths(const real w[3], VertexDepths<true> &r) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        r.iw[k] = reciprocal(w[k]);
+        r.iw2[k] = r.iw[k] * r.iw[k];
+    }
+}
+
+template <bool kDepth>
+__device__ __forceinline__ void gather_back(const RasterArgs &a, int j, BackRecord<kDepth> &r) {
     const TriIds t = load_ids(a, j);
     const real *m = a.bary + 9 * (int64_t)t.tri;
     real4v va = *reinterpret_cast<const real4v *>(a.vertices + t.ia), vb = *reinterpret_cast<const real4v *>(a.vertices + t.ib),
@@ -102,9 +131,7 @@ __device__ __forceinline__ void gather_back(const RasterArgs &a, int j, BackReco
     // saved-order kernel); here, behind all loads, because it is where they are waited for
     asm("" : "+v"(va), "+v"(vb), "+v"(vc));
     r.w[0] = va[3]; r.w[1] = vb[3]; r.w[2] = vc[3];
-    // gradients only: 1 / w to within one unit in the last place, and its square for 1 / (w * w)
-    r.iw[0] = reciprocal(r.w[0]); r.iw[1] = reciprocal(r.w[1]); r.iw[2] = reciprocal(r.w[2]);
-    r.iw2[0] = r.iw[0] * r.iw[0]; r.iw2[1] = r.iw[1] * r.iw[1]; r.iw2[2] = r.iw[2] * r.iw[2];
+    if constexpr (kDepth) vertex_depths(r.w, r);
     r.xy[0] = va[0]; r.xy[1] = va[1]; r.xy[2] = vb[0]; r.xy[3] = vb[1]; r.xy[4] = vc[0]; r.xy[5] = vc[1];
     r.id[0] = t.ia; r.id[1] = t.ib; r.id[2] = t.ic;
 }
@@ -118,22 +145,22 @@ struct BackState {
 
 constexpr int kTerms = 21;  // per vertex v: [7v+0] x, [7v+1] y, [7v+2] w, [7v+3..5] rgb, [7v+6] opacity
 
-// util.h:299-317 scalar interpolate3_backward.
-__device__ __forceinline__ void interp_backward_scalar(real g, const real b[3], const real v[3], const real w[3],
+// util.h:299-317 scalar interpolate3_backward.  -> the reference returns early there (util.h:303) and all results are zero: the
+// caller's to set, once for all of a fragment's and in a branch that a wave rarely takes.  (A selection at every result is a branch
+// around its arithmetic, twelve a fragment: the compiler does not move arithmetic across them.)
+__device__ __forceinline__ bool interp_backward_scalar(real g, const real b[3], const real v[3], const real w[3],
                                                        real gb[3], real gv[3], real gw[3]) {
     const real nom = (b[0] * w[0] * v[0] + b[1] * w[1] * v[1]) + b[2] * w[2] * v[2];
     const real denom = (b[0] * w[0] + b[1] * w[1]) + b[2] * w[2];
-    // all zero where the reference returns early (util.h:303); written as selections, because a branch
-    // around the assignments of three arrays makes the compiler keep them in scratch memory
-    const bool dead = denom * denom < kEffZero;
     const real inv = reciprocal(denom);  // the reference divides nine times, by denom and by its square
     const real inv2 = inv * inv;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        gb[k] = dead ? 0.0f : g * ((v[k] * w[k] * denom - nom * w[k]) * inv2);
-        gv[k] = dead ? 0.0f : g * b[k] * w[k] * inv;
-        gw[k] = dead ? 0.0f : g * (b[k] * v[k] * denom - nom * b[k]) * inv2;  // g * inv2 overflows where w is around 1e-18
+        gb[k] = g * ((v[k] * w[k] * denom - nom * w[k]) * inv2);
+        gv[k] = g * b[k] * w[k] * inv;
+        gw[k] = g * (b[k] * v[k] * denom - nom * b[k]) * inv2;  // g * inv2 overflows where w is around 1e-18
     }
+    return denom * denom < kEffZero;
 }
 
 // process_backward (render.cu:455-538) is evaluated in two parts.  The part that
@@ -147,15 +174,16 @@ __device__ __forceinline__ void interp_backward_scalar(real g, const real b[3], 
 struct FragSeed {
     real d_do;    // derivative w.r.t. the interpolated opacity (:502)
     real gc[3];   // derivative w.r.t. the interpolated colour (:510)
-    real dd_dz;   // derivative w.r.t. the interpolated view depth (:517)
+    real dd_dz;   // derivative w.r.t. the interpolated view depth (:517); with kDepth
 };
 
-// The fragment itself: interpolated opacity, colour and view depth (no state involved).
+// The fragment itself: interpolated opacity, colour and, with kDepth, view depth (no state involved).
 struct FragValue {
     real o, color[3], z;
 };
 
-__device__ __forceinline__ FragValue fragment_value(const BackRecord &r, real b0, real b1, real b2) {
+template <bool kDepth>
+__device__ __forceinline__ FragValue fragment_value(const BackRecord<kDepth> &r, real b0, real b1, real b2) {
     const real w[3] = {r.w[0], r.w[1], r.w[2]};
     FragValue v;
     // The opacity is recomputed exactly as the forward pass computed it: 1 - o can be small, and the
@@ -166,16 +194,17 @@ __device__ __forceinline__ FragValue fragment_value(const BackRecord &r, real b0
 #pragma unroll
     for (int k = 0; k < 3; k++)
         v.color[k] = (b0 * r.col[k] * w[0] + b1 * r.col[3 + k] * w[1] + b2 * r.col[6 + k] * w[2]) * inv_denom;
-    v.z = interp_1(b0, b1, b2, r.iw[0], r.iw[1], r.iw[2]);
+    if constexpr (kDepth) v.z = interp_1(b0, b1, b2, r.iw[0], r.iw[1], r.iw[2]);
     return v;
 }
 
 // The step from one fragment of a pixel to the next one in reverse blend order (render.cu:487-517).
+template <bool kDepth>
 __device__ __forceinline__ FragSeed fragment_chain_step(BackState &st, const FragValue &v) {
-    const real o = v.o, z = v.z;
+    const real o = v.o;
     const real color[3] = {v.color[0], v.color[1], v.color[2]};
     const real om = 1.0f - o;
-    const real inv_om = reciprocal(om);  // the reference divides six derivative terms by om
+    const real inv_om = reciprocal_of_normal(om);  // in [1e-4, 1] or NaN; the reference divides six derivative terms by om
     const real g[3] = {st.g0, st.g1, st.g2};
     real s[3] = {st.s0, st.s1, st.s2};
     real t3[3];
@@ -186,33 +215,47 @@ __device__ __forceinline__ FragSeed fragment_chain_step(BackState &st, const Fra
 #pragma unroll
     for (int k = 0; k < 3; k++) s[k] += color[k] * o * st.alpha;                       // :493
     st.s0 = s[0]; st.s1 = s[1]; st.s2 = s[2];
-    const real ddw_do = st.alpha - st.oa * inv_om;                                    // :494
-    const real dud_do = st.alpha * z - st.zoa * inv_om;                               // :495
-    st.oa = st.oa + o * st.alpha;                                                      // :496
-    st.zoa = st.zoa + z * o * st.alpha;                                                // :497
-    real dd_do = (dud_do - st.final_depth * ddw_do) * st.inv_final_weight * st.gd;    // :499
-    if (st.final_weight < kEffZero) dd_do = 0.0f;
     FragSeed f;
-    f.d_do = drgb_do + dd_do;
+    f.d_do = drgb_do;
     const real ao = st.alpha * o;
     f.gc[0] = ao * g[0]; f.gc[1] = ao * g[1]; f.gc[2] = ao * g[2];                     // :510
-    f.dd_dz = ao * st.gd * st.inv_final_weight;                                        // :517
-    if (st.final_weight < kEffZero) f.dd_dz = 0.0f;
+    if constexpr (kDepth) {
+        const real z = v.z;
+        const real ddw_do = st.alpha - st.oa * inv_om;                                    // :494
+        const real dud_do = st.alpha * z - st.zoa * inv_om;                               // :495
+        st.oa = st.oa + o * st.alpha;                                                      // :496
+        st.zoa = st.zoa + z * o * st.alpha;                                                // :497
+        real dd_do = (dud_do - st.final_depth * ddw_do) * st.inv_final_weight * st.gd;    // :499
+        if (st.final_weight < kEffZero) dd_do = 0.0f;
+        f.d_do = drgb_do + dd_do;
+        f.dd_dz = ao * st.gd * st.inv_final_weight;                                        // :517
+        if (st.final_weight < kEffZero) f.dd_dz = 0.0f;
+    }
     return f;
 }
 
-__device__ __forceinline__ FragSeed fragment_state_step(BackState &st, const BackRecord &r, real b0, real b1, real b2) {
-    return fragment_chain_step(st, fragment_value(r, b0, b1, b2));
+template <bool kDepth>
+__device__ __forceinline__ FragSeed fragment_state_step(BackState &st, const BackRecord<kDepth> &r, real b0, real b1, real b2) {
+    return fragment_chain_step<kDepth>(st, fragment_value(r, b0, b1, b2));
+}
+
+// Without a gradient of the depth: whether the terms by way of it are zeros.  They are where no product in them can be too large
+// for a float.  The coordinates b are positive, so with w and denom = b0 w0 + b1 w1 + b2 w2 in [1e-6, 1e6] the sum of the b
+// is in [1e-12, 1e12], and every factor that a zero meets below 1e31.  (A NaN in w or b makes NaNs of all terms without these.)
+__device__ __forceinline__ bool depth_is_ordinary(const real w[3], real denom) {
+    const real low = 1e-6f, high = 1e6f;
+    return min_number(w[0], w[1], w[2]) > low && max_number(w[0], w[1], w[2]) < high && denom > low && denom < high;
 }
 
 // The order-free part: the 21 gradient terms of one fragment.
-__device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackRecord &r, real b0, real b1, real b2, real px,
+template <bool kDepth>
+__device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackRecord<kDepth> &r, real b0, real b1, real b2, real px,
                                                real py, real out[kTerms]) {
     const real b[3] = {b0, b1, b2};
     const real w[3] = {r.w[0], r.w[1], r.w[2]};
     const real ones[3] = {1.0f, 1.0f, 1.0f};
     real gb_o[3], gv_o[3], gw_o[3];
-    interp_backward_scalar(f.d_do, b, r.op, w, gb_o, gv_o, gw_o);
+    const bool dead = interp_backward_scalar(f.d_do, b, r.op, w, gb_o, gv_o, gw_o);
 
     // vector interpolate3_backward for the colour (util.h:319-355)
     const real *gc = f.gc;
@@ -222,7 +265,6 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
 #pragma unroll
         for (int k = 0; k < 3; k++) nom[k] = (b[0] * w[0] * r.col[k] + b[1] * w[1] * r.col[3 + k]) + b[2] * w[2] * r.col[6 + k];
         const real denom = b[0] * w[0] + b[1] * w[1] + b[2] * w[2];
-        const bool dead = denom * denom < kEffZero;  // util.h:326: all zero (selections, not a branch: see above)
         const real inv = reciprocal(denom);
         const real inv2 = inv * inv;
 #pragma unroll
@@ -234,18 +276,45 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
                 dfb[k] = w[v] * (a * denom - nom[k]) * inv2;
                 dfw[k] = b[v] * a * denom - nom[k] * b[v];
             }
-            gb_c[v] = dead ? 0.0f : (gc[0] * dfb[0] + gc[1] * dfb[1]) + gc[2] * dfb[2];
-            gw_c[v] = dead ? 0.0f : ((gc[0] * dfw[0] + gc[1] * dfw[1]) + gc[2] * dfw[2]) * inv2;
-            scale[v] = dead ? 0.0f : b[v] * w[v] * inv;
+            gb_c[v] = (gc[0] * dfb[0] + gc[1] * dfb[1]) + gc[2] * dfb[2];
+            gw_c[v] = ((gc[0] * dfw[0] + gc[1] * dfw[1]) + gc[2] * dfw[2]) * inv2;
+            scale[v] = b[v] * w[v] * inv;
         }
     }
 
     real gb_z[3], gv_z[3], gw_z[3];
-    interp_backward_scalar(f.dd_dz, b, r.iw, ones, gb_z, gv_z, gw_z);
-
-    real gbary[3];
+    bool dead_z = false;
+    if constexpr (kDepth) dead_z = interp_backward_scalar(f.dd_dz, b, r.iw, ones, gb_z, gv_z, gw_z);
+    if (any_lane(dead || dead_z)) {
 #pragma unroll
-    for (int k = 0; k < 3; k++) gbary[k] = gb_o[k] + gb_c[k] + gb_z[k];  // :527
+        for (int k = 0; k < 3; k++) {
+            if (dead) gb_o[k] = gv_o[k] = gw_o[k] = gb_c[k] = gw_c[k] = scale[k] = 0.0f;  // util.h:303, :326: the same denominator
+            if (dead_z) gb_z[k] = gv_z[k] = gw_z[k] = 0.0f;
+        }
+    }
+    real gbary[3], dw[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        gbary[k] = gb_o[k] + gb_c[k];  // :527
+        dw[k] = gw_o[k] + gw_c[k];     // :530
+    }
+    const auto add_depth = [&](int k, real iw2) {
+        gbary[k] += gb_z[k];
+        dw[k] = dw[k] + gw_z[k] + -gv_z[k] * iw2;  // :523-525
+    };
+    if constexpr (kDepth) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) add_depth(k, r.iw2[k]);
+    } else if (any_lane(!depth_is_ordinary(r.w, (b[0] * w[0] + b[1] * w[1]) + b[2] * w[2]))) {
+        VertexDepths<true> depths;
+        vertex_depths(r.w, depths);
+        dead_z = interp_backward_scalar(0.0f, b, depths.iw, ones, gb_z, gv_z, gw_z);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if (dead_z) gb_z[k] = gv_z[k] = gw_z[k] = 0.0f;
+            add_depth(k, depths.iw2[k]);
+        }
+    }
 
     // util.h:405-455 barycentric_backward (vertex part)
     const real ax = r.xy[0], ay = r.xy[1], bx = r.xy[2], by = r.xy[3], cx = r.xy[4], cy = r.xy[5];
@@ -266,7 +335,6 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
         const real l1 = ((cx - px) * (ay - py) - (cy - py) * (ax - px)) * inv_T;
         const real l2 = ((ax - px) * (by - py) - (ay - py) * (bx - px)) * inv_T;
         const real d = ax * (by - cy) + bx * (-ay + cy) + cx * (ay - by);
-        const bool flat = abs_real(d) < kEffZero;  // util.h:421: zero (selection, not a branch: see above)
         {
             const real inv_d = reciprocal(d);  // of the sum, not of its 18 numerators: 12 multiplications and as many roundings less
             real J[3][2][3];
@@ -292,16 +360,20 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
             for (int v = 0; v < 3; v++)
 #pragma unroll
                 for (int c = 0; c < 2; c++)
-                    dxy[v][c] = flat ? 0.0f : (gbary[0] * J[v][c][0] + gbary[1] * J[v][c][1] + gbary[2] * J[v][c][2]) * inv_d;
+                    dxy[v][c] = (gbary[0] * J[v][c][0] + gbary[1] * J[v][c][1] + gbary[2] * J[v][c][2]) * inv_d;
+            const bool flat = abs_real(d) < kEffZero;  // util.h:421: zero
+            if (any_lane(flat)) {
+#pragma unroll
+                for (int v = 0; v < 3; v++)
+                    if (flat) dxy[v][0] = dxy[v][1] = 0.0f;
+            }
         }
     }
 #pragma unroll
     for (int v = 0; v < 3; v++) {
-        const real dd_dw = -gv_z[v] * r.iw2[v];        // :523-525
-        const real dw = gw_o[v] + gw_c[v] + gw_z[v];   // :530
         out[7 * v + 0] = dxy[v][0];
         out[7 * v + 1] = dxy[v][1];
-        out[7 * v + 2] = dw + dd_dw;
+        out[7 * v + 2] = dw[v];
         out[7 * v + 3] = gc[0] * scale[v];
         out[7 * v + 4] = gc[1] * scale[v];
         out[7 * v + 5] = gc[2] * scale[v];
@@ -310,7 +382,7 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
 }
 
 // One fragment start to finish (used where every pixel has its own order).
-__device__ __forceinline__ void fragment_backward(BackState &st, const BackRecord &r, real b0, real b1, real b2, real px,
+__device__ __forceinline__ void fragment_backward(BackState &st, const BackRecord<true> &r, real b0, real b1, real b2, real px,
                                                   real py, real out[kTerms]) {
     const FragSeed f = fragment_state_step(st, r, b0, b1, b2);
     fragment_terms(f, r, b0, b1, b2, px, py, out);
@@ -337,6 +409,7 @@ __device__ __forceinline__ real *term_address(const BackwardArgs &g, int vertex_
     return g.grad_opacities + at;
 }
 
+template <bool kDepth>
 __device__ __forceinline__ BackState load_back_state(const BackwardArgs &g, const PixelCoord &p) {
     BackState st;
     const real4 gi = g.grad_image[p.index];
@@ -349,6 +422,8 @@ __device__ __forceinline__ BackState load_back_state(const BackwardArgs &g, cons
     st.final_weight = g.weights[p.index];
     st.inv_final_weight = 1.0f / st.final_weight;
     st.final_depth = g.depthmap[p.index];
+    // without a gradient of the depth its part of d_do is 0 times these, and g3 is a factor of d_do only
+    if (!kDepth && !(st.final_weight < kEffZero)) st.g3 += st.final_depth * 0.0f + st.inv_final_weight * 0.0f;
     return st;
 }
 
@@ -475,9 +550,9 @@ __device__ __forceinline__ int wave_max_i32(int v) {
 //      terms of its hit and writes them to a term matrix; three groups of 21 lanes
 //      add up the runs of equal entry and issue one global floating-point atomic
 //      per run and term.
-template <int kLayout>
+template <int kLayout, bool kDepth>
 __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(RasterArgs a, BackwardArgs g) {
-    __shared__ BackRecord s_rec[kBackBatch];
+    __shared__ BackRecord<kDepth> s_rec[kBackBatch];
     __shared__ uint64_t s_ballot[kMaxWaves][kBackBatch];
     __shared__ uint32_t s_base[kMaxWaves][kBackBatch];
     __shared__ int s_tag[kMaxWaves][kWaveSlots];  // (entry | source lane << 8) of a slot
@@ -507,7 +582,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
     const uint64_t *const masks = saved_masks ? g.hit_masks + hit_mask_head_words() : nullptr;
     const int my_last = p.valid ? g.last[p.index] : 0;  // entries [0, my_last) of the list may hold my fragments
     BackState st;
-    if (p.valid) st = load_back_state(g, p);
+    if (p.valid) st = load_back_state<kDepth>(g, p);
     int tile_last = saved_masks ? (int)(int64_t)g.hit_masks[hit_mask_head_index(tile)] : -1;
     if (tile_last < 0) {  // the same for the workgroup: no masks, or its pixels were rendered by several workgroups
         if (tid == 0) s_last = 0;
@@ -562,7 +637,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
                 while (todo) {
                     const int bit = __builtin_ctzll(todo);
                     todo &= todo - 1;
-                    const BackRecord &r = s_rec[64 * wd + bit];
+                    const BackRecord<kDepth> &r = s_rec[64 * wd + bit];
                     real b0, b1, b2;
                     bary_apply(r.m, p.px, p.py, b0, b1, b2);
                     const bool hit = bary_inside(b0, b1, b2) && 64 * wd + bit < mine;
@@ -617,7 +692,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
 #pragma unroll
                     for (int wd = 0; wd < kBackWords; wd++)
                         if ((e >> 6) == wd) m[wd] &= ~(1ull << (e & 63));
-                    const BackRecord &r = s_rec[e];
+                    const BackRecord<kDepth> &r = s_rec[e];
                     real b0, b1, b2;
                     bary_apply(r.m, p.px, p.py, b0, b1, b2);
                     const FragSeed f = fragment_state_step(st, r, b0, b1, b2);
@@ -627,7 +702,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
                     terms[1 * kTermStride + slot] = f.gc[0];
                     terms[2 * kTermStride + slot] = f.gc[1];
                     terms[3 * kTermStride + slot] = f.gc[2];
-                    terms[4 * kTermStride + slot] = f.dd_dz;
+                    if constexpr (kDepth) terms[4 * kTermStride + slot] = f.dd_dz;
                     tags[slot] = e | (lane << 8);
                 }
             }
@@ -645,8 +720,8 @@ __global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(Raste
                 f.gc[0] = terms[1 * kTermStride + lane];
                 f.gc[1] = terms[2 * kTermStride + lane];
                 f.gc[2] = terms[3 * kTermStride + lane];
-                f.dd_dz = terms[4 * kTermStride + lane];
-                const BackRecord &r = s_rec[tag];
+                if constexpr (kDepth) f.dd_dz = terms[4 * kTermStride + lane];
+                const BackRecord<kDepth> &r = s_rec[tag];
                 real b0, b1, b2;
                 bary_apply(r.m, px, py, b0, b1, b2);
                 real term[kTerms];
@@ -724,7 +799,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
     real bound_depth = 0.0f;
     int bound_j = 0;
     if (p.valid) {
-        st = load_back_state(g, p);
+        st = load_back_state<true>(g, p);
         remaining = min(g.ends[p.index], a.max_layers);  // render.cu:642
         bound_depth = g.last_depth[p.index];
         bound_j = start + g.last[p.index];  // one past the last blended entry
@@ -762,7 +837,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
         }
         if (want) {
             for (int i = 0; i < found; i++) {
-                BackRecord r;
+                BackRecord<true> r;
                 gather_back(a, tk.j(i), r);
                 real b0, b1, b2;
                 bary_apply(r.m, p.px, p.py, b0, b1, b2);
@@ -823,38 +898,44 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
 //      columns (ballot matching, groups in order of their lowest slot) of a term
 //      matrix in LDS, three groups of 21 lanes add up the runs of equal entry and issue
 //      one global floating-point atomic per run and term.
-template <int kLayout>
-__global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
-    __shared__ real s_term[kMaxWaves][kTerms * kTermStride];
-    __shared__ int s_rel[kMaxWaves][kWave];         // list position of a slot's fragment, from the tile's start
-    __shared__ int s_tag[kMaxWaves][kWave];         // the same by column of the term matrix
-    __shared__ int s_vertex[kMaxWaves][3 * kWave];  // the three vertex ids of a column's entry
-    __shared__ uint8_t s_src[kMaxWaves][kWave];     // the pixel (lane) of a slot
+// What a wave keeps in LDS.  A workgroup takes it for the waves it has (taken for four always, frames in tiles of 8 x 8, a wave each,
+// had five workgroups a CU: 33 000 triangles 229 us, so 116).
+struct SavedWave {
+    real term[kTerms * kTermStride];
+    int rel[kWave];         // list position of a slot's fragment, from the tile's start
+    int tag[kWave];         // the same by column of the term matrix
+    int vertex[3 * kWave];  // the three vertex ids of a column's entry
+    uint8_t src[kWave];     // the pixel (lane) of a slot
+};
+template <int kLayout, bool kDepth>
+__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
+    extern __shared__ __align__(16) unsigned char s_dyn[];
     if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
+    SavedWave &mem = reinterpret_cast<SavedWave *>(s_dyn)[tid / kWave];
     const TileId tile_id = g.deep ? tile_of_workgroup<kTileBandBackward, kSixteenths>() : tile_of_workgroup<kTileBandBackward, kEighths>();
+    const int slot_of_tile = blockIdx.z * blockDim.x + tid;
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
-    const PixelCoord p = pixel_of_thread(a, tile_id);
+    const PixelCoord p = pixel_of_slot(a, tile_id.x, tile_id.y, slot_of_tile);
     const int rel_bits = 32 - __builtin_clz(max(end - start - 1, 1));  // bits that tell two list positions apart
-    real *terms = s_term[wave];
-    int *tags = s_tag[wave];
-    int *vertices = s_vertex[wave];
+    real *terms = mem.term;
+    int *tags = mem.tag;
+    int *vertices = mem.vertex;
     const TermLane tl = term_lane<kLayout>(g, lane);
 
     BackState st;
     int n = 0;
     if (p.valid) {
-        st = load_back_state(g, p);
+        st = load_back_state<kDepth>(g, p);
         // render.cu:642; fewer than were blended only where a NaN depth had the list blended more than once
         n = min(g.ends[p.index], min(a.max_layers, order_rows(g.order, a, end - start)));
     }
     const int64_t plane = order_stride(g.order, a);
     const bool long_list = end - start > kShortList;  // then the positions' high halves were saved as well
     // The list positions of my steps, one after the other: step s is layer n - 1 - s, a plane further down each time.
-    const uint16_t *next_layer = g.order.low + ((int64_t)(n - 1) * plane + order_first(g.order, p, start, blockIdx.z * blockDim.x + tid));
+    const uint16_t *next_layer = g.order.low + ((int64_t)(n - 1) * plane + order_first(g.order, p, start, slot_of_tile));
     const int64_t high_halves = g.order.high;
     int steps_read = 0;
     auto next_position = [&]() {
@@ -913,8 +994,8 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
         if (lane < first_lane) base += offered;
         const int granted = max(0, min(mine_count, kWave - base));
         const int n_slots = min(kWave, offered);
-        int *rels = s_rel[wave];
-        uint8_t *srcs = s_src[wave];
+        int *rels = mem.rel;
+        uint8_t *srcs = mem.src;
         if (granted > 0) { rels[base] = ahead0; srcs[base] = (uint8_t)lane; }
         if (granted > 1) { rels[base + 1] = ahead1; srcs[base + 1] = (uint8_t)lane; }
         if (granted > 2) { rels[base + 2] = ahead2; srcs[base + 2] = (uint8_t)lane; }
@@ -932,7 +1013,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
         // 2. lane = slot: the record, and the fragment's own values
         const int src = (lane < n_slots) ? srcs[lane] : lane;
         const real px = __shfl(p.px, src, kWave), py = __shfl(p.py, src, kWave);
-        BackRecord r;
+        BackRecord<kDepth> r;
         real b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
         int rel = 0;
         if (lane < n_slots) {
@@ -944,7 +1025,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
             terms[1 * kTermStride + lane] = v.color[0];
             terms[2 * kTermStride + lane] = v.color[1];
             terms[3 * kTermStride + lane] = v.color[2];
-            terms[4 * kTermStride + lane] = v.z;
+            if constexpr (kDepth) terms[4 * kTermStride + lane] = v.z;
         }
         wave_lds_sync();
 
@@ -960,13 +1041,13 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
                 v.color[0] = terms[1 * kTermStride + c];
                 v.color[1] = terms[2 * kTermStride + c];
                 v.color[2] = terms[3 * kTermStride + c];
-                v.z = terms[4 * kTermStride + c];
-                const FragSeed f = fragment_chain_step(st, v);
+                if constexpr (kDepth) v.z = terms[4 * kTermStride + c];
+                const FragSeed f = fragment_chain_step<kDepth>(st, v);
                 terms[0 * kTermStride + c] = f.d_do;
                 terms[1 * kTermStride + c] = f.gc[0];
                 terms[2 * kTermStride + c] = f.gc[1];
                 terms[3 * kTermStride + c] = f.gc[2];
-                terms[4 * kTermStride + c] = f.dd_dz;
+                if constexpr (kDepth) terms[4 * kTermStride + c] = f.dd_dz;
             }
         }
         wave_lds_sync();
@@ -980,7 +1061,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_saved_order_kernel(Rast
             f.gc[0] = terms[1 * kTermStride + lane];
             f.gc[1] = terms[2 * kTermStride + lane];
             f.gc[2] = terms[3 * kTermStride + lane];
-            f.dd_dz = terms[4 * kTermStride + lane];
+            if constexpr (kDepth) f.dd_dz = terms[4 * kTermStride + lane];
         }
         // By the bits that tell positions of the round's range apart: the few positions outside it (a second step behind a
         // first one, by depth, may come later in the list) can be taken together with others, and then make more runs, not
@@ -1070,20 +1151,23 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
     const int layout = (vertex_stride == 4 && color_stride == 3 && opacity_stride == 1)   ? kGradDense
                        : (vertex_stride == 8 && color_stride == 8 && opacity_stride == 8) ? kGradBlock8
                                                                                           : kGradStrided;
-#define TG_LAUNCH_BACKWARD(kernel, grid, block, lds_bytes)                                                  \
-    do {                                                                                                    \
-        if (layout == kGradDense) TG_LAUNCH_AS(#kernel, kernel<kGradDense>, grid, block, lds_bytes, s, a, g);   \
-        else if (layout == kGradBlock8) TG_LAUNCH_AS(#kernel, kernel<kGradBlock8>, grid, block, lds_bytes, s, a, g); \
-        else TG_LAUNCH_AS(#kernel, kernel<kGradStrided>, grid, block, lds_bytes, s, a, g);                      \
+#define TG_LAUNCH_BACKWARD(kernel, grid, block, lds_bytes, ...)                                                                              \
+    do {                                                                                                                                     \
+        if (layout == kGradDense) TG_LAUNCH_AS(#kernel, (kernel<kGradDense __VA_OPT__(,) __VA_ARGS__>), grid, block, lds_bytes, s, a, g);          \
+        else if (layout == kGradBlock8) TG_LAUNCH_AS(#kernel, (kernel<kGradBlock8 __VA_OPT__(,) __VA_ARGS__>), grid, block, lds_bytes, s, a, g);   \
+        else TG_LAUNCH_AS(#kernel, (kernel<kGradStrided __VA_OPT__(,) __VA_ARGS__>), grid, block, lds_bytes, s, a, g);                             \
     } while (0)
     if (!per_pixel_sort) {
         const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, kTileThreads);
-        TG_LAUNCH_BACKWARD(backward_tile_order_kernel, tl.grid, dim3(tl.threads), 0);
+        if (grad_depthmap) TG_LAUNCH_BACKWARD(backward_tile_order_kernel, tl.grid, dim3(tl.threads), 0, true);
+        else TG_LAUNCH_BACKWARD(backward_tile_order_kernel, tl.grid, dim3(tl.threads), 0, false);
         return check_launch("backward_tile_order_kernel");
     }
     if (order.low) {
         const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, kTileThreads);
-        TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), 0);
+        const size_t lds = sizeof(SavedWave) * (tl.threads / kWave);
+        if (grad_depthmap) TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), lds, true);
+        else TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), lds, false);
         return check_launch("backward_saved_order_kernel");
     }
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, pixel_order_threads(kTileThreads));

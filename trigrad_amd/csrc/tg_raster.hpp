@@ -465,6 +465,8 @@ __device__ __forceinline__ uint32_t small_entry(const RasterArgs &a, real extent
 // bary_inside in two operations: a minimum passes NaNs by, as the three comparisons there do.
 __device__ __forceinline__ float min_number(float a, float b, float c) { return __builtin_fminf(__builtin_fminf(a, b), c); }
 __device__ __forceinline__ double min_number(double a, double b, double c) { return __builtin_fmin(__builtin_fmin(a, b), c); }
+__device__ __forceinline__ float max_number(float a, float b, float c) { return __builtin_fmaxf(__builtin_fmaxf(a, b), c); }
+__device__ __forceinline__ double max_number(double a, double b, double c) { return __builtin_fmax(__builtin_fmax(a, b), c); }
 __device__ __forceinline__ bool all_inside(real b0, real b1, real b2) { return !(min_number(b0, b1, b2) < kEffZero); }
 
 template <int kCtrl>
