@@ -1515,3 +1515,25 @@ def test_gradients_where_the_depth_map_has_none(w, mode, cuda):
         np.testing.assert_array_equal(np.isnan(got), np.isnan(want), err_msg=label)
         largest = float(np.abs(want[finite]).max()) if finite.any() else 0.0
         assert_close(f"{w}/{mode}: {label}", np.where(finite, got, 0), np.where(finite, want, 0), 1e-4, 300 * 2.0 ** -24 * largest + 1e-30)
+
+
+@pytest.mark.parametrize("width,height,tw,th", [(513, 512, 16, 16), (512, 512, 16, 16), (478, 480, 16, 16), (500, 452, 16, 16), (448, 512, 16, 16),
+                                                (509, 511, 32, 8), (505, 497, 8, 8), (411, 403, 12, 20)])
+@pytest.mark.parametrize("layers", [32, 40])
+def test_gradients_by_waves_alone_and_in_fours(width, height, tw, th, layers, cuda, oracle):
+    """The saved-order backward kernel runs a wave to a workgroup, or four where the frame's waves (ceil(tile / 64) a tile) are 3585 to
+    4096: numbers of waves on both sides of either edge, tiles of one, two and four waves, numbers of tiles that are no multiple of eight."""
+    import torch
+    import scenes as S
+    import trigrad_amd
+    scene = S.random_soup(1500, width, height, seed=width + layers, sigma_px=14.0, opacity=(0.1, 0.6), varying_w=True)
+    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256, True, layers)
+    gi, gd = _grad_inputs(scene, 4, False)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
+                                    tw, th, True, layers, literal=False, magnitudes=True)
+    d = to_device(scene, cuda)
+    leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+    image, _ = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, tw, th, max_layers=layers)
+    out = torch.autograd.grad(image, leaves, torch.from_numpy(gi).to(cuda))
+    for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+        assert_gradients_close(f"{width}x{height}, tiles of {tw}x{th}, {layers} layers: {label}", g.cpu().numpy(), w, mag)

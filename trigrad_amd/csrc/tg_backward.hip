@@ -898,6 +898,9 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
 //      columns (ballot matching, groups in order of their lowest slot) of a term
 //      matrix in LDS, three groups of 21 lanes add up the runs of equal entry and issue
 //      one global floating-point atomic per run and term.
+// The waves of a tile share nothing, so a workgroup is one wave: its place is free for another tile's when it is done, where
+// workgroups of four wait for the longest of them (saved_order_waves).  In fours and so, us: 10^6 triangles 1057, 1013, 10^5 83.5, 76,
+// 20 000 with a heavy tail on 1920 x 1080 61, 55, a mesh of 1.3 million 185, 180.
 // What a wave keeps in LDS.  A workgroup takes it for the waves it has (taken for four always, frames in tiles of 8 x 8, a wave each,
 // had five workgroups a CU: 33 000 triangles 229 us, so 116).
 struct SavedWave {
@@ -914,8 +917,10 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void backw
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     SavedWave &mem = reinterpret_cast<SavedWave *>(s_dyn)[tid / kWave];
-    const TileId tile_id = g.deep ? tile_of_workgroup<kTileBandBackward, kSixteenths>() : tile_of_workgroup<kTileBandBackward, kEighths>();
-    const int slot_of_tile = blockIdx.z * blockDim.x + tid;
+    const TilePart group = part_of_workgroup();
+    const TileId tile_id = g.deep ? tile_in_turn<kTileBandBackward, kSixteenths>(group.linear, gridDim.x, gridDim.y)
+                                  : tile_in_turn<kTileBandBackward, kEighths>(group.linear, gridDim.x, gridDim.y);
+    const int slot_of_tile = group.part * blockDim.x + tid;
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_slot(a, tile_id.x, tile_id.y, slot_of_tile);
@@ -1117,6 +1122,17 @@ size_t backward_pixel_order_lds_bytes(int n_threads) { return pixel_order_lds_by
 
 using namespace tg;
 
+// Waves of a workgroup of the saved-order kernel.  One, but for a frame whose waves fill the chip once, four for each of its 1024
+// SIMDs (3584 to 4096; 512 x 512 pixels): single waves go five to one SIMD and three to the next, those of a workgroup of four one to
+// each.  200 000 large triangles on 512 x 512: 248 us singly, 231 in fours, 20 000 without a limit on the layers 560 and 551; on
+// 480 x 480 239, 231 and 576, 596.  With fewer waves there is room for all (448 x 448: 222, 228), with more the next one takes the
+// place (528 x 528: 259, 262 and 571, 604).
+static int saved_order_waves(int width, int height, int tile_w, int tile_h) {
+    constexpr int64_t kChipWaves = 4 * 1024;
+    const int64_t waves = (int64_t)ceil_div(width, tile_w) * ceil_div(height, tile_h) * ceil_div(tile_w * tile_h, kWave);
+    return waves > kChipWaves / 8 * 7 && waves <= kChipWaves ? kMaxWaves : 1;
+}
+
 int tg::render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices,
                                   const int32_t *indices, const real *colors, const real *opacities,
                                   const int32_t *sorted_ids, const int32_t *offsets, const real *bary, const real *image,
@@ -1164,7 +1180,7 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
         return check_launch("backward_tile_order_kernel");
     }
     if (order.low) {
-        const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, kTileThreads);
+        const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, saved_order_waves(width, height, tile_w, tile_h) * kWave);
         const size_t lds = sizeof(SavedWave) * (tl.threads / kWave);
         if (grad_depthmap) TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), lds, true);
         else TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), lds, false);

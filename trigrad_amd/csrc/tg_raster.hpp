@@ -109,9 +109,8 @@ constexpr int kChunkForward = TG_XCD_CHUNK_FORWARD;
 constexpr int kManyLayers = 16, kDeepLists = 96;
 struct TileId { int x, y, index; };
 template <int kTileBand, int kChunk>
-__device__ __forceinline__ TileId tile_of_workgroup(int skipped_rows = 0) {  // rows of workgroups in front that are not for tiles
-    const int tiles_x = (int)gridDim.x, tiles_y = (int)gridDim.y - skipped_rows, n = tiles_x * tiles_y;
-    const int linear = (int)((blockIdx.y - skipped_rows) * gridDim.x + blockIdx.x);
+__device__ __forceinline__ TileId tile_in_turn(int linear, int tiles_x, int tiles_y) {
+    const int n = tiles_x * tiles_y;
     TileId t;
 #if TG_XCD_TILES
     const int xcd = linear % kXcds, turn = linear / kXcds;
@@ -140,6 +139,24 @@ __device__ __forceinline__ TileId tile_of_workgroup(int skipped_rows = 0) {  // 
 #endif
     t.index = t.y * tiles_x + t.x;
     return t;
+}
+template <int kTileBand, int kChunk>
+__device__ __forceinline__ TileId tile_of_workgroup(int skipped_rows = 0) {  // rows of workgroups in front that are not for tiles
+    return tile_in_turn<kTileBand, kChunk>((int)((blockIdx.y - skipped_rows) * gridDim.x + blockIdx.x), (int)gridDim.x, (int)gridDim.y - skipped_rows);
+}
+// A launch of gridDim.z workgroups a tile, of which those of one tile follow each other on its XCD: the place of the calling workgroup's
+// tile in the order above, and which of the tile's workgroups it is.
+struct TilePart { int linear, part; };
+__device__ __forceinline__ TilePart part_of_workgroup() {
+    const int tiles = (int)(gridDim.x * gridDim.y), parts = (int)gridDim.z;
+    const int group = (int)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
+    const int whole = tiles / kXcds * kXcds;  // the last tiles, fewer than eight, go as they come
+    if (group >= whole * parts) {
+        const int rest = group - whole * parts;
+        return {whole + rest % (tiles - whole), rest / (tiles - whole)};
+    }
+    const int turn = group / kXcds;
+    return {turn / parts * kXcds + group % kXcds, turn % parts};
 }
 __device__ __forceinline__ PixelCoord pixel_of_thread(const RasterArgs &a, const TileId &t) { return pixel_of_thread(a, t.x, t.y); }
 
