@@ -1537,3 +1537,28 @@ def test_gradients_by_waves_alone_and_in_fours(width, height, tw, th, layers, cu
     out = torch.autograd.grad(image, leaves, torch.from_numpy(gi).to(cuda))
     for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
         assert_gradients_close(f"{width}x{height}, tiles of {tw}x{th}, {layers} layers: {label}", g.cpu().numpy(), w, mag)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 300])
+@pytest.mark.parametrize("width,height,tw,th", [(16, 16, 16, 16), (21, 13, 16, 16), (40, 24, 8, 8), (50, 26, 24, 24), (9, 7, 3, 5)])
+def test_tile_order_gradients_around_blocks_of_a_list(width, height, tw, th, n, cuda, oracle):
+    """In tile order a wave walks its tile's list backwards in blocks of 64 entries and takes the (pixel, entry) hits of a block in
+    rounds of 64: lists around multiples of 64, every pixel with one fragment of a block or with all of them, pixels that stop
+    inside a block, waves without a pixel; with the forward pass's hit masks and without."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    scene = S.random_soup(n, width, height, seed=n + width, sigma_px=9.0, opacity=(0.02, 0.4), varying_w=True)
+    mode = dict(per_pixel_sort=False, max_layers=n + 1)
+    d, want, got, ml = _forward_both(scene, tw, th, mode, cuda, oracle)
+    _check_forward(f"{n} in {width}x{height}", want, got, (th, tw))
+    gi, gd = _grad_inputs(scene, 6, False)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
+                                    tw, th, False, ml, literal=False, magnitudes=True)
+    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
+    for masks in (resume, resume[:4] + (None,)):
+        for depth_gradient in (None, torch.from_numpy(gd).to(cuda)):
+            out = _C.render_backward(torch.from_numpy(gi).to(cuda), depth_gradient, d["vertices"], d["indices"], d["colors"], d["opacities"],
+                                     sorted_ids, offsets, bary, image, depthmap, weights, ends, width, height, tw, th, 1 / 256, False, ml, resume=masks)
+            for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+                assert_gradients_close(f"{n} in {width}x{height}, tiles of {tw}x{th}: {label}", g.cpu().numpy(), w, mag)

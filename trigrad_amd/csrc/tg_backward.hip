@@ -1,4 +1,4 @@
-// tg_backward.hip -- backward of the tile compositor, one workgroup per tile.
+// tg_backward.hip -- backward of the tile compositor, a wave to 64 pixels of a tile.
 //
 // Fragments are visited in exact reverse blend order; the transmittance in front
 // of a fragment is reconstructed by dividing the running value by (1 - opacity),
@@ -11,8 +11,8 @@
 // entries, term) instead of 24 per (pixel, entry).
 //
 // per_pixel_sort = 0 (backward_tile_order_kernel): all pixels of a tile share
-//   the list order, so the tile's list is walked backwards in LDS-staged
-//   batches of 64 entries.
+//   the list order, so every wave walks its tile's list backwards in blocks
+//   of 64 entries.
 // per_pixel_sort = 1 (backward_saved_order_kernel): every
 //   pixel walks the blend order the forward pass saved for it, backwards.
 // per_pixel_sort = 1, no saved order (backward_pixel_order_kernel): the pixel
@@ -39,6 +39,7 @@ struct BackwardArgs {
     real *grad_opacities;
     int vertex_stride, color_stride, opacity_stride;  // scalars from one vertex to the next in the three arrays
     const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
+    int mask_parts, mask_threads; // of the saved hit masks: workgroups of a tile in the forward launch, and their threads
     bool deep;                    // many layers and long lists: which tiles an XCD takes (tile_of_workgroup)
 };
 
@@ -113,8 +114,7 @@ __device__ __forceinline__ void vertex_depths(const real w[3], VertexDepths<true
 }
 
 template <bool kDepth>
-__device__ __forceinline__ void gather_back(const RasterArgs &a, int j, BackRecord<kDepth> &r) {
-    const TriIds t = load_ids(a, j);
+__device__ __forceinline__ void gather_back(const RasterArgs &a, const TriIds &t, BackRecord<kDepth> &r) {
     const real *m = a.bary + 9 * (int64_t)t.tri;
     real4v va = *reinterpret_cast<const real4v *>(a.vertices + t.ia), vb = *reinterpret_cast<const real4v *>(a.vertices + t.ib),
            vc = *reinterpret_cast<const real4v *>(a.vertices + t.ic);
@@ -428,8 +428,7 @@ __device__ __forceinline__ BackState load_back_state(const BackwardArgs &g, cons
 }
 
 
-constexpr int kBackBatch = 64;    // list entries staged per batch
-constexpr int kBackWords = kBackBatch / kWave;  // words of a lane's hit mask per batch
+constexpr int kBackBatch = 64;    // list entries of a block, a word of a lane's hit mask
 constexpr int kWaveSlots = 64;    // hit slots per wave and round: one per lane of the order-free part
 constexpr int kTermStride = 65;   // row stride of the per-wave term matrix (odd: conflict-free columns)
 constexpr int kMaxWaves = kTileThreads / kWave;
@@ -529,211 +528,190 @@ __device__ __forceinline__ int wave_max_i32(int v) {
     return __builtin_amdgcn_readlane(v, kWave - 1);
 }
 
-// Tile-order backward.  LDS floating-point atomics cost about three cycles per lane on
-// gfx950 and direct global atomics collide on the shared vertices, so the
-// per-entry sums are formed with plain LDS stores and loads.  The kernel is bound by
-// latency (LDS round trips, dependent loads), so its LDS and register budgets are set
-// for four workgroups per CU: the records of 64 list entries are staged per batch by
-// the whole workgroup; after that every wave works on its own 64 pixels without
-// workgroup barriers:
-//   1. which entries cover which pixel: the lane's 64-bit mask the forward pass saved
-//      (or the inside tests again, same record for all lanes: LDS broadcast); the
-//      wave's ballot per entry is the transpose of the lanes' masks;
-//   2. the ballots become slot numbers: entries from the far end, lanes in
-//      order inside an entry, so every (pixel, entry) hit of the wave owns one
-//      slot, slots are grouped by entry, and a lane's own hits have increasing
-//      numbers in the order it must visit them (reverse blend order);
-//   3. ordered part, in rounds of 64 slots: every lane walks its own hits and
-//      advances the pixel's transmittance and running sums; each hit leaves
-//      five numbers in its slot;
-//   4. order-free part with every lane busy: lane = slot evaluates the 21 gradient
-//      terms of its hit and writes them to a term matrix; three groups of 21 lanes
-//      add up the runs of equal entry and issue one global floating-point atomic
+// The steps of a round that the two kernels below share.  A round is up to 64 slots, each a fragment of a pixel: what the
+// lanes of its slots and of its pixels hand each other lies in the slot's column of the wave's term matrix.
+template <bool kDepth>
+__device__ __forceinline__ void leave_value(real *terms, int slot, const FragValue &v) {
+    terms[0 * kTermStride + slot] = v.o;
+    terms[1 * kTermStride + slot] = v.color[0];
+    terms[2 * kTermStride + slot] = v.color[1];
+    terms[3 * kTermStride + slot] = v.color[2];
+    if constexpr (kDepth) terms[4 * kTermStride + slot] = v.z;
+}
+// lane = pixel: the ordered part over my slots of the round (increasing slot = the order I must visit them in), which replaces the
+// fragments' values by the numbers that their gradient terms are linear in.
+template <bool kDepth>
+__device__ __forceinline__ void walk_slots(real *terms, uint64_t mine, BackState &st) {
+    while (true) {
+        const bool active = mine != 0;
+        if (__builtin_amdgcn_ballot_w64(active) == 0) break;
+        if (active) {
+            const int c = __builtin_ctzll(mine);
+            mine &= mine - 1;
+            FragValue v;
+            v.o = terms[0 * kTermStride + c];
+            v.color[0] = terms[1 * kTermStride + c];
+            v.color[1] = terms[2 * kTermStride + c];
+            v.color[2] = terms[3 * kTermStride + c];
+            if constexpr (kDepth) v.z = terms[4 * kTermStride + c];
+            const FragSeed f = fragment_chain_step<kDepth>(st, v);
+            terms[0 * kTermStride + c] = f.d_do;
+            terms[1 * kTermStride + c] = f.gc[0];
+            terms[2 * kTermStride + c] = f.gc[1];
+            terms[3 * kTermStride + c] = f.gc[2];
+            if constexpr (kDepth) terms[4 * kTermStride + c] = f.dd_dz;
+        }
+    }
+}
+template <bool kDepth>
+__device__ __forceinline__ FragSeed seed_of_slot(const real *terms, int slot) {
+    FragSeed f;
+    f.d_do = terms[0 * kTermStride + slot];
+    f.gc[0] = terms[1 * kTermStride + slot];
+    f.gc[1] = terms[2 * kTermStride + slot];
+    f.gc[2] = terms[3 * kTermStride + slot];
+    if constexpr (kDepth) f.dd_dz = terms[4 * kTermStride + slot];
+    return f;
+}
+
+// Tile-order backward.  All pixels of a tile share the list order, so a wave walks its tile's list backwards, 64 entries at a
+// time, by itself:
+//   1. which entries cover which pixel: the lane's 64-bit mask the forward pass saved, asked for an entry block ahead (or the inside
+//      tests again); the wave's ballot per entry is the transpose of the lanes' masks;
+//   2. the ballots become slot numbers: entries from the far end, lanes in order inside an entry, so every
+//      (pixel, entry) hit of the wave owns one slot, slots are grouped by entry, and a lane's own hits have increasing numbers in
+//      the order it must visit them (reverse blend order);
+//   then, in rounds of 64 slots:
+//   3. lane = pixel: tells its slots whose they are;
+//   4. lane = slot: gathers the record of its fragment (the entry's triangle and vertex numbers are in LDS) and leaves the
+//      fragment's opacity and colour; lane = pixel: the ordered part over its slots; lane = slot: the 21 gradient terms into a
+//      term matrix, where three groups of 21 lanes add up the runs of equal entry and issue one global floating-point atomic
 //      per run and term.
+// Before, a workgroup of four waves staged every entry's record in LDS, between two barriers a block, each wave evaluated its
+// fragments where their pixels were (three or four turns a round with a third of the lanes busy), and 36 KB of LDS held the CU to
+// four of them.  Now a slot's record is gathered where the fragment is evaluated, by all lanes, entries that cover no pixel of the
+// wave are not read at all, and the waves share nothing: a workgroup is one of them (workgroup_waves), five a SIMD.  us, both with
+// dense gradient arrays: 10^6 triangles 603 -> 577, a mesh of 1.3 million 618 -> 440, 10^5 98 -> 82, 200 000 large ones 245 -> 224,
+// 33 000 in tiles of 8 x 8 203 -> 87.  Asking for a block's vertex numbers a block ahead too leaves seven more registers in scratch
+// memory (mesh 479); 32-bit byte offsets in the gather are ten operations less and change nothing.
+struct TileWave {                // what a wave keeps in LDS
+    real term[kTerms * kTermStride];
+    alignas(16) int id[kBackBatch][4];  // the entries' triangles and vertices
+    uint64_t ballot[kBackBatch]; // the lanes an entry covers
+    uint32_t base[kBackBatch];   // an entry's first slot
+    uint16_t tag[kWaveSlots];    // (entry | source lane << 8) of a slot
+};
 template <int kLayout, bool kDepth>
-__global__ __launch_bounds__(kTileThreads) void backward_tile_order_kernel(RasterArgs a, BackwardArgs g) {
-    __shared__ BackRecord<kDepth> s_rec[kBackBatch];
-    __shared__ uint64_t s_ballot[kMaxWaves][kBackBatch];
-    __shared__ uint32_t s_base[kMaxWaves][kBackBatch];
-    __shared__ int s_tag[kMaxWaves][kWaveSlots];  // (entry | source lane << 8) of a slot
-    __shared__ real s_term[kMaxWaves][kTerms * kTermStride];
-    __shared__ uint8_t s_touch[kBackBatch];
-    __shared__ WaveRect s_rects[kMaxTileWaves];
-    __shared__ int s_last;
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 5) void backward_tile_order_kernel(RasterArgs a, BackwardArgs g) {
+    extern __shared__ __align__(16) unsigned char s_dyn[];
     if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    const int n_waves = blockDim.x / kWave;
-    const TileId tile_id = tile_of_workgroup<kTileBandBackward, kEighths>();
+    int lane = tid & (kWave - 1);
+    TileWave &mem = reinterpret_cast<TileWave *>(s_dyn)[tid / kWave];
+    real *terms = mem.term;
+    const TilePart group = part_of_workgroup();
+    const TileId tile_id = tile_in_turn<kTileBandBackward, kEighths>(group.linear, gridDim.x, gridDim.y);
+    const int slot_of_tile = group.part * blockDim.x + tid;
     const int tile = tile_id.index;
     const int start = a.offsets[tile];
-    const PixelCoord p = pixel_of_thread(a, tile_id);
+    const PixelCoord p = pixel_of_slot(a, tile_id.x, tile_id.y, slot_of_tile);
     const TermLane tl = term_lane<kLayout>(g, lane);
-    uint64_t *ballots = s_ballot[wave];
-    uint32_t *bases = s_base[wave];
-    int *tags = s_tag[wave];
-    real *terms = s_term[wave];
 
-    // With the forward pass's masks comes the number of list entries this workgroup has to walk; else
-    // it is the largest `last` of its pixels.  The pixel's own loads are issued first either way: the
-    // barriers and the staging of the first batch cover their latency.
+    // With the forward pass's masks comes the number of list entries its workgroup has walked; else it is the largest `last` of my pixels.
     const bool saved_masks = g.hit_masks != nullptr;
-    const uint64_t *const masks = saved_masks ? g.hit_masks + hit_mask_head_words() : nullptr;
+    const int64_t mask_slots = (int64_t)g.mask_parts * g.mask_threads;
+    const int first_slot = __builtin_amdgcn_readfirstlane(slot_of_tile);  // of the wave
+    const uint64_t *const masks = g.hit_masks + (int64_t)gridDim.x * gridDim.y * g.mask_parts + first_slot;
     const int my_last = p.valid ? g.last[p.index] : 0;  // entries [0, my_last) of the list may hold my fragments
     BackState st;
     if (p.valid) st = load_back_state<kDepth>(g, p);
-    int tile_last = saved_masks ? (int)(int64_t)g.hit_masks[hit_mask_head_index(tile)] : -1;
-    if (tile_last < 0) {  // the same for the workgroup: no masks, or its pixels were rendered by several workgroups
-        if (tid == 0) s_last = 0;
-        if (!saved_masks) publish_wave_rect(p, s_rects);  // only the repeated inside tests cull by wave rectangle
-        __syncthreads();
-        if (my_last > 0) atomicMax(&s_last, my_last);
-        __syncthreads();
-        tile_last = s_last;
-    }
+    int list_last = saved_masks ? (int)(int64_t)g.hit_masks[(int64_t)tile * g.mask_parts + first_slot / g.mask_threads] : -1;
+    if (list_last < 0) list_last = wave_max_i32(my_last);  // no masks, or its pixels were rendered by several workgroups
+    list_last = __builtin_amdgcn_readfirstlane(list_last);
+    if (list_last == 0) return;
 
-    // Batches are aligned to multiples of kBackBatch from the start of the list (the last one may be
-    // short), so that a batch is whole words of the saved hit masks.
-    const int64_t mask_slots = (int64_t)gridDim.z * blockDim.x, mask_slot = (int64_t)blockIdx.z * blockDim.x + tid;
-    const int hi0 = (tile_last + kBackBatch - 1) / kBackBatch * kBackBatch;
-    for (int hi = hi0; hi > 0; hi -= kBackBatch) {
-        const int lo = hi - kBackBatch;
-        const int nb = min(hi, tile_last) - lo;
-        const int mine = my_last - lo;  // records [0, mine) of this batch are within my range
-        // my saved masks of the batch: asked for here, used after the staging
-        uint64_t m[kBackWords] = {};
-        if (saved_masks) {
-            const int64_t chunk = hit_mask_chunk(start, tile, lo);
+    // Blocks are aligned to multiples of kBackBatch from the start of the list (the last one may be short), so that a block is a whole
+    // word of the saved hit masks.  What a block needs is asked for while the one before it is worked on.
+    const int lo0 = (list_last - 1) / kBackBatch * kBackBatch;
+    const auto triangle_at = [&](int lo) { return a.sorted_ids[start + min(max(lo, 0) + lane, list_last - 1)]; };
+    const auto mask_at = [&](int lo) { return saved_masks && lo >= 0 && lo < my_last ? masks[hit_mask_chunk(start, tile, lo) * mask_slots + (uint32_t)lane] : 0ull; };
+    const auto ids_of = [&](int tri) { const int32_t *v = a.indices + 3 * (int64_t)tri; return TriIds{tri, v[0], v[1], v[2]}; };
+    uint64_t next_mask = mask_at(lo0);
+    int next_triangle = triangle_at(lo0);
+    for (int lo = lo0; lo >= 0; lo -= kBackBatch) {
+        asm volatile("" : "+v"(lane));  // what depends on it is made here, not kept in registers by the loop
+        const int nb = min(kBackBatch, list_last - lo);
+        const int mine = my_last - lo;  // entries [0, mine) of this block are within my range
+        const int triangle = next_triangle;
+        uint64_t m = next_mask;
+        next_triangle = triangle_at(lo - kBackBatch);
+        next_mask = mask_at(lo - kBackBatch);
+        if (__builtin_amdgcn_ballot_w64(mine > 0) != 0) {
+            const TriIds ids = ids_of(triangle);
+            // 1. which entries cover which pixel
+            if (!saved_masks) {
+                real t[9];
 #pragma unroll
-            for (int wd = 0; wd < kBackWords; wd++)
-                if (64 * wd < mine) {
-                    m[wd] = masks[(chunk + wd) * mask_slots + mask_slot];
-                    if (mine < 64 * wd + 64) m[wd] &= (1ull << (mine - 64 * wd)) - 1;  // entries past my last one
-                }
-        }
-        __syncthreads();  // every wave is done with the previous batch
-        for (int e = tid; e < nb; e += blockDim.x) {
-            gather_back(a, start + lo + e, s_rec[e]);
-            if (!saved_masks) s_touch[e] = (uint8_t)waves_touched(s_rec[e].m, s_rects, n_waves);
-        }
-        __syncthreads();
-
-        // 1. which entries cover which pixel: read back what the forward pass saved, or test again
-        //    (then only the entries that can touch this wave's pixels)
-        if (__builtin_amdgcn_ballot_w64(mine > 0) == 0) continue;  // nothing for this wave in the batch
-        if (saved_masks) {
-            // per-entry ballots = the transpose of the lanes' masks
-#pragma unroll
-            for (int wd = 0; wd < kBackWords; wd++) ballots[wd * kWave + lane] = transpose_bits(m[wd], lane);
-        } else {
-#pragma unroll
-            for (int wd = 0; wd < kBackWords; wd++) ballots[wd * kWave + lane] = 0;
+                for (int k = 0; k < 9; k++) t[k] = a.bary[9 * (int64_t)triangle + k];
+                uint64_t hit;
+                m = wave_hits(t, lane < nb, ((a.tw | a.th) & 7) == 0, wave_rect(p), p.px, p.py, hit);
+            }
+            if (mine < kBackBatch) m &= mine > 0 ? (1ull << mine) - 1 : 0ull;  // entries past my last one
+            // 2. slot numbers: lane = entry
+            const uint64_t covered = transpose_bits(m, lane);
+            const uint32_t count = (uint32_t)__builtin_popcountll(covered), incl = wave_inclusive_scan_u32(count);
+            const uint32_t n_hits = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+            mem.ballot[lane] = covered;
+            mem.base[lane] = n_hits - incl;
+            *reinterpret_cast<TriIds *>(mem.id[lane]) = ids;
             wave_lds_sync();
-#pragma unroll
-            for (int wd = 0; wd < kBackWords; wd++) {
-                uint64_t bits = 0;
-                uint64_t todo = wave_candidates(s_touch, 64 * wd, nb, wave);
-                while (todo) {
-                    const int bit = __builtin_ctzll(todo);
-                    todo &= todo - 1;
-                    const BackRecord<kDepth> &r = s_rec[64 * wd + bit];
-                    real b0, b1, b2;
-                    bary_apply(r.m, p.px, p.py, b0, b1, b2);
-                    const bool hit = bary_inside(b0, b1, b2) && 64 * wd + bit < mine;
-                    const uint64_t vote = __builtin_amdgcn_ballot_w64(hit);
-                    if (hit) bits |= 1ull << bit;
-                    if (lane == 0) ballots[64 * wd + bit] = vote;
-                }
-                m[wd] = bits;
-            }
-        }
-        wave_lds_sync();
 
-        // 2. slot numbers of this wave
-        uint32_t n_hits;
-        {
-            // lane l takes entries nb - 1 - kBackWords * l and the kBackWords - 1 before it
-            uint32_t cnt[kBackWords], mine_total = 0;
-#pragma unroll
-            for (int k = 0; k < kBackWords; k++) {
-                const int e = nb - 1 - kBackWords * lane - k;
-                cnt[k] = e >= 0 ? (uint32_t)__builtin_popcountll(ballots[e]) : 0u;
-                mine_total += cnt[k];
-            }
-            const uint32_t incl = wave_inclusive_scan_u32(mine_total);
-            uint32_t base = incl - mine_total;
-#pragma unroll
-            for (int k = 0; k < kBackWords; k++) {
-                const int e = nb - 1 - kBackWords * lane - k;
-                if (e >= 0) bases[e] = base;
-                base += cnt[k];
-            }
-            n_hits = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-        }
-        wave_lds_sync();
-
-        for (uint32_t round0 = 0; round0 < n_hits; round0 += kWaveSlots) {
-            const int n_slots = (int)min((uint32_t)kWaveSlots, n_hits - round0);
-            // 3. ordered part, lane by lane over its own hits
-            while (true) {
-                int e = -1;
-                uint32_t slot = 0;
-#pragma unroll
-                for (int wd = kBackWords - 1; wd >= 0; wd--)
-                    if (e < 0 && m[wd]) e = 64 * wd + top_bit(m[wd]);
-                if (e >= 0) {
-                    slot = bases[e] + lanes_below_mask(ballots[e]) - round0;
-                    if (slot >= (uint32_t)kWaveSlots) e = -1;
+            for (uint32_t round0 = 0; round0 < n_hits; round0 += kWaveSlots) {
+                const int n_slots = (int)min((uint32_t)kWaveSlots, n_hits - round0);
+                // 3. whose the round's slots are
+                uint64_t slots = 0;
+                while (true) {
+                    const int e = m ? top_bit(m) : 0;
+                    const uint32_t slot = mem.base[e] + lanes_below_mask(mem.ballot[e]) - round0;
+                    const bool there = m != 0 && slot < (uint32_t)kWaveSlots;
+                    if (__builtin_amdgcn_ballot_w64(there) == 0) break;
+                    if (there) {
+                        mem.tag[slot] = (uint16_t)(e | (lane << 8));
+                        slots |= 1ull << slot;
+                        m &= ~(1ull << e);
+                    }
                 }
-                const bool active = e >= 0;
-                if (__builtin_amdgcn_ballot_w64(active) == 0) break;
+                wave_lds_sync();
+
+                // 4. the fragments' values, the ordered part, the terms
+                const bool active = lane < n_slots;
+                const int tag = active ? mem.tag[lane] : lane << 8;
+                const int entry = tag & 0xff;
+                // the pixel of the slot, from the lane that owns it
+                const real px = __shfl(p.px, tag >> 8, kWave), py = __shfl(p.py, tag >> 8, kWave);
+                BackRecord<kDepth> r;
+                real b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
                 if (active) {
-#pragma unroll
-                    for (int wd = 0; wd < kBackWords; wd++)
-                        if ((e >> 6) == wd) m[wd] &= ~(1ull << (e & 63));
-                    const BackRecord<kDepth> &r = s_rec[e];
-                    real b0, b1, b2;
-                    bary_apply(r.m, p.px, p.py, b0, b1, b2);
-                    const FragSeed f = fragment_state_step(st, r, b0, b1, b2);
-                    // the five numbers wait in the slot's column of the term matrix, which is free until
-                    // the slot's own lane replaces them by the terms
-                    terms[0 * kTermStride + slot] = f.d_do;
-                    terms[1 * kTermStride + slot] = f.gc[0];
-                    terms[2 * kTermStride + slot] = f.gc[1];
-                    terms[3 * kTermStride + slot] = f.gc[2];
-                    if constexpr (kDepth) terms[4 * kTermStride + slot] = f.dd_dz;
-                    tags[slot] = e | (lane << 8);
+                    gather_back(a, *reinterpret_cast<const TriIds *>(mem.id[entry]), r);
+                    bary_apply(r.m, px, py, b0, b1, b2);
+                    leave_value<kDepth>(terms, lane, fragment_value(r, b0, b1, b2));
                 }
-            }
-            wave_lds_sync();
-
-            // 4. order-free part: lane = slot
-            int tag = -1;
-            if (lane < n_slots) tag = tags[lane] & 0xff;
-            // the pixel of the slot, from the lane that owns it
-            const int src = (lane < n_slots) ? tags[lane] >> 8 : lane;
-            const real px = __shfl(p.px, src, kWave), py = __shfl(p.py, src, kWave);
-            if (lane < n_slots) {
-                FragSeed f;
-                f.d_do = terms[0 * kTermStride + lane];
-                f.gc[0] = terms[1 * kTermStride + lane];
-                f.gc[1] = terms[2 * kTermStride + lane];
-                f.gc[2] = terms[3 * kTermStride + lane];
-                if constexpr (kDepth) f.dd_dz = terms[4 * kTermStride + lane];
-                const BackRecord<kDepth> &r = s_rec[tag];
-                real b0, b1, b2;
-                bary_apply(r.m, px, py, b0, b1, b2);
-                real term[kTerms];
-                fragment_terms(f, r, b0, b1, b2, px, py, term);
+                wave_lds_sync();
+                walk_slots<kDepth>(terms, slots, st);
+                wave_lds_sync();
+                if (active) {
+                    const FragSeed f = seed_of_slot<kDepth>(terms, lane);
+                    real term[kTerms];
+                    fragment_terms(f, r, b0, b1, b2, px, py, term);
 #pragma unroll
-                for (int q = 0; q < kTerms; q++) terms[q * kTermStride + lane] = term[q];
+                    for (int q = 0; q < kTerms; q++) terms[q * kTermStride + lane] = term[q];
+                }
+                const int entry_before = __shfl_up(entry, 1, kWave);
+                const uint64_t heads = __builtin_amdgcn_ballot_w64(active && (lane == 0 || entry != entry_before));
+                wave_lds_sync();
+                add_run_sums(terms, n_slots, heads, tl, [&](int c, int v) { return mem.id[mem.tag[c] & 0xff][1 + v]; });
+                wave_lds_sync();
             }
-            const int tag_before = __shfl_up(tag, 1, kWave);
-            const uint64_t heads = __builtin_amdgcn_ballot_w64(lane < n_slots && (lane == 0 || tag != tag_before));
-            wave_lds_sync();
-            add_run_sums(terms, n_slots, heads, tl, [&](int c, int v) { return s_rec[tags[c] & 0xff].id[v]; });
-            wave_lds_sync();
         }
     }
 }
@@ -838,7 +816,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
         if (want) {
             for (int i = 0; i < found; i++) {
                 BackRecord<true> r;
-                gather_back(a, tk.j(i), r);
+                gather_back(a, load_ids(a, tk.j(i)), r);
                 real b0, b1, b2;
                 bary_apply(r.m, p.px, p.py, b0, b1, b2);
                 if (!bary_inside(b0, b1, b2)) continue;  // cannot happen: the selection tested it
@@ -898,8 +876,8 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
 //      columns (ballot matching, groups in order of their lowest slot) of a term
 //      matrix in LDS, three groups of 21 lanes add up the runs of equal entry and issue
 //      one global floating-point atomic per run and term.
-// The waves of a tile share nothing, so a workgroup is one wave: its place is free for another tile's when it is done, where
-// workgroups of four wait for the longest of them (saved_order_waves).  In fours and so, us: 10^6 triangles 1057, 1013, 10^5 83.5, 76,
+// The waves of a tile share nothing, so a workgroup is one of them: its place is free for another tile's when it is done, where
+// workgroups of four wait for the longest of them (workgroup_waves).  In fours and so, us: 10^6 triangles 1057, 1013, 10^5 83.5, 76,
 // 20 000 with a heavy tail on 1920 x 1080 61, 55, a mesh of 1.3 million 185, 180.
 // What a wave keeps in LDS.  A workgroup takes it for the waves it has (taken for four always, frames in tiles of 8 x 8, a wave each,
 // had five workgroups a CU: 33 000 triangles 229 us, so 116).
@@ -911,7 +889,7 @@ struct SavedWave {
     uint8_t src[kWave];     // the pixel (lane) of a slot
 };
 template <int kLayout, bool kDepth>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 5) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
@@ -1023,51 +1001,21 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 4 : 1) void backw
         int rel = 0;
         if (lane < n_slots) {
             rel = rels[lane];
-            gather_back(a, start + rel, r);
+            gather_back(a, load_ids(a, start + rel), r);
             bary_apply(r.m, px, py, b0, b1, b2);
-            const FragValue v = fragment_value(r, b0, b1, b2);
-            terms[0 * kTermStride + lane] = v.o;
-            terms[1 * kTermStride + lane] = v.color[0];
-            terms[2 * kTermStride + lane] = v.color[1];
-            terms[3 * kTermStride + lane] = v.color[2];
-            if constexpr (kDepth) terms[4 * kTermStride + lane] = v.z;
+            leave_value<kDepth>(terms, lane, fragment_value(r, b0, b1, b2));
         }
         wave_lds_sync();
 
         // 3. lane = pixel: the ordered part
-        while (true) {
-            const bool active = mine != 0;
-            if (__builtin_amdgcn_ballot_w64(active) == 0) break;
-            if (active) {
-                const int c = __builtin_ctzll(mine);
-                mine &= mine - 1;
-                FragValue v;
-                v.o = terms[0 * kTermStride + c];
-                v.color[0] = terms[1 * kTermStride + c];
-                v.color[1] = terms[2 * kTermStride + c];
-                v.color[2] = terms[3 * kTermStride + c];
-                if constexpr (kDepth) v.z = terms[4 * kTermStride + c];
-                const FragSeed f = fragment_chain_step<kDepth>(st, v);
-                terms[0 * kTermStride + c] = f.d_do;
-                terms[1 * kTermStride + c] = f.gc[0];
-                terms[2 * kTermStride + c] = f.gc[1];
-                terms[3 * kTermStride + c] = f.gc[2];
-                if constexpr (kDepth) terms[4 * kTermStride + c] = f.dd_dz;
-            }
-        }
+        walk_slots<kDepth>(terms, mine, st);
         wave_lds_sync();
 
         // 4. lane = slot: the terms, in the column the matching gives the slot
         const bool active = lane < n_slots;
         FragSeed f;
         f.d_do = f.gc[0] = f.gc[1] = f.gc[2] = f.dd_dz = 0.0f;
-        if (active) {
-            f.d_do = terms[0 * kTermStride + lane];
-            f.gc[0] = terms[1 * kTermStride + lane];
-            f.gc[1] = terms[2 * kTermStride + lane];
-            f.gc[2] = terms[3 * kTermStride + lane];
-            if constexpr (kDepth) f.dd_dz = terms[4 * kTermStride + lane];
-        }
+        if (active) f = seed_of_slot<kDepth>(terms, lane);
         // By the bits that tell positions of the round's range apart: the few positions outside it (a second step behind a
         // first one, by depth, may come later in the list) can be taken together with others, and then make more runs, not
         // other ones.
@@ -1127,7 +1075,7 @@ using namespace tg;
 // each.  200 000 large triangles on 512 x 512: 248 us singly, 231 in fours, 20 000 without a limit on the layers 560 and 551; on
 // 480 x 480 239, 231 and 576, 596.  With fewer waves there is room for all (448 x 448: 222, 228), with more the next one takes the
 // place (528 x 528: 259, 262 and 571, 604).
-static int saved_order_waves(int width, int height, int tile_w, int tile_h) {
+static int workgroup_waves(int width, int height, int tile_w, int tile_h) {
     constexpr int64_t kChipWaves = 4 * 1024;
     const int64_t waves = (int64_t)ceil_div(width, tile_w) * ceil_div(height, tile_h) * ceil_div(tile_w * tile_h, kWave);
     return waves > kChipWaves / 8 * 7 && waves <= kChipWaves ? kMaxWaves : 1;
@@ -1159,9 +1107,10 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
     }
     RasterArgs a{(const real4 *)vertices, indices, colors, opacities, sorted_ids, offsets, bary, nullptr, nullptr,
                  width, height, tile_w, tile_h, early_stopping_threshold, max_layers};
+    const TileLaunch forward = tile_launch(width, height, tile_w, tile_h, kTileThreads);  // whose hit masks are read
     BackwardArgs g{(const real4 *)grad_image, grad_depthmap, (const real4 *)image, depthmap, final_weights, ends, last,
                    last_depth, order, per_pixel_sort ? nullptr : hit_masks, grad_vertices, grad_colors, grad_opacities,
-                   vertex_stride, color_stride, opacity_stride, list_status,
+                   vertex_stride, color_stride, opacity_stride, list_status, (int)forward.grid.z, forward.threads,
                    max_layers >= kManyLayers && n_keys / kDeepLists >= (int64_t)ceil_div(width, tile_w) * ceil_div(height, tile_h)};
     hipStream_t s = (hipStream_t)stream;
     const int layout = (vertex_stride == 4 && color_stride == 3 && opacity_stride == 1)   ? kGradDense
@@ -1173,17 +1122,17 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
         else if (layout == kGradBlock8) TG_LAUNCH_AS(#kernel, (kernel<kGradBlock8 __VA_OPT__(,) __VA_ARGS__>), grid, block, lds_bytes, s, a, g);   \
         else TG_LAUNCH_AS(#kernel, (kernel<kGradStrided __VA_OPT__(,) __VA_ARGS__>), grid, block, lds_bytes, s, a, g);                             \
     } while (0)
+    const TileLaunch waves = tile_launch(width, height, tile_w, tile_h, workgroup_waves(width, height, tile_w, tile_h) * kWave);
     if (!per_pixel_sort) {
-        const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, kTileThreads);
-        if (grad_depthmap) TG_LAUNCH_BACKWARD(backward_tile_order_kernel, tl.grid, dim3(tl.threads), 0, true);
-        else TG_LAUNCH_BACKWARD(backward_tile_order_kernel, tl.grid, dim3(tl.threads), 0, false);
+        const size_t lds = sizeof(TileWave) * (waves.threads / kWave);
+        if (grad_depthmap) TG_LAUNCH_BACKWARD(backward_tile_order_kernel, waves.grid, dim3(waves.threads), lds, true);
+        else TG_LAUNCH_BACKWARD(backward_tile_order_kernel, waves.grid, dim3(waves.threads), lds, false);
         return check_launch("backward_tile_order_kernel");
     }
     if (order.low) {
-        const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, saved_order_waves(width, height, tile_w, tile_h) * kWave);
-        const size_t lds = sizeof(SavedWave) * (tl.threads / kWave);
-        if (grad_depthmap) TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), lds, true);
-        else TG_LAUNCH_BACKWARD(backward_saved_order_kernel, tl.grid, dim3(tl.threads), lds, false);
+        const size_t lds = sizeof(SavedWave) * (waves.threads / kWave);
+        if (grad_depthmap) TG_LAUNCH_BACKWARD(backward_saved_order_kernel, waves.grid, dim3(waves.threads), lds, true);
+        else TG_LAUNCH_BACKWARD(backward_saved_order_kernel, waves.grid, dim3(waves.threads), lds, false);
         return check_launch("backward_saved_order_kernel");
     }
     const TileLaunch tl = tile_launch(width, height, tile_w, tile_h, pixel_order_threads(kTileThreads));
