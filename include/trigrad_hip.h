@@ -402,7 +402,12 @@ int tg_split_gradient_block(const tg_real *block, int64_t n_vertices, tg_real *g
  * TG_FRAME_EXPIRED once K is there, [2] the list kernels' status once it is known (TG_FRAME_PENDING before).
  * phases: which parts of the forward pass to launch; TG_FRAME_WAIT then waits for K (the one wait of the call) and
  * sets n_keys and counted.
- * gradients: (V,4), (V,3) and (V,) behind each other; block: (V,8) of scratch with per_pixel_sort. */
+ * gradients: (V,4), (V,3) and (V,) behind each other.  block: (V,8) of scratch, in which they are summed first where
+ * tg_sums_in_block says so (else it is not looked at); may be NULL in tile order, and then they are summed in place. */
+static inline int tg_sums_in_block(int64_t n_vertices, int64_t n_triangles, int64_t width, int64_t height, int per_pixel_sort) {
+    const int64_t pixels = width * height;
+    return n_vertices >= 32768 || (per_pixel_sort ? pixels > 16384 : 3 * n_triangles > 2 * n_vertices && pixels > 65536);
+}
 typedef struct tg_frame {
     const tg_real *vertices;
     const int32_t *indices;

@@ -1562,3 +1562,43 @@ def test_tile_order_gradients_around_blocks_of_a_list(width, height, tw, th, n, 
                                      sorted_ids, offsets, bary, image, depthmap, weights, ends, width, height, tw, th, 1 / 256, False, ml, resume=masks)
             for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
                 assert_gradients_close(f"{n} in {width}x{height}, tiles of {tw}x{th}: {label}", g.cpu().numpy(), w, mag)
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
+@pytest.mark.parametrize("vertices,shared,width,height", [
+    (32767, False, 128, 128), (32768, False, 128, 128), (32770, False, 130, 97), (3000, False, 129, 128), (3000, True, 256, 256),
+    (3000, True, 257, 256), (3000, False, 257, 256)])
+def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height, mode, cuda, oracle):
+    """From 32768 vertices on, in per-pixel order in images of more than 16384 pixels, and in tile order where triangles share vertices in
+    images of more than 65536, the gradients are summed in a (V,8) block, else in the dense arrays: on both sides of the lines, by
+    the frame's call (a first frame, and ones whose plan is there) and by the stage-by-stage route."""
+    import torch
+    import scenes as S
+    import trigrad_amd
+    from trigrad_amd import _C
+    m = MODES[mode]
+    scene = S.random_soup(-(-vertices // 3), width, height, seed=8, sigma_px=3.0, opacity=(0.1, 0.6), varying_w=True)
+    indices = np.minimum(scene["indices"], vertices - 1)
+    if shared:  # every vertex is three triangles': a corner of the next one and of the one after it too
+        indices = np.concatenate([indices, indices[:, [0, 1, 2]] * [1, 1, 0] + np.roll(indices, 1, 0) * [0, 0, 1],
+                                  indices[:, [0, 1, 2]] * [1, 0, 0] + np.roll(indices, 2, 0) * [0, 1, 1]])
+    scene.update(vertices=scene["vertices"][:vertices], colors=scene["colors"][:vertices], opacities=scene["opacities"][:vertices],
+                 indices=np.ascontiguousarray(indices, dtype=np.int32))
+    by_block = vertices >= 32768 or (width > 128 if m["per_pixel_sort"] else shared and width == 257)
+    assert _C._sums_in_block(vertices, scene["indices"].shape[0], width, height, m["per_pixel_sort"]) == by_block
+    d, want, got, ml = _forward_both(scene, 16, 16, m, cuda, oracle)
+    gi, gd = _grad_inputs(scene, 2, False)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, 16, 16,
+                                    m["per_pixel_sort"], ml, literal=False, magnitudes=True)
+    gi = torch.from_numpy(gi).to(cuda)
+    image, depthmap, weights, sorted_ids, offsets, bary, ends, _, resume = got
+    outs = [_C.render_backward(gi, None, d["vertices"], d["indices"], d["colors"], d["opacities"], sorted_ids, offsets, bary, image, depthmap,
+                               weights, ends, width, height, 16, 16, 1 / 256, m["per_pixel_sort"], ml, resume=resume)]
+    leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+    for _ in range(3):
+        image, _ = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, per_pixel_sort=m["per_pixel_sort"], max_layers=m["max_layers"])
+        outs.append(torch.autograd.grad(image, leaves, gi))
+    for out in outs:
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+            assert g.is_contiguous()
+            assert_gradients_close(f"{vertices} vertices/{mode}: {label}", g.cpu().numpy(), w, mag)

@@ -230,13 +230,20 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
     char *kept = (char *)f->kept;
     const int64_t V = f->n_vertices;
     if (V == 0) return 0;
-    // one zero fill for the three gradients.  Tile order: (V,4) | (V,3) | (V,) behind each other.  Per-pixel order issues
-    // five times as many atomics; there the eight gradients of a vertex share a 32-byte sector of a (V,8) block while
-    // the kernel runs, and the three arrays are copied out afterwards.
-    real *sums = f->per_pixel_sort ? f->block : f->gradients;
+    // One zero fill for the three gradients.  Where there are many vertices, or many waves meet in one, the eight gradients of a vertex lie
+    // in a 32-byte sector of a (V,8) block while the kernel runs, and the three arrays are copied out afterwards: the atomics of a run
+    // then fall into three sectors and not nine.  The copy is another launch, and sums of few vertices stay in the L2 whatever their
+    // places, so not for the smallest images, and in tile order, with less than half the atomics, only where vertices are many or
+    // triangles share them.  Kernels, us, dense and by the block with the copy.  Tile order, a soup of 3 * 10^6 vertices 577, 360 + 28,
+    // 3 * 10^5 82, 68 + 6, 9 * 10^4 36.2, 31.7 + 4.8, 5 * 10^4 with a heavy tail 375, 319 + 5, 3 * 10^4 18.8, 18.4 + 2.9; a mesh of
+    // 650 000 on 1920 x 1080 440, 310 + 8, 28 000 on 1235 x 981 91, 62 + 5, 1200 there 124, 58 + 5, 5000 on 500 x 400 26, 23 + 2.4,
+    // on 256 x 256 24.4, 22.4 + 2.4.  Per-pixel order, a soup of 9 * 10^4 43.8, 36.3 + 4.7, of 1500 with a heavy tail on 256 x 256
+    // 98, 92.5 + 4.6, 300 on 128 x 128 38.9, 35.3 + 3.5, 60 on 50 x 50 10.2, 10.1 + 1.4; a mesh of 1200 on 1235 x 981 137, 67 + 5.
+    const bool by_block = f->block && ((uintptr_t)f->block & 15) == 0 && tg_sums_in_block(V, f->n_triangles, f->width, f->height, f->per_pixel_sort != 0);
+    real *sums = by_block ? f->block : f->gradients;
     TG_LAUNCH(zero_gradients_kernel, dim3((unsigned)ceil_div64(2 * V, 256)), dim3(256), 0, (hipStream_t)f->stream, (real4 *)sums, 2 * V);
     if (int e = check_launch("zero_gradients_kernel")) return e;
-    const int stride = f->per_pixel_sort ? 8 : 0;
+    const int stride = by_block ? 8 : 0;
     if (int e = render_backward(f->grad_image, f->grad_depthmap, f->vertices, f->indices, f->colors, f->opacities,
                                 (const int32_t *)(kept + L.ids), (const int32_t *)(kept + L.offsets), (const real *)(kept + L.bary), f->image,
                                 f->depthmap, (const real *)(kept + L.weights), (const int32_t *)(kept + L.ends),
@@ -247,7 +254,7 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
                                 stride ? sums + 7 : sums + 7 * V, stride ? stride : 4, stride ? stride : 3, stride ? stride : 1,
                                 (const uint32_t *)(kept + L.status), f->key_capacity, f->stream))
         return e;
-    if (!f->per_pixel_sort) return 0;
+    if (!by_block) return 0;
     return tg_split_gradient_block(f->block, V, f->gradients, f->gradients + 4 * V, f->gradients + 7 * V, f->stream);
 }
 #endif

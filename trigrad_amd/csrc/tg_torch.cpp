@@ -227,8 +227,8 @@ struct Render : torch::autograd::Function<Render> {
         const at::Tensor gradients = at::empty({8 * n}, on(v, at::kFloat));  // (V,4) | (V,3) | (V,) behind each other
         tg_frame f;
         frame.plan->fill(f, n, i.size(0), frame.max_layers);
-        at::Tensor block;
-        if (f.per_pixel_sort) block = at::empty({8 * n}, on(v, at::kFloat));
+        const bool by_block = tg_sums_in_block(n, f.n_triangles, f.width, f.height, f.per_pixel_sort != 0);
+        const at::Tensor block = by_block ? at::empty({8 * n}, on(v, at::kFloat)) : gradients;
         f.vertices = v.data_ptr<float>();
         f.indices = i.data_ptr<int32_t>();
         f.colors = c.data_ptr<float>();
@@ -240,7 +240,7 @@ struct Render : torch::autograd::Function<Render> {
         f.grad_image = grad_image.data_ptr<float>();
         f.grad_depthmap = grad_depthmap.defined() ? grad_depthmap.data_ptr<float>() : nullptr;
         f.gradients = gradients.data_ptr<float>();
-        f.block = block.defined() ? block.data_ptr<float>() : nullptr;
+        f.block = block.data_ptr<float>();
         check(lib.backward(&f), "tg_frame_backward");
         frame.status->verify();  // everything is launched, and the kernels look at the word themselves
         return {gradients.as_strided({n, 4}, {4, 1}, 0), at::Tensor(), gradients.as_strided({n, 3}, {3, 1}, 4 * n),
