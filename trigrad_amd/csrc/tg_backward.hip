@@ -670,11 +670,11 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
                 const int n_slots = (int)min((uint32_t)kWaveSlots, n_hits - round0);
                 // 3. whose the round's slots are
                 uint64_t slots = 0;
-                while (true) {
+                for (int handed_out = 0; handed_out < n_slots;) {  // a turn hands out one at least: the first one left is its pixel's next
                     const int e = m ? top_bit(m) : 0;
                     const uint32_t slot = mem.base[e] + lanes_below_mask(mem.ballot[e]) - round0;
                     const bool there = m != 0 && slot < (uint32_t)kWaveSlots;
-                    if (__builtin_amdgcn_ballot_w64(there) == 0) break;
+                    handed_out += __builtin_popcountll(__builtin_amdgcn_ballot_w64(there));
                     if (there) {
                         mem.tag[slot] = (uint16_t)(e | (lane << 8));
                         slots |= 1ull << slot;
