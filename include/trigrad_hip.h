@@ -402,12 +402,9 @@ int tg_split_gradient_block(const tg_real *block, int64_t n_vertices, tg_real *g
  * TG_FRAME_EXPIRED once K is there, [2] the list kernels' status once it is known (TG_FRAME_PENDING before).
  * phases: which parts of the forward pass to launch; TG_FRAME_WAIT then waits for K (the one wait of the call) and
  * sets n_keys and counted.
- * gradients: (V,4), (V,3) and (V,) behind each other.  block: (V,8) of scratch, in which they are summed first where
- * tg_sums_in_block says so (else it is not looked at); may be NULL in tile order, and then they are summed in place. */
-static inline int tg_sums_in_block(int64_t n_vertices, int64_t n_triangles, int64_t width, int64_t height, int per_pixel_sort) {
-    const int64_t pixels = width * height;
-    return n_vertices >= 32768 || (per_pixel_sort ? pixels > 16384 : 3 * n_triangles > 2 * n_vertices && pixels > 65536);
-}
+ * gradients: (V,4), (V,3) and (V,) behind each other; block: (V,8) of scratch with per_pixel_sort, or, with
+ * TG_FRAME_GRADIENT_COPIES in the backward call's phases, of tg_frame_gradient_copies times that (any 16-byte aligned pointer where it
+ * is 0). */
 typedef struct tg_frame {
     const tg_real *vertices;
     const int32_t *indices;
@@ -443,6 +440,11 @@ typedef struct tg_frame {
     int64_t scratch_bytes;
     double early_stopping_threshold;
 } tg_frame;
+
+#define TG_FRAME_GRADIENT_COPIES 256
+/* How many (V,8) blocks a frame's gradients are summed in before they are copied out: 0, they are summed in place; 1, a vertex's
+ * eight in one 32-byte sector; or 8, one for each XCD, where its triangles are in many tiles each. */
+int tg_frame_gradient_copies(const tg_frame *f);
 
 #define TG_FRAME_BACKWARD 1     /* flags: a backward pass will follow: save what it needs */
 #define TG_FRAME_ORDER_PLANES 2 /*   ... the blend order in planes (per_pixel_sort, max_layers <= TG_MAX_SAVED_LAYERS) */

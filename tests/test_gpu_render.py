@@ -1567,15 +1567,16 @@ def test_tile_order_gradients_around_blocks_of_a_list(width, height, tw, th, n, 
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
 @pytest.mark.parametrize("vertices,shared,width,height", [
     (32767, False, 128, 128), (32768, False, 128, 128), (32770, False, 130, 97), (3000, False, 129, 128), (3000, True, 256, 256),
-    (3000, True, 257, 256), (3000, False, 257, 256)])
+    (3000, True, 257, 256), (32768, False, 1024, 511), (32768, False, 1024, 512), (32767, False, 1024, 512)])
 def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height, mode, cuda, oracle):
-    """From 32768 vertices on, in per-pixel order in images of more than 16384 pixels, and in tile order where triangles share vertices in
-    images of more than 65536, the gradients are summed in a (V,8) block, else in the dense arrays: on both sides of the lines, by
-    the frame's call (a first frame, and ones whose plan is there) and by the stage-by-stage route."""
+    """In per-pixel order from 32768 vertices on or in images of more than 16384 pixels, and in tile order where triangles share vertices
+    in images of more than 65536 or 32768 vertices are in one of 2^19, the gradients are summed in a (V,8) block, else in the
+    dense arrays: on both sides of the lines, by the frame's call (a first frame, and ones whose plan is there) and by the
+    stage-by-stage route."""
     import torch
     import scenes as S
     import trigrad_amd
-    from trigrad_amd import _C
+    from trigrad_amd import _C, _lib
     m = MODES[mode]
     scene = S.random_soup(-(-vertices // 3), width, height, seed=8, sigma_px=3.0, opacity=(0.1, 0.6), varying_w=True)
     indices = np.minimum(scene["indices"], vertices - 1)
@@ -1584,8 +1585,9 @@ def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height
                                   indices[:, [0, 1, 2]] * [1, 0, 0] + np.roll(indices, 2, 0) * [0, 1, 1]])
     scene.update(vertices=scene["vertices"][:vertices], colors=scene["colors"][:vertices], opacities=scene["opacities"][:vertices],
                  indices=np.ascontiguousarray(indices, dtype=np.int32))
-    by_block = vertices >= 32768 or (width > 128 if m["per_pixel_sort"] else shared and width == 257)
-    assert _C._sums_in_block(vertices, scene["indices"].shape[0], width, height, m["per_pixel_sort"]) == by_block
+    by_block = (vertices >= 32768 or width > 128) if m["per_pixel_sort"] else (shared and width == 257) or (vertices == 32768 and height == 512)
+    kind = _C._FRAME_KIND.pack(vertices, scene["indices"].shape[0], width, height, 16, 16, m["per_pixel_sort"], 32, 0, 0, 0, 0, 0.0)
+    assert _C._gradient_copies(_lib.load(32), kind) == by_block
     d, want, got, ml = _forward_both(scene, 16, 16, m, cuda, oracle)
     gi, gd = _grad_inputs(scene, 2, False)
     wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, 16, 16,
@@ -1602,3 +1604,34 @@ def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height
         for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
             assert g.is_contiguous()
             assert_gradients_close(f"{vertices} vertices/{mode}: {label}", g.cpu().numpy(), w, mag)
+
+
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "A_unlimited", "B_unlimited"])
+@pytest.mark.parametrize("n,sigma,width,height,tw,th,per_waves", [
+    (150, 20.0, 150, 121, 16, 16, True), (150, 20.0, 128, 128, 16, 16, False), (1512, 20.0, 150, 121, 16, 16, True), (1513, 20.0, 150, 121, 16, 16, False), (400, 30.0, 200, 131, 8, 8, True), (400, 4.0, 200, 131, 8, 8, False),
+    (60, 50.0, 160, 160, 32, 32, True)])
+def test_gradients_summed_by_xcds(n, sigma, width, height, tw, th, per_waves, mode, cuda, oracle):
+    """Where triangles are in 24 waves on average each XCD sums the gradients in a block of its own: on both sides of the line, by a first
+    frame (the Python route) and by ones whose plan is there (the module's)."""
+    import torch
+    import scenes as S
+    import trigrad_amd
+    from trigrad_amd import _C, _lib
+    m = MODES[mode]
+    scene = S.random_soup(n, width, height, seed=n, sigma_px=sigma, opacity=(0.05, 0.5), varying_w=True)
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256,
+                         m["per_pixel_sort"], ml)
+    capacity = _C._round_capacity(int(want["offsets"][-1]))
+    kind = _C._FRAME_KIND.pack(3 * n, n, width, height, tw, th, m["per_pixel_sort"], ml, capacity, 0, 0, 0, 0.0)
+    assert (_C._gradient_copies(_lib.load(32), kind) == 8) == per_waves
+    gi, gd = _grad_inputs(scene, 9, True)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, tw, th,
+                                    m["per_pixel_sort"], ml, literal=False, magnitudes=True)
+    d = to_device(scene, cuda)
+    leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+    for _ in range(4):
+        outputs = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, tw, th, per_pixel_sort=m["per_pixel_sort"], max_layers=m["max_layers"])
+        out = torch.autograd.grad(outputs, leaves, (torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda)))
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+            assert_gradients_close(f"{n} triangles/{mode}: {label}", g.cpu().numpy(), w, mag)

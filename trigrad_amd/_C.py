@@ -898,10 +898,12 @@ def _frame_launches(index, stream):
     return lock
 
 
-def _sums_in_block(n_vertices, n_triangles, width, height, per_pixel_sort):
-    """tg_sums_in_block of the C header."""
-    pixels = width * height
-    return n_vertices >= 32768 or (pixels > 16384 if per_pixel_sort else 3 * n_triangles > 2 * n_vertices and pixels > 65536)
+_FRAME_GRADIENT_COPIES = 256  # TG_FRAME_GRADIENT_COPIES of the C header
+
+
+def _gradient_copies(lib, kind):
+    """How many (V,8) blocks the gradients of a frame of a kind (packed) are summed in; 0: they are summed in place."""
+    return lib.tg_frame_gradient_copies(bytes(_FRAME_CALL.size + _FRAME_RESULT.size) + kind)
 
 
 def frame_backward(frame, grad_image, grad_depthmap, vertices, indices, colors, opacities, image, depthmap, kept):
@@ -917,12 +919,12 @@ def frame_backward(frame, grad_image, grad_depthmap, vertices, indices, colors, 
         if grad_depthmap is not None:
             grad_depthmap = grad_depthmap.contiguous()
         gradients = torch.empty((8 * n_vertices,), dtype=torch.float32, device=dev)
-        by_block = _sums_in_block(n_vertices, indices.shape[0], image.shape[1], image.shape[0], plan.per_pixel_sort)
-        block = torch.empty_like(gradients) if by_block else gradients
+        copies = _gradient_copies(lib, plan.kind)
+        block = torch.empty((copies * 8 * n_vertices,), dtype=torch.float32, device=dev) if copies else gradients
         call = bytearray(_FRAME_BYTES)
         call[-_FRAME_KIND.size:] = plan.kind
         _FRAME_CALL.pack_into(call, 0, vertices.data_ptr(), indices.data_ptr(), colors.data_ptr(), opacities.data_ptr(), image.data_ptr(),
-                              depthmap.data_ptr(), kept.data_ptr(), 0, 0, 0, _raw_stream(dev), 0, 0, 0, grad_image.data_ptr(),
+                              depthmap.data_ptr(), kept.data_ptr(), 0, 0, 0, _raw_stream(dev), 0, 0, _FRAME_GRADIENT_COPIES, grad_image.data_ptr(),
                               0 if grad_depthmap is None else grad_depthmap.data_ptr(), gradients.data_ptr(),
                               block.data_ptr())
         code = lib.tg_frame_backward((C.c_char * _FRAME_BYTES).from_buffer(call))
@@ -1150,7 +1152,7 @@ def render_backward(grad_output, grad_depthmap, vertices, indices, colors, opaci
     saves eleven tensors and nothing else) it is taken from `ends` if render_forward's attribute is still
     there, else computed again.  grad_depthmap may be None (no gradient reached the depth map).  grad_strides
     (scalars per vertex in the three arrays the kernel accumulates into) defaults to one (V,8) block or dense arrays by
-    _sums_in_block; the returned tensors are dense either way."""
+    _gradient_copies; the returned tensors are dense either way."""
     _need_cuda(grad_output, vertices)
     if max_layers <= 0:
         max_layers = indices.shape[0] + 1
@@ -1174,7 +1176,8 @@ def render_backward(grad_output, grad_depthmap, vertices, indices, colors, opaci
         # one zero fill for the three gradients: (V,4) | (V,3) | (V,) views of one block, or, for many or shared vertices, the eight
         # gradients of a vertex in a 32-byte sector of a (V,8) block while the kernel runs, copied out afterwards
         V = vertices.shape[0]
-        strides = tuple(grad_strides) if grad_strides is not None else ((8, 8, 8) if _sums_in_block(V, indices.shape[0], width, height, per_pixel_sort) else (4, 3, 1))
+        kind = _FRAME_KIND.pack(V, indices.shape[0], width, height, tile_width, tile_height, bool(per_pixel_sort), max_layers, 0, 0, 0, 0, 0.0)
+        strides = tuple(grad_strides) if grad_strides is not None else ((8, 8, 8) if _gradient_copies(lib, kind) else (4, 3, 1))
         if strides == (4, 3, 1):
             block = torch.zeros((8 * V,), dtype=vertices.dtype, device=dev)
             grad_vertices = block[:4 * V].view(V, 4)

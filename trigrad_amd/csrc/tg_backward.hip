@@ -40,6 +40,7 @@ struct BackwardArgs {
     int vertex_stride, color_stride, opacity_stride;  // scalars from one vertex to the next in the three arrays
     const uint32_t *list_status;  // status word of the kernels that made the lists (TG_STATUS_*); may be null
     int mask_parts, mask_threads; // of the saved hit masks: workgroups of a tile in the forward launch, and their threads
+    int64_t copy_stride;          // scalars from one XCD's gradient arrays to the next one's; 0: all XCDs share them
     bool deep;                    // many layers and long lists: which tiles an XCD takes (tile_of_workgroup)
 };
 
@@ -433,6 +434,12 @@ constexpr int kWaveSlots = 64;    // hit slots per wave and round: one per lane 
 constexpr int kTermStride = 65;   // row stride of the per-wave term matrix (odd: conflict-free columns)
 constexpr int kMaxWaves = kTileThreads / kWave;
 
+// The number of the XCD that runs the calling wave.  What depends on it is where sums are kept, not what they are.
+__device__ __forceinline__ int xcd_number() {
+    constexpr int kXccId = 20, kBits = 4;  // the hardware register and its width
+    return (int)__builtin_amdgcn_s_getreg(kXccId | (kBits - 1) << 11) & (kXcds - 1);
+}
+
 // The run sums' view of a lane: lane = 21 * group + q adds up gradient term q over the group's third
 // of the slots.  What depends on q only is worked out once per kernel.
 struct TermLane {
@@ -451,7 +458,7 @@ __device__ __forceinline__ TermLane term_lane(const BackwardArgs &g, int lane) {
     t.vertex = t.q / 7;
     const int c = t.q - 7 * t.vertex;
     t.stride = term_stride<kLayout>(g, c);
-    t.base = term_address<kLayout>(g, 0, c);
+    t.base = term_address<kLayout>(g, 0, c) + g.copy_stride * xcd_number();
     return t;
 }
 
@@ -1051,12 +1058,17 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
 
 // The three gradient arrays out of the (V,8) block the per-pixel-order kernels accumulate into:
 // one read of the block instead of the three strided ones that three separate copies make.
-__global__ __launch_bounds__(256) void split_gradient_block_kernel(const real4 *__restrict__ block, int64_t n_vertices,
+__global__ __launch_bounds__(256) void split_gradient_block_kernel(const real4 *__restrict__ block, int64_t n_vertices, int copies,
                                                                    real4 *__restrict__ grad_vertices, real *__restrict__ grad_colors,
                                                                    real *__restrict__ grad_opacities) {
     const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (v >= n_vertices) return;
-    const real4 position = block[2 * v], rest = block[2 * v + 1];
+    real4 position = block[2 * v], rest = block[2 * v + 1];
+    for (int k = 1; k < copies; k++) {
+        const real4 a = block[2 * (v + k * n_vertices)], b = block[2 * (v + k * n_vertices) + 1];
+        position.x += a.x; position.y += a.y; position.w += a.w;
+        rest.x += b.x; rest.y += b.y; rest.z += b.z; rest.w += b.w;
+    }
     grad_vertices[v] = position;
     grad_colors[3 * v] = rest.x;
     grad_colors[3 * v + 1] = rest.y;
@@ -1089,7 +1101,7 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
                                   int height, int tile_w,
                                   int tile_h, real early_stopping_threshold, int per_pixel_sort, int max_layers, real *grad_vertices,
                                   real *grad_colors, real *grad_opacities, int vertex_stride, int color_stride,
-                                  int opacity_stride, const uint32_t *list_status, int64_t n_keys, void *stream) {
+                                  int opacity_stride, int64_t copy_stride, const uint32_t *list_status, int64_t n_keys, void *stream) {
     if (int e = check_raster_args("tg_render_backward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!grad_image || !vertices || !indices || !colors || !opacities || !offsets || !bary || !image ||
         !depthmap || !final_weights || !ends || !last || !grad_vertices || !grad_colors || !grad_opacities ||
@@ -1110,7 +1122,7 @@ int tg::render_backward(const real *grad_image, const real *grad_depthmap, const
     const TileLaunch forward = tile_launch(width, height, tile_w, tile_h, kTileThreads);  // whose hit masks are read
     BackwardArgs g{(const real4 *)grad_image, grad_depthmap, (const real4 *)image, depthmap, final_weights, ends, last,
                    last_depth, order, per_pixel_sort ? nullptr : hit_masks, grad_vertices, grad_colors, grad_opacities,
-                   vertex_stride, color_stride, opacity_stride, list_status, (int)forward.grid.z, forward.threads,
+                   vertex_stride, color_stride, opacity_stride, list_status, (int)forward.grid.z, forward.threads, copy_stride,
                    max_layers >= kManyLayers && n_keys / kDeepLists >= (int64_t)ceil_div(width, tile_w) * ceil_div(height, tile_h)};
     hipStream_t s = (hipStream_t)stream;
     const int layout = (vertex_stride == 4 && color_stride == 3 && opacity_stride == 1)   ? kGradDense
@@ -1163,7 +1175,7 @@ extern "C" int tg_render_backward(const real *grad_image, const real *grad_depth
     return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
                            final_weights, ends, last, last_depth, order, hit_masks, width, height, tile_w, tile_h,
                            early_stopping_threshold, per_pixel_sort, max_layers, grad_vertices, grad_colors, grad_opacities,
-                           vertex_stride, color_stride, opacity_stride, nullptr, 0, stream);
+                           vertex_stride, color_stride, opacity_stride, 0, nullptr, 0, stream);
 }
 
 extern "C" int tg_render_backward_pooled(const real *grad_image, const real *grad_depthmap, const real *vertices,
@@ -1181,11 +1193,16 @@ extern "C" int tg_render_backward_pooled(const real *grad_image, const real *gra
     const OrderStore order{const_cast<uint16_t *>(order_pool), n_triangles > kShortList ? n_keys * pixels : 0, pixels};
     return render_backward(grad_image, grad_depthmap, vertices, indices, colors, opacities, sorted_ids, offsets, bary, image, depthmap,
                            final_weights, ends, last, nullptr, order, nullptr, width, height, tile_w, tile_h, early_stopping_threshold,
-                           1, max_layers, grad_vertices, grad_colors, grad_opacities, vertex_stride, color_stride, opacity_stride, nullptr, n_keys, stream);
+                           1, max_layers, grad_vertices, grad_colors, grad_opacities, vertex_stride, color_stride, opacity_stride, 0, nullptr, n_keys, stream);
 }
 
 extern "C" int tg_split_gradient_block(const real *block, int64_t n_vertices, real *grad_vertices, real *grad_colors,
                                        real *grad_opacities, void *stream) {
+    return split_gradient_block(block, n_vertices, 1, grad_vertices, grad_colors, grad_opacities, stream);
+}
+
+int tg::split_gradient_block(const real *block, int64_t n_vertices, int copies, real *grad_vertices, real *grad_colors, real *grad_opacities,
+                             void *stream) {
     if (n_vertices < 0 || n_vertices > (int64_t)0x7fffffff * 256) {
         set_error("tg_split_gradient_block: n_vertices out of range");
         return TG_E_ARG;
@@ -1200,6 +1217,6 @@ extern "C" int tg_split_gradient_block(const real *block, int64_t n_vertices, re
         return TG_E_ARG;
     }
     TG_LAUNCH(split_gradient_block_kernel, dim3((unsigned)ceil_div64(n_vertices, 256)), dim3(256), 0, (hipStream_t)stream,
-              (const real4 *)block, n_vertices, (real4 *)grad_vertices, grad_colors, grad_opacities);
+              (const real4 *)block, n_vertices, copies, (real4 *)grad_vertices, grad_colors, grad_opacities);
     return check_launch("split_gradient_block_kernel");
 }

@@ -14,6 +14,7 @@
 #include <chrono>
 
 #include "tg_frame.hpp"
+#include "tg_gradient_copies.hpp"
 
 namespace tg {
 
@@ -233,17 +234,29 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
     // One zero fill for the three gradients.  Where there are many vertices, or many waves meet in one, the eight gradients of a vertex lie
     // in a 32-byte sector of a (V,8) block while the kernel runs, and the three arrays are copied out afterwards: the atomics of a run
     // then fall into three sectors and not nine.  The copy is another launch, and sums of few vertices stay in the L2 whatever their
-    // places, so not for the smallest images, and in tile order, with less than half the atomics, only where vertices are many or
-    // triangles share them.  Kernels, us, dense and by the block with the copy.  Tile order, a soup of 3 * 10^6 vertices 577, 360 + 28,
+    // places, so not for the smallest images, and in tile order, with less than half the atomics, only where triangles share vertices or
+    // vertices are many and the image is large.  Kernels, us, dense and by the block with the copy.  Tile order, a soup of 3 * 10^6 vertices 577, 360 + 28,
     // 3 * 10^5 82, 68 + 6, 9 * 10^4 36.2, 31.7 + 4.8, 5 * 10^4 with a heavy tail 375, 319 + 5, 3 * 10^4 18.8, 18.4 + 2.9; a mesh of
     // 650 000 on 1920 x 1080 440, 310 + 8, 28 000 on 1235 x 981 91, 62 + 5, 1200 there 124, 58 + 5, 5000 on 500 x 400 26, 23 + 2.4,
     // on 256 x 256 24.4, 22.4 + 2.4.  Per-pixel order, a soup of 9 * 10^4 43.8, 36.3 + 4.7, of 1500 with a heavy tail on 256 x 256
     // 98, 92.5 + 4.6, 300 on 128 x 128 38.9, 35.3 + 3.5, 60 on 50 x 50 10.2, 10.1 + 1.4; a mesh of 1200 on 1235 x 981 137, 67 + 5.
-    const bool by_block = f->block && ((uintptr_t)f->block & 15) == 0 && tg_sums_in_block(V, f->n_triangles, f->width, f->height, f->per_pixel_sort != 0);
-    real *sums = by_block ? f->block : f->gradients;
-    TG_LAUNCH(zero_gradients_kernel, dim3((unsigned)ceil_div64(2 * V, 256)), dim3(256), 0, (hipStream_t)f->stream, (real4 *)sums, 2 * V);
+    // A sector that several XCDs add to goes from L2 to L2, and triangles that cover hundreds of tiles are in all of them.  So each XCD
+    // has a block of its own where triangles are in 24 waves on average (with more vertices than 131072, or than a quarter of the pixels,
+    // the zeros and the copy, 512 bytes a vertex, cost what it gains).  Whole frames, us, one block and eight: heavy tails on 1100 x 1000 to 1230 x 1080, 1291
+    // triangles in per-pixel order 381, 213, 15 800 617, 481, 30 000 728, 514, 2072 in tile order 400, 204, 15 800 436, 296; no
+    // heavy tail, 20 000 large ones 988, 989, 3000 on 1024 x 1024 130, 131.  Below the line: 60 000 with a heavy tail 550, 563,
+    // 33 331 in tiles of 8 x 8 273, 278, a mesh of 20 000 124, 127.
+    const bool copies_fit = f->phases & TG_FRAME_GRADIENT_COPIES;
+    const int copies = copies_fit ? gradient_copies(*f) : f->per_pixel_sort ? 1 : 0;
+    if (copies && (!f->block || ((uintptr_t)f->block & 15))) {
+        set_error("tg_frame_backward: null or misaligned block");
+        return TG_E_ARG;
+    }
+    real *sums = copies ? f->block : f->gradients;
+    const int64_t n4 = 2 * V * max(copies, 1);
+    TG_LAUNCH(zero_gradients_kernel, dim3((unsigned)ceil_div64(n4, 256)), dim3(256), 0, (hipStream_t)f->stream, (real4 *)sums, n4);
     if (int e = check_launch("zero_gradients_kernel")) return e;
-    const int stride = by_block ? 8 : 0;
+    const int stride = copies ? 8 : 0;
     if (int e = render_backward(f->grad_image, f->grad_depthmap, f->vertices, f->indices, f->colors, f->opacities,
                                 (const int32_t *)(kept + L.ids), (const int32_t *)(kept + L.offsets), (const real *)(kept + L.bary), f->image,
                                 f->depthmap, (const real *)(kept + L.weights), (const int32_t *)(kept + L.ends),
@@ -251,13 +264,15 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
                                 frame_order(*f, L, kept), (f->flags & TG_FRAME_HIT_MASKS) ? (const uint64_t *)(kept + L.masks) : nullptr,
                                 (int)f->width, (int)f->height, (int)f->tile_w, (int)f->tile_h, (real)f->early_stopping_threshold,
                                 (int)f->per_pixel_sort, (int)f->max_layers, sums, stride ? sums + 4 : sums + 4 * V,
-                                stride ? sums + 7 : sums + 7 * V, stride ? stride : 4, stride ? stride : 3, stride ? stride : 1,
+                                stride ? sums + 7 : sums + 7 * V, stride ? stride : 4, stride ? stride : 3, stride ? stride : 1, copies > 1 ? 8 * V : 0,
                                 (const uint32_t *)(kept + L.status), f->key_capacity, f->stream))
         return e;
-    if (!by_block) return 0;
-    return tg_split_gradient_block(f->block, V, f->gradients, f->gradients + 4 * V, f->gradients + 7 * V, f->stream);
+    if (!copies) return 0;
+    return split_gradient_block(f->block, V, copies, f->gradients, f->gradients + 4 * V, f->gradients + 7 * V, f->stream);
 }
 #endif
+
+extern "C" int tg_frame_gradient_copies(const tg_frame *f) { return f ? gradient_copies(*f) : 0; }
 
 extern "C" int tg_frame_wait(const uint32_t *host, int word, uint32_t pending, void *stream) {
     if (!host || word < 0 || word > 3) {

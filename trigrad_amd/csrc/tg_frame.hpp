@@ -53,8 +53,10 @@ int render_backward(const real *grad_image, const real *grad_depthmap, const rea
                     const real *depthmap, const real *final_weights, const int32_t *ends, const int32_t *last, const real *last_depth,
                     const OrderStore &order, const uint64_t *hit_masks, int width, int height, int tile_w, int tile_h,
                     real early_stopping_threshold, int per_pixel_sort, int max_layers, real *grad_vertices, real *grad_colors,
-                    real *grad_opacities, int vertex_stride, int color_stride, int opacity_stride, const uint32_t *list_status,
-                    int64_t n_keys, void *stream);  // n_keys: about how many, for what does not have to be right; 0 if it is not known
+                    real *grad_opacities, int vertex_stride, int color_stride, int opacity_stride, int64_t copy_stride,
+                    const uint32_t *list_status, int64_t n_keys, void *stream);  // n_keys: about how many, for what does not have to be right; 0 if it is not known
+// The three arrays out of `copies` (V,8) blocks behind each other: their sum.
+int split_gradient_block(const real *block, int64_t n_vertices, int copies, real *grad_vertices, real *grad_colors, real *grad_opacities, void *stream);
 bool frame_grid_fits(int tiles_x, int tiles_y);  // at most 256 tile columns and rows: the sort passes are the tile's coordinates
 
 }  // namespace tg

@@ -29,7 +29,7 @@
 #include <memory>
 #include <mutex>
 
-#include "../../include/trigrad_hip.h"
+#include "tg_gradient_copies.hpp"
 
 namespace {
 
@@ -227,8 +227,9 @@ struct Render : torch::autograd::Function<Render> {
         const at::Tensor gradients = at::empty({8 * n}, on(v, at::kFloat));  // (V,4) | (V,3) | (V,) behind each other
         tg_frame f;
         frame.plan->fill(f, n, i.size(0), frame.max_layers);
-        const bool by_block = tg_sums_in_block(n, f.n_triangles, f.width, f.height, f.per_pixel_sort != 0);
-        const at::Tensor block = by_block ? at::empty({8 * n}, on(v, at::kFloat)) : gradients;
+        f.phases = TG_FRAME_GRADIENT_COPIES;
+        const int copies = tg::gradient_copies(f);
+        const at::Tensor block = copies ? at::empty({copies * 8 * n}, on(v, at::kFloat)) : gradients;
         f.vertices = v.data_ptr<float>();
         f.indices = i.data_ptr<int32_t>();
         f.colors = c.data_ptr<float>();
