@@ -1518,22 +1518,24 @@ def test_gradients_where_the_depth_map_has_none(w, mode, cuda):
 
 
 @pytest.mark.parametrize("width,height,tw,th", [(513, 512, 16, 16), (512, 512, 16, 16), (478, 480, 16, 16), (500, 452, 16, 16), (448, 512, 16, 16),
-                                                (509, 511, 32, 8), (505, 497, 8, 8), (411, 403, 12, 20)])
-@pytest.mark.parametrize("layers", [32, 40])
+                                                (509, 511, 32, 8), (505, 497, 8, 8), (411, 403, 12, 20), (256, 192, 16, 16), (257, 190, 16, 16)])
+@pytest.mark.parametrize("layers", [32, 40, None])
 def test_gradients_by_waves_alone_and_in_fours(width, height, tw, th, layers, cuda, oracle):
-    """The saved-order backward kernel runs a wave to a workgroup, or four where the frame's waves (ceil(tile / 64) a tile) are 3585 to
-    4096: numbers of waves on both sides of either edge, tiles of one, two and four waves, numbers of tiles that are no multiple of eight."""
+    """The backward kernels run a wave to a workgroup, or four where the frame's waves (ceil(tile / 64) a tile) fill the chip's SIMDs up to
+    four times, the last time to more than three quarters (769 to 1024, 1793 to 2048, ... 4096 waves): numbers of waves on both sides,
+    tiles of one, two and four waves, numbers of tiles that are no multiple of eight; tile order where layers is None."""
     import torch
     import scenes as S
     import trigrad_amd
-    scene = S.random_soup(1500, width, height, seed=width + layers, sigma_px=14.0, opacity=(0.1, 0.6), varying_w=True)
-    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256, True, layers)
+    scene = S.random_soup(1500, width, height, seed=width + (layers or 0), sigma_px=14.0, opacity=(0.1, 0.6), varying_w=True)
+    order, limit = layers is not None, layers or 1501
+    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256, order, limit)
     gi, gd = _grad_inputs(scene, 4, False)
     wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height,
-                                    tw, th, True, layers, literal=False, magnitudes=True)
+                                    tw, th, order, limit, literal=False, magnitudes=True)
     d = to_device(scene, cuda)
     leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
-    image, _ = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, tw, th, max_layers=layers)
+    image, _ = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, tw, th, per_pixel_sort=order, max_layers=limit)
     out = torch.autograd.grad(image, leaves, torch.from_numpy(gi).to(cuda))
     for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
         assert_gradients_close(f"{width}x{height}, tiles of {tw}x{th}, {layers} layers: {label}", g.cpu().numpy(), w, mag)

@@ -1082,15 +1082,16 @@ size_t backward_pixel_order_lds_bytes(int n_threads) { return pixel_order_lds_by
 
 using namespace tg;
 
-// Waves of a workgroup of the saved-order kernel.  One, but for a frame whose waves fill the chip once, four for each of its 1024
-// SIMDs (3584 to 4096; 512 x 512 pixels): single waves go five to one SIMD and three to the next, those of a workgroup of four one to
-// each.  200 000 large triangles on 512 x 512: 248 us singly, 231 in fours, 20 000 without a limit on the layers 560 and 551; on
-// 480 x 480 239, 231 and 576, 596.  With fewer waves there is room for all (448 x 448: 222, 228), with more the next one takes the
-// place (528 x 528: 259, 262 and 571, 604).
+// Waves of a workgroup of the tile-order and the saved-order kernel.  One, but for a frame whose waves all run at once (4096 at most, four
+// for each of 1024 SIMDs) and fill a last layer of the SIMDs to more than three quarters: single waves go two to one SIMD and none to the
+// next, those of a workgroup of four one to each, which counts where it makes the layers one less.  us, singly and in fours, saved
+// order (with a gradient of the depth): 512 x 512 pixels (4096 waves) 248, 231 and 560, 551, 376 x 309 (1920) 230, 217 (251, 234), 256 x 256
+// (1024) 430, 421 (484, 462); tile order, 512 x 512 232, 224, 256 x 256 109, 104.  Else: 448 x 448 (3136) 222, 228, 480 x 480 (3600)
+// 239, 231 and 576, 596, 362 x 362 (2116) 503, 520 (563, 581), 300 x 300 (1444) 168, 171, 528 x 528 (4356) 259, 262 and 571, 604.
 static int workgroup_waves(int width, int height, int tile_w, int tile_h) {
-    constexpr int64_t kChipWaves = 4 * 1024;
+    constexpr int64_t kSimds = 1024;
     const int64_t waves = (int64_t)ceil_div(width, tile_w) * ceil_div(height, tile_h) * ceil_div(tile_w * tile_h, kWave);
-    return waves > kChipWaves / 8 * 7 && waves <= kChipWaves ? kMaxWaves : 1;
+    return waves <= 4 * kSimds && (waves - 1) % kSimds >= kSimds / 4 * 3 ? kMaxWaves : 1;
 }
 
 int tg::render_backward(const real *grad_image, const real *grad_depthmap, const real *vertices,
