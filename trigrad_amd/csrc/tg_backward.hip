@@ -465,12 +465,13 @@ __device__ __forceinline__ TermLane term_lane(const BackwardArgs &g, int lane) {
 // Adds up the runs of equal list entry among the first n slots of a wave's term matrix (row q = term
 // q, rows kTermStride apart; slots of one entry are neighbours) and adds every non-zero run sum to the
 // gradient arrays.  Bit c of `heads` is set where slot c starts a run.  Lane (group, q) owns a fixed third of
-// row q -- slots [0, 22), [22, 44) or [44, 64) -- and turns it into running sums that start over at each head:
+// row q -- slots [0, 21), [21, 42) or [42, 64) -- and turns it into running sums that start over at each head:
 // straight-line code, no branch, no look at the entries; slots from n on hold what an earlier round left, which
 // a running sum carries to later slots only, never into a slot below n.  The last slot of a run, and of a third,
 // then holds a sum to deliver, and every lane walks the ones of its own third.  vertex_at(c, v): vertex id v of
 // the entry in slot c.
-constexpr int kRunSpan = 22;  // slots of a third (the last one has kWave - 2 * kRunSpan = 20)
+// (21, 21 and 22 and not the other way round: the 63 lanes' elements, in banks q + c0 + k, are then 63 banks.)
+constexpr int kRunSpan = 21, kLastSpan = kWave - 2 * kRunSpan;
 // Bit k of x as a mask, all ones or 0.  (The compiler is not to know that: it makes a comparison and a selection of a mask, three
 // operations and a wait for one.)
 __device__ __forceinline__ int bit_mask(int x, int k) {
@@ -486,23 +487,23 @@ __device__ __forceinline__ void add_run_sums(real *terms, int n, uint64_t heads,
     if (t.group >= 3) return;  // the one lane left over; nothing below synchronises the wave
     const int c0 = t.group * kRunSpan;
     real *row = terms + t.q * kTermStride + c0;
-    const bool full = t.group < 2;  // a third of kRunSpan slots
+    const bool last = t.group == 2;  // the third of kLastSpan slots
     {
         const int carries = (int)~(uint32_t)(heads >> c0);  // bit k: slot k goes on with the run of the slot before it
-        real v[kRunSpan];
+        real v[kLastSpan];
 #pragma unroll
-        for (int k = 0; k < kRunSpan; k++) v[k] = (k < kWave - 2 * kRunSpan || full) ? row[k] : 0.0f;
+        for (int k = 0; k < kLastSpan; k++) v[k] = (k < kRunSpan || last) ? row[k] : 0.0f;
         real sum = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kRunSpan; k++) {
+        for (int k = 0; k < kLastSpan; k++) {
             sum = v[k] + masked(sum, bit_mask(carries, k));
-            if (k < kWave - 2 * kRunSpan || full) row[k] = sum;
+            if (k < kRunSpan || last) row[k] = sum;
         }
     }
     // what a lane reads below it wrote itself above: LDS serves a wave's instructions in order
     uint64_t tails = (heads >> 1) | (1ull << (n - 1)) | (1ull << (kRunSpan - 1)) | (1ull << (2 * kRunSpan - 1));
     if (n < kWave) tails &= (1ull << n) - 1;
-    uint32_t mine = (uint32_t)(tails >> c0) & ((1u << (full ? kRunSpan : kWave - 2 * kRunSpan)) - 1);
+    uint32_t mine = (uint32_t)(tails >> c0) & ((1u << (last ? kLastSpan : kRunSpan)) - 1);
     while (mine) {
         // two slots per turn, so that two chains of LDS reads are in flight
         const int k0 = __builtin_ctz(mine);
