@@ -281,6 +281,12 @@ def test_sort_tile_lists_at_the_edges_of_its_rules(longest, cuda):
     np.testing.assert_array_equal(sv.cpu().numpy(), order.astype(np.int32))
 
 
+@pytest.mark.parametrize("longest", [384, 385, 448, 449, 768, 769, 3072, 3073, 5120, 5121, 6144, 6145, 9216, 9217])
+def test_sort_tile_lists_where_a_thread_has_a_pair_more(longest, cuda):
+    """The lengths at which the sorts of a list by a wave and by a workgroup go on to the next number of pairs a thread."""
+    test_sort_tile_lists_at_the_edges_of_its_rules(longest, cuda)
+
+
 @pytest.mark.parametrize("n_tiles,typical", [(2049, 1100), (2048, 1100), (2049, 500), (2049, 2060)])
 def test_sort_of_many_lists_around_the_workgroups_two_sizes(n_tiles, typical, cuda):
     """Most lists of 512 to 2048 pairs, in more than 2048 tiles: sorted by the small kernel up to 2048; else up to 1024."""

@@ -439,7 +439,6 @@ constexpr int kSegWaveCap = kWave * kSegWaveItemsMax;
 // way), none at all 6.4 -> 6.1.  16 pairs per thread spill, and a kernel that has scratch memory takes 4 us more to launch.
 constexpr int kSegLargeThreads = 1024;
 constexpr int kSegLargeItems = 10;
-constexpr int kSegLargeCap = kSegLargeThreads * kSegLargeItems;
 constexpr int kSegStreamItems = 8;                                 // chunk of the pass through memory
 constexpr int kSegLargeGrid = 256;
 
@@ -714,6 +713,7 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
         case 4: segment_sort_in_wave<4>(keys, vals, start, n, lds); break;
         case 5: segment_sort_in_wave<5>(keys, vals, start, n, lds); break;
         case 6: segment_sort_in_wave<6>(keys, vals, start, n, lds); break;
+        case 7: segment_sort_in_wave<7>(keys, vals, start, n, lds); break;
         default: segment_sort_in_wave<8>(keys, vals, start, n, lds); break;
         }
     }
@@ -723,7 +723,9 @@ __global__ __launch_bounds__(kSortThreads) void segment_sort_small_kernel(uint64
         const int len = bounds[w + 1] - bounds[w];
         if (len <= kSegWaveCap || len > medium_cap) continue;
         __syncthreads();  // the waves are done with their own buffers, the previous segment with the shared one
-        if (len <= kSortThreads * 4)
+        if (len <= kSortThreads * 3)
+            segment_sort_in_lds<kSortThreads, 3>(keys, vals, bounds[w], len, s.medium.lds, s.medium.ex_keys, s.medium.ex_vals);
+        else if (len <= kSortThreads * 4)
             segment_sort_in_lds<kSortThreads, 4>(keys, vals, bounds[w], len, s.medium.lds, s.medium.ex_keys, s.medium.ex_vals);
         else
             segment_sort_in_lds<kSortThreads, kSegMediumItems>(keys, vals, bounds[w], len, s.medium.lds, s.medium.ex_keys, s.medium.ex_vals);
@@ -816,11 +818,14 @@ __device__ void segment_sort_through_memory(uint64_t *keys, uint32_t *vals, uint
 }
 
 // Segments longer than medium_cap: few or none, so a workgroup looks through the lengths of its share of the
-// segments, one segment per thread at a time, and takes the long ones in turn.
+// segments, one segment per thread at a time, and takes the long ones in turn.  Its time is that of the pairs a thread has, padding
+// included, so nearly every number of them is an instance (both kernels, us, with 2, 4, 8 and 10 alone and so: 1024 lists around 3700
+// 109, 84; lists of 5200 to 5500 among short ones, 1.3 million triangles of a mesh 99, 89, half a million 77, 67).  Two workgroups a CU,
+// for lists of up to 6144 in 65 KB of LDS and 64 registers, gain 4 % on 1024 lists and lose 7 % on 2500, and are another launch.
 struct LargeSegLds {
     SegLds<kSegLargeThreads> lds;
     uint64_t votes[kSegLargeThreads / kWave];
-    uint32_t ex_keys[kSegLargeCap], ex_vals[kSegLargeCap];
+    uint32_t ex_keys[kSegLargeThreads * kSegLargeItems], ex_vals[kSegLargeThreads * kSegLargeItems];
 };
 __global__ __launch_bounds__(kSegLargeThreads) void segment_sort_large_kernel(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
                                                                              uint32_t *vals_alt, const int32_t *__restrict__ offsets,
@@ -845,16 +850,17 @@ __global__ __launch_bounds__(kSegLargeThreads) void segment_sort_large_kernel(ui
                 todo &= todo - 1;
                 const int64_t start = offsets[seg];
                 const int n = offsets[seg + 1] - offsets[seg];
-                if (n <= kSegLargeThreads * 2)
-                    segment_sort_in_lds<kSegLargeThreads, 2>(keys, vals, start, n, lds, ex_keys, ex_vals);
-                else if (n <= kSegLargeThreads * 4)
-                    segment_sort_in_lds<kSegLargeThreads, 4>(keys, vals, start, n, lds, ex_keys, ex_vals);
-                else if (n <= kSegLargeThreads * 8)
-                    segment_sort_in_lds<kSegLargeThreads, 8>(keys, vals, start, n, lds, ex_keys, ex_vals);
-                else if (n <= kSegLargeCap)
-                    segment_sort_in_lds<kSegLargeThreads, kSegLargeItems>(keys, vals, start, n, lds, ex_keys, ex_vals);
-                else
-                    segment_sort_through_memory(keys, vals, keys_alt, vals_alt, start, n, lds, ex_keys, ex_keys + kRadix);
+                switch ((n - 1) / kSegLargeThreads + 1) {  // pairs a thread
+                case 1: case 2: segment_sort_in_lds<kSegLargeThreads, 2>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                case 3: segment_sort_in_lds<kSegLargeThreads, 3>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                case 4: segment_sort_in_lds<kSegLargeThreads, 4>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                case 5: segment_sort_in_lds<kSegLargeThreads, 5>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                case 6: segment_sort_in_lds<kSegLargeThreads, 6>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                case 7: case 8: segment_sort_in_lds<kSegLargeThreads, 8>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                case 9: segment_sort_in_lds<kSegLargeThreads, 9>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                case kSegLargeItems: segment_sort_in_lds<kSegLargeThreads, kSegLargeItems>(keys, vals, start, n, lds, ex_keys, ex_vals); break;
+                default: segment_sort_through_memory(keys, vals, keys_alt, vals_alt, start, n, lds, ex_keys, ex_keys + kRadix);
+                }
                 __syncthreads();  // the next segment reuses the LDS
             }
         }
