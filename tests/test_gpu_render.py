@@ -184,6 +184,36 @@ def test_crowds_of_small_triangles_match_oracle(n, width, height, tw, th, mode, 
         assert np.array_equal(_shared_out(got, want, tw, th), long & (-(-tw * th // 64) >= 4))
 
 
+@pytest.mark.parametrize("shape", ["tiny", "sliver", "on_centres", "far_corner", "flat"])
+@pytest.mark.parametrize("width,height,tw,th", [(400, 304, 16, 16), (203, 101, 8, 8), (203, 101, 12, 10)])
+def test_triangles_beside_a_waves_pixels(shape, width, height, tw, th, cuda, oracle):
+    """Per-pixel order, batches of 64: a wave leaves out the entries whose vertices are all to one side of its pixels.  Triangles
+    whose edges alone say little of that, or whose matrix is the inverse of their vertices in a few bits only: the images are the
+    oracle's bit for bit."""
+    import scenes as S
+    n = 4000
+    scene = S.random_soup(n, width, height, seed=3, sigma_px=1.0 if shape == "tiny" else 4.0, opacity=(0.05, 0.9), varying_w=True)
+    rng = np.random.default_rng(len(shape))
+    v = scene["vertices"].reshape(n, 3, 4)
+    xy = v[:, :, :2].astype(np.float64)
+    if shape == "sliver":  # the third vertex on the line through the others but for 1e-9 to 1e-2
+        t = rng.uniform(0, 1, (n, 1))
+        xy[:, 2] = xy[:, 0] * (1 - t) + xy[:, 1] * t + 10 ** rng.uniform(-9, -2, (n, 1)) * rng.standard_normal((n, 2))
+    if shape == "on_centres":
+        size = np.array([width, height])
+        xy = (np.floor((xy + 1) / 2 * size) + 0.5) / size * 2 - 1
+    if shape == "far_corner":
+        xy[:, 0] *= 10 ** rng.uniform(0, 6, (n, 1))
+    if shape == "flat":  # two vertices, or all three, with the same x or y up to a few roundings
+        axis = rng.integers(0, 2, n)
+        for k in (1, 2):
+            xy[np.arange(n), k, axis] = xy[np.arange(n), 0, axis] + 1e-7 * rng.standard_normal(n) * (rng.random(n) < 0.8)
+    v[:, :, :2] = xy.astype(np.float32)
+    _, want, got, _ = _forward_both(scene, tw, th, MODES["A_default"], cuda, oracle, frames=2)
+    assert np.diff(want["offsets"]).mean() < 512  # no depth bounds
+    _check_forward(f"{shape}/{width}x{height}/{tw}x{th}", want, got, (th, tw))
+
+
 @pytest.mark.parametrize("mode", ["A_default", "B_unlimited"])
 @pytest.mark.parametrize("n,others,width,lane_by_lane", [(255, 0, 272, False), (256, 0, 272, True), (400, 28_000, 272, False),
                                                          (1023, 70_000, 272, False), (1024, 70_000, 272, True), (90, 0, 16, True),

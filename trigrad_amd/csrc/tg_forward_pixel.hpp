@@ -157,7 +157,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
         constexpr int kTurns = kTileThreads / kStage;
         const int group = kStage == kWave ? wave : tid / kStage, mine = tid & (kStage - 1);  // in turn: whose batch, which of its entries
         const bool ahead = !kInTurn && !a.batch_bounds && (int)blockDim.x >= kStage;
-        DepthParts next;
+        DepthParts<kStage == kWave> next;
         auto start_turns = [&](int first) {  // the records of the kTurns batches from list entry `first` on
             const int j = min(first + tid, end - 1);
             next.fetch_triangle(a, j);
@@ -198,7 +198,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 const int e = kInTurn ? mine : tid;
                 const DepthRecord r = next.record();
                 s_rec[e] = r;
-                s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves) | small_entry(a, r.extent, tests_small));
+                s_touch[e] = (uint8_t)(waves_touched(r.m, s_rects, n_waves, next.reach(r)) | small_entry(a, r.extent, tests_small));
             }
             if (!kInTurn && !ahead) {
                 for (int e = tid; e < nb; e += blockDim.x) {
@@ -423,7 +423,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
                 // a group of the list is 64 entries for each wave
                 const int group = waves * kWave, mine = lane * waves + wave;
                 const auto entry = [&](int first) { return min(start + first + mine, end - 1); };
-                DepthParts next;
+                DepthParts<false> next;
                 const auto fetch_from = [&](int first) {
                     next.fetch_triangle(a, entry(first));
                     next.fetch_matrix(a);
