@@ -174,14 +174,15 @@ def main():
     # through memory for the tile bits only (one pass by tile column, one by tile row) and sorts the depth bits per tile
     # in LDS (one more read and write of every pair).
     model_passes = (_C.key_bits(T) + 7) // 8
-    sweep_n, sweep_ms = prof["sort_sweep_kernel"]
+    sort_pass = "sort_sweep_kernel" if "sort_sweep_kernel" in prof else "sort_few_keys_kernel"  # a few thousand keys: one launch
+    sweep_n, sweep_ms = prof[sort_pass]
     sweep_avg_s = sweep_ms / sweep_n / 1000.0
     sweep_bytes = 24.0 * K
     achieved = sweep_bytes / sweep_avg_s / 1e9
     passes_through_memory = sweep_n // prof_steps
     per_step = {k: v[1] / prof_steps for k, v in prof.items()}
     # binning + sort + ranges: every kernel from the triangles to the sorted tile lists and their offsets
-    sort_kernels = ["fill_zero_kernel", "sort_histogram_kernel", "sort_bases_kernel", "sort_sweep_kernel", "tile_ranges_kernel",
+    sort_kernels = ["fill_zero_kernel", "sort_histogram_kernel", "sort_bases_kernel", "sort_sweep_kernel", "sort_few_keys_kernel", "tile_ranges_kernel",
                     "segment_sort_small_kernel", "segment_sort_large_kernel"]
     bin_sort_kernels = ["bin_count_kernel", "scan_init_kernel", "scan_lookback_kernel", "bin_emit_kernel", "bin_init_kernel",
                         "bin_setup_kernel", "bin_emit_records_kernel", "frame_scan_kernel", "frame_emit_kernel"] + sort_kernels
@@ -212,7 +213,7 @@ def main():
         "config": {"workload": f"config{args.config}: {M} triangles, {W}x{H}, 16x16 tiles, K={K} keys, "
                                f"per_pixel_sort={MODES[args.mode]['per_pixel_sort']}, max_layers={MODES[args.mode]['max_layers']}",
                    "mode": args.mode},
-        "roofline": {"bound": "hbm", "kernel": "sort_sweep_kernel", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+        "roofline": {"bound": "hbm", "kernel": sort_pass, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": traffic_source,
                      "bytes_per_launch": sweep_bytes, "avg_launch_us": sweep_avg_s * 1e6},
     }
