@@ -30,7 +30,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
     int last = 0;
     // an entry's matrix and vertex numbers are asked for while the entries before it are composited, its triangle's number
     // before that; what only the entries that are hit need is read when it is known which they are
-    DepthParts<false> next;
+    DepthParts next;
     const auto entry = [&](int first) { return min(first + tid, end - 1); };
     next.fetch_triangle(a, entry(start));
     next.fetch_matrix(a);

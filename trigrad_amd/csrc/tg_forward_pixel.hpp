@@ -157,7 +157,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
         constexpr int kTurns = kTileThreads / kStage;
         const int group = kStage == kWave ? wave : tid / kStage, mine = tid & (kStage - 1);  // in turn: whose batch, which of its entries
         const bool ahead = !kInTurn && !a.batch_bounds && (int)blockDim.x >= kStage;
-        DepthParts<kStage == kWave> next;
+        std::conditional_t<kStage == kWave, PlacedParts, DepthParts> next;
         auto start_turns = [&](int first) {  // the records of the kTurns batches from list entry `first` on
             const int j = min(first + tid, end - 1);
             next.fetch_triangle(a, j);
@@ -423,7 +423,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
                 // a group of the list is 64 entries for each wave
                 const int group = waves * kWave, mine = lane * waves + wave;
                 const auto entry = [&](int first) { return min(start + first + mine, end - 1); };
-                DepthParts<false> next;
+                DepthParts next;
                 const auto fetch_from = [&](int first) {
                     next.fetch_triangle(a, entry(first));
                     next.fetch_matrix(a);

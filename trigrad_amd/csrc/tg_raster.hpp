@@ -298,15 +298,12 @@ __device__ __forceinline__ V read_three(const T *p) {
     __builtin_memcpy(&v, p, 3 * sizeof(T));
     return v;
 }
-template <bool kWithX>
 struct DepthParts {
-    using Vertex = std::conditional_t<kWithX, real4v, real3v>;  // its last components
-    static constexpr int kY = kWithX;
     int tri;
     int3v id;
     real4v m0, m1;
     real m2;
-    Vertex va, vb, vc;
+    real3v va, vb, vc;  // y, z, w of the vertices
 
     __device__ __forceinline__ void fetch_triangle(const RasterArgs &a, int j) { tri = a.sorted_ids[j]; }
     // the triangle's vertex numbers and matrix
@@ -319,32 +316,42 @@ struct DepthParts {
         m2 = m->c;
     }
     __device__ __forceinline__ void fetch_vertices(const RasterArgs &a) {
-        if constexpr (kWithX) {
-            const real4v *v = reinterpret_cast<const real4v *>(a.vertices);
-            va = v[id.x];
-            vb = v[id.y];
-            vc = v[id.z];
-        } else {
-            const real *v = reinterpret_cast<const real *>(a.vertices) + 1;
-            va = read_three<real3v>(v + 4 * (int64_t)id.x);
-            vb = read_three<real3v>(v + 4 * (int64_t)id.y);
-            vc = read_three<real3v>(v + 4 * (int64_t)id.z);
-        }
+        const real *v = reinterpret_cast<const real *>(a.vertices) + 1;
+        va = read_three<real3v>(v + 4 * (int64_t)id.x);
+        vb = read_three<real3v>(v + 4 * (int64_t)id.y);
+        vc = read_three<real3v>(v + 4 * (int64_t)id.z);
     }
     __device__ __forceinline__ DepthRecord record() const {
         DepthRecord r;
 #pragma unroll
         for (int k = 0; k < 4; k++) { r.m[k] = m0[k]; r.m[4 + k] = m1[k]; }
         r.m[8] = m2;
-        r.z[0] = va[kY + 1]; r.z[1] = vb[kY + 1]; r.z[2] = vc[kY + 1];
-        r.w[0] = va[kY + 2]; r.w[1] = vb[kY + 2]; r.w[2] = vc[kY + 2];
-        r.extent = max3(va[kY], vb[kY], vc[kY]) - min3(va[kY], vb[kY], vc[kY]);
+        r.z[0] = va[1]; r.z[1] = vb[1]; r.z[2] = vc[1];
+        r.w[0] = va[2]; r.w[1] = vb[2]; r.w[2] = vc[2];
+        r.extent = max3(va[0], vb[0], vc[0]) - min3(va[0], vb[0], vc[0]);
         return r;
     }
-    __device__ __forceinline__ Reach reach(const DepthRecord &r) const {
-        if constexpr (kWithX) return triangle_reach(r.m, va[0], va[1], vb[0], vb[1], vc[0], vc[1]);
-        return reaches_everywhere();
+    __device__ __forceinline__ Reach reach(const DepthRecord &) const { return reaches_everywhere(); }
+};
+// The same with x of the vertices: whole vertices, from 16-byte boundaries in both precisions.
+struct __attribute__((packed, aligned(16))) Vertex4 { real4v v; };
+struct PlacedParts : DepthParts {
+    real4v pa, pb, pc;
+
+    __device__ __forceinline__ void fetch_vertices(const RasterArgs &a) {
+        const Vertex4 *v = reinterpret_cast<const Vertex4 *>(a.vertices);
+        pa = v[id.x].v;
+        pb = v[id.y].v;
+        pc = v[id.z].v;
     }
+    __device__ __forceinline__ DepthRecord record() const {
+        DepthParts d = *this;
+        d.va = pa.yzw;
+        d.vb = pb.yzw;
+        d.vc = pc.yzw;
+        return d.record();
+    }
+    __device__ __forceinline__ Reach reach(const DepthRecord &r) const { return triangle_reach(r.m, pa.x, pa.y, pb.x, pb.y, pc.x, pc.y); }
 };
 
 // Saved hit masks (tile order).  The buffer starts with one word per workgroup of the tile launch
