@@ -424,7 +424,7 @@ typedef struct tg_frame {
     const tg_real *grad_depthmap;
     tg_real *gradients;
     tg_real *block;
-    int64_t n_keys;  /* out */
+    int64_t n_keys;  /* out of the forward call; in the backward call: how many the frame has (tg_frame_gradient_copies) */
     int64_t counted; /* out */
     int64_t n_vertices;
     int64_t n_triangles;
@@ -443,7 +443,8 @@ typedef struct tg_frame {
 
 #define TG_FRAME_GRADIENT_COPIES 256
 /* How many (V,8) blocks a frame's gradients are summed in before they are copied out: 0, they are summed in place; 1, a vertex's
- * eight in one 32-byte sector; or 8, one for each XCD, where its triangles are in many tiles each. */
+ * eight in one 32-byte sector; or 8, one for each XCD, where its triangles are in many tiles each (n_keys, as in the backward call; 0,
+ * not known, is never 8). */
 int tg_frame_gradient_copies(const tg_frame *f);
 
 #define TG_FRAME_BACKWARD 1     /* flags: a backward pass will follow: save what it needs */

@@ -280,6 +280,20 @@ def test_buffers_for_a_rounded_number_of_triangles_serve_every_smaller_one(flags
                 assert getattr(sizes[0], field) <= getattr(sizes[1], field)
 
 
+@pytest.mark.parametrize("n_triangles,n_keys,tile,tile_order,pixel_order", [
+    (20, 25, 16, 0, 1), (341, 450, 16, 0, 1), (300, 1499, 16, 0, 1), (300, 1500, 16, 8, 8), (300, 5999, 8, 0, 1), (300, 6000, 8, 8, 8)])
+def test_a_gradient_block_for_each_xcd_by_the_keys_a_frame_has(n_triangles, n_keys, tile, tile_order, pixel_order):
+    """Eight blocks where a triangle is in 20 waves on average, of the keys that were counted: the key buffers have room for
+    more, a first frame's for 65536 more and those that an earlier frame's plan has for any number."""
+    from trigrad_amd import _C, _lib
+    for capacity in (_C._round_capacity(n_keys), 3 * n_triangles + 65536, 1 << 18):
+        for per_pixel_sort, expected in ((0, tile_order), (1, pixel_order)):
+            flags = _C._FRAME_BACKWARD | (_C._FRAME_ORDER_PLANES if per_pixel_sort else _C._FRAME_HIT_MASKS)
+            frame = bytes(_C._FRAME_CALL.size) + _C._FRAME_RESULT.pack(n_keys, 1) + _C._FRAME_KIND.pack(
+                3 * n_triangles, n_triangles, 256, 256, tile, tile, per_pixel_sort, 32, capacity, flags, 0, 0, 0.0)
+            assert _lib.load(32).tg_frame_gradient_copies(frame) == expected
+
+
 @pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
 def test_state_words_of_the_frame_scan_keep_their_place(few, many):
     """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more

@@ -1643,7 +1643,7 @@ def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height
     (150, 20.0, 150, 121, 16, 16, True), (150, 20.0, 128, 128, 16, 16, False), (1512, 20.0, 150, 121, 16, 16, True), (1513, 20.0, 150, 121, 16, 16, False), (400, 30.0, 200, 131, 8, 8, True), (400, 4.0, 200, 131, 8, 8, False),
     (60, 50.0, 160, 160, 32, 32, True)])
 def test_gradients_summed_by_xcds(n, sigma, width, height, tw, th, per_waves, mode, cuda, oracle):
-    """Where triangles are in 24 waves on average each XCD sums the gradients in a block of its own: on both sides of the line, by a first
+    """Where triangles are in 20 waves on average each XCD sums the gradients in a block of its own: on both sides of the line, by a first
     frame (the Python route) and by ones whose plan is there (the module's)."""
     import torch
     import scenes as S
@@ -1654,9 +1654,9 @@ def test_gradients_summed_by_xcds(n, sigma, width, height, tw, th, per_waves, mo
     ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
     want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256,
                          m["per_pixel_sort"], ml)
-    capacity = _C._round_capacity(int(want["offsets"][-1]))
-    kind = _C._FRAME_KIND.pack(3 * n, n, width, height, tw, th, m["per_pixel_sort"], ml, capacity, 0, 0, 0, 0.0)
-    assert (_C._gradient_copies(_lib.load(32), kind) == 8) == per_waves
+    keys = int(want["offsets"][-1])
+    kind = _C._FRAME_KIND.pack(3 * n, n, width, height, tw, th, m["per_pixel_sort"], ml, _C._round_capacity(keys), 0, 0, 0, 0.0)
+    assert (_C._gradient_copies(_lib.load(32), kind, keys) == 8) == per_waves
     gi, gd = _grad_inputs(scene, 9, True)
     wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, tw, th,
                                     m["per_pixel_sort"], ml, literal=False, magnitudes=True)

@@ -901,9 +901,10 @@ def _frame_launches(index, stream):
 _FRAME_GRADIENT_COPIES = 256  # TG_FRAME_GRADIENT_COPIES of the C header
 
 
-def _gradient_copies(lib, kind):
-    """How many (V,8) blocks the gradients of a frame of a kind (packed) are summed in; 0: they are summed in place."""
-    return lib.tg_frame_gradient_copies(bytes(_FRAME_CALL.size + _FRAME_RESULT.size) + kind)
+def _gradient_copies(lib, kind, n_keys=0):
+    """How many (V,8) blocks the gradients of a frame of a kind (packed) with n_keys keys (0: not known) are summed in; 0: they
+    are summed in place."""
+    return lib.tg_frame_gradient_copies(bytes(_FRAME_CALL.size) + _FRAME_RESULT.pack(n_keys, 0) + kind)
 
 
 def frame_backward(frame, grad_image, grad_depthmap, vertices, indices, colors, opacities, image, depthmap, kept):
@@ -919,7 +920,7 @@ def frame_backward(frame, grad_image, grad_depthmap, vertices, indices, colors, 
         if grad_depthmap is not None:
             grad_depthmap = grad_depthmap.contiguous()
         gradients = torch.empty((8 * n_vertices,), dtype=torch.float32, device=dev)
-        copies = _gradient_copies(lib, plan.kind)
+        copies = _gradient_copies(lib, plan.kind, frame.n_keys)
         block = torch.empty((copies * 8 * n_vertices,), dtype=torch.float32, device=dev) if copies else gradients
         call = bytearray(_FRAME_BYTES)
         call[-_FRAME_KIND.size:] = plan.kind
@@ -927,6 +928,7 @@ def frame_backward(frame, grad_image, grad_depthmap, vertices, indices, colors, 
                               depthmap.data_ptr(), kept.data_ptr(), 0, 0, 0, _raw_stream(dev), 0, 0, _FRAME_GRADIENT_COPIES, grad_image.data_ptr(),
                               0 if grad_depthmap is None else grad_depthmap.data_ptr(), gradients.data_ptr(),
                               block.data_ptr())
+        _FRAME_RESULT.pack_into(call, _FRAME_CALL.size, frame.n_keys, 0)
         code = lib.tg_frame_backward((C.c_char * _FRAME_BYTES).from_buffer(call))
         if code:
             _lib.check(code, "tg_frame_backward")

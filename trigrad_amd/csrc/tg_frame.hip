@@ -241,11 +241,13 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
     // on 256 x 256 24.4, 22.4 + 2.4.  Per-pixel order, a soup of 9 * 10^4 43.8, 36.3 + 4.7, of 1500 with a heavy tail on 256 x 256
     // 98, 92.5 + 4.6, 300 on 128 x 128 38.9, 35.3 + 3.5, 60 on 50 x 50 10.2, 10.1 + 1.4; a mesh of 1200 on 1235 x 981 137, 67 + 5.
     // A sector that several XCDs add to goes from L2 to L2, and triangles that cover hundreds of tiles are in all of them.  So each XCD
-    // has a block of its own where triangles are in 24 waves on average (with more vertices than 131072, or than a quarter of the pixels,
-    // the zeros and the copy, 512 bytes a vertex, cost what it gains).  Whole frames, us, one block and eight: heavy tails on 1100 x 1000 to 1230 x 1080, 1291
+    // has a block of its own where triangles are in 20 waves on average, a tile counted as all of its waves (with more vertices than 131072,
+    // or than a quarter of the pixels, the zeros and the copy, 512 bytes a vertex, cost what it gains).  Whole frames, us, one block and eight: heavy tails on 1100 x 1000 to 1230 x 1080, 1291
     // triangles in per-pixel order 381, 213, 15 800 617, 481, 30 000 728, 514, 2072 in tile order 400, 204, 15 800 436, 296; no
     // heavy tail, 20 000 large ones 988, 989, 3000 on 1024 x 1024 130, 131.  Below the line: 60 000 with a heavy tail 550, 563,
-    // 33 331 in tiles of 8 x 8 273, 278, a mesh of 20 000 124, 127.
+    // 33 331 in tiles of 8 x 8 273, 278, a mesh of 20 000 124, 127.  The backward pass alone near it, all of one size: 20 000 on
+    // 1024 x 1024, 15 waves a triangle 63, 71, 21 waves 93, 102; 1000 there, 16 waves 22, 24, 300 on 256 x 256, 20 waves 19.3, 21.4; in tile order
+    // 75, 84 (21 waves), 15.6, 19.2 (20); with a heavy tail, which their mean does not tell, 1500 on 256 x 256, 25 waves 66, 64 and 40, 35.
     const bool copies_fit = f->phases & TG_FRAME_GRADIENT_COPIES;
     const int copies = copies_fit ? gradient_copies(*f) : f->per_pixel_sort ? 1 : 0;
     if (copies && (!f->block || ((uintptr_t)f->block & 15))) {

@@ -228,6 +228,7 @@ struct Render : torch::autograd::Function<Render> {
         tg_frame f;
         frame.plan->fill(f, n, i.size(0), frame.max_layers);
         f.phases = TG_FRAME_GRADIENT_COPIES;
+        f.n_keys = frame.n_keys;
         const int copies = tg::gradient_copies(f);
         const at::Tensor block = copies ? at::empty({copies * 8 * n}, on(v, at::kFloat)) : gradients;
         f.vertices = v.data_ptr<float>();
