@@ -294,6 +294,15 @@ def test_a_gradient_block_for_each_xcd_by_the_keys_a_frame_has(n_triangles, n_ke
             assert _lib.load(32).tg_frame_gradient_copies(frame) == expected
 
 
+@pytest.mark.parametrize("flags,per_pixel_sort,expected", [(1, 1, 1), (1 | 2, 1, 8), (1 | 4, 1, 8), (1 | 4 | 16, 1, 8), (1, 0, 8), (1 | 8, 0, 8)])
+def test_gradient_blocks_for_the_kernels_that_use_them(flags, per_pixel_sort, expected):
+    """The backward kernel for frames without a saved blend order adds to the first block whatever its XCD: there is one."""
+    from trigrad_amd import _C, _lib
+    frame = bytes(_C._FRAME_CALL.size) + _C._FRAME_RESULT.pack(100_000, 1) + _C._FRAME_KIND.pack(
+        3000, 1000, 256, 256, 16, 16, per_pixel_sort, 1001, 200_000, flags, 0, 0, 0.0)
+    assert _lib.load(32).tg_frame_gradient_copies(frame) == expected
+
+
 @pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
 def test_state_words_of_the_frame_scan_keep_their_place(few, many):
     """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more

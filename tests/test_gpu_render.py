@@ -1655,7 +1655,7 @@ def test_gradients_summed_by_xcds(n, sigma, width, height, tw, th, per_waves, mo
     want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256,
                          m["per_pixel_sort"], ml)
     keys = int(want["offsets"][-1])
-    kind = _C._FRAME_KIND.pack(3 * n, n, width, height, tw, th, m["per_pixel_sort"], ml, _C._round_capacity(keys), 0, 0, 0, 0.0)
+    kind = _C._FRAME_KIND.pack(3 * n, n, width, height, tw, th, m["per_pixel_sort"], ml, _C._round_capacity(keys), 15, 0, 0, 0.0)
     assert (_C._gradient_copies(_lib.load(32), kind, keys) == 8) == per_waves
     gi, gd = _grad_inputs(scene, 9, True)
     wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, tw, th,
