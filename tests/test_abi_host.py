@@ -220,15 +220,26 @@ def _device_compile(source, *flags):
                            "--offload-device-only", *flags, os.path.join(build.CSRC, source)], check=True, capture_output=True, text=True).stderr
 
 
+def _assert_no_scratch_memory(source, kernels, flags, tmp_path):
+    report = _device_compile(source, *flags, "-Rpass-analysis=kernel-resource-usage", "-c", "-o", str(tmp_path / "kernels.o"))
+    names = re.findall(r"Function Name: (\S+)", report)
+    scratch = re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", report)
+    assert len(names) == kernels == len(scratch)
+    assert dict(zip(names, scratch)) == dict.fromkeys(names, "0")
+
+
 @pytest.mark.parametrize("flags", [(), ("-DTG_DOUBLE_PRECISION",)])
 def test_forward_kernels_need_no_scratch_memory(flags, tmp_path):
     """Scratch memory costs every launch of a kernel some microseconds: no instance of the forward kernels spills a register
     to it, in neither precision, by the compiler's own report."""
-    report = _device_compile("tg_forward.hip", *flags, "-Rpass-analysis=kernel-resource-usage", "-c", "-o", str(tmp_path / "forward.o"))
-    names = re.findall(r"Function Name: (\S+)", report)
-    scratch = re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", report)
-    assert len(names) == 6 == len(scratch)
-    assert dict(zip(names, scratch)) == dict.fromkeys(names, "0")
+    _assert_no_scratch_memory("tg_forward.hip", 6, flags, tmp_path)
+
+
+@pytest.mark.parametrize("flags", [(), ("-DTG_DOUBLE_PRECISION",)])
+def test_backward_kernels_need_no_scratch_memory(flags, tmp_path):
+    """The same of the backward kernels: three layouts each of the three compositors, two of them with and without a gradient of
+    the depth map, and the split of the gradient blocks."""
+    _assert_no_scratch_memory("tg_backward.hip", 16, flags, tmp_path)
 
 
 @pytest.mark.parametrize("flags,scalar", [((), "float"), (("-DTG_DOUBLE_PRECISION",), "double")])

@@ -662,7 +662,9 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
 #pragma unroll
                 for (int k = 0; k < 9; k++) t[k] = a.bary[9 * (int64_t)triangle + k];
                 uint64_t hit;
-                m = wave_hits(t, lane < nb, ((a.tw | a.th) & 7) == 0, wave_rect(p), p.px, p.py, hit);
+                PixelCoord q = p;
+                asm volatile("" : "+v"(q.px), "+v"(q.py));  // the rectangle is made of them here: kept by the loop it is in scratch memory
+                m = wave_hits(t, lane < nb, ((a.tw | a.th) & 7) == 0, wave_rect(q), q.px, q.py, hit, lane);
             }
             if (mine < kBackBatch) m &= mine > 0 ? (1ull << mine) - 1 : 0ull;  // entries past my last one
             // 2. slot numbers: lane = entry
@@ -896,8 +898,10 @@ struct SavedWave {
     int vertex[3 * kWave];  // the three vertex ids of a column's entry
     uint8_t src[kWave];     // the pixel (lane) of a slot
 };
+// Five waves a SIMD with the (V,8) block only: dense arrays are small frames', of a wave a SIMD at most, and in 96 registers the dense and the
+// strided instance have one and four of theirs in scratch memory.
 template <int kLayout, bool kDepth>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 5) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLayout != kGradBlock8 ? 4 : 5) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;

@@ -658,8 +658,7 @@ __device__ __forceinline__ uint64_t small_entry_hits(const Rec *s_rec, bool mine
 // there is one): 20 or more that can touch the pixels as above, fewer one by one, their matrices read from the lane that has
 // them.  -> bit e: entry e covers the calling lane's pixel; hit: the entries that cover any of the pixels.
 __device__ __forceinline__ uint64_t wave_hits(const real m[9], bool mine, bool by_lane, const WaveRect &rect, real px, real py,
-                                              uint64_t &hit) {
-    int lane = threadIdx.x & (kWave - 1);
+                                              uint64_t &hit, int lane = threadIdx.x & (kWave - 1)) {
     asm volatile("" : "+v"(lane), "+v"(px), "+v"(py));  // the pixels' coordinates by row and column are made here, not kept by the loop around the call
     const bool candidate = mine && rect.x_lo <= rect.x_hi && may_touch(m, rect);
     uint64_t todo = __builtin_amdgcn_ballot_w64(candidate), hits = 0;
