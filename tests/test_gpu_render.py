@@ -1596,6 +1596,18 @@ def test_tile_order_gradients_around_blocks_of_a_list(width, height, tw, th, n, 
                 assert_gradients_close(f"{n} in {width}x{height}, tiles of {tw}x{th}: {label}", g.cpu().numpy(), w, mag)
 
 
+def _blocks_of_a_backward_pass(backward, n_vertices):
+    """Its results, and how many (V,8) blocks it summed the gradients in, by the memory it asked for: 32 bytes a vertex for the gradients
+    and as many for each block."""
+    import torch
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_stats()["requested_bytes.all.current"]
+    results = backward()
+    blocks, rest = divmod(torch.cuda.memory_stats()["requested_bytes.all.peak"] - before, 32 * n_vertices)
+    assert rest == 0
+    return results, blocks - 1
+
+
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
 @pytest.mark.parametrize("vertices,shared,width,height", [
     (32767, False, 128, 128), (32768, False, 128, 128), (32770, False, 130, 97), (3000, False, 129, 128), (3000, True, 256, 256),
@@ -1612,9 +1624,8 @@ def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height
     m = MODES[mode]
     scene = S.random_soup(-(-vertices // 3), width, height, seed=8, sigma_px=3.0, opacity=(0.1, 0.6), varying_w=True)
     indices = np.minimum(scene["indices"], vertices - 1)
-    if shared:  # every vertex is three triangles': a corner of the next one and of the one after it too
-        indices = np.concatenate([indices, indices[:, [0, 1, 2]] * [1, 1, 0] + np.roll(indices, 1, 0) * [0, 0, 1],
-                                  indices[:, [0, 1, 2]] * [1, 0, 0] + np.roll(indices, 2, 0) * [0, 1, 1]])
+    if shared:  # every vertex is three triangles', none of them larger than the others
+        indices = np.concatenate([indices, indices[:, [1, 2, 0]], indices[:, [2, 0, 1]]])
     scene.update(vertices=scene["vertices"][:vertices], colors=scene["colors"][:vertices], opacities=scene["opacities"][:vertices],
                  indices=np.ascontiguousarray(indices, dtype=np.int32))
     by_block = (vertices >= 32768 or width > 128) if m["per_pixel_sort"] else (shared and width == 257) or (vertices == 32768 and height == 512)
@@ -1631,7 +1642,9 @@ def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height
     leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
     for _ in range(3):
         image, _ = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, per_pixel_sort=m["per_pixel_sort"], max_layers=m["max_layers"])
-        outs.append(torch.autograd.grad(image, leaves, gi))
+        out, blocks = _blocks_of_a_backward_pass(lambda: torch.autograd.grad(image, leaves, gi), vertices)
+        assert blocks == by_block
+        outs.append(out)
     for out in outs:
         for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
             assert g.is_contiguous()
@@ -1641,29 +1654,32 @@ def test_gradients_summed_in_a_block_or_in_place(vertices, shared, width, height
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "A_unlimited", "B_unlimited"])
 @pytest.mark.parametrize("n,sigma,width,height,tw,th,per_waves", [
     (150, 20.0, 150, 121, 16, 16, True), (150, 20.0, 128, 128, 16, 16, False), (1512, 20.0, 150, 121, 16, 16, True), (1513, 20.0, 150, 121, 16, 16, False), (400, 30.0, 200, 131, 8, 8, True), (400, 4.0, 200, 131, 8, 8, False),
-    (60, 50.0, 160, 160, 32, 32, True)])
+    (60, 50.0, 160, 160, 32, 32, True), (20, 2.0, 256, 256, 16, 16, False), (341, 2.0, 256, 256, 16, 16, False), (3000, 2.0, 400, 300, 16, 16, False)])
 def test_gradients_summed_by_xcds(n, sigma, width, height, tw, th, per_waves, mode, cuda, oracle):
-    """Where triangles are in 20 waves on average each XCD sums the gradients in a block of its own: on both sides of the line, by a first
-    frame (the Python route) and by ones whose plan is there (the module's)."""
+    """Where triangles are in 20 waves on average each XCD sums the gradients in a block of its own: on both sides of the lines, by a
+    first frame (the Python route, whose buffers have room for 65536 keys more) and by ones whose plan is there (the module's)."""
     import torch
     import scenes as S
     import trigrad_amd
-    from trigrad_amd import _C, _lib
+    from trigrad_amd import _C
     m = MODES[mode]
     scene = S.random_soup(n, width, height, seed=n, sigma_px=sigma, opacity=(0.05, 0.5), varying_w=True)
     ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
     want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256,
                          m["per_pixel_sort"], ml)
-    keys = int(want["offsets"][-1])
-    kind = _C._FRAME_KIND.pack(3 * n, n, width, height, tw, th, m["per_pixel_sort"], ml, _C._round_capacity(keys), 15, 0, 0, 0.0)
-    assert (_C._gradient_copies(_lib.load(32), kind, keys) == 8) == per_waves
     gi, gd = _grad_inputs(scene, 9, True)
     wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, tw, th,
                                     m["per_pixel_sort"], ml, literal=False, magnitudes=True)
     d = to_device(scene, cuda)
     leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
-    for _ in range(4):
+    upstream = (torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda))
+    _C._frame_key_hints.clear()
+    _C._frame_size_hints.clear()
+    _C._module().forget()
+    for frame in range(4):
         outputs = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, tw, th, per_pixel_sort=m["per_pixel_sort"], max_layers=m["max_layers"])
-        out = torch.autograd.grad(outputs, leaves, (torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda)))
+        assert ("RendererBackward" in type(outputs[0].grad_fn).__name__) == (frame == 0)
+        out, blocks = _blocks_of_a_backward_pass(lambda: torch.autograd.grad(outputs, leaves, upstream), 3 * n)
+        assert blocks == (8 if per_waves else int(m["per_pixel_sort"] and width * height > 16384))
         for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
             assert_gradients_close(f"{n} triangles/{mode}: {label}", g.cpu().numpy(), w, mag)
