@@ -1506,6 +1506,16 @@ def _with_w(scene, w):
     return dict(scene, vertices=v)
 
 
+def _assert_same_terms(name, got, want):
+    """Gradients of the same terms, added in another order: NaNs and infinities in the same places, the others within the rounding of a sum
+    of some hundreds of the column's largest (the derivatives of w are 1 / w times those of x and y)."""
+    not_finite = ~np.isfinite(want)
+    np.testing.assert_array_equal(np.where(not_finite, got, 0), np.where(not_finite, want, 0), err_msg=name)
+    for column, (g, w, skip) in enumerate(zip(*(a.reshape(len(a), -1).T for a in (got, want, not_finite)))):
+        largest = float(np.abs(w[~skip]).max(initial=0.0))
+        assert_close(f"{name}, column {column}", np.where(skip, 0, g), np.where(skip, 0, w), 1e-4, 300 * 2.0 ** -24 * largest + 2.0 ** -126)
+
+
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
 @pytest.mark.parametrize("w", ["soup_varying_w", "degenerate", "overlap_mesh_inf_w", "unit_square_negative_z", 0.9e-6, 1.1e-6, 0.9e6, 1.1e6,
                                1e-20, 1e-30, 1e-38, 1e30, 0.0, "around zero", "inf"])
@@ -1540,11 +1550,7 @@ def test_gradients_where_the_depth_map_has_none(w, mode, cuda):
                                offsets, bary, image, depthmap, weights, ends, W, H, tw, th, 1 / 256, m["per_pixel_sort"], ml, resume=resume)
             for g in (None, torch.from_numpy(gd).to(cuda))]
     for label, got, want in zip(("grad_vertices", "grad_colors", "grad_opacities"), *(tuple(g.cpu().numpy() for g in out) for out in outs)):
-        # the same terms, added in another order: within the rounding of a sum of some hundreds of the array's largest
-        finite = np.isfinite(want)
-        np.testing.assert_array_equal(np.isnan(got), np.isnan(want), err_msg=label)
-        largest = float(np.abs(want[finite]).max()) if finite.any() else 0.0
-        assert_close(f"{w}/{mode}: {label}", np.where(finite, got, 0), np.where(finite, want, 0), 1e-4, 300 * 2.0 ** -24 * largest + 1e-30)
+        _assert_same_terms(f"{w}/{mode}: {label}", got, want)
 
 
 @pytest.mark.parametrize("width,height,tw,th", [(513, 512, 16, 16), (512, 512, 16, 16), (478, 480, 16, 16), (500, 452, 16, 16), (448, 512, 16, 16),
