@@ -1518,7 +1518,7 @@ def _assert_same_terms(name, got, want):
 
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
 @pytest.mark.parametrize("w", ["soup_varying_w", "degenerate", "overlap_mesh_inf_w", "unit_square_negative_z", 0.9e-6, 1.1e-6, 0.9e6, 1.1e6,
-                               1e-20, 1e-30, 1e-38, 1e30, 0.0, "around zero", "inf"])
+                               1e-8, 1e-20, 1e-30, 1e-38, 1e30, 0.0, "around zero", "inf"])
 def test_gradients_where_the_depth_map_has_none(w, mode, cuda):
     """A frame whose depth map took no part in the loss has kernels of its own, which leave out what is 0 times the depth's derivatives
     but keep the NaNs it makes where those are not finite: against the general ones with a gradient of zeros."""
