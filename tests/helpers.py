@@ -28,7 +28,7 @@ def assert_close(name, got, want, rtol, atol):
 
 
 # ---- the gradient bar --------------------------------------------------------------------------------------
-# north_star's bar is 1e-4 relative + 1e-6 absolute.  The oracle adds a gradient element's terms into a float64 sum; the
+# The stated bar is 1e-4 relative + 1e-6 absolute.  The oracle adds a gradient element's terms into a float64 sum; the
 # kernels add the same terms in float32 (run sums, then float atomics, in no fixed order).  Where the terms cancel, that
 # alone leaves an error proportional to the sum of their MAGNITUDES, S, whatever the result is: a float32 addition
 # chain of n steps is off by at most n * 2^-24 * S and typically by about 2^-24 * S (the largest factor any test of this

@@ -1,5 +1,5 @@
 """The six host-side component hooks of libtrigrad_hip.so (reference src/trigrad/tests.cu:43-76: barycentric,
-interpolate3_scalar, interpolate3_vector and their backward functions) as the GPU box loads the library: the same
+interpolate3_scalar, interpolate3_vector and their backward functions) as the library is loaded where there is a GPU: the same
 comparisons as tests/test_components.py, run there so that the record of that run covers them, plus a direct call of
 every hook through the C ABI against the oracle, bit for bit."""
 import ctypes as C
@@ -52,7 +52,7 @@ def test_component_hooks_of_the_loaded_library(cuda, oracle):
 
 
 @pytest.mark.parametrize("case", range(8))
-def test_component_functions_on_the_gpu_box(case, cuda, oracle):
+def test_component_functions_beside_a_gpu(case, cuda, oracle):
     T.test_interpolate3_scalar(*T.CASES_I[case], oracle)
     T.test_interpolate3_vector(*T.CASES_V[case], oracle)
     T.test_barycentric(T.CASES_B[case], oracle)

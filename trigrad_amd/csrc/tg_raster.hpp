@@ -1,13 +1,15 @@
 // tg_raster.hpp -- pieces shared by the forward and backward tile kernels.
 //
 // Launch shape: grid (tiles_x, tiles_y, parts); a workgroup of at most 256 threads
-// owns pixels [z*blockDim, (z+1)*blockDim) of its tile in row-major order, so a
-// 16x16 tile is exactly one workgroup of four waves and larger tiles are split
-// into several workgroups that walk the same list.  A tile's sorted list is consumed in
-// batches: up to kBatch threads each gather one list entry (triangle id ->
+// owns pixels [part*blockDim, (part+1)*blockDim) of its tile, so tiles of more are split into several
+// workgroups that walk the same list.
+// Forward, and backward where no blend order was saved: a 16x16 tile is exactly one workgroup of four waves, part = z.
+// The tile's sorted list is consumed in batches: up to kBatch threads each gather one list entry (triangle id ->
 // vertex ids -> vertex data, bary matrix, attributes) into an LDS record, then
 // every pixel thread walks the records; all lanes read the same record at the
 // same time, which LDS serves as a broadcast.
+// The two other backward kernels: a wave works by itself, a workgroup is one or four of them (part_of_workgroup), and nothing is
+// staged; a fragment's record is gathered where the fragment is evaluated.
 #pragma once
 #include "tg_common.hpp"
 
