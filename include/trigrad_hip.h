@@ -403,8 +403,8 @@ int tg_split_gradient_block(const tg_real *block, int64_t n_vertices, tg_real *g
  * phases: which parts of the forward pass to launch; TG_FRAME_WAIT then waits for K (the one wait of the call) and
  * sets n_keys and counted.
  * gradients: (V,4), (V,3) and (V,) behind each other; block: (V,8) of scratch with per_pixel_sort, or, with
- * TG_FRAME_GRADIENT_COPIES in the backward call's phases, of tg_frame_gradient_copies times that (any 16-byte aligned pointer where it
- * is 0). */
+ * TG_FRAME_GRADIENT_COPIES | n << 16 for the backward call's phases, n times that (any 16-byte aligned pointer where n is 0);
+ * n is 0, 1 or 8, and best what tg_frame_gradient_copies says. */
 typedef struct tg_frame {
     const tg_real *vertices;
     const int32_t *indices;
@@ -424,7 +424,7 @@ typedef struct tg_frame {
     const tg_real *grad_depthmap;
     tg_real *gradients;
     tg_real *block;
-    int64_t n_keys;  /* out of the forward call; in the backward call: how many the frame has (tg_frame_gradient_copies) */
+    int64_t n_keys;  /* out */
     int64_t counted; /* out */
     int64_t n_vertices;
     int64_t n_triangles;
@@ -441,10 +441,10 @@ typedef struct tg_frame {
     double early_stopping_threshold;
 } tg_frame;
 
-#define TG_FRAME_GRADIENT_COPIES 256
+#define TG_FRAME_GRADIENT_COPIES 256 /* phases of the backward call: bits 16 and up are the number of blocks */
 /* How many (V,8) blocks a frame's gradients are summed in before they are copied out: 0, they are summed in place; 1, a vertex's
- * eight in one 32-byte sector; or 8, one for each XCD, where its triangles are in many tiles each (n_keys, as in the backward call; 0,
- * not known, is never 8). */
+ * eight in one 32-byte sector; or 8, one for each XCD, where its triangles are in many tiles each (by n_keys, as the
+ * forward call left it; 0, not known, is never 8). */
 int tg_frame_gradient_copies(const tg_frame *f);
 
 #define TG_FRAME_BACKWARD 1     /* flags: a backward pass will follow: save what it needs */

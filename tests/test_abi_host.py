@@ -314,6 +314,22 @@ def test_gradient_blocks_for_the_kernels_that_use_them(flags, per_pixel_sort, ex
     assert _lib.load(32).tg_frame_gradient_copies(frame) == expected
 
 
+def test_backward_frame_takes_the_number_of_blocks_it_is_given():
+    """The block is the caller's, who says how many (V,8) it holds: nothing that may have changed since it was allocated decides.
+    A frame without vertices returns when its arguments are looked at."""
+    from trigrad_amd import _C, _lib
+    lib, somewhere = _lib.load(32), 1 << 20
+    for per_pixel_sort in (0, 1):
+        kind = _C._FramePlan(0, 100, 256, 256, 16, 16, per_pixel_sort, 32, 4096, _C._FRAME_BACKWARD, 0.0).kind
+        for blocks, block, code in ((0, somewhere, 0), (1, somewhere, 0), (8, somewhere, 0), (8, somewhere + 4, -1), (1, 0, -1),
+                                    (2, somewhere, -1), (7, somewhere, -1), (9, somewhere, -1), (-1, somewhere, -1), (8 + (1 << 32), somewhere, -1)):
+            call = bytearray(_C._FRAME_BYTES)
+            _C._FRAME_CALL.pack_into(call, 0, 0, 0, 0, 0, 0, 0, somewhere, 0, 0, 0, 0, 0, 0, _C._FRAME_GRADIENT_COPIES | blocks << 16, 0, 0, somewhere, block)
+            _C._FRAME_RESULT.pack_into(call, _C._FRAME_CALL.size, 1 << 20, 1)
+            call[-_C._FRAME_KIND.size:] = kind
+            assert lib.tg_frame_backward((C.c_char * _C._FRAME_BYTES).from_buffer(call)) == code, (per_pixel_sort, blocks, block)
+
+
 @pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
 def test_state_words_of_the_frame_scan_keep_their_place(few, many):
     """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more

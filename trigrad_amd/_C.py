@@ -925,10 +925,9 @@ def frame_backward(frame, grad_image, grad_depthmap, vertices, indices, colors, 
         call = bytearray(_FRAME_BYTES)
         call[-_FRAME_KIND.size:] = plan.kind
         _FRAME_CALL.pack_into(call, 0, vertices.data_ptr(), indices.data_ptr(), colors.data_ptr(), opacities.data_ptr(), image.data_ptr(),
-                              depthmap.data_ptr(), kept.data_ptr(), 0, 0, 0, _raw_stream(dev), 0, 0, _FRAME_GRADIENT_COPIES, grad_image.data_ptr(),
+                              depthmap.data_ptr(), kept.data_ptr(), 0, 0, 0, _raw_stream(dev), 0, 0, _FRAME_GRADIENT_COPIES | copies << 16, grad_image.data_ptr(),
                               0 if grad_depthmap is None else grad_depthmap.data_ptr(), gradients.data_ptr(),
                               block.data_ptr())
-        _FRAME_RESULT.pack_into(call, _FRAME_CALL.size, frame.n_keys, 0)
         code = lib.tg_frame_backward((C.c_char * _FRAME_BYTES).from_buffer(call))
         if code:
             _lib.check(code, "tg_frame_backward")

@@ -228,6 +228,13 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
         set_error("tg_frame_backward: null, small or misaligned buffer, or a frame rendered without TG_FRAME_BACKWARD");
         return TG_E_ARG;
     }
+    const int64_t given = f->phases >> 16;  // blocks
+    const bool by_count = f->phases & TG_FRAME_GRADIENT_COPIES;
+    const int copies = by_count ? (int)given : f->per_pixel_sort ? 1 : 0;
+    if ((by_count && given != 0 && given != 1 && given != 8) || (copies && (!f->block || ((uintptr_t)f->block & 15)))) {
+        set_error("tg_frame_backward: null or misaligned block, or a number of blocks that is not 0, 1 or 8");
+        return TG_E_ARG;
+    }
     char *kept = (char *)f->kept;
     const int64_t V = f->n_vertices;
     if (V == 0) return 0;
@@ -248,12 +255,6 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
     // 33 331 in tiles of 8 x 8 273, 278, a mesh of 20 000 124, 127.  The backward pass alone near it, all of one size: 20 000 on
     // 1024 x 1024, 15 waves a triangle 63, 71, 21 waves 93, 102; 1000 there, 16 waves 22, 24, 300 on 256 x 256, 20 waves 19.3, 21.4; in tile order
     // 75, 84 (21 waves), 15.6, 19.2 (20); with a heavy tail, which their mean does not tell, 1500 on 256 x 256, 25 waves 66, 64 and 40, 35.
-    const bool copies_fit = f->phases & TG_FRAME_GRADIENT_COPIES;
-    const int copies = copies_fit ? gradient_copies(*f) : f->per_pixel_sort ? 1 : 0;
-    if (copies && (!f->block || ((uintptr_t)f->block & 15))) {
-        set_error("tg_frame_backward: null or misaligned block");
-        return TG_E_ARG;
-    }
     real *sums = copies ? f->block : f->gradients;
     const int64_t n4 = 2 * V * max(copies, 1);
     TG_LAUNCH(zero_gradients_kernel, dim3((unsigned)ceil_div64(n4, 256)), dim3(256), 0, (hipStream_t)f->stream, (real4 *)sums, n4);

@@ -227,9 +227,9 @@ struct Render : torch::autograd::Function<Render> {
         const at::Tensor gradients = at::empty({8 * n}, on(v, at::kFloat));  // (V,4) | (V,3) | (V,) behind each other
         tg_frame f;
         frame.plan->fill(f, n, i.size(0), frame.max_layers);
-        f.phases = TG_FRAME_GRADIENT_COPIES;
         f.n_keys = frame.n_keys;
         const int copies = tg::gradient_copies(f);
+        f.phases = TG_FRAME_GRADIENT_COPIES | (int64_t)copies << 16;
         const at::Tensor block = copies ? at::empty({copies * 8 * n}, on(v, at::kFloat)) : gradients;
         f.vertices = v.data_ptr<float>();
         f.indices = i.data_ptr<int32_t>();
