@@ -1602,6 +1602,34 @@ def test_tile_order_gradients_around_blocks_of_a_list(width, height, tw, th, n, 
                 assert_gradients_close(f"{n} in {width}x{height}, tiles of {tw}x{th}: {label}", g.cpu().numpy(), w, mag)
 
 
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "B_unlimited"])
+@pytest.mark.parametrize("width,height,tw,th", [(1, 1, 16, 16), (2, 1, 16, 16), (5, 3, 16, 16), (8, 8, 8, 8), (64, 1, 64, 1), (9, 9, 8, 8)])
+@pytest.mark.parametrize("n", [1, 2, 5, 63, 65, 130])
+def test_gradients_of_pixels_with_many_slots_of_a_round(n, width, height, tw, th, mode, cuda, oracle):
+    """A round of the backward pass hands the state from one of a pixel's slots to the next in as many turns as a pixel has slots: waves
+    of one pixel, whose fragments fill every slot, of a few, and of 64 with one or many each; with a gradient of the depth map and
+    without one."""
+    import torch
+    import scenes as S
+    import trigrad_amd
+    m = MODES[mode]
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    scene = S.random_soup(n, width, height, seed=n + width, sigma_px=40.0, opacity=(0.01, 0.2), varying_w=True)
+    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, tw, th, 1 / 256,
+                         m["per_pixel_sort"], ml)
+    gi, gd = _grad_inputs(scene, 5, True)
+    d = to_device(scene, cuda)
+    for depth_gradient in (None, gd):
+        wanted = oracle.render_backward(gi, np.zeros_like(gd) if depth_gradient is None else gd, scene["vertices"], scene["indices"], scene["colors"],
+                                        scene["opacities"], want, width, height, tw, th, m["per_pixel_sort"], ml, literal=False, magnitudes=True)
+        leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+        outputs = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, tw, th, per_pixel_sort=m["per_pixel_sort"], max_layers=m["max_layers"])
+        upstream = [torch.from_numpy(x).to(cuda) for x in ((gi,) if depth_gradient is None else (gi, gd))]
+        out = torch.autograd.grad(outputs[:len(upstream)], leaves, upstream)
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+            assert_gradients_close(f"{n} in {width}x{height}/{mode}: {label}", g.cpu().numpy(), w, mag)
+
+
 def _blocks_of_a_backward_pass(backward, n_vertices):
     """Its results, and how many (V,8) blocks it summed the gradients in, by the memory it asked for: 32 bytes a vertex for the gradients
     and as many for each block."""

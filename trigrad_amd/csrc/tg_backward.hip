@@ -139,9 +139,12 @@ __device__ __forceinline__ void gather_back(const RasterArgs &a, const TriIds &t
     r.id[0] = t.ia; r.id[1] = t.ib; r.id[2] = t.ic;
 }
 
-// Reverse-traversal state of one pixel (render.cu:647-653).
-struct BackState {
-    real final_alpha, alpha, s0, s1, s2, oa, zoa, final_weight, final_depth;
+// Reverse-traversal state of one pixel (render.cu:647-653): what a fragment changes, and what it reads only.
+struct ChainState {
+    real alpha, s0, s1, s2, oa, zoa;  // oa, zoa: with kDepth
+};
+struct BackState : ChainState {
+    real final_alpha, final_weight, final_depth;
     real inv_final_weight;  // the reference divides two terms of every fragment by the pixel's final weight
     real g0, g1, g2, g3, gd;  // upstream gradient of this pixel
 };
@@ -201,45 +204,47 @@ __device__ __forceinline__ FragValue fragment_value(const BackRecord<kDepth> &r,
     return v;
 }
 
-// The step from one fragment of a pixel to the next one in reverse blend order (render.cu:487-517).
+// The state behind a fragment, in reverse blend order (render.cu:487-497), from the one in front of it.  om = 1 - o.
 template <bool kDepth>
-__device__ __forceinline__ FragSeed fragment_chain_step(BackState &st, const FragValue &v) {
-    const real o = v.o;
-    const real color[3] = {v.color[0], v.color[1], v.color[2]};
-    const real om = 1.0f - o;
-    const real inv_om = reciprocal_of_normal(om);  // in [1e-4, 1] or NaN; the reference divides six derivative terms by om
-    const real g[3] = {st.g0, st.g1, st.g2};
-    real s[3] = {st.s0, st.s1, st.s2};
+__device__ __forceinline__ ChainState chain_behind(const ChainState &st, const FragValue &v, real om, real inv_om) {
+    ChainState next;
+    next.alpha = quotient(st.alpha, om, inv_om);                                           // :492 (state: kept exact)
+    next.s0 = st.s0 + v.color[0] * v.o * next.alpha;                                       // :493
+    next.s1 = st.s1 + v.color[1] * v.o * next.alpha;
+    next.s2 = st.s2 + v.color[2] * v.o * next.alpha;
+    if constexpr (kDepth) {
+        next.oa = st.oa + v.o * next.alpha;                                                // :496
+        next.zoa = st.zoa + v.z * v.o * next.alpha;                                        // :497
+    }
+    return next;
+}
+// What a fragment's gradient terms are linear in (render.cu:487-517), from the states in front of it and behind it.
+template <bool kDepth>
+__device__ __forceinline__ FragSeed fragment_seed(const ChainState &st, const ChainState &next, const FragValue &v, real inv_om, const BackState &pixel) {
+    const real g[3] = {pixel.g0, pixel.g1, pixel.g2}, s[3] = {st.s0, st.s1, st.s2};
     real t3[3];
 #pragma unroll
-    for (int k = 0; k < 3; k++) t3[k] = (color[k] * st.alpha - s[k]) * inv_om * g[k];
-    const real drgb_do = ((t3[0] + t3[1]) + t3[2]) + st.g3 * (-st.final_alpha * inv_om);  // :491
-    st.alpha = quotient(st.alpha, om, inv_om);                                             // :492 (state: kept exact)
-#pragma unroll
-    for (int k = 0; k < 3; k++) s[k] += color[k] * o * st.alpha;                       // :493
-    st.s0 = s[0]; st.s1 = s[1]; st.s2 = s[2];
+    for (int k = 0; k < 3; k++) t3[k] = (v.color[k] * st.alpha - s[k]) * inv_om * g[k];
     FragSeed f;
-    f.d_do = drgb_do;
-    const real ao = st.alpha * o;
-    f.gc[0] = ao * g[0]; f.gc[1] = ao * g[1]; f.gc[2] = ao * g[2];                     // :510
+    f.d_do = ((t3[0] + t3[1]) + t3[2]) + pixel.g3 * (-pixel.final_alpha * inv_om);         // :491
+    const real ao = next.alpha * v.o;
+    f.gc[0] = ao * g[0]; f.gc[1] = ao * g[1]; f.gc[2] = ao * g[2];                         // :510
     if constexpr (kDepth) {
-        const real z = v.z;
-        const real ddw_do = st.alpha - st.oa * inv_om;                                    // :494
-        const real dud_do = st.alpha * z - st.zoa * inv_om;                               // :495
-        st.oa = st.oa + o * st.alpha;                                                      // :496
-        st.zoa = st.zoa + z * o * st.alpha;                                                // :497
-        real dd_do = (dud_do - st.final_depth * ddw_do) * st.inv_final_weight * st.gd;    // :499
-        if (st.final_weight < kEffZero) dd_do = 0.0f;
-        f.d_do = drgb_do + dd_do;
-        f.dd_dz = ao * st.gd * st.inv_final_weight;                                        // :517
-        if (st.final_weight < kEffZero) f.dd_dz = 0.0f;
+        const real ddw_do = next.alpha - st.oa * inv_om;                                      // :494
+        const real dud_do = next.alpha * v.z - st.zoa * inv_om;                               // :495
+        real dd_do = (dud_do - pixel.final_depth * ddw_do) * pixel.inv_final_weight * pixel.gd;  // :499
+        if (pixel.final_weight < kEffZero) dd_do = 0.0f;
+        f.d_do = f.d_do + dd_do;
+        f.dd_dz = ao * pixel.gd * pixel.inv_final_weight;                                    // :517
+        if (pixel.final_weight < kEffZero) f.dd_dz = 0.0f;
     }
     return f;
 }
-
-template <bool kDepth>
-__device__ __forceinline__ FragSeed fragment_state_step(BackState &st, const BackRecord<kDepth> &r, real b0, real b1, real b2) {
-    return fragment_chain_step<kDepth>(st, fragment_value(r, b0, b1, b2));
+// 1 - o and its reciprocal; in [1e-4, 1] or NaN; the reference divides six derivative terms by it
+struct Remainder { real om, inv; };
+__device__ __forceinline__ Remainder remainder_of(real o) {
+    const real om = 1.0f - o;
+    return {om, reciprocal_of_normal(om)};
 }
 
 // Without a gradient of the depth: whether the terms by way of it are zeros.  They are where no product in them can be too large
@@ -387,7 +392,11 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
 // One fragment start to finish (used where every pixel has its own order).
 __device__ __forceinline__ void fragment_backward(BackState &st, const BackRecord<true> &r, real b0, real b1, real b2, real px,
                                                   real py, real out[kTerms]) {
-    const FragSeed f = fragment_state_step(st, r, b0, b1, b2);
+    const FragValue v = fragment_value(r, b0, b1, b2);
+    const Remainder rem = remainder_of(v.o);
+    const ChainState next = chain_behind<true>(st, v, rem.om, rem.inv);
+    const FragSeed f = fragment_seed<true>(st, next, v, rem.inv, st);
+    static_cast<ChainState &>(st) = next;
     fragment_terms(f, r, b0, b1, b2, px, py, out);
 }
 
@@ -413,18 +422,18 @@ __device__ __forceinline__ real *term_address(const BackwardArgs &g, int vertex_
 }
 
 template <bool kDepth>
-__device__ __forceinline__ BackState load_back_state(const BackwardArgs &g, const PixelCoord &p) {
+__device__ __forceinline__ BackState load_back_state(const BackwardArgs &g, int pixel) {
     BackState st;
-    const real4 gi = g.grad_image[p.index];
+    const real4 gi = g.grad_image[pixel];
     st.g0 = gi.x; st.g1 = gi.y; st.g2 = gi.z; st.g3 = gi.w;
-    st.gd = g.grad_depthmap ? g.grad_depthmap[p.index] : 0.0f;  // null: the depth map took no part in the loss
-    st.final_alpha = g.image[p.index].w;
+    st.gd = g.grad_depthmap ? g.grad_depthmap[pixel] : 0.0f;  // null: the depth map took no part in the loss
+    st.final_alpha = g.image[pixel].w;
     st.alpha = st.final_alpha;
     st.s0 = st.s1 = st.s2 = 0.0f;
     st.oa = st.zoa = 0.0f;
-    st.final_weight = g.weights[p.index];
+    st.final_weight = g.weights[pixel];
     st.inv_final_weight = 1.0f / st.final_weight;
-    st.final_depth = g.depthmap[p.index];
+    st.final_depth = g.depthmap[pixel];
     // without a gradient of the depth its part of d_do is 0 times these, and g3 is a factor of d_do only
     if (!kDepth && !(st.final_weight < kEffZero)) st.g3 += st.final_depth * 0.0f + st.inv_final_weight * 0.0f;
     return st;
@@ -538,51 +547,48 @@ __device__ __forceinline__ int wave_max_i32(int v) {
     return __builtin_amdgcn_readlane(v, kWave - 1);
 }
 
-// The steps of a round that the two kernels below share.  A round is up to 64 slots, each a fragment of a pixel: what the
-// lanes of its slots and of its pixels hand each other lies in the slot's column of the wave's term matrix.
-template <bool kDepth>
-__device__ __forceinline__ void leave_value(real *terms, int slot, const FragValue &v) {
-    terms[0 * kTermStride + slot] = v.o;
-    terms[1 * kTermStride + slot] = v.color[0];
-    terms[2 * kTermStride + slot] = v.color[1];
-    terms[3 * kTermStride + slot] = v.color[2];
-    if constexpr (kDepth) terms[4 * kTermStride + slot] = v.z;
+// The ordered part of a round, lane = slot.  A round is up to 64 slots, each a fragment of a pixel (lane `pixel` of the wave).  Only the
+// carried state goes from slot to slot: a turn hands every slot the state behind the one in front of it in its pixel's order
+// (slot_before; its own number: none of the round is), so after `turns` turns, as many as a pixel has slots at most, all have the right
+// one; those that have it already make it again.  The rest of a fragment is worked out once, by its slot.
+// last_slot: the last of the slots of the calling lane's own pixel, or -1.  Slots that are none have o = 0 and their own number.
+// (Before, the lanes of the pixels walked their slots, and a step, of three or four a round, was 60 instructions that read a fragment's
+// values from LDS and left the seed there; a turn is 24 now.  Saved order: 493 M vector instructions -> 460 M, 10^6 triangles 973 us ->
+// 960, tile order 357 -> 349.)
+template <bool kDepth, typename Take>
+__device__ __forceinline__ ChainState taken(const ChainState &st, const Take &take) {
+    ChainState t;
+    t.alpha = take(st.alpha);
+    t.s0 = take(st.s0); t.s1 = take(st.s1); t.s2 = take(st.s2);
+    if constexpr (kDepth) { t.oa = take(st.oa); t.zoa = take(st.zoa); }
+    return t;
 }
-// lane = pixel: the ordered part over my slots of the round (increasing slot = the order I must visit them in), which replaces the
-// fragments' values by the numbers that their gradient terms are linear in.
 template <bool kDepth>
-__device__ __forceinline__ void walk_slots(real *terms, uint64_t mine, BackState &st) {
-    while (true) {
-        const bool active = mine != 0;
-        if (__builtin_amdgcn_ballot_w64(active) == 0) break;
-        if (active) {
-            const int c = __builtin_ctzll(mine);
-            mine &= mine - 1;
-            FragValue v;
-            v.o = terms[0 * kTermStride + c];
-            v.color[0] = terms[1 * kTermStride + c];
-            v.color[1] = terms[2 * kTermStride + c];
-            v.color[2] = terms[3 * kTermStride + c];
-            if constexpr (kDepth) v.z = terms[4 * kTermStride + c];
-            const FragSeed f = fragment_chain_step<kDepth>(st, v);
-            terms[0 * kTermStride + c] = f.d_do;
-            terms[1 * kTermStride + c] = f.gc[0];
-            terms[2 * kTermStride + c] = f.gc[1];
-            terms[3 * kTermStride + c] = f.gc[2];
-            if constexpr (kDepth) terms[4 * kTermStride + c] = f.dd_dz;
-        }
+__device__ __forceinline__ FragSeed walk_chain(const FragValue &v, int pixel, int slot_before, int turns, int last_slot, BackState &st) {
+    const bool first = slot_before == (int)(threadIdx.x & (kWave - 1));
+    const Remainder rem = remainder_of(v.o);
+    const auto shared = [&](real x) { return __shfl(x, pixel, kWave); };
+    ChainState in = taken<kDepth>(st, shared), out = chain_behind<kDepth>(in, v, rem.om, rem.inv);
+    for (int turn = 1; turn < turns; turn++) {  // wave-uniform
+        const ChainState handed = taken<kDepth>(out, [&](real x) { return __shfl(x, slot_before, kWave); });
+        if (!first) in = handed;
+        out = chain_behind<kDepth>(in, v, rem.om, rem.inv);
     }
-}
-template <bool kDepth>
-__device__ __forceinline__ FragSeed seed_of_slot(const real *terms, int slot) {
-    FragSeed f;
-    f.d_do = terms[0 * kTermStride + slot];
-    f.gc[0] = terms[1 * kTermStride + slot];
-    f.gc[1] = terms[2 * kTermStride + slot];
-    f.gc[2] = terms[3 * kTermStride + slot];
-    if constexpr (kDepth) f.dd_dz = terms[4 * kTermStride + slot];
+    BackState of;  // the slot's pixel's
+    of.g0 = shared(st.g0); of.g1 = shared(st.g1); of.g2 = shared(st.g2); of.g3 = shared(st.g3);
+    of.final_alpha = shared(st.final_alpha);
+    if constexpr (kDepth) {
+        of.gd = shared(st.gd);
+        of.final_weight = shared(st.final_weight); of.final_depth = shared(st.final_depth); of.inv_final_weight = shared(st.inv_final_weight);
+    }
+    const FragSeed f = fragment_seed<kDepth>(in, out, v, rem.inv, of);
+    const int from = max(last_slot, 0);
+    const ChainState end = taken<kDepth>(out, [&](real x) { return __shfl(x, from, kWave); });
+    if (last_slot >= 0) static_cast<ChainState &>(st) = end;
     return f;
 }
+// The value of the lane before; lane 0's own.
+__device__ __forceinline__ int lane_before(int x) { return __builtin_amdgcn_update_dpp(x, x, 0x138, 0xf, 0xf, false); }  // wave_shr:1
 
 // Tile-order backward.  All pixels of a tile share the list order, so a wave walks its tile's list backwards, 64 entries at a
 // time, by itself:
@@ -592,11 +598,10 @@ __device__ __forceinline__ FragSeed seed_of_slot(const real *terms, int slot) {
 //      (pixel, entry) hit of the wave owns one slot, slots are grouped by entry, and a lane's own hits have increasing numbers in
 //      the order it must visit them (reverse blend order);
 //   then, in rounds of 64 slots:
-//   3. lane = pixel: tells its slots whose they are;
-//   4. lane = slot: gathers the record of its fragment (the entry's triangle and vertex numbers are in LDS) and leaves the
-//      fragment's opacity and colour; lane = pixel: the ordered part over its slots; lane = slot: the 21 gradient terms into a
-//      term matrix, where three groups of 21 lanes add up the runs of equal entry and issue one global floating-point atomic
-//      per run and term.
+//   3. lane = pixel: tells its slots whose they are, and which one is in front of them;
+//   4. lane = slot: gathers the record of its fragment (the entry's triangle and vertex numbers are in LDS), the ordered part
+//      (walk_chain), the 21 gradient terms into a term matrix, where three groups of 21 lanes add up the runs of equal entry and
+//      issue one global floating-point atomic per run and term.
 // Before, a workgroup of four waves staged every entry's record in LDS, between two barriers a block, each wave evaluated its
 // fragments where their pixels were (three or four turns a round with a third of the lanes busy), and 36 KB of LDS held the CU to
 // four of them.  Now a slot's record is gathered where the fragment is evaluated, by all lanes, entries that cover no pixel of the
@@ -609,7 +614,7 @@ struct TileWave {                // what a wave keeps in LDS
     alignas(16) int id[kBackBatch][4];  // the entries' triangles and vertices
     uint64_t ballot[kBackBatch]; // the lanes an entry covers
     uint32_t base[kBackBatch];   // an entry's first slot
-    uint16_t tag[kWaveSlots];    // (entry | source lane << 8) of a slot
+    uint32_t tag[kWaveSlots];    // (entry | pixel's lane << 8 | slot in front of it in the pixel's order << 16) of a slot, its own where it is the first
 };
 template <int kLayout, bool kDepth>
 __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 5) void backward_tile_order_kernel(RasterArgs a, BackwardArgs g) {
@@ -633,8 +638,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
     const int first_slot = __builtin_amdgcn_readfirstlane(slot_of_tile);  // of the wave
     const uint64_t *const masks = g.hit_masks + (int64_t)gridDim.x * gridDim.y * g.mask_parts + first_slot;
     const int my_last = p.valid ? g.last[p.index] : 0;  // entries [0, my_last) of the list may hold my fragments
-    BackState st;
-    if (p.valid) st = load_back_state<kDepth>(g, p);
+    BackState st = load_back_state<kDepth>(g, p.valid ? p.index : 0);  // of some pixel where there is none: slots that are none go through the walk as well
     int list_last = saved_masks ? (int)(int64_t)g.hit_masks[(int64_t)tile * g.mask_parts + first_slot / g.mask_threads] : -1;
     if (list_last < 0) list_last = wave_max_i32(my_last);  // no masks, or its pixels were rendered by several workgroups
     list_last = __builtin_amdgcn_readfirstlane(list_last);
@@ -681,15 +685,15 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
             for (uint32_t round0 = 0; round0 < n_hits; round0 += kWaveSlots) {
                 const int n_slots = (int)min((uint32_t)kWaveSlots, n_hits - round0);
                 // 3. whose the round's slots are
-                uint64_t slots = 0;
-                for (int handed_out = 0; handed_out < n_slots;) {  // a turn hands out one at least: the first one left is its pixel's next
+                int last_slot = -1, turns = 0;
+                for (int handed_out = 0; handed_out < n_slots; turns++) {  // a turn hands out one at least: the first one left is its pixel's next
                     const int e = m ? top_bit(m) : 0;
                     const uint32_t slot = mem.base[e] + lanes_below_mask(mem.ballot[e]) - round0;
                     const bool there = m != 0 && slot < (uint32_t)kWaveSlots;
                     handed_out += __builtin_popcountll(__builtin_amdgcn_ballot_w64(there));
                     if (there) {
-                        mem.tag[slot] = (uint16_t)(e | (lane << 8));
-                        slots |= 1ull << slot;
+                        mem.tag[slot] = (uint32_t)e | (uint32_t)lane << 8 | (last_slot >= 0 ? (uint32_t)last_slot : slot) << 16;
+                        last_slot = (int)slot;
                         m &= ~(1ull << e);
                     }
                 }
@@ -697,22 +701,20 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
 
                 // 4. the fragments' values, the ordered part, the terms
                 const bool active = lane < n_slots;
-                const int tag = active ? mem.tag[lane] : lane << 8;
-                const int entry = tag & 0xff;
-                // the pixel of the slot, from the lane that owns it
-                const real px = __shfl(p.px, tag >> 8, kWave), py = __shfl(p.py, tag >> 8, kWave);
+                const uint32_t tag = active ? mem.tag[lane] : (uint32_t)lane << 8 | (uint32_t)lane << 16;
+                const int entry = (int)(tag & 0xff), pixel = (int)(tag >> 8 & 0xff), slot_before = (int)(tag >> 16);
+                const real px = __shfl(p.px, pixel, kWave), py = __shfl(p.py, pixel, kWave);
                 BackRecord<kDepth> r;
                 real b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
+                FragValue value;
+                value.o = value.color[0] = value.color[1] = value.color[2] = value.z = 0.0f;
                 if (active) {
                     gather_back(a, *reinterpret_cast<const TriIds *>(mem.id[entry]), r);
                     bary_apply(r.m, px, py, b0, b1, b2);
-                    leave_value<kDepth>(terms, lane, fragment_value(r, b0, b1, b2));
+                    value = fragment_value(r, b0, b1, b2);
                 }
-                wave_lds_sync();
-                walk_slots<kDepth>(terms, slots, st);
-                wave_lds_sync();
+                const FragSeed f = walk_chain<kDepth>(value, pixel, slot_before, turns, last_slot, st);
                 if (active) {
-                    const FragSeed f = seed_of_slot<kDepth>(terms, lane);
                     real term[kTerms];
                     fragment_terms(f, r, b0, b1, b2, px, py, term);
 #pragma unroll
@@ -789,7 +791,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
     real bound_depth = 0.0f;
     int bound_j = 0;
     if (p.valid) {
-        st = load_back_state<true>(g, p);
+        st = load_back_state<true>(g, p.index);
         remaining = min(g.ends[p.index], a.max_layers);  // render.cu:642
         bound_depth = g.last_depth[p.index];
         bound_j = start + g.last[p.index];  // one past the last blended entry
@@ -871,43 +873,41 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
 // hold different numbers of fragments, so the wave takes its (pixel, step) pairs 64 at a
 // time: a round's 64 slots keep every lane busy whatever the pixels' counts are.  A round
 // takes the pending pairs nearest the far end of the tile's list (every pixel a prefix of
-// its next steps, so its own slots come in the order it must visit them): the slots of a
-// round then hold few different entries.  Per round:
+// its next steps): the slots of a round then hold few different entries.  Per round:
 //   1. lane = pixel: which of my next steps (their list positions are fetched from the
 //      saved order four steps ahead) lie at or above the round's threshold; they get
 //      consecutive slots;
-//   2. lane = slot: gathers the record of its fragment from memory (neighbouring
+//   2. lane = slot: the slots are grouped by entry (ballot matching); a slot takes the
+//      lane, and the column of the term matrix, that this gives it;
+//   3. lane = column: gathers the record of its fragment from memory (neighbouring
 //      pixels hold the same few entries, so the loads hit in cache; staging the tile's
-//      records in LDS first was measured slower, for the workgroups per CU it costs)
-//      and leaves the fragment's own opacity, colour and view depth in the slot;
-//   3. lane = pixel: the ordered part over my slots of the round, which replaces the
-//      five values by the five numbers the gradient terms are linear in;
-//   4. lane = slot: the 21 gradient terms.  LDS floating-point atomics cost about three
-//      cycles per lane on gfx950 and many slots of a round hold the same entry, so the
-//      terms are grouped by entry first: slots with equal entries get consecutive
-//      columns (ballot matching, groups in order of their lowest slot) of a term
-//      matrix in LDS, three groups of 21 lanes add up the runs of equal entry and issue
-//      one global floating-point atomic per run and term.
+//      records in LDS first was measured slower, for the workgroups per CU it costs);
+//   4. the ordered part (walk_chain);
+//   5. the 21 gradient terms into the term matrix, where three groups of 21 lanes add up
+//      the runs of equal entry and issue one global floating-point atomic per run and term
+//      (LDS floating-point atomics cost about three cycles per lane on gfx950).
+// Grouped before the gather and not behind it, four neighbouring lanes, whose addresses the CU takes together, mostly ask for the
+// same lines: 27 lines a load and atomic -> 18, the address unit busy 70 % of the time -> 63.  With the walk by slots (walk_chain), us:
+// 10^6 triangles 958 -> 930, 20 000 without a limit on the layers 523 -> 500, 200 000 large ones 218 -> 210, 33 000 in tiles of 8 x 8
+// 114 -> 110.
 // The waves of a tile share nothing, so a workgroup is one of them: its place is free for another tile's when it is done, where
 // workgroups of four wait for the longest of them (workgroup_waves).  In fours and so, us: 10^6 triangles 1057, 1013, 10^5 83.5, 76,
 // 20 000 with a heavy tail on 1920 x 1080 61, 55, a mesh of 1.3 million 185, 180.
 // What a wave keeps in LDS.  A workgroup takes it for the waves it has (taken for four always, frames in tiles of 8 x 8, a wave each,
 // had five workgroups a CU: 33 000 triangles 229 us, so 116).
+constexpr int kNotFirst = 0x80;  // the slot before is one of the same pixel
 struct SavedWave {
     real term[kTerms * kTermStride];
     int rel[kWave];         // list position of a slot's fragment, from the tile's start
-    int tag[kWave];         // the same by column of the term matrix
     int vertex[3 * kWave];  // the three vertex ids of a column's entry
-    uint8_t src[kWave];     // the pixel (lane) of a slot
+    uint8_t src[kWave];     // the pixel (lane) of a slot, and kNotFirst
 };
-// Five waves a SIMD with the (V,8) block only: dense arrays are small frames', of a wave a SIMD at most, and in 96 registers the dense and the
-// strided instance have one and four of theirs in scratch memory.
 template <int kLayout, bool kDepth>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLayout != kGradBlock8 ? 4 : 5) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 5) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
+    int lane = tid & (kWave - 1);
     SavedWave &mem = reinterpret_cast<SavedWave *>(s_dyn)[tid / kWave];
     const TilePart group = part_of_workgroup();
     const TileId tile_id = g.deep ? tile_in_turn<kTileBandBackward, kSixteenths>(group.linear, gridDim.x, gridDim.y)
@@ -918,14 +918,12 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLa
     const PixelCoord p = pixel_of_slot(a, tile_id.x, tile_id.y, slot_of_tile);
     const int rel_bits = 32 - __builtin_clz(max(end - start - 1, 1));  // bits that tell two list positions apart
     real *terms = mem.term;
-    int *tags = mem.tag;
     int *vertices = mem.vertex;
     const TermLane tl = term_lane<kLayout>(g, lane);
 
-    BackState st;
+    BackState st = load_back_state<kDepth>(g, p.valid ? p.index : 0);  // of some pixel where there is none: slots that are none go through the walk as well
     int n = 0;
     if (p.valid) {
-        st = load_back_state<kDepth>(g, p);
         // render.cu:642; fewer than were blended only where a NaN depth had the list blended more than once
         n = min(g.ends[p.index], min(a.max_layers, order_rows(g.order, a, end - start)));
     }
@@ -961,6 +959,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLa
 
     int span = end - start;  // list positions of the last round, from its threshold to its largest
     for (int round = 0; remaining > 0; round++) {
+        asm volatile("" : "+v"(lane));  // what depends on it is made here, not kept in registers by the loop
         // 1. the round's slots.  A round takes the wave's pending fragments from the far end of the tile's LIST, not step s
         //    of every pixel: a triangle is at another step in each pixel it covers, but at one list position, so the
         //    slots of a round then hold few different entries -- long runs, few atomics, and gathers whose lanes share
@@ -993,11 +992,15 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLa
         const int n_slots = min(kWave, offered);
         int *rels = mem.rel;
         uint8_t *srcs = mem.src;
+        // my slots of the round: neighbours, increasing slot = increasing step
         if (granted > 0) { rels[base] = ahead0; srcs[base] = (uint8_t)lane; }
-        if (granted > 1) { rels[base + 1] = ahead1; srcs[base + 1] = (uint8_t)lane; }
-        if (granted > 2) { rels[base + 2] = ahead2; srcs[base + 2] = (uint8_t)lane; }
-        if (granted > 3) { rels[base + 3] = ahead3; srcs[base + 3] = (uint8_t)lane; }
-        uint64_t mine = granted > 0 ? ((1ull << granted) - 1) << base : 0ull;  // my slots of the round: increasing slot = increasing step
+        if (granted > 1) { rels[base + 1] = ahead1; srcs[base + 1] = (uint8_t)(lane | kNotFirst); }
+        if (granted > 2) { rels[base + 2] = ahead2; srcs[base + 2] = (uint8_t)(lane | kNotFirst); }
+        if (granted > 3) { rels[base + 3] = ahead3; srcs[base + 3] = (uint8_t)(lane | kNotFirst); }
+        const int last_slot = granted > 0 ? base + granted - 1 : -1;
+        int turns = 1;
+#pragma unroll
+        for (int k = 1; k < 4; k++) turns += __builtin_amdgcn_ballot_w64(granted > k) != 0;
 #pragma unroll
         for (int k = 0; k < 4; k++)
             if (granted > k) {
@@ -1007,29 +1010,10 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLa
         remaining -= n_slots;
         wave_lds_sync();
 
-        // 2. lane = slot: the record, and the fragment's own values
-        const int src = (lane < n_slots) ? srcs[lane] : lane;
-        const real px = __shfl(p.px, src, kWave), py = __shfl(p.py, src, kWave);
-        BackRecord<kDepth> r;
-        real b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
-        int rel = 0;
-        if (lane < n_slots) {
-            rel = rels[lane];
-            gather_back(a, load_ids(a, start + rel), r);
-            bary_apply(r.m, px, py, b0, b1, b2);
-            leave_value<kDepth>(terms, lane, fragment_value(r, b0, b1, b2));
-        }
-        wave_lds_sync();
-
-        // 3. lane = pixel: the ordered part
-        walk_slots<kDepth>(terms, mine, st);
-        wave_lds_sync();
-
-        // 4. lane = slot: the terms, in the column the matching gives the slot
+        // 2. The slots grouped by entry (ballot matching, groups in the order of their lowest slot): the column a slot takes.
         const bool active = lane < n_slots;
-        FragSeed f;
-        f.d_do = f.gc[0] = f.gc[1] = f.gc[2] = f.dd_dz = 0.0f;
-        if (active) f = seed_of_slot<kDepth>(terms, lane);
+        const int src = active ? srcs[lane] : lane;
+        int rel = active ? rels[lane] : 0;
         // By the bits that tell positions of the round's range apart: the few positions outside it (a second step behind a
         // first one, by depth, may come later in the list) can be taken together with others, and then make more runs, not
         // other ones.
@@ -1040,24 +1024,43 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLa
             peers &= ~(vote ^ (uint64_t)(int64_t)bit);
         }
         const uint32_t rank = lanes_below_mask(peers);
-        const bool leads = active && rank == 0;
-        const uint32_t size = leads ? (uint32_t)__builtin_popcountll(peers) : 0u;
+        const uint32_t size = active && rank == 0 ? (uint32_t)__builtin_popcountll(peers) : 0u;
         const uint32_t incl = wave_inclusive_scan_u32(size);
-        const int leader = active ? __builtin_ctzll(peers) : lane;
-        const int column = __shfl((int)(incl - size), leader, kWave) + (int)rank;
-        wave_lds_sync();  // every slot's five numbers are in registers before terms take their place
+        int column = __shfl((int)(incl - size), active ? __builtin_ctzll(peers) : lane, kWave) + (int)rank;
+        if (!active) column = lane;
+        const int last_column = __shfl(column, max(last_slot, 0), kWave);
+        const int before = lane_before(column);
+        int tag = (src & (kWave - 1)) | ((src & kNotFirst) ? before : column) << 8;
+        tag = __builtin_amdgcn_ds_permute(column * 4, tag);
+        rel = __builtin_amdgcn_ds_permute(column * 4, rel);
+        const int pixel = tag & 0xff, slot_before = tag >> 8;
+
+        // 3. lane = column: the record, and the fragment's own values
+        const real px = __shfl(p.px, pixel, kWave), py = __shfl(p.py, pixel, kWave);
+        BackRecord<kDepth> r;
+        real b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
+        FragValue value;
+        value.o = value.color[0] = value.color[1] = value.color[2] = value.z = 0.0f;
+        if (active) {
+            gather_back(a, load_ids(a, start + rel), r);
+            bary_apply(r.m, px, py, b0, b1, b2);
+            value = fragment_value(r, b0, b1, b2);
+        }
+        // 4. the ordered part
+        const FragSeed f = walk_chain<kDepth>(value, pixel, slot_before, turns, last_slot >= 0 ? last_column : -1, st);
+        // 5. the terms
         if (active) {
             real term[kTerms];
             fragment_terms(f, r, b0, b1, b2, px, py, term);
 #pragma unroll
-            for (int q = 0; q < kTerms; q++) terms[q * kTermStride + column] = term[q];
-            tags[column] = rel;
+            for (int q = 0; q < kTerms; q++) terms[q * kTermStride + lane] = term[q];
 #pragma unroll
-            for (int k = 0; k < 3; k++) vertices[k * kWave + column] = r.id[k];
+            for (int k = 0; k < 3; k++) vertices[k * kWave + lane] = r.id[k];
         }
-        wave_lds_sync();
         // a column starts a run where its entry differs from the column before
-        const uint64_t heads = __builtin_amdgcn_ballot_w64(lane < n_slots && (lane == 0 || tags[lane] != tags[max(lane - 1, 0)]));
+        const int rel_before = lane_before(rel);
+        const uint64_t heads = __builtin_amdgcn_ballot_w64(active && (lane == 0 || rel != rel_before));
+        wave_lds_sync();
         add_run_sums(terms, n_slots, heads, tl, [&](int c, int v) { return vertices[v * kWave + c]; });
         wave_lds_sync();
     }
