@@ -875,7 +875,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
 // takes the pending pairs nearest the far end of the tile's list (every pixel a prefix of
 // its next steps): the slots of a round then hold few different entries.  Per round:
 //   1. lane = pixel: which of my next steps (their list positions are fetched from the
-//      saved order four steps ahead) lie at or above the round's threshold; they get
+//      saved order kPrefix steps ahead) lie at or above the round's threshold; they get
 //      consecutive slots;
 //   2. lane = slot: the slots are grouped by entry (ballot matching); a slot takes the
 //      lane, and the column of the term matrix, that this gives it;
@@ -895,6 +895,10 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
 // 20 000 with a heavy tail on 1920 x 1080 61, 55, a mesh of 1.3 million 185, 180.
 // What a wave keeps in LDS.  A workgroup takes it for the waves it has (taken for four always, frames in tiles of 8 x 8, a wave each,
 // had five workgroups a CU: 33 000 triangles 229 us, so 116).
+// Steps that a pixel can have in a round.  Fewer are fewer turns of the walk and candidates for a slot, and rounds of more entries (us, 4, 3,
+// 2 steps: 10^6 triangles 942, 912, 947, 20 000 without a limit on the layers 498, 470, 465, a mesh of 1.3 million 175, 177, 184, 10^5 73, 73, 80).
+// With 3, asked for where they stay (fetch_behind) and the pixel's own values after them: 896, 470, 177, 73; 33 000 in tiles of 8 x 8 109 -> 105.
+constexpr int kPrefix = 3;
 constexpr int kNotFirst = 0x80;  // the slot before is one of the same pixel
 struct SavedWave {
     real term[kTerms * kTermStride];
@@ -903,7 +907,7 @@ struct SavedWave {
     uint8_t src[kWave];     // the pixel (lane) of a slot, and kNotFirst
 };
 template <int kLayout, bool kDepth>
-__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 5) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
+__global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLayout == kGradStrided ? 4 : 5) void backward_saved_order_kernel(RasterArgs a, BackwardArgs g) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
     if (lists_invalid(g)) return;  // the same for the whole launch
     const int tid = threadIdx.x;
@@ -921,7 +925,6 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
     int *vertices = mem.vertex;
     const TermLane tl = term_lane<kLayout>(g, lane);
 
-    BackState st = load_back_state<kDepth>(g, p.valid ? p.index : 0);  // of some pixel where there is none: slots that are none go through the walk as well
     int n = 0;
     if (p.valid) {
         // render.cu:642; fewer than were blended only where a NaN depth had the list blended more than once
@@ -929,32 +932,41 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
     }
     const int64_t plane = order_stride(g.order, a);
     const bool long_list = end - start > kShortList;  // then the positions' high halves were saved as well
-    // The list positions of my steps, one after the other: step s is layer n - 1 - s, a plane further down each time.
+    // The list positions of my next three steps, -1 where there is none: below every threshold.  Step s is layer n - 1 - s, so the next
+    // one is `next_layer`, the others lie a plane further down each.
     const uint16_t *next_layer = g.order.low + ((int64_t)(n - 1) * plane + order_first(g.order, p, start, slot_of_tile));
     const int64_t high_halves = g.order.high;
-    int steps_read = 0;
-    auto next_position = [&]() {
-        int position = -1;  // no such step: below every threshold
-        if (steps_read < n) {
-            position = *next_layer;
-            if (long_list) position |= (int)next_layer[high_halves] << 16;
-        }
-        next_layer -= plane;
-        steps_read++;
-        return position;
+    int steps_left = n;
+    int ahead[kPrefix];
+    // The first `kept` of them are there; the others are asked for.  (Each into the register it stays in: one that is moved is waited for,
+    // and while every step taken moved all of them a round waited for as many loads, one after the other, as a pixel had steps in it.)
+    auto fetch_behind = [&](int kept) {
+#pragma unroll
+        for (int i = 0; i < kPrefix; i++)
+            if (kept <= i) {
+                ahead[i] = -1;
+                if (i < steps_left) {
+                    const uint16_t *layer = next_layer - i * plane;
+                    ahead[i] = *layer;
+                    if (long_list) ahead[i] |= (int)layer[high_halves] << 16;
+                }
+            }
     };
-    // the list positions of my next four steps
-    int ahead0 = next_position(), ahead1 = next_position(), ahead2 = next_position(), ahead3 = next_position();
+    fetch_behind(0);
+    BackState st = load_back_state<kDepth>(g, p.valid ? p.index : 0);  // of some pixel where there is none: slots that are none go through the walk as well
     int remaining = __builtin_amdgcn_readlane((int)wave_inclusive_scan_u32((uint32_t)n), kWave - 1);  // the wave's fragments not handed out yet
 
     // How many of my next steps lie at or above list position `threshold`: a prefix of them, so that I visit them in order.
-    // -> the four masks of the lanes whose first, second, ... next step qualifies, and the slots that makes.
+    // -> the slots that makes.
     auto slots_at = [&](int threshold) {
-        const uint64_t first = __builtin_amdgcn_ballot_w64(ahead0 >= threshold);
-        const uint64_t second = first & __builtin_amdgcn_ballot_w64(ahead1 >= threshold);
-        const uint64_t third = second & __builtin_amdgcn_ballot_w64(ahead2 >= threshold);
-        const uint64_t fourth = third & __builtin_amdgcn_ballot_w64(ahead3 >= threshold);
-        return __builtin_popcountll(first) + __builtin_popcountll(second) + __builtin_popcountll(third) + __builtin_popcountll(fourth);
+        uint64_t lanes = ~0ull;
+        int slots = 0;
+#pragma unroll
+        for (int i = 0; i < kPrefix; i++) {
+            lanes &= __builtin_amdgcn_ballot_w64(ahead[i] >= threshold);
+            slots += __builtin_popcountll(lanes);
+        }
+        return slots;
     };
 
     int span = end - start;  // list positions of the last round, from its threshold to its largest
@@ -963,12 +975,12 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
         // 1. the round's slots.  A round takes the wave's pending fragments from the far end of the tile's LIST, not step s
         //    of every pixel: a triangle is at another step in each pixel it covers, but at one list position, so the
         //    slots of a round then hold few different entries -- long runs, few atomics, and gathers whose lanes share
-        //    their cache lines.  Every pixel gives a prefix of its next (at most four) steps, those at or above a
+        //    their cache lines.  Every pixel gives a prefix of its next (at most kPrefix) steps, those at or above a
         //    threshold: the largest threshold that fills the 64 slots.  What overflows is cut off in lane order from a
         //    start lane that moves from round to round, and waits for the next round.
         int threshold = 0, offered = slots_at(0), match_bits = rel_bits;
         if (offered > kWave) {
-            const int top = wave_max_i32(ahead0) + 1;
+            const int top = wave_max_i32(ahead[0]) + 1;
             int high = top;  // slots_at(threshold) >= 64 > slots_at(high) = 0
             int middle = high - 2 * span;  // first twice what the last round took, then halves
             while (high - threshold > 1) {
@@ -980,9 +992,9 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
             span = max(top - threshold, 1);
             match_bits = 32 - __builtin_clz(span);
         }
-        const bool first = ahead0 >= threshold, second = first && ahead1 >= threshold, third = second && ahead2 >= threshold,
-                   fourth = third && ahead3 >= threshold;
-        const int mine_count = (int)first + (int)second + (int)third + (int)fourth;
+        int mine_count = 0;
+#pragma unroll
+        for (int i = 0; i < kPrefix; i++) mine_count += mine_count == i && ahead[i] >= threshold;
         const int taken_incl = (int)wave_inclusive_scan_u32((uint32_t)mine_count);
         const int first_lane = (round * 23) & (kWave - 1);
         const int before_first = __builtin_amdgcn_readlane(taken_incl - mine_count, first_lane);
@@ -993,20 +1005,21 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
         int *rels = mem.rel;
         uint8_t *srcs = mem.src;
         // my slots of the round: neighbours, increasing slot = increasing step
-        if (granted > 0) { rels[base] = ahead0; srcs[base] = (uint8_t)lane; }
-        if (granted > 1) { rels[base + 1] = ahead1; srcs[base + 1] = (uint8_t)(lane | kNotFirst); }
-        if (granted > 2) { rels[base + 2] = ahead2; srcs[base + 2] = (uint8_t)(lane | kNotFirst); }
-        if (granted > 3) { rels[base + 3] = ahead3; srcs[base + 3] = (uint8_t)(lane | kNotFirst); }
-        const int last_slot = granted > 0 ? base + granted - 1 : -1;
         int turns = 1;
 #pragma unroll
-        for (int k = 1; k < 4; k++) turns += __builtin_amdgcn_ballot_w64(granted > k) != 0;
+        for (int i = 0; i < kPrefix; i++) {
+            if (granted > i) { rels[base + i] = ahead[i]; srcs[base + i] = (uint8_t)(i ? lane | kNotFirst : lane); }
+            if (i) turns += __builtin_amdgcn_ballot_w64(granted > i) != 0;
+        }
+        const int last_slot = granted > 0 ? base + granted - 1 : -1;
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (granted > k) {
-                ahead0 = ahead1; ahead1 = ahead2; ahead2 = ahead3;
-                ahead3 = next_position();
-            }
+        for (int i = 0; i + 1 < kPrefix; i++)
+#pragma unroll
+            for (int k = 1; i + k < kPrefix; k++)
+                if (granted == k) ahead[i] = ahead[i + k];
+        steps_left -= granted;
+        next_layer -= granted * plane;
+        if (granted > 0) fetch_behind(kPrefix - granted);
         remaining -= n_slots;
         wave_lds_sync();
 
