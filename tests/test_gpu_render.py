@@ -1630,6 +1630,26 @@ def test_gradients_of_pixels_with_many_slots_of_a_round(n, width, height, tw, th
             assert_gradients_close(f"{n} in {width}x{height}/{mode}: {label}", g.cpu().numpy(), w, mag)
 
 
+@pytest.mark.parametrize("mode", ["A_default", "A_5_layers", "A_40_layers", "A_unlimited"])
+@pytest.mark.parametrize("tw,th", [(16, 16), (8, 8), (6, 5)])
+@pytest.mark.parametrize("n", [1, 22, 23, 24, 31, 32, 33, 64, 65, 140])
+def test_candidates_behind_and_in_front_of_the_last(n, tw, th, mode, cuda, oracle):
+    """A pixel's candidates come in the order of the list, which is not the pixel's where triangles are steep: behind the last candidate,
+    in front of it, and at its depth, in lists with room, at the edge of what is kept in LDS (23 places), and full (32); with one, two
+    and more selections."""
+    import scenes as S
+    rng = np.random.default_rng(n)
+    width, height = 24, 20
+    scene = S.random_soup(n, width, height, seed=n, sigma_px=60.0, opacity=(0.01, 0.2))
+    v = scene["vertices"].reshape(n, 3, 4)
+    v[::3, :, 2] = rng.uniform(0.1, 10.0, (len(v[::3]), 3))  # steep ones, flat ones, and pairs at one depth
+    v[1::3, :, 2] = np.round(v[1::3, :1, 2] * 0.5) + 1.0
+    v[..., 3] = 1.0 / v[..., 2]
+    scene["vertices"] = np.ascontiguousarray(v.reshape(3 * n, 4), np.float32)
+    _, want, got, _ = _forward_both(scene, tw, th, MODES[mode], cuda, oracle)
+    _check_forward(f"{n} candidates/{tw}x{th}/{mode}", want, got, (th, tw))
+
+
 def _blocks_of_a_backward_pass(backward, n_vertices):
     """Its results, and how many (V,8) blocks it summed the gradients in, by the memory it asked for: 32 bytes a vertex for the gradients
     and as many for each block."""

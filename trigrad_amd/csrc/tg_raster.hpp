@@ -728,6 +728,13 @@ __device__ __forceinline__ uint32_t lanes_below_mask(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
+template <int kWords>
+__device__ __forceinline__ bool any_set(const uint64_t m[kWords]) {
+    uint64_t all = 0;
+#pragma unroll
+    for (int wd = 0; wd < kWords; wd++) all |= m[wd];
+    return all != 0;
+}
 // Lowest set bit of a mask of kWords 64-bit words, removed from the mask; -1 if the mask is empty.
 template <int kWords>
 __device__ __forceinline__ int pop_lowest(uint64_t m[kWords]) {
