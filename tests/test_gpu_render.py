@@ -1650,6 +1650,18 @@ def test_candidates_behind_and_in_front_of_the_last(n, tw, th, mode, cuda, oracl
     _check_forward(f"{n} candidates/{tw}x{th}/{mode}", want, got, (th, tw))
 
 
+@pytest.mark.parametrize("mode", ["A_default", "A_unlimited", "B_unlimited"])
+@pytest.mark.parametrize("width,height,tw,th", [(1, 1, 16, 16), (1, 9, 8, 8), (9, 7, 16, 16), (17, 33, 16, 16), (40, 25, 32, 32), (23, 19, 24, 8),
+                                                (50, 47, 40, 24), (129, 9, 128, 8), (20, 21, 10, 6), (33, 5, 7, 8)])
+def test_waves_at_the_edges_of_an_image(width, height, tw, th, mode, cuda, oracle):
+    """The rectangle of a wave's pixels decides which list entries it looks at: whole squares of 8 x 8, those the image cuts, waves
+    without a pixel, and waves that are no squares; tiles of a power of two of squares a row, and of 3 and 5."""
+    import scenes as S
+    scene = S.random_soup(500, width, height, seed=width + height, sigma_px=3.0, opacity=(0.05, 0.4), varying_w=True)
+    _, want, got, _ = _forward_both(scene, tw, th, MODES[mode], cuda, oracle)
+    _check_forward(f"{width}x{height}/{tw}x{th}/{mode}", want, got, (th, tw))
+
+
 def _blocks_of_a_backward_pass(backward, n_vertices):
     """Its results, and how many (V,8) blocks it summed the gradients in, by the memory it asked for: 32 bytes a vertex for the gradients
     and as many for each block."""

@@ -670,7 +670,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
                 uint64_t hit;
                 PixelCoord q = p;
                 asm volatile("" : "+v"(q.px), "+v"(q.py));  // the rectangle is made of them here: kept by the loop it is in scratch memory
-                m = wave_hits(t, lane < nb, ((a.tw | a.th) & 7) == 0, wave_rect(q), q.px, q.py, hit, lane);
+                m = wave_hits(t, lane < nb, ((a.tw | a.th) & 7) == 0, wave_rect(a, q), q.px, q.py, hit, lane);
             }
             if (mine < kBackBatch) m &= mine > 0 ? (1ull << mine) - 1 : 0ull;  // entries past my last one
             // 2. slot numbers: lane = entry
@@ -780,7 +780,7 @@ __global__ __launch_bounds__(kTileThreads) void backward_pixel_order_kernel(Rast
     const int tile = tile_id.index;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_id);
-    publish_wave_rect(p, s_rects);
+    publish_wave_rect(a, p, s_rects);
     const bool tests_small = tests_small_entries(a, end - start, (int)(gridDim.x * gridDim.y));
     const int n_acc = min(end - start, kAccWindow);
     for (int i = tid; i < n_acc * kTerms; i += blockDim.x) s_acc[i] = 0.0f;

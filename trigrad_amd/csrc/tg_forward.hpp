@@ -100,7 +100,7 @@ __device__ __forceinline__ void tile_order_tile(const RasterArgs &a, const Forwa
     const int n_waves = blockDim.x / kWave;
     const int tile = tile_id.index;
     const PixelCoord p = pixel_of_thread(a, tile_id);
-    publish_wave_rect(p, s_rects);
+    publish_wave_rect(a, p, s_rects);
     const bool tests_small = tests_small_entries(a, end - start, (int)(gridDim.x * (gridDim.y - out.long_rows)));
     uint64_t *const masks = out.hit_masks ? out.hit_masks + hit_mask_head_words(out.long_rows) : nullptr;
 

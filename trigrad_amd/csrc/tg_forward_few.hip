@@ -24,7 +24,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
     const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
     const int slot = (blockIdx.z * kMaxTileWaves + part) * kWave + lane;
     const PixelCoord p = pixel_of_slot(a, tile.x, tile.y, slot);
-    const WaveRect rect = wave_rect(p);
+    const WaveRect rect = wave_rect(a, p);
     const bool squares = ((a.tw | a.th) & 7) == 0;
     PixelState s;  // of the first wave
     int last = 0;

@@ -146,7 +146,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     const int tile = tile_y * tiles_x + tile_x;
     const int start = a.offsets[tile], end = a.offsets[tile + 1];
     const PixelCoord p = pixel_of_thread(a, tile_x, tile_y);
-    publish_wave_rect(p, s_rects);
+    publish_wave_rect(a, p, s_rects);
     const bool tests_small = tests_small_entries(a, end - start, n_tiles);
     const int64_t order_step = order_stride(out.order, a);
     const int64_t order_at = order_first(out.order, p, start, blockIdx.z * blockDim.x + threadIdx.x);
@@ -156,9 +156,11 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     real last_depth = -__builtin_inff();  // render.cu:585-586
     int last_j = -1;  // list positions count from the tile's start
     bool active = p.valid && start < end;  // below, a list has a last entry
-    while (true) {
+    for (int selection = 0; start < end; selection++) {
         const bool want = active && s.alpha > a.thr && s.blended < a.max_layers;  // render.cu:588
-        if (!__syncthreads_or(want)) break;
+        // The first time all pixels want what one does.  And what one selection takes is all there is where no more layers are asked for:
+        // a pixel with fewer candidates than that is through with its list.
+        if (selection > 0 && (a.max_layers <= kLayers || !__syncthreads_or(want))) break;
         const int cap = want ? min(kLayers, a.max_layers - s.blended) : 0;
         int found = 0;
         real found_depth = 0.0f;  // of the last candidate
@@ -399,7 +401,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
 
     const int slot = (blockIdx.z * kMaxTileWaves + part) * kWave + lane;
     const PixelCoord p = pixel_of_slot(a, tile.x, tile.y, slot);
-    const WaveRect rect = wave_rect(p);
+    const WaveRect rect = wave_rect(a, p);
     const bool squares = ((a.tw | a.th) & 7) == 0;
 
     PixelState s;  // of the first wave
