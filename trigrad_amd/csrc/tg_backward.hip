@@ -629,7 +629,9 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
     const int slot_of_tile = group.part * blockDim.x + tid;
     const int tile = tile_id.index;
     const int start = a.offsets[tile];
-    const PixelCoord p = pixel_of_slot(a, tile_id.x, tile_id.y, slot_of_tile);
+    PixelCoord p = pixel_of_slot(a, tile_id.x, tile_id.y, slot_of_tile);
+    p.ix = __builtin_amdgcn_readfirstlane(p.ix);  // of the wave's first pixel: all that wave_rect needs, and no register
+    p.iy = __builtin_amdgcn_readfirstlane(p.iy);
     const TermLane tl = term_lane<kLayout>(g, lane);
 
     // With the forward pass's masks comes the number of list entries its workgroup has walked; else it is the largest `last` of my pixels.

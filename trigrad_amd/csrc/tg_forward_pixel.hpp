@@ -118,8 +118,9 @@ struct Candidates {
         tail.read(i - kHead, d, j);
         return d;
     }
+    template <bool kBranch>  // the wave has a branch, as few lists are longer than kHead; it costs two registers
     __device__ __forceinline__ int position(int i) const {
-        if (kHead == kLayers || __builtin_amdgcn_ballot_w64(i >= kHead) == 0) return head.j(i);  // a branch of the wave: few lists are that long
+        if (kHead == kLayers || (kBranch && __builtin_amdgcn_ballot_w64(i >= kHead) == 0)) return head.j(i);
         int j = head.j(min(i, kHead - 1));
         real d = 0.0f;
         tail.read(i - kHead, d, j);
@@ -156,11 +157,11 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
     real last_depth = -__builtin_inff();  // render.cu:585-586
     int last_j = -1;  // list positions count from the tile's start
     bool active = p.valid && start < end;  // below, a list has a last entry
-    for (int selection = 0; start < end; selection++) {
+    for (bool again = false; start < end; again = true) {
         const bool want = active && s.alpha > a.thr && s.blended < a.max_layers;  // render.cu:588
         // The first time all pixels want what one does.  And what one selection takes is all there is where no more layers are asked for:
         // a pixel with fewer candidates than that is through with its list.
-        if (selection > 0 && (a.max_layers <= kLayers || !__syncthreads_or(want))) break;
+        if (again && (a.max_layers <= kLayers || !__syncthreads_or(want))) break;
         const int cap = want ? min(kLayers, a.max_layers - s.blended) : 0;
         int found = 0;
         real found_depth = 0.0f;  // of the last candidate
@@ -284,14 +285,16 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                 // that come from memory overlap.  They are the kernel's peak of registers (two together where three would
                 // do: lists of hundreds 220 -> 226)
                 constexpr int kTogether = kHead < kLayers ? 1 : kInTurn ? 4 : 3;
-                int ahead = tk.position(0);  // one at a time, the next one's position is asked for while this one is blended
+                // one at a time, the next one's position is asked for while this one is blended, where there is a register left for it
+                constexpr bool kAhead = kTogether == 1 && kInTurn;
+                int ahead = kAhead ? tk.template position<kInTurn>(0) : 0;
                 for (int i0 = 0; i0 < todo; i0 += kTogether) {
                     BlendRecord r[kTogether];
                     int rel[kTogether];
 #pragma unroll
                     for (int u = 0; u < kTogether; u++) {
-                        rel[u] = kTogether == 1 ? ahead : tk.position(min(i0 + u, todo - 1));
-                        if (kTogether == 1) ahead = tk.position(min(i0 + 1, kLayers - 1));
+                        rel[u] = kAhead ? ahead : tk.template position<kInTurn>(kTogether == 1 ? i0 : min(i0 + u, todo - 1));
+                        if (kAhead) ahead = tk.template position<kInTurn>(min(i0 + 1, kLayers - 1));
                         if (rel[u] < n_rows) {
                             const real *row = rows + __umul24((uint32_t)rel[u], kBlendWords);
                             real *w = reinterpret_cast<real *>(&r[u]);
@@ -316,7 +319,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                     }
                 }
                 last_depth = todo_depth;
-                last_j = tk.position(todo - 1);
+                last_j = tk.template position<kInTurn>(todo - 1);
                 // fewer candidates than asked for: the list is exhausted, the next
                 // selection would return nothing (render.cu:594)
                 if (found < cap) active = false;
