@@ -452,6 +452,7 @@ int tg_frame_gradient_copies(const tg_frame *f);
 #define TG_FRAME_ORDER_POOL 4   /*   ... the blend order in a pool (tg_order_pool_words) */
 #define TG_FRAME_HIT_MASKS 8    /*   ... the hit masks (tile order) */
 #define TG_FRAME_LIST_BOUNDS 16 /*   depth bounds of the lists (tg_list_bounds) for the per-pixel selection */
+#define TG_FRAME_RECORDS 32     /*   the place of the bary matrices may hold records of all that is read of a triangle instead (tg_frame_has_records) */
 #define TG_FRAME_BIN 1          /* phases */
 #define TG_FRAME_LISTS 2
 #define TG_FRAME_RASTER 4
@@ -463,6 +464,9 @@ int tg_frame_gradient_copies(const tg_frame *f);
 
 int tg_frame_supported(int width, int height, int tile_w, int tile_h);
 int tg_frame_layout(const tg_frame *f, int64_t *out);
+/* Whether the frame makes a record of 32 scalars for each triangle, the first nine of which are its bary matrix, where else the
+ * matrices lie: with TG_FRAME_RECORDS, for many triangles that share few vertices. */
+int tg_frame_has_records(const tg_frame *f);
 int tg_frame_forward(tg_frame *f);
 int tg_frame_backward(const tg_frame *f);
 /* Waits (on the host) until host[word] differs from `pending`. */

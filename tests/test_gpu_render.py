@@ -1662,6 +1662,57 @@ def test_waves_at_the_edges_of_an_image(width, height, tw, th, mode, cuda, oracl
     _check_forward(f"{width}x{height}/{tw}x{th}/{mode}", want, got, (th, tw))
 
 
+@pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "A_unlimited", "B_unlimited"])
+@pytest.mark.parametrize("width,height,tw,th,big", [(520, 410, 16, 16, 0), (301, 203, 8, 8, 0), (300, 200, 32, 32, 3000), (160, 120, 16, 16, 900), (1920, 400, 16, 16, 0)])
+@pytest.mark.parametrize("saved", [True, False])
+def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, big, mode, cuda, monkeypatch):
+    """Many triangles with vertices of their own are rendered from records (TG_FRAME_RECORDS), others from the arrays: the same image, depth
+    map and lists, and gradients the same up to the order of the atomics; tiles of one and several workgroups, frames of few and
+    many, and lists of thousands, which depth bounds and the long tiles' kernels are for; in tile order without the saved hit masks too (in per-pixel order a backward pass
+    without a saved order reads the matrices, so there are no records).  Some triangles name a vertex that is
+    none, some are degenerate or far off the screen, and some attributes are zero or infinite."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    m = MODES[mode]
+    monkeypatch.setattr(_C, "SAVE_HIT_MASKS", saved)
+    monkeypatch.setattr(_C, "SAVE_BLEND_ORDER", saved)
+    n = 160_000 if m["per_pixel_sort"] else 510_000
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    rng = np.random.default_rng(width)
+    scene = S.random_soup(n, width, height, seed=width, sigma_px=0.6, opacity=(0.2, 0.9), varying_w=True)
+    v = scene["vertices"].reshape(n, 3, 4)
+    if big:
+        v[:big, :, :2] = rng.standard_normal((big, 3, 2)) * (6.0 / width)
+    v[5000] = v[5000, :1]
+    v[5001, :, :2] += 1.0e6
+    idx = scene["indices"].copy()
+    idx[5002, 1], idx[5003, 2] = 3 * n, -1
+    scene["colors"][15012:15030] = 0.0
+    scene["colors"][15033:15036] = np.inf
+    d = to_device(dict(scene, indices=idx), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, tw, th, 1 / 256, m["per_pixel_sort"], ml)
+    for _ in range(2):  # the second frame's buffers go by the first one's keys
+        packed, plain = _C.frame_forward(*args), _C.frame_forward(*args, records=False)
+    short = packed[3].plan.capacity <= 800 * (-(-width // tw) * -(-height // th))  # in tile order long lists are left early
+    assert packed[3].records == (saved if m["per_pixel_sort"] else short) and not plain[3].records
+    for a, b in zip(packed[:2], plain[:2]):
+        assert torch.equal(torch.nan_to_num(a, 7.0), torch.nan_to_num(b, 7.0)) and torch.equal(torch.isnan(a), torch.isnan(b))
+    results = [_C._frame_results(*f, width, height, tw, th, m["per_pixel_sort"], ml, n) for f in (packed, plain)]
+    for k in (2, 3, 4, 5, 6):  # weights, sorted ids, offsets, bary matrices, ends
+        a, b = results[0][k], results[1][k]
+        assert a.shape == b.shape and torch.equal(torch.nan_to_num(a.double(), 7.0), torch.nan_to_num(b.double(), 7.0))
+    gi, gd = (torch.from_numpy(x).to(cuda) for x in _grad_inputs(scene, 3, True))
+    for depth_gradient in (None, gd):
+        got, want = (_C.frame_backward(f[3], gi, depth_gradient, *args[:4], f[0], f[1], f[2]) for f in (packed, plain))
+        again = _C.frame_backward(plain[3], gi, depth_gradient, *args[:4], plain[0], plain[1], plain[2])
+        for g, w, w2 in zip(got, want, again):
+            assert torch.equal(torch.isfinite(g), torch.isfinite(w))
+            g, w, w2 = (torch.nan_to_num(x, 0.0, 0.0, 0.0).double() for x in (g, w, w2))
+            # two runs of one route differ by the order of their atomics; the two routes by no more than four times that
+            assert (g - w).norm() <= 4 * (w2 - w).norm() + 1e-6 * w.norm()
+
+
 def _blocks_of_a_backward_pass(backward, n_vertices):
     """Its results, and how many (V,8) blocks it summed the gradients in, by the memory it asked for: 32 bytes a vertex for the gradients
     and as many for each block."""

@@ -650,7 +650,7 @@ def _order_pool(n_keys, n_triangles, tile_width, tile_height, device):
 # ---- a frame in one call ----------------------------------------------------------------------------------
 
 _FRAME_PENDING = 0xFFFFFFFF
-_FRAME_BACKWARD, _FRAME_ORDER_PLANES, _FRAME_ORDER_POOL, _FRAME_HIT_MASKS, _FRAME_LIST_BOUNDS = 1, 2, 4, 8, 16
+_FRAME_BACKWARD, _FRAME_ORDER_PLANES, _FRAME_ORDER_POOL, _FRAME_HIT_MASKS, _FRAME_LIST_BOUNDS, _FRAME_RECORDS = 1, 2, 4, 8, 16, 32
 _FRAME_BIN, _FRAME_LISTS, _FRAME_RASTER, _FRAME_WAIT = 1, 2, 4, 8
 # struct tg_frame of the C header: what changes from call to call in front, then the results, then the frame's kind
 _FRAME_CALL = struct.Struct("<11Q3q4Q")
@@ -725,8 +725,9 @@ def _round_capacity(n):
 
 
 class Frame:
-    """A frame rendered by frame_forward: its plan, the status of its lists and (K) the keys it has."""
-    __slots__ = ("plan", "status", "n_keys")
+    """A frame rendered by frame_forward: its plan, the status of its lists, (K) the keys it has, and whether its triangles'
+    records are where else their bary matrices lie."""
+    __slots__ = ("plan", "status", "n_keys", "records")
 
 
 def render_by_torch_module(vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
@@ -759,7 +760,7 @@ def _leave_plan(kind, for_backward, dev, stream):
     limit = 0 if max_layers == n_triangles + 1 else max_layers  # 0: none
     n_triangles = _round_count(n_triangles)
     plan = _plan_for((0, n_triangles, width, height, tile_width, tile_height, per_pixel_sort,
-                      limit or min(n_triangles + 1, 0x7fffffff), capacity, flags, threshold))
+                      limit or min(n_triangles + 1, 0x7fffffff), capacity, flags | _FRAME_RECORDS, threshold))
     low, high = capacity // 4 if capacity > 1 << 18 else 0, 1 << 30
     if per_pixel_sort:
         # the depth bounds are for lists of a length; a scene that hovers around it keeps what it has
@@ -784,12 +785,12 @@ def frame_supported(vertices, width, height, tile_width, tile_height):
 
 
 def frame_forward(vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
-                  per_pixel_sort, max_layers, for_backward=True, timer=None):
+                  per_pixel_sort, max_layers, for_backward=True, timer=None, records=True):
     """-> (image, depthmap, kept, frame): `kept` is the block that holds what the backward pass reads.
 
     The call launches everything and waits for K only then; a frame with more keys than its buffers were made for (K of the
     last frame of its kind, or of its size by the number of triangles, and an eighth more; else three per triangle) is
-    rendered again into larger ones."""
+    rendered again into larger ones.  records=False: the bary matrices are left in `kept` whatever the frame."""
     global _frame_counter
     lib = _lib.load(32)
     dev = vertices.device
@@ -798,9 +799,9 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
             timer.start("init")
         vertices, indices, colors, opacities = vertices.contiguous(), indices.contiguous(), colors.contiguous(), opacities.contiguous()
         n_triangles, n_vertices = indices.shape[0], vertices.shape[0]
-        flags = 0
+        flags = _FRAME_RECORDS if records else 0
         if for_backward:
-            flags = _FRAME_BACKWARD
+            flags |= _FRAME_BACKWARD
             if not per_pixel_sort:
                 flags |= _FRAME_HIT_MASKS if SAVE_HIT_MASKS else 0
             elif SAVE_BLEND_ORDER:
@@ -879,6 +880,7 @@ def frame_forward(vertices, indices, colors, opacities, width, height, tile_widt
         if timer is None:
             _leave_plan(kind_for(n_keys, _round_capacity(n_keys)), for_backward, dev, stream)
     frame.plan, frame.status, frame.n_keys = plan, status, n_keys
+    frame.records = bool(lib.tg_frame_has_records(bytes(_FRAME_CALL.size + _FRAME_RESULT.size) + plan.kind))
     return image, depthmap, kept, frame
 
 
@@ -961,8 +963,12 @@ def _frame_results(image, depthmap, kept, frame, width, height, tile_width, tile
         order_pool = view("order", words, torch.int16, words)
     resume = Resume((last, last_depth, frame.status, fragments, masks))
     resume.order_pool, resume.pool_keys = order_pool, plan.capacity
+    if frame.records:  # their first nine scalars
+        bary = view("bary", 32 * n_triangles, torch.float32, n_triangles, 32)[:, :9].reshape(n_triangles, 3, 3)
+    else:
+        bary = view("bary", 9 * n_triangles, torch.float32, n_triangles, 3, 3)
     return (image, depthmap, view("weights", pixels, torch.float32, height, width), view("ids", K, torch.int32, K),
-            view("offsets", T + 1, torch.int32, T + 1), view("bary", 9 * n_triangles, torch.float32, n_triangles, 3, 3),
+            view("offsets", T + 1, torch.int32, T + 1), bary,
             view("ends", pixels, torch.int32, height, width), resume)
 
 
@@ -982,7 +988,7 @@ def _forward_full(vertices, indices, colors, opacities, width, height, tile_widt
     if frame_supported(vertices, width, height, tile_width, tile_height):
         image, depthmap, kept, frame = frame_forward(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
                                                      early_stopping_threshold, per_pixel_sort, int(max_layers), for_backward,
-                                                     None if disable_timing else timer)
+                                                     None if disable_timing else timer, records=False)
         timings = timer.stop()
         if not disable_timing:  # the timer has waited for the stream anyway
             if frame.status.failed() and not _tickets_forced:

@@ -69,6 +69,7 @@ SIGNATURES = {
     "tg_frame_forward": (_i, [_p]),
     "tg_frame_backward": (_i, [_p]),
     "tg_frame_gradient_copies": (_i, [_p]),
+    "tg_frame_has_records": (_i, [_p]),
     "tg_frame_wait": (_i, [_p, _i, C.c_uint32, _p]),
     "tg_clip_blocks": (_i64, [_i64]),
     "tg_clip_count": (_i, [_p, _i32, _p, _i64, _p, _p, _p]),

@@ -20,8 +20,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libtrigrad_hip.so")
 LIB_PATH_F64 = os.path.join(LIB_DIR, "libtrigrad_hip_f64.so")  # the same sources with -DTG_DOUBLE_PRECISION
 TORCH_MODULE_PATH = os.path.join(LIB_DIR, "trigrad_torch.so")
 
-SOURCES = ["tg_api.hip", "tg_binning.hip", "tg_scan.hip", "tg_sort.hip", "tg_forward.hip", "tg_forward_few.hip", "tg_backward.hip",
-           "tg_components.hip", "tg_camera.hip", "tg_frame.hip"]
+SOURCES = ["tg_api.hip", "tg_binning.hip", "tg_scan.hip", "tg_sort.hip", "tg_forward.hip", "tg_forward_few.hip", "tg_forward_packed.hip",
+           "tg_backward.hip", "tg_backward_packed.hip", "tg_components.hip", "tg_camera.hip", "tg_frame.hip"]
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",

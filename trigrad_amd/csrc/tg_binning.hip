@@ -20,7 +20,7 @@ namespace tg {
 
 constexpr int kBinThreads = 256;
 
-struct TriXYZ { real ax, ay, az, bx, by, bz, cx, cy, cz; bool ok; };
+struct TriXYZ { real ax, ay, az, bx, by, bz, cx, cy, cz, aw, bw, cw; int ia, ib, ic; bool ok; };
 
 // A triangle that names a vertex outside [0, n_vertices) is treated as
 // degenerate (all coordinates zero) instead of being dereferenced.
@@ -34,6 +34,8 @@ __device__ __forceinline__ TriXYZ load_triangle(const real4 *__restrict__ vertic
     r.ax = a.x; r.ay = a.y; r.az = a.z;
     r.bx = b.x; r.by = b.y; r.bz = b.z;
     r.cx = c.x; r.cy = c.y; r.cz = c.z;
+    r.aw = a.w; r.bw = b.w; r.cw = c.w;
+    r.ia = ia; r.ib = ib; r.ic = ic;
     return r;
 }
 
@@ -592,7 +594,53 @@ __device__ __forceinline__ void write_bary(const TriXYZ &p, real *__restrict__ m
     m[8] = (p.ax * p.by - p.bx * p.ay) / denom;
 }
 
-__global__ __launch_bounds__(kScanThreads) void frame_scan_kernel(const real4 *__restrict__ vertices, int n_vertices,
+// What frame_scan_kernel makes TriangleRecords of, and where they go; null: it makes none.
+struct PackedOut {
+    const real *colors, *opacities;
+    real4 *records;
+};
+// A lane's record, to its wave's place in LDS (kRecordLds bytes).  The pieces of record i are turned by i, else all lanes would meet in
+// four banks.
+constexpr size_t kRecordLds = kWave * sizeof(TriangleRecord);
+__device__ __forceinline__ void make_record(const PackedOut &out, const TriXYZ &p, const real m[9], real4v *lds, int lane) {
+    const auto put = [&](int k, real4v x) { lds[8 * lane + (k ^ (lane & 7))] = x; };
+    const Reach reach = triangle_reach(m, p.ax, p.ay, p.bx, p.by, p.cx, p.cy);
+    put(0, real4v{m[0], m[1], m[2], m[3]});
+    put(1, real4v{m[4], m[5], m[6], m[7]});
+    put(2, real4v{m[8], p.az, p.bz, p.cz});
+    put(3, real4v{p.aw, p.bw, p.cw, int_in_real((int)TriangleRecord::pack_bounds(reach.x_lo, reach.x_hi))});
+    const int id[3] = {p.ok ? p.ia : 0, p.ok ? p.ib : 0, p.ok ? p.ic : 0};  // a triangle that names no vertex is degenerate and in no list
+    const int bounds_y = (int)TriangleRecord::pack_bounds(reach.y_lo, reach.y_hi);
+    real op[3], col[9];
+#pragma unroll
+    for (int v = 0; v < 3; v++) {
+        op[v] = p.ok ? out.opacities[id[v]] : (real)0.0f;
+#pragma unroll
+        for (int k = 0; k < 3; k++) col[3 * v + k] = p.ok ? out.colors[3 * (int64_t)id[v] + k] : (real)0.0f;
+    }
+    put(4, real4v{int_in_real(bounds_y), op[0], op[1], op[2]});
+    put(5, real4v{col[0], col[1], col[2], col[3]});
+    put(6, real4v{col[4], col[5], col[6], col[7]});
+    put(7, real4v{col[8], int_in_real(id[0]), int_in_real(id[1]), int_in_real(id[2])});
+}
+// A wave's 64 records to their places, `first` and those behind it below n_triangles: eight lanes write one record, so that a line is
+// written at once.  (By lane, 16 bytes of 64 lines with every store, the kernel took 117 us for 10^6 triangles.)
+__device__ __forceinline__ void store_records(const real4v *lds, real4 *records, int64_t first, int64_t n_triangles, int lane) {
+    wave_lds_sync();
+    const int piece = lane & 7;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int i = 8 * k + (lane >> 3);
+        if (first + i < n_triangles) reinterpret_cast<real4v *>(records)[8 * (first + i) + piece] = lds[8 * i + (piece ^ (i & 7))];
+    }
+    wave_lds_sync();
+}
+
+// kRecords: with the triangles' records in the place of the bary matrices.  (Instances, because the registers and the LDS of the one
+// make the other slower: a mesh of 1.3 million 43 -> 50 us.  The one with records is held to the 128 registers that let all workgroups
+// of 10^6 triangles run at once.)
+template <bool kRecords>
+__global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1) void frame_scan_kernel(const real4 *__restrict__ vertices, int n_vertices,
                                                                   const int32_t *__restrict__ indices, int n_triangles, int W, int H,
                                                                   int tw, int th, int tiles_x, int tiles_y, uint32_t epoch,
                                                                   uint32_t *__restrict__ tri_offsets, real4 *__restrict__ records,
@@ -600,7 +648,8 @@ __global__ __launch_bounds__(kScanThreads) void frame_scan_kernel(const real4 *_
                                                                   int n_scan_tiles, uint32_t head_capacity, uint32_t *__restrict__ heads,
                                                                   uint32_t *totals, uint32_t *totals_next,
                                                                   real *__restrict__ edges, uint32_t *zero, size_t zero_words,
-                                                                  uint32_t *clear_word, real *__restrict__ bary) {
+                                                                  uint32_t *clear_word, real *__restrict__ bary, PackedOut packed) {
+    extern __shared__ __align__(16) unsigned char s_records[];  // kRecordLds for each wave, with records
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_wave_total[kScanThreads / kWave];
     __shared__ uint32_t s_tile_prefix;
@@ -612,6 +661,7 @@ __global__ __launch_bounds__(kScanThreads) void frame_scan_kernel(const real4 *_
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
+    real4v *const lds_records = reinterpret_cast<real4v *>(s_records + wave * kRecordLds);
     if (totals && tid <= kRadix)
         for (int p = 0; p < kEmitDigitPasses; p++) s_diff[p][tid] = 0;
     if (tid == 0) {
@@ -656,9 +706,16 @@ __global__ __launch_bounds__(kScanThreads) void frame_scan_kernel(const real4 *_
             records[t] = make_real4(A, B, C, int_in_real(r.x0));
             records[(int64_t)n_triangles + t] = make_real4(p.ax, p.ay, p.bx, p.by);
             records[2 * (int64_t)n_triangles + t] = make_real4(p.cx, p.cy, int_in_real(r.y0), int_in_real(r.y1 - r.y0 + 1));
-            if (bary) write_bary(p, bary + 9 * t);
+            if constexpr (kRecords) {
+                real m[9];
+                write_bary(p, m);
+                make_record(packed, p, m, lds_records, lane);
+            } else if (bary) {
+                write_bary(p, bary + 9 * t);
+            }
             rect = r;
         }
+        if constexpr (kRecords) store_records(lds_records, packed.records, t - lane, n_triangles, lane);
         s_count[k * kScanThreads + tid] = count;
         if (totals && count) {
             const uint32_t nx = (uint32_t)(rect.x1 - rect.x0 + 1), ny = (uint32_t)(rect.y1 - rect.y0 + 1);
@@ -1188,7 +1245,7 @@ extern "C" size_t tg_bin_frame_workspace_bytes(int32_t n_triangles, int64_t key_
 int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indices, int32_t n_triangles, int width, int height,
                   int tile_w, int tile_h, uint64_t *keys, uint32_t *values, int64_t key_capacity, uint32_t *total_and_status,
                   void *frame, size_t frame_bytes, uint32_t epoch, void *zero, size_t zero_bytes, uint32_t *clear_word, real *bary,
-                  uint64_t *host_total, void *stream) {
+                  uint64_t *host_total, void *stream, const real *colors, const real *opacities, real4 *records) {
 #ifdef TG_DOUBLE_PRECISION
     set_error("tg_bin_frame: the double build's depth keys take all 64 key bits; use tg_bin_setup and tg_build_tile_lists");
     return TG_E_ARG;
@@ -1216,14 +1273,20 @@ int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indic
         return check_launch("bin_frame_empty_kernel");
     }
     const int n_scan_tiles = (int)ceil_div64(n_triangles, kScanTile);
-    static int resident_cache[kMaxDevices] = {0};
+    static int resident_cache[2][kMaxDevices] = {{0}};
+    static size_t lds_reserved[kMaxDevices] = {0};
+    const auto scan_kernel = records ? frame_scan_kernel<true> : frame_scan_kernel<false>;
+    const size_t lds = records ? kRecordLds * (kScanThreads / kWave) : 0;
+    if (lds)  // with the kernel's own beyond 64 KB
+        if (int e = reserve_lds("tg_bin_frame", (const void *)scan_kernel, lds + 16, lds_reserved)) return e;
     uint32_t *ticket = f.ticket;
-    if (n_scan_tiles <= resident_workgroups((const void *)frame_scan_kernel, kScanThreads, resident_cache)) ticket = nullptr;
+    if (n_scan_tiles <= resident_workgroups((const void *)scan_kernel, kScanThreads, resident_cache[records != nullptr], lds)) ticket = nullptr;
     const GridPlan grid = grid_plan(tiles_x, tiles_y);
-    TG_LAUNCH(frame_scan_kernel, dim3(n_scan_tiles), dim3(kScanThreads), 0, s, (const real4 *)vertices, n_vertices, indices, n_triangles,
+    TG_LAUNCH_AS("frame_scan_kernel", scan_kernel, dim3(n_scan_tiles), dim3(kScanThreads), lds, s, (const real4 *)vertices, n_vertices, indices, n_triangles,
               width, height, tile_w, tile_h, tiles_x, tiles_y, epoch, f.tri_offsets, f.records, total_and_status, ticket, f.states,
               n_scan_tiles, f.head_capacity, f.heads, grid.on ? fused_frame_totals(frame, epoch) : (uint32_t *)nullptr,
-              fused_frame_totals(frame, epoch + 1), f.edges, (uint32_t *)zero, zero_bytes / 4, clear_word, bary);
+              fused_frame_totals(frame, epoch + 1), f.edges, (uint32_t *)zero, zero_bytes / 4, clear_word, bary,
+              PackedOut{colors, opacities, records});
     if (int e = check_launch("frame_scan_kernel")) return e;
     if (key_capacity == 0) return 0;
     // for every key position the buffers hold: the kernel reads K and the workgroups behind it leave at once
@@ -1239,7 +1302,7 @@ extern "C" int tg_bin_frame(const real *vertices, int32_t n_vertices, const int3
                             uint32_t *total_and_status, void *frame, size_t frame_bytes, uint32_t epoch, void *zero,
                             size_t zero_bytes, uint32_t *clear_word, void *stream) {
     return bin_frame(vertices, n_vertices, indices, n_triangles, width, height, tile_w, tile_h, keys, values, key_capacity,
-                     total_and_status, frame, frame_bytes, epoch, zero, zero_bytes, clear_word, nullptr, nullptr, stream);
+                     total_and_status, frame, frame_bytes, epoch, zero, zero_bytes, clear_word, nullptr, nullptr, stream, nullptr, nullptr, nullptr);
 }
 
 namespace tg {

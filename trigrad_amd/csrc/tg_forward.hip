@@ -18,60 +18,6 @@
 
 namespace tg {
 
-// Eight waves per SIMD (63 registers, nothing in scratch memory): 212 -> 194 us against the 73 registers it would take
-// (10^6 triangles, 1920 x 1080).  No bound in double precision: held to the five waves that the LDS allows it spills (8 x 8
-// tiles: 112 -> 123 us).  The tiles with the longest lists are started first, as far as there are workgroups for them; a launch
-// of few workgroups shares their work out instead (forward_tile_order_few_kernel).
-__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
-    __shared__ TileOrderLds s;
-    if (lists_invalid(out)) {  // the same for the whole launch
-        mark_tile_invalid(a, out);
-        return;
-    }
-    const bool first = (int)blockIdx.y < out.long_rows;
-    if (first && long_group(out) >= tiles_started_first(out)) return;
-    const TileId tile = first ? tile_of_index(out.long_tiles.words[1 + long_group(out)]) : tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
-    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
-    if (!first && is_started_first(out, tile.index, end - start)) return;
-    tile_order_tile(a, out, tile, start, end, s);
-}
-
-constexpr int kLongListGroups = 256;    // workgroups that look for the tiles with longer lists
-
-// The tiles whose lists are longer than kShortList, with int positions, where the kernel above does not share them out as long
-// tiles (their launch is saved there, 4.7 us whether there are any or not): few or none, so a small grid looks through the
-// tiles' list lengths (a workgroup through its share of the tiles, one tile per thread at a time) and takes those.
-__global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_kernel(RasterArgs a, ForwardOut out, int tiles_x,
-                                                                                      int tiles_y) {
-    extern __shared__ __align__(16) unsigned char s_dyn[];
-    __shared__ uint8_t s_touch[kSelectBatch];
-    __shared__ WaveRect s_rects[kMaxTileWaves];
-    __shared__ uint64_t s_votes[kMaxTileWaves];
-    if (out.list_status && *out.list_status != TG_STATUS_OK) return;  // the launch before this one has marked every pixel
-    const int tiles = tiles_x * tiles_y;
-    const int share = (tiles + (int)gridDim.x - 1) / (int)gridDim.x;
-    const int first = blockIdx.x * share, past = min(first + share, tiles);
-    const int n_waves = blockDim.x / kWave;
-    for (int base = first; base < past; base += blockDim.x) {
-        const int mine = base + (int)threadIdx.x;
-        const int length = mine < past ? a.offsets[mine + 1] - a.offsets[mine] : 0;
-        const bool is_long = length > kShortList && !(out.long_rows && blockDim.x == kTileThreads && length >= out.long_tiles.limit);
-        const uint64_t vote = __builtin_amdgcn_ballot_w64(is_long);
-        __syncthreads();  // the round before is done with the votes
-        if ((threadIdx.x & (kWave - 1)) == 0) s_votes[threadIdx.x / kWave] = vote;
-        __syncthreads();
-        for (int w = 0; w < n_waves; w++) {
-            uint64_t todo = s_votes[w];
-            while (todo) {  // the same for the whole workgroup
-                const int tile = base + w * kWave + __builtin_ctzll(todo);
-                todo &= todo - 1;
-                __syncthreads();  // the tile before is done with the LDS
-                pixel_order_tile<kSelectBatch, int, false, kLayers>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, tiles, s_dyn, s_touch, s_rects);
-            }
-        }
-    }
-}
-
 // Workgroups for the long tiles where they are shared out, at most: as many as run at once, four a CU; fewer may find too much
 // (1920 x 1080, 200 tiles of 1100 large faint triangles among 60 000 small ones, forward, us: 128 workgroups 630, 512 396, 1024
 // 339, one for each tile 478; without a limit on the layers 1597, 890, 637, 1048; 54 tiles of 32 x 32 in tile order, 256 210, 512
@@ -168,7 +114,7 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
                                  real *image, real *depthmap, real *final_weights, int32_t *ends, int32_t *last,
                                  real *last_depth, const OrderStore &order, uint64_t *hit_masks, const real *batch_bounds,
                                  const int32_t *far_start, const uint32_t *list_status, uint32_t *host_status, int64_t longest,
-                                 const LongTiles &long_tiles, void *stream) {
+                                 const LongTiles &long_tiles, const real4 *records, void *stream) {
     if (int e = check_raster_args("tg_render_forward", width, height, tile_w, tile_h, max_layers)) return e;
     if (!vertices || !indices || !colors || !opacities || !offsets || !bary || !image || !depthmap || !final_weights || !ends) {
         set_error("tg_render_forward: null pointer");
@@ -180,7 +126,8 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     }
     RasterArgs a{(const real4 *)vertices, indices, colors, opacities, sorted_ids, offsets, bary,
                  per_pixel_sort ? batch_bounds : nullptr, (per_pixel_sort && batch_bounds) ? far_start : nullptr,
-                 width, height, tile_w, tile_h, early_stopping_threshold, max_layers};
+                 width, height, tile_w, tile_h, early_stopping_threshold, max_layers, kPacks ? records : nullptr};
+    const bool packed = a.records != nullptr;
     if (batch_bounds && !far_start) {
         set_error("tg_render_forward: batch_bounds come with far_start");
         return TG_E_ARG;
@@ -205,13 +152,14 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
     hipStream_t s = (hipStream_t)stream;
     if (!per_pixel_sort) {
         if (split_tiles)
-            TG_LAUNCH_AS("forward_tile_order_few_kernel", tile_order_few_kernel(), grid, dim3(n_threads), 0, s, a, o);
+            TG_LAUNCH_AS("forward_tile_order_few_kernel", packed ? packed_tile_order_few_kernel() : tile_order_few_kernel(), grid, dim3(n_threads), 0, s, a, o);
         else
-            TG_LAUNCH(forward_tile_order_kernel, grid, dim3(n_threads), 0, s, a, o);
+            TG_LAUNCH_AS("forward_tile_order_kernel", packed ? packed_tile_order_kernel() : forward_tile_order_kernel<false>, grid,
+                         dim3(n_threads), 0, s, a, o);
         return check_launch("forward_tile_order_kernel");
     }
     const size_t lds = pixel_order_lds_bytes(n_threads, kSelectBatch);
-    static size_t lds_reserved[8][kMaxDevices] = {{0}}, lds_reserved_long[kMaxDevices] = {0};
+    static size_t lds_reserved[2][8][kMaxDevices] = {{{0}}}, lds_reserved_long[2][kMaxDevices] = {{0}};
     const bool in_turn = n_threads == kTileThreads;
     const auto launch = [&](void (*kernel)(RasterArgs, ForwardOut), size_t lds_bytes, size_t *reserved) -> int {
         if (int e = reserve_lds("tg_render_forward", (const void *)kernel, lds_bytes, reserved)) return e;
@@ -219,22 +167,25 @@ int tg::render_forward(const real *vertices, const int32_t *indices, const real 
         return check_launch("forward_pixel_order_kernel");
     };
     if (a.batch_bounds)  // they make the batches jump in steps of kSelectBatch
-        return in_turn ? launch(forward_pixel_order_kernel<kSelectBatch, int, true, kLayers>, lds, lds_reserved[0])
-                       : launch(forward_pixel_order_kernel<kSelectBatch, int, false, kLayers>, lds, lds_reserved[1]);
+        return launch(packed    ? packed_pixel_order_bounds_kernel(in_turn)
+                      : in_turn ? forward_pixel_order_kernel<kSelectBatch, int, true, kLayers, false>
+                                : forward_pixel_order_kernel<kSelectBatch, int, false, kLayers, false>, lds, lds_reserved[packed][in_turn]);
     const int places = candidate_places(groups, n_threads);
     const bool all_places = kShortHead < kLayers && places == kLayers;
     const size_t lds_short = pixel_order_lds_bytes(n_threads, kSelectBatchShort, sizeof(uint16_t), places);
-    const auto short_kernel = tiles_help   ? pixel_order_helping_kernel(all_places)
+    const auto short_kernel = packed       ? packed_pixel_order_kernel(tiles_help, all_places, in_turn)
+                              : tiles_help ? pixel_order_helping_kernel(all_places)
                               : all_places ? pixel_order_few_kernel(in_turn)
-                              : in_turn    ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead>
-                                           : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead>;
-    if (int e = launch(short_kernel, lds_short, lds_reserved[tiles_help ? 6 + all_places : 2 + 2 * all_places + in_turn])) return e;
+                              : in_turn    ? forward_pixel_order_kernel<kSelectBatchShort, uint16_t, true, kShortHead, false>
+                                           : forward_pixel_order_kernel<kSelectBatchShort, uint16_t, false, kShortHead, false>;
+    if (int e = launch(short_kernel, lds_short, lds_reserved[packed][tiles_help ? 6 + all_places : 2 + 2 * all_places + in_turn])) return e;
     // no list is too long for 16-bit positions, or those that are are long tiles, which the kernel above has shared out
     if (longest <= kShortList || (in_turn && o.long_rows && long_tiles.limit <= kShortList)) return 0;
-    if (int e = reserve_lds("tg_render_forward", (const void *)forward_pixel_order_long_lists_kernel, lds, lds_reserved_long)) return e;
+    const auto long_kernel = packed ? packed_pixel_order_long_lists_kernel() : forward_pixel_order_long_lists_kernel<false>;
+    if (int e = reserve_lds("tg_render_forward", (const void *)long_kernel, lds, lds_reserved_long[packed])) return e;
     const int tiles = (int)(tl.grid.x * tl.grid.y);
-    TG_LAUNCH(forward_pixel_order_long_lists_kernel, dim3(min(tiles, kLongListGroups), 1, grid.z), dim3(n_threads), lds, s, a, o,
-              (int)tl.grid.x, (int)tl.grid.y);
+    TG_LAUNCH_AS("forward_pixel_order_long_lists_kernel", long_kernel, dim3(min(tiles, kLongListGroups), 1, grid.z), dim3(n_threads), lds, s, a, o,
+                 (int)tl.grid.x, (int)tl.grid.y);
     return check_launch("forward_pixel_order_long_lists_kernel");
 }
 
@@ -251,7 +202,7 @@ extern "C" int tg_render_forward(const real *vertices, const int32_t *indices, c
     const OrderStore order{fragments, (int64_t)max_layers * width * height, 0};
     return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
                           early_stopping_threshold, per_pixel_sort, max_layers, image, depthmap, final_weights, ends, last, last_depth,
-                          order, hit_masks, batch_bounds, far_start, list_status, nullptr, std::numeric_limits<int64_t>::max(), LongTiles(), stream);
+                          order, hit_masks, batch_bounds, far_start, list_status, nullptr, std::numeric_limits<int64_t>::max(), LongTiles(), nullptr, stream);
 }
 
 extern "C" int64_t tg_order_pool_words(int64_t n_keys, int64_t n_triangles, int tile_w, int tile_h) {
@@ -274,5 +225,5 @@ extern "C" int tg_render_forward_pooled(const real *vertices, const int32_t *ind
     const OrderStore order{order_pool, n_triangles > kShortList ? n_keys * pixels : 0, pixels};
     return render_forward(vertices, indices, colors, opacities, sorted_ids, offsets, bary, width, height, tile_w, tile_h,
                           early_stopping_threshold, 1, max_layers, image, depthmap, final_weights, ends, last, last_depth, order, nullptr,
-                          batch_bounds, far_start, list_status, nullptr, n_keys, LongTiles(), stream);
+                          batch_bounds, far_start, list_status, nullptr, n_keys, LongTiles(), nullptr, stream);
 }

@@ -91,6 +91,7 @@ struct TileOrderLds {
     WaveRect rects[kMaxTileWaves];
     int last;
 };
+template <bool kPacked>
 __device__ __forceinline__ void tile_order_tile(const RasterArgs &a, const ForwardOut &out, const TileId &tile_id, int start, int end, TileOrderLds &lds) {
     BlendRecord *s_rec = lds.rec;
     uint8_t *s_touch = lds.touch;
@@ -111,7 +112,7 @@ __device__ __forceinline__ void tile_order_tile(const RasterArgs &a, const Forwa
         if (!__syncthreads_or(running)) break;
         const int nb = min(kBatch, end - batch);
         for (int e = tid; e < nb; e += blockDim.x) {
-            gather_blend(a, batch + e, s_rec[e]);
+            gather_blend<kPacked, true>(a, batch + e, s_rec[e]);
             s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, tests_small));
         }
         __syncthreads();
@@ -161,6 +162,25 @@ __device__ __forceinline__ void tile_order_tile(const RasterArgs &a, const Forwa
     }
 }
 
+// Eight waves per SIMD (63 registers, nothing in scratch memory): 212 -> 194 us against the 73 registers it would take
+// (10^6 triangles, 1920 x 1080).  No bound in double precision: held to the five waves that the LDS allows it spills (8 x 8
+// tiles: 112 -> 123 us).  The tiles with the longest lists are started first, as far as there are workgroups for them; a launch
+// of few workgroups shares their work out instead (forward_tile_order_few_kernel).
+template <bool kPacked>
+__global__ __launch_bounds__(kTileThreads, sizeof(real) == 4 ? 8 : 1) void forward_tile_order_kernel(RasterArgs a, ForwardOut out) {
+    __shared__ TileOrderLds s;
+    if (lists_invalid(out)) {  // the same for the whole launch
+        mark_tile_invalid(a, out);
+        return;
+    }
+    const bool first = (int)blockIdx.y < out.long_rows;
+    if (first && long_group(out) >= tiles_started_first(out)) return;
+    const TileId tile = first ? tile_of_index(out.long_tiles.words[1 + long_group(out)]) : tile_of_workgroup<kTileBandForward, kChunkForward>(out.long_rows);
+    const int start = a.offsets[tile.index], end = a.offsets[tile.index + 1];
+    if (!first && is_started_first(out, tile.index, end - start)) return;
+    tile_order_tile<kPacked>(a, out, tile, start, end, s);
+}
+
 // The kernels of launches with few workgroups (tg_forward_few.hip): forward_tile_order_kernel's, and forward_pixel_order_kernel
 // with all of a candidate list's places in LDS, and where the tiles' workgroups help with the long tiles.  Null in the double
 // build, which has none of them: every launch has all places in LDS there, and long tiles are noted by tg_frame_forward, a call of
@@ -171,5 +191,13 @@ using ForwardKernel = void (*)(RasterArgs, ForwardOut);
 ForwardKernel tile_order_few_kernel();
 ForwardKernel pixel_order_few_kernel(bool in_turn);
 ForwardKernel pixel_order_helping_kernel(bool all_places);
+
+// The instances that read triangles' records (tg_forward_packed.hip).  Null in the double build.
+using LongListsKernel = void (*)(RasterArgs, ForwardOut, int, int);
+ForwardKernel packed_tile_order_kernel();
+ForwardKernel packed_tile_order_few_kernel();
+ForwardKernel packed_pixel_order_kernel(bool tiles_help, bool all_places, bool in_turn);
+ForwardKernel packed_pixel_order_bounds_kernel(bool in_turn);
+LongListsKernel packed_pixel_order_long_lists_kernel();
 
 }  // namespace tg

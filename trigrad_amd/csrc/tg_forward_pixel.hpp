@@ -1,5 +1,6 @@
 // tg_forward_pixel.hpp -- the per-pixel-order forward kernel: selection and blending of one tile, the shared work of a long one.
-// Its instances for launches whose workgroups all run at once are compiled in tg_forward_few.hip, the others in tg_forward.hip.
+// Its instances for launches whose workgroups all run at once are compiled in tg_forward_few.hip, those that read triangles' records in
+// tg_forward_packed.hip, the others in tg_forward.hip.
 #pragma once
 #include "tg_forward.hpp"
 
@@ -131,7 +132,7 @@ struct Candidates {
 // The per-pixel-order forward pass of one tile.  Pos: how a candidate's list position (from the tile's
 // start) is kept.  With uint16_t the candidate lists of a 16x16 tile take 48 KB instead of 64 KB, which
 // together with 64 staged entries lets a CU hold three workgroups instead of two.
-template <int kStage, typename Pos, bool kInTurn, int kHead>  // kStage: list entries staged per batch
+template <int kStage, typename Pos, bool kInTurn, int kHead, bool kPacked>  // kStage: list entries staged per batch
 __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const ForwardOut &out, int tile_x, int tile_y, int tiles_x, int n_tiles,
                                                  unsigned char *s_dyn, uint8_t *s_touch, WaveRect *s_rects) {
     const int n_threads = kInTurn ? kTileThreads : blockDim.x;
@@ -174,7 +175,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
         constexpr int kTurns = kTileThreads / kStage;
         const int group = kStage == kWave ? wave : tid / kStage, mine = tid & (kStage - 1);  // in turn: whose batch, which of its entries
         const bool ahead = !kInTurn && !a.batch_bounds && (int)blockDim.x >= kStage;
-        std::conditional_t<kStage == kWave, PlacedParts, DepthParts> next;
+        std::conditional_t<kPacked, PackedParts, std::conditional_t<kStage == kWave, PlacedParts, DepthParts>> next;
         auto start_turns = [&](int first) {  // the records of the kTurns batches from list entry `first` on
             const int j = min(first + tid, end - 1);
             next.fetch_triangle(a, j);
@@ -219,8 +220,8 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
             }
             if (!kInTurn && !ahead) {
                 for (int e = tid; e < nb; e += blockDim.x) {
-                    gather_depth(a, batch + e, s_rec[e]);
-                    s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves) | small_entry(a, s_rec[e].extent, tests_small));
+                    const Reach reach = gather_depth<kPacked>(a, batch + e, s_rec[e]);
+                    s_touch[e] = (uint8_t)(waves_touched(s_rec[e].m, s_rects, n_waves, reach) | small_entry(a, s_rec[e].extent, tests_small));
                 }
             }
             __syncthreads();
@@ -271,7 +272,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
                                                    (sizeof(real) * kBlendWords)));
         for (int e = tid; e < n_rows; e += blockDim.x) {
             BlendRecord r;
-            gather_blend(a, start + e, r);
+            gather_blend<kPacked>(a, start + e, r);
             const real *w = reinterpret_cast<const real *>(&r);
 #pragma unroll
             for (int k = 0; k < kBlendWords; k++) rows[e * kBlendWords + k] = w[k];
@@ -301,7 +302,7 @@ __device__ __forceinline__ void pixel_order_tile(const RasterArgs &a, const Forw
 #pragma unroll
                             for (int k = 0; k < kBlendWords; k++) w[k] = row[k];
                         } else {
-                            gather_blend(a, start + rel[u], r[u]);
+                            gather_blend<kPacked>(a, start + rel[u], r[u]);
                         }
                     }
 #pragma unroll
@@ -384,7 +385,7 @@ __device__ __forceinline__ int merge_lists(const Shared *shared, const TopKOf<Po
 // 1.3 million triangles of a mesh, 1920 x 1080 (longest list 5200, 221 of at least 1024): 604 -> 332 us; 200 000 around the
 // camera (one list of 8400): 152 -> 117; 81 tiles with lists of some 2600, where depth bounds end the looking early: 105 -> 91.
 // s_quarter: a depth for every thread, with depth bounds; else null.
-template <int kStage, typename Pos, int kHead>
+template <int kStage, typename Pos, int kHead, bool kPacked>
 __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const ForwardOut &out, const TileId &tile, int part, unsigned char *s_dyn,
                                                volatile real *s_quarter) {
     constexpr int kStaged = kStage / kMaxTileWaves;  // records of a wave in LDS at a time
@@ -443,7 +444,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
                 // a group of the list is 64 entries for each wave
                 const int group = waves * kWave, mine = lane * waves + wave;
                 const auto entry = [&](int first) { return min(start + first + mine, end - 1); };
-                DepthParts next;
+                std::conditional_t<kPacked, PackedParts, DepthParts> next;
                 const auto fetch_from = [&](int first) {
                     next.fetch_triangle(a, entry(first));
                     next.fetch_matrix(a);
@@ -532,7 +533,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
                 last_depth = d;
                 last_j = j;
                 BlendRecord r;
-                gather_blend(a, start + j, r);
+                gather_blend<kPacked>(a, start + j, r);
                 if (s.blended < rows_kept) {
                     const int64_t word = order_at + (int64_t)s.blended * order_step;
                     out.order.low[word] = (uint16_t)j;
@@ -553,7 +554,7 @@ __device__ __forceinline__ void long_tile_part(const RasterArgs &a, const Forwar
 // kInTurn: the workgroup has four waves.
 // Workgroups a CU: what their LDS allows.  No bound in double precision: held to two workgroups every instance spills (10^5
 // triangles, 1024 x 1024: 229 us instead of 223, tiles of 8 x 8 190 instead of 168).
-template <int kStage, typename Pos, bool kInTurn, int kHead>
+template <int kStage, typename Pos, bool kInTurn, int kHead, bool kPacked>
 __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kStage != kSelectBatchShort ? 2 : short_list_waves(kHead))
 void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     extern __shared__ __align__(16) unsigned char s_dyn[];
@@ -572,9 +573,9 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
                 const TileId tile = tile_of_index(out.long_tiles.all[item / kMaxTileWaves]);
                 const int part = item % kMaxTileWaves, n = a.offsets[tile.index + 1] - a.offsets[tile.index];
                 if (sizeof(Pos) == sizeof(int) || n <= kShortList)
-                    long_tile_part<kStage, Pos, kHead>(a, out, tile, part, s_dyn, kStage != kWave ? s_quarter : nullptr);
+                    long_tile_part<kStage, Pos, kHead, kPacked>(a, out, tile, part, s_dyn, kStage != kWave ? s_quarter : nullptr);
                 else
-                    long_tile_part<kStage, int, kLongHead>(a, out, tile, part, s_dyn, nullptr);
+                    long_tile_part<kStage, int, kLongHead, kPacked>(a, out, tile, part, s_dyn, nullptr);
             }
             return;
         }
@@ -585,7 +586,44 @@ void forward_pixel_order_kernel(RasterArgs a, ForwardOut out) {
     const int n_entries = a.offsets[tile.index + 1] - a.offsets[tile.index];
     if (sizeof(Pos) < sizeof(int) && n_entries > kShortList) return;
     if (kInTurn ? is_long_tile(out, n_entries) : !first && is_started_first(out, tile.index, n_entries)) return;
-    pixel_order_tile<kStage, Pos, kInTurn, kHead>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
+    pixel_order_tile<kStage, Pos, kInTurn, kHead, kPacked>(a, out, tile.x, tile.y, gridDim.x, gridDim.x * (gridDim.y - out.long_rows), s_dyn, s_touch, s_rects);
+}
+
+constexpr int kLongListGroups = 256;    // workgroups that look for the tiles with longer lists
+
+// The tiles whose lists are longer than kShortList, with int positions, where forward_pixel_order_kernel does not share them out as long
+// tiles (their launch is saved there, 4.7 us whether there are any or not): few or none, so a small grid looks through the
+// tiles' list lengths (a workgroup through its share of the tiles, one tile per thread at a time) and takes those.
+template <bool kPacked>
+__global__ __launch_bounds__(kTileThreads) void forward_pixel_order_long_lists_kernel(RasterArgs a, ForwardOut out, int tiles_x,
+                                                                                      int tiles_y) {
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    __shared__ uint8_t s_touch[kSelectBatch];
+    __shared__ WaveRect s_rects[kMaxTileWaves];
+    __shared__ uint64_t s_votes[kMaxTileWaves];
+    if (out.list_status && *out.list_status != TG_STATUS_OK) return;  // the launch before this one has marked every pixel
+    const int tiles = tiles_x * tiles_y;
+    const int share = (tiles + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int first = blockIdx.x * share, past = min(first + share, tiles);
+    const int n_waves = blockDim.x / kWave;
+    for (int base = first; base < past; base += blockDim.x) {
+        const int mine = base + (int)threadIdx.x;
+        const int length = mine < past ? a.offsets[mine + 1] - a.offsets[mine] : 0;
+        const bool is_long = length > kShortList && !(out.long_rows && blockDim.x == kTileThreads && length >= out.long_tiles.limit);
+        const uint64_t vote = __builtin_amdgcn_ballot_w64(is_long);
+        __syncthreads();  // the round before is done with the votes
+        if ((threadIdx.x & (kWave - 1)) == 0) s_votes[threadIdx.x / kWave] = vote;
+        __syncthreads();
+        for (int w = 0; w < n_waves; w++) {
+            uint64_t todo = s_votes[w];
+            while (todo) {  // the same for the whole workgroup
+                const int tile = base + w * kWave + __builtin_ctzll(todo);
+                todo &= todo - 1;
+                __syncthreads();  // the tile before is done with the LDS
+                pixel_order_tile<kSelectBatch, int, false, kLayers, kPacked>(a, out, tile % tiles_x, tile / tiles_x, tiles_x, tiles, s_dyn, s_touch, s_rects);
+            }
+        }
+    }
 }
 
 }  // namespace tg

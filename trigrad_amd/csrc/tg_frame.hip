@@ -28,6 +28,23 @@ struct FrameLayout {
     int long_limit;                 // list entries that make a tile a long one; 0: the frame has no use for them
 };
 
+// Which frames make triangles' records (TriangleRecord).  They cost the scan 20 us for 10^6 triangles, and the passes gain by every list
+// entry they read: little where neighbouring triangles share vertices, whose lines they share as well (a mesh of 1.3 million, forward, us, 260
+// and 264), where what is read of all triangles is in the L2s anyway, and in tile order, which leaves long lists early.  Soups,
+// frames in us, without and with: per-pixel order, train, 50 000 small triangles on 1024 x 1024 135, 135, 10^5 152, 154, 150 000
+// 173, 172, 200 000 197, 192, 500 000 347, 329, 10^6 670, 586; shown, 10^5 144, 146, 150 000 168, 168, 300 000 245, 237, 10^6
+// 997, 907 (lists of 700).  Tile order, train, 300 000 on 1920 x 1080 247, 251, 500 000 348, 343, 10^6 588, 565 (lists of 270), on 1024 x 1024
+// with lists of 400 573, 542, of 700 611, 609, on 512 x 512 with lists of 2000 549, 551, of 2800 393, 419.
+constexpr int64_t kRecordsTriangles = 150000, kRecordsTrianglesTileOrder = 500000, kRecordsListTileOrder = 800;
+static bool may_have_records(const tg_frame &f) {
+    const bool backward_reads_matrices = (f.flags & TG_FRAME_BACKWARD) && f.per_pixel_sort && !(f.flags & (TG_FRAME_ORDER_PLANES | TG_FRAME_ORDER_POOL));
+    return (f.flags & TG_FRAME_RECORDS) && f.n_triangles >= (f.per_pixel_sort ? kRecordsTriangles : kRecordsTrianglesTileOrder) && !backward_reads_matrices;
+}
+static bool has_records(const tg_frame &f) {
+    const int64_t tiles = ceil_div64(f.width, f.tile_w) * ceil_div64(f.height, f.tile_h);
+    return may_have_records(f) && f.n_vertices >= 2 * f.n_triangles && (f.per_pixel_sort || f.key_capacity <= kRecordsListTileOrder * tiles);
+}
+
 // No size is larger for a smaller number of triangles, all else equal: callers size buffers for a rounded one.
 static FrameLayout frame_layout(const tg_frame &f) {
     FrameLayout L = {};
@@ -39,7 +56,8 @@ static FrameLayout frame_layout(const tg_frame &f) {
     L.status = take(4);  // of the sort
     L.ids = take((size_t)f.key_capacity * 4);
     L.offsets = take((size_t)(tiles + 1) * 4);
-    L.bary = take((size_t)f.n_triangles * 9 * sizeof(real));
+    // the place of the records is that of the matrices; whether they are used goes by the number of vertices too, the size does not
+    L.bary = take((size_t)f.n_triangles * (may_have_records(f) ? sizeof(TriangleRecord) : 9 * sizeof(real)));
     L.weights = take((size_t)pixels * sizeof(real));
     L.ends = take((size_t)pixels * 4);
     if (backward) {
@@ -134,9 +152,12 @@ static int no_frame(const char *fn) {
     return TG_E_ARG;
 }
 extern "C" int tg_frame_layout(const tg_frame *, int64_t *) { return no_frame("tg_frame_layout"); }
+extern "C" int tg_frame_has_records(const tg_frame *) { return 0; }
 extern "C" int tg_frame_forward(tg_frame *) { return no_frame("tg_frame_forward"); }
 extern "C" int tg_frame_backward(const tg_frame *) { return no_frame("tg_frame_backward"); }
 #else
+extern "C" int tg_frame_has_records(const tg_frame *f) { return f && has_records(*f); }
+
 extern "C" int tg_frame_layout(const tg_frame *f, int64_t *out) {
     if (int e = check_frame("tg_frame_layout", f)) return e;
     if (!out) { set_error("tg_frame_layout: null pointer"); return TG_E_ARG; }
@@ -172,6 +193,7 @@ extern "C" int tg_frame_forward(tg_frame *f) {
     uint32_t *ids = (uint32_t *)(kept + L.ids);
     int32_t *offsets = (int32_t *)(kept + L.offsets);
     real *bary = (real *)(kept + L.bary);
+    real4 *records = has_records(*f) ? (real4 *)bary : nullptr;
     volatile uint32_t *host = f->host;
     const int64_t longest = f->key_capacity < f->n_triangles ? f->key_capacity : f->n_triangles;  // a triangle is in a list once
     LongTiles long_tiles;
@@ -183,7 +205,7 @@ extern "C" int tg_frame_forward(tg_frame *f) {
         host[2] = TG_FRAME_PENDING;
         if (int e = bin_frame(f->vertices, V, f->indices, M, W, H, tw, th, keys, ids, f->key_capacity, total_and_status, f->frame,
                               (size_t)f->frame_bytes, (uint32_t)f->epoch, scratch + L.sort, L.zero_bytes, status, bary,
-                              (uint64_t *)f->host, f->stream))
+                              (uint64_t *)f->host, f->stream, f->colors, f->opacities, records))
             return e;
     }
     if (f->phases & TG_FRAME_LISTS) {
@@ -209,7 +231,7 @@ extern "C" int tg_frame_forward(tg_frame *f) {
                                    (real *)(kept + L.weights), (int32_t *)(kept + L.ends), backward ? (int32_t *)(kept + L.last) : nullptr,
                                    backward && f->per_pixel_sort ? (real *)(kept + L.last_depth) : nullptr, frame_order(*f, L, kept),
                                    (f->flags & TG_FRAME_HIT_MASKS) ? (uint64_t *)(kept + L.masks) : nullptr, bounds, far_start, status,
-                                   (uint32_t *)f->host + 2, longest, long_tiles, f->stream))
+                                   (uint32_t *)f->host + 2, longest, long_tiles, records, f->stream))
             return e;
     }
     if (f->phases & TG_FRAME_WAIT) {
@@ -268,7 +290,7 @@ extern "C" int tg_frame_backward(const tg_frame *f) {
                                 (int)f->width, (int)f->height, (int)f->tile_w, (int)f->tile_h, (real)f->early_stopping_threshold,
                                 (int)f->per_pixel_sort, (int)f->max_layers, sums, stride ? sums + 4 : sums + 4 * V,
                                 stride ? sums + 7 : sums + 7 * V, stride ? stride : 4, stride ? stride : 3, stride ? stride : 1, copies > 1 ? 8 * V : 0,
-                                (const uint32_t *)(kept + L.status), f->key_capacity, f->stream))
+                                (const uint32_t *)(kept + L.status), f->key_capacity, has_records(*f) ? (const real4 *)(kept + L.bary) : nullptr, f->stream))
         return e;
     if (!copies) return 0;
     return split_gradient_block(f->block, V, copies, f->gradients, f->gradients + 4 * V, f->gradients + 7 * V, f->stream);
