@@ -1713,6 +1713,27 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
             assert (g - w).norm() <= 4 * (w2 - w).norm() + 1e-6 * w.norm()
 
 
+@pytest.mark.parametrize("n,width,height,tw,sigma", [(1, 64, 64, 16, 9.0), (511, 64, 64, 16, 2.0), (512, 300, 200, 16, 2.0), (513, 300, 200, 8, 6.0), (9000, 500, 400, 8, 6.0),
+                                                     (131071, 640, 480, 16, 1.0), (131072, 640, 480, 16, 0.3), (131073, 640, 480, 16, 1.0),
+                                                     (262144, 1000, 700, 16, 0.5), (262145, 1000, 700, 16, 2.0), (600000, 1000, 700, 16, 3.0)])
+def test_lists_of_frames_around_the_sizes_that_split_the_work_otherwise(n, width, height, tw, sigma, cuda, monkeypatch):
+    """The scan takes 1, 2 or 4 triangles a thread and the sweeps 2, 4 or 8 pairs: frames on both sides of every line have the lists
+    of the route by stages, which knows none of them."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    d = to_device(S.random_soup(n, width, height, seed=n, sigma_px=sigma), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, tw, 16, 1 / 256, True, True, 8)
+    for _ in range(2):  # the second frame's buffers go by the first one's keys
+        got = _C._forward_full(*args)
+    got[8][2].verify()
+    monkeypatch.setattr(_C, "ONE_CALL_FRAME", False)
+    want = _C._forward_full(*args)
+    want[8][2].verify()
+    for k in (0, 1, 3, 4, 6):  # image, depth map, sorted ids, offsets, ends
+        assert torch.equal(got[k], want[k])
+
+
 def _blocks_of_a_backward_pass(backward, n_vertices):
     """Its results, and how many (V,8) blocks it summed the gradients in, by the memory it asked for: 32 bytes a vertex for the gradients
     and as many for each block."""

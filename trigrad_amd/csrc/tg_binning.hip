@@ -636,10 +636,11 @@ __device__ __forceinline__ void store_records(const real4v *lds, real4 *records,
     wave_lds_sync();
 }
 
+// kEach: triangles a thread.
 // kRecords: with the triangles' records in the place of the bary matrices.  (Instances, because the registers and the LDS of the one
 // make the other slower: a mesh of 1.3 million 43 -> 50 us.  The one with records is held to the 128 registers that let all workgroups
 // of 10^6 triangles run at once.)
-template <bool kRecords>
+template <bool kRecords, int kEach>
 __global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1) void frame_scan_kernel(const real4 *__restrict__ vertices, int n_vertices,
                                                                   const int32_t *__restrict__ indices, int n_triangles, int W, int H,
                                                                   int tw, int th, int tiles_x, int tiles_y, uint32_t epoch,
@@ -653,7 +654,8 @@ __global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_wave_total[kScanThreads / kWave];
     __shared__ uint32_t s_tile_prefix;
-    __shared__ uint32_t s_count[kScanTile];
+    constexpr int kTile = kScanThreads * kEach;
+    __shared__ uint32_t s_count[kTile];
     // difference arrays of the keys per tile column and per tile row: a triangle adds its rows at its first column
     // and takes them off behind its last one, likewise for the rows; the running sums are the digit counts
     __shared__ uint32_t s_diff[kEmitDigitPasses][kRadix + 1];
@@ -683,14 +685,14 @@ __global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1
     }
     lds_barrier();
     const int tile = (int)s_tile;
-    const int64_t base = (int64_t)tile * kScanTile + (int64_t)tid * 4;
+    const int64_t base = (int64_t)tile * kTile + (int64_t)tid * kEach;
 
     // Triangle by triangle across the lanes (neighbouring lanes take neighbouring triangles, so the index
     // loads and the record stores of a wave are contiguous); the counts then change hands through LDS so that
-    // every thread scans four consecutive ones.
+    // every thread scans consecutive ones.
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int64_t t = (int64_t)tile * kScanTile + k * kScanThreads + tid;
+    for (int k = 0; k < kEach; k++) {
+        const int64_t t = (int64_t)tile * kTile + k * kScanThreads + tid;
         uint32_t count = 0;
         Rect rect = {0, -1, 0, -1};
         if (t < n_triangles) {
@@ -736,10 +738,9 @@ __global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1
         for (int w = p * (kRadix / kWave); w < wave; w++) keys_of_digit += s_digit_wave[w];
         if (keys_of_digit) atomicAdd(&totals[p * kRadix + d], keys_of_digit);
     }
-    uint32_t x[4];
+    uint32_t x[kEach], thread_sum = 0;
 #pragma unroll
-    for (int k = 0; k < 4; k++) x[k] = s_count[tid * 4 + k];
-    const uint32_t thread_sum = x[0] + x[1] + x[2] + x[3];
+    for (int k = 0; k < kEach; k++) thread_sum += x[k] = s_count[tid * kEach + k];
     const uint32_t incl = wave_inclusive_scan_u32(thread_sum);
     if (lane == kWave - 1) s_wave_total[wave] = incl;
     lds_barrier();
@@ -754,7 +755,7 @@ __global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1
     lds_barrier();
     uint32_t run = s_tile_prefix + s_wave_total[wave] + (incl - thread_sum);
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < kEach; k++) {
         const int64_t t = base + k;
         if (t >= n_triangles) break;
         tri_offsets[t] = run;
@@ -1192,7 +1193,7 @@ namespace tg {
 struct FusedFrame {
     uint32_t *totals;  // two sets of kEmitDigitPasses * kRadix digit totals
     uint32_t *ticket;
-    uint64_t *states;  // one word per kScanTile triangles
+    uint64_t *states;  // one word per kScanTile triangles (for a few hundred thousand there may be four times as many, and room)
     real *edges;       // tiles_x + 1 column edges, then tiles_y + 1 row edges
     uint32_t *heads;   // the owner of every kEmitChunk-th key position
     uint32_t *tri_offsets;
@@ -1272,15 +1273,22 @@ int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indic
         TG_LAUNCH(bin_frame_empty_kernel, dim3(1), dim3(64), 0, s, total_and_status, fused_frame_totals(frame, epoch + 1), clear_word);
         return check_launch("bin_frame_empty_kernel");
     }
-    const int n_scan_tiles = (int)ceil_div64(n_triangles, kScanTile);
-    static int resident_cache[2][kMaxDevices] = {{0}};
-    static size_t lds_reserved[kMaxDevices] = {0};
-    const auto scan_kernel = records ? frame_scan_kernel<true> : frame_scan_kernel<false>;
+    // Triangles a thread: as few as leave the workgroups no more than the CUs, for a frame of less has CUs to spare and waits for one
+    // triangle after the other.  With 1, 2, 4, us: 1000 triangles 5.7, 6.8, 7, 20 000 7.9, 10.0, 14.6, 10^5 10.9, 12.6, 15.9, 140 000 14.2,
+    // 12.6, 15.9, with records 180 000 20.0, 17.1, 23.0, 250 000 23.0, 19.3, 23.4, 350 000 36, 27.7, 24.6, 10^6 93, 79, 67.
+    const int64_t at_once = (int64_t)256 * kScanThreads;
+    const int each = n_triangles <= at_once && !records ? 1 : n_triangles <= 2 * at_once ? 2 : 4;
+    const int n_scan_tiles = (int)ceil_div64(n_triangles, kScanThreads * each);
+    static int resident_cache[2][5][kMaxDevices] = {{{0}}};
+    static size_t lds_reserved[5][kMaxDevices] = {{0}};
+    const auto scan_kernel = each == 1 ? frame_scan_kernel<false, 1>
+                           : each == 2 ? (records ? frame_scan_kernel<true, 2> : frame_scan_kernel<false, 2>)
+                                       : (records ? frame_scan_kernel<true, 4> : frame_scan_kernel<false, 4>);
     const size_t lds = records ? kRecordLds * (kScanThreads / kWave) : 0;
     if (lds)  // with the kernel's own beyond 64 KB
-        if (int e = reserve_lds("tg_bin_frame", (const void *)scan_kernel, lds + 16, lds_reserved)) return e;
+        if (int e = reserve_lds("tg_bin_frame", (const void *)scan_kernel, lds + 16, lds_reserved[each])) return e;
     uint32_t *ticket = f.ticket;
-    if (n_scan_tiles <= resident_workgroups((const void *)scan_kernel, kScanThreads, resident_cache[records != nullptr], lds)) ticket = nullptr;
+    if (n_scan_tiles <= resident_workgroups((const void *)scan_kernel, kScanThreads, resident_cache[records != nullptr][each], lds)) ticket = nullptr;
     const GridPlan grid = grid_plan(tiles_x, tiles_y);
     TG_LAUNCH_AS("frame_scan_kernel", scan_kernel, dim3(n_scan_tiles), dim3(kScanThreads), lds, s, (const real4 *)vertices, n_vertices, indices, n_triangles,
               width, height, tile_w, tile_h, tiles_x, tiles_y, epoch, f.tri_offsets, f.records, total_and_status, ticket, f.states,
