@@ -172,10 +172,11 @@ constexpr int kTerms = 21;  // per vertex v: [7v+0] x, [7v+1] y, [7v+2] w, [7v+3
 // util.h:299-317 scalar interpolate3_backward.  -> the reference returns early there (util.h:303) and all results are zero: the
 // caller's to set, once for all of a fragment's and in a branch that a wave rarely takes.  (A selection at every result is a branch
 // around its arithmetic, twelve a fragment: the compiler does not move arithmetic across them.)
-// denom: of the b w, inv: its reciprocal (the reference divides nine times, by denom and by its square).
-__device__ __forceinline__ bool interp_backward_scalar(real g, const real b[3], const real v[3], const real w[3], real denom, real inv,
+__device__ __forceinline__ bool interp_backward_scalar(real g, const real b[3], const real v[3], const real w[3],
                                                        real gb[3], real gv[3], real gw[3]) {
     const real nom = (b[0] * w[0] * v[0] + b[1] * w[1] * v[1]) + b[2] * w[2] * v[2];
+    const real denom = (b[0] * w[0] + b[1] * w[1]) + b[2] * w[2];
+    const real inv = reciprocal(denom);  // the reference divides nine times, by denom and by its square
     const real inv2 = inv * inv;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -200,11 +201,9 @@ struct FragSeed {
     real dd_dz;   // derivative w.r.t. the interpolated view depth (:517); with kDepth
 };
 
-// The fragment itself: interpolated opacity, colour and, with kDepth, view depth (no state involved); and what all but the depth are
-// divided by, with its reciprocal.
+// The fragment itself: interpolated opacity, colour and, with kDepth, view depth (no state involved).
 struct FragValue {
     real o, color[3], z;
-    real denom, inv_denom;
 };
 
 template <bool kDepth>
@@ -215,11 +214,10 @@ __device__ __forceinline__ FragValue fragment_value(const BackRecord<kDepth> &r,
     // transmittance is reconstructed by dividing by it.  The three colour quotients over the same
     // denominator (util.h:245-250) share its reciprocal.
     v.o = clampf(interp_w(b0, b1, b2, r.op[0], r.op[1], r.op[2], w[0], w[1], w[2]), 0.0f, kMaxOpacity);
-    v.denom = b0 * w[0] + b1 * w[1] + b2 * w[2];
-    v.inv_denom = reciprocal(v.denom);
+    const real inv_denom = reciprocal(b0 * w[0] + b1 * w[1] + b2 * w[2]);
 #pragma unroll
     for (int k = 0; k < 3; k++)
-        v.color[k] = (b0 * r.col[k] * w[0] + b1 * r.col[3 + k] * w[1] + b2 * r.col[6 + k] * w[2]) * v.inv_denom;
+        v.color[k] = (b0 * r.col[k] * w[0] + b1 * r.col[3 + k] * w[1] + b2 * r.col[6 + k] * w[2]) * inv_denom;
     if constexpr (kDepth) v.z = interp_1(b0, b1, b2, r.iw[0], r.iw[1], r.iw[2]);
     return v;
 }
@@ -277,13 +275,13 @@ __device__ __forceinline__ bool depth_is_ordinary(const real w[3], real denom) {
 
 // The order-free part: the 21 gradient terms of one fragment.
 template <bool kDepth>
-__device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackRecord<kDepth> &r, real denom, real inv, real b0, real b1, real b2,
-                                               real px, real py, real out[kTerms]) {
+__device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackRecord<kDepth> &r, real b0, real b1, real b2, real px,
+                                               real py, real out[kTerms]) {
     const real b[3] = {b0, b1, b2};
     const real w[3] = {r.w[0], r.w[1], r.w[2]};
     const real ones[3] = {1.0f, 1.0f, 1.0f};
     real gb_o[3], gv_o[3], gw_o[3];
-    const bool dead = interp_backward_scalar(f.d_do, b, r.op, w, denom, inv, gb_o, gv_o, gw_o);
+    const bool dead = interp_backward_scalar(f.d_do, b, r.op, w, gb_o, gv_o, gw_o);
 
     // vector interpolate3_backward for the colour (util.h:319-355)
     const real *gc = f.gc;
@@ -292,6 +290,8 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
         real nom[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) nom[k] = (b[0] * w[0] * r.col[k] + b[1] * w[1] * r.col[3 + k]) + b[2] * w[2] * r.col[6 + k];
+        const real denom = b[0] * w[0] + b[1] * w[1] + b[2] * w[2];
+        const real inv = reciprocal(denom);
         const real inv2 = inv * inv;
 #pragma unroll
         for (int v = 0; v < 3; v++) {
@@ -299,10 +299,10 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 const real a = r.col[3 * v + k];
-                dfb[k] = a * denom - nom[k];
+                dfb[k] = w[v] * (a * denom - nom[k]) * inv2;
                 dfw[k] = b[v] * a * denom - nom[k] * b[v];
             }
-            gb_c[v] = ((gc[0] * dfb[0] + gc[1] * dfb[1]) + gc[2] * dfb[2]) * (w[v] * inv2);
+            gb_c[v] = (gc[0] * dfb[0] + gc[1] * dfb[1]) + gc[2] * dfb[2];
             gw_c[v] = ((gc[0] * dfw[0] + gc[1] * dfw[1]) + gc[2] * dfw[2]) * inv2;
             scale[v] = b[v] * w[v] * inv;
         }
@@ -310,8 +310,7 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
 
     real gb_z[3], gv_z[3], gw_z[3];
     bool dead_z = false;
-    const real sum = (b[0] + b[1]) + b[2];  // with unit weights
-    if constexpr (kDepth) dead_z = interp_backward_scalar(f.dd_dz, b, r.iw, ones, sum, reciprocal(sum), gb_z, gv_z, gw_z);
+    if constexpr (kDepth) dead_z = interp_backward_scalar(f.dd_dz, b, r.iw, ones, gb_z, gv_z, gw_z);
     if (any_lane(dead || dead_z)) {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -332,10 +331,10 @@ __device__ __forceinline__ void fragment_terms(const FragSeed &f, const BackReco
     if constexpr (kDepth) {
 #pragma unroll
         for (int k = 0; k < 3; k++) add_depth(k, r.iw2[k]);
-    } else if (any_lane(!depth_is_ordinary(r.w, denom))) {
+    } else if (any_lane(!depth_is_ordinary(r.w, (b[0] * w[0] + b[1] * w[1]) + b[2] * w[2]))) {
         VertexDepths<true> depths;
         vertex_depths(r.w, depths);
-        dead_z = interp_backward_scalar(0.0f, b, depths.iw, ones, sum, reciprocal(sum), gb_z, gv_z, gw_z);
+        dead_z = interp_backward_scalar(0.0f, b, depths.iw, ones, gb_z, gv_z, gw_z);
 #pragma unroll
         for (int k = 0; k < 3; k++) {
             if (dead_z) gb_z[k] = gv_z[k] = gw_z[k] = 0.0f;
@@ -416,7 +415,7 @@ __device__ __forceinline__ void fragment_backward(BackState &st, const BackRecor
     const ChainState next = chain_behind<true>(st, v, rem.om, rem.inv);
     const FragSeed f = fragment_seed<true>(st, next, v, rem.inv, st);
     static_cast<ChainState &>(st) = next;
-    fragment_terms(f, r, v.denom, v.inv_denom, b0, b1, b2, px, py, out);
+    fragment_terms(f, r, b0, b1, b2, px, py, out);
 }
 
 // Layout of the three gradient arrays, a template parameter of the kernels so that the two layouts
@@ -728,7 +727,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
                 BackRecord<kDepth> r;
                 real b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
                 FragValue value;
-                value.o = value.color[0] = value.color[1] = value.color[2] = value.z = value.denom = value.inv_denom = 0.0f;
+                value.o = value.color[0] = value.color[1] = value.color[2] = value.z = 0.0f;
                 if (active) {
                     if constexpr (kPacked) gather_packed(a, mem.id[entry][0], r);
                     else gather_back(a, *reinterpret_cast<const TriIds *>(mem.id[entry]), r);
@@ -738,7 +737,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth ? 4 : 
                 const FragSeed f = walk_chain<kDepth>(value, pixel, slot_before, turns, last_slot, st);
                 if (active) {
                     real term[kTerms];
-                    fragment_terms(f, r, value.denom, value.inv_denom, b0, b1, b2, px, py, term);
+                    fragment_terms(f, r, b0, b1, b2, px, py, term);
 #pragma unroll
                     for (int q = 0; q < kTerms; q++) terms[q * kTermStride + lane] = term[q];
                 }
@@ -1075,7 +1074,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLa
         BackRecord<kDepth> r;
         real b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
         FragValue value;
-        value.o = value.color[0] = value.color[1] = value.color[2] = value.z = value.denom = value.inv_denom = 0.0f;
+        value.o = value.color[0] = value.color[1] = value.color[2] = value.z = 0.0f;
         if (active) {
             if constexpr (kPacked) gather_packed(a, a.sorted_ids[start + rel], r);
             else gather_back(a, load_ids(a, start + rel), r);
@@ -1087,7 +1086,7 @@ __global__ __launch_bounds__(kTileThreads, sizeof(real) != 4 ? 1 : kDepth || kLa
         // 5. the terms
         if (active) {
             real term[kTerms];
-            fragment_terms(f, r, value.denom, value.inv_denom, b0, b1, b2, px, py, term);
+            fragment_terms(f, r, b0, b1, b2, px, py, term);
 #pragma unroll
             for (int q = 0; q < kTerms; q++) terms[q * kTermStride + lane] = term[q];
 #pragma unroll
