@@ -197,7 +197,7 @@ __device__ __forceinline__ void wave_match_rank_ballots(const uint32_t (&digit)[
 
 // One pass over digit (key >> shift) & mask, mask < 2^BITS.  `bases`: the exclusive scan of the digit totals,
 // or, with totals_given, the totals themselves (scanned here).
-template <int BITS>
+template <int BITS, int kItems>
 __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_t *__restrict__ keys_in,
                                                                   const uint32_t *__restrict__ vals_in,
                                                                   uint64_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
                                                                   uint32_t *lookback, uint32_t *ticket, uint32_t *status,
                                                                   int unpad_bits, int tiles_x, uint32_t *tile_count,
                                                                   FrameCount frame_count) {
-    constexpr int kDigits = 1 << BITS;
+    constexpr int kDigits = 1 << BITS, kTile = kSweepThreads * kItems;
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_global_delta[kRadix];
     __shared__ uint32_t s_scan_wave[kSweepWaves];
@@ -214,14 +214,15 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
     __shared__ uint32_t s_several_tiles[kRadix];  // with tile_count: the digit's pairs of this sort tile belong to more than one tile
     // The ranking counters are dead once every pair knows its place in the tile,
     // so they share LDS with the permutation buffer (51 KB: three workgroups per CU).
-    __shared__ __align__(16) unsigned char s_raw[kSortTile * 12];
+    constexpr int kMaskOffset = (kSweepWaves + 1) * kRadix * 4;
+    constexpr int kCounterBytes = kMaskOffset + kSweepWaves * kMaskWords * 8;
+    __shared__ __align__(16) unsigned char s_raw[kTile * 12 > kCounterBytes ? kTile * 12 : kCounterBytes];
     uint32_t (*s_wave_count)[kRadix] = reinterpret_cast<uint32_t (*)[kRadix]>(s_raw);
     uint32_t *s_local_start = reinterpret_cast<uint32_t *>(s_raw) + kSweepWaves * kRadix;
-    constexpr int kMaskOffset = (kSweepWaves + 1) * kRadix * 4;
-    static_assert(kMaskOffset % 8 == 0 && kMaskOffset + kSweepWaves * kMaskWords * 8 <= kSortTile * 12, "counters and mask words fit the permutation buffer");
+    static_assert(kMaskOffset % 8 == 0, "the mask words are aligned");
     unsigned long long *s_masks = reinterpret_cast<unsigned long long *>(s_raw + kMaskOffset);  // kSweepWaves sets of kMaskWords
     uint64_t *s_keys = reinterpret_cast<uint64_t *>(s_raw);
-    uint32_t *s_vals = reinterpret_cast<uint32_t *>(s_raw + kSortTile * 8);
+    uint32_t *s_vals = reinterpret_cast<uint32_t *>(s_raw + kTile * 8);
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -244,21 +245,21 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
         base = wave_prefix + base_incl - base;
     }
     const int tile = (int)s_tile;
-    const int64_t tile_base = (int64_t)tile * kSortTile;
+    const int64_t tile_base = (int64_t)tile * kTile;
     // with the number of pairs on the device the grid is made for the buffers' capacity: the rest has nothing to do
     n = frame_count.pairs(n);
-    const int n_tiles = frame_count.word ? (int)((n + kSortTile - 1) / kSortTile) : (int)gridDim.x;
+    const int n_tiles = frame_count.word ? (int)((n + kTile - 1) / kTile) : (int)gridDim.x;
     if (tile >= n_tiles) return;
-    const int n_valid = (int)((n - tile_base) < kSortTile ? (n - tile_base) : kSortTile);
+    const int n_valid = (int)((n - tile_base) < kTile ? (n - tile_base) : kTile);
 
     // Wave-striped loads keep memory order = (wave, item, lane) order.
-    uint64_t key[kSweepItems];
-    uint32_t val[kSweepItems];
-    uint32_t digit[kSweepItems];
-    uint32_t rank[kSweepItems];
-    const int lane_base = wave * (kWave * kSweepItems) + lane;
+    uint64_t key[kItems];
+    uint32_t val[kItems];
+    uint32_t digit[kItems];
+    uint32_t rank[kItems];
+    const int lane_base = wave * (kWave * kItems) + lane;
 #pragma unroll
-    for (int i = 0; i < kSweepItems; i++) {
+    for (int i = 0; i < kItems; i++) {
         const int local = lane_base + i * kWave;
         if (local < n_valid) {
             key[i] = keys_in[tile_base + local];
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
         }
         digit[i] = (uint32_t)(key[i] >> shift) & mask;
     }
-    wave_match_rank<kSweepItems>(digit, s_wave_count[wave], s_masks + wave * kMaskWords, rank);
+    wave_match_rank<kItems>(digit, s_wave_count[wave], s_masks + wave * kMaskWords, rank);
     __syncthreads();
 
     // Thread d owns digit d: per-wave exclusive offsets, tile count, look-back.
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
         }
     }
     // real pairs only: padding always carries the largest digit
-    const uint32_t published = ((uint32_t)tid == mask) ? digit_count - (uint32_t)(kSortTile - n_valid) : digit_count;
+    const uint32_t published = ((uint32_t)tid == mask) ? digit_count - (uint32_t)(kTile - n_valid) : digit_count;
     uint32_t *my_words = lookback + tid;
     if (owns_digit)
         __hip_atomic_store(my_words + (size_t)tile * kDigits, kLbAggregate | published, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -303,10 +304,10 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
     __syncthreads();  // s_local_start is complete
     const uint32_t local_start = s_local_start[tid & (kRadix - 1)];
 #pragma unroll
-    for (int i = 0; i < kSweepItems; i++) rank[i] += s_local_start[digit[i]] + s_wave_count[wave][digit[i]];
+    for (int i = 0; i < kItems; i++) rank[i] += s_local_start[digit[i]] + s_wave_count[wave][digit[i]];
     __syncthreads();  // every pair knows its place: the counters may be overwritten
 #pragma unroll
-    for (int i = 0; i < kSweepItems; i++) {
+    for (int i = 0; i < kItems; i++) {
         s_keys[rank[i]] = key[i];
         s_vals[rank[i]] = val[i];
     }
@@ -394,7 +395,7 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
         __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < kSweepItems; i++) {
+    for (int i = 0; i < kItems; i++) {
         const int pos = i * kSweepThreads + tid;
         if (pos < n_valid) {
             uint64_t k = s_keys[pos];
@@ -991,11 +992,12 @@ __global__ __launch_bounds__(kSortThreads) void tile_ranges_kernel(const uint64_
 }
 
 template <int BITS>
-static void launch_sweep(dim3 grid, hipStream_t s, const uint64_t *kin, const uint32_t *vin, uint64_t *kout, uint32_t *vout,
+static void launch_sweep(int items, dim3 grid, hipStream_t s, const uint64_t *kin, const uint32_t *vin, uint64_t *kout, uint32_t *vout,
                          int64_t n, int shift, uint32_t mask, const uint32_t *bases, int totals_given, uint32_t *lookback,
                          uint32_t *ticket, uint32_t *status, int unpad_bits, int tiles_x, uint32_t *tile_count,
                          FrameCount frame_count) {
-    hipLaunchKernelGGL(sort_sweep_kernel<BITS>, grid, dim3(kSweepThreads), 0, s, kin, vin, kout, vout, n, shift, mask, bases,
+    const auto kernel = items == 2 ? sort_sweep_kernel<BITS, 2> : items == 4 ? sort_sweep_kernel<BITS, 4> : sort_sweep_kernel<BITS, kSweepItems>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kSweepThreads), 0, s, kin, vin, kout, vout, n, shift, mask, bases,
                        totals_given, lookback, ticket, status, unpad_bits, tiles_x, tile_count, frame_count);
 }
 
@@ -1003,7 +1005,8 @@ static void launch_sweep(dim3 grid, hipStream_t s, const uint64_t *kin, const ui
 // exclusive scan of the digit totals or (totals_given) the totals; lookback: per pass n_sort_tiles * kRadix
 // words, zero; tickets: one word per pass, zero.
 // unpad_bits, tiles_x, tile_count: for the last pass of a sort by tile column and row (see the kernel), else 0.
-static int run_sweeps(const char *fn, const PassPlan &plan, int n_sort_tiles, const uint32_t *bases, int totals_given,
+// items: pairs of a sort tile for each of its threads.
+static int run_sweeps(const char *fn, const PassPlan &plan, int items, int n_sort_tiles, const uint32_t *bases, int totals_given,
                       uint32_t *lookback, uint32_t *tickets, uint64_t *keys, uint32_t *values, uint64_t *keys_alt,
                       uint32_t *values_alt, int64_t n, uint32_t *status, hipStream_t s, int unpad_bits = 0, int tiles_x = 0,
                       uint32_t *tile_count = nullptr, FrameCount frame_count = FrameCount()) {
@@ -1011,8 +1014,9 @@ static int run_sweeps(const char *fn, const PassPlan &plan, int n_sort_tiles, co
     uint32_t *vin = values, *vout = values_alt;
     // 534 same-address ticket atomics cost 6 us per pass; a grid that fits the device whole takes its
     // tile numbers from the workgroup ids instead
-    static int resident_cache[kMaxDevices] = {0};
-    const bool whole_grid_resident = n_sort_tiles <= resident_workgroups((const void *)sort_sweep_kernel<kRadixBits>, kSweepThreads, resident_cache);
+    static int resident_cache[kSweepItems + 1][kMaxDevices] = {{0}};
+    const auto widest = items == 2 ? sort_sweep_kernel<kRadixBits, 2> : items == 4 ? sort_sweep_kernel<kRadixBits, 4> : sort_sweep_kernel<kRadixBits, kSweepItems>;
+    const bool whole_grid_resident = n_sort_tiles <= resident_workgroups((const void *)widest, kSweepThreads, resident_cache[items]);
     // one pair of timing events around all passes: a pair per launch would add its own two
     // microseconds to every 24 us kernel
     ProfileScope timed("sort_sweep_kernel", s, plan.passes);
@@ -1026,11 +1030,11 @@ static int run_sweeps(const char *fn, const PassPlan &plan, int n_sort_tiles, co
         const int ub = last ? unpad_bits : 0;
         uint32_t *tc = last ? tile_count : (uint32_t *)nullptr;
         switch (plan.bits[p]) {
-        case 8: launch_sweep<8>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
-        case 7: launch_sweep<7>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
-        case 6: launch_sweep<6>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
-        case 5: launch_sweep<5>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
-        default: launch_sweep<4>(grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        case 8: launch_sweep<8>(items, grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        case 7: launch_sweep<7>(items, grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        case 6: launch_sweep<6>(items, grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        case 5: launch_sweep<5>(items, grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
+        default: launch_sweep<4>(items, grid, s, kin, vin, kout, vout, n, plan.shift[p], mask, b, totals_given, lb, ticket, status, ub, tiles_x, tc, frame_count); break;
         }
         if (int e = check_launch(fn)) return e;
         uint64_t *tk = kin; kin = kout; kout = tk;
@@ -1051,7 +1055,7 @@ static int run_passes(const char *fn, const PassPlan &plan, const SortLayout &L,
     if (int e = check_launch("sort_histogram_kernel")) return e;
     TG_LAUNCH(sort_bases_kernel, dim3(plan.passes), dim3(kBasesThreads), 0, s, partials, L.hist_blocks, bases, status);
     if (int e = check_launch("sort_bases_kernel")) return e;
-    return run_sweeps(fn, plan, L.n_tiles, bases, 0, lookback, tickets, keys, values, keys_alt, values_alt, n, status, s);
+    return run_sweeps(fn, plan, kSweepItems, L.n_tiles, bases, 0, lookback, tickets, keys, values, keys_alt, values_alt, n, status, s);
 }
 
 // Every tile's segment of keys that are ordered by tile sorted by its depth bits in place.  With tile_count (the last sweep
@@ -1199,6 +1203,20 @@ static size_t build_lookback_bytes(int64_t n_keys, int n_tiles) {
     return (size_t)plan.passes * lookback_words_per_pass(n_sort_tiles > 0 ? n_sort_tiles : 1) * 4;
 }
 
+// Pairs a thread of the sweeps: as few as leave a sort tile for each CU, or two, for then a pass is the latency of one tile, which goes with
+// its pairs; more tiles than run at once wait for those before them.  Both passes, us, with 2, 4, 8: 10 000 keys 15.0, 15.4, 18.5, 60 000 18.0,
+// 19.5, 22, 200 000 20.0, 20.7, 24.5, 300 000 21.2, 21.7, 25.3, 500 000 26.8, 26.4, 28.4, 750 000 45, 29.4, 30.8, 1.5 million 76, 51, 38.
+constexpr int kTwoItemTiles = 256, kFourItemTiles = 512;
+static int frame_sweep_items(int64_t n_keys) {
+    return n_keys <= kTwoItemTiles * 2 * kSweepThreads ? 2 : n_keys <= kFourItemTiles * 4 * kSweepThreads ? 4 : kSweepItems;
+}
+static int64_t frame_sort_tiles(int64_t n_keys) { return ceil_div64(n_keys > 0 ? n_keys : 1, kSweepThreads * frame_sweep_items(n_keys)); }
+// The most sort tiles that n_keys or fewer have: a workspace serves fewer keys than it was made for.
+static int64_t most_frame_sort_tiles(int64_t n_keys) {
+    const int items = frame_sweep_items(n_keys);
+    return std::max<int64_t>(frame_sort_tiles(n_keys), items == 2 ? 0 : items == 4 ? kTwoItemTiles : kFourItemTiles);
+}
+
 constexpr size_t kFrameSortHeadBytes = 256;  // tg_build_frame_lists: the sweeps' tickets in front of the look-back words
 extern "C" size_t tg_build_tile_lists_workspace_bytes(int64_t n_keys, int n_tiles) {
     if (n_keys < 0 || n_keys > kSortMaxN || n_tiles <= 0) return 0;
@@ -1260,7 +1278,7 @@ extern "C" int tg_build_tile_lists(const real *records, const uint32_t *tri_offs
     const PassPlan plan = tile_pass_plan(n_tiles);
     const int tiles_x = ceil_div(width, tile_w), tiles_y = ceil_div(height, tile_h);
     uint32_t *tickets = frame_tickets(frame);
-    if (int e = run_sweeps("tg_build_tile_lists", plan, (int)ceil_div64(n_keys, kSortTile), frame_totals(frame, n_triangles, tiles_x, tiles_y),
+    if (int e = run_sweeps("tg_build_tile_lists", plan, kSweepItems, (int)ceil_div64(n_keys, kSortTile), frame_totals(frame, n_triangles, tiles_x, tiles_y),
                            1, lookback, tickets + kSweepTicketWord, keys, values, keys_alt, values_alt, n_keys, status, s))
         return e;
     uint64_t *k = (plan.passes & 1) ? keys_alt : keys, *k_other = (plan.passes & 1) ? keys : keys_alt;
@@ -1278,7 +1296,7 @@ extern "C" size_t tg_build_frame_lists_workspace_bytes(int64_t n_keys, int tiles
     const int n_tiles = tiles_x * tiles_y;
     if (!grid_plan(tiles_x, tiles_y).on) return tg_tile_list_sort_workspace_bytes(n_keys, n_tiles);
     // two passes of at most 256 digits each
-    return kFrameSortHeadBytes + 2 * lookback_words_per_pass(ceil_div64(n_keys > 0 ? n_keys : 1, kSortTile)) * 4 + (size_t)(n_tiles + 1) * 4;
+    return kFrameSortHeadBytes + 2 * lookback_words_per_pass(most_frame_sort_tiles(n_keys)) * 4 + (size_t)(n_tiles + 1) * 4;
 }
 
 bool tg::frame_grid_fits(int tiles_x, int tiles_y) { return grid_plan(tiles_x, tiles_y).on; }
@@ -1314,7 +1332,7 @@ int tg::build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, const uin
         return sort_tile_lists_run("tg_build_frame_lists", keys, values, keys_alt, values_alt, n_keys, n_tiles, offsets, workspace,
                                    workspace_bytes, status, result_in_alt, s);
     if (int e = check_sort_buffers("tg_build_frame_lists", keys, values, keys_alt, values_alt, workspace)) return e;
-    const int n_sort_tiles = (int)ceil_div64(n_keys, kSortTile);
+    const int n_sort_tiles = (int)frame_sort_tiles(n_keys);
     const size_t lookback_bytes = 2 * lookback_words_per_pass(n_sort_tiles) * 4;
     const size_t need = kFrameSortHeadBytes + lookback_bytes + (size_t)(n_tiles + 1) * 4;
     if (workspace_bytes < need) {
@@ -1336,7 +1354,7 @@ int tg::build_frame_lists(void *frame, uint32_t epoch, int64_t n_keys, const uin
         return by_depth ? 0 : sort_segments(keys, values, keys_alt, values_alt, n_keys, n_tiles, offsets, s, nullptr, nullptr, 0, count,
                                             status, longest, LongTiles());
     }
-    if (int e = run_sweeps("tg_build_frame_lists", grid.plan, n_sort_tiles, totals, 1, lookback, tickets, keys, values, keys_alt,
+    if (int e = run_sweeps("tg_build_frame_lists", grid.plan, frame_sweep_items(n_keys), n_sort_tiles, totals, 1, lookback, tickets, keys, values, keys_alt,
                            values_alt, n_keys, status, s, grid.column_bits, tiles_x, tile_count, count))
         return e;
     // two passes: the sorted pairs are back in (keys, values)
