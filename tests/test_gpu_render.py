@@ -1717,7 +1717,7 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
                                                      (131071, 640, 480, 16, 1.0), (131072, 640, 480, 16, 0.3), (131073, 640, 480, 16, 1.0),
                                                      (262144, 1000, 700, 16, 0.5), (262145, 1000, 700, 16, 2.0), (600000, 1000, 700, 16, 3.0)])
 def test_lists_of_frames_around_the_sizes_that_split_the_work_otherwise(n, width, height, tw, sigma, cuda, monkeypatch):
-    """The scan takes 1, 2 or 4 triangles a thread and the sweeps 2, 4 or 8 pairs: frames on both sides of every line have the lists
+    """The scan takes 1, 2 or 4 triangles a thread, the emission 1 or 2 keys and the sweeps 2, 4 or 8 pairs: frames on both sides of every line have the lists
     of the route by stages, which knows none of them."""
     import torch
     import scenes as S

@@ -498,7 +498,7 @@ __global__ __launch_bounds__(kBinThreads) void bin_emit_records_kernel(const rea
 //                     nothing has to be cleared before the launch: a state word of another epoch is "not yet
 //                     written".  The digit totals go to one of two sets in turn (a call counts into one and
 //                     clears the other).  The look-back reads 512 predecessors per round trip.
-// frame_emit_kernel   one workgroup per kEmitChunk key positions.  It reads K from the device, so it is launched
+// frame_emit_kernel   one workgroup per 256 or 512 key positions.  It reads K from the device, so it is launched
 //                     for the capacity of the key buffers before the host knows K.  Per key it runs only those
 //                     of the four clip passes that can change the polygon, and keys that run the same number of
 //                     passes are put on the same wave.
@@ -510,8 +510,8 @@ __global__ __launch_bounds__(kBinThreads) void bin_emit_records_kernel(const rea
 // test of every vertex, whenever they do not: the polygon is the reference's in every case.
 constexpr int kEmitThreads = 256;
 [[maybe_unused]] constexpr int kEmitWaves = kEmitThreads / kWave;
-constexpr int kEmitKeys = 2;  // keys per thread
-constexpr int kEmitChunk = kEmitThreads * kEmitKeys;
+constexpr int kEmitBits = 8;  // key positions a workgroup takes with one key a thread: the least
+static_assert(kEmitThreads == 1 << kEmitBits, "a chunk is a shift");
 constexpr int kFrameMaxTiles = 1 << 21;  // the reciprocal multiply finds a key's column exactly up to here
 constexpr int kFrameTotalsWords = 2 * kEmitDigitPasses * kRadix;  // two sets: a call counts into one and clears the other
 constexpr int kLookSlots = 8;  // state words a lane of the look-back reads per round trip
@@ -649,7 +649,8 @@ __global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1
                                                                   int n_scan_tiles, uint32_t head_capacity, uint32_t *__restrict__ heads,
                                                                   uint32_t *totals, uint32_t *totals_next,
                                                                   real *__restrict__ edges, uint32_t *zero, size_t zero_words,
-                                                                  uint32_t *clear_word, real *__restrict__ bary, PackedOut packed) {
+                                                                  uint32_t *clear_word, real *__restrict__ bary, PackedOut packed,
+                                                                  int chunk_bits) {
     extern __shared__ __align__(16) unsigned char s_records[];  // kRecordLds for each wave, with records
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_wave_total[kScanThreads / kWave];
@@ -760,8 +761,8 @@ __global__ __launch_bounds__(kScanThreads, kRecords && sizeof(real) == 4 ? 4 : 1
         if (t >= n_triangles) break;
         tri_offsets[t] = run;
         if (x[k] != 0) {
-            // triangle t owns the key positions [run, run + x): note for every multiple of kEmitChunk who owns it
-            const uint32_t first = (run + kEmitChunk - 1) / kEmitChunk, last = (run + x[k] - 1) / kEmitChunk;
+            // triangle t owns the key positions [run, run + x): note for every chunk's first one who owns it
+            const uint32_t first = (run + (1u << chunk_bits) - 1) >> chunk_bits, last = (run + x[k] - 1) >> chunk_bits;
             for (uint32_t h = first; h <= last && h < head_capacity; h++) heads[h] = (uint32_t)t;
         }
         run += x[k];
@@ -784,10 +785,11 @@ __device__ __forceinline__ uint32_t wave_inclusive_max_u32(uint32_t v) {
     return v;
 }
 
+template <int kKeys>  // keys a thread
 struct EmitLds {
     PolyLdsOf<kEmitThreads> poly;  // the polygon of the key a thread clips
-    uint32_t owner[kEmitChunk];    // per key position of the chunk: first the marks of the triangles' first keys, then the owners
-    uint16_t queue[kEmitChunk];    // the chunk's keys that need clipping, those with the most passes first
+    uint32_t owner[kKeys * kEmitThreads];  // per key position of the chunk: first the marks of the triangles' first keys, then the owners
+    uint16_t queue[kKeys * kEmitThreads];  // the chunk's keys that need clipping, those with the most passes first
     uint32_t wave_owner[kEmitWaves];
     uint32_t bucket[4];            // keys of the chunk with 4, 3, 2, 1 passes to run
 };
@@ -832,13 +834,15 @@ __device__ __forceinline__ uint32_t frame_key_passes(const FrameKey &k) {
     return todo;
 }
 
+template <int kKeys>
 __global__ __launch_bounds__(kEmitThreads) void frame_emit_kernel(const real4 *__restrict__ records, const uint32_t *__restrict__ tri_offsets,
                                                                   int n_triangles, const uint32_t *__restrict__ total_and_status,
                                                                   uint32_t key_capacity, const uint32_t *__restrict__ heads,
                                                                   uint32_t head_capacity, const real *__restrict__ edges, int tiles_x,
                                                                   int column_bits, uint64_t *__restrict__ keys,
                                                                   uint32_t *__restrict__ payload, uint32_t epoch, uint64_t *host_total) {
-    __shared__ EmitLds L;
+    constexpr int kChunk = kKeys * kEmitThreads;
+    __shared__ EmitLds<kKeys> L;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
@@ -850,52 +854,56 @@ __global__ __launch_bounds__(kEmitThreads) void frame_emit_kernel(const real4 *_
                            __HIP_MEMORY_SCOPE_SYSTEM);
     // keys beyond the buffers are left out; after an expired wait the heads and offsets may be another call's, so no key is made
     const uint32_t n_keys = expired ? 0u : total < key_capacity ? total : key_capacity;
-    const uint32_t k0 = blockIdx.x * (uint32_t)kEmitChunk;
+    const uint32_t k0 = blockIdx.x * (uint32_t)kChunk;
     if (k0 >= n_keys) return;
     // The owners of the chunk's keys lie between the owner of its first key and the owner of the next chunk's
     // first key; the scan noted both (otherwise two uniform binary searches find them).
     int t_first, t_last;
     if (blockIdx.x < head_capacity) {
         t_first = (int)heads[blockIdx.x];
-        t_last = (k0 + kEmitChunk < total && blockIdx.x + 1 < head_capacity) ? (int)heads[blockIdx.x + 1] : n_triangles - 1;
+        t_last = (k0 + kChunk < total && blockIdx.x + 1 < head_capacity) ? (int)heads[blockIdx.x + 1] : n_triangles - 1;
     } else {
-        const uint32_t k_last = (k0 + kEmitChunk <= n_keys ? k0 + kEmitChunk : n_keys) - 1;
+        const uint32_t k_last = (k0 + kChunk <= n_keys ? k0 + kChunk : n_keys) - 1;
         t_first = owner_of_key(tri_offsets, n_triangles, k0);
         t_last = owner_of_key(tri_offsets, n_triangles, k_last);
     }
     const int span = t_last - t_first + 1;
     L.owner[tid] = 0;
-    L.owner[kEmitThreads + tid] = 0;
+    if (kKeys == 2) L.owner[(kKeys - 1) * kEmitThreads + tid] = 0;
     if (tid < 4) L.bucket[tid] = 0;
     lds_barrier();
     // every triangle of the span marks the position of its first key in the chunk with its number (+ 1); of
     // several triangles at one position (all but the last own no key) the last counts
     for (int i = tid; i < span; i += kEmitThreads) {
         const uint32_t off = tri_offsets[t_first + i];
-        if (off < k0 + kEmitChunk) atomicMax(&L.owner[off > k0 ? off - k0 : 0u], (uint32_t)i + 1u);
+        if (off < k0 + kChunk) atomicMax(&L.owner[off > k0 ? off - k0 : 0u], (uint32_t)i + 1u);
     }
     lds_barrier();
     // a running maximum over the marks gives every key position its triangle
     {
-        uint32_t m0 = L.owner[2 * tid], m1 = L.owner[2 * tid + 1];
-        m1 = m1 > m0 ? m1 : m0;
-        const uint32_t wmax = wave_inclusive_max_u32(m1);
+        uint32_t mark[kKeys];
+#pragma unroll
+        for (int i = 0; i < kKeys; i++) {
+            mark[i] = L.owner[kKeys * tid + i];
+            if (i && mark[i - 1] > mark[i]) mark[i] = mark[i - 1];
+        }
+        const uint32_t wmax = wave_inclusive_max_u32(mark[kKeys - 1]);
         if (lane == kWave - 1) L.wave_owner[wave] = wmax;
         uint32_t before = (uint32_t)__shfl_up((int)wmax, 1, kWave);
         if (lane == 0) before = 0;
         lds_barrier();
         for (int w = 0; w < wave; w++) before = L.wave_owner[w] > before ? L.wave_owner[w] : before;
-        L.owner[2 * tid] = m0 > before ? m0 : before;
-        L.owner[2 * tid + 1] = m1 > before ? m1 : before;
+#pragma unroll
+        for (int i = 0; i < kKeys; i++) L.owner[kKeys * tid + i] = mark[i] > before ? mark[i] : before;
     }
     lds_barrier();
 
     // every key of the chunk, neighbouring keys on neighbouring lanes: its tile and the passes it needs.  A key
     // that needs none is done here (its polygon is the triangle, render.cu:262-267); the others queue up by
     // their number of passes.
-    uint32_t entry[kEmitKeys], slot[kEmitKeys];
+    uint32_t entry[kKeys], slot[kKeys];
 #pragma unroll
-    for (int k = 0; k < kEmitKeys; k++) {
+    for (int k = 0; k < kKeys; k++) {
         const uint32_t in_chunk = (uint32_t)k * kEmitThreads + tid, at = k0 + in_chunk;
         uint32_t e = 0, at_slot = 0;
         if (at < n_keys) {
@@ -925,7 +933,7 @@ __global__ __launch_bounds__(kEmitThreads) void frame_emit_kernel(const real4 *_
     const uint32_t b4 = L.bucket[0], b3 = L.bucket[1], b2 = L.bucket[2], b1 = L.bucket[3];
     const uint32_t queued = b4 + b3 + b2 + b1;
 #pragma unroll
-    for (int k = 0; k < kEmitKeys; k++)
+    for (int k = 0; k < kKeys; k++)
         if (entry[k]) {
             const int passes = __builtin_popcount(entry[k] & 15u);
             const uint32_t first = passes == 4 ? 0u : passes == 3 ? b4 : passes == 2 ? b4 + b3 : b4 + b3 + b2;
@@ -937,7 +945,7 @@ __global__ __launch_bounds__(kEmitThreads) void frame_emit_kernel(const real4 *_
     for (uint32_t q = (uint32_t)wave * kWave; q < queued; q += kEmitThreads) {
         if (q + lane >= queued) continue;
         const uint32_t e = L.queue[q + lane];
-        const uint32_t in_chunk = (e >> 4) & (kEmitChunk - 1), at = k0 + in_chunk;
+        const uint32_t in_chunk = (e >> 4) & (kChunk - 1), at = k0 + in_chunk;
         uint32_t todo = e & 15u;
         const uint32_t m = L.owner[in_chunk];
         const int t = t_first + (m ? (int)m - 1 : 0);
@@ -1195,7 +1203,7 @@ struct FusedFrame {
     uint32_t *ticket;
     uint64_t *states;  // one word per kScanTile triangles (for a few hundred thousand there may be four times as many, and room)
     real *edges;       // tiles_x + 1 column edges, then tiles_y + 1 row edges
-    uint32_t *heads;   // the owner of every kEmitChunk-th key position
+    uint32_t *heads;   // the owner of a chunk's first key position, for each chunk
     uint32_t *tri_offsets;
     real4 *records;
     uint32_t head_capacity;
@@ -1213,7 +1221,7 @@ static FusedFrame fused_frame(void *base, int64_t n_triangles, int64_t key_capac
     // for any number where there are more.
     f.states = (uint64_t *)take((size_t)((n_triangles <= 1 << 24 ? 1 << 24 : 1ll << 31) / kScanTile + 1) * 8);
     f.edges = (real *)take((size_t)(tiles_x + tiles_y + 2) * sizeof(real));
-    f.head_capacity = (uint32_t)(key_capacity / kEmitChunk + 2);
+    f.head_capacity = (uint32_t)((key_capacity >> kEmitBits) + 2);
     f.heads = (uint32_t *)take((size_t)f.head_capacity * 4);
     f.tri_offsets = (uint32_t *)take((size_t)n_triangles * 4);
     f.records = (real4 *)take((size_t)n_triangles * kRecordReals * sizeof(real));
@@ -1287,6 +1295,11 @@ int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indic
     const size_t lds = records ? kRecordLds * (kScanThreads / kWave) : 0;
     if (lds)  // with the kernel's own beyond 64 KB
         if (int e = reserve_lds("tg_bin_frame", (const void *)scan_kernel, lds + 16, lds_reserved[each])) return e;
+    // Keys a thread of the emission: one as long as all its workgroups run at once (eight a CU, by their LDS), for then the kernel is
+    // the latency of one; two beyond, where the search for a chunk's owners counts.  Kernel, us, with two and one: 2600 keys 12.4, 8.4,
+    // 216 000 11.5, 9.6, 271 000 around a camera 14.0, 11.1, 277 000 16.3, 12.9, 380 000 16.7, 14.7, 585 000 12.4, 13.8, 1.6 million 25.7, 27.2.
+    constexpr int64_t kOneKeyCapacity = (int64_t)256 * 8 * kEmitThreads;
+    const int chunk_bits = key_capacity <= kOneKeyCapacity ? kEmitBits : kEmitBits + 1;
     uint32_t *ticket = f.ticket;
     if (n_scan_tiles <= resident_workgroups((const void *)scan_kernel, kScanThreads, resident_cache[records != nullptr][each], lds)) ticket = nullptr;
     const GridPlan grid = grid_plan(tiles_x, tiles_y);
@@ -1294,11 +1307,12 @@ int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indic
               width, height, tile_w, tile_h, tiles_x, tiles_y, epoch, f.tri_offsets, f.records, total_and_status, ticket, f.states,
               n_scan_tiles, f.head_capacity, f.heads, grid.on ? fused_frame_totals(frame, epoch) : (uint32_t *)nullptr,
               fused_frame_totals(frame, epoch + 1), f.edges, (uint32_t *)zero, zero_bytes / 4, clear_word, bary,
-              PackedOut{colors, opacities, records});
+              PackedOut{colors, opacities, records}, chunk_bits);
     if (int e = check_launch("frame_scan_kernel")) return e;
     if (key_capacity == 0) return 0;
     // for every key position the buffers hold: the kernel reads K and the workgroups behind it leave at once
-    TG_LAUNCH(frame_emit_kernel, dim3((unsigned)ceil_div64(key_capacity, kEmitChunk)), dim3(kEmitThreads), 0, s, f.records, f.tri_offsets,
+    const auto emit_kernel = chunk_bits == kEmitBits ? frame_emit_kernel<1> : frame_emit_kernel<2>;
+    TG_LAUNCH_AS("frame_emit_kernel", emit_kernel, dim3((unsigned)ceil_div64(key_capacity, 1 << chunk_bits)), dim3(kEmitThreads), 0, s, f.records, f.tri_offsets,
               n_triangles, total_and_status, (uint32_t)key_capacity, f.heads, f.head_capacity, f.edges, tiles_x,
               grid.on ? grid.column_bits : 0, keys, values, epoch, host_total);
     return check_launch("frame_emit_kernel");
