@@ -465,7 +465,10 @@ int tg_frame_gradient_copies(const tg_frame *f);
 int tg_frame_supported(int width, int height, int tile_w, int tile_h);
 int tg_frame_layout(const tg_frame *f, int64_t *out);
 /* Whether the frame makes a record of 32 scalars for each triangle, the first nine of which are its bary matrix, where else the
- * matrices lie: with TG_FRAME_RECORDS, for many triangles that share few vertices. */
+ * matrices lie: with TG_FRAME_RECORDS, for many triangles that share few vertices.  Then TG_FRAME_BIN reads colors and opacities,
+ * which may not be null, and keeps them in the records with the indices and the vertices' z and w: the blend kernels of
+ * TG_FRAME_RASTER and of the backward call take them from there, and from the arrays only the vertices' x and y (backward), so
+ * all of these are to stay as they are in between. */
 int tg_frame_has_records(const tg_frame *f);
 int tg_frame_forward(tg_frame *f);
 int tg_frame_backward(const tg_frame *f);

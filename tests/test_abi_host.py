@@ -330,6 +330,26 @@ def test_backward_frame_takes_the_number_of_blocks_it_is_given():
             assert lib.tg_frame_backward((C.c_char * _C._FRAME_BYTES).from_buffer(call)) == code, (per_pixel_sort, blocks, block)
 
 
+@pytest.mark.parametrize("missing", ["colors", "opacities"])
+@pytest.mark.parametrize("phases", ["_FRAME_BIN", "all"])
+def test_frames_with_records_are_refused_without_what_the_records_are_made_of(phases, missing):
+    """The binning reads colours and opacities where it makes triangles' records: a null one of them is refused there, before
+    anything is launched, and not found out by the kernel."""
+    from trigrad_amd import _C, _lib
+    lib, n, somewhere = _lib.load(32), 1_000_000, 1 << 20
+    plan = _C._FramePlan(3 * n, n, 1920, 1080, 16, 16, 1, 32, 3_000_000, _C._FRAME_RECORDS, 0.0)
+    call = bytearray(_C._FRAME_BYTES)
+    host = (C.c_uint64 * 2)()  # four words
+    phases = _C._FRAME_BIN if phases == "_FRAME_BIN" else _C._FRAME_BIN | _C._FRAME_LISTS | _C._FRAME_RASTER | _C._FRAME_WAIT
+    _C._FRAME_CALL.pack_into(call, 0, somewhere, somewhere, 0 if missing == "colors" else somewhere, 0 if missing == "opacities" else somewhere,
+                             somewhere, somewhere, somewhere, somewhere, somewhere, C.addressof(host), 0, 1,
+                             plan.frame_bytes, phases, 0, 0, 0, 0)
+    call[-_C._FRAME_KIND.size:] = plan.kind
+    assert lib.tg_frame_has_records((C.c_char * _C._FRAME_BYTES).from_buffer(call))
+    assert lib.tg_frame_forward((C.c_char * _C._FRAME_BYTES).from_buffer(call)) == -1
+    assert b"null colors or opacities" in lib.tg_last_error()
+
+
 @pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
 def test_state_words_of_the_frame_scan_keep_their_place(few, many):
     """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more

@@ -1270,6 +1270,10 @@ int tg::bin_frame(const real *vertices, int32_t n_vertices, const int32_t *indic
         set_error("tg_bin_frame: null or misaligned pointer, key_capacity outside [0, 2^30), or an epoch whose low 30 bits are 0");
         return TG_E_ARG;
     }
+    if (records && (!colors || !opacities)) {  // the scan reads them then, in front of the blend kernels' own check
+        set_error("tg_frame_forward: null colors or opacities, which the triangles' records are made of");
+        return TG_E_ARG;
+    }
     const int tiles_x = ceil_div(width, tile_w), tiles_y = ceil_div(height, tile_h);
     const FusedFrame f = fused_frame(frame, n_triangles, key_capacity, tiles_x, tiles_y);
     if (frame_bytes < f.bytes) {
