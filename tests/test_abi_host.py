@@ -350,6 +350,23 @@ def test_frames_with_records_are_refused_without_what_the_records_are_made_of(ph
     assert b"null colors or opacities" in lib.tg_last_error()
 
 
+def test_whether_a_frame_has_records_is_asked_of_any_frame():
+    """A frame that the forward call refuses has none: a size of zero is no division, a null frame no read."""
+    from trigrad_amd import _C, _lib
+    lib, n = _lib.load(32), 1_000_000
+    good = dict(n_vertices=3 * n, n_triangles=n, width=1920, height=1080, tile_w=16, tile_h=16, per_pixel_sort=1, max_layers=32, key_capacity=3_000_000)
+
+    def has_records(**changed):
+        kind = dict(good, **changed)
+        return lib.tg_frame_has_records(bytes(_C._FRAME_CALL.size + _C._FRAME_RESULT.size) + _C._FRAME_KIND.pack(*kind.values(), _C._FRAME_RECORDS, 0, 0, 0.0))
+
+    assert has_records() == 1 and lib.tg_frame_has_records(None) == 0
+    for field in ("width", "height", "tile_w", "tile_h"):
+        for size in (0, -1, -16, 1 << 40):
+            assert has_records(**{field: size}) == 0
+    assert has_records(key_capacity=1 << 30) == 0 and has_records(n_triangles=1 << 31, n_vertices=1 << 33) == 0
+
+
 @pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
 def test_state_words_of_the_frame_scan_keep_their_place(few, many):
     """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more

@@ -156,7 +156,7 @@ extern "C" int tg_frame_has_records(const tg_frame *) { return 0; }
 extern "C" int tg_frame_forward(tg_frame *) { return no_frame("tg_frame_forward"); }
 extern "C" int tg_frame_backward(const tg_frame *) { return no_frame("tg_frame_backward"); }
 #else
-extern "C" int tg_frame_has_records(const tg_frame *f) { return f && has_records(*f); }
+extern "C" int tg_frame_has_records(const tg_frame *f) { return check_frame("tg_frame_has_records", f) == 0 && has_records(*f); }
 
 extern "C" int tg_frame_layout(const tg_frame *f, int64_t *out) {
     if (int e = check_frame("tg_frame_layout", f)) return e;
