@@ -367,6 +367,21 @@ def test_whether_a_frame_has_records_is_asked_of_any_frame():
     assert has_records(key_capacity=1 << 30) == 0 and has_records(n_triangles=1 << 31, n_vertices=1 << 33) == 0
 
 
+@pytest.mark.parametrize("n,keys_of_a_triangle,shown", [(499_999, 1.19, False), (500_000, 2.2, True), (524_288, 2.2, True), (524_289, 1.53, False),
+                                                        (524_289, 1.19, True), (1_000_000, 2.2, False), (1_000_000, 1.53, False),
+                                                        (1_690_000, 1.53, False), (1_700_000, 1.53, True), (1_700_000, 2.2, False), (2_000_000, 1.19, True)])
+def test_shown_frames_in_tile_order_have_records_where_the_forward_pass_alone_gains_by_them(n, keys_of_a_triangle, shown):
+    """In tile order the backward pass gains more by triangles' records than the forward pass, and a frame that is only shown has none:
+    by its triangles and keys.  In per-pixel order, and where a backward pass follows, neither matters."""
+    from trigrad_amd import _C, _lib
+    lib, capacity = _lib.load(32), _C._round_capacity(int(n * keys_of_a_triangle))
+    for per_pixel_sort, flags, expected in ((0, 0, shown), (0, _C._FRAME_BACKWARD | _C._FRAME_HIT_MASKS, n >= 500_000), (0, _C._FRAME_BACKWARD, n >= 500_000),
+                                            (1, 0, True), (1, _C._FRAME_BACKWARD | _C._FRAME_ORDER_PLANES, True), (1, _C._FRAME_BACKWARD, False)):
+        for records, n_vertices in ((1, 3 * n), (0, 3 * n), (1, 2 * n - 1)):
+            kind = _C._FRAME_KIND.pack(n_vertices, n, 1920, 1080, 16, 16, per_pixel_sort, 32, capacity, flags | records * _C._FRAME_RECORDS, 0, 0, 0.0)
+            assert lib.tg_frame_has_records(bytes(_C._FRAME_CALL.size + _C._FRAME_RESULT.size) + kind) == (expected and records and n_vertices == 3 * n)
+
+
 @pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
 def test_state_words_of_the_frame_scan_keep_their_place(few, many):
     """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more

@@ -34,15 +34,28 @@ struct FrameLayout {
 // frames in us, without and with: per-pixel order, train, 50 000 small triangles on 1024 x 1024 135, 135, 10^5 152, 154, 150 000
 // 173, 172, 200 000 197, 192, 500 000 347, 329, 10^6 670, 586; shown, 10^5 144, 146, 150 000 168, 168, 300 000 245, 237, 10^6
 // 997, 907 (lists of 700).  Tile order, train, 300 000 on 1920 x 1080 247, 251, 500 000 348, 343, 10^6 588, 565 (lists of 270), on 1024 x 1024
-// with lists of 400 573, 542, of 700 611, 609, on 512 x 512 with lists of 2000 549, 551, of 2800 393, 419.
+// with lists of 400 573, 542, of 700 611, 609, on 512 x 512 with lists of 2000 549, 551, of 2800 393, 419; with a heavy tail of large
+// triangles it is about the same, 800 000 on 1920 x 1080 707, 706, 1.2 million 818, 829, 2 million 1030, 1030.
+// Tile order, shown: the forward pass alone is to gain what the scan loses.  It does while the scan's workgroups with records are no more
+// than the CUs (524 288 triangles), where triangles are so small that lists are walked to their ends (mean edges of 1.5 pixels, 1.19 keys
+// a triangle), and from where the arrays are more than the memory-side cache holds, unless large triangles end the walks (2.19 keys).
+// 1920 x 1080, mean edges of 1.5, 4, 8 pixels, and of 4 with a heavy tail: 523 000 173, 162 and 193, 190 and 247, 250 and 251, 252; 530 000 179, 176
+// and 202, 208 and 255, 264 and 257, 271; 1.2 million 319, 316 and 357, 376 and 432, 470 and 399, 437; 1.6 million 406, 384 and 467, 463 and 583, 585 and
+// 494, 518; 1.76 million 454, 415 and 501, 495 and 643, 635 and 534, 552; 2.5 million 647, 560 and 754, 693 and 836, 788 and 662, 683.  (A
+// key buffer has room for an eighth and up to a sixteenth more than a frame's keys.)
 constexpr int64_t kRecordsTriangles = 150000, kRecordsTrianglesTileOrder = 500000, kRecordsListTileOrder = 800;
+constexpr int64_t kShownScanAtOnce = 256 * 2048, kShownBeyondCache = 1700000;
 static bool may_have_records(const tg_frame &f) {
     const bool backward_reads_matrices = (f.flags & TG_FRAME_BACKWARD) && f.per_pixel_sort && !(f.flags & (TG_FRAME_ORDER_PLANES | TG_FRAME_ORDER_POOL));
     return (f.flags & TG_FRAME_RECORDS) && f.n_triangles >= (f.per_pixel_sort ? kRecordsTriangles : kRecordsTrianglesTileOrder) && !backward_reads_matrices;
 }
 static bool has_records(const tg_frame &f) {
-    const int64_t tiles = ceil_div64(f.width, f.tile_w) * ceil_div64(f.height, f.tile_h);
-    return may_have_records(f) && f.n_vertices >= 2 * f.n_triangles && (f.per_pixel_sort || f.key_capacity <= kRecordsListTileOrder * tiles);
+    if (!may_have_records(f) || f.n_vertices < 2 * f.n_triangles) return false;
+    if (f.per_pixel_sort) return true;
+    const int64_t tiles = ceil_div64(f.width, f.tile_w) * ceil_div64(f.height, f.tile_h), M = f.n_triangles;
+    if (f.key_capacity > kRecordsListTileOrder * tiles) return false;
+    if ((f.flags & TG_FRAME_BACKWARD) || M <= kShownScanAtOnce) return true;
+    return 2 * f.key_capacity <= (M < kShownBeyondCache ? 3 * M : 4 * M);
 }
 
 // No size is larger for a smaller number of triangles, all else equal: callers size buffers for a rounded one.
