@@ -382,6 +382,42 @@ def test_shown_frames_in_tile_order_have_records_where_the_forward_pass_alone_ga
             assert lib.tg_frame_has_records(bytes(_C._FRAME_CALL.size + _C._FRAME_RESULT.size) + kind) == (expected and records and n_vertices == 3 * n)
 
 
+@pytest.mark.parametrize("per_pixel_sort,flags", [(1, 0), (1, 1 | 2), (1, 1 | 4 | 16), (0, 0), (0, 1 | 8)])
+def test_a_frame_without_records_keeps_no_room_for_them(per_pixel_sort, flags):
+    """A record takes 128 bytes a triangle where a matrix takes 36: a mesh, and a frame of long lists in tile order, keep the matrices' place
+    only, and the plan that later frames share has the room if, and only if, one of them may have records."""
+    from types import SimpleNamespace
+    from unittest import mock
+    from trigrad_amd import _C, _lib
+    left = {}
+    module = SimpleNamespace(remember=lambda key, kind, frame_bytes, low, high: left.update({key: kind}), state_bytes=lambda *_: 1 << 60)
+
+    def kept(n_vertices, n, capacity=3_000_000, records=_C._FRAME_RECORDS):
+        return _C._FramePlan(n_vertices, n, 1920, 1080, 16, 16, per_pixel_sort, 32, capacity, flags | records, 0.0).kept_bytes
+
+    def left_for(n_vertices, n):
+        left.clear()
+        with mock.patch.object(_C, "_module", lambda: module):
+            _C._leave_plan((n_vertices, n, 1920, 1080, 16, 16, per_pixel_sort, 32, 3_000_000, flags, 0.0), bool(flags & 1), SimpleNamespace(index=0), 0)
+        return list(left.items())
+
+    for n in (149_999, 150_000, 155_648, 499_999, 524_288, 524_289, 1_000_000, 1_300_000):
+        n_rounded, least = _C._round_count(n), 150_000 if per_pixel_sort else 500_000
+        assert kept(2 * n - 1, n) == kept(n // 2, n) == kept(3 * n, n, records=0)
+        assert round((kept(2 * n, n) - kept(n, n)) / n, 2) == (92 if n >= least else 0)
+        if not per_pixel_sort:
+            assert kept(3 * n, n, 8_000_000) == kept(3 * n, n, 8_000_000, records=0)
+        keys = set()
+        for n_vertices in (n // 2, 2 * n - 1, 2 * n, 3 * n):
+            (key, kind), = left_for(n_vertices, n)
+            keys.add(key)
+            of_plan = _C._FRAME_KIND.unpack(kind)[10]
+            assert of_plan >= kept(n_vertices, n)
+            assert of_plan == kept(0 if n_vertices < 2 * n else 3 * n_rounded, n_rounded)
+        assert len(keys) == 2
+    assert not left_for(0x7fffffff, (1 << 30) - 1) and len(left_for(0x7fffffff, 1 << 30)) == 1
+
+
 @pytest.mark.parametrize("few,many", [(1, 2049), (2048, 1 << 24), ((1 << 24) + 1, (1 << 25) + 1)])
 def test_state_words_of_the_frame_scan_keep_their_place(few, many):
     """What calls share in a frame state must lie where no call puts anything else, whatever its number of triangles: with more

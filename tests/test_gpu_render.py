@@ -1713,6 +1713,49 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
             assert (g - w).norm() <= 4 * (w2 - w).norm() + 1e-6 * w.norm()
 
 
+@pytest.mark.parametrize("mode,n", [("A_default", 149_999), ("A_default", 150_000), ("A_default", 150_001), ("A_40_layers", 150_037), ("B_unlimited", 499_999),
+                                    ("B_unlimited", 500_000), ("B_unlimited", 500_001)])
+def test_plans_of_frames_around_the_numbers_that_have_records(n, mode, cuda, oracle):
+    """Frames share the plan of a rounded number of triangles: with records and without them, and a mesh behind a soup of as many triangles;
+    the first frame of a kind by the Python route, later ones by the module's."""
+    import torch
+    import scenes as S
+    import trigrad_amd
+    from trigrad_amd import _C
+    m, width, height = MODES[mode], 520, 410
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    soup = S.random_soup(n, width, height, seed=n, sigma_px=0.6, opacity=(0.2, 0.9), varying_w=True)
+    mesh, k = S.random_soup(-(-n // 3), width, height, seed=n + 1, sigma_px=1.0, opacity=(0.2, 0.9), varying_w=True), -(-n // 3)
+    # each of its triangles is cut in three at its middle: four vertices for three
+    a, b, c, middle = *mesh["indices"].T, np.arange(3 * k, 4 * k)
+    mesh["indices"] = np.ascontiguousarray(np.stack([a, b, middle, b, c, middle, c, a, middle], axis=1).reshape(-1, 3)[:n], dtype=np.int32)
+    for name in ("vertices", "colors", "opacities"):
+        x = mesh[name].reshape(k, 3, -1)
+        mesh[name] = np.ascontiguousarray(np.concatenate([x.reshape(3 * k, -1), x.mean(axis=1)]).reshape(4 * k, *mesh[name].shape[1:]), dtype=np.float32)
+    mesh["vertices"][3 * k:, 3] = 1.0 / mesh["vertices"][3 * k:, 2]
+    expected = []
+    for scene in (soup, mesh):
+        want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, 16, 16, 1 / 256, m["per_pixel_sort"], ml)
+        gi, gd = _grad_inputs(scene, 4, True)
+        wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, 16, 16,
+                                        m["per_pixel_sort"], ml, literal=False, magnitudes=True)
+        d = to_device(scene, cuda)
+        plain = _C.frame_forward(d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, 16, 16, 1 / 256, m["per_pixel_sort"], ml, records=False)
+        expected.append((d, plain[:2], [torch.from_numpy(x).to(cuda) for x in (gi, gd)], wanted))
+    _C._module().forget()
+    for kind, routes in ((0, ("Python", "module")), (1, ("Python", "module")), (0, ("module",))):
+        d, plain, upstream, wanted = expected[kind]
+        leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+        for route in routes:
+            outputs = trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, per_pixel_sort=m["per_pixel_sort"], max_layers=m["max_layers"])
+            assert ("RendererBackward" in type(outputs[0].grad_fn).__name__) == (route == "Python")
+            for a, b in zip(outputs, plain):
+                assert torch.equal(a, b)
+            out = torch.autograd.grad(outputs, leaves, upstream)
+            for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+                assert_gradients_close(f"{n}/{mode}/{kind}/{route}: {label}", g.cpu().numpy(), w, mag)
+
+
 @pytest.mark.parametrize("n,width,height,tw,sigma", [(1, 64, 64, 16, 9.0), (511, 64, 64, 16, 2.0), (512, 300, 200, 16, 2.0), (513, 300, 200, 8, 6.0), (9000, 500, 400, 8, 6.0),
                                                      (131071, 640, 480, 16, 1.0), (131072, 640, 480, 16, 0.3), (131073, 640, 480, 16, 1.0),
                                                      (262144, 1000, 700, 16, 0.5), (262145, 1000, 700, 16, 2.0), (600000, 1000, 700, 16, 3.0)])

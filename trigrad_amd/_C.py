@@ -754,12 +754,15 @@ def _module():
 
 
 def _leave_plan(kind, for_backward, dev, stream):
-    """Hands a plan for the frames to come (and a frame state for the stream) to the torch module: for all numbers of vertices,
-    and of triangles up to the rounded one."""
-    _, n_triangles, width, height, tile_width, tile_height, per_pixel_sort, max_layers, capacity, flags, threshold = kind
+    """Hands a plan for the frames to come (and a frame state for the stream) to the torch module: for all numbers of vertices from
+    two a triangle on, or for all below that (whether triangles' records need room goes by it), and of triangles up to the rounded one."""
+    n_vertices, n_triangles, width, height, tile_width, tile_height, per_pixel_sort, max_layers, capacity, flags, threshold = kind
     limit = 0 if max_layers == n_triangles + 1 else max_layers  # 0: none
+    own_vertices = n_vertices >= 2 * n_triangles
     n_triangles = _round_count(n_triangles)
-    plan = _plan_for((0, n_triangles, width, height, tile_width, tile_height, per_pixel_sort,
+    if own_vertices and 2 * n_triangles > 0x7fffffff:
+        return  # no frame has that many vertices: there is no plan to make a room for this one's records by
+    plan = _plan_for((2 * n_triangles if own_vertices else 0, n_triangles, width, height, tile_width, tile_height, per_pixel_sort,
                       limit or min(n_triangles + 1, 0x7fffffff), capacity, flags | _FRAME_RECORDS, threshold))
     low, high = capacity // 4 if capacity > 1 << 18 else 0, 1 << 30
     if per_pixel_sort:
@@ -771,7 +774,8 @@ def _leave_plan(kind, for_backward, dev, stream):
             high = min(high, long_lists + long_lists // 4)
     module = _module()
     key = (dev.index, n_triangles, width, height, tile_width, tile_height,
-           struct.unpack("<q", struct.pack("<d", threshold))[0], per_pixel_sort, limit, 1 if for_backward else 0)
+           struct.unpack("<q", struct.pack("<d", threshold))[0], per_pixel_sort, limit, 1 if for_backward else 0,
+           1 if own_vertices else 0)
     module.remember(key, plan.kind, plan.frame_bytes, low, high)
     if module.state_bytes(dev.index, stream) < plan.frame_bytes:
         size = _state_size(plan.frame_bytes)

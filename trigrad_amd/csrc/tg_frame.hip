@@ -49,16 +49,21 @@ static bool may_have_records(const tg_frame &f) {
     const bool backward_reads_matrices = (f.flags & TG_FRAME_BACKWARD) && f.per_pixel_sort && !(f.flags & (TG_FRAME_ORDER_PLANES | TG_FRAME_ORDER_POOL));
     return (f.flags & TG_FRAME_RECORDS) && f.n_triangles >= (f.per_pixel_sort ? kRecordsTriangles : kRecordsTrianglesTileOrder) && !backward_reads_matrices;
 }
+// Where a frame's buffers have room for records: wherever it or one of fewer triangles has them.  A mesh, which has none, keeps 36 bytes a
+// triangle until its backward pass, and not 128.
+static bool has_room_for_records(const tg_frame &f) {
+    const int64_t tiles = ceil_div64(f.width, f.tile_w) * ceil_div64(f.height, f.tile_h);
+    return may_have_records(f) && f.n_vertices >= 2 * f.n_triangles && (f.per_pixel_sort || f.key_capacity <= kRecordsListTileOrder * tiles);
+}
 static bool has_records(const tg_frame &f) {
-    if (!may_have_records(f) || f.n_vertices < 2 * f.n_triangles) return false;
-    if (f.per_pixel_sort) return true;
-    const int64_t tiles = ceil_div64(f.width, f.tile_w) * ceil_div64(f.height, f.tile_h), M = f.n_triangles;
-    if (f.key_capacity > kRecordsListTileOrder * tiles) return false;
-    if ((f.flags & TG_FRAME_BACKWARD) || M <= kShownScanAtOnce) return true;
+    if (!has_room_for_records(f)) return false;
+    const int64_t M = f.n_triangles;
+    if (f.per_pixel_sort || (f.flags & TG_FRAME_BACKWARD) || M <= kShownScanAtOnce) return true;
     return 2 * f.key_capacity <= (M < kShownBeyondCache ? 3 * M : 4 * M);
 }
 
-// No size is larger for a smaller number of triangles, all else equal: callers size buffers for a rounded one.
+// No size is larger for a smaller number of triangles, all else equal: callers size buffers for a rounded one.  (For records that is so
+// among numbers of triangles with two vertices or more each, and among those with fewer: a plan is for the one or the other.)
 static FrameLayout frame_layout(const tg_frame &f) {
     FrameLayout L = {};
     const int tiles_x = (int)ceil_div64(f.width, f.tile_w), tiles_y = (int)ceil_div64(f.height, f.tile_h), tiles = tiles_x * tiles_y;
@@ -69,8 +74,7 @@ static FrameLayout frame_layout(const tg_frame &f) {
     L.status = take(4);  // of the sort
     L.ids = take((size_t)f.key_capacity * 4);
     L.offsets = take((size_t)(tiles + 1) * 4);
-    // the place of the records is that of the matrices; whether they are used goes by the number of vertices too, the size does not
-    L.bary = take((size_t)f.n_triangles * (may_have_records(f) ? sizeof(TriangleRecord) : 9 * sizeof(real)));
+    L.bary = take((size_t)f.n_triangles * (has_room_for_records(f) ? sizeof(TriangleRecord) : 9 * sizeof(real)));  // the records' place is that of the matrices
     L.weights = take((size_t)pixels * sizeof(real));
     L.ends = take((size_t)pixels * 4);
     if (backward) {

@@ -52,7 +52,8 @@ void check(int code, const char *what) {
 
 // The part of a call that a plan holds: struct tg_frame from n_vertices on.  The counts come with the frame: a viewer that
 // moves through a split scene, or a training loop that adds triangles, has others in every frame.  A plan's sizes are made
-// for the number of triangles rounded up (round_count), and no size a frame needs grows when its count gets smaller.
+// for the number of triangles rounded up (round_count), and no size a frame needs grows when its count gets smaller.  Only triangles
+// with two vertices or more each may have records (tg_frame_has_records), which take room: their plans are others.
 constexpr size_t kKindBytes = sizeof(tg_frame) - offsetof(tg_frame, n_vertices);
 struct Plan {
     std::array<char, kKindBytes> kind;
@@ -65,7 +66,7 @@ struct Plan {
         f.max_layers = max_layers;
     }
 };
-using PlanKey = std::array<int64_t, 10>;
+using PlanKey = std::array<int64_t, 11>;
 
 // As _round_count of the Python side: itself below 32, else up to a multiple of a sixteenth to a thirty-second of itself.
 int64_t round_count(int64_t n) {
@@ -287,7 +288,7 @@ PyObject *py_render(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (layers <= 0) layers = n_triangles + 1;  // no limit
     const PlanKey key = {vertices.device().index(), round_count(n_triangles), PyLong_AsLongLong(args[4]), PyLong_AsLongLong(args[5]),
                          PyLong_AsLongLong(args[6]), PyLong_AsLongLong(args[7]), threshold_bits, args[10] == Py_True,
-                         layers == n_triangles + 1 ? 0 : layers, backward};
+                         layers == n_triangles + 1 ? 0 : layers, backward, n_vertices >= 2 * n_triangles};
     if (PyErr_Occurred()) {  // an integer beyond 64 bits
         PyErr_Clear();
         Py_RETURN_NONE;
@@ -362,20 +363,20 @@ PyObject *py_bind(PyObject *, PyObject *args) {
     Py_RETURN_NONE;
 }
 
-// remember(key of ten integers, plan bytes, frame bytes, keys_low, keys_high): a plan for frames of this kind
+// remember(key of eleven integers, plan bytes, frame bytes, keys_low, keys_high): a plan for frames of this kind
 PyObject *py_remember(PyObject *, PyObject *args) {
     PlanKey key = {};
-    long long k[10], frame_bytes, low, high;
+    long long k[11], frame_bytes, low, high;
     const char *bytes;
     Py_ssize_t size;
-    if (!PyArg_ParseTuple(args, "(LLLLLLLLLL)y#LLL", &k[0], &k[1], &k[2], &k[3], &k[4], &k[5], &k[6], &k[7], &k[8], &k[9], &bytes, &size,
-                          &frame_bytes, &low, &high))
+    if (!PyArg_ParseTuple(args, "(LLLLLLLLLLL)y#LLL", &k[0], &k[1], &k[2], &k[3], &k[4], &k[5], &k[6], &k[7], &k[8], &k[9], &k[10], &bytes,
+                          &size, &frame_bytes, &low, &high))
         return nullptr;
     if ((size_t)size != kKindBytes) {
         PyErr_SetString(PyExc_ValueError, "the plan's constant part has another size");
         return nullptr;
     }
-    for (int j = 0; j < 10; j++) key[j] = k[j];
+    for (int j = 0; j < 11; j++) key[j] = k[j];
     auto plan = std::make_shared<Plan>();
     std::memcpy(plan->kind.data(), bytes, kKindBytes);
     plan->frame_bytes = frame_bytes;
