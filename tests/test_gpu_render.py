@@ -1713,6 +1713,37 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
             assert (g - w).norm() <= 4 * (w2 - w).norm() + 1e-6 * w.norm()
 
 
+def test_reaches_in_records_are_outside_of_their_triangles_and_not_far(cuda):
+    """A record's bounds are steps of 2^-14 rounded to the outside, held in [-2, 2): no triangle's corner is beyond them, those of triangles of
+    some pixels are no further out than two steps and a tenth of a pixel wherever on the screen, and NaN and infinity leave nothing out."""
+    import scenes as S
+    from trigrad_amd import _C
+    n, width, height = 160_037, 1920, 1080
+    scene = S.random_soup(n, width, height, seed=3, sigma_px=3.0, varying_w=True)
+    v = scene["vertices"].reshape(n, 3, 4)
+    v[:1000, :, :2] *= 3.0  # partly and wholly beside the image
+    v[1000, 0, 0], v[1001, 1, 1] = np.nan, np.inf
+    d = to_device(scene, cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, 16, 16, 1 / 256, True, 32)
+    _, _, kept, frame = _C.frame_forward(*args)
+    assert frame.records
+    at = frame.plan.at["bary"]
+    words = kept[at:at + 128 * n].cpu().numpy().view(np.int32).reshape(n, 32)[:, 15:17]
+    lo, hi = ((words << 16) >> 16) / 2.0 ** 14, (words >> 16) / 2.0 ** 14  # (n, 2): x and y
+    xy = v[..., :2].astype(np.float64)
+    least, most = xy.min(axis=1), xy.max(axis=1)
+    fine = np.isfinite(xy).all(axis=(1, 2))
+    top = 2.0 - 2.0 ** -14
+    assert (lo[fine] <= np.maximum(least[fine], -2.0)).all() and (hi[fine] >= np.minimum(most[fine], top)).all()
+    assert (lo[1000:1002] == -2.0).all() and (hi[1000:1002] == top).all()  # in both directions: the matrix is of NaN
+    e = (xy[:, 1:] - xy[:, :1]) * [width / 2, height / 2]
+    longest = np.sqrt(np.maximum(np.maximum((e ** 2).sum(axis=2).max(axis=1), ((e[:, 1] - e[:, 0]) ** 2).sum(axis=1)), 1e-30))
+    round_ones = fine & (np.abs(e[:, 0, 0] * e[:, 1, 1] - e[:, 0, 1] * e[:, 1, 0]) > 3.0 * longest) & (np.abs(xy).max(axis=(1, 2)) < 1.5)
+    assert round_ones.sum() > n // 8
+    slack = 2 * 2.0 ** -14 + 0.1 * np.array([2 / width, 2 / height])
+    assert (least - lo <= slack)[round_ones].all() and (hi - most <= slack)[round_ones].all()
+
+
 @pytest.mark.parametrize("mode,n", [("A_default", 149_999), ("A_default", 150_000), ("A_default", 150_001), ("A_40_layers", 150_037), ("B_unlimited", 499_999),
                                     ("B_unlimited", 500_000), ("B_unlimited", 500_001)])
 def test_plans_of_frames_around_the_numbers_that_have_records(n, mode, cuda, oracle):

@@ -278,7 +278,8 @@ typedef int int3v __attribute__((ext_vector_type(3)));
 // 10^6 triangles on 1920 x 1080, us, without and with: forward per-pixel order 470, 421 and behind a backward pass, whose gradients
 // have taken the caches, 518, 414; tile order 209, 187; backward 911, 880 and 365, 345; the scan 45, 69.  200 000 faint ones, lists of 3700:
 // forward 274, 254, backward 203, 196.
-// The reach is kept in 16 bits a bound, rounded to the outside.
+// The reach is kept in 16 bits a bound, in fixed steps rounded to the outside: a sixteenth of a pixel of 1920 columns or less everywhere
+// (halves, a pixel coarse where the image's edges are: 10^6 triangles, frames, train 1485 -> 1479, shown 591 -> 586).
 struct TriangleRecord {
     real4v q[8];  // matrix 0..3 | matrix 4..7 | matrix 8, z | w, reach in x | reach in y, opacities | colours 0..3 | colours 4..7 | colours 8, vertex numbers
 
@@ -316,14 +317,15 @@ struct TriangleRecord {
     }
     __device__ __forceinline__ int3v vertices() const { return int3v{int_of_real((real)q[7][1]), int_of_real((real)q[7][2]), int_of_real((real)q[7][3])}; }
 
-    // Two bounds as halves, rounded away from each other: a half is within 2^-11 of a number, or 2^-25 beside zero.
+    // Two bounds in steps of 2^-14, rounded away from each other and held in [-2, 2), which no pixel is beyond; NaN leaves nothing out.
     static __device__ __forceinline__ uint32_t pack_bounds(float lo, float hi) {
-        const _Float16 l = (_Float16)(lo - __builtin_fmaf(__builtin_fabsf(lo), 0x1p-10f, 0x1p-20f));
-        const _Float16 h = (_Float16)(hi + __builtin_fmaf(__builtin_fabsf(hi), 0x1p-10f, 0x1p-20f));
-        return (uint32_t)__builtin_bit_cast(uint16_t, l) | (uint32_t)__builtin_bit_cast(uint16_t, h) << 16;
+        constexpr float kStep = 0x1p-14f, kLeast = -2.0f, kMost = 2.0f - kStep;
+        const int l = (int)__builtin_floorf(__builtin_fminf(__builtin_fmaxf(lo, kLeast), kMost) / kStep);
+        const int h = (int)__builtin_ceilf(__builtin_fmaxf(__builtin_fminf(hi, kMost), kLeast) / kStep);
+        return (uint32_t)(uint16_t)l | (uint32_t)h << 16;
     }
-    static __device__ __forceinline__ real lower(real packed) { return (real)__builtin_bit_cast(_Float16, (uint16_t)(uint32_t)int_of_real(packed)); }
-    static __device__ __forceinline__ real upper(real packed) { return (real)__builtin_bit_cast(_Float16, (uint16_t)((uint32_t)int_of_real(packed) >> 16)); }
+    static __device__ __forceinline__ real lower(real packed) { return (real)0x1p-14f * (real)(int16_t)int_of_real(packed); }
+    static __device__ __forceinline__ real upper(real packed) { return (real)0x1p-14f * (real)(int16_t)(int_of_real(packed) >> 16); }
     static __device__ __forceinline__ Reach unpack_reach(real x, real y) { return Reach{lower(x), upper(x), lower(y), upper(y)}; }
     __device__ __forceinline__ Reach reach() const { return unpack_reach(q[3][3], q[4][0]); }
     __device__ __forceinline__ real height() const { return upper(q[4][0]) - lower(q[4][0]); }
