@@ -1713,6 +1713,41 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
             assert (g - w).norm() <= 4 * (w2 - w).norm() + 1e-6 * w.norm()
 
 
+@pytest.mark.parametrize("mode,n", [("A_default", 160_037), ("A_40_layers", 270_011), ("B_unlimited", 510_001), ("A_default", 140_000)])
+def test_timed_frames_run_the_kernels_of_untimed_ones(n, mode, cuda, oracle, monkeypatch):
+    """The stages that record_timing=True times are those of the frame that a user gets without asking: from triangles' records where that
+    one is; the same image and, by the route by stages with the matrices out of the records, the gradients."""
+    import torch
+    import scenes as S
+    import trigrad_amd
+    from trigrad_amd import _C
+    m, width, height = MODES[mode], 520, 410
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    scene = S.random_soup(n, width, height, seed=n, sigma_px=0.6, opacity=(0.2, 0.9), varying_w=True)
+    want = oracle.render(scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], width, height, 16, 16, 1 / 256, m["per_pixel_sort"], ml)
+    gi, gd = _grad_inputs(scene, 6, True)
+    wanted = oracle.render_backward(gi, gd, scene["vertices"], scene["indices"], scene["colors"], scene["opacities"], want, width, height, 16, 16,
+                                    m["per_pixel_sort"], ml, literal=False, magnitudes=True)
+    rendered, frame_forward = [], _C.frame_forward
+
+    def seen(*args, **kwargs):
+        rendered.append(frame_forward(*args, **kwargs))
+        return rendered[-1]
+
+    monkeypatch.setattr(_C, "frame_forward", seen)
+    _C._module().forget()  # an untimed frame by the Python route too
+    d = to_device(scene, cuda)
+    leaves = [d[k].clone().requires_grad_() for k in ("vertices", "colors", "opacities")]
+    frames = [trigrad_amd.render(leaves[0], d["indices"], *leaves[1:], width, height, record_timing=timed, per_pixel_sort=m["per_pixel_sort"],
+                                 max_layers=m["max_layers"]) for timed in (False, True)]
+    assert [f[3].records for f in rendered] == [n != 140_000] * 2 and "rasterization" in frames[1][2]
+    for outputs in frames:
+        assert torch.equal(outputs[0], frames[0][0]) and torch.equal(outputs[1], frames[0][1])
+        out = torch.autograd.grad(outputs[:2], leaves, (torch.from_numpy(gi).to(cuda), torch.from_numpy(gd).to(cuda)))
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), out, wanted[:3], wanted[3:]):
+            assert_gradients_close(f"{n}/{mode}: {label}", g.cpu().numpy(), w, mag)
+
+
 def test_reaches_in_records_are_outside_of_their_triangles_and_not_far(cuda):
     """A record's bounds are steps of 2^-14 rounded to the outside, held in [-2, 2): no triangle's corner is beyond them, those of triangles of
     some pixels are no further out than two steps and a tenth of a pixel wherever on the screen, and NaN and infinity leave nothing out."""

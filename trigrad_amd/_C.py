@@ -989,10 +989,12 @@ def _forward_full(vertices, indices, colors, opacities, width, height, tile_widt
     real = vertices.dtype
     timer = _StageTimer(disable_timing)
     dev = vertices.device
+    # a timed frame runs the kernels that an untimed `render` does, from triangles' records too; without timing this is the caller's who
+    # wants the matrices as they are
     if frame_supported(vertices, width, height, tile_width, tile_height):
         image, depthmap, kept, frame = frame_forward(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
                                                      early_stopping_threshold, per_pixel_sort, int(max_layers), for_backward,
-                                                     None if disable_timing else timer, records=False)
+                                                     None if disable_timing else timer, records=not disable_timing)
         timings = timer.stop()
         if not disable_timing:  # the timer has waited for the stream anyway
             if frame.status.failed() and not _tickets_forced:
