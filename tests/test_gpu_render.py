@@ -1665,9 +1665,10 @@ def test_waves_at_the_edges_of_an_image(width, height, tw, th, mode, cuda, oracl
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "A_unlimited", "B_unlimited"])
 @pytest.mark.parametrize("width,height,tw,th,big", [(520, 410, 16, 16, 0), (301, 203, 8, 8, 0), (300, 200, 32, 32, 3000), (160, 120, 16, 16, 900), (1920, 400, 16, 16, 0)])
 @pytest.mark.parametrize("saved", [True, False])
-def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, big, mode, cuda, monkeypatch):
+def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, big, mode, cuda, oracle, monkeypatch):
     """Many triangles with vertices of their own are rendered from records (TG_FRAME_RECORDS), others from the arrays: the same image, depth
-    map and lists, and gradients the same up to the order of the atomics; tiles of one and several workgroups, frames of few and
+    map and lists, and gradients the same up to the order of the atomics, each of them as near the oracle's as two sums in another order
+    are; tiles of one and several workgroups, frames of few and
     many, and lists of thousands, which depth bounds and the long tiles' kernels are for; in tile order without the saved hit masks too (in per-pixel order a backward pass
     without a saved order reads the matrices, so there are no records).  Some triangles name a vertex that is
     none, some are degenerate or far off the screen, and some attributes are zero or infinite."""
@@ -1677,7 +1678,8 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
     m = MODES[mode]
     monkeypatch.setattr(_C, "SAVE_HIT_MASKS", saved)
     monkeypatch.setattr(_C, "SAVE_BLEND_ORDER", saved)
-    n = 160_000 if m["per_pixel_sort"] else 510_000
+    # two triangles a thread of the scan, and four; a wave's last triangles are fewer than its lanes
+    n = (270_011 if tw == 8 else 160_037) if m["per_pixel_sort"] else 510_001
     ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
     rng = np.random.default_rng(width)
     scene = S.random_soup(n, width, height, seed=width, sigma_px=0.6, opacity=(0.2, 0.9), varying_w=True)
@@ -1703,6 +1705,12 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
         a, b = results[0][k], results[1][k]
         assert a.shape == b.shape and torch.equal(torch.nan_to_num(a.double(), 7.0), torch.nan_to_num(b.double(), 7.0))
     gi, gd = (torch.from_numpy(x).to(cuda) for x in _grad_inputs(scene, 3, True))
+    if packed[3].records:
+        known = dict(scene, indices=scene["indices"].copy())
+        known["indices"][5002:5004] = 0  # in no list either
+        known = [known[k] for k in ("vertices", "indices", "colors", "opacities")]
+        rendered = oracle.render(*known, width, height, tw, th, 1 / 256, m["per_pixel_sort"], ml)
+        known += [rendered, width, height, tw, th, m["per_pixel_sort"], ml]
     for depth_gradient in (None, gd):
         got, want = (_C.frame_backward(f[3], gi, depth_gradient, *args[:4], f[0], f[1], f[2]) for f in (packed, plain))
         again = _C.frame_backward(plain[3], gi, depth_gradient, *args[:4], plain[0], plain[1], plain[2])
@@ -1711,6 +1719,14 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
             g, w, w2 = (torch.nan_to_num(x, 0.0, 0.0, 0.0).double() for x in (g, w, w2))
             # two runs of one route differ by the order of their atomics; the two routes by no more than four times that
             assert (g - w).norm() <= 4 * (w2 - w).norm() + 1e-6 * w.norm()
+        if not packed[3].records:
+            continue
+        wanted = oracle.render_backward(gi.cpu().numpy(), np.zeros((height, width), np.float32) if depth_gradient is None else gd.cpu().numpy(), *known,
+                                        literal=False, magnitudes=True)
+        for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), got, wanted[:3], wanted[3:]):
+            finite = np.isfinite(w) & np.isfinite(mag)  # an infinite colour is not in the sums of all
+            assert finite.mean() > 0.99
+            assert_gradients_close(f"{n} in {width}x{height}/{mode}: {label}", g.cpu().numpy()[finite], w[finite], mag[finite])
 
 
 @pytest.mark.parametrize("mode,n", [("A_default", 160_037), ("A_40_layers", 270_011), ("B_unlimited", 510_001), ("A_default", 140_000)])
