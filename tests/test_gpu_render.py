@@ -1764,6 +1764,23 @@ def test_timed_frames_run_the_kernels_of_untimed_ones(n, mode, cuda, oracle, mon
             assert_gradients_close(f"{n}/{mode}: {label}", g.cpu().numpy(), w, mag)
 
 
+@pytest.mark.parametrize("n,mode", [(160_037, "A_default"), (510_001, "B_unlimited"), (140_000, "A_default")])
+@pytest.mark.parametrize("disable_timing", [True, False])
+def test_matrices_of_render_forward_are_a_dense_array(disable_timing, n, mode, cuda):
+    """render_forward hands out the bary matrices as an array of their own, of frames with timing too, and so a kernel or a view takes them
+    as they are."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    m, width, height = MODES[mode], 520, 410
+    d = to_device(S.random_soup(n, width, height, seed=n, sigma_px=0.6), cuda)
+    bary = _C.render_forward(d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, 16, 16, 1 / 256, disable_timing,
+                             m["per_pixel_sort"], 32)[5]
+    assert bary.shape == (n, 3, 3) and bary.is_contiguous()
+    want = _C.cartesian_to_bary(d["vertices"], d["indices"])
+    assert torch.equal(bary.view(-1), want.view(-1))
+
+
 def test_reaches_in_records_are_outside_of_their_triangles_and_not_far(cuda):
     """A record's bounds are steps of 2^-14 rounded to the outside, held in [-2, 2): no triangle's corner is beyond them, those of triangles of
     some pixels are no further out than two steps and a tenth of a pixel wherever on the screen, and NaN and infinity leave nothing out."""

@@ -977,11 +977,12 @@ def _frame_results(image, depthmap, kept, frame, width, height, tile_width, tile
 
 
 def _forward_full(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
-                  early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward=True):
+                  early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward=True, records=False):
     """render_forward's eight results plus `resume` = (last, last_depth, status_check, fragments, hit_masks):
     what the backward pass needs for its reverse traversal (fragments / hit_masks are None unless the blend
     order / the hit masks were saved) and the status word of the list kernels on its way to the host.
-    for_backward=False: no backward pass will follow, nothing is saved for it."""
+    for_backward=False: no backward pass will follow, nothing is saved for it.  records: the kernels are those of `render`, from triangles'
+    records where the frame has them; the bary matrices are then a view of those, and no dense array."""
     _need_cuda(vertices, indices, colors, opacities)
     verify_finished_frames()
     bits = _bits(vertices)
@@ -989,19 +990,17 @@ def _forward_full(vertices, indices, colors, opacities, width, height, tile_widt
     real = vertices.dtype
     timer = _StageTimer(disable_timing)
     dev = vertices.device
-    # a timed frame runs the kernels that an untimed `render` does, from triangles' records too; without timing this is the caller's who
-    # wants the matrices as they are
     if frame_supported(vertices, width, height, tile_width, tile_height):
         image, depthmap, kept, frame = frame_forward(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
                                                      early_stopping_threshold, per_pixel_sort, int(max_layers), for_backward,
-                                                     None if disable_timing else timer, records=not disable_timing)
+                                                     None if disable_timing else timer, records)
         timings = timer.stop()
         if not disable_timing:  # the timer has waited for the stream anyway
             if frame.status.failed() and not _tickets_forced:
                 # the lists are invalid (and the image NaN): the whole frame once more, its tiles numbered by ticket
                 force_tickets(True)
                 return _forward_full(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
-                                     early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward)
+                                     early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward, records)
             frame.status.checked = False
             frame.status.verify()
         *results, resume = _frame_results(image, depthmap, kept, frame, width, height, tile_width, tile_height, per_pixel_sort,
@@ -1107,7 +1106,7 @@ def _forward_full(vertices, indices, colors, opacities, width, height, tile_widt
                 # the lists are invalid (and the image NaN): the whole frame once more, its tiles numbered by ticket
                 force_tickets(True)
                 return _forward_full(vertices, indices, colors, opacities, width, height, tile_width, tile_height,
-                                     early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward)
+                                     early_stopping_threshold, disable_timing, per_pixel_sort, max_layers, for_backward, records)
             status_check.checked = False
             status_check.verify()
     resume = Resume((last, last_depth, status_check, fragments, hit_masks))

@@ -64,7 +64,8 @@ class Renderer(Function):
             ctx.frame = None
             (image, depthmap, final_weights, sorted_ids, offsets, bary_transforms, ends, timings, resume) = _C._forward_full(
                 vertices, indices, colors, opacities, width, height, tile_width, tile_height, early_stopping_threshold,
-                not record_timing, per_pixel_sort, max_layers, for_backward=any(ctx.needs_input_grad))
+                not record_timing, per_pixel_sort, max_layers, for_backward=any(ctx.needs_input_grad),
+                records=True)  # a timed frame runs the kernels of one without timing
             last, last_depth, status_check, fragments, hit_masks = resume
             # private to this Function: where the reverse traversal starts, and the blend order (per-pixel
             # order, max_layers <= 32) or the hit masks (tile order); the list kernels' status word, which the
