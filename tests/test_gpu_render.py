@@ -1665,10 +1665,9 @@ def test_waves_at_the_edges_of_an_image(width, height, tw, th, mode, cuda, oracl
 @pytest.mark.parametrize("mode", ["A_default", "A_40_layers", "A_unlimited", "B_unlimited"])
 @pytest.mark.parametrize("width,height,tw,th,big", [(520, 410, 16, 16, 0), (301, 203, 8, 8, 0), (300, 200, 32, 32, 3000), (160, 120, 16, 16, 900), (1920, 400, 16, 16, 0)])
 @pytest.mark.parametrize("saved", [True, False])
-def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, big, mode, cuda, oracle, monkeypatch):
+def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, big, mode, cuda, monkeypatch):
     """Many triangles with vertices of their own are rendered from records (TG_FRAME_RECORDS), others from the arrays: the same image, depth
-    map and lists, and gradients the same up to the order of the atomics, each of them as near the oracle's as two sums in another order
-    are; tiles of one and several workgroups, frames of few and
+    map and lists, and gradients the same up to the order of the atomics; tiles of one and several workgroups, frames of few and
     many, and lists of thousands, which depth bounds and the long tiles' kernels are for; in tile order without the saved hit masks too (in per-pixel order a backward pass
     without a saved order reads the matrices, so there are no records).  Some triangles name a vertex that is
     none, some are degenerate or far off the screen, and some attributes are zero or infinite."""
@@ -1678,8 +1677,7 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
     m = MODES[mode]
     monkeypatch.setattr(_C, "SAVE_HIT_MASKS", saved)
     monkeypatch.setattr(_C, "SAVE_BLEND_ORDER", saved)
-    # two triangles a thread of the scan, and four; a wave's last triangles are fewer than its lanes
-    n = (270_011 if tw == 8 else 160_037) if m["per_pixel_sort"] else 510_001
+    n = 160_000 if m["per_pixel_sort"] else 510_000
     ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
     rng = np.random.default_rng(width)
     scene = S.random_soup(n, width, height, seed=width, sigma_px=0.6, opacity=(0.2, 0.9), varying_w=True)
@@ -1705,12 +1703,6 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
         a, b = results[0][k], results[1][k]
         assert a.shape == b.shape and torch.equal(torch.nan_to_num(a.double(), 7.0), torch.nan_to_num(b.double(), 7.0))
     gi, gd = (torch.from_numpy(x).to(cuda) for x in _grad_inputs(scene, 3, True))
-    if packed[3].records:
-        known = dict(scene, indices=scene["indices"].copy())
-        known["indices"][5002:5004] = 0  # in no list either
-        known = [known[k] for k in ("vertices", "indices", "colors", "opacities")]
-        rendered = oracle.render(*known, width, height, tw, th, 1 / 256, m["per_pixel_sort"], ml)
-        known += [rendered, width, height, tw, th, m["per_pixel_sort"], ml]
     for depth_gradient in (None, gd):
         got, want = (_C.frame_backward(f[3], gi, depth_gradient, *args[:4], f[0], f[1], f[2]) for f in (packed, plain))
         again = _C.frame_backward(plain[3], gi, depth_gradient, *args[:4], plain[0], plain[1], plain[2])
@@ -1719,10 +1711,47 @@ def test_frames_with_records_of_their_triangles(saved, width, height, tw, th, bi
             g, w, w2 = (torch.nan_to_num(x, 0.0, 0.0, 0.0).double() for x in (g, w, w2))
             # two runs of one route differ by the order of their atomics; the two routes by no more than four times that
             assert (g - w).norm() <= 4 * (w2 - w).norm() + 1e-6 * w.norm()
-        if not packed[3].records:
-            continue
-        wanted = oracle.render_backward(gi.cpu().numpy(), np.zeros((height, width), np.float32) if depth_gradient is None else gd.cpu().numpy(), *known,
-                                        literal=False, magnitudes=True)
+
+
+# two triangles a thread of the scan, and four; a wave's last triangles are fewer than its lanes
+@pytest.mark.parametrize("width,height,tile,n,mode", [(*size, mode) for size in ((520, 410, 16, 160_037), (301, 203, 8, 270_011), (300, 200, 32, 160_037), (1920, 400, 16, 270_011))
+                                                      for mode in ("A_default", "A_40_layers", "A_unlimited", "B_unlimited")
+                                                      if mode != "B_unlimited" or size[2] < 32])  # in tile order frames of long lists have no records
+def test_gradients_by_element_of_frames_with_records(width, height, tile, n, mode, cuda, oracle):
+    """Each gradient of a frame with triangles' records is as near the oracle's as sums in another order are, and its image, depth map and lists are
+    those without; the last triangles are those of a wave with lanes to spare, some name a vertex that is none, and an infinite colour is
+    in the sums of few."""
+    import torch
+    import scenes as S
+    from trigrad_amd import _C
+    m = MODES[mode]
+    n = n if m["per_pixel_sort"] else 510_001
+    ml = m["max_layers"] if m["max_layers"] > 0 else n + 1
+    scene = S.random_soup(n, width, height, seed=width, sigma_px=0.6, opacity=(0.2, 0.9), varying_w=True)
+    scene["vertices"].reshape(n, 3, 4)[-64:, :, :2] *= 0.3  # on the image
+    scene["colors"][15033:15036] = np.inf
+    idx = scene["indices"].copy()
+    idx[5002, 1], idx[5003, 2] = 3 * n, -1
+    d = to_device(dict(scene, indices=idx), cuda)
+    args = (d["vertices"], d["indices"], d["colors"], d["opacities"], width, height, tile, tile, 1 / 256, m["per_pixel_sort"], ml)
+    for _ in range(2):  # the second frame's buffers go by the first one's keys
+        packed, plain = _C.frame_forward(*args), _C.frame_forward(*args, records=False)
+    assert packed[3].records and not plain[3].records
+    for a, b in zip(packed[:2], plain[:2]):
+        assert torch.equal(torch.nan_to_num(a, 7.0), torch.nan_to_num(b, 7.0)) and torch.equal(torch.isnan(a), torch.isnan(b))
+    results = [_C._frame_results(*f, width, height, tile, tile, m["per_pixel_sort"], ml, n) for f in (packed, plain)]
+    for k in (2, 3, 4, 5, 6):  # weights, sorted ids, offsets, bary matrices, ends
+        a, b = results[0][k], results[1][k]
+        assert a.shape == b.shape and torch.equal(torch.nan_to_num(a.double(), 7.0), torch.nan_to_num(b.double(), 7.0))
+    known = dict(scene, indices=scene["indices"].copy())
+    known["indices"][5002:5004] = 0  # in no list either
+    known = [known[k] for k in ("vertices", "indices", "colors", "opacities")]
+    known += [oracle.render(*known, width, height, tile, tile, 1 / 256, m["per_pixel_sort"], ml), width, height, tile, tile, m["per_pixel_sort"], ml]
+    gi, gd = _grad_inputs(scene, 3, True)
+    for depth_gradient in (None, gd):
+        wanted = oracle.render_backward(gi, np.zeros_like(gd) if depth_gradient is None else gd, *known, literal=False, magnitudes=True)
+        got = _C.frame_backward(packed[3], torch.from_numpy(gi).to(cuda), None if depth_gradient is None else torch.from_numpy(gd).to(cuda),
+                                *args[:4], packed[0], packed[1], packed[2])
         for label, g, w, mag in zip(("grad_vertices", "grad_colors", "grad_opacities"), got, wanted[:3], wanted[3:]):
             finite = np.isfinite(w) & np.isfinite(mag)  # an infinite colour is not in the sums of all
             assert finite.mean() > 0.99
