@@ -452,7 +452,7 @@ int tg_frame_gradient_copies(const tg_frame *f);
 #define TG_FRAME_ORDER_POOL 4   /*   ... the blend order in a pool (tg_order_pool_words) */
 #define TG_FRAME_HIT_MASKS 8    /*   ... the hit masks (tile order) */
 #define TG_FRAME_LIST_BOUNDS 16 /*   depth bounds of the lists (tg_list_bounds) for the per-pixel selection */
-#define TG_FRAME_RECORDS 32     /*   the place of the bary matrices may hold records of all that is read of a triangle instead (tg_frame_has_records) */
+#define TG_FRAME_RECORDS 32     /*   the place of the bary matrices may hold records of what is read of a triangle instead (tg_frame_has_records) */
 #define TG_FRAME_BIN 1          /* phases */
 #define TG_FRAME_LISTS 2
 #define TG_FRAME_RASTER 4

@@ -52,7 +52,7 @@ __device__ __forceinline__ bool lists_invalid(const BackwardArgs &g) { return g.
 // Most losses are of the image alone: kDepth = false is for a frame whose depth map has no gradient.  Its terms by way of the depth
 // are then zeros, a sixth of a fragment's arithmetic, and are left out, but for the cases where they are 0 times infinity: the
 // NaNs that make of a gradient are kept (depth_is_ordinary, load_back_state).  One kind is not: where the depth's derivative by an
-// opacity (fragment_chain_step) overflows although the pixel's depth is finite, which takes a depth beyond 1e34 or one
+// opacity (fragment_seed) overflows although the pixel's depth is finite, which takes a depth beyond 1e34 or one
 // beyond 1e38 times its fragment's opacity, the gradients of that fragment are what the image alone makes them.  The saved-order
 // kernel then needs 96 registers, not 117, and five waves a SIMD find room: 10^6 triangles 1219 -> 1043 us, 20 000 without a limit on the
 // layers 604 -> 541; in tile order 619 -> 594.

@@ -1201,7 +1201,7 @@ namespace tg {
 struct FusedFrame {
     uint32_t *totals;  // two sets of kEmitDigitPasses * kRadix digit totals
     uint32_t *ticket;
-    uint64_t *states;  // one word per kScanTile triangles (for a few hundred thousand there may be four times as many, and room)
+    uint64_t *states;  // one word per workgroup of the scan: for kScanTile triangles, half as many up to 262 144, and a quarter up to 131 072 without records
     real *edges;       // tiles_x + 1 column edges, then tiles_y + 1 row edges
     uint32_t *heads;   // the owner of a chunk's first key position, for each chunk
     uint32_t *tri_offsets;

@@ -272,8 +272,8 @@ typedef real real3v __attribute__((ext_vector_type(3)));
 typedef real real4v __attribute__((ext_vector_type(4)));
 typedef int int3v __attribute__((ext_vector_type(3)));
 
-// All that the passes read of a triangle, in one piece of 128 bytes (a line of the L2): made by frame_scan_kernel, which has its vertices
-// in hand.  A list entry's triangle can be anywhere, and by itself its matrix, vertex numbers, vertices, opacities and colours are on
+// All that the forward pass reads of a triangle, in one piece of 128 bytes (a line of the L2): made by frame_scan_kernel, which has its vertices
+// in hand.  (The backward pass reads x and y of the vertices too, from the array, by the record's vertex numbers.)  A list entry's triangle can be anywhere, and by itself its matrix, vertex numbers, vertices, opacities and colours are on
 // six or seven lines, each fetched whole for a few bytes and through three loads that wait for each other.
 // 10^6 triangles on 1920 x 1080, us, without and with: forward per-pixel order 470, 421 and behind a backward pass, whose gradients
 // have taken the caches, 518, 414; tile order 209, 187; backward 911, 880 and 365, 345; the scan 45, 69.  200 000 faint ones, lists of 3700:

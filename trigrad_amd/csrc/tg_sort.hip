@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kSweepThreads) void sort_sweep_kernel(const uint64_
     __shared__ uint32_t s_base_wave[kSweepWaves];
     __shared__ uint32_t s_several_tiles[kRadix];  // with tile_count: the digit's pairs of this sort tile belong to more than one tile
     // The ranking counters are dead once every pair knows its place in the tile,
-    // so they share LDS with the permutation buffer (51 KB: three workgroups per CU).
+    // so they share LDS with the permutation buffer (with eight pairs a thread 51 KB: three workgroups per CU).
     constexpr int kMaskOffset = (kSweepWaves + 1) * kRadix * 4;
     constexpr int kCounterBytes = kMaskOffset + kSweepWaves * kMaskWords * 8;
     __shared__ __align__(16) unsigned char s_raw[kTile * 12 > kCounterBytes ? kTile * 12 : kCounterBytes];
